@@ -532,6 +532,14 @@ int mllm_hip_softmax(const float* x, float* y, int64_t rows, int64_t len, void* 
  * replaces: CPUTopKOp::forward  mllm/backends/cpu/ops/TopKOp.cpp:20-72 */
 int mllm_hip_topk(const float* x, float* values, int32_t* indices, int64_t rows, int64_t len, int k, int largest, int sorted,
                   void* stream);
+/* The same two with a workspace (its size from the *_bytes call; 0 or a NULL workspace: the calls above).  Few long rows -- the
+ * logits of a vocabulary -- are then cut into pieces with a workgroup each that meet in the workspace, instead of one workgroup
+ * per row: three launches for softmax, two for top-k.  Same values and indices for top-k; softmax adds a row's terms in another order. */
+size_t mllm_hip_softmax_workspace_bytes(int64_t rows, int64_t len);
+int mllm_hip_softmax_ws(const float* x, float* y, int64_t rows, int64_t len, void* workspace, void* stream);
+size_t mllm_hip_topk_workspace_bytes(int64_t rows, int64_t len, int k);
+int mllm_hip_topk_ws(const float* x, float* values, int32_t* indices, int64_t rows, int64_t len, int k, int largest, int sorted,
+                     void* workspace, void* stream);
 /* The MoE gate: scores = softmax(x . W^T) in fp32, the k largest per token in index order, weights divided by their sum
  * when norm_topk_prob.  x [M][H] fp32 or bf16; gate_weight fp32 [E][H]; topk_ids int32 [M][k]; topk_weights fp32 [M][k];
  * scores fp32 [M][E] or NULL.  H % 8 == 0.  With a scores buffer the call is two launches -- the logits with the experts

@@ -74,6 +74,12 @@ def lib():
         L.mllm_hip_set_exp_mode.argtypes = [ci]
         L.mllm_hip_softmax.argtypes = [vp, vp, i64, i64, vp]
         L.mllm_hip_topk.argtypes = [vp, vp, vp, i64, i64, ci, ci, ci, vp]
+        L.mllm_hip_softmax_workspace_bytes.restype = C.c_size_t
+        L.mllm_hip_softmax_workspace_bytes.argtypes = [i64, i64]
+        L.mllm_hip_softmax_ws.argtypes = [vp, vp, i64, i64, vp, vp]
+        L.mllm_hip_topk_workspace_bytes.restype = C.c_size_t
+        L.mllm_hip_topk_workspace_bytes.argtypes = [i64, i64, ci]
+        L.mllm_hip_topk_ws.argtypes = [vp, vp, vp, i64, i64, ci, ci, ci, vp, vp]
         L.mllm_hip_moe_gate.argtypes = [vp, ci, vp, vp, vp, vp, i64, i64, i64, ci, ci, vp]
         L.mllm_hip_moe_gate_set_form.argtypes = [ci]
         L.mllm_hip_w8a8_set_decode.argtypes = [ci]

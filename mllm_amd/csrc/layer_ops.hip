@@ -313,6 +313,81 @@ __global__ __launch_bounds__(SOFTMAX_WG) void softmax_long_rows_kernel(const flo
   }
 }
 
+// Few long rows spread over the chip (mllm_hip_softmax_ws): a row is cut into pieces of SOFTMAX_PIECE elements with a
+// workgroup each, and the row's maximum and sum meet in the caller's workspace, so the operator is three launches: maxima of
+// the pieces, sums of the pieces (which need the row's maximum: the reference's polynomial is not exp(a) exp(b) = exp(a + b)
+// to fp32), results.  A workgroup per row is bound by what one CU can load and by its vector ALU: eight rows of 151 936 take
+// 49 us there and 14.8 here (one row 47 -> 14.2; a launch costs about 2.5 us whatever it does).
+constexpr int SOFTMAX_PIECE = 4096;
+constexpr int SOFTMAX_LONG = 40960;       // up to here one workgroup per row is as fast (32 000: 12.3 us against 13.9; 64 000: 21.7 against 14.1)
+constexpr int SOFTMAX_SPLIT_ROWS = 512;
+__device__ __forceinline__ float block_max_256(float v, float* s_red) {
+  v = wave_max(v);
+  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
+  __syncthreads();
+  return v;
+}
+__device__ __forceinline__ float block_sum_256(float v, float* s_red) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = ((s_red[0] + s_red[1]) + s_red[2]) + s_red[3];
+  __syncthreads();
+  return v;
+}
+// STAGE 0: pmax[row][piece];  1: psum[row][piece];  2: y.  ws: pmax, then psum, of rows * pieces floats each.
+template <int STAGE>
+__global__ __launch_bounds__(256) void softmax_pieces_kernel(const float* __restrict__ x, float* __restrict__ y, float* __restrict__ ws,
+                                                             int len, int exp_accurate) {
+  __shared__ float s_red[4];
+  constexpr int R = SOFTMAX_PIECE / 256;
+  const int tid = threadIdx.x, piece = blockIdx.x, pieces = gridDim.x;
+  const int64_t row = blockIdx.y;
+  float* pmax = ws + row * pieces;
+  float* psum = ws + ((int64_t)gridDim.y + row) * pieces;
+  const float* xr = x + row * len;
+  const int i0 = piece * SOFTMAX_PIECE + tid;
+  float v[R];
+#pragma unroll
+  for (int j = 0; j < R; j++) v[j] = i0 + 256 * j < len ? xr[i0 + 256 * j] : -3.402823466e+38f;
+  if (STAGE == 0) {
+    float mx = v[0];
+#pragma unroll
+    for (int j = 1; j < R; j++) mx = fmaxf(mx, v[j]);
+    mx = block_max_256(mx, s_red);
+    if (tid == 0) pmax[piece] = mx;
+    return;
+  }
+  const bool poly = !exp_accurate;
+  float mx = -3.402823466e+38f;
+  for (int p = tid; p < pieces; p += 256) mx = fmaxf(mx, pmax[p]);
+  float total = 0.f;
+  if (STAGE == 2)
+    for (int p = tid; p < pieces; p += 256) total += psum[p];
+  mx = block_max_256(mx, s_red);
+  float sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    const int i = i0 + 256 * j;
+    if (i < len) {
+      v[j] = softmax_exp(v[j] - mx, poly && i < (len & ~7));
+      sum += v[j];
+    }
+  }
+  if (STAGE == 1) {
+    sum = block_sum_256(sum, s_red);
+    if (tid == 0) psum[piece] = sum;
+  } else {
+    const float inv = 1.f / block_sum_256(total, s_red);
+    float* yr = y + row * len;
+#pragma unroll
+    for (int j = 0; j < R; j++)
+      if (i0 + 256 * j < len) yr[i0 + 256 * j] = v[j] * inv;
+  }
+}
+
 // Rows between the two (2049 to 16 384 elements: the keys of an attention row): a workgroup of four waves per row, the row in
 // registers (16, 32 or 64 elements per thread), one pass over memory; maxima and sums meet in LDS.
 template <int R>
@@ -732,6 +807,148 @@ __global__ __launch_bounds__(NT) void topk_select_rows_kernel(const float* __res
   }
 }
 
+// Few long rows spread over the chip (mllm_hip_topk_ws), k up to 128: a row is cut into pieces of TOPK_PIECE elements, a
+// workgroup selects the k largest keys of its piece into the caller's workspace, and a second launch selects among the
+// pieces' keys.  A workgroup per row is bound by what one CU loads per pass over the row: 20 of eight rows of 151 936 take
+// 110 us there and 12 here, 64 of them 111 and 15.
+//
+// Selection inside a workgroup: keys are unique (value, inverted index).  The k-th largest of the threads' own maxima (found a
+// bit at a time by counting, every wave on its own) is at most the k-th largest value, so the keys at or above it contain the
+// selection, and of keys that are spread over the threads in any order they are few more than k (about 180 at k = 128).  They
+// are collected in LDS and placed by rank, up to 64 of them in the registers of one wave; should they be more than TOPK_CAND
+// (many equal values, or one thread's keys all larger than the other threads'), the k-th key itself is found a bit at a time.
+constexpr int TOPK_PIECE = 4096;
+constexpr int TOPK_CAND = 1024;
+constexpr int TOPK_SPLIT_K = 128;
+constexpr int TOPK_SPLIT_LEN = 4096;
+constexpr int TOPK_SPLIT_ROWS = 512;
+constexpr int TOPK_MERGE_R = 20;  // keys per thread of the second launch, at most
+struct TopkShared {
+  unsigned long long top[256];  // the selection by value
+  unsigned long long cand[TOPK_CAND];
+  uint32_t maxima[256];
+  unsigned count, hits[4];
+};
+__device__ __forceinline__ unsigned long long lane_u64(unsigned long long v, int lane) {  // (lane: the same in every lane)
+  return ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), lane) << 32) |
+         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+}
+// the k largest non-zero keys of the workgroup's 256 R keys (zero = no element), largest first, in sh.top; returns how many there are
+template <int R>
+__device__ __forceinline__ int block_topk_256(const unsigned long long (&key)[R], int k, TopkShared& sh) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  unsigned long long mine = key[0];
+#pragma unroll
+  for (int j = 1; j < R; j++) mine = key[j] > mine ? key[j] : mine;
+  if (tid == 0) sh.count = 0;
+  sh.maxima[tid] = (uint32_t)(mine >> 32);
+  __syncthreads();
+  const u32x4 m4 = *reinterpret_cast<const u32x4*>(&sh.maxima[4 * lane]);  // every wave on its own, four maxima per lane
+  uint32_t b32 = 0;
+  for (int bit = 31; bit >= 0; bit--) {
+    const uint32_t t = b32 | (1u << bit);
+    const int c = __popcll(__ballot(m4.x >= t)) + __popcll(__ballot(m4.y >= t)) + __popcll(__ballot(m4.z >= t)) + __popcll(__ballot(m4.w >= t));
+    if (c >= k) b32 = t;
+  }
+  unsigned long long bound = (unsigned long long)b32 << 32;
+  if (bound == 0) bound = 1;  // fewer than k threads hold an element: every element is wanted
+  auto collect = [&]() {
+#pragma unroll
+    for (int j = 0; j < R; j++)
+      if (key[j] >= bound) {
+        const unsigned pos = atomicAdd(&sh.count, 1u);
+        if (pos < (unsigned)TOPK_CAND) sh.cand[pos] = key[j];
+      }
+    __syncthreads();
+  };
+  collect();
+  if (sh.count > (unsigned)TOPK_CAND) {  // (the same in every thread)
+    unsigned long long kth = 0;
+    for (int bit = 63; bit >= 0; bit--) {
+      const unsigned long long t = kth | (1ull << bit);
+      unsigned c = 0;
+#pragma unroll
+      for (int j = 0; j < R; j++) c += (unsigned)__popcll(__ballot(key[j] >= t));
+      if (lane == 0) sh.hits[wave] = c;
+      __syncthreads();
+      if (sh.hits[0] + sh.hits[1] + sh.hits[2] + sh.hits[3] >= (unsigned)k) kth = t;
+      __syncthreads();
+    }
+    bound = kth;
+    if (tid == 0) sh.count = 0;
+    __syncthreads();
+    collect();  // exactly k
+  }
+  const int n = (int)sh.count;
+  if (n <= 64) {
+    if (wave == 0) {
+      const unsigned long long my = lane < n ? sh.cand[lane] : 0ull;
+      int r = 0;
+      for (int j = 0; j < n; j++) r += lane_u64(my, j) > my ? 1 : 0;
+      if (lane < n && r < k) sh.top[r] = my;
+    }
+  } else {
+    for (int i = tid; i < n; i += 256) {
+      const unsigned long long my = sh.cand[i];
+      int r = 0;
+#pragma unroll 8
+      for (int j = 0; j < n; j++) r += sh.cand[j] > my ? 1 : 0;
+      if (r < k) sh.top[r] = my;
+    }
+  }
+  __syncthreads();
+  return n < k ? n : k;
+}
+template <int VEC>
+__global__ __launch_bounds__(256) void topk_pieces_kernel(const float* __restrict__ x, unsigned long long* __restrict__ ws, int len, int k,
+                                                          int largest) {
+  typedef typename TopkVec<VEC>::T VT;
+  __shared__ TopkShared sh;
+  constexpr int R = TOPK_PIECE / 256, RV = R / VEC;
+  const int tid = threadIdx.x, piece = blockIdx.x;
+  const int64_t row = blockIdx.y;
+  const VT* xr = reinterpret_cast<const VT*>(x + row * len);
+  const int nunits = len / VEC, u0 = piece * (TOPK_PIECE / VEC) + tid;  // (VEC divides len)
+  VT v[RV];
+#pragma unroll
+  for (int j = 0; j < RV; j++) v[j] = u0 + 256 * j < nunits ? xr[u0 + 256 * j] : VT{};
+  unsigned long long key[R];
+#pragma unroll
+  for (int j = 0; j < RV; j++) {
+    const float* f = reinterpret_cast<const float*>(&v[j]);
+#pragma unroll
+    for (int e = 0; e < VEC; e++)
+      key[j * VEC + e] = u0 + 256 * j < nunits ? order_key(f[e], (u0 + 256 * j) * VEC + e, largest != 0) : 0ull;
+  }
+  const int n = block_topk_256<R>(key, k, sh);
+  // the pieces' largest keys first, then their second largest ...: the large ones spread over the threads of the next launch
+  unsigned long long* out = ws + row * gridDim.x * k + piece;
+  for (int t = tid; t < k; t += 256) out[(int64_t)t * gridDim.x] = t < n ? sh.top[t] : 0ull;
+}
+template <int R>
+__global__ __launch_bounds__(256) void topk_merge_kernel(const float* __restrict__ x, const unsigned long long* __restrict__ ws,
+                                                         float* __restrict__ values, int32_t* __restrict__ indices, int len, int n, int k,
+                                                         int sorted) {
+  __shared__ TopkShared sh;
+  const int tid = threadIdx.x;
+  const int64_t row = blockIdx.x;
+  unsigned long long key[R];
+#pragma unroll
+  for (int j = 0; j < R; j++) key[j] = tid + 256 * j < n ? ws[row * n + tid + 256 * j] : 0ull;
+  block_topk_256<R>(key, k, sh);  // (k keys: the row has that many elements)
+  for (int t = tid; t < k; t += 256) {
+    const unsigned long long my = sh.top[t];
+    int r = t;
+    if (!sorted) {
+      r = 0;
+      for (int j = 0; j < k; j++) r += (uint32_t)sh.top[j] > (uint32_t)my ? 1 : 0;  // the inverted index: larger = earlier
+    }
+    const int idx = (int)~(uint32_t)my;
+    values[row * k + r] = x[row * len + idx];
+    indices[row * k + r] = idx;
+  }
+}
+
 // ---- MoE gate: logits = x . W^T (fp32), softmax, top-k, optional normalisation ------------------------------------------
 // A workgroup of sixteen waves takes four tokens: the tokens' activations sit in LDS, every wave walks a sixteenth of the
 // experts (16-byte loads along H, the tokens share each weight load), then wave t finishes token t.
@@ -1029,6 +1246,53 @@ MLLM_API int mllm_hip_topk(const float* x, float* values, int32_t* indices, int6
   else
     hipLaunchKernelGGL(topk_rows_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, (hipStream_t)stream, x, values, indices, rows,
                        (int)len, k, largest, sorted);
+  return (int)hipGetLastError();
+}
+
+// Pieces of a row that few long rows are cut into, 0 where a workgroup per row is the better form
+static int softmax_pieces(int64_t rows, int64_t len) {
+  return len > SOFTMAX_LONG && rows <= SOFTMAX_SPLIT_ROWS && len <= 0x7fffffff ? (int)((len + SOFTMAX_PIECE - 1) / SOFTMAX_PIECE) : 0;
+}
+MLLM_API size_t mllm_hip_softmax_workspace_bytes(int64_t rows, int64_t len) {
+  if (rows <= 0 || len <= 0) return 0;
+  return (size_t)rows * softmax_pieces(rows, len) * 2 * sizeof(float);
+}
+MLLM_API int mllm_hip_softmax_ws(const float* x, float* y, int64_t rows, int64_t len, void* workspace, void* stream) {
+  const int pieces = workspace && rows > 0 && len > 0 ? softmax_pieces(rows, len) : 0;
+  if (!pieces) return mllm_hip_softmax(x, y, rows, len, stream);
+  if (!x || !y) return MLLM_HIP_E_BADARG;
+  if (reinterpret_cast<uintptr_t>(workspace) % 4) return MLLM_HIP_E_ALIGN;
+  const dim3 grid((unsigned)pieces, (unsigned)rows);
+  hipStream_t st = (hipStream_t)stream;
+  float* ws = reinterpret_cast<float*>(workspace);
+  hipLaunchKernelGGL(softmax_pieces_kernel<0>, grid, dim3(256), 0, st, x, y, ws, (int)len, g_exp_accurate);
+  hipLaunchKernelGGL(softmax_pieces_kernel<1>, grid, dim3(256), 0, st, x, y, ws, (int)len, g_exp_accurate);
+  hipLaunchKernelGGL(softmax_pieces_kernel<2>, grid, dim3(256), 0, st, x, y, ws, (int)len, g_exp_accurate);
+  return (int)hipGetLastError();
+}
+
+static int topk_pieces(int64_t rows, int64_t len, int k) {
+  if (len <= TOPK_SPLIT_LEN || rows > TOPK_SPLIT_ROWS || k < 1 || k > TOPK_SPLIT_K || len > 0x7fffffff) return 0;
+  const int64_t pieces = (len + TOPK_PIECE - 1) / TOPK_PIECE;
+  return pieces * k <= 256 * TOPK_MERGE_R ? (int)pieces : 0;
+}
+MLLM_API size_t mllm_hip_topk_workspace_bytes(int64_t rows, int64_t len, int k) {
+  if (rows <= 0 || len <= 0) return 0;
+  return (size_t)rows * topk_pieces(rows, len, k) * (k > 0 ? k : 0) * sizeof(unsigned long long);
+}
+MLLM_API int mllm_hip_topk_ws(const float* x, float* values, int32_t* indices, int64_t rows, int64_t len, int k, int largest, int sorted,
+                              void* workspace, void* stream) {
+  const int pieces = workspace && rows > 0 && len > 0 ? topk_pieces(rows, len, k) : 0;
+  if (!pieces) return mllm_hip_topk(x, values, indices, rows, len, k, largest, sorted, stream);
+  if (!x || !values || !indices) return MLLM_HIP_E_BADARG;
+  if (reinterpret_cast<uintptr_t>(workspace) % 8) return MLLM_HIP_E_ALIGN;
+  const dim3 grid((unsigned)pieces, (unsigned)rows);
+  hipStream_t st = (hipStream_t)stream;
+  unsigned long long* ws = reinterpret_cast<unsigned long long*>(workspace);
+  if (len % 4 == 0 && ((uintptr_t)x & 15) == 0) hipLaunchKernelGGL(topk_pieces_kernel<4>, grid, dim3(256), 0, st, x, ws, (int)len, k, largest);
+  else hipLaunchKernelGGL(topk_pieces_kernel<1>, grid, dim3(256), 0, st, x, ws, (int)len, k, largest);
+  if (pieces * k <= 1024) hipLaunchKernelGGL(topk_merge_kernel<4>, dim3((unsigned)rows), dim3(256), 0, st, x, ws, values, indices, (int)len, pieces * k, k, sorted);
+  else hipLaunchKernelGGL(topk_merge_kernel<TOPK_MERGE_R>, dim3((unsigned)rows), dim3(256), 0, st, x, ws, values, indices, (int)len, pieces * k, k, sorted);
   return (int)hipGetLastError();
 }
 

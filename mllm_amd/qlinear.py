@@ -504,7 +504,10 @@ def softmax(x):
     assert x.is_cuda and x.is_contiguous() and x.dtype == torch.float32
     n = x.shape[-1]
     y = torch.empty_like(x)
-    _lib.check(_lib.lib().mllm_hip_softmax(x.data_ptr(), y.data_ptr(), x.numel() // n, n, _stream()), "mllm_hip_softmax")
+    rows, L = x.numel() // n, _lib.lib()
+    need = L.mllm_hip_softmax_workspace_bytes(rows, n)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda") if need else None
+    _lib.check(L.mllm_hip_softmax_ws(x.data_ptr(), y.data_ptr(), rows, n, _p(ws), _stream()), "mllm_hip_softmax_ws")
     return y
 
 
@@ -513,8 +516,11 @@ def topk(x, k, largest=True, sorted=True):
     n = x.shape[-1]
     v = torch.empty(x.shape[:-1] + (k,), dtype=torch.float32, device="cuda")
     i = torch.empty(x.shape[:-1] + (k,), dtype=torch.int32, device="cuda")
-    _lib.check(_lib.lib().mllm_hip_topk(x.data_ptr(), v.data_ptr(), i.data_ptr(), x.numel() // n, n, k, int(largest),
-                                        int(sorted), _stream()), "mllm_hip_topk")
+    rows, L = x.numel() // n, _lib.lib()
+    need = L.mllm_hip_topk_workspace_bytes(rows, n, k)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda") if need else None
+    _lib.check(L.mllm_hip_topk_ws(x.data_ptr(), v.data_ptr(), i.data_ptr(), rows, n, k, int(largest), int(sorted), _p(ws), _stream()),
+               "mllm_hip_topk_ws")
     return v, i
 
 

@@ -296,6 +296,40 @@ def test_topk_by_radix_select(rows, ln):
             assert np.array_equal(v.cpu().numpy().view(np.uint32), wv.view(np.uint32))
 
 
+@pytest.mark.parametrize("rows,ln", [(1, 40960), (3, 40961), (2, 45056), (5, 45057), (1, 151936)])
+def test_softmax_of_rows_cut_into_pieces(rows, ln):
+    """few long rows meet in a workspace; either side of the length from which they do, whole and ragged last pieces"""
+    x = (synth.rng_for(6, 4500 + ln).standard_normal((rows, ln)) * 3).astype(np.float32)
+    announce("softmax pieces", rows, ln)
+    assert (_lib.lib().mllm_hip_softmax_workspace_bytes(rows, ln) > 0) == (ln > 40960)
+    y = ql.softmax(to_dev(x)).cpu().numpy()
+    want = orc.softmax(x).astype(np.float64)
+    want /= want.sum(-1, keepdims=True)  # without the error of the oracle's one-after-another fp32 sum (1e-5 at 151 936 terms)
+    # a term passes 16 + 8 + 1 + 8 + 2 additions, half an ulp (6e-8) each, plus the quotient's and the product's rounding
+    assert rel_l2(y, want) < 37 * 6e-8
+
+
+@pytest.mark.parametrize("rows,ln,k", [(2, 4096, 8), (3, 4097, 32), (2, 4100, 33), (1, 8193, 64), (2, 20000, 128), (2, 20000, 129), (1, 151936, 128),
+                                       (1, 200003, 128)])
+def test_topk_of_rows_cut_into_pieces(rows, ln, k):
+    """both orders of the result, a last piece of a few elements, k either side of what the pieces serve, a row whose largest
+    elements all fall to one thread (more candidates than are kept), few distinct values"""
+    rng = synth.rng_for(6, 5500 + ln + k)
+    smooth = rng.standard_normal((rows, ln)).astype(np.float32)
+    clustered = smooth.copy()
+    clustered[:, 20:24] += 100.0
+    clustered[:, 1044:1048] += 200.0
+    clustered[:, :1024:4] += 10.0
+    bands = np.round(smooth)
+    announce("topk pieces", rows, ln, k)
+    for x in (smooth, clustered, bands):
+        for largest, srt in ((True, True), (True, False), (False, True)):
+            v, i = ql.topk(to_dev(x), k, largest, srt)
+            wv, wi = orc.topk(x, k, largest, srt)
+            assert np.array_equal(i.cpu().numpy(), wi)
+            assert np.array_equal(v.cpu().numpy().view(np.uint32), wv.view(np.uint32))
+
+
 @pytest.mark.parametrize("M,H,E,k,dtype", [(512, 2048, 128, 8, "f32"), (1, 2048, 128, 8, "f32"), (7, 256, 60, 4, "f32"),
                                            (33, 2048, 128, 8, "bf16"), (5, 64, 8, 2, "f32")])
 def test_moe_gate(M, H, E, k, dtype):
