@@ -16,7 +16,8 @@ BLOCK_BYTES = {Q4_0: 18, Q8_0: 34}
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """the current stream's handle (torch.cuda.current_stream() builds a Stream object first: 2.9 us of a 7 us call)"""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _xdtype(x):
