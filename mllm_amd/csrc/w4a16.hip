@@ -13,6 +13,7 @@
 // Weights are fetched packed (16 bytes = 32 elements per lane), dequantized once per workgroup in registers and staged
 // as bf16 in LDS next to the activation tile; the matrix cores read both operands from LDS.
 #include "qcommon.h"
+#include "wk_gemm.h"
 
 namespace mllmhip {
 
@@ -563,23 +564,104 @@ static int launch_w4a16_nsplit(const W4A16PArgs& a, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
+// The packed matrix as wk_gemm.h reads it: a block is 64 elements, one 16-byte piece of codes per lane and the (scale, -zp * scale)
+// pair of the lane's row; operand d is dword d, dequantized as everywhere else.
+struct W4A16Waves {
+  typedef W4A16PArgs Args;
+  typedef v16f Acc;
+  typedef f32x4 Sum4;
+  typedef bf16x8 X;
+  struct W {
+    u32x4 q;
+    u32x2 sz;
+  };
+  struct Col {
+    uint32_t q, sz;
+    int g64, last;
+  };
+  static __device__ __forceinline__ int kblocks(const Args& a) { return (a.K + 63) / 64; }
+  static __device__ __forceinline__ int row_bytes(const Args& a) { return a.K * 2; }
+  static __device__ __forceinline__ const void* activations(const Args& a) { return a.A; }
+  static __device__ __forceinline__ __amdgpu_buffer_rsrc_t weights(const Args& a) {
+    const int64_t bytes = w4a16_packed_qbytes(a.N, a.K) + w4a16_packed_n(a.N) * (a.K / a.group) * 8;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.P), 0, (uint32_t)bytes, 0x00020000);
+  }
+  static __device__ __forceinline__ Col col(const Args& a, int nb, int lane) {
+    const int kbs = (int)(w4a16_packed_k(a.K) / 64), G = a.K / a.group;
+    nb = min(nb, (int)(w4a16_packed_n(a.N) / 32) - 1);
+    return Col{(uint32_t)((int64_t)nb * kbs * 1024 + lane * 16), (uint32_t)(w4a16_packed_qbytes(a.N, a.K) + ((int64_t)nb * G * 32 + (lane & 31)) * 8),
+               a.group / 64, G - 1};
+  }
+  static __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, const Col& c, int kb, W& w) {
+    w.q = __builtin_amdgcn_raw_buffer_load_b128(r, kb < 0 ? 0xffffffffu : c.q, kb * 1024, 0);
+    w.sz = __builtin_amdgcn_raw_buffer_load_b64(r, kb < 0 ? 0xffffffffu : c.sz, min(kb / c.g64, c.last) * 256, 0);
+  }
+  static __device__ __forceinline__ X operand(const W& w, int d) {
+    uint32_t o[4];
+    dequant8(w.q[d], __uint_as_float(w.sz.x), __uint_as_float(w.sz.y), o);
+    return __builtin_bit_cast(bf16x8, u32x4{o[0], o[1], o[2], o[3]});
+  }
+  static __device__ __forceinline__ Acc mma(const X& w, const X& x, const Acc& acc) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, x, acc, 0, 0, 0); }
+  static __device__ __forceinline__ void store(const Args& a, int m, int n, f32x4 v) {
+    uint16_t* c = a.C + (int64_t)m * a.N + n;
+    if (n + 3 < a.N && a.N % 4 == 0 && reinterpret_cast<uintptr_t>(a.C) % 8 == 0) {
+      if (a.bias) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] += bf16_to_f32(a.bias[n + e]);
+      }
+      *reinterpret_cast<uint2*>(c) = uint2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+      return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (n + e < a.N) c[e] = (uint16_t)pack_bf16(a.bias ? v[e] + bf16_to_f32(a.bias[n + e]) : v[e], 0.f);
+  }
+};
+
 static int g_w4a16_ptile = 0;  // packed path: 0 = heuristic, 1 = 128x384, 2 = 64x384, 3 = 128x128, 4 = 64x128, 5 = 128x256
 
-// Tile choice for the weights-from-global kernel.  128x256 with two workgroups per CU measured best on large problems
-// (one wave's dequantization runs beside the other's MFMAs); smaller tiles only to give every CU work.
-static int launch_w4a16_nsplit_auto(const W4A16PArgs& a, hipStream_t st) {
-  auto tiles = [&](int bm, int bn) { return (int64_t)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
-  int t = g_w4a16_ptile;
-  if (!t) {
-    if (a.M > 64) t = tiles(128, 256) >= 256 ? 5 : tiles(128, 128) >= 128 ? 3 : 4;
-    else t = tiles(64, 384) >= 192 ? 2 : 4;
-  }
-  switch (t) {
-    case 1: return launch_w4a16_nsplit<4, 3, 128, 1>(a, st);
+static int g_w4a16_waves = 1;  // 0: only the weights-from-global tiles (comparison runs and tests)
+
+// Which form runs.  The waves-split-K forms (wk_gemm.h) serve from one token to about the batch whose large tiles fill the chip;
+// 93 x 2048 x 6144: 43.6 -> 12 us, 1 x 2560 x 9728: 16.6 -> 13.4 (a GEMV of fp32 FMAs), 300 x 9728 x 2560: 36 -> 28, 2048 rows as before.
+// The costs are fitted to 98 shapes within 6 to 10 % (rms); the choice by cost is within 0.5 % of the best form on average, 9 % at worst.
+static int launch_w4a16_auto(const W4A16PArgs& a, hipStream_t st) {
+  static const FormCost cost[] = {
+      {32, 32, 0.75f, 1.32f, 2.22f, 0.0906f},   // 16 waves
+      {32, 32, 0.50f, 3.15f, 0.54f, 0.0879f},   // 8 waves, two workgroups per CU
+      {32, 64, 0.75f, 3.20f, 0.85f, 0.1206f},   // 8 waves
+      {64, 64, 0.50f, 3.79f, 0.95f, 0.2008f},   // 4 waves, two workgroups per CU
+      {128, 128, 0.00f, 5.66f, 0.00f, 0.6687f},  // weights-from-global tiles
+      {128, 256, 0.75f, 7.69f, 0.46f, 0.8890f},
+      {128, 384, 1.00f, 3.20f, 12.54f, 1.0826f}};
+  constexpr int waves = 4, forms = 7;
+  int form = -1;
+  switch (g_w4a16_ptile) {
+    case 0: break;
+    case 1: form = 6; break;
+    case 3: form = 4; break;
+    case 5: form = 5; break;
     case 2: return launch_w4a16_nsplit<2, 3, 128, 2>(a, st);
-    case 3: return launch_w4a16_nsplit<4, 1, 64, 3>(a, st);
-    case 5: return launch_w4a16_nsplit<4, 2, 64, 2>(a, st);
     default: return launch_w4a16_nsplit<2, 1, 128, 2>(a, st);
+  }
+  if (form < 0) {
+    float best = 0.f;
+    for (int f = g_w4a16_waves ? 0 : waves; f < forms; f++) {
+      const float c = form_cost(cost[f], a.M, a.N, (a.K + 63) / 64);
+      if (form < 0 || c < best) {
+        best = c;
+        form = f;
+      }
+    }
+  }
+  switch (form) {
+    case 0: return wk_gemm_launch<W4A16Waves, 1, 1, 16, 2>(a, st);
+    case 1: return wk_gemm_launch<W4A16Waves, 1, 1, 8, 3>(a, st);
+    case 2: return wk_gemm_launch<W4A16Waves, 1, 2, 8, 1>(a, st);
+    case 3: return wk_gemm_launch<W4A16Waves, 2, 2, 4, 2>(a, st);
+    case 4: return launch_w4a16_nsplit<4, 1, 64, 3>(a, st);
+    case 5: return launch_w4a16_nsplit<4, 2, 64, 2>(a, st);
+    default: return launch_w4a16_nsplit<4, 3, 128, 1>(a, st);
   }
 }
 
@@ -748,232 +830,13 @@ MLLM_API int mllm_hip_w4a16_prepack(const uint8_t* qw, const uint16_t* scales, c
   return (int)hipGetLastError();
 }
 
-// ---- decode: up to 32 tokens against the packed weights ------------------------------------------------------------------
-// The tile kernels spend a 128-row tile on a decode token (9728 x 2560 at one token: 20 us; 2560 x 9728: 65 us).  Here a
-// workgroup takes one block row of the packed matrix (32 weight rows), its waves stride over the 64-element K blocks, eight
-// blocks requested per wave before the first is dequantized (the first batch ahead of the copy of the tokens' activations
-// into LDS); weights go to bf16 exactly as in the tile kernels (dequant8), the products (exact in fp32) are added by fp32
-// FMAs, the two K halves of a block meet through a wave shuffle, the waves through LDS.  Same rounding points as the tile
-// kernels (weights to bf16, the sum + bias to bf16), fp32 sums in another order.  The kernel is bound by its vector ALU
-// work, which grows with the tokens (9728 x 2560: 12.5 / 14.0 / 17.9 / 25.5 us at one / two / four / eight tokens against 20 us
-// for the tile kernels): it serves one token, the matrix-core form below two and more.
-constexpr int W4G_MAXW = 16;
-template <int MT>
-__global__ __launch_bounds__(W4G_MAXW * 64) void w4a16_gemv_packed_kernel(W4A16PArgs a) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int Kp = (int)w4a16_packed_k(a.K), kbs = Kp / 64, G = a.K / a.group, g64 = a.group / 64;
-  u32x4* sx = reinterpret_cast<u32x4*>(smem);                         // [MT][Kp / 8] bf16 activations, zero past K and M
-  float* s_part = reinterpret_cast<float*>(smem + (size_t)MT * Kp * 2);  // [wave][MT][32]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nthreads = blockDim.x, nwaves = nthreads >> 6;
-  const int r = lane & 31, h = lane >> 5;
-  const int nb = blockIdx.x;
-  const int64_t qbytes = w4a16_packed_qbytes(a.N, a.K);
-  const u32x4* Q = reinterpret_cast<const u32x4*>(a.P) + (size_t)nb * kbs * 64 + lane;
-  const float2* SZ = reinterpret_cast<const float2*>(a.P + qbytes) + (size_t)nb * G * 32 + r;
-  constexpr int UB = 8;
-  u32x4 wv[UB];
-  float2 sz[UB];
-  auto load_batch = [&](int kb0) {
-#pragma unroll
-    for (int u = 0; u < UB; u++) {
-      const int kb = kb0 + u * nwaves;
-      wv[u] = u32x4{0u, 0u, 0u, 0u};
-      sz[u] = float2{0.f, 0.f};
-      if (kb < kbs) {
-        wv[u] = Q[(size_t)kb * 64];
-        sz[u] = SZ[(size_t)min(kb / g64, G - 1) * 32];  // (blocks of the zero padding past K: their codes are zero, as are the activations)
-      }
-    }
-  };
-  load_batch(wave);
-  const int cpr = Kp / 8;  // 16-byte pieces (eight elements) per token
-  for (int i = tid; i < MT * cpr; i += nthreads) {
-    const int m = i / cpr, c = i - m * cpr;
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (m < a.M && c * 8 < a.K) v = *reinterpret_cast<const u32x4*>(a.A + (size_t)m * a.K + c * 8);  // K % 64 == 0
-    sx[i] = v;
-  }
-  __syncthreads();
-  float acc[MT];
-#pragma unroll
-  for (int m = 0; m < MT; m++) acc[m] = 0.f;
-  for (int kb0 = wave; kb0 < kbs; kb0 += nwaves * UB) {
-    if (kb0 != wave) load_batch(kb0);
-#pragma unroll
-    for (int u = 0; u < UB; u++) {
-      const int kb = kb0 + u * nwaves;
-      if (kb < kbs) {  // uniform
-        const uint32_t wd[4] = {wv[u].x, wv[u].y, wv[u].z, wv[u].w};
-#pragma unroll
-        for (int d = 0; d < 4; d++) {  // elements k = 64 kb + 16 d + 8 h + 0..7
-          uint32_t wb[4];
-          dequant8(wd[d], sz[u].x, sz[u].y, wb);
-#pragma unroll
-          for (int m = 0; m < MT; m++) {
-            const u32x4 xv = sx[m * cpr + kb * 8 + 2 * d + h];
-            float s = acc[m];
-            const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
-#pragma unroll
-            for (int p = 0; p < 4; p++) {
-              s = fmaf(__uint_as_float(wb[p] << 16), __uint_as_float(xw[p] << 16), s);
-              s = fmaf(__uint_as_float(wb[p] & 0xffff0000u), __uint_as_float(xw[p] & 0xffff0000u), s);
-            }
-            acc[m] = s;
-          }
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int m = 0; m < MT; m++) {
-    acc[m] += __shfl_xor(acc[m], 32, 64);
-    if (h == 0) s_part[(wave * MT + m) * 32 + r] = acc[m];
-  }
-  __syncthreads();
-  for (int i = tid; i < MT * 32; i += nthreads) {
-    const int m = i >> 5, n = nb * 32 + (i & 31);
-    if (m < a.M && n < a.N) {
-      float f = 0.f;
-      for (int w = 0; w < nwaves; w++) f += s_part[(w * MT + m) * 32 + (i & 31)];
-      if (a.bias) f += bf16_to_f32(a.bias[n]);
-      a.C[(int64_t)m * a.N + n] = (uint16_t)pack_bf16(f, 0.f);
-    }
-  }
-}
-// The same walk with the products on the matrix cores: the packed dword d of a lane IS its operand of the d-th
-// v_mfma_f32_32x32x16_bf16 of the block (row l % 32, eight consecutive k of half l / 32), the other operand the same eight k of
-// token l % 32 from LDS (lanes past the MT tokens staged pass zeros), so a block costs four matrix instructions whatever the
-// token count and the vector ALU does the dequantization only.  acc[4g + e] = C[token l % 32][row 8g + 4 (l / 32) + e]; the
-// waves' sums meet in LDS where the activations were (after a barrier).
-template <int MT>
-__global__ __launch_bounds__(W4G_MAXW * 64) void w4a16_gemv_mfma_packed_kernel(W4A16PArgs a, int cb) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int Kp = (int)w4a16_packed_k(a.K), kbs = Kp / 64, G = a.K / a.group, g64 = a.group / 64;
-  u32x4* sx = reinterpret_cast<u32x4*>(smem);       // [MT][8 cb] bf16 activations of the cb blocks in work, zero past K and M
-  float* s_part = reinterpret_cast<float*>(smem);   // [wave][MT][32], after the loop
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nthreads = blockDim.x, nwaves = nthreads >> 6;
-  const int r = lane & 31, h = lane >> 5;
-  const int nb = blockIdx.x;
-  const int64_t qbytes = w4a16_packed_qbytes(a.N, a.K);
-  const u32x4* Q = reinterpret_cast<const u32x4*>(a.P) + (size_t)nb * kbs * 64 + lane;
-  const float2* SZ = reinterpret_cast<const float2*>(a.P + qbytes) + (size_t)nb * G * 32 + r;
-  constexpr int UB = 8;
-  u32x4 wv[UB];
-  float2 sz[UB];
-  auto load_batch = [&](int kb0, int c1) {
-#pragma unroll
-    for (int u = 0; u < UB; u++) {
-      const int kb = kb0 + u * nwaves;
-      wv[u] = u32x4{0u, 0u, 0u, 0u};
-      sz[u] = float2{0.f, 0.f};
-      if (kb < c1) {
-        wv[u] = Q[(size_t)kb * 64];
-        sz[u] = SZ[(size_t)min(kb / g64, G - 1) * 32];
-      }
-    }
-  };
-  const int cpr = cb * 8;  // 16-byte pieces (eight elements) per token in LDS
-  v16f acc;
-#pragma unroll
-  for (int j = 0; j < 16; j++) acc[j] = 0.f;
-  const bool staged = r < MT;
-  const u32x4* sxr = sx + (size_t)(staged ? r : 0) * cpr + h;
-  // the K blocks in runs of cb (all of them where the tokens' rows fit LDS whole)
-  for (int c0 = 0; c0 < kbs; c0 += cb) {
-  const int c1 = min(c0 + cb, kbs);
-  load_batch(c0 + wave, c1);  // ahead of the copy of the activations
-  if (c0) __syncthreads();    // every wave is done with the previous run's activations
-  for (int i = tid; i < MT * cpr; i += nthreads) {
-    const int m = i / cpr, c = i - m * cpr, gc = c0 * 8 + c;
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (m < a.M && gc * 8 < a.K) v = *reinterpret_cast<const u32x4*>(a.A + (size_t)m * a.K + gc * 8);
-    sx[i] = v;
-  }
-  __syncthreads();
-  for (int kb0 = c0 + wave; kb0 < c1; kb0 += nwaves * UB) {
-    if (kb0 != c0 + wave) load_batch(kb0, c1);
-#pragma unroll
-    for (int u = 0; u < UB; u++) {
-      const int kb = kb0 + u * nwaves;
-      if (kb < c1) {  // uniform
-        const uint32_t wd[4] = {wv[u].x, wv[u].y, wv[u].z, wv[u].w};
-#pragma unroll
-        for (int d = 0; d < 4; d++) {  // elements k = 64 kb + 16 d + 8 h + 0..7
-          uint32_t wb[4];
-          dequant8(wd[d], sz[u].x, sz[u].y, wb);
-          u32x4 xv = {0u, 0u, 0u, 0u};
-          if (staged) xv = sxr[(kb - c0) * 8 + 2 * d];
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, u32x4{wb[0], wb[1], wb[2], wb[3]}),
-                                                        __builtin_bit_cast(bf16x8, xv), acc, 0, 0, 0);
-        }
-      }
-    }
-  }
-  }
-  __syncthreads();  // every wave is done with the activations
-  if (staged) {
-#pragma unroll
-    for (int g = 0; g < 4; g++)
-      *reinterpret_cast<f32x4*>(&s_part[(wave * MT + r) * 32 + 8 * g + 4 * h]) = f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
-  }
-  __syncthreads();
-  for (int i = tid; i < MT * 32; i += nthreads) {
-    const int m = i >> 5, n = nb * 32 + (i & 31);
-    if (m < a.M && n < a.N) {
-      float f = 0.f;
-      for (int w = 0; w < nwaves; w++) f += s_part[(w * MT + m) * 32 + (i & 31)];
-      if (a.bias) f += bf16_to_f32(a.bias[n]);
-      a.C[(int64_t)m * a.N + n] = (uint16_t)pack_bf16(f, 0.f);
-    }
-  }
-}
-static int g_w4a16_decode = 1;  // 0: the tile kernels also for a few tokens (comparison runs and tests)
-static int g_w4a16_decode_mfma_from = 2;  // token counts from this one up take the matrix-core form
-static bool launch_w4a16_gemv_packed(const W4A16PArgs& a, hipStream_t st, int* rc) {
-  if (a.M > 32 || !g_w4a16_decode) return false;
-  const int Kp = (int)w4a16_packed_k(a.K), kbs = Kp / 64;
-  const int nwaves = kbs >= 32 ? W4G_MAXW : 4;
-  const dim3 grid((unsigned)(w4a16_packed_n(a.N) / 32));
-  if (a.M >= g_w4a16_decode_mfma_from) {
-    // 17 to 32 tokens: every lane reads its own token's activations from LDS, and the tile kernels win where N gives them
-    // enough tiles (9728 x 2560 at 32 tokens: 24 us here, 20 there; 6144 x 2048: 11.6 against 16.9)
-    if (a.M > 16 && a.N > 8192) return false;
-    const int MT = a.M <= 8 ? 8 : (a.M <= 16 ? 16 : 32);
-    const int cap = 152 * 1024 / (MT * 128);  // K blocks of MT tokens in 152 KB
-    const int cb = kbs < cap ? kbs : cap;
-    const size_t x_bytes = (size_t)MT * cb * 128, part_bytes = (size_t)nwaves * MT * 32 * 4;
-    const size_t lds = x_bytes > part_bytes ? x_bytes : part_bytes;
-    auto go = [&](auto kern) {
-      if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-        return (int)hipGetLastError();
-      hipLaunchKernelGGL(kern, grid, dim3(nwaves * 64), lds, st, a, cb);
-      return (int)hipGetLastError();
-    };
-    *rc = MT == 8 ? go(w4a16_gemv_mfma_packed_kernel<8>) : MT == 16 ? go(w4a16_gemv_mfma_packed_kernel<16>) : go(w4a16_gemv_mfma_packed_kernel<32>);
-    return true;
-  }
-  if (a.M > 4) return false;
-  const int MT = a.M <= 1 ? 1 : (a.M <= 2 ? 2 : 4);
-  const size_t lds = (size_t)MT * Kp * 2 + (size_t)nwaves * MT * 32 * 4;
-  if (lds > 160 * 1024) return false;
-  auto go = [&](auto kern) {
-    if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-      return (int)hipGetLastError();
-    hipLaunchKernelGGL(kern, grid, dim3(nwaves * 64), lds, st, a);
-    return (int)hipGetLastError();
-  };
-  *rc = MT == 1 ? go(w4a16_gemv_packed_kernel<1>) : MT == 2 ? go(w4a16_gemv_packed_kernel<2>) : go(w4a16_gemv_packed_kernel<4>);
-  return true;
-}
 MLLM_API int mllm_hip_w4a16_set_decode(int gemv) {
   if (gemv != 0 && gemv != 1) return MLLM_HIP_E_BADARG;
-  g_w4a16_decode = gemv;
+  g_w4a16_waves = gemv;
   return 0;
 }
-MLLM_API int mllm_hip_w4a16_set_decode_mfma_from(int tokens) {
-  if (tokens < 1 || tokens > 33) return MLLM_HIP_E_BADARG;
-  g_w4a16_decode_mfma_from = tokens;
-  return 0;
+MLLM_API int mllm_hip_w4a16_set_decode_mfma_from(int tokens) {  // (every token count is on the matrix cores)
+  return tokens < 1 || tokens > 33 ? MLLM_HIP_E_BADARG : 0;
 }
 
 MLLM_API int mllm_hip_w4a16_gemm_packed(const void* a_bf16, const void* packed, const void* bias_bf16, void* c_bf16,
@@ -986,9 +849,7 @@ MLLM_API int mllm_hip_w4a16_gemm_packed(const void* a_bf16, const void* packed, 
   if (reinterpret_cast<uintptr_t>(a_bf16) % 16 || reinterpret_cast<uintptr_t>(packed) % 16) return MLLM_HIP_E_ALIGN;
   W4A16PArgs a{(const uint16_t*)a_bf16, (const uint8_t*)packed, (const uint16_t*)bias_bf16, (uint16_t*)c_bf16,
                (int)M, (int)N, (int)K, group};
-  int rc = 0;
-  if (launch_w4a16_gemv_packed(a, (hipStream_t)stream, &rc)) return rc;  // up to 32 tokens
-  return launch_w4a16_nsplit_auto(a, (hipStream_t)stream);
+  return launch_w4a16_auto(a, (hipStream_t)stream);
 }
 
 MLLM_API int mllm_hip_w4a16_dequantize_packed(const void* packed, void* w_bf16, int64_t N, int64_t K, int group, void* stream) {

@@ -1,0 +1,179 @@
+// Linear with a few dozen to a few hundred activation rows on the matrix cores, for weights packed in MFMA operand order: the
+// waves of a workgroup share ONE output tile and split K.
+//
+// A batch of this size has few output tiles: with 128-row x 256-column tiles and one K loop per tile, 93 rows of a
+// 2048 x 6144 matrix are 16 workgroups on 256 CUs, each walking all of K (43 us for 6 MB of weights).  Here the tile is
+// (32 TM) rows x (32 TN) channels, wave w of NW takes the K blocks w, w + NW, ... (128 bytes of an activation row each), and the
+// waves' sums meet in LDS in wave order: enough workgroups and waves to fill the chip, no workspace, no second launch, the
+// same bits on every run.
+//
+// A wave works on its own: its weights come straight from memory in operand order (1 KB contiguous per load), its activation
+// rows as whole 128-byte lines (8 rows per load instruction; one row per lane would touch 32 lines and be bound by the L1's
+// tag rate) that pass through the wave's own 4 TM KB of LDS, 16-byte pieces placed at piece ^ (row / 2 % 8): conflict-free
+// both ways, and no barrier, since one wave's LDS operations execute in order.  D blocks are in flight per wave in registers.
+//
+// A traits class T supplies Args (tile-independent arguments with members M, N), KB-independent geometry and the operand type:
+//   kblocks(a)                        K blocks of 128 activation bytes
+//   activations(a) / row_bytes(a)     base and length in bytes of a row (16-byte multiple)
+//   struct W                          a block's packed weights of one 32-channel column
+//   Col col(a, nb, lane)              per-lane addressing of column block nb
+//   load(rsrc, col, kb, W&)           requests a block (past the end: zeros)
+//   operand(W, d)                     the lane's operand of matrix instruction d = 0..3
+//   mma(w, x, acc), Acc               the instruction, weights first: acc[4g + e] = C[row l % 32][channel 8g + 4 (l / 32) + e]
+//   store(a, m, n, sum[4])            epilogue of four consecutive channels (n % 4 == 0; may reach past N)
+#pragma once
+#include "qcommon.h"
+
+namespace mllmhip {
+
+template <class T, int TM, int TN, int NW, int D>
+__global__ __launch_bounds__(NW * 64) void wk_gemm_kernel(typename T::Args a) {
+  typedef typename T::Acc Acc;  // sixteen 32-bit sums
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lrow = lane & 31, hi = lane >> 5;
+  const int tilesM = (a.M + 32 * TM - 1) / (32 * TM), tilesN = (a.N + 32 * TN - 1) / (32 * TN);
+  // Row tiles of one column tile are neighbours on ONE XCD (workgroup b runs on XCD b % 8): its L2 fetches their weights once
+  int tile = blockIdx.x;
+  {
+    const int total = tilesM * tilesN, xcd = tile & 7, seq = tile >> 3, per = total >> 3, more = total & 7;
+    tile = xcd * per + min(xcd, more) + seq;
+  }
+  const int m0 = (tile % tilesM) * 32 * TM, n0 = (tile / tilesM) * 32 * TN;
+
+  const uint32_t rowb = (uint32_t)T::row_bytes(a);
+  const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(T::activations(a)), 0, (uint32_t)a.M * rowb, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rW = T::weights(a);
+  // activation piece c of a lane: row 8 c + lane / 8, 16-byte column lane % 8; rows past M repeat the last one (never stored)
+  uint32_t offA[4 * TM];
+#pragma unroll
+  for (int c = 0; c < 4 * TM; c++) offA[c] = (uint32_t)min(m0 + 8 * c + (lane >> 3), a.M - 1) * rowb + (lane & 7) * 16;
+  const uint32_t colb = (lane & 7) * 16;
+  typename T::Col col[TN];
+#pragma unroll
+  for (int j = 0; j < TN; j++) col[j] = T::col(a, n0 / 32 + j, lane);
+
+  unsigned char* stage = smem + wave * (TM * 4096);
+  unsigned char* wr[2];  // pieces c even / odd: (row / 2) % 8 = 4 (c % 2) + lane / 16
+#pragma unroll
+  for (int p = 0; p < 2; p++) wr[p] = stage + (lane >> 3) * 128 + (((lane & 7) ^ ((4 * p + (lane >> 4)) & 7)) * 16);
+  const unsigned char* rd[4];
+#pragma unroll
+  for (int d = 0; d < 4; d++) rd[d] = stage + lrow * 128 + (((2 * d + hi) ^ ((lrow >> 1) & 7)) * 16);
+
+  const int nblk = T::kblocks(a);
+  const int cnt = wave < nblk ? (nblk - wave + NW - 1) / NW : 0;  // blocks of this wave
+
+  u32x4 ga[D][4 * TM];
+  typename T::W w[D][TN];
+  auto request = [&](int s, int it) {
+    const int kb = wave + it * NW;
+    const bool in = it < cnt;
+    const bool ok = in && (uint32_t)kb * 128u + colb < rowb;
+#pragma unroll
+    for (int c = 0; c < 4 * TM; c++) ga[s][c] = __builtin_amdgcn_raw_buffer_load_b128(rA, ok ? offA[c] : 0xffffffffu, kb * 128, 0);
+#pragma unroll
+    for (int j = 0; j < TN; j++) T::load(rW, col[j], in ? kb : -1, w[s][j]);
+  };
+  Acc acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[i][j][r] = 0;
+
+#pragma unroll
+  for (int s = 0; s < D; s++) request(s, s);
+  auto work = [&](int s, int next, bool more) {
+#pragma unroll
+    for (int c = 0; c < 4 * TM; c++) *reinterpret_cast<u32x4*>(wr[c & 1] + c * 1024) = ga[s][c];
+    typename T::W wc[TN];
+#pragma unroll
+    for (int j = 0; j < TN; j++) wc[j] = w[s][j];
+    if (more) request(s, next);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+      typename T::X x[TM];
+#pragma unroll
+      for (int i = 0; i < TM; i++) x[i] = *reinterpret_cast<const typename T::X*>(rd[d] + i * 4096);
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        const typename T::X o = T::operand(wc[j], d);
+#pragma unroll
+        for (int i = 0; i < TM; i++) acc[i][j] = T::mma(o, x[i], acc[i][j]);
+      }
+    }
+  };
+  int it = 0;
+  for (; it + D <= cnt; it += D) {
+#pragma unroll
+    for (int s = 0; s < D; s++) work(s, it + s + D, true);
+  }
+#pragma unroll
+  for (int s = 0; s < D - 1; s++)
+    if (it + s < cnt) work(s, 0, false);
+
+  // the waves' sums meet in LDS: [wave][i][j][g][half] of 33 16-byte slots (32 rows and one of padding)
+  constexpr int PER = TM * TN * 8 * 33;  // slots of a wave
+  typedef typename T::Sum4 Sum4;
+  __syncthreads();
+  Sum4* part = reinterpret_cast<Sum4*>(smem);
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        Sum4 v;
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * g + e];
+        part[wave * PER + ((i * TN + j) * 8 + 2 * g + hi) * 33 + lrow] = v;
+      }
+  __syncthreads();
+  // consecutive lanes take consecutive quads of channels of a row
+  constexpr int QUADS = 8 * TN, OUT = 32 * TM * QUADS;
+#pragma unroll
+  for (int o = tid; o < OUT; o += NW * 64) {
+    const int q = o % QUADS, m = o / QUADS;
+    const int slot = (((m >> 5) * TN + (q >> 3)) * 8 + (q & 7)) * 33 + (m & 31);
+    Sum4 v = part[slot];
+#pragma unroll
+    for (int ww = 1; ww < NW; ww++) v += part[ww * PER + slot];
+    if (m0 + m < a.M) T::store(a, m0 + m, n0 + 4 * q, v);
+  }
+}
+
+template <int TM, int TN, int NW>
+constexpr size_t wk_gemm_lds() {
+  constexpr size_t stage = (size_t)NW * TM * 4096, sums = (size_t)NW * TM * TN * 8 * 33 * 16;
+  return stage > sums ? stage : sums;
+}
+
+template <class T, int TM, int TN, int NW, int D>
+int wk_gemm_launch(const typename T::Args& a, hipStream_t st) {
+  constexpr size_t lds = wk_gemm_lds<TM, TN, NW>();
+  static_assert(lds <= 160 * 1024, "LDS of a CU");
+  auto kern = wk_gemm_kernel<T, TM, TN, NW, D>;
+  if (lds > 64 * 1024)
+    HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  const unsigned grid = (unsigned)(((a.M + 32 * TM - 1) / (32 * TM)) * ((a.N + 32 * TN - 1) / (32 * TN)));
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), lds, st, a);
+  return (int)hipGetLastError();
+}
+
+// What a form of a GEMM is expected to take, in us: fixed + rounds * (round + block * K blocks), where a round is one tile per CU
+// and a partly filled last round counts `whole` of a whole one.  The callers' constants are fitted to measured times over
+// matrices of 1 to 25 M weights and 8 to 2048 rows (each says how well); the form with the least cost is launched.
+struct FormCost {
+  int bm, bn;                         // tile: rows x channels
+  float whole, fixed, round, block;
+};
+inline float form_cost(const FormCost& f, int64_t M, int64_t N, int64_t blocks) {
+  const int64_t tiles = ((M + f.bm - 1) / f.bm) * ((N + f.bn - 1) / f.bn);
+  const float full = (float)((tiles + 255) / 256), part = (float)tiles / 256.f;
+  return f.fixed + (f.whole * full + (1.f - f.whole) * (part > 1.f ? part : 1.f)) * (f.round + f.block * (float)blocks);
+}
+
+}  // namespace mllmhip

@@ -231,3 +231,20 @@ def test_awq_checkpoint_unpack_bit_exact_and_gemm(N, K, group):
     got = _bits(ql.w4a16_gemm_packed(bf16_dev(a_bits), packed, N, None, group))
     want = orc.w4a16_gemm(a_bits, oq, osb, oz, None, group)
     assert rel_l2(synth.bf16_bits_to_fp32(got), synth.bf16_bits_to_fp32(want)) <= TOL
+
+
+@pytest.mark.parametrize("M", [2, 31, 33, 64, 97, 300])
+def test_waves_that_split_k(M):
+    """the forms whose waves share a tile and split K: row tiles of 32 and 64 with ragged ends, fewer K blocks than waves, K blocks that
+    do not divide among the waves, N not a multiple of 4 (element stores) and of 64, a group per K block and fewer"""
+    for N, K, group in ((40, 64, 64), (193, 1088, 64), (1030, 2560, 128), (4100, 768, 256), (256, 6208, 64)):
+        rng = synth.rng_for(2, 1300 + 3 * M + N + K + group)
+        qw, s, zp, _, _ = synth.make_w4a16(rng, N, K, group)
+        a_bits, _ = synth.make_x_bf16(rng, M, K)
+        bias = synth.fp32_to_bf16_bits((rng.standard_normal(N) * 0.1).astype(np.float32))
+        announce("w4a16 waves split K", M, N, K, group)
+        packed = ql.w4a16_prepack(*_dev(qw, s, zp), group)
+        got = _bits(ql.w4a16_gemm_packed(bf16_dev(a_bits), packed, N, bf16_dev(bias), group))
+        want = orc.w4a16_gemm(a_bits, qw, s, zp, bias, group)
+        assert rel_l2(synth.bf16_bits_to_fp32(got), synth.bf16_bits_to_fp32(want)) <= TOL
+        assert (got == want).mean() > 0.95  # the rest one bf16 step apart: a sum in another order next to a rounding edge
