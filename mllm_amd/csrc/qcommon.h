@@ -74,6 +74,10 @@ __device__ __forceinline__ float exp_poly(float x) {
   const int n = (int)fx + 0x7f;
   return y * __int_as_float(n << 23);
 }
+// Workgroup b of `total` runs on XCD b % 8, and every XCD has its own L2: the place in 0 .. total - 1 that gives each XCD one run of
+// neighbouring places (for any total)
+__device__ __forceinline__ int xcd_run(int b, int total) { return (b & 7) * (total >> 3) + min(b & 7, total & 7) + (b >> 3); }
+
 // ---- wavefront reductions with DPP (64-wide waves; a DPP row is 16 lanes) -------------------------------
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {

@@ -413,9 +413,11 @@ __device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int
   unsigned char* patch = smem + 4096;
   static_assert(BN * 4 <= 4096, "bias overlaps the store patch");
   const bool has_bias = a.bias != nullptr;
-  const bool full = m0 + BM <= a.M && n0 + BN <= a.N && a.N % 8 == 0 && reinterpret_cast<uintptr_t>(a.C) % 16 == 0;
-  if (full) {
-    // branch-free path: each 32-row slab of results is turned through LDS so that a wave stores whole rows of the
+  // 16-byte pieces; those of ragged edges fall outside the buffer (whose end a row or column past the tile must not wrap over)
+  const bool pieces = a.N % 8 == 0 && reinterpret_cast<uintptr_t>(a.C) % 16 == 0 && ((int64_t)a.M + BM) * a.N * 2 < ((int64_t)1 << 32);
+  if (pieces) {
+    const __amdgpu_buffer_rsrc_t rC = __builtin_amdgcn_make_buffer_rsrc(a.C, 0, (uint32_t)((int64_t)a.M * a.N * 2), 0x00020000);
+    // each 32-row slab of results is turned through LDS so that a wave stores whole rows of the
     // workgroup's BN columns (runs of whole cache lines, 16 bytes per lane)
     f32x4 bi4[TN][4];
 #pragma unroll
@@ -446,7 +448,9 @@ __device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int
         const int c = lane + 64 * t;
         const int row = wave * 8 + c / CPR, cc = c % CPR;
         const u32x4 v = *reinterpret_cast<const u32x4*>(patch + row * ROWB + cc * 16);
-        *reinterpret_cast<u32x4*>(&a.C[(int64_t)(m0 + i * 32 + row) * a.N + n0 + cc * 8]) = v;
+        const int n = n0 + cc * 8;
+        // (a row past M lies past the end of the buffer)
+        __builtin_amdgcn_raw_buffer_store_b128(v, rC, n < a.N ? (uint32_t)(m0 + i * 32 + row) * (uint32_t)a.N * 2u + (uint32_t)n * 2u : 0xffffffffu, 0, 0);
       }
       if (i + 1 < TM) __syncthreads();
     }
@@ -501,8 +505,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPS, WPS)))
       const int xcd = b & 7, seq = b >> 3, hm = tilesM / 2, qn = big_cols / 4;
       tm = (xcd & 1) * hm + seq % hm;
       tn = (xcd >> 1) * qn + seq / hm;
-    } else if (nbig % 8 == 0) {
-      b = (b % 8) * (nbig / 8) + b / 8;  // one run of tiles per XCD that shares a slice of the weights
+    } else {
+      b = xcd_run(b, nbig);  // one run of tiles per XCD that shares a slice of the weights
       tm = b % tilesM;
       tn = b / tilesM;
     }

@@ -9,6 +9,7 @@
 //                      y = out_dtype( float(acc_int32) * (w_scale[n] * x_scale[m]) + bias[n] )
 // The int32 accumulators are exact, so they match any other exact implementation bit for bit.
 #include "qcommon.h"
+#include "wk_gemm.h"
 
 namespace mllmhip {
 
@@ -322,10 +323,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPS, WPS)))
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 31, hi = lane >> 5;
   const int tilesN = (a.N + BN - 1) / BN, tilesM = (a.M + BM - 1) / BM;
-  const int total = tilesM * tilesN;
-  int tile = blockIdx.x;
-  if (total % 8 == 0) tile = (blockIdx.x % 8) * (total / 8) + blockIdx.x / 8;  // one run of tiles per XCD ...
-  const int m0 = (tile % tilesM) * BM, n0 = (tile / tilesM) * BN;              // ... that shares a slice of the weights
+  const int tile = xcd_run(blockIdx.x, tilesM * tilesN);           // one run of tiles per XCD ...
+  const int m0 = (tile % tilesM) * BM, n0 = (tile / tilesM) * BN;  // ... that shares a slice of the weights
 
   // Rows past the end are clamped to the last row (their results are never stored).  Activation bytes past K belong to
   // the next row and meet zero weights (PK) or do not occur (K % 128 == 0); reads past the buffers return zero.
@@ -425,14 +424,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPS, WPS)))
     sBi[i] = (a.bias && n0 + i < a.N) ? a.bias[n0 + i] : 0.f;
   }
   __syncthreads();
-  // Full tiles with bf16 output only take a branch-free path: the column scales sit in registers, and each 32-row slab
+  // bf16 output only: the column scales sit in registers, and each 32-row slab
   // of results is turned through LDS so that a wave stores whole rows of the workgroup's BN columns (runs of whole
   // cache lines, 16 bytes per lane).
   constexpr int ROWB = 2 * BN + 16;
   unsigned char* patch = smem + 4096;
   static_assert((BM + 2 * BN) * 4 <= 4096, "scales overlap the store patch");
-  const bool full = m0 + BM <= a.M && n0 + BN <= a.N && a.N % 8 == 0 && reinterpret_cast<uintptr_t>(a.C) % 16 == 0;
-  if (full && a.C && !a.acc) {
+  // 16-byte pieces; those of ragged edges fall outside the buffer (whose end a row or column past the tile must not wrap over)
+  const bool pieces = a.N % 8 == 0 && reinterpret_cast<uintptr_t>(a.C) % 16 == 0 && ((int64_t)a.M + BM) * a.N * 2 < ((int64_t)1 << 32);
+  if (pieces && a.C && !a.acc) {
+    const __amdgpu_buffer_rsrc_t rC = __builtin_amdgcn_make_buffer_rsrc(a.C, 0, (uint32_t)((int64_t)a.M * a.N * 2), 0x00020000);
     f32x4 ws4[TN][4], bi4[TN][4];
 #pragma unroll
     for (int j = 0; j < TN; j++)
@@ -467,7 +468,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPS, WPS)))
         const int c = lane + 64 * t;
         const int row = wave * 8 + c / CPR, cc = c % CPR;
         const u32x4 v = *reinterpret_cast<const u32x4*>(patch + row * ROWB + cc * 16);
-        *reinterpret_cast<u32x4*>(&a.C[(int64_t)(m0 + i * 32 + row) * a.N + n0 + cc * 8]) = v;
+        const int n = n0 + cc * 8;
+        // (a row past M lies past the end of the buffer)
+        __builtin_amdgcn_raw_buffer_store_b128(v, rC, n < a.N ? (uint32_t)(m0 + i * 32 + row) * (uint32_t)a.N * 2u + (uint32_t)n * 2u : 0xffffffffu, 0, 0);
       }
       if (i + 1 < TM) __syncthreads();
     }
@@ -558,7 +561,7 @@ MLLM_API int mllm_hip_w8a8_set_tuning(int tile) {
   return 0;
 }
 
-// ---- decode: up to eight tokens against the prepacked weights --------------------------------------------------------------
+// ---- decode: a few tokens against the prepacked weights --------------------------------------------------------------------
 // The tile kernels above spend a 128-row tile on a decode token and leave most CUs idle (9728 x 2560 at one token: 16 us;
 // 2560 x 9728: 41 us).  Here a workgroup takes one block row of the packed matrix (32 weight rows) and its waves stride over
 // the K blocks, eight 1 KB blocks requested per wave before the first is multiplied (the first batch ahead of the copy of
@@ -636,109 +639,66 @@ __global__ __launch_bounds__(W8G_MAXW * 64) void w8a8_gemv_packed_kernel(W8A8Arg
     }
   }
 }
-// The same walk with the sums on the matrix cores: the 16 bytes a lane holds of a packed block ARE its operand of one
-// v_mfma_i32_32x32x32_i8 (row l % 32, sixteen consecutive k of half l / 32), the other operand the same sixteen k of token
-// l % 32 from LDS (lanes past the MT tokens staged pass zeros): one matrix instruction per block whatever the token count, no
-// vector arithmetic in the loop.  The tokens' codes sit in LDS in runs of cb K blocks (all of them where the rows fit whole).
-// acc[4g + e] = C[token l % 32][row 8g + 4 (l / 32) + e]; integer sums, so the same bits as every other form.
-template <int MT>
-__global__ __launch_bounds__(W8G_MAXW * 64) void w8a8_gemv_mfma_packed_kernel(W8A8Args a, int cb) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int Kp = (int)w8a8_packed_k(a.K), kbs = Kp / 32;
-  u32x4* sx = reinterpret_cast<u32x4*>(smem);   // [MT][2 cb] the tokens' codes of the cb blocks in work, zero past K and M
-  int* s_part = reinterpret_cast<int*>(smem);   // [wave][MT][32], after the loop
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nthreads = blockDim.x, nwaves = nthreads >> 6;
-  const int r = lane & 31, h = lane >> 5;
-  const int nb = blockIdx.x;
-  const u32x4* P = reinterpret_cast<const u32x4*>(a.W) + (size_t)nb * kbs * 64 + lane;
-  constexpr int UB = 8;
-  u32x4 wv[UB];
-  auto load_batch = [&](int kb0, int c1) {
-#pragma unroll
-    for (int u = 0; u < UB; u++) {
-      const int kb = kb0 + u * nwaves;
-      wv[u] = u32x4{0u, 0u, 0u, 0u};
-      if (kb < c1) wv[u] = P[(size_t)kb * 64];
-    }
+// The packed matrix as wk_gemm.h reads it: a block is 128 elements, operand d the 16 bytes of the lane's row in the d-th 32 of them.
+// Integer sums are exact, the epilogue is the tile kernels': the same bits as every other form.
+struct W8A8Waves {
+  typedef W8A8Args Args;
+  typedef v16i Acc;
+  typedef v4i Sum4;
+  typedef v4i X;
+  struct W {
+    u32x4 q[4];
   };
-  const int cpr = cb * 2;  // 16-byte pieces per token in LDS
-  v16i acc;
+  typedef uint32_t Col;
+  static __device__ __forceinline__ int kblocks(const Args& a) { return (a.K + 127) / 128; }
+  static __device__ __forceinline__ int row_bytes(const Args& a) { return a.K; }
+  static __device__ __forceinline__ const void* activations(const Args& a) { return a.A; }
+  static __device__ __forceinline__ __amdgpu_buffer_rsrc_t weights(const Args& a) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.W), 0, (uint32_t)(w8a8_packed_n(a.N) * w8a8_packed_k(a.K)), 0x00020000);
+  }
+  static __device__ __forceinline__ Col col(const Args& a, int nb, int lane) {
+    nb = min(nb, (int)(w8a8_packed_n(a.N) / 32) - 1);
+    return (uint32_t)((int64_t)nb * 32 * w8a8_packed_k(a.K) + lane * 16);
+  }
+  static __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, Col c, int kb, W& w) {
 #pragma unroll
-  for (int j = 0; j < 16; j++) acc[j] = 0;
-  const bool staged = r < MT;
-  const u32x4* sxr = sx + (size_t)(staged ? r : 0) * cpr + h;
-  for (int c0 = 0; c0 < kbs; c0 += cb) {
-    const int c1 = min(c0 + cb, kbs);
-    load_batch(c0 + wave, c1);  // ahead of the copy of the codes
-    if (c0) __syncthreads();    // every wave is done with the previous run's codes
-    for (int i = tid; i < MT * cpr; i += nthreads) {
-      const int m = i / cpr, c = i - m * cpr, gc = c0 * 2 + c;
-      u32x4 v = {0u, 0u, 0u, 0u};
-      if (m < a.M && gc * 16 < a.K) v = *reinterpret_cast<const u32x4*>(a.A + (size_t)m * a.K + gc * 16);  // K % 16 == 0
-      sx[i] = v;
-    }
-    __syncthreads();
-    for (int kb0 = c0 + wave; kb0 < c1; kb0 += nwaves * UB) {
-      if (kb0 != c0 + wave) load_batch(kb0, c1);
+    for (int d = 0; d < 4; d++) w.q[d] = __builtin_amdgcn_raw_buffer_load_b128(r, kb < 0 ? 0xffffffffu : c + d * 1024, kb * 4096, 0);
+  }
+  static __device__ __forceinline__ X operand(const W& w, int d) { return __builtin_bit_cast(v4i, w.q[d]); }
+  static __device__ __forceinline__ Acc mma(const X& w, const X& x, const Acc& acc) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(w, x, acc, 0, 0, 0); }
+  static __device__ __forceinline__ void store(const Args& a, int m, int n, const v4i& v) {
+    const int64_t at = (int64_t)m * a.N + n;
+    float f[4];
+    if (a.C) {
+      const float xs = a.xs[m];
 #pragma unroll
-      for (int u = 0; u < UB; u++) {
-        const int kb = kb0 + u * nwaves;
-        if (kb < c1) {  // uniform
-          u32x4 xv = {0u, 0u, 0u, 0u};
-          if (staged) xv = sxr[(kb - c0) * 2];
-          acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(v4i, wv[u]), __builtin_bit_cast(v4i, xv), acc, 0, 0, 0);
-        }
+      for (int e = 0; e < 4; e++) {
+        f[e] = n + e < a.N ? (float)v[e] * (a.ws[n + e] * xs) : 0.f;
+        if (a.bias && n + e < a.N) f[e] += a.bias[n + e];
+      }
+      if (n + 3 < a.N && a.N % 4 == 0 && reinterpret_cast<uintptr_t>(a.C) % 8 == 0) {
+        *reinterpret_cast<uint2*>(a.C + at) = uint2{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3])};
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (n + e < a.N) a.C[at + e] = (uint16_t)pack_bf16(f[e], 0.f);
       }
     }
-  }
-  __syncthreads();  // every wave is done with the codes
-  if (staged) {
+    if (a.acc) {
 #pragma unroll
-    for (int g = 0; g < 4; g++)
-      *reinterpret_cast<v4i*>(&s_part[(wave * MT + r) * 32 + 8 * g + 4 * h]) = v4i{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
-  }
-  __syncthreads();
-  for (int i = tid; i < MT * 32; i += nthreads) {
-    const int m = i >> 5, n = nb * 32 + (i & 31);
-    if (m < a.M && n < a.N) {
-      int v = 0;
-      for (int w = 0; w < nwaves; w++) v += s_part[(w * MT + m) * 32 + (i & 31)];
-      if (a.acc) a.acc[(int64_t)m * a.N + n] = v;
-      if (a.C) {
-        float f = (float)v * (a.ws[n] * a.xs[m]);
-        if (a.bias) f += a.bias[n];
-        a.C[(int64_t)m * a.N + n] = (uint16_t)pack_bf16(f, 0.f);
-      }
+      for (int e = 0; e < 4; e++)
+        if (n + e < a.N) a.acc[at + e] = v[e];
     }
   }
-}
-// false where the kernels above do not apply
-static int g_w8a8_decode = 1;  // 0: the tile kernels also for a few tokens (comparison runs and tests)
-static int g_w8a8_decode_mfma_from = 5;  // token counts from this one up take the matrix-core form (two to four: the dot form is
-                                         // faster, 9728 x 2560 at four tokens 11.3 against 12.9 us)
+};
+static int g_w8a8_decode = 1;  // 0: only the weights-from-global tiles (comparison runs and tests)
+static int g_w8a8_decode_mfma_from = 5;  // token counts from this one up take the matrix cores (at four tokens the two are even: 6144 x 2048
+                                         // 5.9 us here, 6.1 there; 2560 x 9728 10.4 against 9.5; at one 5.3 / 6.1 and 8.1 / 9.4)
+// false where the dot kernel does not apply
 static bool launch_w8a8_gemv_packed(const W8A8Args& a, hipStream_t st, int* rc) {
-  if (a.M > 32 || !g_w8a8_decode) return false;
+  if (a.M >= g_w8a8_decode_mfma_from || !g_w8a8_decode) return false;
   const int Kp = (int)w8a8_packed_k(a.K), kbs = Kp / 32;
   const int nwaves = kbs >= 32 ? W8G_MAXW : 4;
-  if (a.M >= g_w8a8_decode_mfma_from) {
-    // 17 to 32 tokens: every lane reads its own token's codes from LDS, and the tile kernels win where N gives them enough
-    // tiles (9728 x 2560 at 32 tokens: 21.6 us here, 17.1 there; 2560 x 9728: 28.4 against 43.5)
-    if (a.M > 16 && a.N > 8192) return false;
-    const int MT = a.M <= 8 ? 8 : (a.M <= 16 ? 16 : 32);
-    const int cap = 152 * 1024 / (MT * 32);  // K blocks of MT tokens in 152 KB
-    const int cb = kbs < cap ? kbs : cap;
-    const size_t x_bytes = (size_t)MT * cb * 32, part_bytes = (size_t)nwaves * MT * 32 * 4;
-    const size_t lds = x_bytes > part_bytes ? x_bytes : part_bytes;
-    const dim3 grid((unsigned)(w8a8_packed_n(a.N) / 32));
-    auto go = [&](auto kern) {
-      if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-        return (int)hipGetLastError();
-      hipLaunchKernelGGL(kern, grid, dim3(nwaves * 64), lds, st, a, cb);
-      return (int)hipGetLastError();
-    };
-    *rc = MT == 8 ? go(w8a8_gemv_mfma_packed_kernel<8>) : MT == 16 ? go(w8a8_gemv_mfma_packed_kernel<16>) : go(w8a8_gemv_mfma_packed_kernel<32>);
-    return true;
-  }
   if (a.M > 8) return false;
   const int MT = a.M <= 1 ? 1 : (a.M <= 2 ? 2 : (a.M <= 4 ? 4 : 8));
   const size_t lds = (size_t)MT * Kp + (size_t)nwaves * MT * 32 * 4;
@@ -752,6 +712,42 @@ static bool launch_w8a8_gemv_packed(const W8A8Args& a, hipStream_t st, int* rc) 
   };
   *rc = MT == 1 ? go(w8a8_gemv_packed_kernel<1>) : MT == 2 ? go(w8a8_gemv_packed_kernel<2>) : MT == 4 ? go(w8a8_gemv_packed_kernel<4>) : go(w8a8_gemv_packed_kernel<8>);
   return true;
+}
+// Which matrix-core form runs against packed weights.  Waves that split K (wk_gemm.h) from a few tokens to about the batch whose
+// large tiles fill the chip (93 x 2560 x 9728: 38 -> 11 us, 300 x 2560 x 9728: 41 -> 20, 32 x 4096 x 4096: 13.5 -> 7.6), then the
+// weights-from-global tiles.  The costs are fitted to 170 shapes within 6 to 11 % (rms); the choice by cost is within 1 % of
+// the best form on average, 17 % at worst.
+static int launch_w8a8_packed_auto(const W8A8Args& a, hipStream_t st) {
+  static const FormCost cost[] = {
+      {32, 32, 0.50f, 2.89f, 0.79f, 0.1048f},   // 8 waves, two workgroups per CU
+      {32, 64, 1.00f, 1.94f, 2.55f, 0.1276f},   // 8 waves
+      {64, 64, 1.00f, 0.89f, 4.64f, 0.1776f},   // 8 waves
+      {64, 128, 0.00f, 3.34f, 0.00f, 0.4102f},  // weights-from-global tiles
+      {128, 128, 0.50f, 2.82f, 1.34f, 0.5597f},
+      {128, 256, 0.75f, 0.00f, 6.71f, 0.6615f},
+      {64, 384, 0.75f, 0.00f, 5.22f, 0.5796f},
+      {128, 384, 1.00f, 0.00f, 9.57f, 0.8600f}};
+  constexpr int forms = 8;
+  if (g_w8a8_ntile || !g_w8a8_decode) return launch_w8a8_nsplit_auto<true>(a, st);
+  int form = 0;
+  float best = 0.f;
+  for (int f = 0; f < forms; f++) {
+    const float c = form_cost(cost[f], a.M, a.N, (a.K + 127) / 128);
+    if (f == 0 || c < best) {
+      best = c;
+      form = f;
+    }
+  }
+  switch (form) {
+    case 0: return wk_gemm_launch<W8A8Waves, 1, 1, 8, 2>(a, st);
+    case 1: return wk_gemm_launch<W8A8Waves, 1, 2, 8, 1>(a, st);
+    case 2: return wk_gemm_launch<W8A8Waves, 2, 2, 8, 1>(a, st);
+    case 3: return launch_w8a8_nsplit<2, 1, true, 2>(a, st);
+    case 4: return launch_w8a8_nsplit<4, 1, true, 2>(a, st);
+    case 5: return launch_w8a8_nsplit<4, 2, true, 2>(a, st);
+    case 6: return launch_w8a8_nsplit<2, 3, true, 2>(a, st);
+    default: return launch_w8a8_nsplit<4, 3, true, 1>(a, st);
+  }
 }
 MLLM_API int mllm_hip_w8a8_set_decode(int gemv) {
   if (gemv != 0 && gemv != 1) return MLLM_HIP_E_BADARG;
@@ -845,8 +841,8 @@ MLLM_API int mllm_hip_w8a8_gemm_packed(const int8_t* xq, const float* x_scale, c
   if (reinterpret_cast<uintptr_t>(xq) % 16 || reinterpret_cast<uintptr_t>(W_packed) % 16) return MLLM_HIP_E_ALIGN;
   W8A8Args a{xq, reinterpret_cast<const int8_t*>(W_packed), x_scale, w_scale, bias, (uint16_t*)out_bf16, acc_out, (int)M, (int)N, (int)K};
   int rc = 0;
-  if (launch_w8a8_gemv_packed(a, (hipStream_t)stream, &rc)) return rc;  // up to 32 tokens
-  return launch_w8a8_nsplit_auto<true>(a, (hipStream_t)stream);
+  if (launch_w8a8_gemv_packed(a, (hipStream_t)stream, &rc)) return rc;  // up to four tokens
+  return launch_w8a8_packed_auto(a, (hipStream_t)stream);
 }
 
 MLLM_API size_t mllm_hip_w8a8_workspace_bytes(int64_t M, int64_t K) {

@@ -33,12 +33,8 @@ __global__ __launch_bounds__(NW * 64) void wk_gemm_kernel(typename T::Args a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 31, hi = lane >> 5;
   const int tilesM = (a.M + 32 * TM - 1) / (32 * TM), tilesN = (a.N + 32 * TN - 1) / (32 * TN);
-  // Row tiles of one column tile are neighbours on ONE XCD (workgroup b runs on XCD b % 8): its L2 fetches their weights once
-  int tile = blockIdx.x;
-  {
-    const int total = tilesM * tilesN, xcd = tile & 7, seq = tile >> 3, per = total >> 3, more = total & 7;
-    tile = xcd * per + min(xcd, more) + seq;
-  }
+  // row tiles of one column tile are neighbours on ONE XCD: its L2 fetches their weights once
+  const int tile = xcd_run(blockIdx.x, tilesM * tilesN);
   const int m0 = (tile % tilesM) * 32 * TM, n0 = (tile / tilesM) * 32 * TN;
 
   const uint32_t rowb = (uint32_t)T::row_bytes(a);

@@ -198,3 +198,26 @@ def test_argument_errors():
     assert L.mllm_hip_w8a8_prepack(t.data_ptr(), 64, 40, o.data_ptr(), None) == -2
     assert L.mllm_hip_w8a8_prepack(None, 64, 64, o.data_ptr(), None) == -1
     assert L.mllm_hip_w8a8_packed_bytes(33, 130) == 64 * 256
+
+
+@pytest.mark.parametrize("M", [5, 31, 33, 64, 97, 300])
+def test_waves_that_split_k(M):
+    """the forms whose waves share a tile and split K: row tiles of 32 and 64 with ragged ends, fewer K blocks than waves, K blocks that
+    do not divide among the waves, N not a multiple of 4 (element stores) and of 64; same bits as the oracle"""
+    L = _lib.lib()
+    for N, K in ((40, 64), (193, 1104), (1030, 2560), (4100, 784), (256, 6160)):
+        rng = synth.rng_for(3, 1300 + 3 * M + N + K)
+        a_bits, W, w_scale = synth.make_w8a8(rng, M, N, K)
+        bias = (rng.standard_normal(N) * 0.1).astype(np.float32)
+        announce("w8a8 waves split K", M, N, K)
+        q, s = ql.per_token_quant_int8(bf16_dev(a_bits))
+        packed = ql.w8a8_prepack(to_dev(W))
+        y, acc = ql.w8a8_gemm_packed(q, s, packed, N, to_dev(w_scale), to_dev(bias), want_acc=True)
+        want = q.cpu().numpy().astype(np.int64) @ W.astype(np.int64).T
+        assert np.array_equal(acc.cpu().numpy(), want)
+        assert L.mllm_hip_w8a8_set_decode(0) == 0
+        try:
+            yt = ql.w8a8_gemm_packed(q, s, packed, N, to_dev(w_scale), to_dev(bias))
+        finally:
+            assert L.mllm_hip_w8a8_set_decode(1) == 0
+        assert torch.equal(y.view(torch.int16), yt.view(torch.int16))
