@@ -224,10 +224,11 @@ int mllm_hip_q_gemm_prepack(int wtype, const void* blocks, int weight_scale_mode
 size_t mllm_hip_linear_q_gemm_workspace_bytes(int64_t M, int64_t K);
 int mllm_hip_linear_q_gemm(int wtype, const void* gemm_packed, const void* x, int x_dtype, const float* bias, float* y,
                            int64_t M, int64_t N, int64_t K, int act_scale_mode, void* workspace, void* stream);
-/* The same Linear for short batches (a prompt of up to 1024 rows): its M/128 x N/256 tiles would occupy a fraction of the chip,
- * so K is cut into up to eight ranges that run as separate workgroups and a small second kernel adds their partial results
- * in range order (deterministic).  Same operands and arithmetic; the fp32 sum over K is grouped by range.  Any M is
- * accepted (where cutting K does not pay it is the call above).  workspace: 256-byte aligned. */
+/* The same Linear with a larger workspace, for batches whose M/128 x N/256 tiles would occupy a fraction of the chip: where it
+ * pays, K is cut into up to eight ranges that run as separate workgroups and a small second kernel adds their partial results
+ * in range order (deterministic).  Same operands and arithmetic; the fp32 sum over K is grouped by range.  Any M is accepted
+ * (where cutting K does not pay it is the call above).  workspace: 256-byte aligned.
+ * Both calls choose among their forms by expected cost: up to a few hundred rows the waves of a workgroup split K of a small tile. */
 size_t mllm_hip_linear_q_gemm_short_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int mllm_hip_linear_q_gemm_short(int wtype, const void* gemm_packed, const void* x, int x_dtype, const float* bias, float* y,
                                  int64_t M, int64_t N, int64_t K, int act_scale_mode, void* workspace, void* stream);

@@ -11,6 +11,7 @@
 // a lane owns one output channel: its weight scale is a scalar per block and stores are contiguous across lanes.
 #include "qgemv_kernel.h"
 #include "qgemm_layout.h"
+#include "wk_gemm.h"
 
 namespace mllmhip {
 
@@ -562,7 +563,27 @@ struct QG2Args {
   int x86_scale;
   int ksplit;            // one-matrix mode: K is cut into this many ranges (blockIdx.z), each writing its own partial result
   float* partial;        // [ksplit][a_rows][N] when ksplit > 1
+  int halves;            // a plain Linear: workgroups of eight waves, each four of them half of K
+  int big_cols;          // a plain Linear (no tile list): column tiles that run as full-height tiles
 };
+
+// the scale of dword d (K elements 16 d .. 16 d + 15 of a 64-element step) in both halves; for Q4_K also the offset
+template <int WT>
+__device__ __forceinline__ f16x2 qg_scale2(const uint32_t (&s)[qg_scale_dwords(WT)], int d) {
+  uint32_t h;
+  if constexpr (WT == MLLM_HIP_Q6_K) {
+    const uint32_t v = s[d >> 1];
+    h = (d & 1) ? (v >> 16) : (v & 0xffffu);
+  } else {
+    h = d < 2 ? (s[0] & 0xffffu) : (s[0] >> 16);
+  }
+  return __builtin_bit_cast(f16x2, h | (h << 16));
+}
+template <int WT>
+__device__ __forceinline__ f16x2 qg_offset2(const uint32_t (&s)[qg_scale_dwords(WT)], int d) {
+  const uint32_t v = s[qg_scale_dwords(WT) - 1], h = d < 2 ? (v & 0xffffu) : (v >> 16);
+  return __builtin_bit_cast(f16x2, h | (h << 16));
+}
 
 // pair `b` (elements 2b, 2b+1) of the eight weights of one MFMA step, scaled: one dword of two fp16.  With PREC == 2 also
 // the rounding residual of the product (exact: the error of a product of two fp16 numbers is an fp16 number).
@@ -597,9 +618,11 @@ __device__ __forceinline__ uint32_t qg_pair(const u32x4 (&rq)[qg_nibbles(WT) ? 1
 // (wh*xh + wl*xh + wh*xl): the operands are then exact and the result is the fp32 sum of exact products.  The gate/up
 // stage needs it: its output is re-quantized to Q8_0, and a relative perturbation eps of the values in front of that
 // rounding step flips codes often enough to come out as about sqrt(eps/40) in relative L2.
-template <int WT, int NW, int TM, int TN, int PREC>
+// G == 2 (one matrix): eight waves, the second four take the second half of K with a stage of their own; their sums join the first
+// four's through LDS.
+template <int WT, int NW, int TM, int TN, int PREC, int G = 1>
 __device__ __forceinline__ void qg_tile(const QG2Args& a, const int e, const int row0, const int rows, const int n0,
-                                        unsigned char* smem) {
+                                        unsigned char* smem_all) {
   constexpr int BK = 64, LDK = 2 * BK + 16, KS = BK / 16;
   constexpr int BM = TM * 32, WN = TN * 32;
   constexpr int CA = TM;  // 16-byte activation chunks per thread and K step: 32 TM rows x 8 chunks over 256 threads
@@ -607,7 +630,10 @@ __device__ __forceinline__ void qg_tile(const QG2Args& a, const int e, const int
   constexpr int QW = qg_nibbles(WT) ? 1 : 2;
   constexpr int SDW = qg_scale_dwords(WT);
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  static_assert(G == 1 || NW == 1, "halves of K: one matrix");
+  const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  unsigned char* const smem = smem_all + group * 2 * STAGE;
+  const int tid = G == 1 ? threadIdx.x : threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 31, hi = lane >> 5;
   const int Kp = (int)qg_kp(a.K), kbs = Kp / 64, nbs = (int)(qg_np(a.N) / 32);
   const int64_t qbytes = qg_qbytes(WT, a.N, a.K), wbytes = qg_bytes(WT, a.N, a.K);
@@ -694,27 +720,17 @@ __device__ __forceinline__ void qg_tile(const QG2Args& a, const int e, const int
         loadS(rs[set][w][j], w, j, kb);
       }
   };
-  // the scale of dword d (K elements 16 d .. 16 d + 15 of the step) in both halves; for Q4_K also the offset
-  auto scale2 = [&](const uint32_t (&s)[SDW], int d) -> f16x2 {
-    uint32_t h;
-    if constexpr (WT == MLLM_HIP_Q6_K) {
-      const uint32_t v = s[d >> 1];
-      h = (d & 1) ? (v >> 16) : (v & 0xffffu);
-    } else {
-      h = d < 2 ? (s[0] & 0xffffu) : (s[0] >> 16);
-    }
-    return __builtin_bit_cast(f16x2, h | (h << 16));
-  };
-  auto offset2 = [&](const uint32_t (&s)[SDW], int d) -> f16x2 {
-    const uint32_t h = d < 2 ? (s[SDW - 1] & 0xffffu) : (s[SDW - 1] >> 16);
-    return __builtin_bit_cast(f16x2, h | (h << 16));
-  };
-  // K range of this workgroup: all of it, or (short batches, one matrix) range blockIdx.z of a.ksplit, written to its own
-  // partial result; the ranges start at even K steps
-  int kt0 = 0, kt1 = Kp / BK;  // even
+  // K range of these waves: all of it, one of the G halves, or (short batches, one matrix) range blockIdx.z of a.ksplit, written to its
+  // own partial result; the ranges start at even K steps
+  int kt0 = 0, kt1 = Kp / BK, idle = 0;  // even
   float* outp = a.out;
   const float* biasp = a.bias;
-  if (NW == 1 && a.ksplit > 1) {
+  if (G == 2) {
+    const int per = (kt1 / 2 + 1) / 2 * 2, all = kt1;
+    kt0 = group * per;
+    kt1 = min(all, kt0 + per);
+    idle = per - (kt1 - kt0);
+  } else if (NW == 1 && a.ksplit > 1) {
     const int per = ((kt1 + a.ksplit - 1) / a.ksplit + 1) / 2 * 2;
     kt0 = (int)blockIdx.z * per;
     kt1 = min(kt1, kt0 + per);
@@ -731,7 +747,7 @@ __device__ __forceinline__ void qg_tile(const QG2Args& a, const int e, const int
   for (int w = 0; w < NW; w++)
 #pragma unroll
     for (int j = 0; j < TN; j++) {
-      const f16x2 dd = scale2(rs[0][w][j], 0), dm = offset2(rs[0][w][j], 0);
+      const f16x2 dd = qg_scale2<WT>(rs[0][w][j], 0), dm = qg_offset2<WT>(rs[0][w][j], 0);
       uint32_t o[4], ol[4] = {0, 0, 0, 0};
 #pragma unroll
       for (int b = 0; b < 4; b++) o[b] = qg_pair<WT, PREC>(rq[0][w][j], 0, b, dd, dm, ol[b]);
@@ -761,7 +777,7 @@ __device__ __forceinline__ void qg_tile(const QG2Args& a, const int e, const int
 #pragma unroll
         for (int j = 0; j < TN; j++) {
           // the dequantization of the next step's operand is cut into TM pieces, one pinned into the shadow of each MFMA
-          const f16x2 dd = scale2(rs[ns][w][j], nd), dm = offset2(rs[ns][w][j], nd);
+          const f16x2 dd = qg_scale2<WT>(rs[ns][w][j], nd), dm = qg_offset2<WT>(rs[ns][w][j], nd);
           uint32_t o[4], ol[4] = {0, 0, 0, 0};
 #pragma unroll
           for (int i = 0; i < TM; i++) {
@@ -790,30 +806,82 @@ __device__ __forceinline__ void qg_tile(const QG2Args& a, const int e, const int
     kstep(std::integral_constant<int, 0>{}, kt);
     kstep(std::integral_constant<int, 1>{}, kt + 1);
   }
+  for (int i = 0; i < idle; i++) __syncthreads();  // the barriers of the steps the other half of K still has
   __syncthreads();
+  if (G == 2) {
+    f32x4* part = reinterpret_cast<f32x4*>(smem_all);
+    if (group == 1) {
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int g = 0; g < 4; g++)
+            part[(((wave * TN + j) * TM + i) * 4 + g) * 64 + lane] = f32x4{acc[0][j][i][4 * g], acc[0][j][i][4 * g + 1], acc[0][j][i][4 * g + 2], acc[0][j][i][4 * g + 3]};
+    }
+    __syncthreads();
+    if (group == 0) {
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int g = 0; g < 4; g++) {
+            const f32x4 v = part[(((wave * TN + j) * TM + i) * 4 + g) * 64 + lane];
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc[0][j][i][4 * g + q] += v[q];
+          }
+    }
+    __syncthreads();
+  }
 
   // acc[w][j][i][4g+e] = result[row0 + 32i + lrow][n0 + wave*WN + 32j + 8g + 4hi + e]
-  if (NW == 1) {
+  if (NW == 1 && a.N % 4 == 0) {
+    // each 32-row slab is turned through LDS so that a wave stores whole rows of the workgroup's columns, 16 bytes per lane (a lane's
+    // own quads lie in 32 different rows: 2048 x 9728 x 2560 128 -> 125 us)
+    constexpr int BN = 4 * WN, ROWB = 4 * BN + 16, QPR = BN / 4;  // QPR: 16-byte pieces per row
+    constexpr int RPW = 8 / G;                                    // rows per wave
+    static_assert(RPW * QPR % 64 == 0, "a wave stores whole rows");
+    const int wall = group * 4 + wave;
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+      if (group == 0) {
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+          for (int g = 0; g < 4; g++)
+            *reinterpret_cast<f32x4*>(smem_all + lrow * ROWB + (wave * WN + j * 32 + 8 * g + 4 * hi) * 4) =
+                f32x4{acc[0][j][i][4 * g], acc[0][j][i][4 * g + 1], acc[0][j][i][4 * g + 2], acc[0][j][i][4 * g + 3]};
+      }
+      __syncthreads();
+      const int q = lane % QPR, n = n0 + 4 * q;
+      f32x4 bi = {0.f, 0.f, 0.f, 0.f};
+      if (biasp && n < a.N) bi = *reinterpret_cast<const f32x4*>(biasp + n);
+#pragma unroll
+      for (int t = 0; t < RPW * QPR / 64; t++) {
+        const int rl = wall * RPW + t * (64 / QPR) + lane / QPR, r = i * 32 + rl;
+        f32x4 v = *reinterpret_cast<const f32x4*>(smem_all + rl * ROWB + q * 16);
+        if (biasp) v += bi;
+        if (r < rows && n < a.N) {
+          const int pos = row0 + r;
+          *reinterpret_cast<f32x4*>(outp + (int64_t)(a.o_index ? a.o_index[pos] : pos) * a.N + n) = v;
+        }
+      }
+      if (i + 1 < TM) __syncthreads();
+    }
+  } else if (NW == 1) {
 #pragma unroll
     for (int i = 0; i < TM; i++) {
       const int r = i * 32 + lrow;
-      if (r < rows) {
+      if (r < rows && group == 0) {
         const int pos = row0 + r;
         float* orow = outp + (int64_t)(a.o_index ? a.o_index[pos] : pos) * a.N;
 #pragma unroll
         for (int j = 0; j < TN; j++)
 #pragma unroll
-          for (int g = 0; g < 4; g++) {
-            const int n = n0 + wave * WN + j * 32 + 8 * g + 4 * hi;
-            f32x4 v = {acc[0][j][i][4 * g], acc[0][j][i][4 * g + 1], acc[0][j][i][4 * g + 2], acc[0][j][i][4 * g + 3]};
-            if (n + 3 < a.N && a.N % 4 == 0) {
-              if (biasp) v += *reinterpret_cast<const f32x4*>(biasp + n);
-              *reinterpret_cast<f32x4*>(orow + n) = v;
-            } else {
-#pragma unroll
-              for (int e2 = 0; e2 < 4; e2++)
-                if (n + e2 < a.N) orow[n + e2] = biasp ? v[e2] + biasp[n + e2] : v[e2];
-            }
+          for (int q = 0; q < 16; q++) {
+            const int n = n0 + wave * WN + j * 32 + 8 * (q / 4) + 4 * hi + q % 4;
+            if (n < a.N) orow[n] = biasp ? acc[0][j][i][q] + biasp[n] : acc[0][j][i][q];
           }
       }
     }
@@ -858,38 +926,87 @@ __device__ __forceinline__ void qg_tile(const QG2Args& a, const int e, const int
   }
 }
 
+constexpr int QG_TILE_H = 128;
+constexpr int QG_SLOTS = 512;  // tiles in flight: two workgroups on each of 256 CUs
+
 // MODE 0: one matrix, 128 x 256 tiles, one-term operands.  MODE 1: gate and up together with two-term operands; a tile of
 // the list is cut into halves of 64 rows (blockIdx.z) x 128 channels.
 // The tile height follows the rows the tile really has: short tiles skip the MFMAs of empty row blocks.
-template <int WT, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void qg_kernel(QG2Args a) {
+template <int WT, int MODE, int G = 1>
+__global__ __launch_bounds__(256 * G) __attribute__((amdgpu_waves_per_eu(2, 2))) void qg_kernel(QG2Args a) {
   extern __shared__ __align__(16) unsigned char smem[];
-  const int t = blockIdx.x;
-  if (t >= min(a.ntiles[0], (int)gridDim.x)) return;
-  const int e = a.tile_expert[t];
-  int row0 = a.tile_row0[t], rows = a.tile_rows[t];
+  int e, row0, rows, n0 = blockIdx.y * (MODE == 1 ? 128 : 256);
+  if (MODE == 1 || a.ntiles) {
+    const int t = blockIdx.x;
+    if (t >= min(a.ntiles[0], (int)gridDim.x)) return;
+    e = a.tile_expert[t];
+    row0 = a.tile_row0[t];
+    rows = a.tile_rows[t];
+  } else {
+    // A plain Linear.  The column tiles behind big_cols run as half-height tiles, which are the first workgroups of the grid: the
+    // full-height tiles fill whole rounds of the chip, and short tiles share their CUs with full ones.
+    const int tilesM = (a.a_rows + QG_TILE_H - 1) / QG_TILE_H, tilesH = (a.a_rows + QG_TILE_H / 2 - 1) / (QG_TILE_H / 2);
+    const int nbig = tilesM * a.big_cols, nsmall = (int)gridDim.x - nbig;
+    int b = (int)blockIdx.x - nsmall;
+    e = 0;
+    if (b < 0) {
+      b = (int)blockIdx.x;
+      row0 = b % tilesH * (QG_TILE_H / 2);
+      rows = min(QG_TILE_H / 2, a.a_rows - row0);
+      n0 = (a.big_cols + b / tilesH) * 256;
+    } else {
+      int tm, tn;
+      if (tilesM % 2 == 0 && a.big_cols % 4 == 0) {  // an XCD takes half of the rows of a quarter of the columns
+        const int xcd = b & 7, seq = b >> 3, hm = tilesM / 2, qn = a.big_cols / 4;
+        tm = (xcd & 1) * hm + seq % hm;
+        tn = (xcd >> 1) * qn + seq / hm;
+      } else {
+        b = xcd_run(b, nbig);
+        tm = b % tilesM;
+        tn = b / tilesM;
+      }
+      row0 = tm * QG_TILE_H;
+      rows = min(QG_TILE_H, a.a_rows - row0);
+      n0 = tn * 256;
+    }
+  }
   if constexpr (MODE == 1) {
-    const int n0 = blockIdx.y * 128;
     row0 += 64 * blockIdx.z;
     rows -= 64 * blockIdx.z;
     if (rows <= 0) return;
     if (rows > 32) qg_tile<WT, 2, 2, 1, 2>(a, e, row0, min(rows, 64), n0, smem);
     else qg_tile<WT, 2, 1, 1, 2>(a, e, row0, rows, n0, smem);
   } else {
-    const int n0 = blockIdx.y * 256;
-    if (rows > 64) qg_tile<WT, 1, 4, 2, 1>(a, e, row0, rows, n0, smem);
-    else if (rows > 32) qg_tile<WT, 1, 2, 2, 1>(a, e, row0, rows, n0, smem);
-    else qg_tile<WT, 1, 1, 2, 1>(a, e, row0, rows, n0, smem);
+    if (rows > 64) qg_tile<WT, 1, 4, 2, 1, G>(a, e, row0, rows, n0, smem);
+    else if (rows > 32) qg_tile<WT, 1, 2, 2, 1, G>(a, e, row0, rows, n0, smem);
+    else qg_tile<WT, 1, 1, 2, 1, G>(a, e, row0, rows, n0, smem);
   }
 }
-
-constexpr int QG_TILE_H = 128;
 
 template <int MODE>
 static int launch_qg(const QG2Args& a, unsigned max_tiles, hipStream_t st) {
   constexpr int TN = MODE == 1 ? 1 : 2;
-  const dim3 grid(max_tiles, (unsigned)((a.N + 128 * TN - 1) / (128 * TN)), MODE == 1 ? 2 : (unsigned)(a.ksplit > 1 ? a.ksplit : 1));
-  const size_t lds = 2 * (size_t)QG_TILE_H * (2 * 64 + 16);  // MODE 1: half the rows, value + residual
+  dim3 grid(max_tiles, (unsigned)((a.N + 128 * TN - 1) / (128 * TN)), MODE == 1 ? 2 : (unsigned)(a.ksplit > 1 ? a.ksplit : 1));
+  if (MODE == 0 && !a.ntiles) {
+    const int64_t cols = grid.y, tilesH = (a.a_rows + QG_TILE_H / 2 - 1) / (QG_TILE_H / 2);
+    grid.x = (unsigned)(max_tiles * a.big_cols + tilesH * (cols - a.big_cols));
+    grid.y = 1;
+  }
+  if (MODE == 0 && a.halves) {
+    constexpr size_t lds = 128 * 1024;  // the sums of four waves
+    auto go = [&](auto kern) {
+      HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      hipLaunchKernelGGL(kern, grid, dim3(512), lds, st, a);
+      return (int)hipGetLastError();
+    };
+    switch (a.wtype) {
+      case MLLM_HIP_Q4_0: return go(qg_kernel<MLLM_HIP_Q4_0, 0, 2>);
+      case MLLM_HIP_Q8_0: return go(qg_kernel<MLLM_HIP_Q8_0, 0, 2>);
+      case MLLM_HIP_Q4_K: return go(qg_kernel<MLLM_HIP_Q4_K, 0, 2>);
+      default: return go(qg_kernel<MLLM_HIP_Q6_K, 0, 2>);
+    }
+  }
+  const size_t lds = 2 * (size_t)QG_TILE_H * (2 * 64 + 16);  // MODE 1: half the rows, value + residual (and the 32 rows of 256 sums of the epilogue)
   if (a.wtype == MLLM_HIP_Q4_0) hipLaunchKernelGGL((qg_kernel<MLLM_HIP_Q4_0, MODE>), grid, dim3(256), lds, st, a);
   else if (a.wtype == MLLM_HIP_Q8_0) hipLaunchKernelGGL((qg_kernel<MLLM_HIP_Q8_0, MODE>), grid, dim3(256), lds, st, a);
   else if constexpr (MODE == 0) {  // the super-block formats: plain Linear only
@@ -1735,6 +1852,80 @@ static int launch_tiles(int wtype, const QGemmArgs& a, unsigned max_tiles, hipSt
   return wtype == MLLM_HIP_Q4_0 ? launch(qgemm_tile_kernel<MLLM_HIP_Q4_0, MODE>) : launch(qgemm_tile_kernel<MLLM_HIP_Q8_0, MODE>);
 }
 
+// The gemm-packed matrix as wk_gemm.h reads it: a block is 64 elements, operand d the lane's eight weights of the d-th 16 of them,
+// dequantized to fp16 as in qg_tile.
+struct QWavesArgs {
+  const char* W;
+  const uint16_t* xh;  // fp16 [M][K]
+  const float* bias;   // [N] or null
+  float* y;            // [M][N]
+  int M, N, K;
+};
+template <int WT>
+struct QWaves {
+  typedef QWavesArgs Args;
+  typedef v16f Acc;
+  typedef f32x4 Sum4;
+  typedef f16x8 X;
+  static constexpr int QW = qg_nibbles(WT) ? 1 : 2, SDW = qg_scale_dwords(WT);
+  struct W {
+    u32x4 q[QW];
+    uint32_t s[SDW];
+  };
+  struct Col {
+    uint32_t q, s;
+  };
+  static __device__ __forceinline__ int kblocks(const Args& a) { return (a.K + 63) / 64; }
+  static __device__ __forceinline__ int row_bytes(const Args& a) { return a.K * 2; }
+  static __device__ __forceinline__ const void* activations(const Args& a) { return a.xh; }
+  static __device__ __forceinline__ __amdgpu_buffer_rsrc_t weights(const Args& a) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.W), 0, (uint32_t)qg_bytes(WT, a.N, a.K), 0x00020000);
+  }
+  static __device__ __forceinline__ Col col(const Args& a, int nb, int lane) {
+    const int64_t kbs = qg_kp(a.K) / 64;
+    nb = min(nb, (int)(qg_np(a.N) / 32) - 1);
+    return Col{(uint32_t)(nb * kbs * (1024 * QW) + lane * 16), (uint32_t)(qg_qbytes(WT, a.N, a.K) + (nb * kbs * 32 + (lane & 31)) * 4 * SDW)};
+  }
+  static __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, const Col& c, int kb, W& w) {
+#pragma unroll
+    for (int p = 0; p < QW; p++) w.q[p] = __builtin_amdgcn_raw_buffer_load_b128(r, kb < 0 ? 0xffffffffu : c.q, (kb * QW + p) * 1024, 0);
+    if constexpr (SDW == 1) {
+      w.s[0] = __builtin_amdgcn_raw_buffer_load_b32(r, kb < 0 ? 0xffffffffu : c.s, kb * 128, 0);
+    } else {
+      const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, kb < 0 ? 0xffffffffu : c.s, kb * 256, 0);
+      w.s[0] = v.x;
+      w.s[1] = v.y;
+    }
+  }
+  static __device__ __forceinline__ X operand(const W& w, int d) {
+    const f16x2 dd = qg_scale2<WT>(w.s, d), dm = qg_offset2<WT>(w.s, d);
+    uint32_t o[4], lo;
+#pragma unroll
+    for (int b = 0; b < 4; b++) o[b] = qg_pair<WT, 1>(w.q, d, b, dd, dm, lo);
+    return __builtin_bit_cast(f16x8, u32x4{o[0], o[1], o[2], o[3]});
+  }
+  static __device__ __forceinline__ Acc mma(const X& w, const X& x, const Acc& acc) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(w, x, acc, 0, 0, 0); }
+  static __device__ __forceinline__ void store(const Args& a, int m, int n, f32x4 v) {
+    float* y = a.y + (int64_t)m * a.N + n;
+    if (n + 3 < a.N && a.N % 4 == 0) {
+      if (a.bias) v += *reinterpret_cast<const f32x4*>(a.bias + n);
+      *reinterpret_cast<f32x4*>(y) = v;
+      return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (n + e < a.N) y[e] = a.bias ? v[e] + a.bias[n + e] : v[e];
+  }
+};
+template <int WT>
+static int launch_q_waves(int form, const QWavesArgs& a, hipStream_t st) {
+  switch (form) {
+    case 0: return wk_gemm_launch<QWaves<WT>, 1, 1, 8, 2>(a, st);
+    case 1: return wk_gemm_launch<QWaves<WT>, 1, 2, 8, 1>(a, st);
+    default: return wk_gemm_launch<QWaves<WT>, 2, 2, 4, 2>(a, st);
+  }
+}
+
 // y = sum over the K ranges of their partial results (in range order) + bias
 __global__ __launch_bounds__(256) void qg_reduce_kernel(const float* __restrict__ partial, int Z, int64_t MN, int N, const float* __restrict__ bias,
                                                         float* __restrict__ y) {
@@ -1746,46 +1937,83 @@ __global__ __launch_bounds__(256) void qg_reduce_kernel(const float* __restrict_
   *reinterpret_cast<f32x4*>(y + i) = v;
 }
 
-// Short batches: a Linear of a few hundred rows has M/128 x N/256 tiles, far fewer than the chip has CUs (gate projection of
-// the 4B layer at 128 rows: 38 workgroups, down: 10), and each streams its weights two K steps ahead only.  K is therefore
-// cut into up to eight ranges that run as separate workgroups and leave partial results, summed by a small second kernel
-// in range order.  Number of ranges: enough for about one workgroup per CU, at most 24 MB of partial results (their round trip through memory is what the second kernel costs); up to 1024 rows.
-int qg_short_splits(int64_t M, int64_t N, int64_t K) {
-  if (M > 1024 || N % 4) return 1;
-  const int64_t tiles = ((M + QG_TILE_H - 1) / QG_TILE_H) * ((N + 255) / 256);
-  const int KT = (int)(qg_kp(K) / 64);
-  int z = (int)((256 + tiles - 1) / tiles);
-  if (z > 8) z = 8;
-  while (z > 1 && (int64_t)z * M * N * 4 > (24 << 20)) z--;
-  if (z <= 1) return 1;
-  const int per = ((KT + z - 1) / z + 1) / 2 * 2;
-  return (KT + per - 1) / per;  // no empty range
+// How a Linear runs.  Up to a few hundred rows its M/128 x N/256 tiles are far fewer than the chip has CUs (gate projection of the
+// 4B layer at 128 rows: 38, down: 10), so there is a choice:
+//   waves   the waves of a workgroup split K of a small tile (wk_gemm.h; forms 0..2 of launch_q_waves)
+//   halves  128 x 256 tiles by eight waves, four for each half of K: two waves per SIMD where a tile has a CU to itself
+//   ranges  128 x 256 tiles by four waves, K cut into up to eight ranges that run as separate workgroups, leave partial results and
+//           are added by a small second kernel in range order; one range: the plain form, with half-height tiles for a short
+//           last round
+// The expected cost of each, in us, is fitted to 130 shapes of 1 to 28 M weights and 93 to 2048 rows within 4 to 9 % (rms; form 0: 17 %);
+// the choice is within 1.2 % of the best form on average, 14 % at worst.  131 x 2560 x 9728 (Q6_K, with the activations' kernel):
+// 33.6 -> 26 us, 93 x 6144 x 2048 (Q4_0) 27 -> 14, 700 x 6144 x 2048 43.7 -> 39, 2048 x 2048 x 6144 102 -> 80.
+struct QLinearPlan {
+  int waves;   // form of launch_q_waves, or -1
+  int halves;
+  int ranges;
+};
+static QLinearPlan q_linear_plan(int64_t M, int64_t N, int64_t K, bool ranges_fit) {
+  static const FormCost waves[] = {{32, 32, 0.0f, 1.22f, 0.36f, 0.1026f}, {32, 64, 0.5f, 1.72f, 0.97f, 0.1251f}, {64, 64, 0.5f, 2.22f, 1.86f, 0.2001f}};
+  const int64_t blocks = (K + 63) / 64;
+  const float mn = (float)M * (float)N * 1e-6f;
+  QLinearPlan best{-1, 0, 1};
+  float least = 0.f;
+  auto offer = [&](float cost, const QLinearPlan& p) {
+    if (least == 0.f || cost < least) {
+      least = cost;
+      best = p;
+    }
+  };
+  for (int f = 0; f < 3; f++) offer(form_cost(waves[f], M, N, blocks), QLinearPlan{f, 0, 1});
+  // a ragged last tile of 128 rows runs as 64 or 32
+  const int64_t rest = M % QG_TILE_H;
+  const float tiles = ((float)(M / QG_TILE_H) + (rest == 0 ? 0.f : rest > 64 ? 1.f : rest > 32 ? 0.7f : 0.5f)) * (float)((N + 255) / 256);
+  offer(5.52f + ceilf(tiles / 256.f) * (1.56f + 0.6155f * (float)blocks) + 1.874f * mn, QLinearPlan{-1, 1, 1});
+  for (int z = 1; z <= 8; z++) {
+    if (z > 1 && (!ranges_fit || N % 4 || (float)z * mn > 16.f)) break;  // 64 MB of partial results at most
+    const int64_t per = ((blocks + z - 1) / z + 1) / 2 * 2;
+    if ((blocks + per - 1) / per != z) continue;  // no empty range
+    const float t = tiles * (float)z, rounds = t <= 256.f ? 1.f : t <= 512.f ? 1.5f : 1.5f * (0.5f * ceilf(t / 512.f) + t / 1024.f);
+    offer(4.75f + rounds * (3.80f + 0.793f * (float)per) + 0.895f * mn + (z > 1 ? 0.804f * (float)(z + 1) * mn + 2.76f : 0.f), QLinearPlan{-1, 0, z});
+  }
+  return best;
 }
 size_t qg_partial_bytes(int64_t M, int64_t N, int64_t K) {
-  const int z = qg_short_splits(M, N, K);
+  const int z = q_linear_plan(M, N, K, true).ranges;
   return z > 1 ? align_up((size_t)z * M * N * 4, 256) : 0;
 }
 
-size_t qg_route_bytes(int64_t M) {
-  Carver c(nullptr);
-  carve_route(c, 1, M);
-  return c.used;
-}
 int qg_linear_run(int wtype, const void* gemm_packed, const uint16_t* xh, const float* bias, float* y, int64_t M, int64_t N,
-                  int64_t K, void* route_ws, void* partial_ws, hipStream_t st) {
-  Carver c(route_ws);
-  RouteOut ro = carve_route(c, 1, M);
-  RC_RET(launch_identity_tiles(M, QG_TILE_H, ro, st));
+                  int64_t K, void* partial_ws, hipStream_t st) {
+  const QLinearPlan plan = q_linear_plan(M, N, K, partial_ws != nullptr);
+  if (plan.waves >= 0) {
+    const QWavesArgs w{reinterpret_cast<const char*>(gemm_packed), xh, bias, y, (int)M, (int)N, (int)K};
+    switch (wtype) {
+      case MLLM_HIP_Q4_0: return launch_q_waves<MLLM_HIP_Q4_0>(plan.waves, w, st);
+      case MLLM_HIP_Q8_0: return launch_q_waves<MLLM_HIP_Q8_0>(plan.waves, w, st);
+      case MLLM_HIP_Q4_K: return launch_q_waves<MLLM_HIP_Q4_K>(plan.waves, w, st);
+      default: return launch_q_waves<MLLM_HIP_Q6_K>(plan.waves, w, st);
+    }
+  }
   QG2Args a{};
   a.W0 = a.W1 = reinterpret_cast<const char*>(gemm_packed);
   a.wstride = 0;
   a.xh = xh; a.a_index = nullptr; a.a_div = 1; a.a_rows = (int)M;
   a.o_index = nullptr; a.out = y; a.bias = bias;
-  a.tile_expert = ro.tile_expert; a.tile_row0 = ro.tile_row0; a.tile_rows = ro.tile_rows; a.ntiles = ro.ntiles;
   a.N = (int)N; a.K = (int)K; a.wtype = wtype; a.x86_scale = 0;
-  a.ksplit = partial_ws ? qg_short_splits(M, N, K) : 1;
+  a.ksplit = plan.ranges;
+  a.halves = plan.halves;
   a.partial = reinterpret_cast<float*>(partial_ws);
-  const int rc = launch_qg<0>(a, (unsigned)((M + QG_TILE_H - 1) / QG_TILE_H), st);
+  const int64_t tilesM = (M + QG_TILE_H - 1) / QG_TILE_H, cols = (N + 255) / 256, total = tilesM * cols;
+  a.big_cols = (int)cols;
+  if (a.ksplit <= 1 && !a.halves && total > QG_SLOTS && total % QG_SLOTS) {
+    // columns whose full tiles fill whole rounds; the others as half-height tiles if that ends earlier (such a tile takes about 0.6 of
+    // a full one: it dequantizes the same weights for half the rows)
+    const int64_t big = total / QG_SLOTS * QG_SLOTS / tilesM, halves = (cols - big) * ((M + QG_TILE_H / 2 - 1) / (QG_TILE_H / 2));
+    const double with_tail = (double)((big * tilesM + QG_SLOTS - 1) / QG_SLOTS) + 0.6 * (double)((halves + QG_SLOTS - 1) / QG_SLOTS);
+    if (with_tail < (double)((total + QG_SLOTS - 1) / QG_SLOTS)) a.big_cols = (int)big;
+  }
+  const int rc = launch_qg<0>(a, (unsigned)tilesM, st);
   if (rc || a.ksplit <= 1) return rc;
   hipLaunchKernelGGL(qg_reduce_kernel, dim3((unsigned)((M * N / 4 + 255) / 256)), dim3(256), 0, st, a.partial, a.ksplit, M * N, (int)N, bias, y);
   return (int)hipGetLastError();
@@ -2016,7 +2244,6 @@ MLLM_API size_t mllm_hip_linear_q_gemm_workspace_bytes(int64_t M, int64_t K) {
   if (M <= 0 || K <= 0 || K % QK) return 0;
   Carver c(nullptr);
   c.take<uint16_t>((size_t)M * K);
-  carve_route(c, 1, M);
   return c.used;
 }
 
@@ -2037,13 +2264,13 @@ MLLM_API int mllm_hip_linear_q_gemm(int wtype, const void* gemm_packed, const vo
   const int64_t nblocks = M * (K / QK);
   hipLaunchKernelGGL(qg_act_kernel, dim3((unsigned)((nblocks + 127) / 128)), dim3(128), 0, st, x, x_dtype, xh,
                      (uint16_t*)nullptr, nblocks, act_scale_mode == MLLM_HIP_SCALE_X86_REF);
-  return qg_linear_run(wtype, gemm_packed, xh, bias, y, M, N, K, c.p + c.used, nullptr, st);
+  return qg_linear_run(wtype, gemm_packed, xh, bias, y, M, N, K, nullptr, st);
 }
 
-// the same for short batches (M <= 256 gains; any M is accepted): K cut into ranges, see qg_short_splits
+// the same with room for the partial results of K ranges (behind the activations, on a 256-byte line of their own)
 MLLM_API size_t mllm_hip_linear_q_gemm_short_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % QK) return 0;
-  return mllm_hip_linear_q_gemm_workspace_bytes(M, K) + qg_partial_bytes(M, N, K);
+  return align_up(mllm_hip_linear_q_gemm_workspace_bytes(M, K), 256) + 256 + qg_partial_bytes(M, N, K);
 }
 MLLM_API int mllm_hip_linear_q_gemm_short(int wtype, const void* gemm_packed, const void* x, int x_dtype, const float* bias, float* y,
                                           int64_t M, int64_t N, int64_t K, int act_scale_mode, void* workspace, void* stream) {
@@ -2061,9 +2288,8 @@ MLLM_API int mllm_hip_linear_q_gemm_short(int wtype, const void* gemm_packed, co
   const int64_t nblocks = M * (K / QK);
   hipLaunchKernelGGL(qg_act_kernel, dim3((unsigned)((nblocks + 127) / 128)), dim3(128), 0, st, x, x_dtype, xh,
                      (uint16_t*)nullptr, nblocks, act_scale_mode == MLLM_HIP_SCALE_X86_REF);
-  void* route = c.p + c.used;
-  void* partial = qg_partial_bytes(M, N, K) ? c.p + mllm_hip_linear_q_gemm_workspace_bytes(M, K) : nullptr;
-  return qg_linear_run(wtype, gemm_packed, xh, bias, y, M, N, K, route, partial, st);
+  void* partial = qg_partial_bytes(M, N, K) ? c.p + align_up(mllm_hip_linear_q_gemm_workspace_bytes(M, K), 256) : nullptr;
+  return qg_linear_run(wtype, gemm_packed, xh, bias, y, M, N, K, partial, st);
 }
 
 namespace mllmhip {

@@ -86,6 +86,26 @@ def test_linear_q_gemm_short_batches(wtype, M, N, K):
     assert rel_l2(ys, ql.linear_q_gemm(w, to_dev(x), to_dev(bias)).cpu().numpy()) < 2e-6
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 40, 64), (33, 200, 96), (49, 5000, 1504), (97, 1030, 2048 + 32), (300, 520, 4096), (129, 3000, 9728),
+                                   (700, 6144, 2048 + 64), (1300, 3000, 3008), (1500, 2560, 9728), (2048, 2048, 6144), (2000, 9728, 512)])
+def test_linear_q_gemm_forms(M, N, K):
+    """the forms a Linear takes from a few rows to a long prompt: waves that split K (tiles of 32 and 64, ragged, K blocks that do not
+    divide), halves of K in one workgroup (odd numbers of K steps), K ranges, half-height tiles in a short last round; element stores
+    (N % 4 != 0).  Sampled rows, the last ones among them, against the oracle; the two calls agree on all rows up to the order of sums"""
+    for wtype in (0, 1) if M < 1000 else (0,):
+        rng = synth.rng_for(4, 900 + M + N % 97 + wtype)
+        W = synth.make_weight(rng, wtype, N, K)
+        w = ql.PackedQWeight(wtype, torch.from_numpy(W), layout="gemm")
+        x = synth.make_x_fp32(rng, M, K)
+        bias = rng.standard_normal(N).astype(np.float32)
+        announce("linear_q_gemm forms", wtype, M, N, K)
+        ys = ql.linear_q_gemm(w, to_dev(x), to_dev(bias), short=True).cpu().numpy()
+        rows = np.unique(np.concatenate([rng.integers(0, M, 6), np.arange(max(0, M - 2), M)]))
+        assert rel_l2(ys[rows], orc.linear_q(x[rows], W, wtype, bias)) < GEMM_TOL
+        # fp32 sums of K products in two orders: about sqrt(K) * 2^-24 apart, relative to the result's own size
+        assert rel_l2(ys, ql.linear_q_gemm(w, to_dev(x), to_dev(bias)).cpu().numpy()) < 4 * np.sqrt(K) * 2.0 ** -24
+
+
 def test_linear_q_gemm_exact_when_operands_fit_fp16():
     """Weights and activations chosen so that dW*qW and dX*qX are exactly representable in fp16 and every partial sum in
     fp32: then the matrix-core path must equal the reference arithmetic bit for bit (a wrong nibble order, scale pairing,
