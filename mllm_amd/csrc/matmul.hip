@@ -3,14 +3,14 @@
 // loop of mllm/backends/cpu/kernels/common/ggml/matmul.cpp / mllm_blas).  Not a quantized path.
 //   fp32 operands   v_mfma_f32_32x32x2f32: exact fp32 products, fp32 accumulation (the CPU's arithmetic in another order)
 //   bf16 / fp16     v_mfma_f32_32x32x16_{bf16,f16}: exact products, fp32 accumulation, one rounding of the result
-// One launch covers the whole batch (blockIdx.z walks it; a stride of 0 broadcasts an operand).
+// One launch covers the whole batch (a stride of 0 broadcasts an operand).
 //
-// Workgroup = 2 x 2 waves, each wave (32 TM) x (32 TN) outputs, K step 32.  Both operand tiles sit in LDS as [row][k] with
-// 16 bytes of padding per row, whichever way the tensor is laid out in memory (an operand that is contiguous along its row
-// index is transposed on its way into LDS).  Inside a K step lane half h takes k = 16 h .. 16 h + 15 of its row, for both
+// Workgroup = 2 x 2 waves, each wave (32 TM) x (32 TN) outputs, K step 32.  Both operand tiles sit in LDS with
+// 16 bytes of padding per row, as [row][k] whichever way the tensor is laid out in memory (fp32 [K][rows] operands stay [k][row]).  Inside a K step lane half h takes k = 16 h .. 16 h + 15 of its row, for both
 // operands alike: the order in which an MFMA walks k is free, and this way every lane fetches its operands of the whole
 // step with 16-byte LDS reads.
 #include <algorithm>
+#include <cmath>
 
 #include "qcommon.h"
 
@@ -26,7 +26,7 @@ struct MMArgs {
   void* C;
   int M, N, K, batch;
   int64_t sA, sB, sC;  // batch strides in elements
-  int vecA, vecB;      // 16-byte loads allowed (base, leading dimension and batch stride all multiples of 16 bytes)
+  int vecA, vecB;      // aligned 16-byte loads of whole rows (base, leading dimension and batch stride all multiples of 16 bytes)
 };
 
 template <int DT>
@@ -38,15 +38,27 @@ struct MMElem<MLLM_HIP_F32> {
   using type = float;
 };
 
-// One operand tile of ROWS x 32 elements from global memory into registers, then into LDS as [row][k].
-// CONTIG_K: the tensor is [rows][K] (k contiguous); otherwise it is [K][rows].
+// One operand tile of ROWS x 32 elements from global memory into registers, then into LDS.
+// CONTIG_K: the tensor is [rows][K] (k contiguous); otherwise it is [K][rows].  In LDS the tile is [row][k], except that an fp32
+// tensor [K][rows] stays [k][row]: v_mfma_f32_32x32x2f32 takes one k per lane half, so a lane's operand is one dword and
+// neighbouring lanes read neighbouring dwords.  A 16-bit tensor [K][rows] is loaded as two neighbouring k of four rows per
+// thread and vector, which makes one dword of LDS per row.
+// Whole tiles load whole vectors whatever the alignment of the rows (odd row lengths among them); rows past the end repeat the
+// last ones (their results are never stored).  A K step that ends behind K, and a last tile of rows that are not a multiple of
+// the vector in a [K][rows] tensor, load element by element with zeros outside.
 template <typename E, int ROWS, bool CONTIG_K>
 struct MMTile {
   static constexpr int VE = 16 / (int)sizeof(E);
-  static constexpr int LDK = 32 + VE;
-  static constexpr int NV = ROWS * 32 / VE / 256;  // 16-byte vectors per thread
+  static constexpr bool KROWS = !CONTIG_K && sizeof(E) == 4;   // [k][row] in LDS
+  static constexpr bool PAIRS = !CONTIG_K && sizeof(E) == 2;   // two k of four rows per vector
+  static constexpr int RV = CONTIG_K ? 1 : 4;                  // rows of a vector
+  static constexpr int LD = KROWS ? ROWS + VE : 32 + VE;
+  static constexpr int SIZE = KROWS ? 32 * LD : ROWS * LD;     // elements in LDS
+  static constexpr int NV = ROWS * 32 / VE / 256;              // 16-byte vectors per thread
   static_assert(ROWS * 32 / VE % 256 == 0, "tile must split evenly over 256 threads");
   u32x4 v[NV];
+  const E* p[NV];
+  bool whole;
 
   static __device__ __forceinline__ uint32_t bits(E e) {
     if constexpr (sizeof(E) == 4) return __builtin_bit_cast(uint32_t, e);
@@ -59,157 +71,195 @@ struct MMTile {
     if constexpr (sizeof(E) == 4) return __builtin_bit_cast(E, d);
     else return (E)d;
   }
-
-  __device__ __forceinline__ void load(const E* __restrict__ X, int row0, int k0, int rows, int K, bool vec) {
+  static __device__ __forceinline__ void place(int c, int& r, int& k) {  // first element of vector c of this thread inside the tile
+    const int idx = c * 256 + (int)threadIdx.x;
+    if (CONTIG_K) r = idx / (32 / VE), k = (idx % (32 / VE)) * VE;
+    else if (PAIRS) k = idx / (ROWS / 4) * 2, r = (idx % (ROWS / 4)) * 4;
+    else k = idx / (ROWS / VE), r = (idx % (ROWS / VE)) * VE;
+  }
+  __device__ __forceinline__ void start(const E* __restrict__ X, int row0, int rows, int K) {
+    whole = CONTIG_K || (rows >= RV && (row0 + ROWS <= rows || rows % RV == 0));  // (the same in every thread)
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
-      const int idx = c * 256 + (int)threadIdx.x;
       int r, k;
-      int64_t off;
-      if (CONTIG_K) {
-        r = row0 + idx / (32 / VE), k = k0 + (idx % (32 / VE)) * VE;
-        off = (int64_t)r * K + k;
-      } else {
-        k = k0 + idx / (ROWS / VE), r = row0 + (idx % (ROWS / VE)) * VE;
-        off = (int64_t)k * rows + r;
-      }
-      if (vec) {
-        u32x4 q = {0u, 0u, 0u, 0u};
-        if (r < rows && k < K) q = *reinterpret_cast<const u32x4*>(X + off);
-        v[c] = q;
-      } else {
-        u32x4 q = {0u, 0u, 0u, 0u};
+      place(c, r, k);
+      if (CONTIG_K) p[c] = X + (int64_t)min(row0 + r, rows - 1) * K + k;
+      else p[c] = X + (int64_t)k * rows + (whole ? min(row0 + r, rows - RV) : 0);
+    }
+  }
+  __device__ __forceinline__ void load(const E* __restrict__ X, int row0, int k0, int rows, int K) {
+    if (whole && k0 + 32 <= K) {
+      const int64_t step = CONTIG_K ? (int64_t)k0 : (int64_t)k0 * rows;
 #pragma unroll
-        for (int j = 0; j < VE; ++j) {
-          const bool ok = CONTIG_K ? (r < rows && k + j < K) : (r + j < rows && k < K);
-          const uint32_t e = ok ? bits(X[off + j]) : 0u;
-          if constexpr (sizeof(E) == 4) q[j] = e;
-          else q[j >> 1] |= e << (16 * (j & 1));
+      for (int c = 0; c < NV; ++c) {
+        if constexpr (PAIRS) {
+          u32x2 lo, hi;
+          __builtin_memcpy(&lo, p[c] + step, 8);
+          __builtin_memcpy(&hi, p[c] + step + rows, 8);
+          v[c] = u32x4{lo.x, lo.y, hi.x, hi.y};
+        } else {
+          __builtin_memcpy(&v[c], p[c] + step, 16);
         }
-        v[c] = q;
       }
+      return;
+    }
+#pragma unroll
+    for (int c = 0; c < NV; ++c) {
+      int r, k;
+      place(c, r, k);
+      r += row0;
+      k += k0;
+      u32x4 q = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int j = 0; j < VE; ++j) {
+        const int rj = CONTIG_K ? r : PAIRS ? r + j % 4 : r + j, kj = CONTIG_K ? k + j : PAIRS ? k + j / 4 : k;
+        const uint32_t e = rj < rows && kj < K ? bits(X[CONTIG_K ? (int64_t)rj * K + kj : (int64_t)kj * rows + rj]) : 0u;
+        if constexpr (sizeof(E) == 4) q[j] = e;
+        else q[j >> 1] |= e << (16 * (j & 1));
+      }
+      v[c] = q;
     }
   }
   __device__ __forceinline__ void store(E* __restrict__ s) const {
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
-      const int idx = c * 256 + (int)threadIdx.x;
-      if (CONTIG_K) {
-        const int r = idx / (32 / VE), k = (idx % (32 / VE)) * VE;
-        *reinterpret_cast<u32x4*>(s + r * LDK + k) = v[c];
+      int r, k;
+      place(c, r, k);
+      if constexpr (CONTIG_K) {
+        *reinterpret_cast<u32x4*>(s + r * LD + k) = v[c];
+      } else if constexpr (KROWS) {
+        *reinterpret_cast<u32x4*>(s + k * LD + r) = v[c];
       } else {
-        const int k = idx / (ROWS / VE), r = (idx % (ROWS / VE)) * VE;
 #pragma unroll
-        for (int j = 0; j < VE; ++j) s[(r + j) * LDK + k] = elem(v[c], j);
+        for (int j = 0; j < 4; ++j)
+          *reinterpret_cast<uint32_t*>(s + (r + j) * LD + k) = __builtin_amdgcn_perm(v[c][2 + (j >> 1)], v[c][j >> 1], j & 1 ? 0x07060302u : 0x05040100u);
       }
     }
   }
+  // fp32: the operand of instruction 4 q + s of a K step (k = 16 h + 4 q + s) for s = 0 .. 3, row r of the tile
+  static __device__ __forceinline__ f32x4 four(const E* __restrict__ s, int r, int h, int q) {
+    static_assert(sizeof(E) == 4 || !KROWS, "");
+    const float* f = reinterpret_cast<const float*>(s);
+    if constexpr (!KROWS) return *reinterpret_cast<const f32x4*>(f + r * LD + 16 * h + 4 * q);
+    else return f32x4{f[(16 * h + 4 * q) * LD + r], f[(16 * h + 4 * q + 1) * LD + r], f[(16 * h + 4 * q + 2) * LD + r], f[(16 * h + 4 * q + 3) * LD + r]};
+  }
 };
 
+// Bound by the matrix pipe in fp32 (157 TFLOP/s nominal), by LDS reads and the output in 16 bits.  The next K step is loaded into
+// registers during this one's matrix instructions.  One LDS stage: a second one halves the workgroups of a CU, which hide
+// the barriers better (fp32 8 x 3108 x 777 x 128: 59 us, 62 with two stages).  The tiles of one batch entry are
+// neighbours on one XCD, whose L2 then holds that entry's operands.  16 bits, large tile: 128 registers, four waves per SIMD instead of
+// three (4096 x 4096 x 4096 bf16: 236 -> 180 us).
+//   (heads x rows x keys x d) fp32 8 x 3108 x 777 x 128: scores 80 -> 59 us, values 97 -> 65; bf16 33 -> 23, 70 -> 26 (odd row lengths
+//   loaded element by element and transposed through 16 two-byte LDS stores before)
 template <int DT, bool TA, bool TB, int TM, int TN>
-__global__ __launch_bounds__(256) void matmul_kernel(MMArgs a) {
+__global__ __launch_bounds__(256, (TM * TN == 4 && DT != MLLM_HIP_F32) ? 4 : 1) void matmul_kernel(MMArgs a) {
   using E = typename MMElem<DT>::type;
-  constexpr int VE = 16 / (int)sizeof(E), LDK = 32 + VE;
   constexpr int BM = 64 * TM, BN = 64 * TN;
-  __shared__ __align__(16) E sA[BM * LDK];
-  __shared__ __align__(16) E sB[BN * LDK];
+  // A is [M][K], or [K][M] when transposed; B is [K][N], or [N][K] when transposed
+  typedef MMTile<E, BM, !TA> TileA;
+  typedef MMTile<E, BN, TB> TileB;
+  __shared__ __align__(16) E sA[TileA::SIZE];
+  __shared__ __align__(16) E sB[TileB::SIZE];
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave >> 1, wn = wave & 1, r = lane & 31, h = lane >> 5;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
   const int KT = (a.K + 31) / 32;
+  const int tilesM = (a.M + BM - 1) / BM, tilesN = (a.N + BN - 1) / BN, tiles = tilesM * tilesN;
+  const int t = xcd_run(blockIdx.x, gridDim.x), z = t / tiles, in = t - z * tiles;
+  const int n0 = in / tilesM * BN, m0 = in % tilesM * BM;
+  const E* A = reinterpret_cast<const E*>(a.A) + z * a.sA;
+  const E* B = reinterpret_cast<const E*>(a.B) + z * a.sB;
+  E* C = reinterpret_cast<E*>(a.C) + z * a.sC;
 
-  for (int z = blockIdx.z; z < a.batch; z += gridDim.z) {
-    const E* A = reinterpret_cast<const E*>(a.A) + z * a.sA;
-    const E* B = reinterpret_cast<const E*>(a.B) + z * a.sB;
-    E* C = reinterpret_cast<E*>(a.C) + z * a.sC;
+  TileA ta;
+  TileB tb;
+  mm_f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
-    // A is [M][K], or [K][M] when transposed; B is [K][N], or [N][K] when transposed
-    MMTile<E, BM, !TA> ta;
-    MMTile<E, BN, TB> tb;
-    mm_f32x16 acc[TM][TN];
+  ta.start(A, m0, a.M, a.K);
+  tb.start(B, n0, a.N, a.K);
+  ta.load(A, m0, 0, a.M, a.K);
+  tb.load(B, n0, 0, a.N, a.K);
+  for (int kt = 0; kt < KT; ++kt) {
+    __syncthreads();  // the previous step's LDS reads are done
+    ta.store(sA);
+    tb.store(sB);
+    __syncthreads();
+    if (kt + 1 < KT) {
+      ta.load(A, m0, (kt + 1) * 32, a.M, a.K);
+      tb.load(B, n0, (kt + 1) * 32, a.N, a.K);
+    }
+    if constexpr (DT == MLLM_HIP_F32) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+      for (int q = 0; q < 4; ++q) {  // four k of this lane's sixteen at a time
+        f32x4 fa[TM], fb[TN];
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+        for (int i = 0; i < TM; ++i) fa[i] = TileA::four(sA, wm * 32 * TM + i * 32 + r, h, q);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-
-    ta.load(A, m0, 0, a.M, a.K, a.vecA);
-    tb.load(B, n0, 0, a.N, a.K, a.vecB);
-    for (int kt = 0; kt < KT; ++kt) {
-      __syncthreads();  // the previous step's LDS reads are done
-      ta.store(sA);
-      tb.store(sB);
-      __syncthreads();
-      if (kt + 1 < KT) {
-        ta.load(A, m0, (kt + 1) * 32, a.M, a.K, a.vecA);
-        tb.load(B, n0, (kt + 1) * 32, a.N, a.K, a.vecB);
-      }
-      if constexpr (DT == MLLM_HIP_F32) {
+        for (int j = 0; j < TN; ++j) fb[j] = TileB::four(sB, wn * 32 * TN + j * 32 + r, h, q);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {  // four k of this lane's sixteen at a time
-          f32x4 fa[TM], fb[TN];
-#pragma unroll
-          for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const f32x4*>(sA + (wm * 32 * TM + i * 32 + r) * LDK + 16 * h + 4 * q);
-#pragma unroll
-          for (int j = 0; j < TN; ++j) fb[j] = *reinterpret_cast<const f32x4*>(sB + (wn * 32 * TN + j * 32 + r) * LDK + 16 * h + 4 * q);
-#pragma unroll
-          for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-              for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][s], fb[j][s], acc[i][j], 0, 0, 0);
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          u32x4 fa[TM], fb[TN];
-#pragma unroll
-          for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const u32x4*>(sA + (wm * 32 * TM + i * 32 + r) * LDK + 16 * h + 8 * q);
-#pragma unroll
-          for (int j = 0; j < TN; ++j) fb[j] = *reinterpret_cast<const u32x4*>(sB + (wn * 32 * TN + j * 32 + r) * LDK + 16 * h + 8 * q);
+        for (int s = 0; s < 4; ++s)
 #pragma unroll
           for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-              if constexpr (DT == MLLM_HIP_BF16)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mm_bf16x8, fa[i]),
-                                                                    __builtin_bit_cast(mm_bf16x8, fb[j]), acc[i][j], 0, 0, 0);
-              else
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mm_f16x8, fa[i]),
-                                                                   __builtin_bit_cast(mm_f16x8, fb[j]), acc[i][j], 0, 0, 0);
-            }
-        }
+            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][s], fb[j][s], acc[i][j], 0, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        u32x4 fa[TM], fb[TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const u32x4*>(sA + (wm * 32 * TM + i * 32 + r) * TileA::LD + 16 * h + 8 * q);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fb[j] = *reinterpret_cast<const u32x4*>(sB + (wn * 32 * TN + j * 32 + r) * TileB::LD + 16 * h + 8 * q);
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            if constexpr (DT == MLLM_HIP_BF16)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mm_bf16x8, fa[i]),
+                                                                  __builtin_bit_cast(mm_bf16x8, fb[j]), acc[i][j], 0, 0, 0);
+            else
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mm_f16x8, fa[i]),
+                                                                 __builtin_bit_cast(mm_f16x8, fb[j]), acc[i][j], 0, 0, 0);
+          }
       }
     }
+  }
 
-    // 32x32 accumulator layout: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32
+  // 32x32 accumulator layout: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32
+  auto put = [&](int m, int n, float f) {
+    if constexpr (DT == MLLM_HIP_F32) C[(int64_t)m * a.N + n] = f;
+    else if constexpr (DT == MLLM_HIP_BF16) C[(int64_t)m * a.N + n] = f32_to_bf16(f);
+    else C[(int64_t)m * a.N + n] = f32_to_f16bits(f);
+  };
+  const bool full = m0 + BM <= a.M && n0 + BN <= a.N;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = n0 + wn * 32 * TN + j * 32 + r;
+  for (int j = 0; j < TN; ++j) {
+    const int n = n0 + wn * 32 * TN + j * 32 + r;
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int m = m0 + wm * 32 * TM + i * 32 + 8 * (v / 4) + 4 * h + (v % 4);
-          if (n < a.N && m < a.M) {
-            const float f = acc[i][j][v];
-            if constexpr (DT == MLLM_HIP_F32) C[(int64_t)m * a.N + n] = f;
-            else if constexpr (DT == MLLM_HIP_BF16) C[(int64_t)m * a.N + n] = f32_to_bf16(f);
-            else C[(int64_t)m * a.N + n] = f32_to_f16bits(f);
-          }
-        }
-    }
+      for (int v = 0; v < 16; ++v) {
+        const int m = m0 + wm * 32 * TM + i * 32 + 8 * (v / 4) + 4 * h + (v % 4);
+        if (full || (n < a.N && m < a.M)) put(m, n, acc[i][j][v]);
+      }
   }
 }
 
 // Up to four rows of A [M][K] against B [K][N] (attention probabilities x values of a decode token): a GEMV per row, bound by
 // reading B once, which the tile kernel above walks with one workgroup per 64 columns and a K step at a time (32 heads x
 // 8192 x 128 bf16: 158 us, 0.43 TB/s).  Here a workgroup of sixteen waves takes 2^lpr_log2 x VE columns (VE elements = 16
-// bytes per lane); a wave reads 64 >> lpr_log2 rows of B per pass, the waves stride over K, four passes requested before the
-// first is multiplied; fp32 sums per lane, then over the lanes of a column (wave shuffles), then over the waves in order
-// through LDS.  Exact products, fp32 sums in another order than the tile kernel's.
+// bytes per lane); a lane takes four neighbouring k per pass, whose elements of A are one load per row (one load per element of A
+// beside each load of B bound the kernel before: 8 x 4 x 8000 x 128 bf16 48.6 -> 20.9 us), the waves stride over K; fp32 sums per lane,
+// then over the lanes of a column (wave shuffles), then over the waves in order through LDS.  Exact products, fp32 sums in
+// another order than the tile kernel's.  The column blocks of a batch entry run on one XCD: they share the cache lines of B.
 template <int DT>
 __device__ __forceinline__ float mm_to_f32(typename MMElem<DT>::type e) {
   if constexpr (DT == MLLM_HIP_F32) return e;
@@ -218,68 +268,73 @@ __device__ __forceinline__ float mm_to_f32(typename MMElem<DT>::type e) {
 }
 constexpr int MMR_WAVES = 16;
 template <int DT, int MR>
-__global__ __launch_bounds__(MMR_WAVES * 64) void matmul_rows_kernel(MMArgs a, int lpr_log2) {
+__global__ __launch_bounds__(MMR_WAVES * 64) void matmul_rows_kernel(MMArgs a, int lpr_log2, int col_blocks) {
   using E = typename MMElem<DT>::type;
-  constexpr int VE = 16 / (int)sizeof(E);
+  constexpr int VE = 16 / (int)sizeof(E), UB = 4;
+  typedef E AV __attribute__((ext_vector_type(UB)));
   extern __shared__ __align__(16) unsigned char mmr_smem[];
   float* s_part = reinterpret_cast<float*>(mmr_smem);  // [wave][row][column of the workgroup]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lpr = 1 << lpr_log2, rpw = 64 >> lpr_log2, ncols = lpr * VE;
   const int col = (lane & (lpr - 1)) * VE, sub = lane >> lpr_log2;
-  const int n0 = (int)blockIdx.x * ncols + col;
-  const int kstep = MMR_WAVES * rpw;
-  constexpr int UB = 4;
-  for (int z = blockIdx.y; z < a.batch; z += gridDim.y) {
-    const E* A = reinterpret_cast<const E*>(a.A) + z * a.sA;
-    const E* B = reinterpret_cast<const E*>(a.B) + z * a.sB;
-    E* C = reinterpret_cast<E*>(a.C) + z * a.sC;
-    float acc[MR][VE];
+  const int b = xcd_run(blockIdx.x, gridDim.x), z = b / col_blocks, nb = (b - z * col_blocks) * ncols;
+  const int n0 = nb + col, nc = min(n0, a.N - VE);  // (N % VE == 0: a lane's columns are all inside or all outside)
+  const E* A = reinterpret_cast<const E*>(a.A) + z * a.sA;
+  const E* B = reinterpret_cast<const E*>(a.B) + z * a.sB + nc;
+  E* C = reinterpret_cast<E*>(a.C) + z * a.sC;
+  const E* Am[MR];
 #pragma unroll
-    for (int m = 0; m < MR; m++)
+  for (int m = 0; m < MR; m++) Am[m] = A + (int64_t)min(m, a.M - 1) * a.K;
+  float acc[MR][VE];
 #pragma unroll
-      for (int j = 0; j < VE; j++) acc[m][j] = 0.f;
-    for (int k0 = wave * rpw + sub; k0 < a.K; k0 += kstep * UB) {
-      u32x4 bv[UB];
-      E av[UB][MR];
+  for (int m = 0; m < MR; m++)
 #pragma unroll
-      for (int u = 0; u < UB; u++) {
-        const int k = k0 + u * kstep;
-        const bool ok = k < a.K && n0 < a.N;  // (N is a multiple of VE here: a lane's columns are all inside or all outside)
-        bv[u] = u32x4{0u, 0u, 0u, 0u};
-        if (ok) bv[u] = *reinterpret_cast<const u32x4*>(B + (int64_t)k * a.N + n0);
+    for (int j = 0; j < VE; j++) acc[m][j] = 0.f;
+  auto mac = [&](u32x4 bv, int m, E e) {
+    const float am = mm_to_f32<DT>(e);
 #pragma unroll
-        for (int m = 0; m < MR; m++) av[u][m] = (ok && m < a.M) ? A[(int64_t)m * a.K + k] : (E)0;
-      }
+    for (int j = 0; j < VE; j++) acc[m][j] = fmaf(am, mm_to_f32<DT>(MMTile<E, 64, true>::elem(bv, j)), acc[m][j]);
+  };
+  const int kstep = MMR_WAVES * rpw * UB;
+  int k = (wave * rpw + sub) * UB;
+#pragma unroll 2
+  for (; k + UB <= a.K; k += kstep) {
+    u32x4 bv[UB];
+    AV av[MR];
 #pragma unroll
-      for (int u = 0; u < UB; u++)
+    for (int u = 0; u < UB; u++) bv[u] = *reinterpret_cast<const u32x4*>(B + (int64_t)(k + u) * a.N);
 #pragma unroll
-        for (int m = 0; m < MR; m++) {
-          const float am = mm_to_f32<DT>(av[u][m]);
+    for (int m = 0; m < MR; m++) __builtin_memcpy(&av[m], Am[m] + k, sizeof(AV));
 #pragma unroll
-          for (int j = 0; j < VE; j++) acc[m][j] = fmaf(am, mm_to_f32<DT>(MMTile<E, 64, true>::elem(bv[u], j)), acc[m][j]);
-        }
+    for (int u = 0; u < UB; u++)
+#pragma unroll
+      for (int m = 0; m < MR; m++) mac(bv[u], m, av[m][u]);
+  }
+  for (; k < a.K; k++) {  // one lane group of one wave ends here at most
+    const u32x4 bv = *reinterpret_cast<const u32x4*>(B + (int64_t)k * a.N);
+#pragma unroll
+    for (int m = 0; m < MR; m++) mac(bv, m, Am[m][k]);
+    if (k + 1 == a.K) break;
+  }
+#pragma unroll
+  for (int m = 0; m < MR; m++)
+#pragma unroll
+    for (int j = 0; j < VE; j++) {
+      float v = acc[m][j];
+      for (int off = lpr; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
+      if (sub == 0) s_part[((size_t)wave * MR + m) * ncols + col + j] = v;
     }
+  __syncthreads();
+  for (int i = tid; i < MR * ncols; i += MMR_WAVES * 64) {
+    const int m = i / ncols, c = i - m * ncols, n = nb + c;
+    if (m < a.M && n < a.N) {
+      float f = 0.f;
 #pragma unroll
-    for (int m = 0; m < MR; m++)
-#pragma unroll
-      for (int j = 0; j < VE; j++) {
-        float v = acc[m][j];
-        for (int off = lpr; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
-        if (sub == 0) s_part[((size_t)wave * MR + m) * ncols + col + j] = v;
-      }
-    __syncthreads();
-    for (int i = tid; i < MR * ncols; i += MMR_WAVES * 64) {
-      const int m = i / ncols, c = i - m * ncols, n = (int)blockIdx.x * ncols + c;
-      if (m < a.M && n < a.N) {
-        float f = 0.f;
-#pragma unroll
-        for (int w = 0; w < MMR_WAVES; w++) f += s_part[((size_t)w * MR + m) * ncols + c];
-        if constexpr (DT == MLLM_HIP_F32) C[(int64_t)m * a.N + n] = f;
-        else if constexpr (DT == MLLM_HIP_BF16) C[(int64_t)m * a.N + n] = f32_to_bf16(f);
-        else C[(int64_t)m * a.N + n] = f32_to_f16bits(f);
-      }
+      for (int w = 0; w < MMR_WAVES; w++) f += s_part[((size_t)w * MR + m) * ncols + c];
+      if constexpr (DT == MLLM_HIP_F32) C[(int64_t)m * a.N + n] = f;
+      else if constexpr (DT == MLLM_HIP_BF16) C[(int64_t)m * a.N + n] = f32_to_bf16(f);
+      else C[(int64_t)m * a.N + n] = f32_to_f16bits(f);
     }
-    __syncthreads();
   }
 }
 // the launch shape of the kernel above; false where it does not apply (the tile kernel then)
@@ -294,13 +349,115 @@ static bool launch_matmul_rows(const MMArgs& a, hipStream_t st, int* rc) {
   const int mr = a.M <= 1 ? 1 : (a.M <= 2 ? 2 : 4);
   while (lg > 0 && (size_t)MMR_WAVES * mr * (VE << lg) * sizeof(float) > 64 * 1024) lg--;  // the waves' partial sums fit 64 KB of LDS
   const int ncols = VE << lg;
-  const dim3 grid((unsigned)((a.N + ncols - 1) / ncols), (unsigned)std::min(a.batch, 65535));
-  const size_t lds = (size_t)MMR_WAVES * 4 * ncols * sizeof(float);
-  if (a.M <= 1) hipLaunchKernelGGL((matmul_rows_kernel<DT, 1>), grid, dim3(MMR_WAVES * 64), lds / 4, st, a, lg);
-  else if (a.M <= 2) hipLaunchKernelGGL((matmul_rows_kernel<DT, 2>), grid, dim3(MMR_WAVES * 64), lds / 2, st, a, lg);
-  else hipLaunchKernelGGL((matmul_rows_kernel<DT, 4>), grid, dim3(MMR_WAVES * 64), lds, st, a, lg);
+  const int64_t cols = (a.N + ncols - 1) / ncols;
+  if (cols * a.batch > 0x7fffffff) return false;
+  const dim3 grid((unsigned)(cols * a.batch));
+  const size_t lds = (size_t)MMR_WAVES * mr * ncols * sizeof(float);
+  if (mr == 1) hipLaunchKernelGGL((matmul_rows_kernel<DT, 1>), grid, dim3(MMR_WAVES * 64), lds, st, a, lg, (int)cols);
+  else if (mr == 2) hipLaunchKernelGGL((matmul_rows_kernel<DT, 2>), grid, dim3(MMR_WAVES * 64), lds, st, a, lg, (int)cols);
+  else hipLaunchKernelGGL((matmul_rows_kernel<DT, 4>), grid, dim3(MMR_WAVES * 64), lds, st, a, lg, (int)cols);
   *rc = (int)hipGetLastError();
   return true;
+}
+
+// Up to four rows of A [M][K] against B [N][K] (a decode token's queries x keys): dot products, bound by reading B once.  The tile
+// kernel multiplies 64 rows for them, which in fp32 takes as long as the read.  A group of 2^g_log2 lanes holds 16-byte pieces of the
+// rows of A and takes UB rows of B, all requested before the first is multiplied; the lanes' sums meet through wave shuffles.
+// fp32: 8 x 4 x 8000 x 128 13.7 -> 9.8 us (3.3 TB/s), 8 x 1 x 8000 x 128 13.5 -> 5.5; bf16: 8 x 1 x 8000 x 128 5.6 -> 4.2.  1 x 1 x 64 x 2048 (router logits): fp32 52.6 -> 11.3,
+// bf16 21.8 -> 5.4.
+template <int DT, int MR, int UB>
+__global__ __launch_bounds__(256) void matmul_dots_kernel(MMArgs a, int g_log2, int col_blocks) {
+  using E = typename MMElem<DT>::type;
+  constexpr int VE = 16 / (int)sizeof(E);
+  __shared__ float s_out[MR][256 * UB / 4];  // at least four lanes per row of B
+  const int tid = threadIdx.x, g = 1 << g_log2, sub = tid & (g - 1), groups = 256 >> g_log2, grp = tid >> g_log2, per = groups * UB;
+  const int b = xcd_run(blockIdx.x, gridDim.x), z = b / col_blocks, n0 = (b - z * col_blocks) * per;
+  const E* A = reinterpret_cast<const E*>(a.A) + z * a.sA;
+  const E* B = reinterpret_cast<const E*>(a.B) + z * a.sB;
+  E* C = reinterpret_cast<E*>(a.C) + z * a.sC;
+  float acc[UB][MR];
+#pragma unroll
+  for (int u = 0; u < UB; u++)
+#pragma unroll
+    for (int m = 0; m < MR; m++) acc[u][m] = 0.f;
+#pragma unroll UB == 1 ? 4 : 1
+  for (int k = sub * VE; k < a.K; k += g * VE) {  // (K % VE == 0; once for rows of up to 64 pieces)
+    u32x4 av[MR], bv[UB];
+#pragma unroll
+    for (int m = 0; m < MR; m++) av[m] = *reinterpret_cast<const u32x4*>(A + (int64_t)min(m, a.M - 1) * a.K + k);
+#pragma unroll
+    for (int u = 0; u < UB; u++) bv[u] = *reinterpret_cast<const u32x4*>(B + (int64_t)min(n0 + grp + u * groups, a.N - 1) * a.K + k);
+#pragma unroll
+    for (int u = 0; u < UB; u++)
+#pragma unroll
+      for (int j = 0; j < VE; j++) {
+        const float bf = mm_to_f32<DT>(MMTile<E, 64, true>::elem(bv[u], j));
+#pragma unroll
+        for (int m = 0; m < MR; m++) acc[u][m] = fmaf(mm_to_f32<DT>(MMTile<E, 64, true>::elem(av[m], j)), bf, acc[u][m]);
+      }
+  }
+#pragma unroll
+  for (int u = 0; u < UB; u++)
+#pragma unroll
+    for (int m = 0; m < MR; m++) {
+      float v = acc[u][m];
+      v += dpp_f<0xB1>(v);  // (a group has four lanes or more)
+      v += dpp_f<0x4E>(v);
+      if (g > 4) v += dpp_f<0x141>(v);
+      if (g > 8) v += dpp_f<0x140>(v);
+      if (g > 16) v += __shfl_xor(v, 16, 64);
+      if (g > 32) v += __shfl_xor(v, 32, 64);
+      if (sub == 0) s_out[m][u * groups + grp] = v;
+    }
+  __syncthreads();
+  for (int i = tid; i < MR * per; i += 256) {
+    const int m = i / per, c = i - m * per;
+    if (m < a.M && n0 + c < a.N) {
+      const float f = s_out[m][c];
+      if constexpr (DT == MLLM_HIP_F32) C[(int64_t)m * a.N + n0 + c] = f;
+      else if constexpr (DT == MLLM_HIP_BF16) C[(int64_t)m * a.N + n0 + c] = f32_to_bf16(f);
+      else C[(int64_t)m * a.N + n0 + c] = f32_to_f16bits(f);
+    }
+  }
+}
+// the launch shape of the kernel above; false where it does not apply (the tile kernel then: 16-bit operands with three or four
+// short rows cost less there, 5.8 against 6.0 us at 8 x 4 x 8000 x 128; 1 x 4 x 64 x 2048: 18.7 / 6.0)
+template <int DT>
+static bool launch_matmul_dots(const MMArgs& a, hipStream_t st, int* rc) {
+  constexpr int VE = 16 / (int)sizeof(typename MMElem<DT>::type);
+  if (a.M > 4 || (a.M > 2 && DT != MLLM_HIP_F32 && a.K < 256) || !a.vecA || !a.vecB) return false;  // (aligned rows: K % VE == 0)
+  int lg = 2;
+  while (lg < 6 && (VE << lg) < a.K) lg++;
+  if (((int64_t)a.N + 3) / 4 * a.batch > 0x7fffffff) return false;  // (a workgroup takes four rows of B at least)
+  auto go = [&](auto kern, int ub) {
+    const int per = (256 >> lg) * ub;
+    const int64_t cols = ((int64_t)a.N + per - 1) / per;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(cols * a.batch)), dim3(256), 0, st, a, lg, (int)cols);
+    return (int)hipGetLastError();
+  };
+  // four rows of B per group where that leaves 128 workgroups or more, else one (8 x 4 x 8000 x 128 fp32: 9.8 us / 13.1; 2 x 4 x
+  // 777 x 128: 5.0 / 4.1)
+  const int64_t per4 = (256 >> lg) * 4;
+  if ((a.N + per4 - 1) / per4 * a.batch >= 128)
+    *rc = a.M <= 1 ? go(matmul_dots_kernel<DT, 1, 4>, 4) : a.M <= 2 ? go(matmul_dots_kernel<DT, 2, 4>, 4) : go(matmul_dots_kernel<DT, 4, 4>, 4);
+  else
+    *rc = a.M <= 1 ? go(matmul_dots_kernel<DT, 1, 1>, 1) : a.M <= 2 ? go(matmul_dots_kernel<DT, 2, 1>, 1) : go(matmul_dots_kernel<DT, 4, 1>, 1);
+  return true;
+}
+
+// The tile of 128 x 128 or of 64 x 64.  A wave of the larger one does four matrix instructions per pair of operand reads
+// instead of one per pair, but fewer workgroups fit a CU and the last round and the edges of the output stay emptier.
+//   fp32 (bound by the matrix pipe, two large tiles per CU at a time): rounds over the 256 CUs; 2048 x 4096 x 1000: 138 us large, 153
+//     small; 3000 x 3000 x 3000 (2.25 rounds): 604 / 527; K = 64 is mostly epilogue: 4 x 4000 x 1000 x 64: 34 / 31
+//   16 bits (bound by loads and LDS, more workgroups per CU hide them): us of a K of 2048 against tiles per CU, B [N][K]: 4096 x 4096 x 4096
+//     180 large, 298 small, 1000 x 3000 x 700: 24 / 20; where an operand is [K][rows] the large tile gains less (4096^3: 340 / 371)
+template <int DT, bool TA, bool TB>
+static bool matmul_large_tile(const MMArgs& a) {
+  const double large = (double)((a.M + 127) / 128) * ((a.N + 127) / 128) * a.batch / 256;
+  const double small = (double)((a.M + 63) / 64) * ((a.N + 63) / 64) * a.batch / 256;
+  if (DT == MLLM_HIP_F32) return a.K >= 128 && 4. * std::ceil(large) < 1.13 * std::ceil(small);
+  if (a.K < 256) return false;
+  return !TA && TB ? 30. + 17. * large < 9. + 9.3 * small : 40. + 36. * large < 11.7 * small;
 }
 
 template <int DT, bool TA, bool TB>
@@ -309,17 +466,27 @@ static int launch_matmul(const MMArgs& a, hipStream_t st) {
     int rc = 0;
     if (launch_matmul_rows<DT>(a, st, &rc)) return rc;
   }
-  // the small tile where the large one would leave most of the 256 CUs without a workgroup
-  const int64_t big = (int64_t)((a.M + 127) / 128) * ((a.N + 127) / 128) * a.batch;
-  const unsigned gz = (unsigned)std::min(a.batch, 65535);
-  if (big >= 256 && a.M > 64 && a.N > 64) {
-    hipLaunchKernelGGL((matmul_kernel<DT, TA, TB, 2, 2>), dim3((unsigned)((a.N + 127) / 128), (unsigned)((a.M + 127) / 128), gz),
-                       dim3(256), 0, st, a);
-  } else {
-    hipLaunchKernelGGL((matmul_kernel<DT, TA, TB, 1, 1>), dim3((unsigned)((a.N + 63) / 64), (unsigned)((a.M + 63) / 64), gz),
-                       dim3(256), 0, st, a);
+  if constexpr (!TA && TB) {
+    int rc = 0;
+    if (launch_matmul_dots<DT>(a, st, &rc)) return rc;
   }
-  return (int)hipGetLastError();
+  auto go = [&](auto kern, int side) {
+    const int64_t tiles = (int64_t)((a.M + side - 1) / side) * ((a.N + side - 1) / side);
+    if (tiles > 0x7fffffff) return MLLM_HIP_E_SHAPE;
+    const int most = (int)std::min<int64_t>(a.batch, 0x7fffffff / tiles);  // batch entries per launch
+    using E = typename MMElem<DT>::type;
+    for (int z = 0; z < a.batch; z += most) {
+      MMArgs p = a;
+      p.A = reinterpret_cast<const E*>(a.A) + z * a.sA;
+      p.B = reinterpret_cast<const E*>(a.B) + z * a.sB;
+      p.C = reinterpret_cast<E*>(a.C) + z * a.sC;
+      p.batch = std::min(most, a.batch - z);
+      hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * p.batch)), dim3(256), 0, st, p);
+    }
+    return (int)hipGetLastError();
+  };
+  if (matmul_large_tile<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 2, 2>, 128);
+  return go(matmul_kernel<DT, TA, TB, 1, 1>, 64);
 }
 
 template <int DT>

@@ -83,3 +83,26 @@ def test_matmul_16_bit(batch, M, N, K, ta, tb, dtype):
     assert rel_l2(c.float().numpy(), want.float().numpy()) <= 1e-3
     # and against the unrounded float64 result: no worse than one rounding of the result type
     assert rel_l2(c.float().numpy(), _ref(a.float().numpy(), b.float().numpy(), ta, tb)) <= (3e-3 if dtype == "bf16" else 4e-4)
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("batch,M,N,K,ta,tb", [
+    # either tile (the larger one from many tiles on), rows past the end repeated, K steps that end behind K, [K][rows] operands
+    # whose rows are or are not a multiple of a vector, fewer rows than a vector
+    (1, 2050, 2174, 257, False, True), (33, 513, 387, 290, False, False), (1, 2177, 2049, 288, True, True), (3, 65, 63, 33, False, False),
+    (2, 3, 2, 64, True, False), (2, 66, 68, 96, True, False), (2, 5, 3, 31, False, False), (1, 64, 7, 320, True, False),
+    # up to four rows: dot products (one and four rows of B per group, groups of 4 to 64 lanes, several pieces per lane), values
+    (1, 4, 5, 8, False, True), (1, 1, 63, 2056, False, True), (40, 4, 401, 128, False, True), (7, 2, 1030, 264, False, True),
+    (1, 3, 64, 2048, False, True), (9, 3, 520, 1027, False, False), (1, 4, 8, 259, False, False)])
+def test_matmul_forms_at_their_edges(batch, M, N, K, ta, tb, dtype):
+    """fp32: products of integers up to 8 and their sums (<= 64 K < 2^24) are exact, so the result is the integer product; 16 bits:
+    the same sums, rounded once to the result type"""
+    rng = synth.rng_for(6, 2000 + batch + M + N + K)
+    td = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    a = rng.integers(-8, 9, (batch, K, M) if ta else (batch, M, K)).astype(np.float32)
+    b = rng.integers(-8, 9, (batch, N, K) if tb else (batch, K, N)).astype(np.float32)
+    announce("matmul %s %s ta=%d tb=%d" % (dtype, (batch, M, N, K), ta, tb))
+    c = ql.matmul(torch.from_numpy(a).to(td).cuda(), torch.from_numpy(b).to(td).cuda(), ta, tb).cpu()
+    a, b = torch.from_numpy(a), torch.from_numpy(b)
+    want = torch.matmul(a.transpose(1, 2).contiguous() if ta else a, b.transpose(1, 2).contiguous() if tb else b).to(td)
+    assert torch.equal(c, want)
