@@ -377,7 +377,8 @@ int mllm_hip_moe_ffn_q(int wtype, const void* gate_packed, const void* up_packed
  * Qwen3-MoE recipe quantizes to; activations Q8_K in front of every projection): gate_packed / up_packed / down_packed are E
  * matrices packed by mllm_hip_kq_prepack back to back, mllm_hip_kq_packed_bytes(wtype, I, H) resp. (wtype, H, I) apart.
  * H % 256 == 0, I % 256 == 0, T * k <= 65535, E <= 3072.  Up to one (token, expert) pair per expert (Q6_K: half) every pair runs as one
- * GEMV row (three or four launches; the decode form, an expert's weights are read once per pair that uses it).  Beyond that
+ * GEMV row (three or four launches; the decode form, an expert's weights are read once per pair that uses it); from 16
+ * pairs on the workgroups of that form find the pairs that share an expert and take up to eight at once.  Beyond that
  * the pairs are sorted by expert and run as tiles of eight rows on the matrix cores (the grouped form: x and h quantized
  * to Q8_K once, an expert's weights read once per eight pairs; seven launches), same arithmetic; from four pairs per expert
  * on (Q4_K) as tiles of 32 rows, the weights as the second operand of 32 x 32 matrix instructions (an expert's weights read
@@ -431,34 +432,27 @@ int mllm_hip_kq_quantize_weight_blocks(int wtype, const float* w, void* blocks, 
                                        void* stream);
 /* y[M][N] fp32 = x[M][K] (fp32 or bf16) * W^T + bias.  K % 256 == 0.  Up to eight rows per launch (decode); more rows run
  * as groups of eight, each streaming the weights again.  workspace (mllm_hip_kq_workspace_bytes, may be NULL): from three
- * rows on x is quantized once by a small kernel and the GEMV copies that image instead of quantizing in every workgroup
- * (same results bit for bit). */
+ * rows on, where every workgroup would have more than a little to quantize, x is quantized once by a small kernel and the
+ * GEMV copies that image (same results bit for bit). */
 size_t mllm_hip_kq_workspace_bytes(int64_t M, int64_t K);
 /* Up to four Linears that share the activations and K in one launch (q/k/v, gate/up), as mllm_hip_linear_q_gemv_multi. */
 int mllm_hip_linear_kq_multi(int wtype, int nparts, const mllm_hip_gemv_part* parts, const void* x, int x_dtype, int64_t M, int64_t K,
                              void* workspace, void* stream);
-/* The same with the size of the workspace stated.  A workspace of mllm_hip_kq_workspace_bytes_n(M, K, N_total) bytes (N_total =
- * the sum of the parts' N) also has room for partial sums: launches of three to eight rows on the matrix-core kernels whose
- * rows have more than 2560 elements (Q6_K: more than 5120) then give every K slice a workgroup of its own, which quantizes
- * just its part of x (no separate quantization launch), and the slices meet in that room.  Same results bit for bit.  The arrival counters
- * belong to the workspace address as for mllm_hip_linear_q_gemv_multi: one launch at a time per workspace, and
- * mllm_hip_gemv_workspace_release before the memory is freed.  A smaller workspace (at least mllm_hip_kq_workspace_bytes)
- * is used as by mllm_hip_linear_kq_multi; less than that is MLLM_HIP_E_BADARG.
+/* The same with the size of the workspace stated: at least mllm_hip_kq_workspace_bytes, less is MLLM_HIP_E_BADARG.  (What
+ * mllm_hip_kq_workspace_bytes_n(M, K, N_total) asks for beyond that, N_total = the sum of the parts' N, is not needed by
+ * the present kernels: the K slices of a tile meet in LDS.)  One launch at a time per workspace.
  * replaces: the same call sites as mllm_hip_linear_kq (the workspace has no counterpart in the reference). */
 size_t mllm_hip_kq_workspace_bytes_n(int64_t M, int64_t K, int64_t N_total);
 int mllm_hip_linear_kq_multi_ws(int wtype, int nparts, const mllm_hip_gemv_part* parts, const void* x, int x_dtype, int64_t M, int64_t K,
                                 void* workspace, size_t workspace_bytes, void* stream);
-/* Comparison runs and tests: mode 0 keeps the K slices of every launch in one workgroup even where the workspace has room
- * for partial sums; -1 (the default) lets them meet in global memory where a row has at least four slices (more than
- * 2560 elements; Q6_K: eight slices, more than 5120 elements), 1 from two slices on; waves_per_wg = row tiles of a workgroup in that form (1..8, 0 = chosen per launch).
- * Same results bit for bit in every setting. */
+/* Checks its arguments (mode -1..1, waves_per_wg 0..8) and changes nothing: the form it chose, K slices that meet in the
+ * workspace, gave way to slices that meet in LDS.  Kept for callers that set it. */
 int mllm_hip_kq_set_slice_meeting(int mode, int waves_per_wg);
 /* Tuning override of the decode GEMV: lanes per weight row (8/16/32/64), waves per workgroup (1/2/4), units a lane keeps in
  * flight per row (1/2/4; more than one only for up to two activation rows); 0 = heuristic. */
 int mllm_hip_kq_set_tuning(int lanes_per_row, int waves_per_wg, int units_in_flight);
-/* Three to eight rows take their sub-block sums from the matrix cores as the Q4_0 kernel of that kind does (Q4_K always, Q6_K
- * with five to eight rows, and with three or four rows of more than 4096 elements, where it measured faster).  path = 1 keeps every launch on the dot4
- * kernel, 2 uses the matrix-core kernels wherever they fit (comparison runs, tests), 0 restores the default. */
+/* Three to eight rows take their sub-block sums from the matrix cores (rows of up to 15 872 elements).  path = 1 keeps
+ * every launch on the dot4 kernel; 0 and 2 are the default (comparison runs, tests). */
 int mllm_hip_kq_set_path(int path);
 int mllm_hip_linear_kq(int wtype, const void* packed, const void* x, int x_dtype, const float* bias, float* y, int64_t M, int64_t N,
                        int64_t K, void* workspace, void* stream);

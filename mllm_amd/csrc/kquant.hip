@@ -678,949 +678,14 @@ static int launch_kq(const KGemvArgs& a, hipStream_t st) {
 }
 
 
-// ---- Q4_K, three to eight rows: sub-block sums on the matrix cores ---------------------------------------------------------
-// The dot4 kernel above needs the activation codes of every row from LDS for every weight unit and is bound by those reads
-// from three rows on (17 us per 9728 x 2560 projection at eight rows against 7 at one).  Here v_mfma_i32_16x16x64_i8 makes
-// the sums of one 32-element sub-block, as in the Q4_0 kernel of this kind (qgemv_mfma.hip): the instruction sums over
-// K = 64, and the sums of different sub-blocks are kept apart by the activation operand.  A 16-byte record of the nibble
-// plane holds 16 elements of sub-block 2c (low nibbles) and the same 16 of sub-block 2c+1 (high nibbles); lane group g of
-// the weight operand holds record 4j + g of the lane's weight row, so the low-nibble instruction sees sub-block 4j in
-// groups 0,1 and sub-block 4j+2 in groups 2,3 (the high-nibble instruction 4j+1 and 4j+3).  Output column 8 q + t gets the
-// codes of (that sub-block, activation row t) in groups 2q, 2q+1 and zeros in the other two: one instruction = the sums of
-// two sub-blocks for eight rows, every lane of the result useful.
-// Scaling per lane (four consecutive weight rows of one activation row):
-//   acc = fma(fp32(d*sc) * dx, float(isum), acc);  acc = fma(-(fp32(dmin*m) * dx), float(sum of the row's 32 codes), acc)
-// the reference's sum (vec_dot_q4_K_q8_K: integer sums per super-block, then d*dx and dmin*dx) regrouped; the integer parts
-// are exact, the fp32 roundings differ in order only.
-// Order and batching of the requests in front of the loop (measured on the 4B layer shapes; the values compiled in are the
-// fastest): KMF_WEIGHTS_FIRST 1 asks for the slice's weights before the quantized image is copied -- the image, which every
-// wave needs before the first barrier, then comes back behind them (layer at eight rows 58.3 us against 54.2);
-// KMF_COPY_UNROLL = image pieces a thread requests before it stores the first (10: the down projection gets slower);
-// KMF_QUANT_BATCH = activation items a thread requests before it quantizes the first.
-#ifndef KMF_WEIGHTS_FIRST
-#define KMF_WEIGHTS_FIRST 0
-#endif
-#ifndef KMF_QUANT_BATCH
-#define KMF_QUANT_BATCH 4
-#endif
-#ifndef KMF_COPY_UNROLL
-#define KMF_COPY_UNROLL 5
-#endif
 typedef int kv4i __attribute__((ext_vector_type(4)));
-constexpr int KMF_NG = 10;  // groups of four sub-blocks per trip, at most (the launcher takes 6 or 8 for shorter slices)
+#include "kquant_rows.h"
 
-static int kmf_slices(int nb32) {
-  int s = 1;
-  while (s < 8 && nb32 > 40 * s) s *= 2;
-  return s;
-}
-
-// blockDim = nwaves * 64; a workgroup holds nwaves / S row tiles (16 weight rows), S K-slices each; nbs = sub-blocks per slice
-// (a multiple of 8: whole super-blocks).
-// LDS: xc [nb32 + xpad][MT] 32 bytes: the 32 codes of (sub-block, row); xs [nb32 + xpad][MT] {dx, sum of the 32 codes}
-//      (xpad = how far the last trip of the last slice reaches past the row: zeros); one zero record;
-//      ws per wave [whole trips][16 rows] fp32 d*sc, then the same of dmin*m (after the loop: the wave's four sums for the
-//      wave of slice 0).
-// NG = groups of four sub-blocks per trip: the slice in one trip where it fits (6, 8 or 10), so that neither registers nor
-// LDS rows are held for sub-blocks the slice does not have -- with K = 2048 three workgroups fit a CU instead of two.
-// K slices spread over workgroups (blockIdx.z = slice group): where they meet.  SG = 1: all slices of a tile in one workgroup.
-struct KMeet {
-  int SG;              // slice groups (= gridDim.z); a workgroup holds slices [z S, z S + S)
-  int lrows;           // sub-blocks a workgroup keeps in LDS: its slices' plus what their last trips reach past them
-  float* part;         // [x column of the grid][wave][slice group][32 lanes] four partial sums
-  unsigned* counters;  // one per x column (cstride counters apart), zero between launches
-  int cstride;
-};
-// host side: what a caller's workspace offers for it (key = the workspace address that owns the counter block)
-struct KMeetRoom {
-  const void* key;
-  void* part;
-  size_t part_bytes;
-};
-int gemv_counter_block(const void* workspace, hipStream_t st, unsigned** out);  // qgemv_mfma.hip
-constexpr int KQ_NOT_TAKEN = 1;  // a launcher's answer when the launch does not suit it (also gemv_counter_block's when no block is free)
-template <int XT, int MT, int NG = KMF_NG>
-__global__ __launch_bounds__(512) void kq4_gemv_mfma_kernel(KGemvArgs a, int S, int nbs, KMeet km) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int TRIP = 4 * NG;
-  const int nsb = a.nsb, nb32 = nsb * 8, K = nsb * QK_K;
-  const int tid = threadIdx.x, lane = tid & 63, nthreads = blockDim.x, nwaves = nthreads >> 6;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int pidx = 0;
-#pragma unroll
-  for (int p = 1; p < KQ_MAX_PARTS; p++)
-    if (p < a.nparts && (int)blockIdx.x >= a.wg_start[p]) pidx = p;
-  const KGemvPart& pt = a.part[pidx];
-  const KTile mt = kq_tile(a);
-  if (!mt.active) return;  // uniform, ahead of every barrier
-  const int N = pt.N;
-  const int tiles_wg = nwaves / S;
-  const int tile = ((int)blockIdx.x - a.wg_start[pidx]) * tiles_wg + wave / S;
-  const int sg = km.SG > 1 ? (int)blockIdx.z : 0;
-  const int slice = sg * S + wave % S;
-  const int row0 = tile * 16;
-  const bool tile_ok = row0 < N;
-  const int b0 = slice * nbs, b1 = min(nb32, b0 + nbs);
-  const int kb0 = min(nb32, sg * S * nbs), kb1 = min(nb32, kb0 + S * nbs);  // the workgroup's sub-blocks; LDS rows count from kb0
-  const int nloc = kb1 - kb0, lrows = km.lrows;
-
-  const int wsb = (nbs + TRIP - 1) / TRIP * TRIP;
-  u32x4* xc = reinterpret_cast<u32x4*>(smem);                        // [((sb - kb0) * MT + m) * 2 + half]
-  u32x4* zrec = xc + (size_t)lrows * MT * 2;
-  u32x2* xs = reinterpret_cast<u32x2*>(zrec + 1);                    // [(sb - kb0) * MT + m]
-  float* ws_all = reinterpret_cast<float*>(xs + (size_t)lrows * MT);
-  float* ws_ds = ws_all + (size_t)wave * 2 * wsb * 16;
-  float* ws_dm = ws_ds + (size_t)wsb * 16;
-  f32x4* red = reinterpret_cast<f32x4*>(ws_ds);  // the wave's scale table, dead after the loop (2 wsb x 64 bytes >= 1 KB)
-  int* s_flag = reinterpret_cast<int*>(ws_all + (size_t)nwaves * 2 * wsb * 16);
-
-  // ---- 1. weight scale records of the tile and slice: one 16-byte record per (row, super-block) --------------------------
-  const uint32_t sbt = (uint32_t)N * (uint32_t)nsb;
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(kq_at(pt.w.a, mt.eoff)), 0, sbt * 128u, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsc = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(kq_at(pt.w.s, mt.eoff)), 0, sbt * 16u, 0x00020000);
-  const int spb = nbs >> 3;  // super-blocks per slice (at most 8)
-  const __amdgpu_buffer_rsrc_t rdd = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kq_at(pt.w.d, mt.eoff)), 0, sbt * 4u, 0x00020000);
-  u32x4 sc[2];
-  uint32_t scd[2];
-#pragma unroll
-  for (int k = 0; k < 2; k++) {
-    const int ch = lane + 64 * k;
-    const int r = ch / spb, si = ch - r * spb;
-    const int sb256 = (b0 >> 3) + si;
-    const bool ok = tile_ok && r < 16 && row0 + r < N && sb256 < nsb;
-    const uint32_t rec = (uint32_t)(row0 + r) * (uint32_t)nsb + (uint32_t)sb256;
-    sc[k] = __builtin_amdgcn_raw_buffer_load_b128(rsc, ok ? rec * 16u : KBUF_OOB, 0, KBUF_NT);
-    scd[k] = __builtin_amdgcn_raw_buffer_load_b32(rdd, ok ? rec * 4u : KBUF_OOB, 0, KBUF_NT);
-  }
-  // ---- 2. weight codes: lane (row c, group g) takes records b0 + 4 j + g ------------------------------------------------------
-  const int c = lane & 15, g = lane >> 4;
-  const bool row_ok = tile_ok && row0 + c < N;
-  const uint32_t rbase = (uint32_t)(row0 + c) * (uint32_t)nb32;
-  u32x4 wq[NG];
-  auto load_groups = [&](int bb) {
-#pragma unroll
-    for (int j = 0; j < NG; j++) {
-      const int b = bb + 4 * j + g;
-      wq[j] = __builtin_amdgcn_raw_buffer_load_b128(ra, (row_ok && b < b1) ? (rbase + (uint32_t)b) * 16u : KBUF_OOB, 0, KBUF_NT);
-    }
-  };
-  if (KMF_WEIGHTS_FIRST && XT == KQ_IMAGE) load_groups(b0);
-  __asm__ volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-
-  // ---- 3. activations into LDS -------------------------------------------------------------------------------------------------
-  if (XT == KQ_IMAGE) {  // codes [R][K], sums of 16 as int16 [R][K/16], scales [R][nsb]; R = MT, or the rows of a MoE image
-    const size_t R = a.img_rows ? (size_t)a.img_rows : (size_t)MT;
-    const u32x4* codes = reinterpret_cast<const u32x4*>(a.x);
-    const uint32_t* pairs = reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(a.x) + R * K);
-    const float* dd = reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.x) + R * K + R * nsb * 32);
-    // Thread (row m = tid % MT, piece tid / MT): a wave reads 128 contiguous bytes of each of its rows and writes 1 KB of
-    // contiguous LDS.  The pieces of a batch are all requested before the first is stored, and the sums and scales before
-    // the codes: one round trip to memory per batch, where a copy row by row and pass by pass took one per pass.
-    const int m = tid & (MT - 1), p0 = tid / MT, pstep = nthreads / MT;
-    const size_t src = (size_t)kq_tile_in_row(a, mt, m);
-    constexpr int CS = 3;
-    uint32_t pr[CS];
-    float dv[CS];
-#pragma unroll
-    for (int u = 0; u < CS; u++) {
-      const int sb = p0 + u * pstep;
-      if (sb < nloc) {
-        pr[u] = pairs[src * nb32 + kb0 + sb];
-        dv[u] = dd[src * nsb + ((kb0 + sb) >> 3)];
-      }
-    }
-    for (int r0 = p0; r0 < 2 * nloc; r0 += pstep * KMF_COPY_UNROLL) {
-      u32x4 cv[KMF_COPY_UNROLL];
-#pragma unroll
-      for (int u = 0; u < KMF_COPY_UNROLL; u++) {
-        const int r = r0 + u * pstep;
-        if (r < 2 * nloc) cv[u] = codes[(src * nb32 + kb0) * 2 + r];
-      }
-#pragma unroll
-      for (int u = 0; u < KMF_COPY_UNROLL; u++) {
-        const int r = r0 + u * pstep;
-        if (r < 2 * nloc) xc[((size_t)(r >> 1) * MT + m) * 2 + (r & 1)] = cv[u];
-      }
-    }
-    auto put_sums = [&](int sb, uint32_t pair, float d) {
-      const int bsum = (int)(int16_t)(pair & 0xffffu) + (int)(int16_t)(pair >> 16);
-      xs[(size_t)sb * MT + m] = u32x2{__float_as_uint(d), (uint32_t)bsum};
-    };
-#pragma unroll
-    for (int u = 0; u < CS; u++)
-      if (p0 + u * pstep < nloc) put_sums(p0 + u * pstep, pr[u], dv[u]);
-    for (int sb = p0 + CS * pstep; sb < nloc; sb += pstep) put_sums(sb, pairs[src * nb32 + kb0 + sb], dd[src * nsb + ((kb0 + sb) >> 3)]);
-  } else {
-    const int ipr = K >> 3;     // items (eight elements) per row; 32 consecutive items = one super-block
-    const int iwg = nloc << 2;  // of them in this workgroup's sub-blocks (whole super-blocks)
-    const int nitems = MT * iwg;
-    const float inv_iwg = 1.0f / (float)iwg;
-    // (the items of a batch are all requested before the first is quantized: one round trip to memory per batch)
-    constexpr int QI = KMF_QUANT_BATCH;
-    for (int it0 = tid; it0 < nitems; it0 += nthreads * QI) {  // whole half-waves: nitems and nthreads are multiples of 32
-      float v[QI][8];
-#pragma unroll
-      for (int u = 0; u < QI; u++) {
-        const int it = it0 + u * nthreads;
-        const int m = (int)(((float)it + 0.5f) * inv_iwg), i = it - m * iwg;  // it / iwg: far from rounding trouble
-#pragma unroll
-        for (int e = 0; e < 8; e++) v[u][e] = 0.f;
-        if (it < nitems && m < a.M) load8<XT == KQ_IMAGE ? MLLM_HIP_F32 : XT>(a.x, ((int64_t)m * ipr + 4 * kb0 + i) * 8, v[u]);
-      }
-      if (it0 == tid) load_groups(b0);  // the weights right behind the first batch: they arrive while it is quantized
-#pragma unroll
-      for (int u = 0; u < QI; u++) {
-        const int it = it0 + u * nthreads;
-        if (it >= nitems) break;
-        const int m = (int)(((float)it + 0.5f) * inv_iwg), i = it - m * iwg;
-        const Q8KItem qi = quantize_q8k_item(v[u], lane);
-        int s32 = qi.sum8 + __builtin_amdgcn_update_dpp(0, qi.sum8, 0xB1, 0xf, 0xf, true);
-        s32 += __builtin_amdgcn_update_dpp(0, s32, 0x4E, 0xf, 0xf, true);
-        const int sb = i >> 2, part = i & 3;  // sub-block (from kb0), which 8 of its 32 codes
-        reinterpret_cast<u32x2*>(xc + ((size_t)sb * MT + m) * 2 + (part >> 1))[part & 1] = u32x2{qi.q0, qi.q1};
-        if (part == 0) xs[(size_t)sb * MT + m] = u32x2{__float_as_uint(qi.d), (uint32_t)s32};
-      }
-    }
-  }
-  if (!KMF_WEIGHTS_FIRST && XT == KQ_IMAGE) load_groups(b0);
-  if (XT != KQ_IMAGE && tid >= (nloc << 2) * MT) load_groups(b0);  // (threads without an item to quantize)
-  if (tid == 0) zrec[0] = u32x4{0u, 0u, 0u, 0u};
-  for (int i = tid; i < (lrows - nloc) * MT * 2; i += nthreads) xc[(size_t)nloc * MT * 2 + i] = u32x4{0u, 0u, 0u, 0u};
-  for (int i = tid; i < (lrows - nloc) * MT; i += nthreads) xs[(size_t)nloc * MT + i] = u32x2{0u, 0u};
-  // weight scales: fp32 d*sc and dmin*m per (sub-block of the slice, row); zero past the row and in the rest of the last trip
-#pragma unroll
-  for (int k = 0; k < 2; k++) {
-    const int ch = lane + 64 * k;
-    const int r = ch / spb, si = ch - r * spb;
-    if (r < 16) {
-      const bool in = (b0 >> 3) + si < nsb;
-      const float d = f16bits_to_f32((uint16_t)(scd[k] & 0xffffu)), dmin = f16bits_to_f32((uint16_t)(scd[k] >> 16));
-      const uint32_t rec[4] = {sc[k].x, sc[k].y, sc[k].z, sc[k].w};  // per pair of sub-blocks {sc, sc, m, m}
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        ws_ds[(8 * si + j) * 16 + r] = in ? d * (float)((rec[j >> 1] >> (8 * (j & 1))) & 0xffu) : 0.f;
-        ws_dm[(8 * si + j) * 16 + r] = in ? dmin * (float)((rec[j >> 1] >> (16 + 8 * (j & 1))) & 0xffu) : 0.f;
-      }
-    }
-  }
-  for (int i = nbs * 16 + lane; i < wsb * 16; i += 64) {
-    ws_ds[i] = 0.f;
-    ws_dm[i] = 0.f;
-  }
-  __syncthreads();
-
-  // ---- 4. sub-block sums on the matrix cores, scaling on the vector ALU (software-pipelined over groups of four) --------------
-  const int q2 = (lane & 15) >> 3, t = lane & 7, tm = t & (MT - 1);
-  const bool mine = (g >> 1) == q2;  // the lane groups that supply this column's codes
-  const int half = g & 1;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int bb = b0; bb < b1; bb += TRIP) {
-    if (bb != b0) load_groups(bb);
-    const u32x4* bl = mine ? xc + ((size_t)(bb - kb0 + 2 * q2) * MT + tm) * 2 + half : zrec;
-    const int bstep = mine ? 8 * MT : 0;  // four sub-blocks further per group
-    const u32x2* xsl = xs + (size_t)(bb - kb0 + 2 * q2) * MT + tm;
-    const float* dsl = ws_ds + (bb - b0 + 2 * q2) * 16 + 4 * g;
-    const float* dml = ws_dm + (bb - b0 + 2 * q2) * 16 + 4 * g;
-    u32x4 Bl[2], Bh[2];
-    u32x2 sx[2][2];
-    f32x4 ds[2][2], dm[2][2];
-    kv4i D[2][2];
-    auto fetch_b = [&](int set, int j) {
-      Bl[set] = bl[j * bstep];
-      Bh[set] = bl[j * bstep + (mine ? 2 * MT : 0)];
-    };
-    auto fetch_s = [&](int set, int j) {
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        sx[set][h] = xsl[(4 * j + h) * MT];
-        ds[set][h] = *reinterpret_cast<const f32x4*>(dsl + (4 * j + h) * 16);
-        dm[set][h] = *reinterpret_cast<const f32x4*>(dml + (4 * j + h) * 16);
-      }
-    };
-    auto issue = [&](int set, int j) {
-      const u32x4 w = wq[j];
-      const kv4i Al = {(int)(w.x & 0x0f0f0f0fu), (int)(w.y & 0x0f0f0f0fu), (int)(w.z & 0x0f0f0f0fu), (int)(w.w & 0x0f0f0f0fu)};
-      const kv4i Ah = {(int)((w.x >> 4) & 0x0f0f0f0fu), (int)((w.y >> 4) & 0x0f0f0f0fu), (int)((w.z >> 4) & 0x0f0f0f0fu),
-                       (int)((w.w >> 4) & 0x0f0f0f0fu)};
-      D[set][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(Al, __builtin_bit_cast(kv4i, Bl[set]), kv4i{0, 0, 0, 0}, 0, 0, 0);
-      D[set][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(Ah, __builtin_bit_cast(kv4i, Bh[set]), kv4i{0, 0, 0, 0}, 0, 0, 0);
-    };
-    auto scale = [&](int set, int j) {
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        const bool live = bb + 4 * j + 2 * q2 + h < b1;
-        const float dx = live ? __uint_as_float(sx[set][h].x) : 0.f;
-        const float bs = (float)(int)sx[set][h].y;
-        acc.x = fmaf(ds[set][h].x * dx, (float)D[set][h].x, acc.x);
-        acc.y = fmaf(ds[set][h].y * dx, (float)D[set][h].y, acc.y);
-        acc.z = fmaf(ds[set][h].z * dx, (float)D[set][h].z, acc.z);
-        acc.w = fmaf(ds[set][h].w * dx, (float)D[set][h].w, acc.w);
-        acc.x = fmaf(-(dm[set][h].x * dx), bs, acc.x);
-        acc.y = fmaf(-(dm[set][h].y * dx), bs, acc.y);
-        acc.z = fmaf(-(dm[set][h].z * dx), bs, acc.z);
-        acc.w = fmaf(-(dm[set][h].w * dx), bs, acc.w);
-      }
-    };
-    fetch_b(0, 0);
-#pragma unroll
-    for (int j = 0; j < NG; j++) {
-      issue(j & 1, j);
-      if (j + 1 < NG) fetch_b((j + 1) & 1, j + 1);
-      fetch_s(j & 1, j);
-      __builtin_amdgcn_sched_barrier(0);
-      if (j > 0) scale((j - 1) & 1, j - 1);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    scale((NG - 1) & 1, NG - 1);
-  }
-  {  // the two lanes of an activation row (sub-blocks = 0,1 and 2,3 mod 4)
-    acc.x += __shfl_xor(acc.x, 8, 64);
-    acc.y += __shfl_xor(acc.y, 8, 64);
-    acc.z += __shfl_xor(acc.z, 8, 64);
-    acc.w += __shfl_xor(acc.w, 8, 64);
-  }
-
-  // ---- 5. slices of a tile in slice order, bias ------------------------------------------------------------------------------
-  if (S > 1) {
-    red[lane] = acc;
-    __syncthreads();
-    if (wave % S != 0) return;
-    for (int s = 1; s < S; s++) {
-      const f32x4 o = reinterpret_cast<const f32x4*>(ws_ds + (size_t)s * 2 * wsb * 16)[lane];  // the table of wave + s
-      acc.x += o.x; acc.y += o.y; acc.z += o.z; acc.w += o.w;
-    }
-  }
-  if (km.SG > 1) {
-    // The slice groups of a grid column meet in global memory (S = 1 here: every wave is a tile).  Ordering, step by step:
-    // partial sums leave with device-scope stores; every wave waits until the memory system has acknowledged its stores
-    // (s_waitcnt vmcnt(0): stores count in vmcnt until acknowledged); the workgroup barrier; thread 0 counts the workgroup
-    // in with a device-scope atomic add; the workgroup that sees the last count reads all partial sums with device-scope
-    // loads issued after a second barrier, and adds them in slice order: the bits of the one-workgroup form.
-    const int SG = km.SG;
-    const int li = 8 * g + t;
-    float* pbase = km.part + (((size_t)blockIdx.x * nwaves + wave) * SG) * 128;
-    if (q2 == 0) {
-      float* dst = pbase + (size_t)sg * 128 + 4 * li;
-      __hip_atomic_store(dst + 0, acc.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(dst + 1, acc.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(dst + 2, acc.z, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(dst + 3, acc.w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (tid == 0) {
-      unsigned* cnt = km.counters + (size_t)blockIdx.x * km.cstride;
-      const unsigned old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const int last = old == (unsigned)(SG - 1);
-      if (last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
-      *s_flag = last;
-    }
-    __syncthreads();
-    if (!*s_flag) return;
-    if (q2 == 0) {  // (at most eight slice groups; their loads are in flight together)
-      float pv[8][4];
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const float* src = pbase + (size_t)min(u, SG - 1) * 128 + 4 * li;
-#pragma unroll
-        for (int e = 0; e < 4; e++) pv[u][e] = __hip_atomic_load(src + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      acc = f32x4{pv[0][0], pv[0][1], pv[0][2], pv[0][3]};
-#pragma unroll
-      for (int u = 1; u < 8; u++)
-        if (u < SG) { acc.x += pv[u][0]; acc.y += pv[u][1]; acc.z += pv[u][2]; acc.w += pv[u][3]; }
-    }
-  }
-  if (!tile_ok || q2 != 0 || t >= MT || t >= mt.rows) return;
-  const int n = row0 + 4 * g;
-  const float v[4] = {acc.x, acc.y, acc.z, acc.w};
-  float* yrow = pt.y + (int64_t)kq_tile_out_row(a, mt, t) * N;
-#pragma unroll
-  for (int e = 0; e < 4; e++)
-    if (n + e < N) yrow[n + e] = pt.bias ? v[e] + pt.bias[n + e] : v[e];
-}
-
-static int kmf_groups(int nbs) { return nbs <= 24 ? 6 : (nbs <= 32 ? 8 : KMF_NG); }
-// how far the last trip of a slice reads past the row's nb32 sub-blocks (whole trips from the slice's first sub-block)
-static int kmf_xpad(int nb32, int S, int nbs) {
-  const int trip = 4 * kmf_groups(nbs);
-  int pad = 0;
-  for (int s = 0; s < S; s++) {
-    const int b0 = s * nbs, b1 = std::min(nb32, b0 + nbs);
-    if (b1 > b0) pad = std::max(pad, b0 + ((b1 - b0 - 1) / trip + 1) * trip - nb32);
-  }
-  return pad;
-}
-template <int MT>
-static size_t kmf_lds_bytes(int nb32, int nbs, int nwaves, int S) {
-  const int trip = 4 * kmf_groups(nbs);
-  const int wsb = (nbs + trip - 1) / trip * trip, rows = nb32 + kmf_xpad(nb32, S, nbs);
-  return (size_t)rows * MT * 32 + 16 + (size_t)rows * MT * 8 + (size_t)nwaves * 2 * wsb * 64 + 16;
-}
-// the same with one slice per workgroup (slice groups over the grid's z): the slice's sub-blocks in whole trips
-template <int MT>
-static size_t kmf_lds_bytes_z(int nbs, int nwaves) {
-  const int trip = 4 * kmf_groups(nbs);
-  const int wsb = (nbs + trip - 1) / trip * trip;
-  return (size_t)wsb * MT * 32 + 16 + (size_t)wsb * MT * 8 + (size_t)nwaves * 2 * wsb * 64 + 16;
-}
-static bool kq4_mfma_fits(int MT, int nsb) {
-  const int nb32 = nsb * 8;
-  if (nb32 > 512) return false;  // scale records: at most 128 per wave
-  const int S = kmf_slices(nb32);
-  const int nbs = ((nb32 + S - 1) / S + 7) / 8 * 8;
-  return (MT == 4 ? kmf_lds_bytes<4>(nb32, nbs, 8, S) : kmf_lds_bytes<8>(nb32, nbs, 8, S)) <= 160 * 1024;
-}
-// room for the partial sums of a launch whose slices meet in global memory (0: its slices share a workgroup anyway)
-static size_t kmf_part_bytes(int nsb, int64_t n_total, int nparts) {
-  const int S = std::max(kmf_slices(nsb * 8), nsb > 5 ? (nsb > 10 ? (nsb > 20 ? 8 : 4) : 2) : 1);  // (Q4_K's slices, Q6_K's: k6mf_split)
-  if (S < 2) return 0;
-  return (size_t)((n_total + 15) / 16 + (int64_t)nparts * 8) * S * 512;
-}
-int g_kq_meet = -1, g_kq_meet_waves = 0, g_kq_meet_min = 4;  // (mllm_hip_kq_set_slice_meeting)
-// row tiles (= waves) per workgroup of a launch whose K slices meet in memory: four to six, the first that needs the fewest
-// rounds of 256 workgroups (measured with Q4_K on 2560 x 9728 with eight slices: 12.6 / 11.4 / 12.4 us with four / five /
-// six at four rows, five = exactly 256 workgroups; 2560 x 4096 with four slices: 8.8 / 8.9 / 9.8, and 9.2 with three)
-static int kq_meet_waves(const KGemvArgs& a, int SG) {
-  int nwaves = g_kq_meet_waves;
-  if (!nwaves) {
-    int64_t best = 0;
-    for (int nw = 4; nw <= 6; nw++) {
-      int64_t wgs = 0;
-      for (int p = 0; p < a.nparts; p++) wgs += ((a.part[p].N + 15) / 16 + nw - 1) / nw;
-      const int64_t rounds = (wgs * SG + 255) / 256;
-      if (!best || rounds < best) {
-        best = rounds;
-        nwaves = nw;
-      }
-    }
-  }
-  return nwaves;
-}
-template <int XT, int MT>
-static int launch_kq4_mfma_z(const KGemvArgs& a_in, const KMeetRoom& room, hipStream_t st) {
-  KGemvArgs a = a_in;
-  const int nb32 = a.nsb * 8;
-  const int SG = kmf_slices(nb32);
-  const int nbs = ((nb32 + SG - 1) / SG + 7) / 8 * 8;
-  const int nwaves = kq_meet_waves(a, SG);
-  unsigned grid = 0;
-  for (int p = 0; p < a.nparts; p++) {
-    a.wg_start[p] = (int)grid;
-    grid += (unsigned)(((a.part[p].N + 15) / 16 + nwaves - 1) / nwaves);
-  }
-  a.wg_start[a.nparts] = (int)grid;
-  if (SG < 2 || g_kq_meet == 0 || !room.part || (size_t)grid * nwaves * SG * 512 > room.part_bytes || grid > 1024u) return KQ_NOT_TAKEN;
-  KMeet km{};
-  km.SG = SG;
-  const int trip = 4 * kmf_groups(nbs);
-  km.lrows = (nbs + trip - 1) / trip * trip;
-  km.part = static_cast<float*>(room.part);
-  RC_RET(gemv_counter_block(room.key, st, &km.counters));
-  km.cstride = 1;
-  while (km.cstride < 32 && (size_t)grid * km.cstride * 2 <= 1024u) km.cstride *= 2;
-  const size_t lds = kmf_lds_bytes_z<MT>(nbs, nwaves);
-  auto go = [&](auto kern) {
-    if (lds > 64 * 1024)
-      HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, dim3(grid, 1, (unsigned)SG), dim3(nwaves * 64), lds, st, a, 1, nbs, km);
-    return (int)hipGetLastError();
-  };
-  switch (kmf_groups(nbs)) {
-    case 6: return go(kq4_gemv_mfma_kernel<XT, MT, 6>);
-    case 8: return go(kq4_gemv_mfma_kernel<XT, MT, 8>);
-    default: return go(kq4_gemv_mfma_kernel<XT, MT, KMF_NG>);
-  }
-}
-template <int XT, int MT>
-static int launch_kq4_mfma_t(const KGemvArgs& a_in, hipStream_t st, unsigned grid_y = 1) {
-  KGemvArgs a = a_in;
-  const int nb32 = a.nsb * 8;
-  const int S = kmf_slices(nb32);
-  const int nbs = ((nb32 + S - 1) / S + 7) / 8 * 8;
-  // (MoE row tiles, grid_y > 1: the tile's eight image rows are staged once per workgroup; eight waves = 64 weight rows per
-  // staging instead of 32: Q4_K 512 tokens 491 -> 458 us.  The Q6_K kernel, with two waves per SIMD, loses with eight: 780 -> 915)
-  int nwaves = XT == KQ_IMAGE ? (grid_y > 1 ? (g_kq_NW ? g_kq_NW : 8) : 4) : 8;
-  if (nwaves < S) nwaves = S;
-  const int tiles_wg = nwaves / S;
-  unsigned grid = 0;
-  for (int p = 0; p < a.nparts; p++) {
-    a.wg_start[p] = (int)grid;
-    grid += (unsigned)(((a.part[p].N + 15) / 16 + tiles_wg - 1) / tiles_wg);
-  }
-  a.wg_start[a.nparts] = (int)grid;
-  const size_t lds = kmf_lds_bytes<MT>(nb32, nbs, nwaves, S);
-  if (lds > 160 * 1024) return MLLM_HIP_E_SHAPE;
-  KMeet km{};
-  km.SG = 1;
-  km.lrows = nb32 + kmf_xpad(nb32, S, nbs);
-  auto go = [&](auto kern) {
-    if (lds > 64 * 1024)
-      HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, dim3(grid, grid_y), dim3(nwaves * 64), lds, st, a, S, nbs, km);
-    return (int)hipGetLastError();
-  };
-  switch (kmf_groups(nbs)) {
-    case 6: return go(kq4_gemv_mfma_kernel<XT, MT, 6>);
-    case 8: return go(kq4_gemv_mfma_kernel<XT, MT, 8>);
-    default: return go(kq4_gemv_mfma_kernel<XT, MT, KMF_NG>);
-  }
-}
-template <int XT>
-static int launch_kq4_mfma(const KGemvArgs& a, hipStream_t st) {
-  return a.M <= 4 ? launch_kq4_mfma_t<XT, 4>(a, st) : launch_kq4_mfma_t<XT, 8>(a, st);
-}
-// ---- Q6_K, three to eight rows: the same on 16-element units -------------------------------------------------------------------
-// Q6_K scales 16 elements at a time, which is exactly what one lane supplies to the K = 64 instruction: lane group g of the
-// weight operand holds one 16-element unit, and output column 4 q + t gets the codes of (unit q of the four, activation row
-// t) in lane group q and zeros elsewhere: one instruction = the sums of four units for four rows.  A 16-byte record of the
-// low-nibble plane serves two units (low and high nibbles) with the matching 16 bytes of the bit-pair plane; the codes stay
-// unsigned (0..63) and the offset of 32 goes into the sum as -32 * (sum of the unit's 16 activation codes), which the Q8_K
-// quantization delivers anyway.  Scaling per lane: acc = fma(fp32(d * sc) * dx, float(isum - 32 * bsum), acc).
-// Step st of a trip = half a super-block (records 4 (st & 1) + g of super-block st / 2): low nibbles are units 8 (st & 1) + g,
-// high nibbles units 8 (st & 1) + 4 + g.
-constexpr int K6_ST = 10;  // steps per trip, at most: five super-blocks (the launcher takes fewer for shorter slices)
-// ST = steps per trip: the slice in one trip where it fits (6, 8 or 10); xpad = super-blocks the last trip of a slice reaches
-// past the row (zeros in LDS)
-template <int XT, int MT, int ST = K6_ST>
-__global__ __launch_bounds__(512) void kq6_gemv_mfma_kernel(KGemvArgs a, int S, int sps, KMeet km) {  // sps = super-blocks per slice; km.lrows in super-blocks
-  extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int TH = MT / 4;
-  constexpr int TSB = ST / 2;  // super-blocks per trip
-  const int nsb = a.nsb, nu = nsb * 16, K = nsb * QK_K;
-  const int tid = threadIdx.x, lane = tid & 63, nthreads = blockDim.x, nwaves = nthreads >> 6;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int pidx = 0;
-#pragma unroll
-  for (int p = 1; p < KQ_MAX_PARTS; p++)
-    if (p < a.nparts && (int)blockIdx.x >= a.wg_start[p]) pidx = p;
-  const KGemvPart& pt = a.part[pidx];
-  const KTile mt = kq_tile(a);
-  if (!mt.active) return;  // uniform, ahead of every barrier
-  const int N = pt.N;
-  const int tiles_wg = nwaves / S;
-  const int tile = ((int)blockIdx.x - a.wg_start[pidx]) * tiles_wg + wave / S;
-  const int sg = km.SG > 1 ? (int)blockIdx.z : 0;  // slice group: the workgroup's slices are [sg S, sg S + S)
-  const int slice = sg * S + wave % S;
-  const int row0 = tile * 16;
-  const bool tile_ok = row0 < N;
-  const int s0 = slice * sps, s1 = min(nsb, s0 + sps);  // this wave's super-blocks
-  const int ks0 = min(nsb, sg * S * sps), ks1 = min(nsb, ks0 + S * sps);  // the workgroup's; LDS rows count from ks0
-  const int nloc = ks1 - ks0, lsb = km.lrows, nul = nloc * 16;
-
-  const int wsu = (sps + TSB - 1) / TSB * TSB * 16;  // units of weight scales per wave: whole trips
-  u32x4* xc = reinterpret_cast<u32x4*>(smem);                     // [(unit - 16 ks0) * MT + m] the unit's 16 codes
-  u32x4* zrec = xc + (size_t)lsb * 16 * MT;
-  int* bs16 = reinterpret_cast<int*>(zrec + 1);                   // [(unit - 16 ks0) * MT + m] sum of the unit's codes
-  float* dxs = reinterpret_cast<float*>(bs16 + (size_t)lsb * 16 * MT);  // [(super-block - ks0) * MT + m]
-  float* ws_all = dxs + (size_t)lsb * MT;
-  float* ws = ws_all + (size_t)wave * wsu * 16;
-  int* s_flag = reinterpret_cast<int*>(ws_all + (size_t)nwaves * wsu * 16);
-  f32x4* red = reinterpret_cast<f32x4*>(smem) + (size_t)wave * TH * 64;  // takes the place of the codes once every wave is done with them
-
-  const uint32_t sbt = (uint32_t)N * (uint32_t)nsb;
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(kq_at(pt.w.a, mt.eoff)), 0, sbt * 128u, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(kq_at(pt.w.h, mt.eoff)), 0, sbt * 64u, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsc = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(kq_at(pt.w.s, mt.eoff)), 0, sbt * 16u, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kq_at(pt.w.d, mt.eoff)), 0, sbt * 2u, 0x00020000);
-  // ---- 1. weight scales of the tile and slice: 16 int8 and one fp16 per (row, super-block) -------------------------------------
-  u32x4 sc[2];
-  uint16_t scd[2];
-#pragma unroll
-  for (int k = 0; k < 2; k++) {
-    const int ch = lane + 64 * k;
-    const int r = ch / sps, si = ch - r * sps;
-    const bool ok = tile_ok && r < 16 && row0 + r < N && s0 + si < nsb;
-    const uint32_t idx = (uint32_t)(row0 + r) * (uint32_t)nsb + (uint32_t)(s0 + si);
-    sc[k] = __builtin_amdgcn_raw_buffer_load_b128(rsc, ok ? idx * 16u : KBUF_OOB, 0, KBUF_NT);
-    scd[k] = __builtin_amdgcn_raw_buffer_load_b16(rd, ok ? idx * 2u : KBUF_OOB, 0, KBUF_NT);
-  }
-  // ---- 2. weight codes: lane (row c, group g), step st: low-nibble record 4 (st & 1) + g and bit-pair record 2 (st & 1) + (g & 1)
-  const int c = lane & 15, g = lane >> 4;
-  const bool row_ok = tile_ok && row0 + c < N;
-  const uint32_t rbase = (uint32_t)(row0 + c) * (uint32_t)nsb;
-  u32x4 wl[ST], wh[ST];
-  auto load_steps = [&](int sb0) {
-#pragma unroll
-    for (int st = 0; st < ST; st++) {
-      const int sb = sb0 + (st >> 1);
-      const bool ok = row_ok && sb < s1;
-      wl[st] = __builtin_amdgcn_raw_buffer_load_b128(ra, ok ? ((rbase + (uint32_t)sb) * 8u + 4u * (st & 1) + (uint32_t)g) * 16u : KBUF_OOB, 0, KBUF_NT);
-      wh[st] = __builtin_amdgcn_raw_buffer_load_b128(rh, ok ? ((rbase + (uint32_t)sb) * 4u + 2u * (st & 1) + (uint32_t)(g & 1)) * 16u : KBUF_OOB, 0, KBUF_NT);
-    }
-  };
-  // (MoE row tiles -- short rows, the slice is one trip -- ask for the weights first: behind the image copy they would be a
-  // second round trip to memory in a kernel that is little more than its prologue; all-Q6_K experts, 512 tokens: 250 us this
-  // way, 256 the other)
-  const bool wfirst = KMF_WEIGHTS_FIRST || a.tile_expert != nullptr;  // uniform
-  if (wfirst && XT == KQ_IMAGE) load_steps(s0);
-  __asm__ volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-
-  // ---- 3. activations into LDS -------------------------------------------------------------------------------------------------
-  if (XT == KQ_IMAGE) {  // codes [R][K], sums of 16 as int16 [R][K/16], scales [R][nsb]; R = MT, or the rows of a MoE image
-    const size_t R = a.img_rows ? (size_t)a.img_rows : (size_t)MT;
-    const u32x4* codes = reinterpret_cast<const u32x4*>(a.x);
-    const int16_t* sums = reinterpret_cast<const int16_t*>(reinterpret_cast<const char*>(a.x) + R * K);
-    const float* dd = reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.x) + R * K + R * nsb * 32);
-    // thread (row m = tid % MT, unit tid / MT), a batch of units requested before the first is stored, as in the Q4_K kernel
-    const int m = tid & (MT - 1), p0 = tid / MT, pstep = nthreads / MT;
-    const size_t src = (size_t)kq_tile_in_row(a, mt, m);
-    float dv[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-      if (p0 + i * pstep < nloc) dv[i] = dd[src * nsb + ks0 + p0 + i * pstep];
-    for (int u0 = p0; u0 < nul; u0 += pstep * KMF_COPY_UNROLL) {
-      u32x4 cv[KMF_COPY_UNROLL];
-      int16_t sv[KMF_COPY_UNROLL];
-#pragma unroll
-      for (int i = 0; i < KMF_COPY_UNROLL; i++) {
-        const int u = u0 + i * pstep;
-        if (u < nul) {
-          cv[i] = codes[src * nu + ks0 * 16 + u];
-          sv[i] = sums[src * nu + ks0 * 16 + u];
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < KMF_COPY_UNROLL; i++) {
-        const int u = u0 + i * pstep;
-        if (u < nul) {
-          xc[(size_t)u * MT + m] = cv[i];
-          bs16[(size_t)u * MT + m] = (int)sv[i];
-        }
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-      if (p0 + i * pstep < nloc) dxs[(p0 + i * pstep) * MT + m] = dv[i];
-    for (int sb = p0 + 2 * pstep; sb < nloc; sb += pstep) dxs[sb * MT + m] = dd[src * nsb + ks0 + sb];
-  } else {
-    const int ipr = K >> 3;      // items (eight elements) per row
-    const int iwg = nloc << 5;   // of them in this workgroup's super-blocks
-    const int nitems = MT * iwg;
-    const float inv_iwg = 1.0f / (float)iwg;
-    constexpr int QI = KMF_QUANT_BATCH;  // (a batch of items is requested before the first is quantized)
-    for (int it0 = tid; it0 < nitems; it0 += nthreads * QI) {  // whole half-waves
-      float v[QI][8];
-#pragma unroll
-      for (int b = 0; b < QI; b++) {
-        const int it = it0 + b * nthreads;
-        const int m = (int)(((float)it + 0.5f) * inv_iwg), i = it - m * iwg;
-#pragma unroll
-        for (int e = 0; e < 8; e++) v[b][e] = 0.f;
-        if (it < nitems && m < a.M) load8<XT == KQ_IMAGE ? MLLM_HIP_F32 : XT>(a.x, ((int64_t)m * ipr + 32 * ks0 + i) * 8, v[b]);
-      }
-      if (it0 == tid) load_steps(s0);  // the weights right behind the first batch: they arrive while it is quantized
-#pragma unroll
-      for (int b = 0; b < QI; b++) {
-        const int it = it0 + b * nthreads;
-        if (it >= nitems) break;
-        const Q8KItem qi = quantize_q8k_item(v[b], lane);
-        const int s16 = qi.sum8 + __builtin_amdgcn_update_dpp(0, qi.sum8, 0xB1, 0xf, 0xf, true);
-        const int m = (int)(((float)it + 0.5f) * inv_iwg), i = it - m * iwg;
-        const int u = i >> 1;
-        reinterpret_cast<u32x2*>(xc + (size_t)u * MT + m)[i & 1] = u32x2{qi.q0, qi.q1};
-        if ((i & 1) == 0) bs16[(size_t)u * MT + m] = s16;
-        if ((i & 31) == 0) dxs[(i >> 5) * MT + m] = qi.d;
-      }
-    }
-  }
-  if (!wfirst && XT == KQ_IMAGE) load_steps(s0);
-  if (XT != KQ_IMAGE && tid >= (nloc << 5) * MT) load_steps(s0);  // (threads without an item to quantize)
-  if (tid == 0) zrec[0] = u32x4{0u, 0u, 0u, 0u};
-  for (int i = tid; i < (lsb - nloc) * 16 * MT; i += nthreads) {
-    xc[(size_t)nul * MT + i] = u32x4{0u, 0u, 0u, 0u};
-    bs16[(size_t)nul * MT + i] = 0;
-  }
-  for (int i = tid; i < (lsb - nloc) * MT; i += nthreads) dxs[nloc * MT + i] = 0.f;
-#pragma unroll
-  for (int k = 0; k < 2; k++) {
-    const int ch = lane + 64 * k;
-    const int r = ch / sps, si = ch - r * sps;
-    if (r < 16) {
-      const float d = (s0 + si < nsb) ? f16bits_to_f32(scd[k]) : 0.f;
-      const uint32_t wds[4] = {sc[k].x, sc[k].y, sc[k].z, sc[k].w};
-#pragma unroll
-      for (int j = 0; j < 16; j++) ws[(16 * si + j) * 16 + r] = d * (float)(int8_t)(wds[j >> 2] >> (8 * (j & 3)));
-    }
-  }
-  for (int i = sps * 256 + lane; i < wsu * 16; i += 64) ws[i] = 0.f;
-  __syncthreads();
-
-  // ---- 4. unit sums on the matrix cores, scaling on the vector ALU ----------------------------------------------------------------
-  const int q = (lane & 15) >> 2, tt = lane & 3;
-  const bool mine = g == q;
-  const int shl = 2 * (g >> 1);  // this lane's low-nibble units take bit pair g / 2 of the high plane, its high-nibble units g / 2 + 2
-  f32x4 acc[TH];
-#pragma unroll
-  for (int h = 0; h < TH; h++) acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int sb0 = s0; sb0 < s1; sb0 += TSB) {
-    if (sb0 != s0) load_steps(sb0);
-    const int u0 = (sb0 - ks0) * 16;  // first unit of the trip in LDS
-    const u32x4* bl[TH];
-    const int* bsl[TH];
-    const float* dxl[TH];
-#pragma unroll
-    for (int h = 0; h < TH; h++) {
-      bl[h] = mine ? xc + (size_t)(u0 + q) * MT + 4 * h + tt : zrec;
-      bsl[h] = bs16 + (size_t)(u0 + q) * MT + 4 * h + tt;
-      dxl[h] = dxs + (sb0 - ks0) * MT + 4 * h + tt;
-    }
-    const int bstep = mine ? MT : 0;
-    const float* wsl = ws + (size_t)((sb0 - s0) * 16 + q) * 16 + 4 * g;
-    u32x4 B[2][2][TH];
-    int bs[2][2][TH];
-    float dxv[2][TH];
-    f32x4 dsv[2][2];
-    kv4i D[2][2][TH];
-    auto fetch_b = [&](int set, int st) {  // units 8 st + q (low nibbles) and 8 st + 4 + q (high)
-#pragma unroll
-      for (int h = 0; h < TH; h++) {
-        B[set][0][h] = bl[h][(8 * st) * bstep];
-        B[set][1][h] = bl[h][(8 * st + 4) * bstep];
-      }
-    };
-    auto fetch_s = [&](int set, int st) {
-#pragma unroll
-      for (int h = 0; h < TH; h++) {
-        bs[set][0][h] = bsl[h][(8 * st) * MT];
-        bs[set][1][h] = bsl[h][(8 * st + 4) * MT];
-        dxv[set][h] = dxl[h][(st >> 1) * MT];
-      }
-      dsv[set][0] = *reinterpret_cast<const f32x4*>(wsl + (8 * st) * 16);
-      dsv[set][1] = *reinterpret_cast<const f32x4*>(wsl + (8 * st + 4) * 16);
-    };
-    auto issue = [&](int set, int st) {
-      const uint32_t l4[4] = {wl[st].x, wl[st].y, wl[st].z, wl[st].w};
-      const uint32_t h4[4] = {wh[st].x, wh[st].y, wh[st].z, wh[st].w};
-      kv4i Alo, Ahi;
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const uint32_t hs = h4[e] >> shl;
-        Alo[e] = (int)((l4[e] & 0x0f0f0f0fu) | ((hs & 0x03030303u) << 4));
-        Ahi[e] = (int)(((l4[e] >> 4) & 0x0f0f0f0fu) | (((hs >> 4) & 0x03030303u) << 4));
-      }
-#pragma unroll
-      for (int h = 0; h < TH; h++) {
-        D[set][0][h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(Alo, __builtin_bit_cast(kv4i, B[set][0][h]), kv4i{0, 0, 0, 0}, 0, 0, 0);
-        D[set][1][h] = __builtin_amdgcn_mfma_i32_16x16x64_i8(Ahi, __builtin_bit_cast(kv4i, B[set][1][h]), kv4i{0, 0, 0, 0}, 0, 0, 0);
-      }
-    };
-    auto scale = [&](int set, int st) {
-      const bool live = sb0 + (st >> 1) < s1;  // uniform
-#pragma unroll
-      for (int h = 0; h < TH; h++) {
-        const float dx = live ? dxv[set][h] : 0.f;
-#pragma unroll
-        for (int w = 0; w < 2; w++) {
-          const int corr = -32 * bs[set][w][h];  // the codes went in as 0..63
-          acc[h].x = fmaf(dsv[set][w].x * dx, (float)(D[set][w][h].x + corr), acc[h].x);
-          acc[h].y = fmaf(dsv[set][w].y * dx, (float)(D[set][w][h].y + corr), acc[h].y);
-          acc[h].z = fmaf(dsv[set][w].z * dx, (float)(D[set][w][h].z + corr), acc[h].z);
-          acc[h].w = fmaf(dsv[set][w].w * dx, (float)(D[set][w][h].w + corr), acc[h].w);
-        }
-      }
-    };
-    fetch_b(0, 0);
-#pragma unroll
-    for (int st = 0; st < ST; st++) {
-      issue(st & 1, st);
-      if (st + 1 < ST) fetch_b((st + 1) & 1, st + 1);
-      fetch_s(st & 1, st);
-      __builtin_amdgcn_sched_barrier(0);
-      if (st > 0) scale((st - 1) & 1, st - 1);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    scale((ST - 1) & 1, ST - 1);
-  }
-#pragma unroll
-  for (int h = 0; h < TH; h++) {  // the four lanes of an activation row (units = 0..3 mod 4)
-    float v[4] = {acc[h].x, acc[h].y, acc[h].z, acc[h].w};
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      v[e] += __shfl_xor(v[e], 4, 64);
-      v[e] += __shfl_xor(v[e], 8, 64);
-    }
-    acc[h] = f32x4{v[0], v[1], v[2], v[3]};
-  }
-
-  // ---- 5. slices of a tile in slice order, bias ------------------------------------------------------------------------------
-  if (S > 1) {
-    __syncthreads();
-#pragma unroll
-    for (int h = 0; h < TH; h++) red[h * 64 + lane] = acc[h];
-    __syncthreads();
-    if (wave % S != 0) return;
-    for (int s = 1; s < S; s++)
-#pragma unroll
-      for (int h = 0; h < TH; h++) {
-        const f32x4 o = red[(size_t)s * TH * 64 + h * 64 + lane];
-        acc[h].x += o.x; acc[h].y += o.y; acc[h].z += o.z; acc[h].w += o.w;
-      }
-  }
-  if (km.SG > 1) {  // the slice groups of a grid column meet in global memory, as in the Q4_K kernel (S = 1 here: every wave is a tile)
-    const int SG = km.SG;
-    const int li = 4 * g + tt;
-    float* pbase = km.part + (((size_t)blockIdx.x * nwaves + wave) * SG) * 128;
-    if (q == 0) {
-#pragma unroll
-      for (int h = 0; h < TH; h++) {
-        float* dst = pbase + (size_t)sg * 128 + (16 * h + li) * 4;
-        __hip_atomic_store(dst + 0, acc[h].x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(dst + 1, acc[h].y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(dst + 2, acc[h].z, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(dst + 3, acc[h].w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (tid == 0) {
-      unsigned* cnt = km.counters + (size_t)blockIdx.x * km.cstride;
-      const unsigned old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const int last = old == (unsigned)(SG - 1);
-      if (last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
-      *s_flag = last;
-    }
-    __syncthreads();
-    if (!*s_flag) return;
-    if (q == 0) {
-#pragma unroll
-      for (int h = 0; h < TH; h++) {
-        float pv[8][4];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const float* src = pbase + (size_t)min(u, SG - 1) * 128 + (16 * h + li) * 4;
-#pragma unroll
-          for (int e = 0; e < 4; e++) pv[u][e] = __hip_atomic_load(src + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        acc[h] = f32x4{pv[0][0], pv[0][1], pv[0][2], pv[0][3]};
-#pragma unroll
-        for (int u = 1; u < 8; u++)
-          if (u < SG) { acc[h].x += pv[u][0]; acc[h].y += pv[u][1]; acc[h].z += pv[u][2]; acc[h].w += pv[u][3]; }
-      }
-    }
-  }
-  if (!tile_ok || q != 0) return;
-  const int n = row0 + 4 * g;
-#pragma unroll
-  for (int h = 0; h < TH; h++) {
-    const int t = 4 * h + tt;
-    if (t >= mt.rows) continue;
-    const float v[4] = {acc[h].x, acc[h].y, acc[h].z, acc[h].w};
-    float* yrow = pt.y + (int64_t)kq_tile_out_row(a, mt, t) * N;
-#pragma unroll
-    for (int e = 0; e < 4; e++)
-      if (n + e < N) yrow[n + e] = pt.bias ? v[e] + pt.bias[n + e] : v[e];
-  }
-}
-
-static int k6mf_steps(int sps) { return sps <= 3 ? 6 : (sps <= 4 ? 8 : K6_ST); }
-// super-blocks the last trip of a slice reads past the row (whole trips from the slice's first super-block)
-static int k6mf_xpad(int nsb, int S, int sps) {
-  const int tsb = k6mf_steps(sps) / 2;
-  int pad = 0;
-  for (int s = 0; s < S; s++) {
-    const int s0 = s * sps, s1 = std::min(nsb, s0 + sps);
-    if (s1 > s0) pad = std::max(pad, s0 + ((s1 - s0 - 1) / tsb + 1) * tsb - nsb);
-  }
-  return pad;
-}
-template <int MT>
-static size_t k6mf_lds_bytes(int nsb, int sps, int nwaves, int S) {
-  const int tsb = k6mf_steps(sps) / 2, rows = nsb + k6mf_xpad(nsb, S, sps);
-  const int wsu = (sps + tsb - 1) / tsb * tsb * 16;
-  const size_t need = (size_t)rows * 16 * MT * 16 + 16 + (size_t)rows * 16 * MT * 4 + (size_t)rows * MT * 4 + (size_t)nwaves * wsu * 64 + 16;
-  // the partial sums of the slices reuse the code area: it must hold them
-  return std::max(need, (size_t)nwaves * (MT / 4) * 1024);
-}
-// the same with one slice per workgroup (slice groups over the grid's z): the slice's super-blocks in whole trips
-template <int MT>
-static size_t k6mf_lds_bytes_z(int sps, int nwaves) {
-  const int tsb = k6mf_steps(sps) / 2, rows = (sps + tsb - 1) / tsb * tsb;
-  return (size_t)rows * 16 * MT * 16 + 16 + (size_t)rows * 16 * MT * 4 + (size_t)rows * MT * 4 + (size_t)nwaves * rows * 16 * 64 + 16;
-}
-static void k6mf_split(int nsb, int& S, int& sps) {
-  S = 1;
-  while (S < 8 && nsb > 5 * S) S *= 2;
-  sps = (nsb + S - 1) / S;
-}
-static bool kq6_mfma_fits(int MT, int nsb) {
-  int S, sps;
-  k6mf_split(nsb, S, sps);
-  if (sps > 8) return false;  // scale records: at most 128 per wave
-  return (MT == 4 ? k6mf_lds_bytes<4>(nsb, sps, 8, S) : k6mf_lds_bytes<8>(nsb, sps, 8, S)) <= 160 * 1024;
-}
-static int kq_meet_waves(const KGemvArgs& a, int SG);
-// every K slice a workgroup of its own (four to six row tiles), meeting in the caller's workspace: as launch_kq4_mfma_z
-template <int XT, int MT>
-static int launch_kq6_mfma_z(const KGemvArgs& a_in, const KMeetRoom& room, hipStream_t st) {
-  KGemvArgs a = a_in;
-  int SG, sps;
-  k6mf_split(a.nsb, SG, sps);
-  const int nwaves = kq_meet_waves(a, SG);
-  unsigned grid = 0;
-  for (int p = 0; p < a.nparts; p++) {
-    a.wg_start[p] = (int)grid;
-    grid += (unsigned)(((a.part[p].N + 15) / 16 + nwaves - 1) / nwaves);
-  }
-  a.wg_start[a.nparts] = (int)grid;
-  if (SG < 2 || sps > 8 || g_kq_meet == 0 || !room.part || (size_t)grid * nwaves * SG * 512 > room.part_bytes || grid > 1024u) return KQ_NOT_TAKEN;
-  KMeet km{};
-  km.SG = SG;
-  const int tsb = k6mf_steps(sps) / 2;
-  km.lrows = (sps + tsb - 1) / tsb * tsb;
-  km.part = static_cast<float*>(room.part);
-  RC_RET(gemv_counter_block(room.key, st, &km.counters));
-  km.cstride = 1;
-  while (km.cstride < 32 && (size_t)grid * km.cstride * 2 <= 1024u) km.cstride *= 2;
-  const size_t lds = k6mf_lds_bytes_z<MT>(sps, nwaves);
-  auto go = [&](auto kern) {
-    if (lds > 64 * 1024)
-      HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, dim3(grid, 1, (unsigned)SG), dim3(nwaves * 64), lds, st, a, 1, sps, km);
-    return (int)hipGetLastError();
-  };
-  switch (k6mf_steps(sps)) {
-    case 6: return go(kq6_gemv_mfma_kernel<XT, MT, 6>);
-    case 8: return go(kq6_gemv_mfma_kernel<XT, MT, 8>);
-    default: return go(kq6_gemv_mfma_kernel<XT, MT, K6_ST>);
-  }
-}
-template <int XT, int MT>
-static int launch_kq6_mfma_t(const KGemvArgs& a_in, hipStream_t st, unsigned grid_y = 1) {
-  KGemvArgs a = a_in;
-  int S, sps;
-  k6mf_split(a.nsb, S, sps);
-  int nwaves = XT == KQ_IMAGE ? 4 : 8;
-  if (nwaves < S) nwaves = S;
-  const int tiles_wg = nwaves / S;
-  unsigned grid = 0;
-  for (int p = 0; p < a.nparts; p++) {
-    a.wg_start[p] = (int)grid;
-    grid += (unsigned)(((a.part[p].N + 15) / 16 + tiles_wg - 1) / tiles_wg);
-  }
-  a.wg_start[a.nparts] = (int)grid;
-  const size_t lds = k6mf_lds_bytes<MT>(a.nsb, sps, nwaves, S);
-  if (lds > 160 * 1024) return MLLM_HIP_E_SHAPE;
-  KMeet km{};
-  km.SG = 1;
-  km.lrows = a.nsb + k6mf_xpad(a.nsb, S, sps);
-  auto go = [&](auto kern) {
-    if (lds > 64 * 1024)
-      HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(kern, dim3(grid, grid_y), dim3(nwaves * 64), lds, st, a, S, sps, km);
-    return (int)hipGetLastError();
-  };
-  switch (k6mf_steps(sps)) {
-    case 6: return go(kq6_gemv_mfma_kernel<XT, MT, 6>);
-    case 8: return go(kq6_gemv_mfma_kernel<XT, MT, 8>);
-    default: return go(kq6_gemv_mfma_kernel<XT, MT, K6_ST>);
-  }
-}
-template <int XT>
-static int launch_kq6_mfma(const KGemvArgs& a, hipStream_t st) {
-  return a.M <= 4 ? launch_kq6_mfma_t<XT, 4>(a, st) : launch_kq6_mfma_t<XT, 8>(a, st);
+// What mllm_hip_kq_workspace_bytes_n adds to the image: room for partial sums of K slices that no kernel leaves there any more (the
+// slices of a tile meet in LDS); the size stays what callers were told.
+static size_t kq_part_bytes(int nsb, int64_t n_total) {
+  const int S = nsb > 5 ? (nsb > 10 ? (nsb > 20 ? 8 : 4) : 2) : 1;
+  return S < 2 ? 0 : (size_t)((n_total + 15) / 16 + (int64_t)KQ_MAX_PARTS * 8) * S * 512;
 }
 
 static int g_kq_path = 0;  // 1: always the dot4 kernel, 2: the matrix-core kernels wherever they fit (comparison runs and tests)
@@ -1745,9 +810,6 @@ MLLM_API int mllm_hip_kq_set_path(int path) {
 }
 MLLM_API int mllm_hip_kq_set_slice_meeting(int mode, int waves_per_wg) {
   if (mode < -1 || mode > 1 || (waves_per_wg != 0 && (waves_per_wg < 1 || waves_per_wg > 8))) return MLLM_HIP_E_BADARG;
-  g_kq_meet = mode;
-  g_kq_meet_min = mode == 1 ? 2 : 4;
-  g_kq_meet_waves = waves_per_wg;
   return 0;
 }
 
@@ -1806,7 +868,7 @@ MLLM_API size_t mllm_hip_kq_workspace_bytes(int64_t M, int64_t K) {
 MLLM_API size_t mllm_hip_kq_workspace_bytes_n(int64_t M, int64_t K, int64_t N_total) {
   const size_t img = mllm_hip_kq_workspace_bytes(M, K);
   if (!img || N_total <= 0) return img;
-  return align_up(img, 256) + kmf_part_bytes((int)(K / QK_K), N_total, KQ_MAX_PARTS);
+  return align_up(img, 256) + kq_part_bytes((int)(K / QK_K), N_total);
 }
 
 MLLM_API int mllm_hip_linear_kq_multi(int wtype, int nparts, const mllm_hip_gemv_part* parts, const void* x, int x_dtype, int64_t M,
@@ -1829,14 +891,7 @@ MLLM_API int mllm_hip_linear_kq_multi_ws(int wtype, int nparts, const mllm_hip_g
   const int nsb = (int)(K / QK_K);
   hipStream_t st = (hipStream_t)stream;
   int rc = 0;
-  const size_t img_bytes = mllm_hip_kq_workspace_bytes(M, K);
-  if (workspace && workspace_bytes < img_bytes) return MLLM_HIP_E_BADARG;
-  // what lies behind the image serves the partial sums of K slices that meet in global memory
-  KMeetRoom room{workspace, nullptr, 0};
-  if (workspace && workspace_bytes > align_up(img_bytes, 256)) {
-    room.part = reinterpret_cast<char*>(workspace) + align_up(img_bytes, 256);
-    room.part_bytes = workspace_bytes - align_up(img_bytes, 256);
-  }
+  if (workspace && workspace_bytes < mllm_hip_kq_workspace_bytes(M, K)) return MLLM_HIP_E_BADARG;
   for (int64_t m0 = 0; m0 < M; m0 += 8) {  // more than eight rows: groups of eight (each streams the weights again)
     const int rows = (int)(M - m0 < 8 ? M - m0 : 8);
     const void* xg = reinterpret_cast<const char*>(x) + m0 * xrow;
@@ -1847,31 +902,21 @@ MLLM_API int mllm_hip_linear_kq_multi_ws(int wtype, int nparts, const mllm_hip_g
     a.x = xg;
     a.M = rows;
     a.nsb = nsb;
-    // Q4_K: from three rows on.  Q6_K (heavier unpacking, 200 registers): from five rows on, and with three or four rows of
-    // more than 4096 elements (4B layer shapes q+k+v / o / gate+up / down, dot4 -> matrix cores: eight rows 14.8 / 13.8 / 33.3 /
-    // 19.7 -> 13.8 / 12.6 / 25.0 / 19.7 us; four rows 11.1 / 10.1 / 24.1 / 17.8 -> 12.1 / 10.6 / 21.3 / 16.2).
-    // The rule looks at the weight type, the number of rows and the row length only: a projection gives the same bits alone
-    // and as a part of a launch.
-    const bool mfma = rows >= 3 && g_kq_path != 1 &&
-                      (wtype == MLLM_HIP_Q4_K ? kq4_mfma_fits(rows <= 4 ? 4 : 8, nsb)
-                                              : (rows > 4 || nsb > 16 || g_kq_path == 2) && kq6_mfma_fits(rows <= 4 ? 4 : 8, nsb));
-    int k6S = 1, k6sps = 0;
-    k6mf_split(nsb, k6S, k6sps);
-    // (Q6_K: from eight slices on; with four, 2560 x 4096 at eight rows, the one-workgroup form measured 12.7 us against 13.4)
-    if (mfma && room.part && g_kq_meet != 0 &&
-        (wtype == MLLM_HIP_Q4_K ? kmf_slices(nsb * 8) >= g_kq_meet_min : k6S >= (g_kq_meet == 1 ? 2 : 8))) {
-      // long rows: every workgroup takes one K slice and quantizes just that part of x itself; the slices meet in the workspace
-      const bool f32 = x_dtype == MLLM_HIP_F32, r4 = rows <= 4;
-      if (wtype == MLLM_HIP_Q4_K)
-        rc = r4 ? (f32 ? launch_kq4_mfma_z<MLLM_HIP_F32, 4>(a, room, st) : launch_kq4_mfma_z<MLLM_HIP_BF16, 4>(a, room, st))
-                : (f32 ? launch_kq4_mfma_z<MLLM_HIP_F32, 8>(a, room, st) : launch_kq4_mfma_z<MLLM_HIP_BF16, 8>(a, room, st));
-      else
-        rc = r4 ? (f32 ? launch_kq6_mfma_z<MLLM_HIP_F32, 4>(a, room, st) : launch_kq6_mfma_z<MLLM_HIP_BF16, 4>(a, room, st))
-                : (f32 ? launch_kq6_mfma_z<MLLM_HIP_F32, 8>(a, room, st) : launch_kq6_mfma_z<MLLM_HIP_BF16, 8>(a, room, st));
-      if (rc == 0) continue;
-      if (rc != KQ_NOT_TAKEN) return rc;
-    }
-    if (workspace && rows >= 3) {
+    // From three rows on the matrix cores, while the rows' codes fit the LDS.  The rule looks at the number of rows and the row
+    // length only: a projection gives the same bits alone and as a part of a launch.
+    if (rows >= 3 && g_kq_path != 1 && kr_fits(nsb)) {
+      // Quantized once, by a launch of its own, where every workgroup would have more than three items of eight elements per
+      // thread to quantize (q+k+v, gate+up of 2560 and o of 4096 elements, own launch / in the workgroups, us: three rows 7.8 / 6.7,
+      // 11.8 / 10.1, 7.5 / 6.9; five 8.0 / 7.6, 12.0 / 11.2, 7.5 / 8.2; eight 8.1 / 8.9, 12.3 / 12.4, 7.6 / 10.0).  Same bits.
+      if (workspace && rows * nsb * 32 > 3 * kr_threads(wtype, a)) {
+        hipLaunchKernelGGL(kr_image_kernel, dim3((unsigned)((nsb * 32 + 255) / 256), (unsigned)rows), dim3(256), 0, st, xg, x_dtype,
+                           reinterpret_cast<unsigned char*>(workspace), nsb, rows);
+        a.x = workspace;
+        rc = launch_kq_rows_any<KQ_IMAGE>(wtype, a, st);
+      } else {
+        rc = x_dtype == MLLM_HIP_F32 ? launch_kq_rows_any<MLLM_HIP_F32>(wtype, a, st) : launch_kq_rows_any<MLLM_HIP_BF16>(wtype, a, st);
+      }
+    } else if (workspace && rows >= 3) {
       // several rows: quantize once for all workgroups; the GEMV then copies the image instead of quantizing
       const int MT = rows <= 4 ? 4 : 8;
       int8_t* img = reinterpret_cast<int8_t*>(workspace);
@@ -1880,12 +925,7 @@ MLLM_API int mllm_hip_linear_kq_multi_ws(int wtype, int nparts, const mllm_hip_g
                          reinterpret_cast<float*>(img + (size_t)MT * K + (size_t)MT * nsb * 32),
                          reinterpret_cast<int16_t*>(img + (size_t)MT * K), nitems, (int64_t)rows * K / 8);
       a.x = img;
-      if (mfma) rc = wtype == MLLM_HIP_Q4_K ? launch_kq4_mfma<KQ_IMAGE>(a, st) : launch_kq6_mfma<KQ_IMAGE>(a, st);
-      else rc = wtype == MLLM_HIP_Q4_K ? launch_kq<MLLM_HIP_Q4_K, KQ_IMAGE>(a, st) : launch_kq<MLLM_HIP_Q6_K, KQ_IMAGE>(a, st);
-    } else if (mfma && wtype == MLLM_HIP_Q4_K) {
-      rc = x_dtype == MLLM_HIP_F32 ? launch_kq4_mfma<MLLM_HIP_F32>(a, st) : launch_kq4_mfma<MLLM_HIP_BF16>(a, st);
-    } else if (mfma) {
-      rc = x_dtype == MLLM_HIP_F32 ? launch_kq6_mfma<MLLM_HIP_F32>(a, st) : launch_kq6_mfma<MLLM_HIP_BF16>(a, st);
+      rc = wtype == MLLM_HIP_Q4_K ? launch_kq<MLLM_HIP_Q4_K, KQ_IMAGE>(a, st) : launch_kq<MLLM_HIP_Q6_K, KQ_IMAGE>(a, st);
     } else if (wtype == MLLM_HIP_Q4_K) {
       rc = x_dtype == MLLM_HIP_F32 ? launch_kq<MLLM_HIP_Q4_K, MLLM_HIP_F32>(a, st) : launch_kq<MLLM_HIP_Q4_K, MLLM_HIP_BF16>(a, st);
     } else {
@@ -1910,7 +950,7 @@ MLLM_API int mllm_hip_linear_kq(int wtype, const void* packed, const void* x, in
 namespace mllmhip {
 int exp_mode_accurate();  // layer_ops.hip: the setting of mllm_hip_set_exp_mode
 int kq_moe_gemv(int wtype, int nparts, const void* const* packed0, float* const* ys, int64_t N, int64_t K, const void* x, int x_dtype,
-                const float* x2, const int32_t* ids, int E, int slots, int slot_div, hipStream_t st) {
+                const float* x2, const int32_t* ids, int E, int slots, int slot_div, bool grouped, hipStream_t st) {
   if (x2 && x_dtype != MLLM_HIP_F32) return MLLM_HIP_E_BADARG;
   if (nparts < 1 || nparts > KQ_MAX_PARTS || slots < 1 || slots > 65535) return MLLM_HIP_E_SHAPE;
   KGemvArgs a{};
@@ -1926,6 +966,11 @@ int kq_moe_gemv(int wtype, int nparts, const void* const* packed0, float* const*
   a.slot_div = slot_div;
   a.slot_div_slots = slots;
   a.estride = kq_packed_bytes(wtype, N, K);
+  if (grouped) {
+    a.M = 8;
+    return x_dtype == MLLM_HIP_F32 ? launch_kq_rows_any<MLLM_HIP_F32>(wtype, a, st, (unsigned)slots)
+                                   : launch_kq_rows_any<MLLM_HIP_BF16>(wtype, a, st, (unsigned)slots);
+  }
   if (wtype == MLLM_HIP_Q4_K)
     return x_dtype == MLLM_HIP_F32 ? launch_kq<MLLM_HIP_Q4_K, MLLM_HIP_F32>(a, st) : launch_kq<MLLM_HIP_Q4_K, MLLM_HIP_BF16>(a, st);
   return x_dtype == MLLM_HIP_F32 ? launch_kq<MLLM_HIP_Q6_K, MLLM_HIP_F32>(a, st) : launch_kq<MLLM_HIP_Q6_K, MLLM_HIP_BF16>(a, st);
@@ -1944,7 +989,8 @@ int kq_quantize_image(const void* x, int x_dtype, void* image, int64_t rows, int
   return (int)hipGetLastError();
 }
 bool kq_moe_tiles_fit(int wtype, int64_t K) {
-  return wtype == MLLM_HIP_Q4_K ? kq4_mfma_fits(8, (int)(K / QK_K)) : kq6_mfma_fits(8, (int)(K / QK_K));
+  (void)wtype;
+  return kr_fits((int)(K / QK_K));
 }
 // MoE row tiles on the matrix-core kernels: tile t (blockIdx.y) = up to eight expert-sorted positions of expert tile_expert[t];
 // its rows read image rows row_ids[pos] / row_div (null: pos) and write rows out_ids[pos] (null: pos) of ys[p].
@@ -1962,7 +1008,7 @@ int kq_moe_tiles_gemv(int wtype, int nparts, const void* const* packed0, float* 
   a.tile_expert = tile_expert; a.tile_row0 = tile_row0; a.tile_rows = tile_rows; a.ntiles = ntiles;
   a.row_ids = row_ids; a.out_ids = out_ids; a.row_div = row_div > 0 ? row_div : 1;
   a.img_rows = (int)img_rows;
-  return wtype == MLLM_HIP_Q4_K ? launch_kq4_mfma_t<KQ_IMAGE, 8>(a, st, max_tiles) : launch_kq6_mfma_t<KQ_IMAGE, 8>(a, st, max_tiles);
+  return launch_kq_rows_any<KQ_IMAGE>(wtype, a, st, max_tiles);
 }
 }  // namespace mllmhip
 

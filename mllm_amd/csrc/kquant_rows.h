@@ -1,0 +1,486 @@
+// Q4_K / Q6_K weights x three to eight activation rows (or the rows of an MoE expert) on the matrix cores.  Included by
+// kquant.hip behind KGemvArgs, the Q8_K quantizer and load8.
+//
+// A tile is sixteen weight rows (channels) x up to eight activation rows x all of K.  The weights are the SECOND operand of
+// v_mfma_i32_16x16x64_i8, so that a lane owns ONE channel and the scales it needs are bytes of its own channel's record:
+// no table of scales in LDS, one byte extract per scale.  The instruction sums over K = 64 and every 32 (Q4_K) or 16 (Q6_K) elements
+// have a scale of their own, so the ACTIVATION operand keeps them apart: its sixteen rows are (sub-block pair member q, row m)
+// resp. (unit q of four, four of the rows), with zeros outside the lane group(s) that hold sub-block q.
+//   Q4_K  lane (channel c = l % 16, g = l / 16) holds record 4 j + g of its channel's super-block: the low-nibble instruction
+//         sees sub-block 4 j in groups 0, 1 and 4 j + 2 in groups 2, 3 (high nibbles one further); its four results are rows
+//         4 (g % 2) .. + 3 of the sub-block of q = g / 2.  I += sc * D; the minimum term accumulates in the matrix pipe: the same
+//         activation operand against the byte m in all sixteen places (one v_perm) sums m * code.
+//   Q6_K  group g's record is exactly one unit of 16 elements: D = sum over unit g of (code - 32) * x for four rows (the
+//         -32 is a first instruction against a constant operand), I += sc * D.  Five to eight rows: a second instruction.
+// Per super-block acc = fma(fp32(d * dx), float(I), acc) (and the minimum term): the reference's vec_dot (integer sums per
+// super-block, then d * dx) with the sums of a super-block split over two (Q4_K) or four lanes.
+//
+// What bounds it (time stamps written by the kernel, gate + up of 9728 x 2560 at five rows, us after the start): the codes back
+// 2.2, all waves past the barrier 3.8, the last wave's loop done 7.9, end 8.4 -- the weights, 28 MB, flow from 1.5 on.  Kept
+// short by spreading K over the waves of a workgroup (one tile's waves meet in LDS, not in memory), by requests for activations ahead
+// of every wave's weights, and by loading whole lines: with weights loaded in the operand's own order (sixteen rows per instruction) the
+// L1's tags were the bottleneck and the last wave passed the barrier at 10.7.  Five rows, us with the quantization (before: K slices as
+// workgroups that met in memory, or scale tables in LDS): q+k+v 9.9 -> 7.5, o 9.6 -> 7.5, gate+up 14.7 -> 11.2, down (Q6_K, 2560 x
+// 9728) 17.3 -> 12.6; 20 MB of the last take 4 us at the copy rate of the card.
+// K is cut into slices of KR_SPS super-blocks whatever the launch shape; a slice is summed in one chain and the slices are added in
+// order, by one wave or over several: the bits depend on the weight type and K alone.
+#pragma once
+
+constexpr int KR_SPS = 2;                      // super-blocks per slice
+constexpr int KR_SB_LDS = 16 * 8 * 16;         // codes of a super-block, at most: [unit of 16][rows] 16 bytes
+constexpr size_t KR_LDS_MAX = 160 * 1024;
+// the image in memory: codes [super-block][unit][rows][16], then scales [super-block][8]
+static int kr_slices(int nsb) { return (nsb + KR_SPS - 1) / KR_SPS; }
+// super-blocks of weights a wave has in flight: two, one where the registers of a second set would spill (more in flight, four, measured
+// slower: every wave then queues its requests for weights ahead of other waves' activations)
+constexpr int kr_depth(bool q4, int th) { return q4 || th == 1 ? 2 : 1; }
+constexpr int kr_stage_bytes(bool q4) { return q4 ? 2048 + 1024 + 256 : 2048 + 1024 + 1024 + 128; }  // per wave: codes [, bit pairs], scales, d
+static size_t kr_lds_bytes(bool q4, int nsb, int tiles, int waves_per_tile) {
+  return (size_t)(nsb + 1) * KR_SB_LDS + (size_t)nsb * 32 + 64 + (size_t)tiles * waves_per_tile * kr_stage_bytes(q4) +
+         (waves_per_tile > 1 ? (size_t)tiles * kr_slices(nsb) * 512 : 0);
+}
+static bool kr_fits(int nsb) { return kr_lds_bytes(false, nsb, 1, 4) <= KR_LDS_MAX; }
+
+// the activation rows -> the image
+__global__ __launch_bounds__(256) void kr_image_kernel(const void* __restrict__ x, int x_dtype, unsigned char* __restrict__ image, int nsb, int rows) {
+  const int it = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;  // item (eight elements) of row m; whole half-waves
+  if (it >= nsb * 32) return;
+  float v[8];
+  const int64_t e = ((int64_t)m * nsb * 32 + it) * 8;
+  if (x_dtype == MLLM_HIP_F32) load8<MLLM_HIP_F32>(x, e, v);
+  else load8<MLLM_HIP_BF16>(x, e, v);
+  const Q8KItem r = quantize_q8k_item(v, threadIdx.x & 63);
+  reinterpret_cast<u32x2*>(image)[((it >> 1) * rows + m) * 2 + (it & 1)] = u32x2{r.q0, r.q1};
+  if ((it & 31) == 0) reinterpret_cast<float*>(image + (size_t)nsb * 256 * rows)[(it >> 5) * 8 + m] = r.d;
+}
+
+// sum over lane bit 5 (permlane32) / bit 4 (permlane16) of two values at once: lanes with the bit clear keep a's, the others b's
+__device__ __forceinline__ float kr_fold32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float kr_fold16(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// a trip's weights on their way: whole 128-byte lines (lanes 8 r .. 8 r + 7 hold row r's super-block; one row per lane, the operand's own
+// order, would touch 64 lines per instruction and was bound by the L1's tag rate)
+template <int WT, int DEPTH>
+struct KrWeights {
+  u32x4 a[DEPTH][2], s;                             // rows l / 8 and 8 + l / 8, piece l % 8; scale record of (row l / 4, super-block l % 4)
+  u32x4 h[WT == MLLM_HIP_Q4_K ? 1 : DEPTH];         // Q6_K: row l / 4, piece l % 4
+  uint32_t d;                                         // as s
+};
+
+// blockDim = tiles per workgroup * P waves (wave = tile * P + p); XT: fp32 / bf16 activations, quantized by the workgroup, or the
+// image (KQ_IMAGE: of these eight rows; MoE row tiles: codes [rows][K], sums, scales of all rows, gathered).
+// TH = groups of four rows (Q4_K: always two).
+template <int WT, int XT, int TH>
+__global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr bool Q4 = WT == MLLM_HIP_Q4_K;
+  constexpr int DEPTH = kr_depth(Q4, TH);
+  const int nsb = a.nsb, K = nsb * QK_K;
+  const int tid = threadIdx.x, lane = tid & 63, nthreads = blockDim.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tiles_wg = (nthreads >> 6) / P, tl = wave / P, p = wave - tl * P;
+  int pidx = 0;
+#pragma unroll
+  for (int i = 1; i < KQ_MAX_PARTS; i++)
+    if (i < a.nparts && (int)blockIdx.x >= a.wg_start[i]) pidx = i;
+  const KGemvPart& pt = a.part[pidx];
+  const int N = pt.N;
+
+  u32x4* xc = reinterpret_cast<u32x4*>(smem);                                 // [unit][R rows] 16 codes
+  unsigned char* zblk = smem + (size_t)nsb * KR_SB_LDS;                       // one super-block of zeros
+  float* dxs = reinterpret_cast<float*>(zblk + KR_SB_LDS);                    // [super-block][8]
+  int* s_rows = reinterpret_cast<int*>(dxs + (size_t)nsb * 8);                // [8] MoE pairs: the tile's slots; [8]: how many
+  // a wave's own stage, where lines become operands: pieces of 16 bytes, conflict-free both ways (one wave's LDS operations execute in order)
+  unsigned char* stage = reinterpret_cast<unsigned char*>(s_rows) + 64 + (size_t)wave * kr_stage_bytes(Q4);
+  f32x2* part = reinterpret_cast<f32x2*>(reinterpret_cast<unsigned char*>(s_rows) + 64 + (size_t)(nthreads >> 6) * kr_stage_bytes(Q4));  // [tile][slice][lane]
+
+  constexpr int GROUP = Q4 ? 8 : 4 * TH;
+  // ---- which rows -----------------------------------------------------------------------------------------------------------
+  KTile mt = kq_tile(a);
+  if (!mt.active) return;  // uniform, ahead of every barrier
+  if (a.slot_ids) {
+    // MoE pairs: the pairs of one expert are found by the workgroups themselves.  Slot blockIdx.y works if it is the first of
+    // its expert's slots, or the ninth (GROUP = 8), ...; it takes the next eight.  No routing launch, weights read once per expert.
+    const int mine = blockIdx.y, e = a.slot_ids[mine];
+    if (e < 0 || e >= a.slot_E) return;
+    int before = 0, total = 0;
+    for (int c = 0; c < a.slot_div_slots; c += 64) {
+      const int s = c + lane;
+      const bool same = s < a.slot_div_slots && a.slot_ids[min(s, a.slot_div_slots - 1)] == e;
+      const unsigned long long b = __ballot(same);
+      const int ahead = total + __popcll(b & ((1ull << lane) - 1ull));  // this expert's slots ahead of s
+      if (mine >= c) before += __popcll(mine - c >= 64 ? b : b & ((1ull << (mine - c)) - 1ull));
+      // (mine's own rank is known once its chunk has been seen; slots behind it only count from then on)
+      if (same && s >= mine && ahead - before < GROUP) {
+        if (wave == 0) s_rows[ahead - before] = s;
+      }
+      total += __popcll(b);
+    }
+    if (before % GROUP) return;  // uniform
+    mt.rows = min(GROUP, total - before);
+    mt.eoff = (size_t)e * a.estride;
+    __syncthreads();
+  }
+  const int R = mt.rows;
+  auto in_row = [&](int m) -> int64_t { return a.slot_ids ? (int64_t)(s_rows[m] / a.slot_div) : (int64_t)kq_tile_in_row(a, mt, m); };
+
+  // ---- 1. activations requested, then the wave's first super-blocks of weights (memory requests return in order) ------------
+  const int c = lane & 15, g = lane >> 4;
+  const int row0 = (((int)blockIdx.x - a.wg_start[pidx]) * tiles_wg + tl) * 16;
+  const uint32_t sbt = (uint32_t)N * (uint32_t)nsb;
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(kq_at(pt.w.a, mt.eoff)), 0, sbt * 128u, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(kq_at(Q4 ? pt.w.a : pt.w.h, mt.eoff)), 0, sbt * 64u, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsc = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(kq_at(pt.w.s, mt.eoff)), 0, sbt * 16u, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kq_at(pt.w.d, mt.eoff)), 0, sbt * (Q4 ? 4u : 2u), 0x00020000);
+  const int S = (nsb + KR_SPS - 1) / KR_SPS;
+  const int sl0 = p * S / P, sl1 = (p + 1) * S / P;                // this wave's slices
+  const int sb0 = sl0 * KR_SPS, sb1 = min(nsb, sl1 * KR_SPS);      // and super-blocks
+  const uint32_t rb8 = (uint32_t)(row0 + (lane >> 3)) * (uint32_t)nsb, rb4 = (uint32_t)(row0 + (lane >> 2)) * (uint32_t)nsb;
+  const bool ok8[2] = {row0 + (lane >> 3) < N, row0 + 8 + (lane >> 3) < N}, ok4 = row0 + (lane >> 2) < N;
+  KrWeights<WT, DEPTH> w;
+  auto load_sb = [&](int i, int sb) {
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+      w.a[i][t] = __builtin_amdgcn_raw_buffer_load_b128(
+          ra, ok8[t] && sb < sb1 ? (rb8 + (uint32_t)(8 * t * nsb + sb)) * 128u + (uint32_t)(lane & 7) * 16u : KBUF_OOB, 0, KBUF_NT);
+    if constexpr (!Q4)
+      w.h[i] = __builtin_amdgcn_raw_buffer_load_b128(rh, ok4 && sb < sb1 ? (rb4 + (uint32_t)sb) * 64u + (uint32_t)(lane & 3) * 16u : KBUF_OOB, 0, KBUF_NT);
+  };
+  auto load_scales = [&](int sb) {
+    const int si = sb + (lane & 3);
+    const bool ok = ok4 && (lane & 3) < DEPTH && si < sb1;
+    w.s = __builtin_amdgcn_raw_buffer_load_b128(rsc, ok ? (rb4 + (uint32_t)si) * 16u : KBUF_OOB, 0, KBUF_NT);
+    if constexpr (Q4) w.d = __builtin_amdgcn_raw_buffer_load_b32(rd, ok ? (rb4 + (uint32_t)si) * 4u : KBUF_OOB, 0, KBUF_NT);
+    else w.d = __builtin_amdgcn_raw_buffer_load_b16(rd, ok ? (rb4 + (uint32_t)si) * 2u : KBUF_OOB, 0, KBUF_NT);
+  };
+  // (behind a barrier, so that the requests for activations of ALL waves are ahead of any weights: the L1 answers in order)
+  auto load_first = [&]() {
+    __asm__ volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    load_scales(sb0);
+#pragma unroll
+    for (int i = 0; i < DEPTH; i++) load_sb(i, sb0 + i);
+    __asm__ volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  for (int i = tid; i < KR_SB_LDS / 16; i += nthreads) reinterpret_cast<u32x4*>(zblk)[i] = u32x4{0u, 0u, 0u, 0u};
+  if (XT == KQ_IMAGE && !a.tile_expert) {
+    const u32x4* src = reinterpret_cast<const u32x4*>(a.x);
+    const int n16 = nsb * 16 * R;
+    constexpr int U = 6;
+    u32x4 v[U];
+    float dv = 0.f;
+    if (tid < nsb * 8) dv = reinterpret_cast<const float*>(src + n16)[tid];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (tid + u * nthreads < n16) v[u] = src[tid + u * nthreads];
+    load_first();
+    if (tid < nsb * 8) dxs[tid] = dv;
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (tid + u * nthreads < n16) xc[tid + u * nthreads] = v[u];
+    for (int i = tid + U * nthreads; i < n16; i += nthreads) xc[i] = src[i];
+    for (int i = tid + nthreads; i < nsb * 8; i += nthreads) dxs[i] = reinterpret_cast<const float*>(src + n16)[i];
+  } else if (XT == KQ_IMAGE) {  // rows gathered from codes [R][K], sums of 16 [R][K/16], scales [R][nsb]
+    const size_t RI = (size_t)a.img_rows;
+    const u32x4* codes = reinterpret_cast<const u32x4*>(a.x);
+    const float* dd = reinterpret_cast<const float*>(reinterpret_cast<const char*>(a.x) + RI * K + RI * nsb * 32);
+    const int m = tid & 7, p0 = tid >> 3, pstep = nthreads >> 3, nu = m < R ? nsb * 16 : 0;
+    const size_t src = (size_t)kq_tile_in_row(a, mt, m) * (size_t)nsb;  // in super-blocks
+    constexpr int U = 4;
+    u32x4 v[U];
+    float dv = 0.f;
+    if (p0 < nsb) dv = dd[src + p0];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (p0 + u * pstep < nu) v[u] = codes[src * 16 + p0 + u * pstep];
+    load_first();
+    if (p0 < nsb) dxs[p0 * 8 + m] = dv;
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (p0 + u * pstep < nu) xc[(p0 + u * pstep) * R + m] = v[u];
+    for (int u = p0 + U * pstep; u < nu; u += pstep) xc[u * R + m] = codes[src * 16 + u];
+    for (int sb = p0 + pstep; sb < nsb; sb += pstep) dxs[sb * 8 + m] = dd[src + sb];
+  } else {
+    // quantized here: items of eight elements, 32 consecutive ones = a super-block; rows past the tile's are left as they are
+    // (a row's results depend on its own codes only, and theirs are dropped)
+    constexpr int XL = XT == KQ_IMAGE ? MLLM_HIP_F32 : XT;
+    const int ipr = nsb * 32, nitems = mt.rows * ipr;
+    const float inv = 1.0f / (float)ipr;
+    constexpr int U = 2;  // items a thread requests ahead of the weights
+    const bool prod = XT == MLLM_HIP_F32 && a.x2 != nullptr;  // uniform
+    auto fetch = [&](int it, float (&v)[8], float (&f)[8]) {
+      const int m = (int)(((float)it + 0.5f) * inv), i = it - m * ipr;  // it / ipr: far from rounding trouble
+      const int64_t e = (in_row(m) * ipr + i) * 8;
+      load8<XL>(a.x, e, v);
+      if (prod) load8<MLLM_HIP_F32>(a.x2, e, f);
+    };
+    auto put = [&](int it, float (&v)[8], const float (&f)[8]) {
+      const int m = (int)(((float)it + 0.5f) * inv), i = it - m * ipr;
+      if (prod) silu_mul8(v, f, a.silu_accurate);
+      const Q8KItem q = quantize_q8k_item(v, lane);
+      reinterpret_cast<u32x2*>(xc)[((i >> 1) * R + m) * 2 + (i & 1)] = u32x2{q.q0, q.q1};
+      if ((i & 31) == 0) dxs[(i >> 5) * 8 + m] = q.d;
+    };
+    float v[U][8] = {}, f[U][8] = {};
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (tid + u * nthreads < nitems) fetch(tid + u * nthreads, v[u], f[u]);
+    load_first();
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (tid + u * nthreads < nitems) put(tid + u * nthreads, v[u], f[u]);  // whole half-waves
+    for (int it = tid + U * nthreads; it < nitems; it += nthreads) {
+      float v1[8], f1[8] = {};
+      fetch(it, v1, f1);
+      put(it, v1, f1);
+    }
+  }
+  __syncthreads();
+
+  // ---- 2. a super-block: sums on the matrix cores, scales as integers ---------------------------------------------------------
+  const int i16 = lane & 15;                      // the activation operand's row
+  const int q = Q4 ? i16 >> 3 : i16 >> 2;          // sub-block (unit) it belongs to
+  const int im = Q4 ? i16 & 7 : i16 & 3;           // and its row (Q6_K: of the first four)
+  // the lane groups that supply its codes; the others read zeros
+  const bool act = Q4 ? (g >> 1) == q : g == q;
+  const int u0 = Q4 ? 4 * q + (g & 1) : q, R16 = R * 16;
+  const unsigned char* xb[Q4 ? 1 : TH];
+  uint32_t xstep[Q4 ? 1 : TH];
+#pragma unroll
+  for (int h = 0; h < (Q4 ? 1 : TH); h++) {
+    const bool on = act && im + 4 * h < R;
+    xb[h] = on ? smem + u0 * R16 + (im + 4 * h) * 16 : zblk;
+    xstep[h] = on ? (uint32_t)(16 * R16) : 0u;
+  }
+  const float* dxl = dxs + (Q4 ? 4 * (g & 1) : 0);
+  constexpr int NA = Q4 ? 4 : 4 * TH;  // accumulators
+  float acc[NA], tot[2] = {0.f, 0.f};
+#pragma unroll
+  for (int r = 0; r < NA; r++) acc[r] = 0.f;
+  const uint32_t bsel = (uint32_t)g * 8u;
+  const kv4i zero = {0, 0, 0, 0}, m32 = {(int)0xe0e0e0e0u, (int)0xe0e0e0e0u, (int)0xe0e0e0e0u, (int)0xe0e0e0e0u};
+  u32x4* st_a = reinterpret_cast<u32x4*>(stage);                   // [16 rows][8] piece ^ (row / 2 % 8)
+  u32x4* st_s = st_a + 128;                                        // [16 rows][4] super-block ^ (row / 4)
+  u32x4* st_h = st_s + 64;                                         // Q6_K: [16 rows][4] piece ^ (row / 4)
+  uint32_t* st_d = reinterpret_cast<uint32_t*>(stage + 3072);      // Q4_K: [16 rows][4]
+  uint16_t* st_d6 = reinterpret_cast<uint16_t*>(stage + 4096);     // Q6_K: [16 rows][4]
+  const int wra = (lane >> 3) * 8 + ((lane & 7) ^ ((lane >> 4) & 7)), wrb = wra ^ 4;  // rows l / 8 and 8 + l / 8
+  const int wr4 = (lane & ~3) + ((lane & 3) ^ (lane >> 4));                           // row l / 4: (row / 4) = l / 16
+  auto put_scales = [&]() {
+    st_s[wr4] = w.s;
+    if constexpr (Q4) st_d[lane] = w.d;
+    else st_d6[lane] = (uint16_t)w.d;
+  };
+  auto put_sb = [&](int i) {
+    st_a[wra] = w.a[i][0];
+    st_a[64 + wrb] = w.a[i][1];
+    if constexpr (!Q4) st_h[wr4] = w.h[i];
+  };
+  struct {
+    u32x4 a[2], h[2], s4;
+    uint32_t s[2], d;
+  } u;
+  auto take_sb = [&](int i) {
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      u.a[j] = st_a[c * 8 + ((4 * j + g) ^ (c >> 1))];
+      if constexpr (Q4) u.s[j] = reinterpret_cast<const uint32_t*>(st_s + c * 4 + (i ^ (c >> 2)))[2 * j + (g >> 1)];
+      else u.h[j] = st_h[c * 4 + ((2 * j + (g & 1)) ^ (c >> 2))];
+    }
+    if constexpr (Q4) {
+      u.d = st_d[c * 4 + i];
+    } else {
+      u.s4 = st_s[c * 4 + (i ^ (c >> 2))];
+      u.d = st_d6[c * 4 + i];
+    }
+  };
+  auto compute = [&](int sb) {
+    if constexpr (Q4) {
+      int I[4] = {0, 0, 0, 0};
+      kv4i mn = zero;
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const unsigned char* x = xb[0] + (uint32_t)sb * xstep[0] + 8 * j * R16;
+        const kv4i xl = *reinterpret_cast<const kv4i*>(x), xh = *reinterpret_cast<const kv4i*>(x + 2 * R16);
+        kv4i wl, wh;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          wl[e] = (int)(u.a[j][e] & 0x0f0f0f0fu);
+          wh[e] = (int)((u.a[j][e] >> 4) & 0x0f0f0f0fu);
+        }
+        const int ml = (int)__builtin_amdgcn_perm(0u, u.s[j], 0x02020202u), mh = (int)__builtin_amdgcn_perm(0u, u.s[j], 0x03030303u);
+        const kv4i dl = __builtin_amdgcn_mfma_i32_16x16x64_i8(xl, wl, zero, 0, 0, 0);
+        const kv4i dh = __builtin_amdgcn_mfma_i32_16x16x64_i8(xh, wh, zero, 0, 0, 0);
+        mn = __builtin_amdgcn_mfma_i32_16x16x64_i8(xl, kv4i{ml, ml, ml, ml}, mn, 0, 0, 0);
+        mn = __builtin_amdgcn_mfma_i32_16x16x64_i8(xh, kv4i{mh, mh, mh, mh}, mn, 0, 0, 0);
+        const int sl = (int)(u.s[j] & 0xffu), sh = (int)((u.s[j] >> 8) & 0xffu);
+#pragma unroll
+        for (int r = 0; r < 4; r++) I[r] += __mul24(sl, dl[r]) + __mul24(sh, dh[r]);
+      }
+      const float d = f16bits_to_f32((uint16_t)(u.d & 0xffffu)), dmin = f16bits_to_f32((uint16_t)(u.d >> 16));
+      const f32x4 dx = *reinterpret_cast<const f32x4*>(dxl + sb * 8);
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        acc[r] = fmaf(dx[r] * d, (float)I[r], acc[r]);
+        acc[r] = fmaf(-(dx[r] * dmin), (float)mn[r], acc[r]);
+      }
+    } else {
+      int I[NA];
+#pragma unroll
+      for (int r = 0; r < NA; r++) I[r] = 0;
+      const uint32_t shl = 2u * (uint32_t)(g >> 1);  // low-nibble units of this group take bit pair g / 2, high-nibble units g / 2 + 2
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        kv4i wl, wh;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const uint32_t hs = u.h[j][e] >> shl;
+          wl[e] = (int)((u.a[j][e] & 0x0f0f0f0fu) | ((hs & 0x03030303u) << 4));
+          wh[e] = (int)(((u.a[j][e] >> 4) & 0x0f0f0f0fu) | (hs & 0x30303030u));
+        }
+        const int sl = (int)(u.s4[2 * j] << (24 - bsel)) >> 24, sh = (int)(u.s4[2 * j + 1] << (24 - bsel)) >> 24;
+#pragma unroll
+        for (int h = 0; h < TH; h++) {
+          const unsigned char* x = xb[h] + (uint32_t)sb * xstep[h] + 8 * j * R16;
+          const kv4i xl = *reinterpret_cast<const kv4i*>(x), xh = *reinterpret_cast<const kv4i*>(x + 4 * R16);
+          kv4i dl = __builtin_amdgcn_mfma_i32_16x16x64_i8(xl, m32, zero, 0, 0, 0);
+          kv4i dh = __builtin_amdgcn_mfma_i32_16x16x64_i8(xh, m32, zero, 0, 0, 0);
+          dl = __builtin_amdgcn_mfma_i32_16x16x64_i8(xl, wl, dl, 0, 0, 0);
+          dh = __builtin_amdgcn_mfma_i32_16x16x64_i8(xh, wh, dh, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; r++) I[4 * h + r] += __mul24(sl, dl[r]) + __mul24(sh, dh[r]);
+        }
+      }
+      const float d = f16bits_to_f32((uint16_t)u.d);
+#pragma unroll
+      for (int h = 0; h < TH; h++) {
+        const f32x4 dx = *reinterpret_cast<const f32x4*>(dxl + sb * 8 + 4 * h);
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[4 * h + r] = fmaf(dx[r] * d, (float)I[4 * h + r], acc[4 * h + r]);
+      }
+    }
+  };
+  // the end of a slice: the lanes of a channel meet.  Afterwards lane (c, g) holds two rows of channel c:
+  //   Q4_K 4 (g % 2) + g / 2 and that + 2;  Q6_K 2 (g % 2) + g / 2 and that + 4
+  auto flush = [&](int slice) {
+    f32x2 v;
+    if constexpr (Q4) {
+      v = f32x2{kr_fold32(acc[0], acc[1]), kr_fold32(acc[2], acc[3])};
+    } else {
+      v.x = kr_fold16(kr_fold32(acc[0], acc[1]), kr_fold32(acc[2], acc[3]));
+      v.y = TH == 2 ? kr_fold16(kr_fold32(acc[NA - 4], acc[NA - 3]), kr_fold32(acc[NA - 2], acc[NA - 1])) : 0.f;
+    }
+#pragma unroll
+    for (int r = 0; r < NA; r++) acc[r] = 0.f;
+    if (P > 1) {
+      part[(tl * S + slice) * 64 + lane] = v;
+    } else if (slice == 0) {
+      tot[0] = v.x;
+      tot[1] = v.y;
+    } else {
+      tot[0] += v.x;
+      tot[1] += v.y;
+    }
+  };
+  for (int sb = sb0; sb < sb1; sb += DEPTH) {
+    put_scales();
+    load_scales(sb + DEPTH);  // (past the wave's last one: fetches nothing)
+#pragma unroll
+    for (int i = 0; i < DEPTH; i++) {
+      if (sb + i < sb1) {  // uniform
+        put_sb(i);
+        __builtin_amdgcn_wave_barrier();
+        take_sb(i);
+        __builtin_amdgcn_wave_barrier();
+      }
+      load_sb(i, sb + DEPTH + i);
+      __builtin_amdgcn_sched_barrier(0);
+      if (sb + i < sb1) {
+        compute(sb + i);
+        if ((sb + i + 1) % KR_SPS == 0 || sb + i + 1 == nsb) flush((sb + i) / KR_SPS);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  // ---- 3. slices in order, bias ----------------------------------------------------------------------------------------------
+  if (P > 1) {
+    __syncthreads();
+    if (p != 0) return;
+    const f32x2 v0 = part[tl * S * 64 + lane];
+    tot[0] = v0.x;
+    tot[1] = v0.y;
+#pragma unroll 4
+    for (int s = 1; s < S; s++) {
+      const f32x2 v = part[(tl * S + s) * 64 + lane];
+      tot[0] += v.x;
+      tot[1] += v.y;
+    }
+  }
+  const int n = row0 + c;
+  if (n >= N) return;
+  const float bias = pt.bias ? pt.bias[n] : 0.f;
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const int m = Q4 ? 4 * (g & 1) + (g >> 1) + 2 * k : 2 * (g & 1) + (g >> 1) + 4 * k;
+    if (m >= mt.rows) continue;
+    const int64_t orow = a.slot_ids ? (int64_t)s_rows[m] : (int64_t)kq_tile_out_row(a, mt, m);
+    pt.y[orow * N + n] = pt.bias ? tot[k] + bias : tot[k];
+  }
+}
+
+// Tiles per workgroup and waves per tile.  A plain Linear: about one workgroup per CU, up to sixteen waves in it, none with more
+// slices than needed (2560 x 9728: one tile of ten waves 12.6 us, two tiles of eight 18; 2 x 9728 x 2560 in tiles x waves: 5 x 2
+// 12.0, 8 x 1 12.6, 2 x 8 17.2).  MoE: thousands of workgroups, small ones that share a CU (48 us with 4 x 1 for eight tokens,
+// 60 with 8 x 1, 65 with 2 x 2).
+struct KrShape {
+  int tiles, waves;
+};
+static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y) {
+  int64_t tiles = 0;
+  for (int i = 0; i < a.nparts; i++) tiles += (a.part[i].N + 15) / 16;
+  const int S = kr_slices(a.nsb);
+  const bool moe = a.slot_ids || a.tile_expert;
+  int tw = (int)std::min<int64_t>(moe ? 4 : 8, (tiles * grid_y + 255) / 256);
+  int P = moe ? 1 : std::min(S, tw >= 5 ? 10 / tw : 16 / tw);
+  while (P > 1 && (S + P - 2) / (P - 1) == (S + P - 1) / P) P--;
+  while (P > 1 && kr_lds_bytes(q4, a.nsb, 1, P) > KR_LDS_MAX) P--;
+  while (tw > 1 && kr_lds_bytes(q4, a.nsb, tw, P) > KR_LDS_MAX) tw--;
+  return KrShape{tw, P};
+}
+static int kr_threads(int wtype, const KGemvArgs& a) {
+  const KrShape s = kr_shape(wtype == MLLM_HIP_Q4_K, a, 1);
+  return s.tiles * s.waves * 64;
+}
+template <int WT, int XT, int TH>
+static int launch_kq_rows(const KGemvArgs& a_in, hipStream_t st, unsigned grid_y = 1) {
+  KGemvArgs a = a_in;
+  const KrShape shape = kr_shape(WT == MLLM_HIP_Q4_K, a, grid_y);
+  const int tw = shape.tiles, P = shape.waves;
+  const size_t lds = kr_lds_bytes(WT == MLLM_HIP_Q4_K, a.nsb, tw, P);
+  if (lds > KR_LDS_MAX) return MLLM_HIP_E_SHAPE;
+  unsigned grid = 0;
+  for (int i = 0; i < a.nparts; i++) {
+    a.wg_start[i] = (int)grid;
+    grid += (unsigned)(((a.part[i].N + 15) / 16 + tw - 1) / tw);
+  }
+  a.wg_start[a.nparts] = (int)grid;
+  auto kern = kq_rows_kernel<WT, XT, TH>;
+  if (lds > 64 * 1024)
+    HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(kern, dim3(grid, grid_y), dim3(tw * P * 64), lds, st, a, P);
+  return (int)hipGetLastError();
+}
+template <int XT>
+static int launch_kq_rows_any(int wtype, const KGemvArgs& a, hipStream_t st, unsigned grid_y = 1) {
+  if (wtype == MLLM_HIP_Q4_K) return launch_kq_rows<MLLM_HIP_Q4_K, XT, 2>(a, st, grid_y);
+  return a.M <= 4 ? launch_kq_rows<MLLM_HIP_Q6_K, XT, 1>(a, st, grid_y) : launch_kq_rows<MLLM_HIP_Q6_K, XT, 2>(a, st, grid_y);
+}

@@ -2448,7 +2448,7 @@ MLLM_API int mllm_hip_moe_ffn_q_gemm(int wtype, const void* gate_packed, const v
 // rows on the matrix-core kernels instead (the grouped form).
 namespace mllmhip {
 int kq_moe_gemv(int wtype, int nparts, const void* const* packed0, float* const* ys, int64_t N, int64_t K, const void* x, int x_dtype,
-                const float* x2, const int32_t* ids, int E, int slots, int slot_div, hipStream_t st);
+                const float* x2, const int32_t* ids, int E, int slots, int slot_div, bool grouped, hipStream_t st);
 size_t kq_image_bytes(int64_t rows, int64_t K);
 int kq_quantize_image(const void* x, int x_dtype, void* image, int64_t rows, int64_t K, hipStream_t st);
 bool kq_moe_tiles_fit(int wtype, int64_t K);
@@ -2518,8 +2518,6 @@ MLLM_API int mllm_hip_moe_ffn_kq2(int wtype, int wtype_down, const void* gate_pa
   // x and h are quantized to Q8_K once (bit-exact images), the tiles gather their rows from the images.
   const bool tiles_ok = E <= MOE_MAX_EXPERTS && kq_moe_tiles_fit(wtype, H) && kq_moe_tiles_fit(wtype_down, I) &&
                         (size_t)E + (size_t)slots / KQ_MOE_TILE + 1 <= 65535;
-  // measured at 128 experts, top-8 (pairs / tiles, us): Q4_K 16 tokens 80 / 84, 24: 112 / 97, 32: 145 / 112, 64: 289 / 153,
-  // 512: 2182 / 480; Q6_K 8 tokens 79 / 77, 16: 142 / 126, 32: 260 / 165, 512: 3976 / 760
   const bool many = (wtype == MLLM_HIP_Q4_K && wtype_down == MLLM_HIP_Q4_K) ? slots > E : 2 * slots > E;
   // Four pairs per expert and more: tiles of 32 rows, weights as the second operand of 32 x 32 matrix instructions (one pass
   // over an expert's weights per 32 pairs, one unpacking per 32 rows).  Same integer arithmetic; silu(gate) * up is formed where
@@ -2544,7 +2542,12 @@ MLLM_API int mllm_hip_moe_ffn_kq2(int wtype, int wtype_down, const void* gate_pa
                        (int)H, k, E);
     return (int)hipGetLastError();
   }
-  if (tiles_ok && (g_moe_kq_path == 2 || ((g_moe_kq_path == 0 || g_moe_kq_path == 3) && many))) {
+  // 16 pairs to one pair per expert: the workgroups find an expert's pairs themselves and take up to eight at a time (kquant_rows.h),
+  // without a routing launch; from one pair per expert on the sorted tiles.  128 experts, top-8, Q4_K / Q6_K, us, pairs one by
+  // one / grouped / sorted tiles: one token 15.0 / 17.2 / 24.4, two 21.7 / 20.2 / 29.4, eight 60.9 / 48.5 / 53.5, 16 - / 70.2 / 69.0,
+  // 32 - / 107 / 91
+  const bool grouped = g_moe_kq_path == 0 && kq_moe_tiles_fit(wtype, H) && kq_moe_tiles_fit(wtype_down, I) && slots >= 16 && slots < E && slots <= 512;
+  if (tiles_ok && (g_moe_kq_path == 2 || ((g_moe_kq_path == 0 || g_moe_kq_path == 3) && many && !grouped))) {
     const unsigned max_tiles = (unsigned)(E + slots / KQ_MOE_TILE + 1);
     RC_RET(launch_route(topk_ids, slots, E, KQ_MOE_TILE, w.ro, st));
     RC_RET(kq_quantize_image(x, x_dtype, w.ximg, T, H, st));
@@ -2566,19 +2569,19 @@ MLLM_API int mllm_hip_moe_ffn_kq2(int wtype, int wtype_down, const void* gate_pa
   }
   const void* gu[2] = {gate_packed, up_packed};
   float* guy[2] = {g, u};
-  int rc = kq_moe_gemv(wtype, 2, gu, guy, I, H, x, x_dtype, nullptr, topk_ids, E, slots, k, st);
+  int rc = kq_moe_gemv(wtype, 2, gu, guy, I, H, x, x_dtype, nullptr, topk_ids, E, slots, k, grouped, st);
   if (rc) return rc;
   // silu(g) * u: up to 32 pairs it is formed where the down GEMV reads its activations (same fp32 operations; one launch
   // fewer: one token 17.8 -> 16.4 us); with more pairs every down workgroup reading g and u costs more than the elementwise
   // launch (eight tokens 50 against 48 us)
   const void* dn[1] = {down_packed};
   float* dny[1] = {per};
-  if (slots <= 32) {
-    rc = kq_moe_gemv(wtype_down, 1, dn, dny, H, I, g, MLLM_HIP_F32, u, topk_ids, E, slots, 1, st);
+  if (slots <= (grouped ? 128 : 32)) {
+    rc = kq_moe_gemv(wtype_down, 1, dn, dny, H, I, g, MLLM_HIP_F32, u, topk_ids, E, slots, 1, grouped, st);
   } else {
     rc = mllm_hip_silu_mul(g, u, h, MLLM_HIP_F32, slots, I, nullptr, MLLM_HIP_SCALE_IEEE, stream);
     if (rc) return rc;
-    rc = kq_moe_gemv(wtype_down, 1, dn, dny, H, I, h, MLLM_HIP_F32, nullptr, topk_ids, E, slots, 1, st);
+    rc = kq_moe_gemv(wtype_down, 1, dn, dny, H, I, h, MLLM_HIP_F32, nullptr, topk_ids, E, slots, 1, grouped, st);
   }
   if (rc) return rc;
   const int64_t total = T * H;

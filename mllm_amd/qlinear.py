@@ -664,8 +664,7 @@ def linear_kq_gemm(w, x, bias=None, out=None, workspace=None, short=False):
 
 
 def linear_kq(w, x, bias=None, out=None, workspace=None):
-    """workspace (kq_workspace): from three rows on, x is quantized once by a small kernel instead of in every workgroup;
-    with room for partial sums (kq_workspace(M, K, N)), long Q4_K rows are cut into K slices with a workgroup each"""
+    """workspace (kq_workspace): from three rows on, x is quantized once by a small kernel where that is cheaper than in every workgroup"""
     assert w.layout == "gemv" and x.is_cuda and x.is_contiguous() and x.dim() == 2 and x.shape[1] == w.K
     M = x.shape[0]
     y = out if out is not None else torch.empty((M, w.N), dtype=torch.float32, device="cuda")

@@ -241,6 +241,47 @@ def test_k_slices_that_meet_in_the_workspace_give_the_same_bits(wtype, M):
 
 
 @pytest.mark.parametrize("wtype", [2, 3])
+@pytest.mark.parametrize("M,Ns,K", [(3, (1, 16, 17), 256), (4, (15,), 768), (5, (4097, 33), 1280), (8, (16 * 1400 + 3,), 512), (6, (40,), 15872),
+                                    (7, (9, 70), 16128)])
+def test_rows_kernel_edges(wtype, M, Ns, K):
+    """three to eight rows: part and odd tiles of 16 channels, one to many tiles per workgroup, odd numbers of super-blocks, the
+    longest rows whose codes fit the LDS and the first that do not, with a workspace and without"""
+    rng = synth.rng_for(7, 1700 + M + 50 * wtype)
+    Ws = [synth.make_weight(rng, wtype, N, K) for N in Ns]
+    ws = [ql.PackedKWeight(wtype, torch.from_numpy(W)) for W in Ws]
+    xf = synth.make_x_fp32(rng, M, K)
+    announce("kq rows", wtype, M, Ns, K)
+    ys = ql.linear_kq_multi(ws, to_dev(xf))
+    yw = ql.linear_kq_multi(ws, to_dev(xf), workspace=ql.kq_workspace(M, K))
+    for W, y, y2 in zip(Ws, ys, yw):
+        assert torch.equal(y, y2)
+        assert rel_l2(y.cpu().numpy(), orc.linear_kq(xf, W, wtype, None, orc.SCALE_X86_REF)) < 2e-6
+
+
+@pytest.mark.parametrize("wtype,T,E,k,shared", [(2, 8, 64, 2, 0), (3, 9, 64, 3, 19), (2, 31, 128, 4, 124), (3, 20, 256, 8, 9)])
+def test_moe_pairs_that_find_their_expert_group(wtype, T, E, k, shared):
+    """16 pairs up to one per expert: groups of up to eight pairs of an expert (shared = how many slots name expert 3, so that some
+    experts have one, exactly eight, nine and many pairs), invalid ids among them, against one GEMV row per pair"""
+    rng = synth.rng_for(9, 7300 + wtype + T + E)
+    L, H, I = _lib.lib(), 256, 512
+    g, u, d = (ql.PackedKExperts(wtype, torch.from_numpy(synth.make_weight(rng, wtype, E * n, K).reshape(E, n, K // 256, -1)))
+               for n, K in ((I, H), (I, H), (H, I)))
+    ids = rng.integers(0, E, size=(T, k)).astype(np.int32)
+    ids.reshape(-1)[:shared] = 3
+    ids[T - 1, k - 1], ids[0, k - 1] = -1, E
+    w = rng.random((T, k)).astype(np.float32)
+    x = to_dev(synth.make_x_fp32(rng, T, H))
+    announce("moe groups", wtype, T, E, k, shared)
+    y = ql.moe_ffn_kq(g, u, d, x, to_dev(ids), to_dev(w)).cpu().numpy()
+    assert L.mllm_hip_moe_kq_set_path(1) == 0
+    try:
+        y1 = ql.moe_ffn_kq(g, u, d, x, to_dev(ids), to_dev(w)).cpu().numpy()
+    finally:
+        assert L.mllm_hip_moe_kq_set_path(0) == 0
+    assert rel_l2(y, y1) < 1e-5, rel_l2(y, y1)
+
+
+@pytest.mark.parametrize("wtype", [2, 3])
 def test_units_in_flight_do_not_change_the_bits(wtype):
     """one or two rows: a lane adds its units in the same order whether the row is requested whole before the quantization of
     x (the default for Q4_K rows of up to 96 / 128 units) or trip by trip (mllm_hip_kq_set_tuning with units in flight)"""
