@@ -317,9 +317,11 @@ __global__ __launch_bounds__(SOFTMAX_WG) void softmax_long_rows_kernel(const flo
 // workgroup each, and the row's maximum and sum meet in the caller's workspace, so the operator is three launches: maxima of
 // the pieces, sums of the pieces (which need the row's maximum: the reference's polynomial is not exp(a) exp(b) = exp(a + b)
 // to fp32), results.  A workgroup per row is bound by what one CU can load and by its vector ALU: eight rows of 151 936 take
-// 49 us there and 14.8 here (one row 47 -> 14.2; a launch costs about 2.5 us whatever it does).
+// 49 us there and 11.4 here (one row 47 -> 9.3; a launch costs about 2.5 us whatever it does).  A piece inside the polynomial's
+// range has no branch per element, so that its exponentials overlap (with the branches: 14.8 and 13.5); pieces of 2048 elements
+// are no faster.
 constexpr int SOFTMAX_PIECE = 4096;
-constexpr int SOFTMAX_LONG = 40960;       // up to here one workgroup per row is as fast (32 000: 12.3 us against 13.9; 64 000: 21.7 against 14.1)
+constexpr int SOFTMAX_LONG = 40960;       // up to here one workgroup per row is as fast (32 000: 12.3 us against 13.9 with a branch per element; 64 000: 21.7 against 9.9)
 constexpr int SOFTMAX_SPLIT_ROWS = 512;
 __device__ __forceinline__ float block_max_256(float v, float* s_red) {
   v = wave_max(v);
@@ -368,12 +370,20 @@ __global__ __launch_bounds__(256) void softmax_pieces_kernel(const float* __rest
     for (int p = tid; p < pieces; p += 256) total += psum[p];
   mx = block_max_256(mx, s_red);
   float sum = 0.f;
+  if (poly && (int64_t)(piece + 1) * SOFTMAX_PIECE <= (len & ~7)) {  // (uniform) the whole piece takes the polynomial
 #pragma unroll
-  for (int j = 0; j < R; j++) {
-    const int i = i0 + 256 * j;
-    if (i < len) {
-      v[j] = softmax_exp(v[j] - mx, poly && i < (len & ~7));
+    for (int j = 0; j < R; j++) {
+      v[j] = exp_poly(v[j] - mx);
       sum += v[j];
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const int i = i0 + 256 * j;
+      if (i < len) {
+        v[j] = softmax_exp(v[j] - mx, poly && i < (len & ~7));
+        sum += v[j];
+      }
     }
   }
   if (STAGE == 1) {
