@@ -376,11 +376,12 @@ int mllm_hip_moe_ffn_q(int wtype, const void* gate_packed, const void* up_packed
 /* The same expert FFN with the experts in the super-block formats (MLLM_HIP_Q4_K / MLLM_HIP_Q6_K, the formats the shipped
  * Qwen3-MoE recipe quantizes to; activations Q8_K in front of every projection): gate_packed / up_packed / down_packed are E
  * matrices packed by mllm_hip_kq_prepack back to back, mllm_hip_kq_packed_bytes(wtype, I, H) resp. (wtype, H, I) apart.
- * H % 256 == 0, I % 256 == 0, T * k <= 65535, E <= 3072.  Up to one (token, expert) pair per expert (Q6_K: half) every pair runs as one
- * GEMV row (three or four launches; the decode form, an expert's weights are read once per pair that uses it); from 16
- * pairs on the workgroups of that form find the pairs that share an expert and take up to eight at once.  Beyond that
- * the pairs are sorted by expert and run as tiles of eight rows on the matrix cores (the grouped form: x and h quantized
- * to Q8_K once, an expert's weights read once per eight pairs; seven launches), same arithmetic; from four pairs per expert
+ * H % 256 == 0, I % 256 == 0, T * k <= 65535, E <= 3072.  Up to one (token, expert) pair per expert (with Q6_K: half) every pair runs as
+ * one GEMV row (three or four launches; the decode form, an expert's weights are read once per pair that uses it; Q6_K rows of 768 to
+ * 1536 elements with 16 to 512 pairs: once per four pairs, which their workgroups find, same bits).  Beyond that the pairs run as tiles
+ * of eight rows on the matrix cores, same arithmetic with the fp32 sums in another order: with Q6_K and 16 to 512 pairs, but less than
+ * one per expert, found by the workgroups (three or four launches), else sorted by expert (x and h quantized to Q8_K once, an
+ * expert's weights read once per eight pairs; seven launches; same bits).  From four pairs per expert
  * on (Q4_K) as tiles of 32 rows, the weights as the second operand of 32 x 32 matrix instructions (an expert's weights read
  * and unpacked once per 32 pairs), the same integers.
  * replaces: the same loop over experts with Q4_K / Q6_K Linear ops, modeling_qwen3_moe_fa2.hpp:98-100,175-238 */

@@ -947,10 +947,12 @@ MLLM_API int mllm_hip_linear_kq(int wtype, const void* packed, const void* x, in
 // nparts sibling matrices per expert (gate and up, or down alone), packed0[p] = expert 0's matrix of part p, the experts'
 // matrices mllm_hip_kq_packed_bytes(wtype, N, K) apart; slot s multiplies activation row s / slot_div by the matrices of
 // expert ids[s] and writes row s of ys[p] ([slots][N]).  x2 (fp32, same rows as x): the activation is silu(x) * x2.
+// form: KQ_MOE_PAIRS one by one; KQ_MOE_GROUPS the workgroups find the pairs that share an expert, same bits (kq_moe_groups_fit);
+// KQ_MOE_TILES they find them too, up to eight, with the sums of the sorted tiles.
 namespace mllmhip {
 int exp_mode_accurate();  // layer_ops.hip: the setting of mllm_hip_set_exp_mode
 int kq_moe_gemv(int wtype, int nparts, const void* const* packed0, float* const* ys, int64_t N, int64_t K, const void* x, int x_dtype,
-                const float* x2, const int32_t* ids, int E, int slots, int slot_div, bool grouped, hipStream_t st) {
+                const float* x2, const int32_t* ids, int E, int slots, int slot_div, int form, hipStream_t st) {
   if (x2 && x_dtype != MLLM_HIP_F32) return MLLM_HIP_E_BADARG;
   if (nparts < 1 || nparts > KQ_MAX_PARTS || slots < 1 || slots > 65535) return MLLM_HIP_E_SHAPE;
   KGemvArgs a{};
@@ -966,17 +968,33 @@ int kq_moe_gemv(int wtype, int nparts, const void* const* packed0, float* const*
   a.slot_div = slot_div;
   a.slot_div_slots = slots;
   a.estride = kq_packed_bytes(wtype, N, K);
-  if (grouped) {
+  if (form == KQ_MOE_GROUPS) {
+    if (wtype != MLLM_HIP_Q6_K) return MLLM_HIP_E_BADARG;
+    a.M = 4;
+    return x_dtype == MLLM_HIP_F32 ? launch_kq_rows<MLLM_HIP_Q6_K, MLLM_HIP_F32, 1, KR_PAIRS>(a, st, (unsigned)slots)
+                                   : launch_kq_rows<MLLM_HIP_Q6_K, MLLM_HIP_BF16, 1, KR_PAIRS>(a, st, (unsigned)slots);
+  }
+  if (form == KQ_MOE_TILES) {
     a.M = 8;
-    return x_dtype == MLLM_HIP_F32 ? launch_kq_rows_any<MLLM_HIP_F32>(wtype, a, st, (unsigned)slots)
-                                   : launch_kq_rows_any<MLLM_HIP_BF16>(wtype, a, st, (unsigned)slots);
+    return x_dtype == MLLM_HIP_F32 ? launch_kq_rows_any<MLLM_HIP_F32, KR_TILES>(wtype, a, st, (unsigned)slots)
+                                   : launch_kq_rows_any<MLLM_HIP_BF16, KR_TILES>(wtype, a, st, (unsigned)slots);
   }
   if (wtype == MLLM_HIP_Q4_K)
     return x_dtype == MLLM_HIP_F32 ? launch_kq<MLLM_HIP_Q4_K, MLLM_HIP_F32>(a, st) : launch_kq<MLLM_HIP_Q4_K, MLLM_HIP_BF16>(a, st);
   return x_dtype == MLLM_HIP_F32 ? launch_kq<MLLM_HIP_Q6_K, MLLM_HIP_F32>(a, st) : launch_kq<MLLM_HIP_Q6_K, MLLM_HIP_BF16>(a, st);
 }
 
-// The Q8_K image of `rows` activation rows of K elements (codes [rows][K], sums of 16 [rows][K/16] int16, scales
+// Groups of pairs pay for Q6_K rows of three to six super-blocks (the dot4 kernel's sixteen lanes then hold a row in one or two
+// trips and wait for each) from about 32 k rows of weights in the launch on.  128 to 512 experts, us of the layer, pairs one by one / in
+// groups: down 2048 x 768 at 16 / 24 / 64 pairs 0.91 / 0.83 / 0.76 of the time, 4096 x 1024 0.90 / 0.90 / 0.78, 1024 x 1024 1.05 /
+// 0.98 / 0.82; two super-blocks 1.01 to 1.15, eight 0.96 to 1.14 of it; gate + up of 2 x 512 x 1024 1.07 / 0.99 / 0.81, of 2 x 768 x 2048
+// 1.01 to 1.15.  (Q4_K: 0.95 to 1.2 over the same sizes.)  The search walks the slots, hence at most 512.
+bool kq_moe_groups_fit(int wtype, int64_t rows, int64_t K, int slots) {
+  const int64_t nsb = K / QK_K;
+  return wtype == MLLM_HIP_Q6_K && nsb >= 3 && nsb <= 6 && slots >= 16 && slots <= 512 && rows * slots >= 32768 && !g_kq_G && !g_kq_NW && !g_kq_U;
+}
+
+// The Q8_K image of `rows` activation rows (codes [rows][K], sums of 16 [rows][K/16] int16, scales
 // [rows][K/256]) at `image`: what the matrix-core kernels copy into LDS.
 size_t kq_image_bytes(int64_t rows, int64_t K) { return (size_t)rows * K + (size_t)rows * (K / 16) * 2 + (size_t)rows * (K / QK_K) * 4; }
 int kq_quantize_image(const void* x, int x_dtype, void* image, int64_t rows, int64_t K, hipStream_t st) {
@@ -1008,7 +1026,7 @@ int kq_moe_tiles_gemv(int wtype, int nparts, const void* const* packed0, float* 
   a.tile_expert = tile_expert; a.tile_row0 = tile_row0; a.tile_rows = tile_rows; a.ntiles = ntiles;
   a.row_ids = row_ids; a.out_ids = out_ids; a.row_div = row_div > 0 ? row_div : 1;
   a.img_rows = (int)img_rows;
-  return launch_kq_rows_any<KQ_IMAGE>(wtype, a, st, max_tiles);
+  return launch_kq_rows_any<KQ_IMAGE, KR_TILES>(wtype, a, st, max_tiles);
 }
 }  // namespace mllmhip
 

@@ -42,4 +42,7 @@ __host__ __device__ inline KView kq_view(int wtype, const void* packed, int64_t 
   return v;
 }
 
+// how the pairs of an MoE layer run in kq_moe_gemv (kquant.hip)
+enum { KQ_MOE_PAIRS, KQ_MOE_GROUPS, KQ_MOE_TILES };
+
 }  // namespace mllmhip

@@ -24,6 +24,17 @@
 // 9728) 17.3 -> 12.6; 20 MB of the last take 4 us at the copy rate of the card.
 // K is cut into slices of KR_SPS super-blocks whatever the launch shape; a slice is summed in one chain and the slices are added in
 // order, by one wave or over several: the bits depend on the weight type and K alone.
+//
+// MoE layers quantize twice more behind these sums, and the router of the next layer picks by them: a last bit that moves one code of h
+// or x over a rounding edge is 1e-4 to 1e-3 of a token's output.  A form that serves an MoE layer therefore keeps the fp32 order of the
+// form it stands in for (the integer sums are the same in all):
+//   KR_TILES  eight rows of an expert.  Every sub-block (Q6_K: unit of 16) is scaled on its own, acc = fma((d * sc) * dx, D, acc), Q4_K's
+//             minimum behind it, acc = fma(-((dmin * m) * dx), sum of the codes, acc); a lane group's chain runs over the slice
+//             (kr_moe_slice), the lane groups meet pairwise (0 + 1) + (2 + 3), then the slices in order.
+//   KR_PAIRS  Q6_K pairs in groups of four, in the order of the dot4 kernel on sixteen lanes per weight row: units of 64 elements
+//             (scaled int sum, then acc = fma(dx * d, sum, acc)) in sixteen chains, unit modulo 16, added as a binary tree.
+//             Bound by the weights of the experts in use; a Q4_K / Q6_K layer of 128 experts of 2048 x 768, top-8, two / four / eight tokens:
+//             22.5 / 35.1 / 59.7 -> 19.9 / 27.7 / 43.7 us against one dot4 row per pair.
 #pragma once
 
 constexpr int KR_SPS = 2;                      // super-blocks per slice
@@ -31,6 +42,12 @@ constexpr int KR_SB_LDS = 16 * 8 * 16;         // codes of a super-block, at mos
 constexpr size_t KR_LDS_MAX = 160 * 1024;
 // the image in memory: codes [super-block][unit][rows][16], then scales [super-block][8]
 static int kr_slices(int nsb) { return (nsb + KR_SPS - 1) / KR_SPS; }
+// super-blocks of a slice in MoE layers: up to five while there are at most eight slices
+__device__ __forceinline__ int kr_moe_slice(int nsb) {
+  int s = 1;
+  while (s < 8 && nsb > 5 * s) s *= 2;
+  return (nsb + s - 1) / s;
+}
 // super-blocks of weights a wave has in flight: two, one where the registers of a second set would spill (more in flight, four, measured
 // slower: every wave then queues its requests for weights ahead of other waves' activations)
 constexpr int kr_depth(bool q4, int th) { return q4 || th == 1 ? 2 : 1; }
@@ -59,6 +76,10 @@ __device__ __forceinline__ float kr_fold32(float a, float b) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+__device__ __forceinline__ int kr_fold32i(int a, int b) {
+  const auto r = __builtin_amdgcn_permlane32_swap((uint32_t)a, (uint32_t)b, false, false);
+  return (int)(r[0] + r[1]);
+}
 __device__ __forceinline__ float kr_fold16(float a, float b) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
@@ -75,12 +96,15 @@ struct KrWeights {
 
 // blockDim = tiles per workgroup * P waves (wave = tile * P + p); XT: fp32 / bf16 activations, quantized by the workgroup, or the
 // image (KQ_IMAGE: of these eight rows; MoE row tiles: codes [rows][K], sums, scales of all rows, gathered).
-// TH = groups of four rows (Q4_K: always two).
-template <int WT, int XT, int TH>
+// TH = groups of four rows (Q4_K: always two).  ORDER: the sums, see above; in MoE layers one wave per tile.
+enum { KR_LINEAR, KR_TILES, KR_PAIRS };
+template <int WT, int XT, int TH, int ORDER>
 __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr bool Q4 = WT == MLLM_HIP_Q4_K;
-  constexpr int DEPTH = kr_depth(Q4, TH);
+  constexpr bool TILES = ORDER == KR_TILES, PAIRS = ORDER == KR_PAIRS;
+  static_assert(!PAIRS || (!Q4 && TH == 1), "pairs in groups: Q6_K, groups of four");
+  constexpr int DEPTH = kr_depth(Q4, PAIRS ? 2 : TH);  // (pairs: sixteen accumulators)
   const int nsb = a.nsb, K = nsb * QK_K;
   const int tid = threadIdx.x, lane = tid & 63, nthreads = blockDim.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -106,7 +130,7 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
   if (!mt.active) return;  // uniform, ahead of every barrier
   if (a.slot_ids) {
     // MoE pairs: the pairs of one expert are found by the workgroups themselves.  Slot blockIdx.y works if it is the first of
-    // its expert's slots, or the ninth (GROUP = 8), ...; it takes the next eight.  No routing launch, weights read once per expert.
+    // its expert's slots, or the one after a group of GROUP, ...; it takes the next GROUP.  No routing launch, weights read once per expert.
     const int mine = blockIdx.y, e = a.slot_ids[mine];
     if (e < 0 || e >= a.slot_E) return;
     int before = 0, total = 0;
@@ -138,9 +162,10 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
   const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(kq_at(Q4 ? pt.w.a : pt.w.h, mt.eoff)), 0, sbt * 64u, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsc = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(kq_at(pt.w.s, mt.eoff)), 0, sbt * 16u, 0x00020000);
   const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kq_at(pt.w.d, mt.eoff)), 0, sbt * (Q4 ? 4u : 2u), 0x00020000);
-  const int S = (nsb + KR_SPS - 1) / KR_SPS;
+  const int sps = PAIRS ? nsb : TILES ? kr_moe_slice(nsb) : KR_SPS;
+  const int S = (nsb + sps - 1) / sps;
   const int sl0 = p * S / P, sl1 = (p + 1) * S / P;                // this wave's slices
-  const int sb0 = sl0 * KR_SPS, sb1 = min(nsb, sl1 * KR_SPS);      // and super-blocks
+  const int sb0 = sl0 * sps, sb1 = min(nsb, sl1 * sps);            // and super-blocks
   const uint32_t rb8 = (uint32_t)(row0 + (lane >> 3)) * (uint32_t)nsb, rb4 = (uint32_t)(row0 + (lane >> 2)) * (uint32_t)nsb;
   const bool ok8[2] = {row0 + (lane >> 3) < N, row0 + 8 + (lane >> 3) < N}, ok4 = row0 + (lane >> 2) < N;
   KrWeights<WT, DEPTH> w;
@@ -261,12 +286,13 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
     xstep[h] = on ? (uint32_t)(16 * R16) : 0u;
   }
   const float* dxl = dxs + (Q4 ? 4 * (g & 1) : 0);
-  constexpr int NA = Q4 ? 4 : 4 * TH;  // accumulators
+  constexpr int NA = PAIRS ? 16 : Q4 ? 4 : 4 * TH;  // accumulators (pairs: super-block modulo 4, half, row)
   float acc[NA], tot[2] = {0.f, 0.f};
 #pragma unroll
   for (int r = 0; r < NA; r++) acc[r] = 0.f;
   const uint32_t bsel = (uint32_t)g * 8u;
-  const kv4i zero = {0, 0, 0, 0}, m32 = {(int)0xe0e0e0e0u, (int)0xe0e0e0e0u, (int)0xe0e0e0e0u, (int)0xe0e0e0e0u};
+  const kv4i zero = {0, 0, 0, 0}, m32 = {(int)0xe0e0e0e0u, (int)0xe0e0e0e0u, (int)0xe0e0e0e0u, (int)0xe0e0e0e0u},
+             ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
   u32x4* st_a = reinterpret_cast<u32x4*>(stage);                   // [16 rows][8] piece ^ (row / 2 % 8)
   u32x4* st_s = st_a + 128;                                        // [16 rows][4] super-block ^ (row / 4)
   u32x4* st_h = st_s + 64;                                         // Q6_K: [16 rows][4] piece ^ (row / 4)
@@ -302,8 +328,31 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
       u.d = st_d6[c * 4 + i];
     }
   };
-  auto compute = [&](int sb) {
-    if constexpr (Q4) {
+  // (part: the super-block modulo 4, a constant; used by pairs only)
+  auto compute = [&](int sb, int part) {
+    if constexpr (Q4 && TILES) {
+      const float d = f16bits_to_f32((uint16_t)(u.d & 0xffffu)), dmin = f16bits_to_f32((uint16_t)(u.d >> 16));
+      const f32x4 dx = *reinterpret_cast<const f32x4*>(dxl + sb * 8);
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const unsigned char* x = xb[0] + (uint32_t)sb * xstep[0] + 8 * j * R16;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {  // sub-blocks 4 j + 2 q (low nibbles) and the next one (high nibbles)
+          const kv4i xv = *reinterpret_cast<const kv4i*>(x + 2 * h * R16);
+          kv4i wv;
+#pragma unroll
+          for (int e = 0; e < 4; e++) wv[e] = (int)((u.a[j][e] >> (4 * h)) & 0x0f0f0f0fu);
+          const kv4i D = __builtin_amdgcn_mfma_i32_16x16x64_i8(xv, wv, zero, 0, 0, 0);
+          const kv4i X = __builtin_amdgcn_mfma_i32_16x16x64_i8(xv, ones, zero, 0, 0, 0);  // sums of the codes
+          const float ds = d * (float)((u.s[j] >> (8 * h)) & 0xffu), dm = dmin * (float)((u.s[j] >> (16 + 8 * h)) & 0xffu);
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            acc[r] = fmaf(ds * dx[r], (float)D[r], acc[r]);
+            acc[r] = fmaf(-(dm * dx[r]), (float)X[r], acc[r]);
+          }
+        }
+      }
+    } else if constexpr (Q4) {
       int I[4] = {0, 0, 0, 0};
       kv4i mn = zero;
 #pragma unroll
@@ -333,9 +382,13 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
         acc[r] = fmaf(-(dx[r] * dmin), (float)mn[r], acc[r]);
       }
     } else {
-      int I[NA];
+      int I[4 * TH];
 #pragma unroll
-      for (int r = 0; r < NA; r++) I[r] = 0;
+      for (int r = 0; r < 4 * TH; r++) I[r] = 0;
+      const float d = f16bits_to_f32((uint16_t)u.d);
+      f32x4 dx[TH];
+#pragma unroll
+      for (int h = 0; h < TH; h++) dx[h] = *reinterpret_cast<const f32x4*>(dxl + sb * 8 + 4 * h);
       const uint32_t shl = 2u * (uint32_t)(g >> 1);  // low-nibble units of this group take bit pair g / 2, high-nibble units g / 2 + 2
 #pragma unroll
       for (int j = 0; j < 2; j++) {
@@ -347,6 +400,8 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
           wh[e] = (int)(((u.a[j][e] >> 4) & 0x0f0f0f0fu) | (hs & 0x30303030u));
         }
         const int sl = (int)(u.s4[2 * j] << (24 - bsel)) >> 24, sh = (int)(u.s4[2 * j + 1] << (24 - bsel)) >> 24;
+        const float dsl = d * (float)sl, dsh = d * (float)sh;
+        int U[4 * TH];  // pairs: this lane's share of a unit's sum
 #pragma unroll
         for (int h = 0; h < TH; h++) {
           const unsigned char* x = xb[h] + (uint32_t)sb * xstep[h] + 8 * j * R16;
@@ -356,24 +411,47 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
           dl = __builtin_amdgcn_mfma_i32_16x16x64_i8(xl, wl, dl, 0, 0, 0);
           dh = __builtin_amdgcn_mfma_i32_16x16x64_i8(xh, wh, dh, 0, 0, 0);
 #pragma unroll
-          for (int r = 0; r < 4; r++) I[4 * h + r] += __mul24(sl, dl[r]) + __mul24(sh, dh[r]);
+          for (int r = 0; r < 4; r++) {
+            if constexpr (TILES) {
+              acc[4 * h + r] = fmaf(dsl * dx[h][r], (float)dl[r], acc[4 * h + r]);
+              acc[4 * h + r] = fmaf(dsh * dx[h][r], (float)dh[r], acc[4 * h + r]);
+            } else if constexpr (PAIRS) {
+              U[r] = __mul24(sl, dl[r]) + __mul24(sh, dh[r]);
+            } else {
+              I[4 * h + r] += __mul24(sl, dl[r]) + __mul24(sh, dh[r]);
+            }
+          }
+        }
+        if constexpr (PAIRS) {  // records g and g + 2 make one unit of 64: lane groups 0, 1 keep rows 0, 2, groups 2, 3 rows 1, 3
+          const int s01 = kr_fold32i(U[0], U[1]), s23 = kr_fold32i(U[2], U[3]);
+          acc[4 * part + 2 * j] = fmaf((g >> 1 ? dx[0][1] : dx[0][0]) * d, (float)s01, acc[4 * part + 2 * j]);
+          acc[4 * part + 2 * j + 1] = fmaf((g >> 1 ? dx[0][3] : dx[0][2]) * d, (float)s23, acc[4 * part + 2 * j + 1]);
         }
       }
-      const float d = f16bits_to_f32((uint16_t)u.d);
+      if constexpr (ORDER == KR_LINEAR) {
 #pragma unroll
-      for (int h = 0; h < TH; h++) {
-        const f32x4 dx = *reinterpret_cast<const f32x4*>(dxl + sb * 8 + 4 * h);
+        for (int h = 0; h < TH; h++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) acc[4 * h + r] = fmaf(dx[r] * d, (float)I[4 * h + r], acc[4 * h + r]);
+          for (int r = 0; r < 4; r++) acc[4 * h + r] = fmaf(dx[h][r] * d, (float)I[4 * h + r], acc[4 * h + r]);
       }
     }
   };
   // the end of a slice: the lanes of a channel meet.  Afterwards lane (c, g) holds two rows of channel c:
-  //   Q4_K 4 (g % 2) + g / 2 and that + 2;  Q6_K 2 (g % 2) + g / 2 and that + 4
-  auto flush = [&](int slice) {
+  //   Q4_K 4 (g % 2) + g / 2 and that + 2;  Q6_K 2 (g % 2) + g / 2 and that + 4 (tiles: g and that + 4)
+  //   pairs: the row 2 (g % 2) + g / 2
+  int slice = sl0, left = sps;  // left: super-blocks up to the end of the slice
+  auto flush = [&]() {
     f32x2 v;
-    if constexpr (Q4) {
+    if constexpr (PAIRS) {
+      float s[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) s[i] = kr_fold16(acc[2 * i], acc[2 * i + 1]);
+      v = f32x2{((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7])), 0.f};
+    } else if constexpr (Q4) {
       v = f32x2{kr_fold32(acc[0], acc[1]), kr_fold32(acc[2], acc[3])};
+    } else if constexpr (TILES) {  // (units 0, 1 and 2, 3 first)
+      v.x = kr_fold32(kr_fold16(acc[0], acc[1]), kr_fold16(acc[2], acc[3]));
+      v.y = TH == 2 ? kr_fold32(kr_fold16(acc[NA - 4], acc[NA - 3]), kr_fold16(acc[NA - 2], acc[NA - 1])) : 0.f;
     } else {
       v.x = kr_fold16(kr_fold32(acc[0], acc[1]), kr_fold32(acc[2], acc[3]));
       v.y = TH == 2 ? kr_fold16(kr_fold32(acc[NA - 4], acc[NA - 3]), kr_fold32(acc[NA - 2], acc[NA - 1])) : 0.f;
@@ -389,25 +467,33 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
       tot[0] += v.x;
       tot[1] += v.y;
     }
+    slice++;
+    left = sps;
   };
-  for (int sb = sb0; sb < sb1; sb += DEPTH) {
-    put_scales();
-    load_scales(sb + DEPTH);  // (past the wave's last one: fetches nothing)
+  constexpr int TRIPS = PAIRS ? 4 / DEPTH : 1;  // (pairs: the super-block modulo 4 is a constant)
+  for (int t0 = sb0; t0 < sb1; t0 += TRIPS * DEPTH) {
 #pragma unroll
-    for (int i = 0; i < DEPTH; i++) {
-      if (sb + i < sb1) {  // uniform
-        put_sb(i);
-        __builtin_amdgcn_wave_barrier();
-        take_sb(i);
-        __builtin_amdgcn_wave_barrier();
+    for (int t = 0; t < TRIPS; t++) {
+      const int sb = t0 + t * DEPTH;
+      if (t && sb >= sb1) break;  // uniform
+      put_scales();
+      load_scales(sb + DEPTH);  // (past the wave's last one: fetches nothing)
+#pragma unroll
+      for (int i = 0; i < DEPTH; i++) {
+        if (sb + i < sb1) {  // uniform
+          put_sb(i);
+          __builtin_amdgcn_wave_barrier();
+          take_sb(i);
+          __builtin_amdgcn_wave_barrier();
+        }
+        load_sb(i, sb + DEPTH + i);
+        __builtin_amdgcn_sched_barrier(0);
+        if (sb + i < sb1) {
+          compute(sb + i, t * DEPTH + i);
+          if (--left == 0 || sb + i + 1 == nsb) flush();
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      load_sb(i, sb + DEPTH + i);
-      __builtin_amdgcn_sched_barrier(0);
-      if (sb + i < sb1) {
-        compute(sb + i);
-        if ((sb + i + 1) % KR_SPS == 0 || sb + i + 1 == nsb) flush((sb + i) / KR_SPS);
-      }
-      __builtin_amdgcn_sched_barrier(0);
     }
   }
 
@@ -429,8 +515,8 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
   if (n >= N) return;
   const float bias = pt.bias ? pt.bias[n] : 0.f;
 #pragma unroll
-  for (int k = 0; k < 2; k++) {
-    const int m = Q4 ? 4 * (g & 1) + (g >> 1) + 2 * k : 2 * (g & 1) + (g >> 1) + 4 * k;
+  for (int k = 0; k < (PAIRS ? 1 : 2); k++) {
+    const int m = Q4 ? 4 * (g & 1) + (g >> 1) + 2 * k : (TILES ? g : 2 * (g & 1) + (g >> 1)) + 4 * k;
     if (m >= mt.rows) continue;
     const int64_t orow = a.slot_ids ? (int64_t)s_rows[m] : (int64_t)kq_tile_out_row(a, mt, m);
     pt.y[orow * N + n] = pt.bias ? tot[k] + bias : tot[k];
@@ -460,7 +546,7 @@ static int kr_threads(int wtype, const KGemvArgs& a) {
   const KrShape s = kr_shape(wtype == MLLM_HIP_Q4_K, a, 1);
   return s.tiles * s.waves * 64;
 }
-template <int WT, int XT, int TH>
+template <int WT, int XT, int TH, int ORDER>
 static int launch_kq_rows(const KGemvArgs& a_in, hipStream_t st, unsigned grid_y = 1) {
   KGemvArgs a = a_in;
   const KrShape shape = kr_shape(WT == MLLM_HIP_Q4_K, a, grid_y);
@@ -473,14 +559,14 @@ static int launch_kq_rows(const KGemvArgs& a_in, hipStream_t st, unsigned grid_y
     grid += (unsigned)(((a.part[i].N + 15) / 16 + tw - 1) / tw);
   }
   a.wg_start[a.nparts] = (int)grid;
-  auto kern = kq_rows_kernel<WT, XT, TH>;
+  auto kern = kq_rows_kernel<WT, XT, TH, ORDER>;
   if (lds > 64 * 1024)
     HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   hipLaunchKernelGGL(kern, dim3(grid, grid_y), dim3(tw * P * 64), lds, st, a, P);
   return (int)hipGetLastError();
 }
-template <int XT>
+template <int XT, int ORDER = KR_LINEAR>
 static int launch_kq_rows_any(int wtype, const KGemvArgs& a, hipStream_t st, unsigned grid_y = 1) {
-  if (wtype == MLLM_HIP_Q4_K) return launch_kq_rows<MLLM_HIP_Q4_K, XT, 2>(a, st, grid_y);
-  return a.M <= 4 ? launch_kq_rows<MLLM_HIP_Q6_K, XT, 1>(a, st, grid_y) : launch_kq_rows<MLLM_HIP_Q6_K, XT, 2>(a, st, grid_y);
+  if (wtype == MLLM_HIP_Q4_K) return launch_kq_rows<MLLM_HIP_Q4_K, XT, 2, ORDER>(a, st, grid_y);
+  return a.M <= 4 ? launch_kq_rows<MLLM_HIP_Q6_K, XT, 1, ORDER>(a, st, grid_y) : launch_kq_rows<MLLM_HIP_Q6_K, XT, 2, ORDER>(a, st, grid_y);
 }

@@ -11,6 +11,7 @@
 // a lane owns one output channel: its weight scale is a scalar per block and stores are contiguous across lanes.
 #include "qgemv_kernel.h"
 #include "qgemm_layout.h"
+#include "kquant_layout.h"
 #include "wk_gemm.h"
 
 namespace mllmhip {
@@ -2448,7 +2449,8 @@ MLLM_API int mllm_hip_moe_ffn_q_gemm(int wtype, const void* gate_packed, const v
 // rows on the matrix-core kernels instead (the grouped form).
 namespace mllmhip {
 int kq_moe_gemv(int wtype, int nparts, const void* const* packed0, float* const* ys, int64_t N, int64_t K, const void* x, int x_dtype,
-                const float* x2, const int32_t* ids, int E, int slots, int slot_div, bool grouped, hipStream_t st);
+                const float* x2, const int32_t* ids, int E, int slots, int slot_div, int form, hipStream_t st);
+bool kq_moe_groups_fit(int wtype, int64_t rows, int64_t K, int slots);
 size_t kq_image_bytes(int64_t rows, int64_t K);
 int kq_quantize_image(const void* x, int x_dtype, void* image, int64_t rows, int64_t K, hipStream_t st);
 bool kq_moe_tiles_fit(int wtype, int64_t K);
@@ -2542,12 +2544,11 @@ MLLM_API int mllm_hip_moe_ffn_kq2(int wtype, int wtype_down, const void* gate_pa
                        (int)H, k, E);
     return (int)hipGetLastError();
   }
-  // 16 pairs to one pair per expert: the workgroups find an expert's pairs themselves and take up to eight at a time (kquant_rows.h),
-  // without a routing launch; from one pair per expert on the sorted tiles.  128 experts, top-8, Q4_K / Q6_K, us, pairs one by
-  // one / grouped / sorted tiles: one token 15.0 / 17.2 / 24.4, two 21.7 / 20.2 / 29.4, eight 60.9 / 48.5 / 53.5, 16 - / 70.2 / 69.0,
-  // 32 - / 107 / 91
-  const bool grouped = g_moe_kq_path == 0 && kq_moe_tiles_fit(wtype, H) && kq_moe_tiles_fit(wtype_down, I) && slots >= 16 && slots < E && slots <= 512;
-  if (tiles_ok && (g_moe_kq_path == 2 || ((g_moe_kq_path == 0 || g_moe_kq_path == 3) && many && !grouped))) {
+  // Such tiles with 16 pairs to less than one pair per expert: the workgroups find an expert's pairs themselves and take up to
+  // eight at a time (kquant_rows.h), without a routing launch; same bits.  Q4_K / Q6_K, 128 experts, top-8, us, sorted tiles / this: 2048 x
+  // 768 nine tokens 56.6 / 54.4, twelve 62.3 / 61.8, fifteen 67.6 / 68.8; 1024 x 512 nine 31.5 / 27.2, twelve 33.8 / 30.8
+  const bool unsorted = g_moe_kq_path == 0 && tiles_ok && many && slots >= 16 && slots < E && slots <= 512;
+  if (tiles_ok && (g_moe_kq_path == 2 || ((g_moe_kq_path == 0 || g_moe_kq_path == 3) && many && !unsorted))) {
     const unsigned max_tiles = (unsigned)(E + slots / KQ_MOE_TILE + 1);
     RC_RET(launch_route(topk_ids, slots, E, KQ_MOE_TILE, w.ro, st));
     RC_RET(kq_quantize_image(x, x_dtype, w.ximg, T, H, st));
@@ -2569,19 +2570,23 @@ MLLM_API int mllm_hip_moe_ffn_kq2(int wtype, int wtype_down, const void* gate_pa
   }
   const void* gu[2] = {gate_packed, up_packed};
   float* guy[2] = {g, u};
-  int rc = kq_moe_gemv(wtype, 2, gu, guy, I, H, x, x_dtype, nullptr, topk_ids, E, slots, k, grouped, st);
+  auto form = [&](int wt, int64_t rows, int64_t K) {
+    return unsorted ? KQ_MOE_TILES : g_moe_kq_path == 0 && kq_moe_groups_fit(wt, rows, K, slots) ? KQ_MOE_GROUPS : KQ_MOE_PAIRS;
+  };
+  const int form_down = form(wtype_down, H, I);
+  int rc = kq_moe_gemv(wtype, 2, gu, guy, I, H, x, x_dtype, nullptr, topk_ids, E, slots, k, form(wtype, 2 * I, H), st);
   if (rc) return rc;
   // silu(g) * u: up to 32 pairs it is formed where the down GEMV reads its activations (same fp32 operations; one launch
   // fewer: one token 17.8 -> 16.4 us); with more pairs every down workgroup reading g and u costs more than the elementwise
-  // launch (eight tokens 50 against 48 us)
+  // launch (eight tokens 50 against 48 us), where the workgroups share an expert's pairs from about 128 on
   const void* dn[1] = {down_packed};
   float* dny[1] = {per};
-  if (slots <= (grouped ? 128 : 32)) {
-    rc = kq_moe_gemv(wtype_down, 1, dn, dny, H, I, g, MLLM_HIP_F32, u, topk_ids, E, slots, 1, grouped, st);
+  if (slots <= (form_down != KQ_MOE_PAIRS ? 128 : 32)) {
+    rc = kq_moe_gemv(wtype_down, 1, dn, dny, H, I, g, MLLM_HIP_F32, u, topk_ids, E, slots, 1, form_down, st);
   } else {
     rc = mllm_hip_silu_mul(g, u, h, MLLM_HIP_F32, slots, I, nullptr, MLLM_HIP_SCALE_IEEE, stream);
     if (rc) return rc;
-    rc = kq_moe_gemv(wtype_down, 1, dn, dny, H, I, h, MLLM_HIP_F32, nullptr, topk_ids, E, slots, 1, grouped, st);
+    rc = kq_moe_gemv(wtype_down, 1, dn, dny, H, I, h, MLLM_HIP_F32, nullptr, topk_ids, E, slots, 1, form_down, st);
   }
   if (rc) return rc;
   const int64_t total = T * H;

@@ -258,27 +258,102 @@ def test_rows_kernel_edges(wtype, M, Ns, K):
         assert rel_l2(y.cpu().numpy(), orc.linear_kq(xf, W, wtype, None, orc.SCALE_X86_REF)) < 2e-6
 
 
-@pytest.mark.parametrize("wtype,T,E,k,shared", [(2, 8, 64, 2, 0), (3, 9, 64, 3, 19), (2, 31, 128, 4, 124), (3, 20, 256, 8, 9)])
-def test_moe_pairs_that_find_their_expert_group(wtype, T, E, k, shared):
-    """16 pairs up to one per expert: groups of up to eight pairs of an expert (shared = how many slots name expert 3, so that some
-    experts have one, exactly eight, nine and many pairs), invalid ids among them, against one GEMV row per pair"""
-    rng = synth.rng_for(9, 7300 + wtype + T + E)
-    L, H, I = _lib.lib(), 256, 512
-    g, u, d = (ql.PackedKExperts(wtype, torch.from_numpy(synth.make_weight(rng, wtype, E * n, K).reshape(E, n, K // 256, -1)))
-               for n, K in ((I, H), (I, H), (H, I)))
+@pytest.mark.parametrize("wtype,H,I,T,E,k,shared,same_as", [
+    # pairs one by one, pairs in groups of four (Q6_K, three to six super-blocks; gate / up, down or both), at the edges of that rule
+    (2, 768, 1024, 16, 64, 2, 19, 1), (3, 2048, 768, 8, 64, 2, 0, 1), (3, 1024, 512, 11, 64, 2, 9, 1), (3, 1024, 2048, 4, 64, 4, 5, 1),
+    ((2, 3), 2048, 768, 9, 64, 3, 19, 1), ((2, 3), 2048, 1536, 31, 256, 4, 124, 1), ((3, 2), 1536, 1024, 15, 64, 2, 30, 1), (3, 1280, 1280, 13, 128, 2, 13, 1),
+    # less than one pair per expert, with the sums of the sorted tiles
+    (3, 256, 512, 20, 256, 8, 9, 2), ((2, 3), 512, 256, 17, 64, 3, 0, 2), ((3, 2), 1792, 256, 31, 128, 4, 124, 2)])
+def test_moe_pairs_that_find_their_expert_group(wtype, H, I, T, E, k, shared, same_as):
+    """MoE pairs whose workgroups find the pairs that share an expert give the bits of the form they stand in for: one GEMV row per
+    pair (1) or the sorted tiles (2).  shared = how many slots name expert 3, so that some experts have one, exactly a group's,
+    one more and many pairs; invalid ids among them; against the oracle"""
+    wtype, wdown = wtype if isinstance(wtype, tuple) else (wtype, wtype)
+    rng = synth.rng_for(9, 7300 + wtype + 5 * wdown + T + H + I + E)
+    L = _lib.lib()
+    Wg, Wu, Wd = (synth.make_weight(rng, wt, E * n, K).reshape(E, n, K // 256, -1) for wt, n, K in ((wtype, I, H), (wtype, I, H), (wdown, H, I)))
+    g, u, d = (ql.PackedKExperts(wt, torch.from_numpy(W)) for wt, W in ((wtype, Wg), (wtype, Wu), (wdown, Wd)))
     ids = rng.integers(0, E, size=(T, k)).astype(np.int32)
     ids.reshape(-1)[:shared] = 3
     ids[T - 1, k - 1], ids[0, k - 1] = -1, E
     w = rng.random((T, k)).astype(np.float32)
-    x = to_dev(synth.make_x_fp32(rng, T, H))
-    announce("moe groups", wtype, T, E, k, shared)
-    y = ql.moe_ffn_kq(g, u, d, x, to_dev(ids), to_dev(w)).cpu().numpy()
-    assert L.mllm_hip_moe_kq_set_path(1) == 0
+    xf = synth.make_x_fp32(rng, T, H)
+    bits, xb = synth.make_x_bf16(rng, T, H)
+    announce("moe groups", wtype, wdown, H, I, T, E, k, shared)
+    run = lambda: [ql.moe_ffn_kq(g, u, d, x, to_dev(ids), to_dev(w)) for x in (to_dev(xf), bf16_dev(bits))]  # noqa: E731
+    y = run()
+    assert L.mllm_hip_moe_kq_set_path(same_as) == 0
     try:
-        y1 = ql.moe_ffn_kq(g, u, d, x, to_dev(ids), to_dev(w)).cpu().numpy()
+        y1 = run()
     finally:
         assert L.mllm_hip_moe_kq_set_path(0) == 0
-    assert rel_l2(y, y1) < 1e-5, rel_l2(y, y1)
+    assert torch.equal(y[0], y1[0]) and torch.equal(y[1], y1[1])
+    assert rel_l2(y[0].cpu().numpy(), orc.moe_ffn_kq(xf, ids, w, Wg, Wu, Wd, wtype, wtype_down=wdown)) < 1e-3
+
+
+def _fma(a, b, c):
+    """fp32 fma: the product is exact in 64 bits, the sum rounded there first (a tie of the second rounding: once in 2^29)"""
+    a, b, c = (np.asarray(v, np.float64) for v in (a, b, c))
+    return (a * b + c).astype(np.float32)
+
+
+def _moe_tile_sums(x, W, wtype):
+    """codes [M, K] x W [N, K/256, block] in the fp32 order of the MoE tiles (kquant_rows.h): every sub-block of 32 (Q6_K: unit of
+    16) scaled on its own, a chain per lane group over a slice, lane groups pairwise, slices in order"""
+    codes, d, _ = orc.quantize_rows_q8_K(x)
+    (M, K), N = codes.shape, W.shape[0]
+    nsb, f32 = K // 256, np.float32
+    half = lambda a: np.ascontiguousarray(a).view(np.float16).astype(f32)[..., 0]  # noqa: E731
+    if wtype == 2:
+        sc12, qs, dw, dmin = W[:, :, 4:16].astype(np.int32), W[:, :, 16:144].reshape(N, nsb, 4, 32), half(W[:, :, 0:2]), half(W[:, :, 2:4])
+        q = np.stack([qs & 15, qs >> 4], axis=3).reshape(N, nsb, 8, 32).astype(np.int32)
+        lo, hi = sc12[:, :, 0:4], sc12[:, :, 4:8]
+        sc = np.concatenate([lo & 63, (sc12[:, :, 8:] & 15) | ((lo >> 6) << 4)], axis=2)
+        mn = np.concatenate([hi & 63, (sc12[:, :, 8:] >> 4) | ((hi >> 6) << 4)], axis=2)
+        size, groups, steps = 32, 2, [(4 * j + h, 2) for j in range(2) for h in range(2)]  # sub-block of group 0, step to the next group's
+    else:
+        l, h = W[:, :, :128].reshape(N, nsb, 2, 2, 32).astype(np.int32), W[:, :, 128:192].reshape(N, nsb, 2, 32).astype(np.int32)
+        sc, dw = W[:, :, 192:208].view(np.int8).astype(np.int32), half(W[:, :, 208:210])
+        q = np.stack([(l[:, :, :, 0] & 15) | (h & 3) << 4, (l[:, :, :, 1] & 15) | (h >> 2 & 3) << 4, (l[:, :, :, 0] >> 4) | (h >> 4 & 3) << 4,
+                      (l[:, :, :, 1] >> 4) | (h >> 6) << 4], axis=3).reshape(N, nsb, 16, 16) - 32
+        size, groups, steps = 16, 4, [(8 * j + 4 * h, 1) for j in range(2) for h in range(2)]
+    c = codes.astype(np.int32).reshape(M, nsb, 256 // size, size)
+    D, X = np.einsum("nbse,mbse->bsmn", q, c), c.sum(-1)
+    slices = 1
+    while slices < 8 and nsb > 5 * slices:
+        slices *= 2
+    per, total = -(-nsb // slices), None
+    for s in range(0, nsb, per):
+        acc = [np.zeros((M, N), f32) for _ in range(groups)]
+        for b in range(s, min(nsb, s + per)):
+            dx = d[:, b, None]
+            for first, stride in steps:
+                for i in range(groups):
+                    k = first + stride * i
+                    acc[i] = _fma((dw[:, b] * sc[:, b, k].astype(f32)) * dx, D[b, k], acc[i])
+                    if wtype == 2:
+                        acc[i] = _fma(-((dmin[:, b] * mn[:, b, k].astype(f32)) * dx), X[:, b, k, None], acc[i])
+        v = acc[0] + acc[1] if groups == 2 else (acc[0] + acc[1]) + (acc[2] + acc[3])
+        total = v if total is None else total + v
+    return total
+
+
+@pytest.mark.parametrize("wtype,wdown,E,H,I", [(2, 2, 8, 2816, 512), (3, 3, 8, 2816, 512), (2, 3, 40, 1536, 512), (3, 2, 40, 512, 1536)])
+def test_moe_tiles_keep_the_order_of_their_sums(wtype, wdown, E, H, I):
+    """eight-row tiles, sorted (8 experts) and found by the workgroups (40): bit for bit the stated fp32 order, through SiLU, the
+    second quantization and the weighted sum (one pair per token)"""
+    T, rng = 24, synth.rng_for(9, 7500 + wtype + 5 * wdown + E)
+    Wg, Wu, Wd = (synth.make_weight(rng, wt, E * n, K).reshape(E, n, K // 256, -1) for wt, n, K in ((wtype, I, H), (wtype, I, H), (wdown, H, I)))
+    g, u, d = (ql.PackedKExperts(wt, torch.from_numpy(W)) for wt, W in ((wtype, Wg), (wtype, Wu), (wdown, Wd)))
+    ids, w, x = rng.integers(0, E, size=(T, 1)).astype(np.int32), rng.random((T, 1)).astype(np.float32), synth.make_x_fp32(rng, T, H)
+    announce("moe tile order", wtype, wdown, E, H, I)
+    y = ql.moe_ffn_kq(g, u, d, to_dev(x), to_dev(ids), to_dev(w)).cpu().numpy()
+    want = np.empty_like(y)
+    for e in np.unique(ids):
+        rows = np.nonzero(ids[:, 0] == e)[0]
+        h = ql.silu_mul(to_dev(_moe_tile_sums(x[rows], Wg[e], wtype)), to_dev(_moe_tile_sums(x[rows], Wu[e], wtype))).cpu().numpy()
+        want[rows] = _moe_tile_sums(h, Wd[e], wdown) * w[rows]
+    assert np.array_equal(y, want)
 
 
 @pytest.mark.parametrize("wtype", [2, 3])
