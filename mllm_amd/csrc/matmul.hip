@@ -29,6 +29,14 @@ struct MMArgs {
   int vecA, vecB;      // aligned 16-byte loads of whole rows (base, leading dimension and batch stride all multiples of 16 bytes)
 };
 
+// The grid of a launch of `total` workgroups (below 2^31): HIP counts the work-items of a dimension in 32 bits, which 2^24 workgroups of
+// 256 threads no longer fit, so that more than 2^21 are rows of 2^21 (a multiple of the XCDs).  The last row may reach past the end.
+static dim3 mm_grid(int64_t total) {
+  constexpr int64_t ROW = 1 << 21;
+  return total <= ROW ? dim3((unsigned)total) : dim3((unsigned)ROW, (unsigned)((total + ROW - 1) / ROW));
+}
+__device__ __forceinline__ int mm_block() { return (int)(blockIdx.y * gridDim.x + blockIdx.x); }
+
 template <int DT>
 struct MMElem {
   using type = uint16_t;
@@ -166,7 +174,8 @@ __global__ __launch_bounds__(256, (TM * TN == 4 && DT != MLLM_HIP_F32) ? 4 : 1) 
   const int wm = wave >> 1, wn = wave & 1, r = lane & 31, h = lane >> 5;
   const int KT = (a.K + 31) / 32;
   const int tilesM = (a.M + BM - 1) / BM, tilesN = (a.N + BN - 1) / BN, tiles = tilesM * tilesN;
-  const int t = xcd_run(blockIdx.x, gridDim.x), z = t / tiles, in = t - z * tiles;
+  if (mm_block() >= tiles * a.batch) return;  // (uniform)
+  const int t = xcd_run(mm_block(), tiles * a.batch), z = t / tiles, in = t - z * tiles;
   const int n0 = in / tilesM * BN, m0 = in % tilesM * BM;
   const E* A = reinterpret_cast<const E*>(a.A) + z * a.sA;
   const E* B = reinterpret_cast<const E*>(a.B) + z * a.sB;
@@ -277,7 +286,8 @@ __global__ __launch_bounds__(MMR_WAVES * 64) void matmul_rows_kernel(MMArgs a, i
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lpr = 1 << lpr_log2, rpw = 64 >> lpr_log2, ncols = lpr * VE;
   const int col = (lane & (lpr - 1)) * VE, sub = lane >> lpr_log2;
-  const int b = xcd_run(blockIdx.x, gridDim.x), z = b / col_blocks, nb = (b - z * col_blocks) * ncols;
+  if (mm_block() >= col_blocks * a.batch) return;  // (uniform)
+  const int b = xcd_run(mm_block(), col_blocks * a.batch), z = b / col_blocks, nb = (b - z * col_blocks) * ncols;
   const int n0 = nb + col, nc = min(n0, a.N - VE);  // (N % VE == 0: a lane's columns are all inside or all outside)
   const E* A = reinterpret_cast<const E*>(a.A) + z * a.sA;
   const E* B = reinterpret_cast<const E*>(a.B) + z * a.sB + nc;
@@ -351,7 +361,7 @@ static bool launch_matmul_rows(const MMArgs& a, hipStream_t st, int* rc) {
   const int ncols = VE << lg;
   const int64_t cols = (a.N + ncols - 1) / ncols;
   if (cols * a.batch > 0x7fffffff) return false;
-  const dim3 grid((unsigned)(cols * a.batch));
+  const dim3 grid = mm_grid(cols * a.batch);
   const size_t lds = (size_t)MMR_WAVES * mr * ncols * sizeof(float);
   if (mr == 1) hipLaunchKernelGGL((matmul_rows_kernel<DT, 1>), grid, dim3(MMR_WAVES * 64), lds, st, a, lg, (int)cols);
   else if (mr == 2) hipLaunchKernelGGL((matmul_rows_kernel<DT, 2>), grid, dim3(MMR_WAVES * 64), lds, st, a, lg, (int)cols);
@@ -371,7 +381,8 @@ __global__ __launch_bounds__(256) void matmul_dots_kernel(MMArgs a, int g_log2, 
   constexpr int VE = 16 / (int)sizeof(E);
   __shared__ float s_out[MR][256 * UB / 4];  // at least four lanes per row of B
   const int tid = threadIdx.x, g = 1 << g_log2, sub = tid & (g - 1), groups = 256 >> g_log2, grp = tid >> g_log2, per = groups * UB;
-  const int b = xcd_run(blockIdx.x, gridDim.x), z = b / col_blocks, n0 = (b - z * col_blocks) * per;
+  if (mm_block() >= col_blocks * a.batch) return;  // (uniform)
+  const int b = xcd_run(mm_block(), col_blocks * a.batch), z = b / col_blocks, n0 = (b - z * col_blocks) * per;
   const E* A = reinterpret_cast<const E*>(a.A) + z * a.sA;
   const E* B = reinterpret_cast<const E*>(a.B) + z * a.sB;
   E* C = reinterpret_cast<E*>(a.C) + z * a.sC;
@@ -432,7 +443,7 @@ static bool launch_matmul_dots(const MMArgs& a, hipStream_t st, int* rc) {
   auto go = [&](auto kern, int ub) {
     const int per = (256 >> lg) * ub;
     const int64_t cols = ((int64_t)a.N + per - 1) / per;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(cols * a.batch)), dim3(256), 0, st, a, lg, (int)cols);
+    hipLaunchKernelGGL(kern, mm_grid(cols * a.batch), dim3(256), 0, st, a, lg, (int)cols);
     return (int)hipGetLastError();
   };
   // four rows of B per group where that leaves 128 workgroups or more, else one (8 x 4 x 8000 x 128 fp32: 9.8 us / 13.1; 2 x 4 x
@@ -481,7 +492,7 @@ static int launch_matmul(const MMArgs& a, hipStream_t st) {
       p.B = reinterpret_cast<const E*>(a.B) + z * a.sB;
       p.C = reinterpret_cast<E*>(a.C) + z * a.sC;
       p.batch = std::min(most, a.batch - z);
-      hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * p.batch)), dim3(256), 0, st, p);
+      hipLaunchKernelGGL(kern, mm_grid(tiles * p.batch), dim3(256), 0, st, p);
     }
     return (int)hipGetLastError();
   };

@@ -106,3 +106,24 @@ def test_matmul_forms_at_their_edges(batch, M, N, K, ta, tb, dtype):
     a, b = torch.from_numpy(a), torch.from_numpy(b)
     want = torch.matmul(a.transpose(1, 2).contiguous() if ta else a, b.transpose(1, 2).contiguous() if tb else b).to(td)
     assert torch.equal(c, want)
+
+
+def test_matmul_batches_beyond_a_grid_dimension():
+    """more workgroups than a grid dimension's 32 bits of work-items hold (2^24 of 256 threads, 2^22 of 1024), once per kernel: tiles,
+    dot products, values; small integers, exact"""
+    n = (1 << 24) + 3
+    g = torch.Generator(device="cuda").manual_seed(5)
+    ints = lambda *shape, top=8, dtype=torch.float32: torch.randint(0, top, shape, device="cuda", generator=g, dtype=torch.int8).to(dtype)  # noqa: E731
+    a, b = ints(n, 1, 1), ints(n, 1, 1)
+    announce("matmul of 2^24 + 3 products")
+    assert torch.equal(ql.matmul(a, b), a * b)
+    a, b = ints(n, 1, 4), ints(n, 1, 4)
+    announce("matmul of 2^24 + 3 dot products")
+    assert torch.equal(ql.matmul(a, b, False, True), (a * b).sum(-1, keepdim=True))
+    del a, b
+    n = (1 << 22) + 3
+    a, b = ints(n, 1, 256, top=2, dtype=torch.bfloat16), ints(256, 8, top=2, dtype=torch.bfloat16)  # sums up to 256: exact in bf16
+    announce("matmul of 2^22 + 3 value products")
+    c = ql.matmul(a, b)
+    for i in range(0, n, 1 << 20):
+        assert torch.equal(c[i:i + (1 << 20), 0].float(), torch.mm(a[i:i + (1 << 20), 0].float(), b.float()))
