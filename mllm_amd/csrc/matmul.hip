@@ -36,6 +36,11 @@ static dim3 mm_grid(int64_t total) {
   return total <= ROW ? dim3((unsigned)total) : dim3((unsigned)ROW, (unsigned)((total + ROW - 1) / ROW));
 }
 __device__ __forceinline__ int mm_block() { return (int)(blockIdx.y * gridDim.x + blockIdx.x); }
+// n / d for the same n in every lane; inv = mm_inv(d, n's bound): a division instruction sequence costs a small product as much as a K step
+static uint32_t mm_inv(int64_t d, int64_t bound) { return d > 1 && bound <= 65536 ? (uint32_t)(((1ull << 32) + d - 1) / d) : 0u; }
+__device__ __forceinline__ int mm_div(int n, int d, uint32_t inv) {
+  return d == 1 ? n : inv ? (int)__umulhi((uint32_t)n, inv) : n / d;  // (n, d < 2^16: exact)
+}
 
 template <int DT>
 struct MMElem {
@@ -53,8 +58,10 @@ struct MMElem<MLLM_HIP_F32> {
 // thread and vector, which makes one dword of LDS per row.
 // Whole tiles load whole vectors whatever the alignment of the rows (odd row lengths among them); rows past the end repeat the
 // last ones (their results are never stored).  A K step that ends behind K, and a last tile of rows that are not a multiple of
-// the vector in a [K][rows] tensor, load element by element with zeros outside.
-template <typename E, int ROWS, bool CONTIG_K>
+// the vector in a [K][rows] tensor, load element by element with zeros outside; VECTORS: the shape has neither but K steps whose
+// vectors lie inside or outside as a whole (mm_vectors below), and no element by element code: the short products that this is for
+// are bound by their few K steps (bf16 1000 x 8 x 8 x 8: 4.7 us by elements, 3.3; 8 x 800 x 64 x 200 5.7 / 4.8).
+template <typename E, int ROWS, bool CONTIG_K, bool VECTORS>
 struct MMTile {
   static constexpr int VE = 16 / (int)sizeof(E);
   static constexpr bool KROWS = !CONTIG_K && sizeof(E) == 4;   // [k][row] in LDS
@@ -86,7 +93,7 @@ struct MMTile {
     else k = idx / (ROWS / VE), r = (idx % (ROWS / VE)) * VE;
   }
   __device__ __forceinline__ void start(const E* __restrict__ X, int row0, int rows, int K) {
-    whole = CONTIG_K || (rows >= RV && (row0 + ROWS <= rows || rows % RV == 0));  // (the same in every thread)
+    whole = CONTIG_K || VECTORS || (rows >= RV && (row0 + ROWS <= rows || rows % RV == 0));  // (the same in every thread)
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
       int r, k;
@@ -95,19 +102,33 @@ struct MMTile {
       else p[c] = X + (int64_t)k * rows + (whole ? min(row0 + r, rows - RV) : 0);
     }
   }
+  static __device__ __forceinline__ u32x4 vector(const E* __restrict__ at, int rows) {
+    u32x4 q;
+    if constexpr (PAIRS) {
+      u32x2 lo, hi;
+      __builtin_memcpy(&lo, at, 8);
+      __builtin_memcpy(&hi, at + rows, 8);
+      q = u32x4{lo.x, lo.y, hi.x, hi.y};
+    } else {
+      __builtin_memcpy(&q, at, 16);
+    }
+    return q;
+  }
   __device__ __forceinline__ void load(const E* __restrict__ X, int row0, int k0, int rows, int K) {
-    if (whole && k0 + 32 <= K) {
+    if (VECTORS ? k0 + 32 <= K : whole && k0 + 32 <= K) {
+      const int64_t step = CONTIG_K ? (int64_t)k0 : (int64_t)k0 * rows;
+#pragma unroll
+      for (int c = 0; c < NV; ++c) v[c] = vector(p[c] + step, rows);
+      return;
+    }
+    if constexpr (VECTORS) {
       const int64_t step = CONTIG_K ? (int64_t)k0 : (int64_t)k0 * rows;
 #pragma unroll
       for (int c = 0; c < NV; ++c) {
-        if constexpr (PAIRS) {
-          u32x2 lo, hi;
-          __builtin_memcpy(&lo, p[c] + step, 8);
-          __builtin_memcpy(&hi, p[c] + step + rows, 8);
-          v[c] = u32x4{lo.x, lo.y, hi.x, hi.y};
-        } else {
-          __builtin_memcpy(&v[c], p[c] + step, 16);
-        }
+        int r, k;
+        place(c, r, k);
+        v[c] = u32x4{0u, 0u, 0u, 0u};
+        if (k0 + k < K) v[c] = vector(p[c] + step, rows);
       }
       return;
     }
@@ -160,23 +181,23 @@ struct MMTile {
 // three (4096 x 4096 x 4096 bf16: 236 -> 180 us).
 //   (heads x rows x keys x d) fp32 8 x 3108 x 777 x 128: scores 80 -> 59 us, values 97 -> 65; bf16 33 -> 23, 70 -> 26 (odd row lengths
 //   loaded element by element and transposed through 16 two-byte LDS stores before)
-template <int DT, bool TA, bool TB, int TM, int TN>
-__global__ __launch_bounds__(256, (TM * TN == 4 && DT != MLLM_HIP_F32) ? 4 : 1) void matmul_kernel(MMArgs a) {
+template <int DT, bool TA, bool TB, int TM, int TN, bool VECTORS>
+__global__ __launch_bounds__(256, (TM * TN == 4 && DT != MLLM_HIP_F32) ? 4 : 1) void matmul_kernel(MMArgs a, int tiles, int tilesM, uint32_t inv_tiles, uint32_t inv_tilesM) {
   using E = typename MMElem<DT>::type;
   constexpr int BM = 64 * TM, BN = 64 * TN;
   // A is [M][K], or [K][M] when transposed; B is [K][N], or [N][K] when transposed
-  typedef MMTile<E, BM, !TA> TileA;
-  typedef MMTile<E, BN, TB> TileB;
+  typedef MMTile<E, BM, !TA, VECTORS> TileA;
+  typedef MMTile<E, BN, TB, VECTORS> TileB;
   __shared__ __align__(16) E sA[TileA::SIZE];
   __shared__ __align__(16) E sB[TileB::SIZE];
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave >> 1, wn = wave & 1, r = lane & 31, h = lane >> 5;
   const int KT = (a.K + 31) / 32;
-  const int tilesM = (a.M + BM - 1) / BM, tilesN = (a.N + BN - 1) / BN, tiles = tilesM * tilesN;
-  if (mm_block() >= tiles * a.batch) return;  // (uniform)
-  const int t = xcd_run(mm_block(), tiles * a.batch), z = t / tiles, in = t - z * tiles;
-  const int n0 = in / tilesM * BN, m0 = in % tilesM * BM;
+  const int total = tiles * a.batch, b = mm_block();
+  if (b >= total) return;  // (uniform)
+  const int t = xcd_run(b, total), z = mm_div(t, tiles, inv_tiles), in = t - z * tiles;
+  const int tn = mm_div(in, tilesM, inv_tilesM), n0 = tn * BN, m0 = (in - tn * tilesM) * BM;
   const E* A = reinterpret_cast<const E*>(a.A) + z * a.sA;
   const E* B = reinterpret_cast<const E*>(a.B) + z * a.sB;
   E* C = reinterpret_cast<E*>(a.C) + z * a.sC;
@@ -277,7 +298,7 @@ __device__ __forceinline__ float mm_to_f32(typename MMElem<DT>::type e) {
 }
 constexpr int MMR_WAVES = 16;
 template <int DT, int MR>
-__global__ __launch_bounds__(MMR_WAVES * 64) void matmul_rows_kernel(MMArgs a, int lpr_log2, int col_blocks) {
+__global__ __launch_bounds__(MMR_WAVES * 64) void matmul_rows_kernel(MMArgs a, int lpr_log2, int col_blocks, uint32_t inv_blocks) {
   using E = typename MMElem<DT>::type;
   constexpr int VE = 16 / (int)sizeof(E), UB = 4;
   typedef E AV __attribute__((ext_vector_type(UB)));
@@ -286,8 +307,9 @@ __global__ __launch_bounds__(MMR_WAVES * 64) void matmul_rows_kernel(MMArgs a, i
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lpr = 1 << lpr_log2, rpw = 64 >> lpr_log2, ncols = lpr * VE;
   const int col = (lane & (lpr - 1)) * VE, sub = lane >> lpr_log2;
-  if (mm_block() >= col_blocks * a.batch) return;  // (uniform)
-  const int b = xcd_run(mm_block(), col_blocks * a.batch), z = b / col_blocks, nb = (b - z * col_blocks) * ncols;
+  const int total = col_blocks * a.batch;
+  if (mm_block() >= total) return;  // (uniform)
+  const int b = xcd_run(mm_block(), total), z = mm_div(b, col_blocks, inv_blocks), nb = (b - z * col_blocks) * ncols;
   const int n0 = nb + col, nc = min(n0, a.N - VE);  // (N % VE == 0: a lane's columns are all inside or all outside)
   const E* A = reinterpret_cast<const E*>(a.A) + z * a.sA;
   const E* B = reinterpret_cast<const E*>(a.B) + z * a.sB + nc;
@@ -303,7 +325,7 @@ __global__ __launch_bounds__(MMR_WAVES * 64) void matmul_rows_kernel(MMArgs a, i
   auto mac = [&](u32x4 bv, int m, E e) {
     const float am = mm_to_f32<DT>(e);
 #pragma unroll
-    for (int j = 0; j < VE; j++) acc[m][j] = fmaf(am, mm_to_f32<DT>(MMTile<E, 64, true>::elem(bv, j)), acc[m][j]);
+    for (int j = 0; j < VE; j++) acc[m][j] = fmaf(am, mm_to_f32<DT>(MMTile<E, 64, true, false>::elem(bv, j)), acc[m][j]);
   };
   const int kstep = MMR_WAVES * rpw * UB;
   int k = (wave * rpw + sub) * UB;
@@ -362,10 +384,11 @@ static bool launch_matmul_rows(const MMArgs& a, hipStream_t st, int* rc) {
   const int64_t cols = (a.N + ncols - 1) / ncols;
   if (cols * a.batch > 0x7fffffff) return false;
   const dim3 grid = mm_grid(cols * a.batch);
+  const uint32_t inv = mm_inv(cols, cols * a.batch);
   const size_t lds = (size_t)MMR_WAVES * mr * ncols * sizeof(float);
-  if (mr == 1) hipLaunchKernelGGL((matmul_rows_kernel<DT, 1>), grid, dim3(MMR_WAVES * 64), lds, st, a, lg, (int)cols);
-  else if (mr == 2) hipLaunchKernelGGL((matmul_rows_kernel<DT, 2>), grid, dim3(MMR_WAVES * 64), lds, st, a, lg, (int)cols);
-  else hipLaunchKernelGGL((matmul_rows_kernel<DT, 4>), grid, dim3(MMR_WAVES * 64), lds, st, a, lg, (int)cols);
+  if (mr == 1) hipLaunchKernelGGL((matmul_rows_kernel<DT, 1>), grid, dim3(MMR_WAVES * 64), lds, st, a, lg, (int)cols, inv);
+  else if (mr == 2) hipLaunchKernelGGL((matmul_rows_kernel<DT, 2>), grid, dim3(MMR_WAVES * 64), lds, st, a, lg, (int)cols, inv);
+  else hipLaunchKernelGGL((matmul_rows_kernel<DT, 4>), grid, dim3(MMR_WAVES * 64), lds, st, a, lg, (int)cols, inv);
   *rc = (int)hipGetLastError();
   return true;
 }
@@ -376,13 +399,14 @@ static bool launch_matmul_rows(const MMArgs& a, hipStream_t st, int* rc) {
 // fp32: 8 x 4 x 8000 x 128 13.7 -> 9.8 us (3.3 TB/s), 8 x 1 x 8000 x 128 13.5 -> 5.5; bf16: 8 x 1 x 8000 x 128 5.6 -> 4.2.  1 x 1 x 64 x 2048 (router logits): fp32 52.6 -> 11.3,
 // bf16 21.8 -> 5.4.
 template <int DT, int MR, int UB>
-__global__ __launch_bounds__(256) void matmul_dots_kernel(MMArgs a, int g_log2, int col_blocks) {
+__global__ __launch_bounds__(256) void matmul_dots_kernel(MMArgs a, int g_log2, int col_blocks, uint32_t inv_blocks) {
   using E = typename MMElem<DT>::type;
   constexpr int VE = 16 / (int)sizeof(E);
   __shared__ float s_out[MR][256 * UB / 4];  // at least four lanes per row of B
   const int tid = threadIdx.x, g = 1 << g_log2, sub = tid & (g - 1), groups = 256 >> g_log2, grp = tid >> g_log2, per = groups * UB;
-  if (mm_block() >= col_blocks * a.batch) return;  // (uniform)
-  const int b = xcd_run(mm_block(), col_blocks * a.batch), z = b / col_blocks, n0 = (b - z * col_blocks) * per;
+  const int total = col_blocks * a.batch;
+  if (mm_block() >= total) return;  // (uniform)
+  const int b = xcd_run(mm_block(), total), z = mm_div(b, col_blocks, inv_blocks), n0 = (b - z * col_blocks) * per;
   const E* A = reinterpret_cast<const E*>(a.A) + z * a.sA;
   const E* B = reinterpret_cast<const E*>(a.B) + z * a.sB;
   E* C = reinterpret_cast<E*>(a.C) + z * a.sC;
@@ -402,9 +426,9 @@ __global__ __launch_bounds__(256) void matmul_dots_kernel(MMArgs a, int g_log2, 
     for (int u = 0; u < UB; u++)
 #pragma unroll
       for (int j = 0; j < VE; j++) {
-        const float bf = mm_to_f32<DT>(MMTile<E, 64, true>::elem(bv[u], j));
+        const float bf = mm_to_f32<DT>(MMTile<E, 64, true, false>::elem(bv[u], j));
 #pragma unroll
-        for (int m = 0; m < MR; m++) acc[u][m] = fmaf(mm_to_f32<DT>(MMTile<E, 64, true>::elem(av[m], j)), bf, acc[u][m]);
+        for (int m = 0; m < MR; m++) acc[u][m] = fmaf(mm_to_f32<DT>(MMTile<E, 64, true, false>::elem(av[m], j)), bf, acc[u][m]);
       }
   }
 #pragma unroll
@@ -443,7 +467,7 @@ static bool launch_matmul_dots(const MMArgs& a, hipStream_t st, int* rc) {
   auto go = [&](auto kern, int ub) {
     const int per = (256 >> lg) * ub;
     const int64_t cols = ((int64_t)a.N + per - 1) / per;
-    hipLaunchKernelGGL(kern, mm_grid(cols * a.batch), dim3(256), 0, st, a, lg, (int)cols);
+    hipLaunchKernelGGL(kern, mm_grid(cols * a.batch), dim3(256), 0, st, a, lg, (int)cols, mm_inv(cols, cols * a.batch));
     return (int)hipGetLastError();
   };
   // four rows of B per group where that leaves 128 workgroups or more, else one (8 x 4 x 8000 x 128 fp32: 9.8 us / 13.1; 2 x 4 x
@@ -471,6 +495,17 @@ static bool matmul_large_tile(const MMArgs& a) {
   return !TA && TB ? 30. + 17. * large < 9. + 9.3 * small : 40. + 36. * large < 11.7 * small;
 }
 
+// A short product all of whose vectors lie inside K and the rows, or outside K, as a whole (whatever the alignment in memory).  From K =
+// 512 on the two are even (1000 x 1000 x 1000 bf16 17.1 / 17.1 us, fp32 26.4 / 26.4 to 27.4); whole K steps gain 0.1 to 0.3 us of a
+// launch (64 x 128 x 128 x 128 bf16 4.44 -> 4.21) and nothing in many rounds (fp32 8 x 3108 x 777 x 128: 58.4 / 59.8).
+template <int DT, bool TA, bool TB>
+static bool mm_vectors(const MMArgs& a) {
+  constexpr bool f32 = DT == MLLM_HIP_F32;
+  if (a.K >= 512 || (a.K % 32 == 0 && (double)((a.M + 63) / 64) * ((a.N + 63) / 64) * a.batch > 1024)) return false;
+  auto fits = [&](bool contig_k, int rows) { return contig_k ? a.K % (f32 ? 4 : 8) == 0 : rows % 4 == 0 && (f32 || a.K % 2 == 0); };
+  return fits(!TA, a.M) && fits(TB, a.N);
+}
+
 template <int DT, bool TA, bool TB>
 static int launch_matmul(const MMArgs& a, hipStream_t st) {
   if constexpr (!TA && !TB) {
@@ -482,7 +517,7 @@ static int launch_matmul(const MMArgs& a, hipStream_t st) {
     if (launch_matmul_dots<DT>(a, st, &rc)) return rc;
   }
   auto go = [&](auto kern, int side) {
-    const int64_t tiles = (int64_t)((a.M + side - 1) / side) * ((a.N + side - 1) / side);
+    const int64_t tilesM = (a.M + side - 1) / side, tiles = tilesM * ((a.N + side - 1) / side);
     if (tiles > 0x7fffffff) return MLLM_HIP_E_SHAPE;
     const int most = (int)std::min<int64_t>(a.batch, 0x7fffffff / tiles);  // batch entries per launch
     using E = typename MMElem<DT>::type;
@@ -492,12 +527,13 @@ static int launch_matmul(const MMArgs& a, hipStream_t st) {
       p.B = reinterpret_cast<const E*>(a.B) + z * a.sB;
       p.C = reinterpret_cast<E*>(a.C) + z * a.sC;
       p.batch = std::min(most, a.batch - z);
-      hipLaunchKernelGGL(kern, mm_grid(tiles * p.batch), dim3(256), 0, st, p);
+      hipLaunchKernelGGL(kern, mm_grid(tiles * p.batch), dim3(256), 0, st, p, (int)tiles, (int)tilesM, mm_inv(tiles, tiles * p.batch), mm_inv(tilesM, tiles));
     }
     return (int)hipGetLastError();
   };
-  if (matmul_large_tile<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 2, 2>, 128);
-  return go(matmul_kernel<DT, TA, TB, 1, 1>, 64);
+  if (matmul_large_tile<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 2, 2, false>, 128);
+  if (mm_vectors<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 1, 1, true>, 64);
+  return go(matmul_kernel<DT, TA, TB, 1, 1, false>, 64);
 }
 
 template <int DT>

@@ -108,6 +108,21 @@ def test_matmul_forms_at_their_edges(batch, M, N, K, ta, tb, dtype):
     assert torch.equal(c, want)
 
 
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("batch,M,N,K", [(16, 16, 16, 16), (1000, 8, 8, 8), (1, 300, 132, 40), (3, 68, 60, 24), (2, 64, 128, 504), (5, 12, 8, 56)])
+def test_short_matmuls_of_whole_vectors(batch, M, N, K, ta, tb, dtype):
+    """K steps that end behind K with every vector inside or outside it, rows that end inside a tile: exact as above"""
+    rng = synth.rng_for(6, 3000 + batch + M + N + K)
+    td = torch.float32 if dtype == "fp32" else torch.bfloat16
+    a = torch.from_numpy(rng.integers(-8, 9, (batch, K, M) if ta else (batch, M, K)).astype(np.float32))
+    b = torch.from_numpy(rng.integers(-8, 9, (batch, N, K) if tb else (batch, K, N)).astype(np.float32))
+    announce("matmul of whole vectors %s %s ta=%d tb=%d" % (dtype, (batch, M, N, K), ta, tb))
+    c = ql.matmul(a.to(td).cuda(), b.to(td).cuda(), ta, tb).cpu()
+    want = torch.matmul(a.transpose(1, 2).contiguous() if ta else a, b.transpose(1, 2).contiguous() if tb else b).to(td)
+    assert torch.equal(c, want)
+
+
 def test_matmul_batches_beyond_a_grid_dimension():
     """more workgroups than a grid dimension's 32 bits of work-items hold (2^24 of 256 threads, 2^22 of 1024), once per kernel: tiles,
     dot products, values; small integers, exact"""
