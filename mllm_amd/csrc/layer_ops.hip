@@ -1281,25 +1281,32 @@ MLLM_API int mllm_hip_softmax_ws(const float* x, float* y, int64_t rows, int64_t
   return (int)hipGetLastError();
 }
 
-static int topk_pieces(int64_t rows, int64_t len, int k) {
+// Pieces of a row, 0 where a workgroup per row is the better form.  vec: rows of whole aligned 16-byte vectors.  The largest 50, us, a
+// workgroup per row / pieces: 8 rows of 4100 elements 20.9 / 14.8, of 8192 26.0 / 15.0, of 151 936 113 / 16.6; 512 rows of 8192 29.0 / 18.8.
+// Element by element the pieces load slower than the row's workgroup, which holds up to 8192 elements in registers: 8 rows of 4097
+// 12.6 / 16.6, of 8191 14.1 / 15.5, of 8193 26.7 / 15.3; where the rows need a second round of workgroups pieces pay there too (300
+// rows of 4097: 0.87 of the time).
+static int topk_pieces(int64_t rows, int64_t len, int k, bool vec) {
   if (len <= TOPK_SPLIT_LEN || rows > TOPK_SPLIT_ROWS || k < 1 || k > TOPK_SPLIT_K || len > 0x7fffffff) return 0;
+  if (!vec && len <= 8192 && rows <= 256) return 0;
   const int64_t pieces = (len + TOPK_PIECE - 1) / TOPK_PIECE;
   return pieces * k <= 256 * TOPK_MERGE_R ? (int)pieces : 0;
 }
 MLLM_API size_t mllm_hip_topk_workspace_bytes(int64_t rows, int64_t len, int k) {
   if (rows <= 0 || len <= 0) return 0;
-  return (size_t)rows * topk_pieces(rows, len, k) * (k > 0 ? k : 0) * sizeof(unsigned long long);
+  return (size_t)rows * topk_pieces(rows, len, k, len % 4 == 0) * (k > 0 ? k : 0) * sizeof(unsigned long long);
 }
 MLLM_API int mllm_hip_topk_ws(const float* x, float* values, int32_t* indices, int64_t rows, int64_t len, int k, int largest, int sorted,
                               void* workspace, void* stream) {
-  const int pieces = workspace && rows > 0 && len > 0 ? topk_pieces(rows, len, k) : 0;
+  const bool vec = len % 4 == 0 && ((uintptr_t)x & 15) == 0;
+  const int pieces = workspace && rows > 0 && len > 0 ? topk_pieces(rows, len, k, vec) : 0;
   if (!pieces) return mllm_hip_topk(x, values, indices, rows, len, k, largest, sorted, stream);
   if (!x || !values || !indices) return MLLM_HIP_E_BADARG;
   if (reinterpret_cast<uintptr_t>(workspace) % 8) return MLLM_HIP_E_ALIGN;
   const dim3 grid((unsigned)pieces, (unsigned)rows);
   hipStream_t st = (hipStream_t)stream;
   unsigned long long* ws = reinterpret_cast<unsigned long long*>(workspace);
-  if (len % 4 == 0 && ((uintptr_t)x & 15) == 0) hipLaunchKernelGGL(topk_pieces_kernel<4>, grid, dim3(256), 0, st, x, ws, (int)len, k, largest);
+  if (vec) hipLaunchKernelGGL(topk_pieces_kernel<4>, grid, dim3(256), 0, st, x, ws, (int)len, k, largest);
   else hipLaunchKernelGGL(topk_pieces_kernel<1>, grid, dim3(256), 0, st, x, ws, (int)len, k, largest);
   if (pieces * k <= 1024) hipLaunchKernelGGL(topk_merge_kernel<4>, dim3((unsigned)rows), dim3(256), 0, st, x, ws, values, indices, (int)len, pieces * k, k, sorted);
   else hipLaunchKernelGGL(topk_merge_kernel<TOPK_MERGE_R>, dim3((unsigned)rows), dim3(256), 0, st, x, ws, values, indices, (int)len, pieces * k, k, sorted);

@@ -143,6 +143,14 @@ def test_entry_point_rejects_bad_argument(name, idx, bad, code):
     assert rc == code, "%s with argument %d = %r returned %d, expected %d" % (name, idx, bad, rc, code)
 
 
+def test_topk_is_cut_into_pieces_only_where_that_is_faster():
+    """rows without whole vectors of up to 8192 elements stay one workgroup's work while that is one round of workgroups"""
+    room = _lib.lib().mllm_hip_topk_workspace_bytes
+    for rows, ln, k, pieces in ((8, 4096, 50, 0), (8, 4097, 50, 0), (1, 8191, 1, 0), (256, 5001, 128, 0), (257, 4097, 50, 2), (8, 4100, 50, 2), (8, 8192, 50, 2),
+                                (8, 8193, 50, 3), (8, 151936, 128, 38), (512, 151936, 20, 38), (513, 151936, 20, 0), (8, 151936, 129, 0)):
+        assert room(rows, ln, k) == rows * pieces * k * 8, (rows, ln, k)
+
+
 def test_size_helpers_return_zero_for_shapes_they_do_not_take():
     L = _lib.lib()
     assert L.mllm_hip_q_packed_bytes(Q4_0, 64, 48) == 0

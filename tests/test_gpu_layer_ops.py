@@ -310,7 +310,7 @@ def test_softmax_of_rows_cut_into_pieces(rows, ln):
 
 
 @pytest.mark.parametrize("rows,ln,k", [(2, 4096, 8), (3, 4097, 32), (2, 4100, 33), (1, 8193, 64), (2, 20000, 128), (2, 20000, 129), (1, 151936, 128),
-                                       (1, 200003, 128)])
+                                       (1, 200003, 128), (257, 4097, 50)])
 def test_topk_of_rows_cut_into_pieces(rows, ln, k):
     """both orders of the result, a last piece of a few elements, k either side of what the pieces serve, a row whose largest
     elements all fall to one thread (more candidates than are kept), few distinct values"""
