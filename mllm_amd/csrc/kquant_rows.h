@@ -530,7 +530,7 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
 struct KrShape {
   int tiles, waves;
 };
-static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y) {
+static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y, bool quantizes = false) {
   int64_t tiles = 0;
   for (int i = 0; i < a.nparts; i++) tiles += (a.part[i].N + 15) / 16;
   const int S = kr_slices(a.nsb);
@@ -538,6 +538,10 @@ static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y) {
   int tw = (int)std::min<int64_t>(moe ? 4 : 8, (tiles * grid_y + 255) / 256);
   int P = moe ? 1 : std::min(S, tw >= 5 ? 10 / tw : 16 / tw);
   while (P > 1 && (S + P - 2) / (P - 1) == (S + P - 1) / P) P--;
+  // one tile per workgroup that quantizes x itself: waves without a slice share that, two items per thread (up to eight waves; 1024 x 1024
+  // Q6_K at three / four / eight rows 5.8 / 6.3 / 8.9 -> 5.2 / 5.3 / 6.5 us, Q4_K at eight 8.3 -> 6.0; with more tiles the added waves cost
+  // more than they take over, 6144 x 2048 Q6_K at eight rows 8.4 -> 9.5)
+  if (quantizes && !moe && tw == 1) P = std::max(P, std::min(8, (a.M * a.nsb * 32 + 127) / 128));
   while (P > 1 && kr_lds_bytes(q4, a.nsb, 1, P) > KR_LDS_MAX) P--;
   while (tw > 1 && kr_lds_bytes(q4, a.nsb, tw, P) > KR_LDS_MAX) tw--;
   return KrShape{tw, P};
@@ -549,7 +553,7 @@ static int kr_threads(int wtype, const KGemvArgs& a) {
 template <int WT, int XT, int TH, int ORDER>
 static int launch_kq_rows(const KGemvArgs& a_in, hipStream_t st, unsigned grid_y = 1) {
   KGemvArgs a = a_in;
-  const KrShape shape = kr_shape(WT == MLLM_HIP_Q4_K, a, grid_y);
+  const KrShape shape = kr_shape(WT == MLLM_HIP_Q4_K, a, grid_y, XT != KQ_IMAGE);
   const int tw = shape.tiles, P = shape.waves;
   const size_t lds = kr_lds_bytes(WT == MLLM_HIP_Q4_K, a.nsb, tw, P);
   if (lds > KR_LDS_MAX) return MLLM_HIP_E_SHAPE;

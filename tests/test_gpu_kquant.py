@@ -241,11 +241,11 @@ def test_k_slices_that_meet_in_the_workspace_give_the_same_bits(wtype, M):
 
 
 @pytest.mark.parametrize("wtype", [2, 3])
-@pytest.mark.parametrize("M,Ns,K", [(3, (1, 16, 17), 256), (4, (15,), 768), (5, (4097, 33), 1280), (8, (16 * 1400 + 3,), 512), (6, (40,), 15872),
+@pytest.mark.parametrize("M,Ns,K", [(3, (1, 16, 17), 256), (4, (15,), 768), (8, (33,), 1024), (5, (4097, 33), 1280), (8, (16 * 1400 + 3,), 512), (6, (40,), 15872),
                                     (7, (9, 70), 16128)])
 def test_rows_kernel_edges(wtype, M, Ns, K):
-    """three to eight rows: part and odd tiles of 16 channels, one to many tiles per workgroup, odd numbers of super-blocks, the
-    longest rows whose codes fit the LDS and the first that do not, with a workspace and without"""
+    """three to eight rows: part and odd tiles of 16 channels, one to many tiles per workgroup, odd numbers of super-blocks, more waves
+    than slices, the longest rows whose codes fit the LDS and the first that do not, with a workspace and without"""
     rng = synth.rng_for(7, 1700 + M + 50 * wtype)
     Ws = [synth.make_weight(rng, wtype, N, K) for N in Ns]
     ws = [ql.PackedKWeight(wtype, torch.from_numpy(W)) for W in Ws]
