@@ -1080,7 +1080,7 @@ MLLM_API int mllm_hip_linear_kq_gemm(int wtype, const void* gemm_packed, const v
 // the same with room for the partial results of K ranges that run as separate workgroups
 MLLM_API size_t mllm_hip_linear_kq_gemm_short_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % QK_K) return 0;
-  return mllm_hip_linear_kq_gemm_workspace_bytes(M, K) + 256 + qg_partial_bytes(M, N, K);
+  return mllm_hip_linear_kq_gemm_workspace_bytes(M, K) + 256 + qg_partial_bytes(MLLM_HIP_Q4_K, M, N, K);
 }
 MLLM_API int mllm_hip_linear_kq_gemm_short(int wtype, const void* gemm_packed, const void* x, int x_dtype, const float* bias, float* y,
                                            int64_t M, int64_t N, int64_t K, void* workspace, void* stream) {
@@ -1095,6 +1095,6 @@ MLLM_API int mllm_hip_linear_kq_gemm_short(int wtype, const void* gemm_packed, c
   const int64_t nitems = M * K / 8;
   hipLaunchKernelGGL(kq_act_f16_kernel, dim3((unsigned)((nitems + 255) / 256)), dim3(256), 0, st, x, x_dtype, xh, nitems);
   char* base = reinterpret_cast<char*>(workspace);
-  void* partial = qg_partial_bytes(M, N, K) ? base + mllm_hip_linear_kq_gemm_workspace_bytes(M, K) : nullptr;
+  void* partial = qg_partial_bytes(MLLM_HIP_Q4_K, M, N, K) ? base + mllm_hip_linear_kq_gemm_workspace_bytes(M, K) : nullptr;
   return qg_linear_run(wtype, gemm_packed, xh, bias, y, M, N, K, partial, st);
 }

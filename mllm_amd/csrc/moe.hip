@@ -970,8 +970,13 @@ __global__ __launch_bounds__(256 * G) __attribute__((amdgpu_waves_per_eu(2, 2)))
       rows = min(QG_TILE_H / 2, a.a_rows - row0);
       n0 = (a.big_cols + b / tilesH) * 256;
     } else {
+      // Row tiles in multiples of eight, from 16 on: in the grid's order an XCD takes every eighth of them, whose activations stay in its
+      // L2 (1.00 to 1.11 of the time otherwise over 110 shapes of 2048 to 8192 rows; 0.90 to 1.04 with eight row tiles).
       int tm, tn;
-      if (tilesM % 2 == 0 && a.big_cols % 4 == 0) {  // an XCD takes half of the rows of a quarter of the columns
+      if (tilesM % 8 == 0 && tilesM >= 16) {
+        tm = b % tilesM;
+        tn = b / tilesM;
+      } else if (tilesM % 2 == 0 && a.big_cols % 4 == 0) {  // an XCD takes half of the rows of a quarter of the columns
         const int xcd = b & 7, seq = b >> 3, hm = tilesM / 2, qn = a.big_cols / 4;
         tm = (xcd & 1) * hm + seq % hm;
         tn = (xcd >> 1) * qn + seq / hm;
@@ -1959,18 +1964,63 @@ __global__ __launch_bounds__(256) void qg_reduce_kernel(const float* __restrict_
 //   ranges  128 x 256 tiles by four waves, K cut into up to eight ranges that run as separate workgroups, leave partial results and
 //           are added by a small second kernel in range order; one range: the plain form, with half-height tiles for a short
 //           last round
-// The expected cost of each, in us, is fitted to 130 shapes of 1 to 28 M weights and 93 to 2048 rows within 4 to 9 % (rms; form 0: 17 %);
-// the choice is within 1.2 % of the best form on average, 14 % at worst.  131 x 2560 x 9728 (Q6_K, with the activations' kernel):
-// 33.6 -> 26 us, 93 x 6144 x 2048 (Q4_0) 27 -> 14, 700 x 6144 x 2048 43.7 -> 39, 2048 x 2048 x 6144 102 -> 80.
+// 131 x 2560 x 9728 (Q6_K, with the activations' kernel): 33.6 -> 23.2 us, 93 x 6144 x 2048 (Q4_0) 27 -> 14, 700 x 6144 x 2048 43.7 -> 39,
+// 2048 x 2048 x 6144 102 -> 80.
 struct QLinearPlan {
   int waves;   // form of launch_q_waves, or -1
   int halves;
   int ranges;
 };
-static QLinearPlan q_linear_plan(int64_t M, int64_t N, int64_t K, bool ranges_fit) {
-  static const FormCost waves[] = {{32, 32, 0.0f, 1.22f, 0.36f, 0.1026f}, {32, 64, 0.5f, 1.72f, 0.97f, 0.1251f}, {64, 64, 0.5f, 2.22f, 1.86f, 0.2001f}};
-  const int64_t blocks = (K + 63) / 64;
-  const float mn = (float)M * (float)N * 1e-6f;
+static int g_q_gemm_form = 0;  // mllm_hip_q_gemm_set_form
+static bool q_ranges_exist(int64_t N, int64_t blocks, int z) {  // whole even ranges, none of them empty
+  const int64_t per = ((blocks + z - 1) / z + 1) / 2 * 2;
+  return z == 1 || (N % 4 == 0 && (blocks + per - 1) / per == z);
+}
+// What each form is expected to take, in us with the activations' kernel, fitted per format to 340 shapes each (random, 33 to 2048 rows,
+// weights of 512 to 9728 either way; the rms errors stand in the table).  Over 1360 such shapes the form chosen takes 1.005 times the best
+// form's time on average (19 % more at worst) and is more than 2 % slower than the one range or the ranges by rows and columns alone that
+// ran before in 5 of them (595 x 1016 x 8704 Q4_K 37.4 -> 39.3 us at most); from 33 to 4096 rows of up to 151 936 channels 3 of 520 (404 x
+// 17776 x 512 Q4_K 29.3 -> 32.9).  With one table for all formats, K products and ragged last tiles at a price, a choice was up to 18 %
+// slower than those (63 x 9328 x 8704 Q6_K 41.4 -> 48.9, 345 x 1480 x 8704 Q6_K 33.9 -> 39.1, 424 x 6432 x 5376 Q4_K 56.2 -> 63.3).
+struct QFormCost {
+  float waves[3][6];  // per form: how a partly filled last round counts, fixed, round, round and 64 of K, 1e6 M K (read again by every
+  float halves[6];    // column tile), 1e6 M N
+  float ranges[8];    // two workgroups on a CU, part of a last round; fixed, round, round and 64 of K, M K, M N, M N per partial result
+};
+static const QFormCost& q_form_cost(int wtype) {
+  static const QFormCost cost[] = {
+      {{{0.75f, 5.194f, 0.7106f, 0.0662f, 3.222f, 0.06239f},
+        {0.75f, 5.554f, 0.1751f, 0.1086f, 1.942f, 1.997f},
+        {0.5f, 6.718f, 0.f, 0.1817f, 1.876f, 1.659f}},
+       {1.f, 8.318f, 0.3028f, 0.6705f, 0.6885f, 1.894f},
+       {1.5f, 0.5f, 11.4f, 0.005467f, 0.7897f, 1.398f, 0.7408f, 1.058f}},  // Q4_0: 4 / 4 / 5 / 4 / 6 %
+      {{{0.75f, 5.465f, 0.4136f, 0.0751f, 3.046f, 1.154f},
+        {1.f, 5.928f, 0.f, 0.1192f, 1.86f, 2.248f},
+        {0.5f, 7.359f, 0.f, 0.2f, 1.889f, 1.413f}},
+       {1.f, 6.389f, 2.611f, 0.6195f, 1.174f, 1.848f},
+       {1.6f, 0.5f, 11.23f, 0.f, 0.7656f, 1.514f, 0.6784f, 1.075f}},  // Q8_0: 4 / 4 / 5 / 7 / 7 %
+      {{{0.75f, 5.412f, 0.5444f, 0.06797f, 3.148f, 0.8011f},
+        {1.f, 5.739f, 0.04121f, 0.1086f, 1.952f, 2.302f},
+        {0.5f, 7.01f, 0.f, 0.1872f, 1.97f, 1.559f}},
+       {1.f, 10.17f, 0.05216f, 0.6293f, 0.906f, 1.662f},
+       {1.5f, 0.75f, 12.58f, 0.f, 0.763f, 1.45f, 0.7756f, 1.005f}},  // Q4_K: 3 / 3 / 5 / 4 / 6 %
+      {{{1.f, 4.986f, 0.6891f, 0.08025f, 3.059f, 2.38f},
+        {1.f, 6.076f, 0.f, 0.1191f, 1.771f, 2.268f},
+        {0.5f, 7.235f, 0.f, 0.2001f, 1.852f, 1.482f}},
+       {1.f, 2.535f, 7.217f, 0.6381f, 1.067f, 1.459f},
+       {1.7f, 0.5f, 12.05f, 0.f, 0.7532f, 1.344f, 0.6954f, 1.035f}},  // Q6_K: 4 / 3 / 5 / 4 / 6 %
+  };
+  return cost[wtype == MLLM_HIP_Q4_0 ? 0 : wtype == MLLM_HIP_Q8_0 ? 1 : wtype == MLLM_HIP_Q4_K ? 2 : 3];
+}
+static QLinearPlan q_linear_plan(int wtype, int64_t M, int64_t N, int64_t K, bool ranges_fit) {
+  const int64_t blocks = (K + 63) / 64, cols = (N + 255) / 256, tilesM = (M + QG_TILE_H - 1) / QG_TILE_H;
+  if (g_q_gemm_form) {
+    const int z = g_q_gemm_form - 4;
+    return g_q_gemm_form <= 3 ? QLinearPlan{g_q_gemm_form - 1, 0, 1} : z == 0 ? QLinearPlan{-1, 1, 1}
+           : QLinearPlan{-1, 0, ranges_fit && q_ranges_exist(N, blocks, z) ? z : 1};
+  }
+  const QFormCost& c = q_form_cost(wtype);
+  const float mk = (float)M * (float)K * 1e-6f, mn = (float)M * (float)N * 1e-6f;
   QLinearPlan best{-1, 0, 1};
   float least = 0.f;
   auto offer = [&](float cost, const QLinearPlan& p) {
@@ -1979,28 +2029,39 @@ static QLinearPlan q_linear_plan(int64_t M, int64_t N, int64_t K, bool ranges_fi
       best = p;
     }
   };
-  for (int f = 0; f < 3; f++) offer(form_cost(waves[f], M, N, blocks), QLinearPlan{f, 0, 1});
+  auto whole = [&](const float* f, float full, float part) {  // one workgroup on a CU at a time, or as good as
+    const float rounds = f[0] * full + (1.f - f[0]) * std::max(1.f, part);
+    return f[1] + rounds * (f[2] + f[3] * (float)blocks) + f[4] * mk + f[5] * mn;
+  };
+  static const int rows[3] = {32, 32, 64}, chans[3] = {32, 64, 64};
+  for (int f = 0; f < 3; f++) {
+    const int64_t tiles = ((M + rows[f] - 1) / rows[f]) * ((N + chans[f] - 1) / chans[f]);
+    offer(whole(c.waves[f], (float)((tiles + 255) / 256), (float)tiles / 256.f), QLinearPlan{f, 0, 1});
+  }
   // a ragged last tile of 128 rows runs as 64 or 32
   const int64_t rest = M % QG_TILE_H;
-  const float tiles = ((float)(M / QG_TILE_H) + (rest == 0 ? 0.f : rest > 64 ? 1.f : rest > 32 ? 0.7f : 0.5f)) * (float)((N + 255) / 256);
-  offer(5.52f + ceilf(tiles / 256.f) * (1.56f + 0.6155f * (float)blocks) + 1.874f * mn, QLinearPlan{-1, 1, 1});
+  const float tiles = ((float)(M / QG_TILE_H) + (rest == 0 ? 0.f : rest > 64 ? 1.f : rest > 32 ? 0.7f : 0.5f)) * (float)cols;
+  offer(whole(c.halves, ceilf(tiles / 256.f), tiles / 256.f), QLinearPlan{-1, 1, 1});
   for (int z = 1; z <= 8; z++) {
-    if (z > 1 && (!ranges_fit || N % 4 || (float)z * mn > 16.f)) break;  // 64 MB of partial results at most
-    const int64_t per = ((blocks + z - 1) / z + 1) / 2 * 2;
-    if ((blocks + per - 1) / per != z) continue;  // no empty range
-    const float t = tiles * (float)z, rounds = t <= 256.f ? 1.f : t <= 512.f ? 1.5f : 1.5f * (0.5f * ceilf(t / 512.f) + t / 1024.f);
-    offer(4.75f + rounds * (3.80f + 0.793f * (float)per) + 0.895f * mn + (z > 1 ? 0.804f * (float)(z + 1) * mn + 2.76f : 0.f), QLinearPlan{-1, 0, z});
+    if (z > 1 && (!ranges_fit || (float)z * mn > 16.f)) break;  // 64 MB of partial results at most
+    if (!q_ranges_exist(N, blocks, z)) continue;
+    const int64_t per = ((blocks + z - 1) / z + 1) / 2 * 2, t = tilesM * cols * z;
+    const float* f = c.ranges;
+    const float rounds = t <= 256 ? 1.f : t <= 512 ? f[0] : f[0] * (f[1] * (float)((t + 511) / 512) + (1.f - f[1]) * (float)t / 512.f);
+    offer(f[2] + rounds * (f[3] + f[4] * (float)per) + f[5] * mk + f[6] * mn + (z > 1 ? f[7] * (float)(z + 1) * mn : 0.f), QLinearPlan{-1, 0, z});
   }
   return best;
 }
-size_t qg_partial_bytes(int64_t M, int64_t N, int64_t K) {
-  const int z = q_linear_plan(M, N, K, true).ranges;
+size_t qg_partial_bytes(int wtype, int64_t M, int64_t N, int64_t K) {  // the same for both types of a call (their plans may differ)
+  const bool kq = wtype == MLLM_HIP_Q4_K || wtype == MLLM_HIP_Q6_K;
+  const int z = std::max(q_linear_plan(kq ? MLLM_HIP_Q4_K : MLLM_HIP_Q4_0, M, N, K, true).ranges,
+                         q_linear_plan(kq ? MLLM_HIP_Q6_K : MLLM_HIP_Q8_0, M, N, K, true).ranges);
   return z > 1 ? align_up((size_t)z * M * N * 4, 256) : 0;
 }
 
 int qg_linear_run(int wtype, const void* gemm_packed, const uint16_t* xh, const float* bias, float* y, int64_t M, int64_t N,
                   int64_t K, void* partial_ws, hipStream_t st) {
-  const QLinearPlan plan = q_linear_plan(M, N, K, partial_ws != nullptr);
+  const QLinearPlan plan = q_linear_plan(wtype, M, N, K, partial_ws != nullptr);
   if (plan.waves >= 0) {
     const QWavesArgs w{reinterpret_cast<const char*>(gemm_packed), xh, bias, y, (int)M, (int)N, (int)K};
     switch (wtype) {
@@ -2021,12 +2082,12 @@ int qg_linear_run(int wtype, const void* gemm_packed, const uint16_t* xh, const 
   a.partial = reinterpret_cast<float*>(partial_ws);
   const int64_t tilesM = (M + QG_TILE_H - 1) / QG_TILE_H, cols = (N + 255) / 256, total = tilesM * cols;
   a.big_cols = (int)cols;
-  if (a.ksplit <= 1 && !a.halves && total > QG_SLOTS && total % QG_SLOTS) {
-    // columns whose full tiles fill whole rounds; the others as half-height tiles if that ends earlier (such a tile takes about 0.6 of
-    // a full one: it dequantizes the same weights for half the rows)
-    const int64_t big = total / QG_SLOTS * QG_SLOTS / tilesM, halves = (cols - big) * ((M + QG_TILE_H / 2 - 1) / (QG_TILE_H / 2));
-    const double with_tail = (double)((big * tilesM + QG_SLOTS - 1) / QG_SLOTS) + 0.6 * (double)((halves + QG_SLOTS - 1) / QG_SLOTS);
-    if (with_tail < (double)((total + QG_SLOTS - 1) / QG_SLOTS)) a.big_cols = (int)big;
+  const int64_t last = total % QG_SLOTS;
+  if (a.ksplit <= 1 && !a.halves && total > QG_SLOTS && total < 4 * QG_SLOTS && last && last < QG_SLOTS / 4) {
+    // A last round that is less than a quarter full: the columns whose full tiles fill whole rounds, the others as half-height tiles (such
+    // a tile takes about 0.6 of a full one: it dequantizes the same weights for half the rows).  Over 180 shapes of 513 to 2600 tiles: 0.89
+    // to 0.99 of the time there, 1.01 to 1.09 where the last round is fuller, 0.93 to 1.06 from four rounds on.
+    a.big_cols = (int)(total / QG_SLOTS * QG_SLOTS / tilesM);
   }
   const int rc = launch_qg<0>(a, (unsigned)tilesM, st);
   if (rc || a.ksplit <= 1) return rc;
@@ -2255,6 +2316,18 @@ MLLM_API int mllm_hip_q_gemm_prepack(int wtype, const void* blocks, int weight_s
   return (int)hipGetLastError();
 }
 
+MLLM_API int mllm_hip_q_gemm_set_form(int form) {
+  if (form < 0 || form > 12) return MLLM_HIP_E_BADARG;
+  g_q_gemm_form = form;
+  return 0;
+}
+MLLM_API int mllm_hip_q_gemm_form(int wtype, int64_t M, int64_t N, int64_t K, int short_call) {
+  if (wtype != MLLM_HIP_Q4_0 && wtype != MLLM_HIP_Q8_0 && wtype != MLLM_HIP_Q4_K && wtype != MLLM_HIP_Q6_K) return 0;
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const QLinearPlan p = q_linear_plan(wtype, M, N, K, short_call && qg_partial_bytes(wtype, M, N, K));
+  return p.waves >= 0 ? 1 + p.waves : p.halves ? 4 : 4 + p.ranges;
+}
+
 MLLM_API size_t mllm_hip_linear_q_gemm_workspace_bytes(int64_t M, int64_t K) {
   if (M <= 0 || K <= 0 || K % QK) return 0;
   Carver c(nullptr);
@@ -2285,7 +2358,7 @@ MLLM_API int mllm_hip_linear_q_gemm(int wtype, const void* gemm_packed, const vo
 // the same with room for the partial results of K ranges (behind the activations, on a 256-byte line of their own)
 MLLM_API size_t mllm_hip_linear_q_gemm_short_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % QK) return 0;
-  return align_up(mllm_hip_linear_q_gemm_workspace_bytes(M, K), 256) + 256 + qg_partial_bytes(M, N, K);
+  return align_up(mllm_hip_linear_q_gemm_workspace_bytes(M, K), 256) + 256 + qg_partial_bytes(MLLM_HIP_Q4_0, M, N, K);
 }
 MLLM_API int mllm_hip_linear_q_gemm_short(int wtype, const void* gemm_packed, const void* x, int x_dtype, const float* bias, float* y,
                                           int64_t M, int64_t N, int64_t K, int act_scale_mode, void* workspace, void* stream) {
@@ -2303,7 +2376,7 @@ MLLM_API int mllm_hip_linear_q_gemm_short(int wtype, const void* gemm_packed, co
   const int64_t nblocks = M * (K / QK);
   hipLaunchKernelGGL(qg_act_kernel, dim3((unsigned)((nblocks + 63) / 64)), dim3(256), 0, st, x, x_dtype, xh,
                      (uint16_t*)nullptr, nblocks, act_scale_mode == MLLM_HIP_SCALE_X86_REF);
-  void* partial = qg_partial_bytes(M, N, K) ? c.p + align_up(mllm_hip_linear_q_gemm_workspace_bytes(M, K), 256) : nullptr;
+  void* partial = qg_partial_bytes(MLLM_HIP_Q4_0, M, N, K) ? c.p + align_up(mllm_hip_linear_q_gemm_workspace_bytes(M, K), 256) : nullptr;
   return qg_linear_run(wtype, gemm_packed, xh, bias, y, M, N, K, partial, st);
 }
 

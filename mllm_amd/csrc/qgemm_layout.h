@@ -22,9 +22,9 @@ __host__ __device__ inline int64_t qg_bytes(int wtype, int64_t N, int64_t K) {
 }
 
 // y[M][N] fp32 = xh[M][K] (fp16) * W^T + bias on the matrix cores, in the form with the least expected cost.
-// partial_ws: null, or qg_partial_bytes(M, N, K) bytes (256-byte aligned), with which K may be cut into ranges that run as separate
+// partial_ws: null, or qg_partial_bytes(wtype, M, N, K) bytes (256-byte aligned), with which K may be cut into ranges that run as separate
 // workgroups (qg_partial_bytes returns 0 where that does not pay; pass null then)
-size_t qg_partial_bytes(int64_t M, int64_t N, int64_t K);
+size_t qg_partial_bytes(int wtype, int64_t M, int64_t N, int64_t K);
 int qg_linear_run(int wtype, const void* gemm_packed, const uint16_t* xh, const float* bias, float* y, int64_t M, int64_t N,
                   int64_t K, void* partial_ws, hipStream_t st);
 

@@ -89,6 +89,8 @@ def _cases():
         "mllm_hip_w8a8_set_decode_mfma_from": ([5], [(0, 0, BADARG), (0, 34, BADARG)]),
         "mllm_hip_w4a16_set_decode": ([1], [(0, 2, BADARG), (0, -1, BADARG)]),
         "mllm_hip_w4a16_set_decode_mfma_from": ([2], [(0, 0, BADARG), (0, 34, BADARG)]),
+        "mllm_hip_q_gemm_set_form": ([0], [(0, 13, BADARG), (0, -1, BADARG)]),
+        "mllm_hip_q_gemm_form": ([Q4_0, 64, 64, 256, 1], [(0, 5, 0), (1, 0, 0), (2, 0, 0), (3, -1, 0)]),
         "mllm_hip_moe_gate_set_form": ([1], [(0, 2, BADARG), (0, -1, BADARG)]),
         "mllm_hip_kq_gemm_prepack": ([Q4_K, P, 0, P, 8, 256, None], [(0, Q8_0, BADARG), (1, None, BADARG), (5, 96, SHAPE)]),
         "mllm_hip_linear_kq_gemm": ([Q4_K, P, P, F32, None, P, 16, 8, 256, P, None],
@@ -149,6 +151,30 @@ def test_topk_is_cut_into_pieces_only_where_that_is_faster():
     for rows, ln, k, pieces in ((8, 4096, 50, 0), (8, 4097, 50, 0), (1, 8191, 1, 0), (256, 5001, 128, 0), (257, 4097, 50, 2), (8, 4100, 50, 2), (8, 8192, 50, 2),
                                 (8, 8193, 50, 3), (8, 151936, 128, 38), (512, 151936, 20, 38), (513, 151936, 20, 0), (8, 151936, 129, 0)):
         assert room(rows, ln, k) == rows * pieces * k * 8, (rows, ln, k)
+
+
+@pytest.mark.parametrize("wtype,M,N,K,forms", [
+    (Q6_K, 54, 6144, 2048, (2,)), (Q6_K, 138, 2288, 1536, (2,)), (Q4_K, 394, 2560, 9728, (10,)), (Q4_0, 415, 5640, 8768, (9,)),
+    (Q6_K, 316, 8880, 7424, (6, 8)), (Q4_0, 1956, 760, 4832, (8, 9, 10)), (Q6_K, 114, 2560, 9728, (2,))])
+def test_q_gemm_takes_a_form_that_measures_fast(wtype, M, N, K, forms):
+    """shapes at which a choice by rows, columns and K steps alone was 10 to 23 % slower than the forms here (measured, all twelve)"""
+    assert _lib.lib().mllm_hip_q_gemm_form(wtype, M, N, K, 1) in forms
+    assert _lib.lib().mllm_hip_q_gemm_form(wtype, M, N, K, 0) <= 5  # no room for partial results: no ranges
+
+
+@pytest.mark.parametrize("M,N,K", [(200, 2560, 9728), (200, 2558, 9728), (70, 260, 160), (200, 1024, 640), (512, 512, 65536)])
+def test_q_gemm_has_room_for_the_ranges_of_each_format(M, N, K):
+    """partial results of the larger of a call's two formats, 64 MB at most; none where no format takes ranges or N % 4"""
+    L = _lib.lib()
+    up = lambda b: (b + 255) // 256 * 256
+    for types, room, plain in (((Q4_0, Q8_0), L.mllm_hip_linear_q_gemm_short_workspace_bytes, up(L.mllm_hip_linear_q_gemm_workspace_bytes(M, K))),
+                               ((Q4_K, Q6_K), L.mllm_hip_linear_kq_gemm_short_workspace_bytes, L.mllm_hip_linear_kq_gemm_workspace_bytes(M, K))):
+        if K % 256 and Q4_K in types:
+            continue
+        z = max(max(1, L.mllm_hip_q_gemm_form(t, M, N, K, 1) - 4) for t in types)
+        partial = room(M, N, K) - plain - 256
+        assert partial == (up(z * M * N * 4) if z > 1 else 0) and partial <= 64 << 20
+        assert N % 4 == 0 or z == 1
 
 
 def test_size_helpers_return_zero_for_shapes_they_do_not_take():

@@ -69,16 +69,21 @@ def test_linear_q_gemm_any_m(wtype, M, N, K):
 
 
 @pytest.mark.parametrize("wtype", [0, 1])
-@pytest.mark.parametrize("M,N,K", [(16, 9728, 2560), (128, 2560, 9728), (200, 1024, 640), (256, 6144, 2560), (40, 132, 4096 + 128)])
+@pytest.mark.parametrize("M,N,K", [(16, 9728, 2560), (128, 2560, 9728), (200, 1024, 640), (256, 6144, 2560), (40, 132, 4096 + 128),
+                                   (200, 2560, 9728), (256, 2560, 9728), (394, 2560, 9728)])
 def test_linear_q_gemm_short_batches(wtype, M, N, K):
-    """short prompts: K ranges as separate workgroups + reduction, against the oracle and the unsplit call"""
+    """short prompts with the larger workspace, against the oracle and the unsplit call; the long rows of 200 and more tokens run as K
+    ranges in separate workgroups + reduction, which the workspace has room for"""
     rng = synth.rng_for(4, 600 + M + N % 97 + wtype)
     W = synth.make_weight(rng, wtype, N, K)
     w = ql.PackedQWeight(wtype, torch.from_numpy(W), layout="gemm")
     x = synth.make_x_fp32(rng, M, K)
     bias = rng.standard_normal(N).astype(np.float32)
     announce("linear_q_gemm short", wtype, M, N, K)
-    assert _lib.lib().mllm_hip_linear_q_gemm_short_workspace_bytes(M, N, K) > _lib.lib().mllm_hip_linear_q_gemm_workspace_bytes(M, K)
+    ranges = _lib.lib().mllm_hip_q_gemm_form(wtype, M, N, K, 1) - 4
+    assert (ranges > 1) == (M >= 200 and K == 9728)
+    assert ranges <= 1 or (_lib.lib().mllm_hip_linear_q_gemm_short_workspace_bytes(M, N, K) >=
+                           _lib.lib().mllm_hip_linear_q_gemm_workspace_bytes(M, K) + 256 + ranges * M * N * 4)
     ys = ql.linear_q_gemm(w, to_dev(x), to_dev(bias), short=True).cpu().numpy()
     rows = rng.integers(0, M, 8)
     want = orc.linear_q(x[rows], W, wtype, bias)
@@ -89,9 +94,8 @@ def test_linear_q_gemm_short_batches(wtype, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(3, 40, 64), (33, 200, 96), (49, 5000, 1504), (97, 1030, 2048 + 32), (300, 520, 4096), (129, 3000, 9728),
                                    (700, 6144, 2048 + 64), (1300, 3000, 3008), (1500, 2560, 9728), (2048, 2048, 6144), (2000, 9728, 512)])
 def test_linear_q_gemm_forms(M, N, K):
-    """the forms a Linear takes from a few rows to a long prompt: waves that split K (tiles of 32 and 64, ragged, K blocks that do not
-    divide), halves of K in one workgroup (odd numbers of K steps), K ranges, half-height tiles in a short last round; element stores
-    (N % 4 != 0).  Sampled rows, the last ones among them, against the oracle; the two calls agree on all rows up to the order of sums"""
+    """whatever form a Linear takes from a few rows to a long prompt.  Sampled rows, the last ones among them, against the oracle; the two
+    calls agree on all rows up to the order of sums"""
     for wtype in (0, 1) if M < 1000 else (0,):
         rng = synth.rng_for(4, 900 + M + N % 97 + wtype)
         W = synth.make_weight(rng, wtype, N, K)
@@ -104,6 +108,61 @@ def test_linear_q_gemm_forms(M, N, K):
         assert rel_l2(ys[rows], orc.linear_q(x[rows], W, wtype, bias)) < GEMM_TOL
         # fp32 sums of K products in two orders: about sqrt(K) * 2^-24 apart, relative to the result's own size
         assert rel_l2(ys, ql.linear_q_gemm(w, to_dev(x), to_dev(bias)).cpu().numpy()) < 4 * np.sqrt(K) * 2.0 ** -24
+
+
+# ragged tiles of every form, N % 4 != 0 (element stores, no ranges), odd and even numbers of K steps, fewer K steps than waves or ranges;
+# a last round that runs in half-height tiles (3 x 172 = 516 tiles); 16 row tiles, which keep the grid's order
+FORM_SHAPES = [(1, 5, 256), (37, 70, 768), (65, 100, 256), (150, 196, 2304), (131, 260, 8448), (33, 264, 17 * 256), (300, 43_900, 256), (2040, 700, 512)]
+FORM_SHAPES_32 = [(70, 260, 9 * 32), (129, 36, 32), (97, 132, 15 * 64 + 32)]  # not in super-blocks of 256
+
+
+@pytest.mark.parametrize("wtype,M,N,K", [(t, *s) for t in range(4) for s in FORM_SHAPES + (FORM_SHAPES_32 if t < 2 else [])])
+def test_q_gemm_every_form_exact(wtype, M, N, K):
+    """unit block scales, small codes and integer activations that quantize to themselves: every operand is an integer that fp16 holds
+    and every partial sum, in any order, stays below 2^24, so each form gives the integer product exactly"""
+    L = _lib.lib()
+    kq = wtype >= 2
+    rng = synth.rng_for(4, 1200 + M + N + K + wtype)
+    W = synth.make_weight(rng, wtype, N, K)
+    x = rng.integers(-3, 4, (M, K)).astype(np.float32)
+    one = np.array([0x00, 0x3c], np.uint8)
+    if wtype == 0:
+        W.reshape(N, K // 32, -1)[:, :, 0:2] = one
+    elif wtype == 1:
+        W.reshape(N, K // 32, -1)[:, :, 0:2] = one
+        W.reshape(N, K // 32, -1)[:, :, 2:] = rng.integers(-9, 10, (N, K // 32, 32)).astype(np.int8).view(np.uint8)
+    elif wtype == 2:
+        W[:, :, 0:2] = W[:, :, 2:4] = one
+    else:
+        W[:, :, 208:210] = one
+        W[:, :, 192:208] = rng.integers(-3, 4, (N, K // 256, 16)).astype(np.int8).view(np.uint8)
+    if kq:
+        x[:, ::256] = -128.0  # the largest magnitude, -128: scale 1
+        wd = orc.dequantize_k(W, wtype, orc.SCALE_IEEE).astype(np.float32)
+        w = ql.PackedKWeight(wtype, torch.from_numpy(W), layout="gemm")
+        run = lambda short: ql.linear_kq_gemm(w, to_dev(x), to_dev(bias), short=short)
+    else:
+        x[:, ::32] = 127.0
+        b = W.reshape(N, K // 32, -1)[:, :, 2:]
+        wd = (np.concatenate([b & 15, b >> 4], 2).astype(np.float32) - 8 if wtype == 0 else b.view(np.int8).astype(np.float32)).reshape(N, K)
+        w = ql.PackedQWeight(wtype, torch.from_numpy(W), layout="gemm")
+        run = lambda short: ql.linear_q_gemm(w, to_dev(x), to_dev(bias), ql.SCALE_IEEE, short=short)
+    bias = rng.integers(-50, 51, N).astype(np.float32)
+    assert np.abs(wd).max() <= 2048 and np.abs(wd).sum(1).max() * 3 + np.abs(wd[:, ::256 if kq else 32]).sum(1).max() * 128 + 50 < 2 ** 24
+    want = x @ wd.T + bias  # exact: no partial sum leaves 2^24
+    blocks = (K + 63) // 64
+    try:
+        for form in range(1, 13):
+            assert L.mllm_hip_q_gemm_set_form(form) == 0
+            per = ((blocks + form - 5) // max(form - 4, 1) + 1) // 2 * 2
+            ranges = form < 6 or (N % 4 == 0 and -(-blocks // per) == form - 4)  # else whole tiles
+            assert L.mllm_hip_q_gemm_form(wtype, M, N, K, 1) == (form if ranges else 5)
+            announce("q gemm form", form, wtype, M, N, K)
+            assert np.array_equal(run(True).cpu().numpy(), want), form
+            if form <= 5:
+                assert np.array_equal(run(False).cpu().numpy(), want), form
+    finally:
+        assert L.mllm_hip_q_gemm_set_form(0) == 0
 
 
 def test_linear_q_gemm_exact_when_operands_fit_fp16():
