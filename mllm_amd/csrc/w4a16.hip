@@ -627,7 +627,7 @@ static int g_w4a16_ptile = 0;  // packed path: 0 = heuristic, 1 = 128x384, 2 = 6
 static int g_w4a16_waves = 1;  // 0: only the weights-from-global tiles (comparison runs and tests)
 
 // Which form runs.  The waves-split-K forms (wk_gemm.h) serve from one token to about the batch whose large tiles fill the chip;
-// 93 x 2048 x 6144: 43.6 -> 12 us, 1 x 2560 x 9728: 16.6 -> 13.4 (a GEMV of fp32 FMAs), 300 x 9728 x 2560: 36 -> 28, 2048 rows as before.
+// 93 x 2048 x 6144: 43.6 -> 10.5 us, 1 x 2560 x 9728: 15.9 (a GEMV of fp32 FMAs) -> 11.9, 300 x 9728 x 2560: 36 -> 28, 2048 rows as before.
 // The costs are fitted to 98 shapes within 6 to 10 % (rms); the choice by cost is within 0.5 % of the best form on average, 9 % at worst.
 static int launch_w4a16_auto(const W4A16PArgs& a, hipStream_t st) {
   static const FormCost cost[] = {
@@ -657,6 +657,11 @@ static int launch_w4a16_auto(const W4A16PArgs& a, hipStream_t st) {
         form = f;
       }
     }
+  }
+  if (a.M <= 8) switch (form) {  // one piece of eight rows; faster at every size measured (512 to 22016 channels, K 512 to 11008)
+    case 0: return wk_gemm_launch<W4A16Waves, 1, 1, 16, 2, 1>(a, st);
+    case 1: return wk_gemm_launch<W4A16Waves, 1, 1, 8, 3, 1>(a, st);
+    case 2: return wk_gemm_launch<W4A16Waves, 1, 2, 8, 1, 1>(a, st);
   }
   switch (form) {
     case 0: return wk_gemm_launch<W4A16Waves, 1, 1, 16, 2>(a, st);

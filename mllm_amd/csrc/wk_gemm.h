@@ -12,6 +12,11 @@
 // tag rate) that pass through the wave's own 4 TM KB of LDS, 16-byte pieces placed at piece ^ (row / 2 % 8): conflict-free
 // both ways, and no barrier, since one wave's LDS operations execute in order.  D blocks are in flight per wave in registers.
 //
+// RP: how many 8-row pieces of a 32-row tile are loaded, staged and summed (4: all).  Up to eight rows need one: the matrix instructions'
+// other columns then hold whatever the LDS held, which reaches no sum of a stored row.  Same bits; W4A16, one to eight tokens: 2048 x 2048
+// 5.85 -> 5.1 us, 6144 x 2048 6.2 -> 5.5, 2560 x 9728 14.0 -> 11.9 (a GEMV of fp32 FMAs took 5.5 / 5.9 / 15.9 for one token), 22016 x 4096
+// 18.9 -> 18.7.
+//
 // A traits class T supplies Args (tile-independent arguments with members M, N), KB-independent geometry and the operand type:
 //   kblocks(a)                        K blocks of 128 activation bytes
 //   activations(a) / row_bytes(a)     base and length in bytes of a row (16-byte multiple)
@@ -26,7 +31,7 @@
 
 namespace mllmhip {
 
-template <class T, int TM, int TN, int NW, int D>
+template <class T, int TM, int TN, int NW, int D, int RP = 4>
 __global__ __launch_bounds__(NW * 64) void wk_gemm_kernel(typename T::Args a) {
   typedef typename T::Acc Acc;  // sixteen 32-bit sums
   extern __shared__ __align__(16) unsigned char smem[];
@@ -41,9 +46,10 @@ __global__ __launch_bounds__(NW * 64) void wk_gemm_kernel(typename T::Args a) {
   const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(T::activations(a)), 0, (uint32_t)a.M * rowb, 0x00020000);
   const __amdgpu_buffer_rsrc_t rW = T::weights(a);
   // activation piece c of a lane: row 8 c + lane / 8, 16-byte column lane % 8; rows past M repeat the last one (never stored)
-  uint32_t offA[4 * TM];
+  constexpr int CA = RP * TM;
+  uint32_t offA[CA];
 #pragma unroll
-  for (int c = 0; c < 4 * TM; c++) offA[c] = (uint32_t)min(m0 + 8 * c + (lane >> 3), a.M - 1) * rowb + (lane & 7) * 16;
+  for (int c = 0; c < CA; c++) offA[c] = (uint32_t)min(m0 + 8 * c + (lane >> 3), a.M - 1) * rowb + (lane & 7) * 16;
   const uint32_t colb = (lane & 7) * 16;
   typename T::Col col[TN];
 #pragma unroll
@@ -60,14 +66,14 @@ __global__ __launch_bounds__(NW * 64) void wk_gemm_kernel(typename T::Args a) {
   const int nblk = T::kblocks(a);
   const int cnt = wave < nblk ? (nblk - wave + NW - 1) / NW : 0;  // blocks of this wave
 
-  u32x4 ga[D][4 * TM];
+  u32x4 ga[D][CA];
   typename T::W w[D][TN];
   auto request = [&](int s, int it) {
     const int kb = wave + it * NW;
     const bool in = it < cnt;
     const bool ok = in && (uint32_t)kb * 128u + colb < rowb;
 #pragma unroll
-    for (int c = 0; c < 4 * TM; c++) ga[s][c] = __builtin_amdgcn_raw_buffer_load_b128(rA, ok ? offA[c] : 0xffffffffu, kb * 128, 0);
+    for (int c = 0; c < CA; c++) ga[s][c] = __builtin_amdgcn_raw_buffer_load_b128(rA, ok ? offA[c] : 0xffffffffu, kb * 128, 0);
 #pragma unroll
     for (int j = 0; j < TN; j++) T::load(rW, col[j], in ? kb : -1, w[s][j]);
   };
@@ -83,7 +89,7 @@ __global__ __launch_bounds__(NW * 64) void wk_gemm_kernel(typename T::Args a) {
   for (int s = 0; s < D; s++) request(s, s);
   auto work = [&](int s, int next, bool more) {
 #pragma unroll
-    for (int c = 0; c < 4 * TM; c++) *reinterpret_cast<u32x4*>(wr[c & 1] + c * 1024) = ga[s][c];
+    for (int c = 0; c < CA; c++) *reinterpret_cast<u32x4*>(wr[c & 1] + c * 1024) = ga[s][c];
     typename T::W wc[TN];
 #pragma unroll
     for (int j = 0; j < TN; j++) wc[j] = w[s][j];
@@ -125,11 +131,11 @@ __global__ __launch_bounds__(NW * 64) void wk_gemm_kernel(typename T::Args a) {
         Sum4 v;
 #pragma unroll
         for (int e = 0; e < 4; e++) v[e] = acc[i][j][4 * g + e];
-        part[wave * PER + ((i * TN + j) * 8 + 2 * g + hi) * 33 + lrow] = v;
+        if (RP == 4 || lrow < 8 * RP) part[wave * PER + ((i * TN + j) * 8 + 2 * g + hi) * 33 + lrow] = v;
       }
   __syncthreads();
   // consecutive lanes take consecutive quads of channels of a row
-  constexpr int QUADS = 8 * TN, OUT = 32 * TM * QUADS;
+  constexpr int QUADS = 8 * TN, OUT = 8 * RP * TM * QUADS;
 #pragma unroll
   for (int o = tid; o < OUT; o += NW * 64) {
     const int q = o % QUADS, m = o / QUADS;
@@ -147,11 +153,13 @@ constexpr size_t wk_gemm_lds() {
   return stage > sums ? stage : sums;
 }
 
-template <class T, int TM, int TN, int NW, int D>
+template <class T, int TM, int TN, int NW, int D, int RP = 4>
 int wk_gemm_launch(const typename T::Args& a, hipStream_t st) {
   constexpr size_t lds = wk_gemm_lds<TM, TN, NW>();
   static_assert(lds <= 160 * 1024, "LDS of a CU");
-  auto kern = wk_gemm_kernel<T, TM, TN, NW, D>;
+  static_assert(RP == 4 || TM == 1, "fewer rows than a tile: one row tile");
+  if (a.M > 8 * RP * TM && RP < 4) return MLLM_HIP_E_BADARG;
+  auto kern = wk_gemm_kernel<T, TM, TN, NW, D, RP>;
   if (lds > 64 * 1024)
     HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   const unsigned grid = (unsigned)(((a.M + 32 * TM - 1) / (32 * TM)) * ((a.N + 32 * TN - 1) / (32 * TN)));

@@ -143,6 +143,23 @@ def _decode_gemv_cases(L, M):
     assert L.mllm_hip_w4a16_set_decode(2) == -1
 
 
+@pytest.mark.parametrize("M", [1, 5, 8])
+def test_one_piece_of_eight_rows_gives_the_bits_of_the_whole_tile(M):
+    """up to eight tokens load and sum one piece of a 32-row tile; 9 and 32 tokens take the same form with all four (the costs depend on
+    the tiles only).  16 waves, 8 waves and 8 waves on 64 channels, ragged N, N % 4 != 0, one K block and K blocks that do not divide;
+    rows past the batch of NaN and infinities must not reach it"""
+    for N, K, group in ((40, 64, 64), (1030, 1984, 64), (33, 8192, 128), (8195, 128, 64), (8202, 2048, 128), (40_001, 64, 64)):
+        rng = synth.rng_for(2, 1700 + M + N + K)
+        qw, s, zp, _, _ = synth.make_w4a16(rng, N, K, group)
+        a_bits, _ = synth.make_x_bf16(rng, 32, K)
+        a_bits[9:] = np.resize(np.array([0x7fc0, 0x7f80, 0xff80], np.uint16), a_bits[9:].shape)
+        bias = bf16_dev(synth.fp32_to_bf16_bits((rng.standard_normal(N) * 0.1).astype(np.float32)))
+        announce("w4a16 eight rows", M, N, K, group)
+        packed = ql.w4a16_prepack(*_dev(qw, s, zp), group)
+        got, nine, all32 = (_bits(ql.w4a16_gemm_packed(bf16_dev(a_bits[:m]), packed, N, bias, group)) for m in (M, 9, 32))
+        assert np.array_equal(got, nine[:M]) and np.array_equal(got, all32[:M])
+
+
 @pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 16 + 5])
 def test_gemm_packed_every_tile(tile):
     M, N, K, group = 200, 800, 384, 128
