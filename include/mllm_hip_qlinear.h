@@ -568,6 +568,9 @@ int mllm_hip_matmul_batched(const void* A, const void* B, void* C, int dtype, in
 /* batch = 1, fp32 */
 int mllm_hip_matmul_f32(const float* A, const float* B, float* C, int64_t M, int64_t N, int64_t K, int transpose_a,
                         int transpose_b, void* stream);
+/* Comparison runs and tests: products on tiles of 64 x 64 or 128 x 128 whatever the size (up to four rows stay with the kernels for few
+ * rows); 0: by size.  No counterpart in the reference. */
+int mllm_hip_matmul_set_tile(int side);
 
 #ifdef __cplusplus
 }

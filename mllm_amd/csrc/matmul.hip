@@ -486,8 +486,10 @@ static bool launch_matmul_dots(const MMArgs& a, hipStream_t st, int* rc) {
 //     small; 3000 x 3000 x 3000 (2.25 rounds): 604 / 527; K = 64 is mostly epilogue: 4 x 4000 x 1000 x 64: 34 / 31
 //   16 bits (bound by loads and LDS, more workgroups per CU hide them): us of a K of 2048 against tiles per CU, B [N][K]: 4096 x 4096 x 4096
 //     180 large, 298 small, 1000 x 3000 x 700: 24 / 20; where an operand is [K][rows] the large tile gains less (4096^3: 340 / 371)
+static int g_matmul_tile = 0;  // mllm_hip_matmul_set_tile
 template <int DT, bool TA, bool TB>
 static bool matmul_large_tile(const MMArgs& a) {
+  if (g_matmul_tile) return g_matmul_tile == 128;
   const double large = (double)((a.M + 127) / 128) * ((a.N + 127) / 128) * a.batch / 256;
   const double small = (double)((a.M + 63) / 64) * ((a.N + 63) / 64) * a.batch / 256;
   if (DT == MLLM_HIP_F32) return a.K >= 128 && 4. * std::ceil(large) < 1.13 * std::ceil(small);
@@ -572,6 +574,12 @@ MLLM_API int mllm_hip_matmul_batched(const void* A, const void* B, void* C, int 
     case MLLM_HIP_BF16: return launch_matmul_t<MLLM_HIP_BF16>(a, transpose_a, transpose_b, st);
     default: return launch_matmul_t<MLLM_HIP_F16>(a, transpose_a, transpose_b, st);
   }
+}
+
+MLLM_API int mllm_hip_matmul_set_tile(int side) {
+  if (side != 0 && side != 64 && side != 128) return MLLM_HIP_E_BADARG;
+  g_matmul_tile = side;
+  return 0;
 }
 
 MLLM_API int mllm_hip_matmul_f32(const float* A, const float* B, float* C, int64_t M, int64_t N, int64_t K, int transpose_a,

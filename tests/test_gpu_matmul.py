@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from mllm_amd import qlinear as ql, synth
+from mllm_amd import _lib, qlinear as ql, synth
 from gpu_util import announce, rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -87,7 +87,7 @@ def test_matmul_16_bit(batch, M, N, K, ta, tb, dtype):
 
 @pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
 @pytest.mark.parametrize("batch,M,N,K,ta,tb", [
-    # either tile (the larger one from many tiles on), rows past the end repeated, K steps that end behind K, [K][rows] operands
+    # tiles (the larger one for the first shape in 16 bits), rows past the end repeated, K steps that end behind K, [K][rows] operands
     # whose rows are or are not a multiple of a vector, fewer rows than a vector
     (1, 2050, 2174, 257, False, True), (33, 513, 387, 290, False, False), (1, 2177, 2049, 288, True, True), (3, 65, 63, 33, False, False),
     (2, 3, 2, 64, True, False), (2, 66, 68, 96, True, False), (2, 5, 3, 31, False, False), (1, 64, 7, 320, True, False),
@@ -108,6 +108,28 @@ def test_matmul_forms_at_their_edges(batch, M, N, K, ta, tb, dtype):
     assert torch.equal(c, want)
 
 
+@pytest.mark.parametrize("side", [64, 128])
+@pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("batch,M,N,K", [(3, 130, 262, 37), (2, 257, 129, 160), (1, 128, 256, 31), (2, 66, 68, 290), (2, 7, 5, 33), (5, 300, 132, 64),
+                                         (1, 770, 642, 163), (1, 768, 644, 1024)])
+def test_matmul_on_each_tile(batch, M, N, K, ta, tb, dtype, side):
+    """either tile in every order: ragged and whole tiles, rows that are and are not a multiple of a vector, K steps that end behind K, K
+    of one step and less; exact as above"""
+    rng = synth.rng_for(6, 4000 + batch + M + N + K)
+    td = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    a = torch.from_numpy(rng.integers(-8, 9, (batch, K, M) if ta else (batch, M, K)).astype(np.float32))
+    b = torch.from_numpy(rng.integers(-8, 9, (batch, N, K) if tb else (batch, K, N)).astype(np.float32))
+    announce("matmul tile %d %s %s ta=%d tb=%d" % (side, dtype, (batch, M, N, K), ta, tb))
+    try:
+        assert _lib.lib().mllm_hip_matmul_set_tile(side) == 0
+        c = ql.matmul(a.to(td).cuda(), b.to(td).cuda(), ta, tb).cpu()
+    finally:
+        assert _lib.lib().mllm_hip_matmul_set_tile(0) == 0
+    want = torch.matmul(a.transpose(1, 2).contiguous() if ta else a, b.transpose(1, 2).contiguous() if tb else b).to(td)
+    assert torch.equal(c, want)
+
+
 @pytest.mark.parametrize("dtype", ["fp32", "bf16"])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("batch,M,N,K", [(16, 16, 16, 16), (1000, 8, 8, 8), (1, 300, 132, 40), (3, 68, 60, 24), (2, 64, 128, 504), (5, 12, 8, 56)])
@@ -121,6 +143,30 @@ def test_short_matmuls_of_whole_vectors(batch, M, N, K, ta, tb, dtype):
     c = ql.matmul(a.to(td).cuda(), b.to(td).cuda(), ta, tb).cpu()
     want = torch.matmul(a.transpose(1, 2).contiguous() if ta else a, b.transpose(1, 2).contiguous() if tb else b).to(td)
     assert torch.equal(c, want)
+
+
+@pytest.mark.parametrize("side", [0, 64, 128])
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(70, 130, 37), (129, 66, 64), (5, 133, 100)])
+def test_matmul_keeps_infinities_and_nan_in_their_rows(M, N, K, ta, tb, dtype, side):
+    """a row past the end repeats the last one, and what lies past K is zero on both sides: an infinity or a NaN reaches the results of its
+    own row and column alone, also from the last row and the last k"""
+    rng = synth.rng_for(6, 5000 + M + N + K)
+    td = torch.float32 if dtype == "fp32" else torch.bfloat16
+    a = torch.from_numpy(rng.integers(1, 9, (M, K)).astype(np.float32))
+    b = torch.from_numpy(rng.integers(1, 9, (N, K)).astype(np.float32))
+    a[M - 1, K - 1], a[0, 0], b[N - 1, K - 1], b[1, 0] = float("inf"), float("nan"), float("-inf"), float("inf")
+    want = torch.matmul(a, b.t().contiguous()).to(td)
+    ad, bd = a.t().contiguous() if ta else a, b if tb else b.t().contiguous()
+    announce("matmul of infinities %s %s ta=%d tb=%d tile %d" % (dtype, (M, N, K), ta, tb, side))
+    try:
+        assert _lib.lib().mllm_hip_matmul_set_tile(side) == 0
+        c = ql.matmul(ad.to(td).cuda(), bd.to(td).cuda(), ta, tb).cpu()
+    finally:
+        assert _lib.lib().mllm_hip_matmul_set_tile(0) == 0
+    assert want[0].isnan().all() and want[M - 1, N - 1].isnan() and want[M - 1, 0].isinf() and want.isfinite().sum() == (M - 2) * (N - 2)
+    assert torch.equal(c.isnan(), want.isnan()) and torch.equal(c.nan_to_num(nan=0.), want.nan_to_num(nan=0.))
 
 
 def test_matmul_batches_beyond_a_grid_dimension():

@@ -83,7 +83,7 @@ def _pack_reference(W):
     return Wp.reshape(Np // 32, 32, Kp // 32, 2, 16).transpose(0, 2, 3, 1, 4).reshape(-1)
 
 
-# shapes that reach each tile of the weights-from-global kernel: 128x384, 64x384, 128x128, 64x128, and ragged edges
+# whatever form a shape takes (waves that split K, tiles of 64x128), ragged edges
 PACKED_SHAPES = REF_SHAPES + [(300, 200, 48), (257, 193, 80), (1536, 6144, 256), (512, 9216, 128), (1024, 3072, 128),
                               (200, 800, 144)]
 
@@ -108,6 +108,33 @@ def test_gemm_packed_bit_exact(M, N, K):
     assert np.array_equal(_bits(y), wy)
     assert np.array_equal(_bits(y1), wy)
     assert np.array_equal(_bits(yb), wyb)
+
+
+@pytest.mark.parametrize("M,N,K", [(131, 200, 144), (257, 193, 80), (65, 1030, 16), (70, 392, 272), (33, 776, 1040), (300, 385, 384)])
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5])
+def test_gemm_packed_every_tile_bit_exact(tile, M, N, K):
+    """each tile of the weights-from-global kernel at ragged rows and channels (N % 8 == 0: whole stores that the buffer's bound cuts; else
+    by elements), one K step and an odd number of them; with and without the accumulators, with bias: the oracle's bits"""
+    rng = synth.rng_for(3, 400 + M * 11 + N + K)
+    xq = rng.integers(-127, 128, (M, K), dtype=np.int8)
+    W = rng.integers(-127, 128, (N, K), dtype=np.int8)
+    xs = ((rng.random(M) + 0.01) * 0.01).astype(np.float32)
+    ws = ((rng.random(N) + 0.01) * 0.01).astype(np.float32)
+    bias = (rng.standard_normal(N) * 0.01).astype(np.float32)
+    announce("w8a8 packed tile", tile, M, N, K)
+    Wp = ql.w8a8_prepack(to_dev(W))
+    wacc, wy = orc.w8a8_gemm(xq, xs, W, ws, None)
+    _, wyb = orc.w8a8_gemm(xq, xs, W, ws, bias)
+    L = _lib.lib()
+    try:
+        assert L.mllm_hip_w8a8_nsplit_set_tuning(tile) == 0
+        y, acc = ql.w8a8_gemm_packed(to_dev(xq), to_dev(xs), Wp, N, to_dev(ws), None, want_acc=True)
+        y1 = ql.w8a8_gemm_packed(to_dev(xq), to_dev(xs), Wp, N, to_dev(ws), None)
+        yb = ql.w8a8_gemm_packed(to_dev(xq), to_dev(xs), Wp, N, to_dev(ws), to_dev(bias))
+    finally:
+        assert L.mllm_hip_w8a8_nsplit_set_tuning(0) == 0
+    assert np.array_equal(acc.cpu().numpy(), wacc)
+    assert np.array_equal(_bits(y), wy) and np.array_equal(_bits(y1), wy) and np.array_equal(_bits(yb), wyb)
 
 
 @pytest.mark.parametrize("M,mfma_from", [(1, 5), (2, 5), (3, 5), (5, 33), (8, 33), (1, 1), (2, 2), (3, 2), (5, 5), (8, 5), (13, 5), (16, 5),
@@ -202,10 +229,22 @@ def test_argument_errors():
 
 @pytest.mark.parametrize("M", [5, 31, 33, 64, 97, 300])
 def test_waves_that_split_k(M):
-    """the forms whose waves share a tile and split K: row tiles of 32 and 64 with ragged ends, fewer K blocks than waves, K blocks that
-    do not divide among the waves, N not a multiple of 4 (element stores) and of 64; same bits as the oracle"""
+    """the forms whose waves share a tile and split K (32x32 at most of these shapes, 64x128 tiles at K of one block): ragged ends, fewer K
+    blocks than waves, K blocks that do not divide among the waves, N not a multiple of 4 (element stores) and of 64; same bits as the
+    oracle"""
+    _waves_cases(((M, N, K) for N, K in ((40, 64), (40, 144), (193, 1104), (1030, 2560), (4100, 784), (256, 6160))))
+
+
+def test_waves_that_split_k_of_larger_tiles():
+    """tiles of 32x64 (70 x 4100 x 784, 33 x 6002 x 1104, 300 x 1030 x 2560, 31 x 9001 x 2560 by the cost of each form) and of 64x64 (97 x
+    4101 x 2560, 65 x 6002 x 2560, 33 x 9001 x 2560, 300 x 3002 x 2576): ragged ends, N % 4 != 0, K blocks that do not divide"""
+    _waves_cases(((70, 4100, 784), (33, 6002, 1104), (300, 1030, 2560), (31, 9001, 2560), (97, 4101, 2560), (65, 6002, 2560), (33, 9001, 2560),
+                  (300, 3002, 2576)))
+
+
+def _waves_cases(shapes):
     L = _lib.lib()
-    for N, K in ((40, 64), (193, 1104), (1030, 2560), (4100, 784), (256, 6160)):
+    for M, N, K in shapes:
         rng = synth.rng_for(3, 1300 + 3 * M + N + K)
         a_bits, W, w_scale = synth.make_w8a8(rng, M, N, K)
         bias = (rng.standard_normal(N) * 0.1).astype(np.float32)
@@ -213,7 +252,7 @@ def test_waves_that_split_k(M):
         q, s = ql.per_token_quant_int8(bf16_dev(a_bits))
         packed = ql.w8a8_prepack(to_dev(W))
         y, acc = ql.w8a8_gemm_packed(q, s, packed, N, to_dev(w_scale), to_dev(bias), want_acc=True)
-        want = q.cpu().numpy().astype(np.int64) @ W.astype(np.int64).T
+        want = (q.cpu().numpy().astype(np.float64) @ W.astype(np.float64).T).astype(np.int64)  # exact
         assert np.array_equal(acc.cpu().numpy(), want)
         assert L.mllm_hip_w8a8_set_decode(0) == 0
         try:
