@@ -156,7 +156,7 @@ def test_matmul_keeps_infinities_and_nan_in_their_rows(M, N, K, ta, tb, dtype, s
     td = torch.float32 if dtype == "fp32" else torch.bfloat16
     a = torch.from_numpy(rng.integers(1, 9, (M, K)).astype(np.float32))
     b = torch.from_numpy(rng.integers(1, 9, (N, K)).astype(np.float32))
-    a[M - 1, K - 1], a[0, 0], b[N - 1, K - 1], b[1, 0] = float("inf"), float("nan"), float("-inf"), float("inf")
+    a[M - 1, K - 1], a[0, 0], b[N - 1, K - 2], b[1, 0] = float("inf"), float("nan"), float("-inf"), float("inf")
     want = torch.matmul(a, b.t().contiguous()).to(td)
     ad, bd = a.t().contiguous() if ta else a, b if tb else b.t().contiguous()
     announce("matmul of infinities %s %s ta=%d tb=%d tile %d" % (dtype, (M, N, K), ta, tb, side))
