@@ -446,9 +446,9 @@ size_t mllm_hip_kq_workspace_bytes(int64_t M, int64_t K);
 /* Up to four Linears that share the activations and K in one launch (q/k/v, gate/up), as mllm_hip_linear_q_gemv_multi. */
 int mllm_hip_linear_kq_multi(int wtype, int nparts, const mllm_hip_gemv_part* parts, const void* x, int x_dtype, int64_t M, int64_t K,
                              void* workspace, void* stream);
-/* The same with the size of the workspace stated: at least mllm_hip_kq_workspace_bytes, less is MLLM_HIP_E_BADARG.  (What
- * mllm_hip_kq_workspace_bytes_n(M, K, N_total) asks for beyond that, N_total = the sum of the parts' N, is not needed by
- * the present kernels: the K slices of a tile meet in LDS.)  One launch at a time per workspace.
+/* The same with the size of the workspace stated: at least mllm_hip_kq_workspace_bytes, less is MLLM_HIP_E_BADARG.
+ * mllm_hip_kq_workspace_bytes_n(M, K, N_total) is that size (the K slices of a tile meet in LDS and need no room for partial sums;
+ * N_total, the sum of the parts' N, is not looked at).  One launch at a time per workspace.
  * replaces: the same call sites as mllm_hip_linear_kq (the workspace has no counterpart in the reference). */
 size_t mllm_hip_kq_workspace_bytes_n(int64_t M, int64_t K, int64_t N_total);
 int mllm_hip_linear_kq_multi_ws(int wtype, int nparts, const mllm_hip_gemv_part* parts, const void* x, int x_dtype, int64_t M, int64_t K,
@@ -462,6 +462,9 @@ int mllm_hip_kq_set_tuning(int lanes_per_row, int waves_per_wg, int units_in_fli
 /* Three to eight rows take their sub-block sums from the matrix cores (rows of up to 15 872 elements).  path = 1 keeps
  * every launch on the dot4 kernel; 0 and 2 are the default (comparison runs, tests). */
 int mllm_hip_kq_set_path(int path);
+/* Those launches' tiles of 16 channels per workgroup (1..8) and waves per tile (tiles * waves <= 16; fewer of both where the LDS is too
+ * small): same bits.  0, 0: by size (comparison runs, tests).  No counterpart in the reference. */
+int mllm_hip_kq_set_rows_shape(int tiles, int waves);
 int mllm_hip_linear_kq(int wtype, const void* packed, const void* x, int x_dtype, const float* bias, float* y, int64_t M, int64_t N,
                        int64_t K, void* workspace, void* stream);
 /* Many rows (prefill) on the matrix cores, as mllm_hip_linear_q_gemm: fp16 operands with the scales folded in

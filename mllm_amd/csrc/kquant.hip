@@ -681,14 +681,7 @@ static int launch_kq(const KGemvArgs& a, hipStream_t st) {
 typedef int kv4i __attribute__((ext_vector_type(4)));
 #include "kquant_rows.h"
 
-// What mllm_hip_kq_workspace_bytes_n adds to the image: room for partial sums of K slices that no kernel leaves there any more (the
-// slices of a tile meet in LDS); the size stays what callers were told.
-static size_t kq_part_bytes(int nsb, int64_t n_total) {
-  const int S = nsb > 5 ? (nsb > 10 ? (nsb > 20 ? 8 : 4) : 2) : 1;
-  return S < 2 ? 0 : (size_t)((n_total + 15) / 16 + (int64_t)KQ_MAX_PARTS * 8) * S * 512;
-}
-
-static int g_kq_path = 0;  // 1: always the dot4 kernel, 2: the matrix-core kernels wherever they fit (comparison runs and tests)
+static int g_kq_path = 0;  // 1: always the dot4 kernel (comparison runs and tests); 0 and 2: the matrix-core kernel wherever it fits
 
 
 // ---- many rows: the matrix-core GEMM of the block formats (moe.hip, qg_kernel) with these weights -------------------------
@@ -813,6 +806,13 @@ MLLM_API int mllm_hip_kq_set_slice_meeting(int mode, int waves_per_wg) {
   return 0;
 }
 
+MLLM_API int mllm_hip_kq_set_rows_shape(int tiles, int waves) {
+  const bool off = tiles == 0 && waves == 0;
+  if (!off && (tiles < 1 || tiles > 8 || waves < 1 || tiles * waves > 16)) return MLLM_HIP_E_BADARG;
+  g_kr_shape = KrShape{tiles, waves};
+  return 0;
+}
+
 MLLM_API int mllm_hip_kq_set_tuning(int lanes_per_row, int waves_per_wg, int units_in_flight) {
   auto ok = [](int v, std::initializer_list<int> allowed) {
     for (int x : allowed)
@@ -866,9 +866,8 @@ MLLM_API size_t mllm_hip_kq_workspace_bytes(int64_t M, int64_t K) {
 }
 
 MLLM_API size_t mllm_hip_kq_workspace_bytes_n(int64_t M, int64_t K, int64_t N_total) {
-  const size_t img = mllm_hip_kq_workspace_bytes(M, K);
-  if (!img || N_total <= 0) return img;
-  return align_up(img, 256) + kq_part_bytes((int)(K / QK_K), N_total);
+  (void)N_total;  // (the K slices of a tile meet in LDS)
+  return mllm_hip_kq_workspace_bytes(M, K);
 }
 
 MLLM_API int mllm_hip_linear_kq_multi(int wtype, int nparts, const mllm_hip_gemv_part* parts, const void* x, int x_dtype, int64_t M,
@@ -1006,8 +1005,7 @@ int kq_quantize_image(const void* x, int x_dtype, void* image, int64_t rows, int
                      nitems);
   return (int)hipGetLastError();
 }
-bool kq_moe_tiles_fit(int wtype, int64_t K) {
-  (void)wtype;
+bool kq_moe_tiles_fit(int64_t K) {
   return kr_fits((int)(K / QK_K));
 }
 // MoE row tiles on the matrix-core kernels: tile t (blockIdx.y) = up to eight expert-sorted positions of expert tile_expert[t];

@@ -530,6 +530,7 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
 struct KrShape {
   int tiles, waves;
 };
+static KrShape g_kr_shape{0, 0};  // mllm_hip_kq_set_rows_shape
 static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y, bool quantizes = false) {
   int64_t tiles = 0;
   for (int i = 0; i < a.nparts; i++) tiles += (a.part[i].N + 15) / 16;
@@ -542,6 +543,7 @@ static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y, bool quant
   // Q6_K at three / four / eight rows 5.8 / 6.3 / 8.9 -> 5.2 / 5.3 / 6.5 us, Q4_K at eight 8.3 -> 6.0; with more tiles the added waves cost
   // more than they take over, 6144 x 2048 Q6_K at eight rows 8.4 -> 9.5)
   if (quantizes && !moe && tw == 1) P = std::max(P, std::min(8, (a.M * a.nsb * 32 + 127) / 128));
+  if (g_kr_shape.tiles && !moe) tw = g_kr_shape.tiles, P = g_kr_shape.waves;
   while (P > 1 && kr_lds_bytes(q4, a.nsb, 1, P) > KR_LDS_MAX) P--;
   while (tw > 1 && kr_lds_bytes(q4, a.nsb, tw, P) > KR_LDS_MAX) tw--;
   return KrShape{tw, P};

@@ -2526,7 +2526,7 @@ int kq_moe_gemv(int wtype, int nparts, const void* const* packed0, float* const*
 bool kq_moe_groups_fit(int wtype, int64_t rows, int64_t K, int slots);
 size_t kq_image_bytes(int64_t rows, int64_t K);
 int kq_quantize_image(const void* x, int x_dtype, void* image, int64_t rows, int64_t K, hipStream_t st);
-bool kq_moe_tiles_fit(int wtype, int64_t K);
+bool kq_moe_tiles_fit(int64_t K);
 int kq_moe_tiles_gemv(int wtype, int nparts, const void* const* packed0, float* const* ys, int64_t N, int64_t K, const void* image,
                       int64_t img_rows, const int* tile_expert, const int* tile_row0, const int* tile_rows, const int* ntiles,
                       unsigned max_tiles, const int* row_ids, int row_div, const int* out_ids, hipStream_t st);
@@ -2591,7 +2591,7 @@ MLLM_API int mllm_hip_moe_ffn_kq2(int wtype, int wtype_down, const void* gate_pa
   // More than about one pair per expert (Q6_K: half a pair): the pairs are sorted by expert and run as tiles of eight rows on the matrix-core
   // kernels, so an expert's matrices are streamed once per eight pairs instead of once per pair (the grouped form).
   // x and h are quantized to Q8_K once (bit-exact images), the tiles gather their rows from the images.
-  const bool tiles_ok = E <= MOE_MAX_EXPERTS && kq_moe_tiles_fit(wtype, H) && kq_moe_tiles_fit(wtype_down, I) &&
+  const bool tiles_ok = E <= MOE_MAX_EXPERTS && kq_moe_tiles_fit(H) && kq_moe_tiles_fit(I) &&
                         (size_t)E + (size_t)slots / KQ_MOE_TILE + 1 <= 65535;
   const bool many = (wtype == MLLM_HIP_Q4_K && wtype_down == MLLM_HIP_Q4_K) ? slots > E : 2 * slots > E;
   // Four pairs per expert and more: tiles of 32 rows, weights as the second operand of 32 x 32 matrix instructions (one pass

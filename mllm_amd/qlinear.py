@@ -642,10 +642,8 @@ def moe_ffn_kq(gate, up, down, x, topk_ids, topk_w, workspace=None, out=None):
 
 
 def kq_workspace(M, K, N_total=0):
-    """N_total (the sum of the N of a launch's parts) > 0: with room for the partial sums of K slices that meet in global memory"""
-    L = _lib.lib()
-    size = L.mllm_hip_kq_workspace_bytes_n(M, K, N_total) if N_total else L.mllm_hip_kq_workspace_bytes(M, K)
-    return torch.empty(size, dtype=torch.uint8, device="cuda")
+    """room for the quantized image of a group of eight rows; N_total (the sum of the N of a launch's parts) does not matter"""
+    return torch.empty(_lib.lib().mllm_hip_kq_workspace_bytes(M, K), dtype=torch.uint8, device="cuda")
 
 
 def linear_kq_gemm(w, x, bias=None, out=None, workspace=None, short=False):

@@ -83,6 +83,7 @@ def _cases():
         "mllm_hip_linear_kq_multi_ws": ([Q4_K, 1, part, P, BF16, 4, 256, P, 8 * 256 + 8 * 36, None],
                                         [(0, Q4_0, BADARG), (1, 0, BADARG), (1, 5, BADARG), (2, None, BADARG), (3, None, BADARG),
                                          (4, IMAGE, BADARG), (5, 0, BADARG), (6, 320, SHAPE), (7, ODD, ALIGN), (8, 8 * 256 + 8 * 36 - 1, BADARG)]),
+        "mllm_hip_kq_set_rows_shape": ([0, 0], [(0, 1, BADARG), (1, 1, BADARG), (0, -1, BADARG)]),
         "mllm_hip_kq_set_slice_meeting": ([-1, 0], [(0, 2, BADARG), (0, -2, BADARG), (1, 9, BADARG), (1, -1, BADARG)]),
         # switches for comparison runs: anything but 0 and 1 is refused and leaves the setting alone
         "mllm_hip_w8a8_set_decode": ([1], [(0, 2, BADARG), (0, -1, BADARG)]),
@@ -193,7 +194,6 @@ def test_size_helpers_return_zero_for_shapes_they_do_not_take():
     assert L.mllm_hip_w4a16_packed_bytes(64, 256, 100) == 0
     assert L.mllm_hip_moe_kq_workspace_bytes(4, 128, 256, 8, 2) == 0
     assert L.mllm_hip_kq_workspace_bytes_n(4, 128, 64) == 0
-    # room for partial sums only where a row has K slices: 256 elements have none, 4096 have four
-    assert 0 <= L.mllm_hip_kq_workspace_bytes_n(4, 256, 64) - L.mllm_hip_kq_workspace_bytes(4, 256) < 256
-    assert L.mllm_hip_kq_workspace_bytes_n(4, 4096, 64) >= L.mllm_hip_kq_workspace_bytes(4, 4096) + 4 * 4 * 512
-    assert L.mllm_hip_kq_workspace_bytes_n(4, 4096, 0) == L.mllm_hip_kq_workspace_bytes(4, 4096)
+    # no kernel leaves partial sums there: the image alone, whatever the channels
+    for k, n in ((256, 64), (4096, 64), (4096, 0), (9728, 9728)):
+        assert L.mllm_hip_kq_workspace_bytes_n(4, k, n) == L.mllm_hip_kq_workspace_bytes(4, k) > 8 * k
