@@ -321,7 +321,14 @@ __global__ __launch_bounds__(SOFTMAX_WG) void softmax_long_rows_kernel(const flo
 // range has no branch per element, so that its exponentials overlap (with the branches: 14.8 and 13.5); pieces of 2048 elements
 // are no faster.
 constexpr int SOFTMAX_PIECE = 4096;
-constexpr int SOFTMAX_LONG = 40960;       // up to here one workgroup per row is as fast (32 000: 12.3 us against 13.9 with a branch per element; 64 000: 21.7 against 9.9)
+// In a graph, us, a workgroup per row / pieces (which do not get slower below their limits: the limits are not where the two meet):
+//   1 to 16 rows of 8192: 7.1 / 9.0, 16 384: 13.4 / 9.3, 20 480: 9.0 / 9.4, 32 000: 12.0 / 10.4, 40 960: 14.7 / 9.6, 64 000: 21.4 / 10.2
+//   256 rows of 20 480: 16.6 / 17.4, 40 960: 32.0 / 33.4, 64 000: 48.5 / 46.1;  512 rows of 24 576: 36.6 / 38.0, 40 960: 60.4 / 56.1, 64 000: 101 /
+//   83, 151 936: 308 / 231;  1024 rows of 40 960: 131 / 106, 151 936: 603 / 455
+// Up to 16 rows the pieces win from about 22 000 elements on (and from 12 288 to 16 384, where one workgroup holds the row in registers),
+// with 256 rows from about 50 000.  The limit dates from pieces with a branch per element (32 000: 13.9) and lies late for few rows: from
+// 24 000 on no number of rows up to 512 loses more than 4 %.
+constexpr int SOFTMAX_LONG = 40960;
 constexpr int SOFTMAX_SPLIT_ROWS = 512;
 __device__ __forceinline__ float block_max_256(float v, float* s_red) {
   v = wave_max(v);
@@ -827,6 +834,10 @@ __global__ __launch_bounds__(NT) void topk_select_rows_kernel(const float* __res
 // selection, and of keys that are spread over the threads in any order they are few more than k (about 180 at k = 128).  They
 // are collected in LDS and placed by rank, up to 64 of them in the registers of one wave; should they be more than TOPK_CAND
 // (many equal values, or one thread's keys all larger than the other threads'), the k-th key itself is found a bit at a time.
+// Limits, in a graph, us, a workgroup per row / pieces, the largest 1 | 50 | 128: 8 rows of 4100: 17.6 / 8.6 | 19.1 / 12.9 | 21.3 / 13.9 (up to
+// 4096 a row is one piece, and the second launch has nothing to merge), of 151 936: 109 / 9.3 | 111 / 15.0 | 113 / 23.5; 512 rows of 4100: 19.0 /
+// 11.7 | 20.9 / 16.8 | 24.1 / 19.4, of 151 936: 256 / 76 | 260 / 101 | 264 / 143.  Pieces win on either side of 512 rows (1024 rows of 4100:
+// 38.2 / 23.5, of 151 936: 511 / 187, the largest 50); the limits bound the workspace, 512 x 38 pieces x 128 keys of 8 bytes: 20 MB.
 constexpr int TOPK_PIECE = 4096;
 constexpr int TOPK_CAND = 1024;
 constexpr int TOPK_SPLIT_K = 128;

@@ -309,6 +309,69 @@ def test_softmax_of_rows_cut_into_pieces(rows, ln):
     assert rel_l2(y, want) < 37 * 6e-8
 
 
+@pytest.mark.parametrize("ln", [40_961, 45_056, 151_936])
+def test_softmax_pieces_treat_infinities_and_nan_as_whole_rows_do(ln):
+    """a piece of -inf alone, a row of -inf, of the type's lowest value, an +inf, a NaN in a full piece and in the last one, -0.0 (the
+    polynomial clamps its argument, also an infinity or a NaN; expf of the last ln % 8 does not): one workgroup per row's results, up to the order of the sum (pieces of 4096, then their sums: 2 (16 + 8 + 38) roundings at most)"""
+    inf, nan, low = float("inf"), float("nan"), float(np.finfo(np.float32).min)
+    x = torch.randn((10, ln), generator=torch.Generator().manual_seed(ln))
+    x[0, 4096:8192] = -inf
+    x[1] = -inf
+    x[2] = low
+    x[3, ln - 1] = inf
+    x[4, 5000] = nan
+    x[5, ln - 1] = nan
+    x[6, :ln - 1] = -inf
+    x[7] = -0.0
+    x[8, 0], x[8, ln - 1] = inf, -inf
+    x[9, 8192:] = low
+    xd = x.cuda()
+    announce("softmax pieces infinities", ln)
+    y = ql.softmax(xd)
+    assert _lib.lib().mllm_hip_softmax_workspace_bytes(10, ln) > 0
+    want = torch.empty_like(xd)
+    _lib.check(_lib.lib().mllm_hip_softmax(xd.data_ptr(), want.data_ptr(), 10, ln, ql._stream()), "mllm_hip_softmax")
+    y, want = y.cpu(), want.cpu()
+    assert torch.equal(y.isnan(), want.isnan())
+    ok = ~want.isnan()
+    assert ((y[ok] - want[ok]).abs() <= 124 * 2.0 ** -24 * want[ok]).all()
+
+
+@pytest.mark.parametrize("ln", [4100, 8193, 151_936])
+@pytest.mark.parametrize("k", [1, 50, 128])
+def test_topk_pieces_order_infinities_nan_and_zeros_as_whole_rows_do(ln, k):
+    """infinities of both signs, NaN of both signs, zeros of both signs (equal: the lowest index first), a row of each alone, pieces of
+    fewer finite values than k: the values and indices of one workgroup per row, largest and smallest, sorted"""
+    inf, nan = float("inf"), float("nan")
+    g = torch.Generator().manual_seed(ln + k)
+    x = torch.randn((10, ln), generator=g)
+    x[0, torch.randperm(ln, generator=g)[:40]] = inf
+    x[0, torch.randperm(ln, generator=g)[:40]] = -inf
+    x[1] = -inf
+    x[2] = inf
+    x[3] = nan
+    x[4, torch.randperm(ln, generator=g)[:30]] = nan
+    x[4, torch.randperm(ln, generator=g)[:30]] = -nan
+    x[5] = torch.where(torch.rand(ln, generator=g) < 0.5, 0.0, -0.0)
+    x[6, :] = -inf
+    x[6, ln - 3:] = torch.tensor([-0.0, 0.0, 1.0])
+    x[7, : ln // 2] = -0.0
+    x[8, 4096:] = -inf
+    x[9] = float(np.finfo(np.float32).min)
+    xd = x.cuda()
+    L = _lib.lib()
+    assert L.mllm_hip_topk_workspace_bytes(10, ln, k) > 0 or (ln % 4 and ln <= 8192)
+    for largest in (True, False):
+        announce("topk pieces infinities", ln, k, largest)
+        v, i = ql.topk(xd, k, largest, True)
+        wv, wi = torch.empty_like(v), torch.empty_like(i)
+        _lib.check(L.mllm_hip_topk(xd.data_ptr(), wv.data_ptr(), wi.data_ptr(), 10, ln, k, int(largest), 1, ql._stream()), "mllm_hip_topk")
+        assert torch.equal(i, wi) and torch.equal(v.view(torch.int32), wv.view(torch.int32))
+        finite = [0, 1, 2, 5, 6, 7, 8, 9]  # (torch puts every NaN first and leaves the order of equal values open)
+        t = torch.topk(x[finite], k, dim=1, largest=largest).values
+        assert torch.equal(v.cpu()[finite] + 0.0, t + 0.0)
+
+
 @pytest.mark.parametrize("rows,ln,k", [(2, 4096, 8), (3, 4097, 32), (2, 4100, 33), (1, 8193, 64), (2, 20000, 128), (2, 20000, 129), (1, 151936, 128),
                                        (1, 200003, 128), (257, 4097, 50)])
 def test_topk_of_rows_cut_into_pieces(rows, ln, k):
