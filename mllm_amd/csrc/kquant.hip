@@ -813,6 +813,17 @@ MLLM_API int mllm_hip_kq_set_rows_shape(int tiles, int waves) {
   return 0;
 }
 
+MLLM_API int mllm_hip_kq_rows_shape(int wtype, int64_t M, int64_t N, int64_t K) {
+  if ((wtype != MLLM_HIP_Q4_K && wtype != MLLM_HIP_Q6_K) || M < 3 || M > 8 || N <= 0 || N > 0x7fffffff || K <= 0 || K % QK_K || !kr_fits((int)(K / QK_K))) return 0;
+  KGemvArgs a{};
+  a.M = (int)M;
+  a.nsb = (int)(K / QK_K);
+  a.nparts = 1;
+  a.part[0].N = (int)N;
+  const KrShape s = kr_shape(wtype == MLLM_HIP_Q4_K, a, 1);
+  return s.tiles * 16 + s.waves;
+}
+
 MLLM_API int mllm_hip_kq_set_tuning(int lanes_per_row, int waves_per_wg, int units_in_flight) {
   auto ok = [](int v, std::initializer_list<int> allowed) {
     for (int x : allowed)

@@ -539,6 +539,11 @@ static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y, bool quant
   int tw = (int)std::min<int64_t>(moe ? 4 : 8, (tiles * grid_y + 255) / 256);
   int P = moe ? 1 : std::min(S, tw >= 5 ? 10 / tw : 16 / tw);
   while (P > 1 && (S + P - 2) / (P - 1) == (S + P - 1) / P) P--;
+  // One tile per workgroup and more than twelve slices: waves with two slices each, up to six rows and where x is quantized ahead (13 to
+  // 16 waves with one slice each have nothing in flight beside it and start later; fewer waves also make the image pay from three rows
+  // on).  13 to 16 slices, 128 to 4096 channels, us, a slice / two per wave: 3 x 2048 x 8192 Q4_K 10.1 / 8.8, Q6_K 10.8 / 9.5; 6 x 1024 x
+  // 7168 8.84 / 8.67, 10.1 / 9.9; eight rows 8.96 / 9.26, 10.2 / 10.5; with twelve slices 8.36 / 8.46, 9.1 / 9.9.
+  if (!quantizes && !moe && tw == 1 && P > 12 && P == S && a.M <= 6) P = (S + 1) / 2;
   // one tile per workgroup that quantizes x itself: waves without a slice share that, two items per thread (up to eight waves; 1024 x 1024
   // Q6_K at three / four / eight rows 5.8 / 6.3 / 8.9 -> 5.2 / 5.3 / 6.5 us, Q4_K at eight 8.3 -> 6.0; with more tiles the added waves cost
   // more than they take over, 6144 x 2048 Q6_K at eight rows 8.4 -> 9.5)

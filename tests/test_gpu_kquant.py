@@ -239,7 +239,7 @@ def test_rows_give_the_same_bits_in_every_launch_shape(wtype, M):
 
 
 @pytest.mark.parametrize("wtype", [2, 3])
-@pytest.mark.parametrize("M,Ns,K", [(3, (1, 16, 17), 256), (4, (15,), 768), (8, (33,), 1024), (5, (4097, 33), 1280), (8, (16 * 1400 + 3,), 512), (6, (40,), 15872),
+@pytest.mark.parametrize("M,Ns,K", [(3, (1, 16, 17), 256), (4, (15,), 768), (8, (33,), 1024), (5, (4097, 33), 1280), (8, (16 * 1400 + 3,), 512), (6, (40,), 15872), (6, (90,), 6912),
                                     (7, (9, 70), 16128)])
 def test_rows_kernel_edges(wtype, M, Ns, K):
     """three to eight rows: part and odd tiles of 16 channels, one to many tiles per workgroup, odd numbers of super-blocks, more waves
