@@ -813,14 +813,16 @@ MLLM_API int mllm_hip_kq_set_rows_shape(int tiles, int waves) {
   return 0;
 }
 
-MLLM_API int mllm_hip_kq_rows_shape(int wtype, int64_t M, int64_t N, int64_t K) {
-  if ((wtype != MLLM_HIP_Q4_K && wtype != MLLM_HIP_Q6_K) || M < 3 || M > 8 || N <= 0 || N > 0x7fffffff || K <= 0 || K % QK_K || !kr_fits((int)(K / QK_K))) return 0;
+MLLM_API int mllm_hip_kq_rows_shape(int wtype, int64_t M, int64_t N, int64_t K, int row_tiles) {
+  if ((wtype != MLLM_HIP_Q4_K && wtype != MLLM_HIP_Q6_K) || M < 3 || M > 8 || N <= 0 || N > 0x7fffffff || K <= 0 || K % QK_K || !kr_fits((int)(K / QK_K)) || row_tiles < 0 || row_tiles > 65535) return 0;
+  const int id = 0;
   KGemvArgs a{};
+  if (row_tiles) a.tile_expert = &id;
   a.M = (int)M;
   a.nsb = (int)(K / QK_K);
   a.nparts = 1;
   a.part[0].N = (int)N;
-  const KrShape s = kr_shape(wtype == MLLM_HIP_Q4_K, a, 1);
+  const KrShape s = kr_shape(wtype == MLLM_HIP_Q4_K, a, row_tiles ? (unsigned)row_tiles : 1u);
   return s.tiles * 16 + s.waves;
 }
 

@@ -43,7 +43,7 @@ constexpr size_t KR_LDS_MAX = 160 * 1024;
 // the image in memory: codes [super-block][unit][rows][16], then scales [super-block][8]
 static int kr_slices(int nsb) { return (nsb + KR_SPS - 1) / KR_SPS; }
 // super-blocks of a slice in MoE layers: up to five while there are at most eight slices
-__device__ __forceinline__ int kr_moe_slice(int nsb) {
+__host__ __device__ __forceinline__ int kr_moe_slice(int nsb) {
   int s = 1;
   while (s < 8 && nsb > 5 * s) s *= 2;
   return (nsb + s - 1) / s;
@@ -96,7 +96,7 @@ struct KrWeights {
 
 // blockDim = tiles per workgroup * P waves (wave = tile * P + p); XT: fp32 / bf16 activations, quantized by the workgroup, or the
 // image (KQ_IMAGE: of these eight rows; MoE row tiles: codes [rows][K], sums, scales of all rows, gathered).
-// TH = groups of four rows (Q4_K: always two).  ORDER: the sums, see above; in MoE layers one wave per tile.
+// TH = groups of four rows (Q4_K: always two).  ORDER: the sums, see above; pairs: one wave per tile.
 enum { KR_LINEAR, KR_TILES, KR_PAIRS };
 template <int WT, int XT, int TH, int ORDER>
 __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
@@ -526,12 +526,15 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
 // Tiles per workgroup and waves per tile.  A plain Linear: about one workgroup per CU, up to sixteen waves in it, none with more
 // slices than needed (2560 x 9728: one tile of ten waves 12.6 us, two tiles of eight 18; 2 x 9728 x 2560 in tiles x waves: 5 x 2
 // 12.0, 8 x 1 12.6, 2 x 8 17.2).  MoE: thousands of workgroups, small ones that share a CU (48 us with 4 x 1 for eight tokens,
-// 60 with 8 x 1, 65 with 2 x 2).
+// 60 with 8 x 1, 65 with 2 x 2).  Tiles of rows of more than ten super-blocks (four slices or more) or with few tiles spread the slices over
+// waves, or one wave's walk along K is what the layer waits for.  Experts, us of the layer, tiles x 1 / this: 8 x 512 x 3584, 5 and 28 tokens
+// Q4_K / Q6_K 33.5 / 26.4, 36.6 / 28.2; 8 x 4096 x 768 Q4_K, 5 tokens 31.8 / 27.6; 32 x 4096 x 1536 Q4_K, 18 tokens 73.5 / 70.1 (2 x 4: 74.7),
+// Q6_K 103.6 / 95.4 (4 x 2: 110.9); 4 x 2048 x 2048 Q6_K, 4 tokens 31.2 / 28.2.  Six to ten super-blocks and many tiles: 0.83 to 1.07 of the time.
 struct KrShape {
   int tiles, waves;
 };
 static KrShape g_kr_shape{0, 0};  // mllm_hip_kq_set_rows_shape
-static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y, bool quantizes = false) {
+static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y, bool quantizes = false, bool pairs = false) {
   int64_t tiles = 0;
   for (int i = 0; i < a.nparts; i++) tiles += (a.part[i].N + 15) / 16;
   const int S = kr_slices(a.nsb);
@@ -548,6 +551,16 @@ static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y, bool quant
   // Q6_K at three / four / eight rows 5.8 / 6.3 / 8.9 -> 5.2 / 5.3 / 6.5 us, Q4_K at eight 8.3 -> 6.0; with more tiles the added waves cost
   // more than they take over, 6144 x 2048 Q6_K at eight rows 8.4 -> 9.5)
   if (quantizes && !moe && tw == 1) P = std::max(P, std::min(8, (a.M * a.nsb * 32 + 127) / 128));
+  if (moe && !pairs) {
+    const int slices = (a.nsb + kr_moe_slice(a.nsb) - 1) / kr_moe_slice(a.nsb);
+    if (slices >= 4) {
+      P = q4 && tw == 4 ? 2 : 4;
+      tw = q4 && tw == 4 ? 4 : std::min(tw, 2);
+    } else if (slices == 2 && tw < 4) {
+      P = 2;
+      tw = std::min(tw, 2);
+    }
+  }
   if (g_kr_shape.tiles && !moe) tw = g_kr_shape.tiles, P = g_kr_shape.waves;
   while (P > 1 && kr_lds_bytes(q4, a.nsb, 1, P) > KR_LDS_MAX) P--;
   while (tw > 1 && kr_lds_bytes(q4, a.nsb, tw, P) > KR_LDS_MAX) tw--;
@@ -560,7 +573,7 @@ static int kr_threads(int wtype, const KGemvArgs& a) {
 template <int WT, int XT, int TH, int ORDER>
 static int launch_kq_rows(const KGemvArgs& a_in, hipStream_t st, unsigned grid_y = 1) {
   KGemvArgs a = a_in;
-  const KrShape shape = kr_shape(WT == MLLM_HIP_Q4_K, a, grid_y, XT != KQ_IMAGE);
+  const KrShape shape = kr_shape(WT == MLLM_HIP_Q4_K, a, grid_y, XT != KQ_IMAGE, ORDER == KR_PAIRS);
   const int tw = shape.tiles, P = shape.waves;
   const size_t lds = kr_lds_bytes(WT == MLLM_HIP_Q4_K, a.nsb, tw, P);
   if (lds > KR_LDS_MAX) return MLLM_HIP_E_SHAPE;

@@ -84,7 +84,7 @@ def _cases():
                                         [(0, Q4_0, BADARG), (1, 0, BADARG), (1, 5, BADARG), (2, None, BADARG), (3, None, BADARG),
                                          (4, IMAGE, BADARG), (5, 0, BADARG), (6, 320, SHAPE), (7, ODD, ALIGN), (8, 8 * 256 + 8 * 36 - 1, BADARG)]),
         "mllm_hip_kq_set_rows_shape": ([0, 0], [(0, 1, BADARG), (1, 1, BADARG), (0, -1, BADARG)]),
-        "mllm_hip_kq_rows_shape": ([Q4_K, 5, 64, 4096], [(0, Q4_0, 0), (1, 2, 0), (1, 9, 0), (2, 0, 0), (3, 320, 0), (3, 16128, 0)]),
+        "mllm_hip_kq_rows_shape": ([Q4_K, 5, 64, 4096, 0], [(0, Q4_0, 0), (1, 2, 0), (1, 9, 0), (2, 0, 0), (3, 320, 0), (3, 16128, 0), (4, -1, 0)]),
         "mllm_hip_kq_set_slice_meeting": ([-1, 0], [(0, 2, BADARG), (0, -2, BADARG), (1, 9, BADARG), (1, -1, BADARG)]),
         # switches for comparison runs: anything but 0 and 1 is refused and leaves the setting alone
         "mllm_hip_w8a8_set_decode": ([1], [(0, 2, BADARG), (0, -1, BADARG)]),
@@ -154,8 +154,18 @@ def test_long_rows_of_few_channels_take_two_slices_per_wave(wtype, N):
     """three to six rows of 13 to 16 K slices, one tile per workgroup: a wave per slice was 3 to 17 % slower than two slices per wave"""
     shape = _lib.lib().mllm_hip_kq_rows_shape
     for K, waves in ((6144, 12), (6400, 7), (6656, 7), (7168, 7), (7680, 8), (8192, 8), (8448, 9)):
-        assert [shape(wtype, M, N, K) - 16 for M in (3, 4, 6)] == [waves] * 3
-    assert shape(wtype, 8, N, 8192) == 16 + 16 and shape(wtype, 3, 4112, 8192) == 2 * 16 + 8
+        assert [shape(wtype, M, N, K, 0) - 16 for M in (3, 4, 6)] == [waves] * 3
+    assert shape(wtype, 8, N, 8192, 0) == 16 + 16 and shape(wtype, 3, 4112, 8192, 0) == 2 * 16 + 8
+
+
+def test_moe_tiles_of_long_rows_spread_their_slices_over_waves():
+    """one wave per tile walked all of K: 4 to 21 % slower than a workgroup per slice with eight experts of 3584 or 4096 elements"""
+    shape = lambda *a: divmod(_lib.lib().mllm_hip_kq_rows_shape(*a), 16)  # noqa: E731
+    for wtype in (Q4_K, Q6_K):
+        assert shape(wtype, 8, 512, 3584, 10) == (2, 4) and shape(wtype, 8, 512, 3584, 5) == (1, 4)
+        assert shape(wtype, 8, 2048, 2048, 5) == (2, 2) and shape(wtype, 8, 16, 1536, 9) == (1, 2)
+        assert shape(wtype, 8, 2048, 768, 100) == (4, 1) and shape(wtype, 8, 1536, 2048, 129) == (4, 1)
+    assert shape(Q4_K, 8, 2 * 768, 4096, 10) == (4, 2) and shape(Q6_K, 8, 2 * 768, 4096, 10) == (2, 4)
 
 
 def test_topk_is_cut_into_pieces_only_where_that_is_faster():

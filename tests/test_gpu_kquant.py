@@ -336,10 +336,11 @@ def _moe_tile_sums(x, W, wtype):
     return total
 
 
-@pytest.mark.parametrize("wtype,wdown,E,H,I", [(2, 2, 8, 2816, 512), (3, 3, 8, 2816, 512), (2, 3, 40, 1536, 512), (3, 2, 40, 512, 1536)])
+@pytest.mark.parametrize("wtype,wdown,E,H,I", [(2, 2, 8, 2816, 512), (3, 3, 8, 2816, 512), (2, 3, 40, 1536, 512), (3, 2, 40, 512, 1536), (2, 3, 8, 512, 3584),
+                                               (3, 2, 8, 4096, 256), (3, 2, 8, 512, 2048), (3, 2, 40, 4096, 512)])
 def test_moe_tiles_keep_the_order_of_their_sums(wtype, wdown, E, H, I):
-    """eight-row tiles, sorted (8 experts) and found by the workgroups (40): bit for bit the stated fp32 order, through SiLU, the
-    second quantization and the weighted sum (one pair per token)"""
+    """eight-row tiles (three pairs per expert and less), sorted (8 experts) and found by the workgroups (40), slices one after another and
+    spread over waves: bit for bit the stated fp32 order, through SiLU, the second quantization and the weighted sum (one pair per token)"""
     T, rng = 24, synth.rng_for(9, 7500 + wtype + 5 * wdown + E)
     Wg, Wu, Wd = (synth.make_weight(rng, wt, E * n, K).reshape(E, n, K // 256, -1) for wt, n, K in ((wtype, I, H), (wtype, I, H), (wdown, H, I)))
     g, u, d = (ql.PackedKExperts(wt, torch.from_numpy(W)) for wt, W in ((wtype, Wg), (wtype, Wu), (wdown, Wd)))
