@@ -58,11 +58,14 @@ struct MMElem<MLLM_HIP_F32> {
 // thread and vector, which makes one dword of LDS per row.
 // Whole tiles load whole vectors whatever the alignment of the rows (odd row lengths among them); rows past the end repeat the
 // last ones (their results are never stored).  A K step that ends behind K, and a last tile of rows that are not a multiple of
-// the vector in a [K][rows] tensor, load element by element with zeros outside; VECTORS: the shape has neither but K steps whose
+// the vector in a [K][rows] tensor, load element by element with zeros outside; MM_VECTORS: the shape has neither but K steps whose
 // vectors lie inside or outside as a whole (mm_vectors below), and no element by element code: the short products that this is for
-// are bound by their few K steps (bf16 1000 x 8 x 8 x 8: 4.7 us by elements, 3.3; 8 x 800 x 64 x 200 5.7 / 4.8).
-template <typename E, int ROWS, bool CONTIG_K, bool VECTORS>
+// are bound by their few K steps (bf16 1000 x 8 x 8 x 8: 4.7 us by elements, 3.3; 8 x 800 x 64 x 200 5.7 / 4.8).  MM_STEP: one K step, element
+// by element and nothing else: 0.3 to 0.5 us of a launch are waits for code (8 x 69 x 7 x 18 bf16 4.84 us with the general form's, 4.4).
+enum { MM_ANY, MM_VECTORS, MM_STEP };
+template <typename E, int ROWS, bool CONTIG_K, int FORM>
 struct MMTile {
+  static constexpr bool VECTORS = FORM == MM_VECTORS;
   static constexpr int VE = 16 / (int)sizeof(E);
   static constexpr bool KROWS = !CONTIG_K && sizeof(E) == 4;   // [k][row] in LDS
   static constexpr bool PAIRS = !CONTIG_K && sizeof(E) == 2;   // two k of four rows per vector
@@ -93,6 +96,7 @@ struct MMTile {
     else k = idx / (ROWS / VE), r = (idx % (ROWS / VE)) * VE;
   }
   __device__ __forceinline__ void start(const E* __restrict__ X, int row0, int rows, int K) {
+    if (FORM == MM_STEP) return;
     whole = CONTIG_K || VECTORS || (rows >= RV && (row0 + ROWS <= rows || rows % RV == 0));  // (the same in every thread)
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
@@ -115,7 +119,7 @@ struct MMTile {
     return q;
   }
   __device__ __forceinline__ void load(const E* __restrict__ X, int row0, int k0, int rows, int K) {
-    if (VECTORS ? k0 + 32 <= K : whole && k0 + 32 <= K) {
+    if (FORM != MM_STEP && (VECTORS || whole) && k0 + 32 <= K) {
       const int64_t step = CONTIG_K ? (int64_t)k0 : (int64_t)k0 * rows;
 #pragma unroll
       for (int c = 0; c < NV; ++c) v[c] = vector(p[c] + step, rows);
@@ -181,19 +185,19 @@ struct MMTile {
 // three (4096 x 4096 x 4096 bf16: 236 -> 180 us).
 //   (heads x rows x keys x d) fp32 8 x 3108 x 777 x 128: scores 80 -> 59 us, values 97 -> 65; bf16 33 -> 23, 70 -> 26 (odd row lengths
 //   loaded element by element and transposed through 16 two-byte LDS stores before)
-template <int DT, bool TA, bool TB, int TM, int TN, bool VECTORS>
+template <int DT, bool TA, bool TB, int TM, int TN, int FORM>
 __global__ __launch_bounds__(256, (TM * TN == 4 && DT != MLLM_HIP_F32) ? 4 : 1) void matmul_kernel(MMArgs a, int tiles, int tilesM, uint32_t inv_tiles, uint32_t inv_tilesM) {
   using E = typename MMElem<DT>::type;
   constexpr int BM = 64 * TM, BN = 64 * TN;
   // A is [M][K], or [K][M] when transposed; B is [K][N], or [N][K] when transposed
-  typedef MMTile<E, BM, !TA, VECTORS> TileA;
-  typedef MMTile<E, BN, TB, VECTORS> TileB;
+  typedef MMTile<E, BM, !TA, FORM> TileA;
+  typedef MMTile<E, BN, TB, FORM> TileB;
   __shared__ __align__(16) E sA[TileA::SIZE];
   __shared__ __align__(16) E sB[TileB::SIZE];
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave >> 1, wn = wave & 1, r = lane & 31, h = lane >> 5;
-  const int KT = (a.K + 31) / 32;
+  const int KT = FORM == MM_STEP ? 1 : (a.K + 31) / 32;
   const int total = tiles * a.batch, b = mm_block();
   if (b >= total) return;  // (uniform)
   const int t = xcd_run(b, total), z = mm_div(t, tiles, inv_tiles), in = t - z * tiles;
@@ -325,7 +329,7 @@ __global__ __launch_bounds__(MMR_WAVES * 64) void matmul_rows_kernel(MMArgs a, i
   auto mac = [&](u32x4 bv, int m, E e) {
     const float am = mm_to_f32<DT>(e);
 #pragma unroll
-    for (int j = 0; j < VE; j++) acc[m][j] = fmaf(am, mm_to_f32<DT>(MMTile<E, 64, true, false>::elem(bv, j)), acc[m][j]);
+    for (int j = 0; j < VE; j++) acc[m][j] = fmaf(am, mm_to_f32<DT>(MMTile<E, 64, true, MM_ANY>::elem(bv, j)), acc[m][j]);
   };
   const int kstep = MMR_WAVES * rpw * UB;
   int k = (wave * rpw + sub) * UB;
@@ -426,9 +430,9 @@ __global__ __launch_bounds__(256) void matmul_dots_kernel(MMArgs a, int g_log2, 
     for (int u = 0; u < UB; u++)
 #pragma unroll
       for (int j = 0; j < VE; j++) {
-        const float bf = mm_to_f32<DT>(MMTile<E, 64, true, false>::elem(bv[u], j));
+        const float bf = mm_to_f32<DT>(MMTile<E, 64, true, MM_ANY>::elem(bv[u], j));
 #pragma unroll
-        for (int m = 0; m < MR; m++) acc[u][m] = fmaf(mm_to_f32<DT>(MMTile<E, 64, true, false>::elem(av[m], j)), bf, acc[u][m]);
+        for (int m = 0; m < MR; m++) acc[u][m] = fmaf(mm_to_f32<DT>(MMTile<E, 64, true, MM_ANY>::elem(av[m], j)), bf, acc[u][m]);
       }
   }
 #pragma unroll
@@ -533,9 +537,10 @@ static int launch_matmul(const MMArgs& a, hipStream_t st) {
     }
     return (int)hipGetLastError();
   };
-  if (matmul_large_tile<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 2, 2, false>, 128);
-  if (mm_vectors<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 1, 1, true>, 64);
-  return go(matmul_kernel<DT, TA, TB, 1, 1, false>, 64);
+  if (matmul_large_tile<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 2, 2, MM_ANY>, 128);
+  if (mm_vectors<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 1, 1, MM_VECTORS>, 64);
+  if (a.K <= 32) return go(matmul_kernel<DT, TA, TB, 1, 1, MM_STEP>, 64);
+  return go(matmul_kernel<DT, TA, TB, 1, 1, MM_ANY>, 64);
 }
 
 template <int DT>
