@@ -62,7 +62,8 @@ struct MMElem<MLLM_HIP_F32> {
 // vectors lie inside or outside as a whole (mm_vectors below), and no element by element code: the short products that this is for
 // are bound by their few K steps (bf16 1000 x 8 x 8 x 8: 4.7 us by elements, 3.3; 8 x 800 x 64 x 200 5.7 / 4.8).  MM_STEP: one K step, element
 // by element and nothing else: 0.3 to 0.5 us of a launch are waits for code (8 x 69 x 7 x 18 bf16 4.84 us with the general form's, 4.4).
-enum { MM_ANY, MM_VECTORS, MM_STEP };
+// MM_NARROW: rows past the end are not requested again but stay zero (mm_narrow below).
+enum { MM_ANY, MM_VECTORS, MM_STEP, MM_NARROW };
 template <typename E, int ROWS, bool CONTIG_K, int FORM>
 struct MMTile {
   static constexpr bool VECTORS = FORM == MM_VECTORS;
@@ -76,7 +77,7 @@ struct MMTile {
   static_assert(ROWS * 32 / VE % 256 == 0, "tile must split evenly over 256 threads");
   u32x4 v[NV];
   const E* p[NV];
-  bool whole;
+  bool whole, inside[FORM == MM_NARROW ? NV : 1];
 
   static __device__ __forceinline__ uint32_t bits(E e) {
     if constexpr (sizeof(E) == 4) return __builtin_bit_cast(uint32_t, e);
@@ -102,6 +103,10 @@ struct MMTile {
     for (int c = 0; c < NV; ++c) {
       int r, k;
       place(c, r, k);
+      if constexpr (FORM == MM_NARROW) {
+        inside[c] = row0 + r < rows;
+        v[c] = u32x4{0u, 0u, 0u, 0u};
+      }
       if (CONTIG_K) p[c] = X + (int64_t)min(row0 + r, rows - 1) * K + k;
       else p[c] = X + (int64_t)k * rows + (whole ? min(row0 + r, rows - RV) : 0);
     }
@@ -122,7 +127,8 @@ struct MMTile {
     if (FORM != MM_STEP && (VECTORS || whole) && k0 + 32 <= K) {
       const int64_t step = CONTIG_K ? (int64_t)k0 : (int64_t)k0 * rows;
 #pragma unroll
-      for (int c = 0; c < NV; ++c) v[c] = vector(p[c] + step, rows);
+      for (int c = 0; c < NV; ++c)
+        if (FORM != MM_NARROW || inside[FORM == MM_NARROW ? c : 0]) v[c] = vector(p[c] + step, rows);
       return;
     }
     if constexpr (VECTORS) {
@@ -191,7 +197,7 @@ __global__ __launch_bounds__(256, (TM * TN == 4 && DT != MLLM_HIP_F32) ? 4 : 1) 
   constexpr int BM = 64 * TM, BN = 64 * TN;
   // A is [M][K], or [K][M] when transposed; B is [K][N], or [N][K] when transposed
   typedef MMTile<E, BM, !TA, FORM> TileA;
-  typedef MMTile<E, BN, TB, FORM> TileB;
+  typedef MMTile<E, BN, TB, FORM == MM_NARROW ? MM_ANY : FORM> TileB;
   __shared__ __align__(16) E sA[TileA::SIZE];
   __shared__ __align__(16) E sB[TileB::SIZE];
 
@@ -512,6 +518,15 @@ static bool mm_vectors(const MMArgs& a) {
   return fits(!TA, a.M) && fits(TB, a.N);
 }
 
+// Few rows of A against many of B, fp32 [M][K] x [N][K]: the tile's other rows would repeat A's last one through the L1, whose requests are
+// what such a product waits for when it fills the chip.  us, repeated / left out: 33 x 12 x 2732 x 1080 171 / 146, 48 x 8 x 2840 x 624 127 /
+// 113, 16 x 20 x 3148 x 692 (800 tiles) 59.1 / 56.8; with fewer tiles the branch costs more (10 x 20 x 920 x 432, 150 tiles: 12.6 / 13.3),
+// in the other orders and in 16 bits up to 1.6 times as much.
+template <int DT, bool TA, bool TB>
+static bool mm_narrow(const MMArgs& a) {
+  return DT == MLLM_HIP_F32 && !TA && TB && a.M <= 32 && (int64_t)((a.N + 63) / 64) * a.batch >= 800;
+}
+
 template <int DT, bool TA, bool TB>
 static int launch_matmul(const MMArgs& a, hipStream_t st) {
   if constexpr (!TA && !TB) {
@@ -538,6 +553,9 @@ static int launch_matmul(const MMArgs& a, hipStream_t st) {
     return (int)hipGetLastError();
   };
   if (matmul_large_tile<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 2, 2, MM_ANY>, 128);
+  if constexpr (DT == MLLM_HIP_F32 && !TA && TB) {
+    if (a.K > 32 && mm_narrow<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 1, 1, MM_NARROW>, 64);
+  }
   if (mm_vectors<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 1, 1, MM_VECTORS>, 64);
   if (a.K <= 32) return go(matmul_kernel<DT, TA, TB, 1, 1, MM_STEP>, 64);
   return go(matmul_kernel<DT, TA, TB, 1, 1, MM_ANY>, 64);

@@ -147,9 +147,11 @@ def test_short_matmuls_of_whole_vectors(batch, M, N, K, ta, tb, dtype):
 
 @pytest.mark.parametrize("dtype", ["fp32", "bf16", "fp16"])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
-@pytest.mark.parametrize("batch,M,N,K", [(4, 70, 7, 18), (1, 65, 130, 1), (2, 5, 3, 32), (3, 67, 129, 31), (2, 130, 66, 5)])
-def test_matmul_of_one_k_step(batch, M, N, K, ta, tb, dtype):
-    """one K step loaded element by element: exact as above, and an infinity in the last row and a NaN at the last k stay in their own row and column"""
+@pytest.mark.parametrize("batch,M,N,K", [(4, 70, 7, 18), (1, 65, 130, 1), (2, 5, 3, 32), (3, 67, 129, 31), (2, 130, 66, 5), (100, 12, 520, 132),
+                                         (101, 31, 513, 37), (40, 32, 1280, 64), (90, 5, 577, 33)])
+def test_matmul_of_one_k_step_and_of_few_rows_by_many(batch, M, N, K, ta, tb, dtype):
+    """one K step loaded element by element; up to 32 rows x [N][K] over 800 tiles and more (fp32: rows past the end left out), the last K
+    step ending behind K: exact as above, and an infinity in the last row and a NaN at the last k stay in their own row and column"""
     rng = synth.rng_for(6, 6000 + batch + M + N + K)
     td = {"fp32": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
     a = torch.from_numpy(rng.integers(1, 9, (batch, M, K)).astype(np.float32))
@@ -158,7 +160,7 @@ def test_matmul_of_one_k_step(batch, M, N, K, ta, tb, dtype):
     b[:, 1, K - 1], a[:, M - 1, 0] = float("nan"), float("inf")
     want = torch.matmul(a, b.transpose(1, 2).contiguous())
     assert want[:, :M - 1].isfinite().sum() == batch * (M - 1) * (N - 1) and want[:, M - 1, N - 1].isinf().all()
-    announce("matmul one step %s %s ta=%d tb=%d" % (dtype, (batch, M, N, K), ta, tb))
+    announce("matmul one step / narrow %s %s ta=%d tb=%d" % (dtype, (batch, M, N, K), ta, tb))
     ad, bd = a.transpose(1, 2).contiguous() if ta else a, b if tb else b.transpose(1, 2).contiguous()
     c = ql.matmul(ad.to(td).cuda(), bd.to(td).cuda(), ta, tb).cpu()
     want = want.to(td)
