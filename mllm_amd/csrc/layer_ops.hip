@@ -824,7 +824,7 @@ __global__ __launch_bounds__(NT) void topk_select_rows_kernel(const float* __res
   }
 }
 
-// Few long rows spread over the chip (mllm_hip_topk_ws), k up to 128: a row is cut into pieces of TOPK_PIECE elements, a
+// Few long rows spread over the chip (mllm_hip_topk_ws), k up to 128: a row is cut into equal pieces of at most TOPK_PIECE elements, a
 // workgroup selects the k largest keys of its piece into the caller's workspace, and a second launch selects among the
 // pieces' keys.  A workgroup per row is bound by what one CU loads per pass over the row: 20 of eight rows of 151 936 take
 // 110 us there and 12 here, 64 of them 111 and 15.
@@ -834,6 +834,8 @@ __global__ __launch_bounds__(NT) void topk_select_rows_kernel(const float* __res
 // selection, and of keys that are spread over the threads in any order they are few more than k (about 180 at k = 128).  They
 // are collected in LDS and placed by rank, up to 64 of them in the registers of one wave; should they be more than TOPK_CAND
 // (many equal values, or one thread's keys all larger than the other threads'), the k-th key itself is found a bit at a time.
+// Equal pieces, so that every thread has elements: a last piece of 432 (12 720 cut at 4096s) gave 108 threads four each, all of them
+// candidates for the largest 128 (256 rows of 12 720: 37.8 us, 19.7 in equal pieces, 20.3 as a workgroup per row).
 // Limits, in a graph, us, a workgroup per row / pieces, the largest 1 | 50 | 128: 8 rows of 4100: 17.6 / 8.6 | 19.1 / 12.9 | 21.3 / 13.9 (up to
 // 4096 a row is one piece, and the second launch has nothing to merge), of 151 936: 109 / 9.3 | 111 / 15.0 | 113 / 23.5; 512 rows of 4100: 19.0 /
 // 11.7 | 20.9 / 16.8 | 24.1 / 19.4, of 151 936: 256 / 76 | 260 / 101 | 264 / 143.  Pieces win on either side of 512 rows (1024 rows of 4100:
@@ -921,7 +923,7 @@ __device__ __forceinline__ int block_topk_256(const unsigned long long (&key)[R]
   return n < k ? n : k;
 }
 template <int VEC>
-__global__ __launch_bounds__(256) void topk_pieces_kernel(const float* __restrict__ x, unsigned long long* __restrict__ ws, int len, int k,
+__global__ __launch_bounds__(256) void topk_pieces_kernel(const float* __restrict__ x, unsigned long long* __restrict__ ws, int len, int per, int k,
                                                           int largest) {
   typedef typename TopkVec<VEC>::T VT;
   __shared__ TopkShared sh;
@@ -929,17 +931,17 @@ __global__ __launch_bounds__(256) void topk_pieces_kernel(const float* __restric
   const int tid = threadIdx.x, piece = blockIdx.x;
   const int64_t row = blockIdx.y;
   const VT* xr = reinterpret_cast<const VT*>(x + row * len);
-  const int nunits = len / VEC, u0 = piece * (TOPK_PIECE / VEC) + tid;  // (VEC divides len)
+  const int u0 = piece * per + tid, end = min(len / VEC, (piece + 1) * per);  // per: vectors of a piece (VEC divides len)
   VT v[RV];
 #pragma unroll
-  for (int j = 0; j < RV; j++) v[j] = u0 + 256 * j < nunits ? xr[u0 + 256 * j] : VT{};
+  for (int j = 0; j < RV; j++) v[j] = u0 + 256 * j < end ? xr[u0 + 256 * j] : VT{};
   unsigned long long key[R];
 #pragma unroll
   for (int j = 0; j < RV; j++) {
     const float* f = reinterpret_cast<const float*>(&v[j]);
 #pragma unroll
     for (int e = 0; e < VEC; e++)
-      key[j * VEC + e] = u0 + 256 * j < nunits ? order_key(f[e], (u0 + 256 * j) * VEC + e, largest != 0) : 0ull;
+      key[j * VEC + e] = u0 + 256 * j < end ? order_key(f[e], (u0 + 256 * j) * VEC + e, largest != 0) : 0ull;
   }
   const int n = block_topk_256<R>(key, k, sh);
   // the pieces' largest keys first, then their second largest ...: the large ones spread over the threads of the next launch
@@ -1317,8 +1319,9 @@ MLLM_API int mllm_hip_topk_ws(const float* x, float* values, int32_t* indices, i
   const dim3 grid((unsigned)pieces, (unsigned)rows);
   hipStream_t st = (hipStream_t)stream;
   unsigned long long* ws = reinterpret_cast<unsigned long long*>(workspace);
-  if (vec) hipLaunchKernelGGL(topk_pieces_kernel<4>, grid, dim3(256), 0, st, x, ws, (int)len, k, largest);
-  else hipLaunchKernelGGL(topk_pieces_kernel<1>, grid, dim3(256), 0, st, x, ws, (int)len, k, largest);
+  const int units = (int)(vec ? len / 4 : len), per = (units + pieces - 1) / pieces;  // (at most TOPK_PIECE elements)
+  if (vec) hipLaunchKernelGGL(topk_pieces_kernel<4>, grid, dim3(256), 0, st, x, ws, (int)len, per, k, largest);
+  else hipLaunchKernelGGL(topk_pieces_kernel<1>, grid, dim3(256), 0, st, x, ws, (int)len, per, k, largest);
   if (pieces * k <= 1024) hipLaunchKernelGGL(topk_merge_kernel<4>, dim3((unsigned)rows), dim3(256), 0, st, x, ws, values, indices, (int)len, pieces * k, k, sorted);
   else hipLaunchKernelGGL(topk_merge_kernel<TOPK_MERGE_R>, dim3((unsigned)rows), dim3(256), 0, st, x, ws, values, indices, (int)len, pieces * k, k, sorted);
   return (int)hipGetLastError();

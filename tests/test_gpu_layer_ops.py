@@ -393,6 +393,23 @@ def test_topk_of_rows_cut_into_pieces(rows, ln, k):
             assert np.array_equal(v.cpu().numpy().view(np.uint32), wv.view(np.uint32))
 
 
+@pytest.mark.parametrize("rows,ln,k", [(3, 12_720, 128), (2, 12_300, 50), (2, 8197, 64), (1, 163_844, 60), (300, 4099, 107), (1, 20_971_008, 1)])
+def test_topk_pieces_are_equal(rows, ln, k):
+    """every piece of a row leaves k keys, whatever the row's length is over the longest piece (a short last piece makes each of its elements a
+    candidate, or has fewer than k), and the selection is one workgroup's per row"""
+    L = _lib.lib()
+    x = torch.randn((rows, ln), device="cuda", generator=torch.Generator("cuda").manual_seed(ln))
+    need = L.mllm_hip_topk_workspace_bytes(rows, ln, k)
+    assert need == rows * ((ln + 4095) // 4096) * k * 8
+    announce("topk equal pieces", rows, ln, k)
+    ws = torch.zeros(need // 8, dtype=torch.int64, device="cuda")
+    v, i, wv, wi = (torch.empty((rows, k), dtype=t, device="cuda") for t in (torch.float32, torch.int32) * 2)
+    _lib.check(L.mllm_hip_topk_ws(x.data_ptr(), v.data_ptr(), i.data_ptr(), rows, ln, k, 1, 1, ws.data_ptr(), ql._stream()), "mllm_hip_topk_ws")
+    _lib.check(L.mllm_hip_topk(x.data_ptr(), wv.data_ptr(), wi.data_ptr(), rows, ln, k, 1, 1, ql._stream()), "mllm_hip_topk")
+    assert (ws != 0).all()
+    assert torch.equal(i, wi) and torch.equal(v, wv)
+
+
 @pytest.mark.parametrize("M,H,E,k,dtype", [(512, 2048, 128, 8, "f32"), (1, 2048, 128, 8, "f32"), (7, 256, 60, 4, "f32"),
                                            (33, 2048, 128, 8, "bf16"), (5, 64, 8, 2, "f32")])
 def test_moe_gate(M, H, E, k, dtype):
