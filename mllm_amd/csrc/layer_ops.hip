@@ -326,9 +326,11 @@ constexpr int SOFTMAX_PIECE = 4096;
 //   256 rows of 20 480: 16.6 / 17.4, 40 960: 32.0 / 33.4, 64 000: 48.5 / 46.1;  512 rows of 24 576: 36.6 / 38.0, 40 960: 60.4 / 56.1, 64 000: 101 /
 //   83, 151 936: 308 / 231;  1024 rows of 40 960: 131 / 106, 151 936: 603 / 455
 // Up to 16 rows the pieces win from about 22 000 elements on (and from 12 288 to 16 384, where one workgroup holds the row in registers),
-// with 256 rows from about 50 000.  The limit dates from pieces with a branch per element (32 000: 13.9) and lies late for few rows: from
-// 24 000 on no number of rows up to 512 loses more than 4 %.
+// with 256 rows from about 50 000: 193 to 256 rows are one whole round of the chip for the form of a workgroup per row, which stays up to
+// there (233 x 46 120: 33.8 / 35.7; 192 x 50 000 30.7 / 30.9, 256 x 50 000 39.1 / 39.0, 256 x 56 000 43.1 / 42.3, 320 x 40 968 43.1 / 40.0).
+// The other limit dates from pieces with a branch per element (32 000: 13.9) and lies late for few rows.
 constexpr int SOFTMAX_LONG = 40960;
+constexpr int SOFTMAX_LONG_ROUND = 50000;  // with 193 to 256 rows
 constexpr int SOFTMAX_SPLIT_ROWS = 512;
 __device__ __forceinline__ float block_max_256(float v, float* s_red) {
   v = wave_max(v);
@@ -1274,7 +1276,7 @@ MLLM_API int mllm_hip_topk(const float* x, float* values, int32_t* indices, int6
 
 // Pieces of a row that few long rows are cut into, 0 where a workgroup per row is the better form
 static int softmax_pieces(int64_t rows, int64_t len) {
-  return len > SOFTMAX_LONG && rows <= SOFTMAX_SPLIT_ROWS && len <= 0x7fffffff ? (int)((len + SOFTMAX_PIECE - 1) / SOFTMAX_PIECE) : 0;
+  return len > (rows > 192 && rows <= 256 ? SOFTMAX_LONG_ROUND : SOFTMAX_LONG) && rows <= SOFTMAX_SPLIT_ROWS && len <= 0x7fffffff ? (int)((len + SOFTMAX_PIECE - 1) / SOFTMAX_PIECE) : 0;
 }
 MLLM_API size_t mllm_hip_softmax_workspace_bytes(int64_t rows, int64_t len) {
   if (rows <= 0 || len <= 0) return 0;

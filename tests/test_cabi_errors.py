@@ -168,6 +168,14 @@ def test_moe_tiles_of_long_rows_spread_their_slices_over_waves():
     assert shape(Q4_K, 8, 2 * 768, 4096, 10) == (4, 2) and shape(Q6_K, 8, 2 * 768, 4096, 10) == (2, 4)
 
 
+def test_softmax_is_cut_into_pieces_only_where_that_is_not_slower():
+    """193 to 256 rows, one whole round of workgroups, stay a workgroup per row up to 50 000 elements"""
+    room = _lib.lib().mllm_hip_softmax_workspace_bytes
+    for rows, ln, pieces in ((1, 40960, 0), (1, 40961, 11), (192, 40968, 11), (193, 46120, 0), (256, 50000, 0), (256, 50001, 13), (257, 40968, 11),
+                             (512, 40968, 11), (513, 151936, 0)):
+        assert room(rows, ln) == rows * pieces * 8, (rows, ln)
+
+
 def test_topk_is_cut_into_pieces_only_where_that_is_faster():
     """rows without whole vectors of up to 8192 elements stay one workgroup's work while that is one round of workgroups"""
     room = _lib.lib().mllm_hip_topk_workspace_bytes
