@@ -640,6 +640,11 @@ static int launch_w4a16_auto(const W4A16PArgs& a, hipStream_t st) {
       {128, 384, 1.00f, 3.20f, 12.54f, 1.0826f}};
   constexpr int waves = 4, forms = 7;
   int form = -1;
+  // Up to eight K blocks and 64 rows: four waves, since of more most have nothing to multiply and all of them meet.  us, as many waves as
+  // below / four: 1 x 1440 x 128 3.76 / 2.85, 8 x 4096 x 512 3.99 / 3.26, 32 x 9728 x 512 4.44 / 4.40, 64 x 9728 x 128 5.40 / 3.84 (a GEMV of
+  // fp32 FMAs took 3.4 for the first)
+  if (!g_w4a16_ptile && g_w4a16_waves && a.K <= 512 && a.M <= 64)
+    return a.M <= 8 ? wk_gemm_launch<W4A16Waves, 1, 1, 4, 1, 1>(a, st) : wk_gemm_launch<W4A16Waves, 1, 1, 4, 1>(a, st);
   switch (g_w4a16_ptile) {
     case 0: break;
     case 1: form = 6; break;

@@ -138,9 +138,9 @@ def test_decode_gemv_packed_vs_oracle_and_tiles(M):
 @pytest.mark.parametrize("M", [1, 5, 8])
 def test_one_piece_of_eight_rows_gives_the_bits_of_the_whole_tile(M):
     """up to eight tokens load and sum one piece of a 32-row tile; 9 and 32 tokens take the same form with all four (the costs depend on
-    the tiles only).  16 waves, 8 waves and 8 waves on 64 channels, ragged N, N % 4 != 0, one K block and K blocks that do not divide;
+    the tiles only).  16 waves, 8 waves, 8 waves on 64 channels and 4 waves (K up to 512), ragged N, N % 4 != 0, one K block and K blocks that do not divide;
     rows past the batch of NaN and infinities must not reach it"""
-    for N, K, group in ((40, 64, 64), (1030, 1984, 64), (33, 8192, 128), (8195, 128, 64), (8202, 2048, 128), (40_001, 64, 64)):
+    for N, K, group in ((40, 64, 64), (1030, 448, 64), (77, 512, 128), (77, 576, 64), (1030, 1984, 64), (33, 8192, 128), (8195, 128, 64), (8202, 2048, 128), (40_001, 64, 64)):
         rng = synth.rng_for(2, 1700 + M + N + K)
         qw, s, zp, _, _ = synth.make_w4a16(rng, N, K, group)
         a_bits, _ = synth.make_x_bf16(rng, 32, K)
