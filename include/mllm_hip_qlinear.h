@@ -306,6 +306,9 @@ int mllm_hip_w8a8_set_decode_mfma_from(int tokens);
 /* Tile override for the weights-from-global kernel (packed entry points and tile 4 above): 0 heuristic, 1 = 128x384,
  * 2 = 64x384, 3 = 128x128, 4 = 64x128, 5 = 128x256. */
 int mllm_hip_w8a8_nsplit_set_tuning(int tile);
+/* The form that a product of this size takes against prepacked weights: 1 / 2 / 3 waves that split K of a tile of 32x32 / 32x64 / 64x64, 4 / 5 / 6 /
+ * 7 / 8 tiles of 64x128 / 128x128 / 128x256 / 64x384 / 128x384, 9 the dot form.  Host only, overrides aside.  No counterpart in the reference. */
+int mllm_hip_w8a8_packed_form(int64_t M, int64_t N, int64_t K);
 
 /* ---------------------------------------------------------------------------------------------------------
  * W4A16 Linear (prefill): bf16 activations x uint4 weights, per-group fp16 scale and uint4 zero-point
@@ -362,6 +365,9 @@ int mllm_hip_w4a16_set_decode_mfma_from(int tokens);
 /* Tile override for the packed GEMM: 0 heuristic, 1 = 128x384, 2 = 64x384, 3 = 128x128, 4 = 64x128, 5 = 128x256;
  * + 16 switches off the half-height tiles that shorten a partly filled last round. */
 int mllm_hip_w4a16_packed_set_tuning(int tile);
+/* The form that a product of this size takes: waves that split K of a tile of 32x32 by 1: sixteen, 2: eight, 10: four, 3: 32x64, 4: 64x64; tiles of
+ * 5: 128x128, 6: 128x256, 7: 128x384, 8: 64x128, 9: 64x384.  Host only, overrides aside.  No counterpart in the reference. */
+int mllm_hip_w4a16_packed_form(int64_t M, int64_t N, int64_t K);
 
 /* ---------------------------------------------------------------------------------------------------------
  * MoE expert FFN over expert-sorted tokens, Q4_0 / Q8_0 expert weights

@@ -130,6 +130,7 @@ def lib():
         L.mllm_hip_w8a8_linear.argtypes = [vp, ci, vp, vp, vp, vp, i64, i64, i64, vp, vp]
         L.mllm_hip_w8a8_set_tuning.argtypes = [ci]
         L.mllm_hip_w8a8_nsplit_set_tuning.argtypes = [ci]
+        L.mllm_hip_w8a8_packed_form.argtypes = [i64, i64, i64]
         L.mllm_hip_w8a8_packed_bytes.restype = C.c_size_t
         L.mllm_hip_w8a8_packed_bytes.argtypes = [i64, i64]
         L.mllm_hip_w8a8_prepack.argtypes = [vp, i64, i64, vp, vp]
@@ -140,6 +141,7 @@ def lib():
         L.mllm_hip_w4a16_from_awq.argtypes = [vp, vp, vp, i64, i64, ci, vp, vp, vp, vp]
         L.mllm_hip_w4a16_set_tuning.argtypes = [ci]
         L.mllm_hip_w4a16_packed_set_tuning.argtypes = [ci]
+        L.mllm_hip_w4a16_packed_form.argtypes = [i64, i64, i64]
         L.mllm_hip_w4a16_packed_bytes.restype = C.c_size_t
         L.mllm_hip_w4a16_packed_bytes.argtypes = [i64, i64, ci]
         L.mllm_hip_w4a16_prepack.argtypes = [vp, vp, vp, i64, i64, ci, vp, vp]

@@ -628,45 +628,53 @@ static int g_w4a16_waves = 1;  // 0: only the weights-from-global tiles (compari
 
 // Which form runs.  The waves-split-K forms (wk_gemm.h) serve from one token to about the batch whose large tiles fill the chip;
 // 93 x 2048 x 6144: 43.6 -> 10.5 us, 1 x 2560 x 9728: 15.9 (a GEMV of fp32 FMAs) -> 11.9, 300 x 9728 x 2560: 36 -> 28, 2048 rows as before.
-// The costs are fitted to 98 shapes within 6 to 10 % (rms); the choice by cost is within 0.5 % of the best form on average, 9 % at worst.
-static int launch_w4a16_auto(const W4A16PArgs& a, hipStream_t st) {
-  static const FormCost cost[] = {
-      {32, 32, 0.75f, 1.32f, 2.22f, 0.0906f},   // 16 waves
-      {32, 32, 0.50f, 3.15f, 0.54f, 0.0879f},   // 8 waves, two workgroups per CU
-      {32, 64, 0.75f, 3.20f, 0.85f, 0.1206f},   // 8 waves
-      {64, 64, 0.50f, 3.79f, 0.95f, 0.2008f},   // 4 waves, two workgroups per CU
-      {128, 128, 0.00f, 5.66f, 0.00f, 0.6687f},  // weights-from-global tiles
-      {128, 256, 0.75f, 7.69f, 0.46f, 0.8890f},
-      {128, 384, 1.00f, 3.20f, 12.54f, 1.0826f}};
-  constexpr int waves = 4, forms = 7;
-  int form = -1;
+// Two tables: where tiles of 128 x 256 would be fewer than 192, costs fitted to 1703 random shapes (5 to 6000 rows, 64 to 22 000 channels, K 64
+// to 10 000) within 4 to 8 % (rms, where a form is near the best); from 192 tiles on, costs fitted to 98 shapes of 512 and more channels, which
+// are within 0.2 % of the best form there on average, 8 % at worst.  Over all the choice takes 1.009 times the best form's time (28 % more at
+// worst, 1194 x 392 x 8960; more than 10 % in 34) and is more than 5 % slower than the tiles by rows and columns alone that ran before in 7;
+// the second table for all sizes, without the tiles of 64 rows, made that 1.037, 266 and 130 (3500 x 456 x 1280: 18.3 us, 14.0 now).
+static int w4a16_packed_form(int64_t M, int64_t N, int64_t K, bool tiles_only) {
   // Up to eight K blocks and 64 rows: four waves, since of more most have nothing to multiply and all of them meet.  us, as many waves as
   // below / four: 1 x 1440 x 128 3.76 / 2.85, 8 x 4096 x 512 3.99 / 3.26, 32 x 9728 x 512 4.44 / 4.40, 64 x 9728 x 128 5.40 / 3.84 (a GEMV of
   // fp32 FMAs took 3.4 for the first)
-  if (!g_w4a16_ptile && g_w4a16_waves && a.K <= 512 && a.M <= 64)
-    return a.M <= 8 ? wk_gemm_launch<W4A16Waves, 1, 1, 4, 1, 1>(a, st) : wk_gemm_launch<W4A16Waves, 1, 1, 4, 1>(a, st);
-  switch (g_w4a16_ptile) {
-    case 0: break;
-    case 1: form = 6; break;
-    case 3: form = 4; break;
-    case 5: form = 5; break;
-    case 2: return launch_w4a16_nsplit<2, 3, 128, 2>(a, st);
-    default: return launch_w4a16_nsplit<2, 1, 128, 2>(a, st);
-  }
-  if (form < 0) {
-    float best = 0.f;
-    for (int f = g_w4a16_waves ? 0 : waves; f < forms; f++) {
-      const float c = form_cost(cost[f], a.M, a.N, (a.K + 63) / 64);
-      if (form < 0 || c < best) {
-        best = c;
-        form = f;
-      }
+  if (!tiles_only && K <= 512 && M <= 64) return 9;
+  constexpr int waves = 4, most = 9;
+  static const FormCost few[most] = {
+      {32, 32, 1, 1.0f, 1.00f, 2.408f, 1.616f, 0.06823f, 0.292f, 3.379f},     // 16 waves
+      {32, 32, 1, 1.0f, 0.75f, 3.452f, 0.1624f, 0.07441f, 0.3295f, 2.168f},   // 8 waves, two workgroups per CU
+      {32, 64, 1, 1.0f, 1.00f, 3.91f, 0.1143f, 0.1137f, 0.1157f, 1.484f},     // 8 waves
+      {64, 64, 1, 1.0f, 0.75f, 4.599f, 0.03457f, 0.1918f, 0.2428f, 0.9395f},  // 4 waves, two workgroups per CU
+      {128, 128, 3, 0.7f, 0.25f, 4.537f, 0.f, 0.631f, 0.288f, 0.3427f},       // weights-from-global tiles
+      {128, 256, 1, 1.0f, 0.50f, 5.655f, 0.f, 0.8938f, 0.1696f, 0.3077f},
+      {128, 384, 1, 1.0f, 1.00f, 4.017f, 3.449f, 1.104f, 0.1419f, 0.348f},
+      {64, 128, 2, 0.6f, 0.50f, 3.84f, 0.1499f, 0.4126f, 0.1031f, 0.5252f},
+      {64, 384, 1, 1.0f, 0.50f, 5.6f, 0.f, 0.8473f, 0.1218f, 0.3584f}};
+  static const FormCost many[] = {{32, 32, 1, 1.f, 0.75f, 1.32f, 2.22f, 0.0906f, 0.f, 0.f},   {32, 32, 1, 1.f, 0.50f, 3.15f, 0.54f, 0.0879f, 0.f, 0.f},
+                                  {32, 64, 1, 1.f, 0.75f, 3.20f, 0.85f, 0.1206f, 0.f, 0.f},   {64, 64, 1, 1.f, 0.50f, 3.79f, 0.95f, 0.2008f, 0.f, 0.f},
+                                  {128, 128, 1, 1.f, 0.00f, 5.66f, 0.f, 0.6687f, 0.f, 0.f},   {128, 256, 1, 1.f, 0.75f, 7.69f, 0.46f, 0.8890f, 0.f, 0.f},
+                                  {128, 384, 1, 1.f, 1.00f, 3.20f, 12.54f, 1.0826f, 0.f, 0.f}};
+  const bool large = ((M + 127) / 128) * ((N + 255) / 256) >= 192;
+  const FormCost* cost = large ? many : few;
+  const int forms = large ? 7 : most;
+  int form = -1;
+  float best = 0.f;
+  for (int f = tiles_only ? waves : 0; f < forms; f++) {
+    const float c = form_cost(cost[f], M, N, K, (K + 63) / 64);
+    if (form < 0 || c < best) {
+      best = c;
+      form = f;
     }
   }
+  return form;
+}
+static int launch_w4a16_auto(const W4A16PArgs& a, hipStream_t st) {
+  static const int tiles[] = {-1, 6, 8, 4, 7, 5};  // of g_w4a16_ptile
+  const int form = g_w4a16_ptile ? tiles[g_w4a16_ptile] : w4a16_packed_form(a.M, a.N, a.K, !g_w4a16_waves);
   if (a.M <= 8) switch (form) {  // one piece of eight rows; faster at every size measured (512 to 22016 channels, K 512 to 11008)
     case 0: return wk_gemm_launch<W4A16Waves, 1, 1, 16, 2, 1>(a, st);
     case 1: return wk_gemm_launch<W4A16Waves, 1, 1, 8, 3, 1>(a, st);
     case 2: return wk_gemm_launch<W4A16Waves, 1, 2, 8, 1, 1>(a, st);
+    case 9: return wk_gemm_launch<W4A16Waves, 1, 1, 4, 1, 1>(a, st);
   }
   switch (form) {
     case 0: return wk_gemm_launch<W4A16Waves, 1, 1, 16, 2>(a, st);
@@ -675,7 +683,10 @@ static int launch_w4a16_auto(const W4A16PArgs& a, hipStream_t st) {
     case 3: return wk_gemm_launch<W4A16Waves, 2, 2, 4, 2>(a, st);
     case 4: return launch_w4a16_nsplit<4, 1, 64, 3>(a, st);
     case 5: return launch_w4a16_nsplit<4, 2, 64, 2>(a, st);
-    default: return launch_w4a16_nsplit<4, 3, 128, 1>(a, st);
+    case 6: return launch_w4a16_nsplit<4, 3, 128, 1>(a, st);
+    case 7: return launch_w4a16_nsplit<2, 1, 128, 2>(a, st);
+    case 8: return launch_w4a16_nsplit<2, 3, 128, 2>(a, st);
+    default: return wk_gemm_launch<W4A16Waves, 1, 1, 4, 1>(a, st);
   }
 }
 
@@ -703,6 +714,9 @@ MLLM_API int mllm_hip_w4a16_set_tuning(int tile) {
   return 0;
 }
 
+MLLM_API int mllm_hip_w4a16_packed_form(int64_t M, int64_t N, int64_t K) {
+  return M < 1 || N < 1 || K < 1 ? 0 : 1 + w4a16_packed_form(M, N, K, false);
+}
 MLLM_API int mllm_hip_w4a16_packed_set_tuning(int tile) {
   if (tile < 0 || (tile & 15) > 5 || tile > 31) return MLLM_HIP_E_BADARG;
   g_w4a16_ptile = tile & 15;

@@ -715,30 +715,41 @@ static bool launch_w8a8_gemv_packed(const W8A8Args& a, hipStream_t st, int* rc) 
 }
 // Which matrix-core form runs against packed weights.  Waves that split K (wk_gemm.h) from a few tokens to about the batch whose
 // large tiles fill the chip (93 x 2560 x 9728: 38 -> 11 us, 300 x 2560 x 9728: 41 -> 20, 32 x 4096 x 4096: 13.5 -> 7.6), then the
-// weights-from-global tiles.  The costs are fitted to 170 shapes within 6 to 11 % (rms); the choice by cost is within 1 % of
-// the best form on average, 17 % at worst.
-static int launch_w8a8_packed_auto(const W8A8Args& a, hipStream_t st) {
-  static const FormCost cost[] = {
-      {32, 32, 0.50f, 2.89f, 0.79f, 0.1048f},   // 8 waves, two workgroups per CU
-      {32, 64, 1.00f, 1.94f, 2.55f, 0.1276f},   // 8 waves
-      {64, 64, 1.00f, 0.89f, 4.64f, 0.1776f},   // 8 waves
-      {64, 128, 0.00f, 3.34f, 0.00f, 0.4102f},  // weights-from-global tiles
-      {128, 128, 0.50f, 2.82f, 1.34f, 0.5597f},
-      {128, 256, 0.75f, 0.00f, 6.71f, 0.6615f},
-      {64, 384, 0.75f, 0.00f, 5.22f, 0.5796f},
-      {128, 384, 1.00f, 0.00f, 9.57f, 0.8600f}};
+// weights-from-global tiles.  Over 1850 random shapes (5 to 6000 rows, 64 to 22 000 channels, K 64 to 10 000) the choice takes 1.008 times the
+// best form's time on average (40 % more at worst, 814 x 1200 x 3200; more than 10 % in 43) and is more than 5 % slower than the tiles by
+// rows and columns alone that ran before in 17 (2806 x 208 x 3968: 14.7, 11.5 at most).  More than 32 rows: fitted to 1300 of them within 5 to
+// 8 % (rms, where a form is near the best); a table fitted to 170 shapes of 93 rows and more, without the prices of M K and M N, made the
+// choice 1.021, 169 and 97 (1811 x 264 x 1280 7.6 us, 6.4 now), but is as good up to 32 rows (1.009 of the best) and stays there.
+static int w8a8_packed_form(int64_t M, int64_t N, int64_t K) {
   constexpr int forms = 8;
-  if (g_w8a8_ntile || !g_w8a8_decode) return launch_w8a8_nsplit_auto<true>(a, st);
+  static const FormCost many[forms] = {
+      {32, 32, 1, 1.0f, 0.75f, 3.143f, 0.5845f, 0.08189f, 0.0852f, 0.8638f},  // 8 waves, two workgroups per CU
+      {32, 64, 1, 1.0f, 1.00f, 2.442f, 1.744f, 0.1177f, 0.08201f, 1.227f},    // 8 waves
+      {64, 64, 1, 1.0f, 1.00f, 2.549f, 2.125f, 0.1942f, 0.1198f, 1.73f},      // 8 waves
+      {64, 128, 1, 1.0f, 0.75f, 3.462f, 0.3554f, 0.2758f, 0.05724f, 0.4347f},  // weights-from-global tiles
+      {128, 128, 1, 1.0f, 0.50f, 4.155f, 0.355f, 0.501f, 0.2004f, 0.3674f},
+      {128, 256, 1, 1.0f, 1.00f, 5.54f, 0.f, 0.7006f, 0.1384f, 0.3784f},
+      {64, 384, 1, 1.0f, 1.00f, 4.842f, 0.03656f, 0.5477f, 0.07742f, 0.48f},
+      {128, 384, 1, 1.0f, 1.00f, 3.357f, 4.175f, 0.9135f, 0.3508f, 0.3465f}};
+  static const FormCost few[forms] = {{32, 32, 1, 1.f, 0.50f, 2.89f, 0.79f, 0.1048f, 0.f, 0.f},   {32, 64, 1, 1.f, 1.00f, 1.94f, 2.55f, 0.1276f, 0.f, 0.f},
+                                      {64, 64, 1, 1.f, 1.00f, 0.89f, 4.64f, 0.1776f, 0.f, 0.f},   {64, 128, 1, 1.f, 0.00f, 3.34f, 0.f, 0.4102f, 0.f, 0.f},
+                                      {128, 128, 1, 1.f, 0.50f, 2.82f, 1.34f, 0.5597f, 0.f, 0.f}, {128, 256, 1, 1.f, 0.75f, 0.f, 6.71f, 0.6615f, 0.f, 0.f},
+                                      {64, 384, 1, 1.f, 0.75f, 0.f, 5.22f, 0.5796f, 0.f, 0.f},    {128, 384, 1, 1.f, 1.00f, 0.f, 9.57f, 0.86f, 0.f, 0.f}};
+  const FormCost* cost = M <= 32 ? few : many;
   int form = 0;
   float best = 0.f;
   for (int f = 0; f < forms; f++) {
-    const float c = form_cost(cost[f], a.M, a.N, (a.K + 127) / 128);
+    const float c = form_cost(cost[f], M, N, K, (K + 127) / 128);
     if (f == 0 || c < best) {
       best = c;
       form = f;
     }
   }
-  switch (form) {
+  return form;
+}
+static int launch_w8a8_packed_auto(const W8A8Args& a, hipStream_t st) {
+  if (g_w8a8_ntile || !g_w8a8_decode) return launch_w8a8_nsplit_auto<true>(a, st);
+  switch (w8a8_packed_form(a.M, a.N, a.K)) {
     case 0: return wk_gemm_launch<W8A8Waves, 1, 1, 8, 2>(a, st);
     case 1: return wk_gemm_launch<W8A8Waves, 1, 2, 8, 1>(a, st);
     case 2: return wk_gemm_launch<W8A8Waves, 2, 2, 8, 1>(a, st);
@@ -748,6 +759,10 @@ static int launch_w8a8_packed_auto(const W8A8Args& a, hipStream_t st) {
     case 6: return launch_w8a8_nsplit<2, 3, true, 2>(a, st);
     default: return launch_w8a8_nsplit<4, 3, true, 1>(a, st);
   }
+}
+MLLM_API int mllm_hip_w8a8_packed_form(int64_t M, int64_t N, int64_t K) {
+  if (M < 1 || N < 1 || K < 1) return 0;
+  return M < 5 ? 9 : 1 + w8a8_packed_form(M, N, K);
 }
 MLLM_API int mllm_hip_w8a8_set_decode(int gemv) {
   if (gemv != 0 && gemv != 1) return MLLM_HIP_E_BADARG;

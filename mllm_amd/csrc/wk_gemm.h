@@ -167,17 +167,21 @@ int wk_gemm_launch(const typename T::Args& a, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-// What a form of a GEMM is expected to take, in us: fixed + rounds * (round + block * K blocks), where a round is one tile per CU
-// and a partly filled last round counts `whole` of a whole one.  The callers' constants are fitted to measured times over
-// matrices of 1 to 25 M weights and 8 to 2048 rows (each says how well); the form with the least cost is launched.
+// What a form of a GEMM is expected to take, in us: fixed + rounds * (round + block * K blocks) + mk * M K + mn * M N (in millions).  A round
+// is one tile per CU; up to `cap` tiles share a CU, each further one at `share` of the first, and a partly filled last round counts `whole` of a
+// whole one.  The callers' constants are fitted to measured times (each says how well); the form with the least cost is launched.
+// Up to 32 rows the choice looks at the tiles alone: a row's bits do not depend on how many rows come with it.
 struct FormCost {
-  int bm, bn;                         // tile: rows x channels
-  float whole, fixed, round, block;
+  int bm, bn, cap;                    // tile: rows x channels
+  float share, whole, fixed, round, block, mk, mn;
 };
-inline float form_cost(const FormCost& f, int64_t M, int64_t N, int64_t blocks) {
-  const int64_t tiles = ((M + f.bm - 1) / f.bm) * ((N + f.bn - 1) / f.bn);
-  const float full = (float)((tiles + 255) / 256), part = (float)tiles / 256.f;
-  return f.fixed + (f.whole * full + (1.f - f.whole) * (part > 1.f ? part : 1.f)) * (f.round + f.block * (float)blocks);
+inline float form_cost(const FormCost& f, int64_t M, int64_t N, int64_t K, int64_t blocks) {
+  const int64_t tiles = ((M + f.bm - 1) / f.bm) * ((N + f.bn - 1) / f.bn), chip = 256 * (int64_t)f.cap;
+  const float part = (float)tiles / 256.f, m = 1e-6f * (float)(M > 32 ? M : 32);
+  float rounds;
+  if (tiles <= chip) rounds = 1.f + f.share * (f.whole * (float)((tiles + 255) / 256) + (1.f - f.whole) * (part > 1.f ? part : 1.f) - 1.f);
+  else rounds = (1.f + f.share * (float)(f.cap - 1)) * (f.whole * (float)((tiles + chip - 1) / chip) + (1.f - f.whole) * part / (float)f.cap);
+  return f.fixed + rounds * (f.round + f.block * (float)blocks) + m * (f.mk * (float)K + f.mn * (float)N);
 }
 
 }  // namespace mllmhip

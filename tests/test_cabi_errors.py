@@ -92,6 +92,8 @@ def _cases():
         "mllm_hip_w4a16_set_decode": ([1], [(0, 2, BADARG), (0, -1, BADARG)]),
         "mllm_hip_w4a16_set_decode_mfma_from": ([2], [(0, 0, BADARG), (0, 34, BADARG)]),
         "mllm_hip_q_gemm_set_form": ([0], [(0, 13, BADARG), (0, -1, BADARG)]),
+        "mllm_hip_w8a8_packed_form": ([64, 64, 64], [(0, 0, 0), (1, -1, 0), (2, 0, 0)]),
+        "mllm_hip_w4a16_packed_form": ([64, 64, 64], [(0, 0, 0), (1, -1, 0), (2, 0, 0)]),
         "mllm_hip_q_gemm_form": ([Q4_0, 64, 64, 256, 1], [(0, 5, 0), (1, 0, 0), (2, 0, 0), (3, -1, 0)]),
         "mllm_hip_moe_gate_set_form": ([1], [(0, 2, BADARG), (0, -1, BADARG)]),
         "mllm_hip_kq_gemm_prepack": ([Q4_K, P, 0, P, 8, 256, None], [(0, Q8_0, BADARG), (1, None, BADARG), (5, 96, SHAPE)]),
@@ -174,6 +176,25 @@ def test_softmax_is_cut_into_pieces_only_where_that_is_not_slower():
     for rows, ln, pieces in ((1, 40960, 0), (1, 40961, 11), (192, 40968, 11), (193, 46120, 0), (256, 50000, 0), (256, 50001, 13), (257, 40968, 11),
                              (512, 40968, 11), (513, 151936, 0)):
         assert room(rows, ln) == rows * pieces * 8, (rows, ln)
+
+
+@pytest.mark.parametrize("M,N,K,form", [(1811, 264, 1280, 4), (381, 1480, 1664, 4), (3409, 1176, 704, 7), (1117, 872, 1344, 4), (169, 4592, 1216, 4),
+                                        (2048, 6144, 2048, 8), (93, 2560, 9728, 1), (20, 1968, 192, 1)])
+def test_w8a8_takes_a_form_that_measures_fast(M, N, K, form):
+    """shapes at which a choice by tiles and K steps alone took 13 to 26 % longer than this form (the first five), and where it took it"""
+    L = _lib.lib()
+    assert L.mllm_hip_w8a8_packed_form(M, N, K) == form
+    assert [L.mllm_hip_w8a8_packed_form(t, N, K) for t in (1, 4)] == [9, 9] and len({L.mllm_hip_w8a8_packed_form(t, N, K) for t in (5, 17, 32)}) == 1
+
+
+@pytest.mark.parametrize("M,N,K,form", [(3500, 456, 1280, 8), (4580, 576, 512, 8), (5226, 376, 2688, 8), (738, 2720, 384, 8), (2048, 9728, 2560, 6), (93, 2048, 6144, 2),
+                                        (64, 9728, 128, 10), (1, 1440, 512, 10), (65, 9728, 128, 8), (64, 9728, 576, 4)])
+def test_w4a16_takes_a_form_that_measures_fast(M, N, K, form):
+    """shapes at which a choice without tiles of 64 rows took 23 to 33 % longer (the first four), few K blocks, and a long prompt; the tokens of
+    a decode step take one form however many there are"""
+    L = _lib.lib()
+    assert L.mllm_hip_w4a16_packed_form(M, N, K) == form
+    assert len({L.mllm_hip_w4a16_packed_form(t, N, K) for t in (1, 5, 9, 32)}) == 1
 
 
 def test_topk_is_cut_into_pieces_only_where_that_is_faster():

@@ -236,10 +236,10 @@ def test_waves_that_split_k(M):
 
 
 def test_waves_that_split_k_of_larger_tiles():
-    """tiles of 32x64 (70 x 4100 x 784, 33 x 6002 x 1104, 300 x 1030 x 2560, 31 x 9001 x 2560 by the cost of each form) and of 64x64 (97 x
-    4101 x 2560, 65 x 6002 x 2560, 33 x 9001 x 2560, 300 x 3002 x 2576): ragged ends, N % 4 != 0, K blocks that do not divide"""
-    _waves_cases(((70, 4100, 784), (33, 6002, 1104), (300, 1030, 2560), (31, 9001, 2560), (97, 4101, 2560), (65, 6002, 2560), (33, 9001, 2560),
-                  (300, 3002, 2576)))
+    """tiles of 32x64 and of 64x64: ragged ends, N % 4 != 0, K blocks that do not divide"""
+    small, large = ((70, 4100, 784), (33, 6002, 1104), (300, 1030, 2560), (31, 9001, 2560)), ((97, 4101, 2560), (65, 6002, 2560), (33, 9001, 2560), (120, 4101, 2576))
+    assert [_lib.lib().mllm_hip_w8a8_packed_form(*s) for s in small + large] == [2] * 4 + [3] * 4
+    _waves_cases(small + large)
 
 
 def _waves_cases(shapes):
