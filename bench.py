@@ -597,8 +597,8 @@ def main():
             _, ev = timed(graphed(lambda: [ql.linear_kq(w, x1, out=y1) for w in ws]), 3, 2)
             res["%s_gate_proj_us" % kname] = ev / (3 * N_LAYERS) * 1e6
             del ws
-            # the four launches of a layer (q+k+v | o | gate+up | down) at eight rows over 12 layers' weights, with workspaces
-            # that have room for the partial sums of K slices
+            # the four launches of a layer (q+k+v | o | gate+up | down) at eight rows over 12 layers' weights, with workspaces for
+            # the quantized image of the rows
             kpool = [{name: ql.PackedKWeight.synthetic(kt, n, k, gen) for name, (n, k) in shapes.items()} for _ in range(12)]
             xs8 = {k: torch.randn((8, k), device="cuda", generator=gen).to(torch.bfloat16) for k in (2560, 4096, 9728)}
             ys8 = {name: torch.empty((8, n), dtype=torch.float32, device="cuda") for name, (n, _) in shapes.items()}
@@ -667,7 +667,7 @@ def main():
             kpool = [{name: ql.PackedKWeight.synthetic(kt, n, k, gen) for name, (n, k) in shapes.items()} for _ in range(N_LAYERS)]
             for M in (1, 8):
                 xs, ys = make_io(M)
-                kws = {k: ql.kq_workspace(M, k, 2 * 9728) for k in (2560, 4096, 9728)}  # (with room for partial sums of K slices)
+                kws = {k: ql.kq_workspace(M, k, 2 * 9728) for k in (2560, 4096, 9728)}  # (room for the quantized image)
 
                 def kstep():  # sibling projections share a launch: qkv | o | gate+up | down
                     for l in kpool:
