@@ -246,9 +246,20 @@ def test_awq_checkpoint_unpack_bit_exact_and_gemm(N, K, group):
 
 @pytest.mark.parametrize("M", [2, 31, 33, 64, 97, 300])
 def test_waves_that_split_k(M):
-    """the forms whose waves share a tile and split K: row tiles of 32 and 64 with ragged ends, fewer K blocks than waves, K blocks that
-    do not divide among the waves, N not a multiple of 4 (element stores) and of 64, a group per K block and fewer"""
-    for N, K, group in ((40, 64, 64), (193, 1088, 64), (1030, 2560, 128), (4100, 768, 256), (256, 6208, 64)):
+    """the forms whose waves share a tile and split K: ragged ends, fewer K blocks than waves, K blocks that do not divide among the waves,
+    N not a multiple of 4 (element stores) and of 64, a group per K block and fewer"""
+    _waves_cases((M, *s) for s in ((40, 64, 64), (193, 1088, 64), (1030, 2560, 128), (4100, 768, 256), (256, 6208, 64)))
+
+
+def test_waves_that_split_k_of_larger_tiles():
+    """tiles of 32x64, of 64x64 and of 64x128 (whole K): ragged rows and channels, N % 4 != 0, K blocks that do not divide"""
+    shapes = ((65, 3002, 576, 64), (45, 4101, 704, 64), (131, 4101, 576, 64), (97, 6002, 640, 128), (193, 6002, 576, 64), (300, 4101, 704, 64))
+    assert [_lib.lib().mllm_hip_w4a16_packed_form(*s[:3]) for s in shapes] == [3, 3, 4, 4, 8, 8]
+    _waves_cases(shapes)
+
+
+def _waves_cases(shapes):
+    for M, N, K, group in shapes:
         rng = synth.rng_for(2, 1300 + 3 * M + N + K + group)
         qw, s, zp, _, _ = synth.make_w4a16(rng, N, K, group)
         a_bits, _ = synth.make_x_bf16(rng, M, K)

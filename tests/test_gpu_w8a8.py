@@ -229,8 +229,8 @@ def test_argument_errors():
 
 @pytest.mark.parametrize("M", [5, 31, 33, 64, 97, 300])
 def test_waves_that_split_k(M):
-    """the forms whose waves share a tile and split K (32x32 at most of these shapes, 64x128 tiles at K of one block): ragged ends, fewer K
-    blocks than waves, K blocks that do not divide among the waves, N not a multiple of 4 (element stores) and of 64; same bits as the
+    """tiles of 32x32 whose waves split K (at most of these shapes; else 32x64, or 64x128 and whole K): ragged ends, fewer K blocks than waves,
+    K blocks that do not divide among the waves, N not a multiple of 4 (element stores) and of 64; same bits as the
     oracle"""
     _waves_cases(((M, N, K) for N, K in ((40, 64), (40, 144), (193, 1104), (1030, 2560), (4100, 784), (256, 6160))))
 
