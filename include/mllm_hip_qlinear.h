@@ -570,8 +570,8 @@ int mllm_hip_moe_gate_set_form(int two_launches);
  * Activation x activation MatMul on the matrix cores (the backend's kMatMul slot; not a quantized path)
  * replaces: CPUMatMulOp::forward  mllm/backends/cpu/ops/MatMulOp.cpp:19-90 (shapes :30-44, default kernel choice :47-61)
  * C[b][M][N] = op(A[b]) * op(B[b]), op(X) = X or X^T; A[b] is [M][K] ([K][M] when transposed), B[b] is [K][N] ([N][K]
- * when transposed).  dtype MLLM_HIP_F32, MLLM_HIP_BF16 or MLLM_HIP_F16 for all three tensors; products are exact and
- * summed in fp32, 16-bit results are rounded once to nearest even.  Batch entry b starts stride_x * b elements after
+ * when transposed).  dtype MLLM_HIP_F32, MLLM_HIP_BF16 or MLLM_HIP_F16 for all three tensors; products are exact (larger fp32
+ * calls: to within 2^-26 of a product) and summed in fp32, 16-bit results are rounded once to nearest even.  Batch entry b starts stride_x * b elements after
  * entry 0 (stride_b = 0 multiplies every A[b] by the same B); the whole batch is one launch.
  * ------------------------------------------------------------------------------------------------------- */
 int mllm_hip_matmul_batched(const void* A, const void* B, void* C, int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
@@ -583,6 +583,10 @@ int mllm_hip_matmul_f32(const float* A, const float* B, float* C, int64_t M, int
 /* Comparison runs and tests: products on tiles of 64 x 64 or 128 x 128 whatever the size (up to four rows stay with the kernels for few
  * rows); 0: by size.  No counterpart in the reference. */
 int mllm_hip_matmul_set_tile(int side);
+/* The same for fp32 products from bf16 parts: -1 never, 64 or 128 on that tile (K >= 16; up to four rows as above), 0 by size (and never while
+ * mllm_hip_matmul_set_tile is not 0).  mllm_hip_matmul_split_side: the tile that a call's tiles would run on, 0: fp32 instructions. */
+int mllm_hip_matmul_set_split(int side);
+int mllm_hip_matmul_split_side(int64_t batch, int64_t M, int64_t N, int64_t K, int transpose_a, int transpose_b);
 
 #ifdef __cplusplus
 }

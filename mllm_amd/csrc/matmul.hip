@@ -1,7 +1,8 @@
 // Activation x activation MatMul on the matrix cores (the kMatMul factory slot of the backend: attention scores, attention
 // x values and the MoE gate logits of the reference run through it, mllm/backends/cpu/ops/MatMulOp.cpp:27-61 with the batch
 // loop of mllm/backends/cpu/kernels/common/ggml/matmul.cpp / mllm_blas).  Not a quantized path.
-//   fp32 operands   v_mfma_f32_32x32x2f32: exact fp32 products, fp32 accumulation (the CPU's arithmetic in another order)
+//   fp32 operands   v_mfma_f32_32x32x2f32: exact fp32 products, fp32 accumulation (the CPU's arithmetic in another order); larger products from
+//                   three bf16 parts per operand, to within 2^-26 of a product (matmul_split_kernel)
 //   bf16 / fp16     v_mfma_f32_32x32x16_{bf16,f16}: exact products, fp32 accumulation, one rounding of the result
 // One launch covers the whole batch (a stride of 0 broadcasts an operand).
 //
@@ -64,7 +65,7 @@ struct MMElem<MLLM_HIP_F32> {
 // by element and nothing else: 0.3 to 0.5 us of a launch are waits for code (8 x 69 x 7 x 18 bf16 4.84 us with the general form's, 4.4).
 // MM_NARROW: rows past the end are not requested again but stay zero (mm_narrow below).
 enum { MM_ANY, MM_VECTORS, MM_STEP, MM_NARROW };
-template <typename E, int ROWS, bool CONTIG_K, int FORM>
+template <typename E, int ROWS, bool CONTIG_K, int FORM, int NT = 256>
 struct MMTile {
   static constexpr bool VECTORS = FORM == MM_VECTORS;
   static constexpr int VE = 16 / (int)sizeof(E);
@@ -73,8 +74,8 @@ struct MMTile {
   static constexpr int RV = CONTIG_K ? 1 : 4;                  // rows of a vector
   static constexpr int LD = KROWS ? ROWS + VE : 32 + VE;
   static constexpr int SIZE = KROWS ? 32 * LD : ROWS * LD;     // elements in LDS
-  static constexpr int NV = ROWS * 32 / VE / 256;              // 16-byte vectors per thread
-  static_assert(ROWS * 32 / VE % 256 == 0, "tile must split evenly over 256 threads");
+  static constexpr int NV = ROWS * 32 / VE / NT;               // 16-byte vectors per thread
+  static_assert(ROWS * 32 / VE % NT == 0, "tile must split evenly over the threads");
   u32x4 v[NV];
   const E* p[NV];
   bool whole, inside[FORM == MM_NARROW ? NV : 1];
@@ -91,7 +92,7 @@ struct MMTile {
     else return (E)d;
   }
   static __device__ __forceinline__ void place(int c, int& r, int& k) {  // first element of vector c of this thread inside the tile
-    const int idx = c * 256 + (int)threadIdx.x;
+    const int idx = c * NT + (int)threadIdx.x;
     if (CONTIG_K) r = idx / (32 / VE), k = (idx % (32 / VE)) * VE;
     else if (PAIRS) k = idx / (ROWS / 4) * 2, r = (idx % (ROWS / 4)) * 4;
     else k = idx / (ROWS / VE), r = (idx % (ROWS / VE)) * VE;
@@ -184,7 +185,47 @@ struct MMTile {
   }
 };
 
-// Bound by the matrix pipe in fp32 (157 TFLOP/s nominal), by LDS reads and the output in 16 bits.  The next K step is loaded into
+// one K step of fp32 instructions from the two tiles in LDS
+template <typename TileA, typename TileB, int TM, int TN>
+__device__ __forceinline__ void mm_f32_step(const float* sA, const float* sB, int wm, int wn, int r, int h, mm_f32x16 (&acc)[TM][TN]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {  // four k of this lane's sixteen at a time
+    f32x4 fa[TM], fb[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) fa[i] = TileA::four(sA, wm * 32 * TM + i * 32 + r, h, q);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) fb[j] = TileB::four(sB, wn * 32 * TN + j * 32 + r, h, q);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][s], fb[j][s], acc[i][j], 0, 0, 0);
+  }
+}
+template <int DT, int TM, int TN, int BM, int BN>
+__device__ __forceinline__ void mm_store(const MMArgs& a, typename MMElem<DT>::type* C, int m0, int n0, int wm, int wn, int r, int h, const mm_f32x16 (&acc)[TM][TN]) {
+  // 32x32 accumulator layout: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32
+  auto put = [&](int m, int n, float f) {
+    if constexpr (DT == MLLM_HIP_F32) C[(int64_t)m * a.N + n] = f;
+    else if constexpr (DT == MLLM_HIP_BF16) C[(int64_t)m * a.N + n] = f32_to_bf16(f);
+    else C[(int64_t)m * a.N + n] = f32_to_f16bits(f);
+  };
+  const bool full = m0 + BM <= a.M && n0 + BN <= a.N;
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = n0 + wn * 32 * TN + j * 32 + r;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int m = m0 + wm * 32 * TM + i * 32 + 8 * (v / 4) + 4 * h + (v % 4);
+        if (full || (n < a.N && m < a.M)) put(m, n, acc[i][j][v]);
+      }
+  }
+}
+
+// Bound by the matrix pipe in fp32 (157 TFLOP/s nominal; larger fp32 products run in matmul_split_kernel), by LDS reads and the output in 16 bits.  The next K step is loaded into
 // registers during this one's matrix instructions.  One LDS stage: a second one halves the workgroups of a CU, which hide
 // the barriers better (fp32 8 x 3108 x 777 x 128: 59 us, 62 with two stages).  The tiles of one batch entry are
 // neighbours on one XCD, whose L2 then holds that entry's operands.  16 bits, large tile: 128 registers, four waves per SIMD instead of
@@ -236,20 +277,7 @@ __global__ __launch_bounds__(256, (TM * TN == 4 && DT != MLLM_HIP_F32) ? 4 : 1) 
       tb.load(B, n0, (kt + 1) * 32, a.N, a.K);
     }
     if constexpr (DT == MLLM_HIP_F32) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {  // four k of this lane's sixteen at a time
-        f32x4 fa[TM], fb[TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) fa[i] = TileA::four(sA, wm * 32 * TM + i * 32 + r, h, q);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) fb[j] = TileB::four(sB, wn * 32 * TN + j * 32 + r, h, q);
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-          for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i][s], fb[j][s], acc[i][j], 0, 0, 0);
-      }
+      mm_f32_step<TileA, TileB, TM, TN>(sA, sB, wm, wn, r, h, acc);
     } else {
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
@@ -273,23 +301,233 @@ __global__ __launch_bounds__(256, (TM * TN == 4 && DT != MLLM_HIP_F32) ? 4 : 1) 
     }
   }
 
-  // 32x32 accumulator layout: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32
-  auto put = [&](int m, int n, float f) {
-    if constexpr (DT == MLLM_HIP_F32) C[(int64_t)m * a.N + n] = f;
-    else if constexpr (DT == MLLM_HIP_BF16) C[(int64_t)m * a.N + n] = f32_to_bf16(f);
-    else C[(int64_t)m * a.N + n] = f32_to_f16bits(f);
-  };
-  const bool full = m0 + BM <= a.M && n0 + BN <= a.N;
+  mm_store<DT, TM, TN, BM, BN>(a, C, m0, n0, wm, wn, r, h, acc);
+}
+
+// fp32 operands on the bf16 matrix instructions, which do sixteen times the products per clock.  A float is the sum of three bf16 numbers,
+// exactly: x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1.  Six of the nine products are multiplied, the smallest first; the three left out
+// are below 2^-26 of a product.  An instruction adds sixteen of them before it rounds, so the result is nearer to 64 bits than that of the fp32
+// instructions, which add two (8 x 3108 x 777 x 128: 1.63e-7 of the norm against 2.03e-7, x 128 x 777: 4.3e-7 against 5.0e-7).
+// Bound by the matrix pipe at the clock it holds under this load, by LDS reads (nine 16-byte reads per twelve instructions; a wave tile of 32 x
+// 64) and by the splitting (six vector instructions per element), which share the issue slots: about 27 us per 128 k of 8 x 3072 x 768, where the
+// matrix instructions alone take 17 and the fp32 ones 45.  K steps of sixteen in two LDS buffers, one barrier each; two (large tile) to five
+// workgroups per CU.  One LDS buffer with steps of 32, operands read a step ahead, and tiles of 64 x 128 with four waves were no faster.
+//   8 x 3108 x 777 x 128 (scores): 65 -> 46 us, x 128 x 777 (values): 66 -> 43; 8 x 4096 x 1024 x 128: 93 -> 62
+struct MMParts {
+  uint32_t p[3];
+};
+__device__ __forceinline__ MMParts mm_split(float a, float b) {  // two neighbouring k of a row
+  MMParts s;
+  s.p[0] = pack_bf16(a, b);
+  a -= __uint_as_float(s.p[0] << 16), b -= __uint_as_float(s.p[0] & 0xffff0000u);
+  s.p[1] = pack_bf16(a, b);
+  a -= __uint_as_float(s.p[1] << 16), b -= __uint_as_float(s.p[1] & 0xffff0000u);
+  s.p[2] = pack_bf16(a, b);
+  return s;
+}
+// An operand tile of ROWS x 16 elements (K >= 16): in LDS [row][part][k], 16 bytes of padding per row (16-byte reads of neighbouring rows
+// meet different banks).  A last K step that ends behind K is moved back to end at K, and what the step before it has multiplied is zero
+// in it: every load is whole, without a branch.  Rows past the end repeat the last one.
+template <int ROWS, bool CONTIG_K, int NT>
+struct MMSplitTile {
+  static constexpr int LD = 3 * 32 + 16, SIZE = ROWS * LD;  // bytes
+  static constexpr int NV = ROWS * 4 / NT;                  // vectors of four k per thread: of as many rows, or [K][rows] of one row
+  static_assert(ROWS * 4 % NT == 0 && NT % ROWS == 0, "tile must split evenly over the threads");
+  __amdgpu_buffer_rsrc_t rsrc;
+  uint32_t off[CONTIG_K ? NV : 1], ld;
+  u32x4 v[2][NV];  // two K steps in flight
+  static __device__ __forceinline__ int row(int c) { return CONTIG_K ? (int)threadIdx.x / 4 + c * (NT / 4) : (int)threadIdx.x % ROWS; }
+  static __device__ __forceinline__ int kfirst(int c) {  // of the step's 16
+    return CONTIG_K ? (int)threadIdx.x % 4 * 4 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / ROWS) * 4 * NV + 4 * c;  // (the same in a wave: ROWS >= 64)
+  }
+  __device__ __forceinline__ void start(const float* X, int row0, int rows, int K) {
+    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(X), 0, (uint32_t)rows * (uint32_t)K * 4u, 0x00020000);
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int n = n0 + wn * 32 * TN + j * 32 + r;
+    for (int c = 0; c < (CONTIG_K ? NV : 1); c++) {
+      const uint32_t r = (uint32_t)min(row0 + row(c), rows - 1);
+      off[c] = CONTIG_K ? (r * (uint32_t)K + kfirst(c)) * 4u : r * 4u;
+    }
+    ld = (uint32_t)rows * 4u;
+  }
+  __device__ __forceinline__ void load(int d, int k) {  // k: the first of the step's 16
+#pragma unroll
+    for (int c = 0; c < NV; c++) {
+      if constexpr (CONTIG_K) {
+        v[d][c] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[c], k * 4, 0);
+      } else {
+        const uint32_t at = (uint32_t)(k + kfirst(c)) * ld;
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[d][c][e] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, off[0], at + e * ld, 0);
+      }
+    }
+  }
+  // skip: how many k of the step are not its own
+  __device__ __forceinline__ void store(unsigned char* s, int d, int skip, float& most) {
+    if (__builtin_expect(skip != 0, 0)) {
+      asm volatile("");  // (a branch: selects in every step cost more)
+#pragma unroll
+      for (int c = 0; c < NV; c++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (kfirst(c) + e < skip) v[d][c][e] = 0u;
+    }
+    MMParts a[2 * NV];
+#pragma unroll
+    for (int c = 0; c < NV; c++) {
+      const f32x4 x = __builtin_bit_cast(f32x4, v[d][c]);
+      most = fmaxf(fmaxf(most, fabsf(x[0])), fabsf(x[1]));
+      most = fmaxf(fmaxf(most, fabsf(x[2])), fabsf(x[3]));
+      a[2 * c] = mm_split(x[0], x[1]), a[2 * c + 1] = mm_split(x[2], x[3]);
+    }
+    if constexpr (!CONTIG_K && NV == 2) {
+      unsigned char* at = s + row(0) * LD + kfirst(0) * 2;
+#pragma unroll
+      for (int i = 0; i < 3; i++) *reinterpret_cast<u32x4*>(at + 32 * i) = u32x4{a[0].p[i], a[1].p[i], a[2].p[i], a[3].p[i]};
+    } else {
+#pragma unroll
+      for (int c = 0; c < NV; c++) {
+        unsigned char* at = s + row(c) * LD + kfirst(c) * 2;
+#pragma unroll
+        for (int i = 0; i < 3; i++) *reinterpret_cast<u32x2*>(at + 32 * i) = u32x2{a[2 * c].p[i], a[2 * c + 1].p[i]};
+      }
+    }
+  }
+};
+
+template <bool TA, bool TB, int WM, int WN, int TM, int TN>
+__global__ __launch_bounds__(WM * WN * 64, 4) void matmul_split_kernel(MMArgs a, int tiles, int tilesM, uint32_t inv_tiles, uint32_t inv_tilesM) {
+  constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, NT = WM * WN * 64;
+  typedef MMSplitTile<BM, !TA, NT> SplitA;
+  typedef MMSplitTile<BN, TB, NT> SplitB;
+  typedef MMTile<float, BM, !TA, MM_ANY, NT> TileA;
+  typedef MMTile<float, BN, TB, MM_ANY, NT> TileB;
+  constexpr int BUF = SplitA::SIZE + SplitB::SIZE, F32 = (TileA::SIZE + TileB::SIZE) * 4;
+  __shared__ __align__(16) unsigned char smem[2 * BUF > F32 ? 2 * BUF : F32];
+
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = wave / WN, wn = wave % WN, r = lane & 31, h = lane >> 5;
+  const int total = tiles * a.batch, b = mm_block();
+  if (b >= total) return;  // (uniform)
+  const int t = xcd_run(b, total), z = mm_div(t, tiles, inv_tiles), in = t - z * tiles;
+  const int tn = mm_div(in, tilesM, inv_tilesM), n0 = tn * BN, m0 = (in - tn * tilesM) * BM;
+  const float* A = reinterpret_cast<const float*>(a.A) + z * a.sA;
+  const float* B = reinterpret_cast<const float*>(a.B) + z * a.sB;
+  float* C = reinterpret_cast<float*>(a.C) + z * a.sC;
+
+  mm_f32x16 acc[TM][TN];
+  auto clear = [&]() {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  };
+  clear();
+  float most = 0.f;
+  {
+    SplitA ta;
+    SplitB tb;
+    ta.start(A, m0, a.M, a.K);
+    tb.start(B, n0, a.N, a.K);
+    const int steps = (a.K + 15) / 16;
+    auto load = [&](int d, int step) {  // (past the last step: that one again)
+      const int k = min(step * 16, a.K - 16);
+      ta.load(d, k);
+      tb.load(d, k);
+    };
+    auto store = [&](int d, int skip) {  // d = step % 2
+      ta.store(smem + d * BUF, d, skip, most);
+      tb.store(smem + d * BUF + SplitA::SIZE, d, skip, most);
+    };
+    const unsigned char *pa = smem + (wm * 32 * TM + r) * SplitA::LD + 16 * h, *pb = smem + SplitA::SIZE + (wn * 32 * TN + r) * SplitB::LD + 16 * h;
+    auto skip = [&](int step) { return max(step * 16 + 16 - a.K, 0); };
+    load(0, 0);
+    load(1, 1);
+    store(0, 0);
+    load(0, 2);
+    __syncthreads();
+    // step s's tile is in LDS, steps s + 1 and s + 2 are on their way (past the end the last step again, which nothing reads)
+    auto work = [&](int d, int step, int skip) {
+      mm_bf16x8 fa[TM][3], fb[TN][3];
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int u = 0; u < 3; ++u) fa[i][u] = *reinterpret_cast<const mm_bf16x8*>(pa + d * BUF + i * 32 * SplitA::LD + u * 32);
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int u = 0; u < 3; ++u) fb[j][u] = *reinterpret_cast<const mm_bf16x8*>(pb + d * BUF + j * 32 * SplitB::LD + u * 32);
+      __builtin_amdgcn_sched_barrier(0);
+      store(1 - d, skip);
+      load(1 - d, step + 3);
+      __builtin_amdgcn_sched_barrier(0);
+      auto mma = [&](int u, int w) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][u], fb[j][w], acc[i][j], 0, 0, 0);
+      };
+      mma(2, 0), mma(0, 2), mma(1, 1), mma(1, 0), mma(0, 1), mma(0, 0);
+      __syncthreads();
+    };
+    int step = 0;
+    for (; step + 3 < steps; step += 2) work(0, step, 0), work(1, step + 1, 0);
+#pragma unroll 1
+    for (; step < steps; step += 2) {
+      work(0, step, skip(step + 1));
+      if (step + 1 < steps) work(1, step + 1, skip(step + 2));
+    }
+  }
+  // An infinity or a NaN in an operand, and a float that rounds to an infinity in bf16, leave a NaN here.  Parts below 2^-133 vanish: at most
+  // 2^-103 of a product of operands below 2^30.  A tile with a NaN, an infinity, a larger operand or a sum between 0 and 2^-66 is multiplied
+  // again with fp32 instructions.
+  constexpr uint32_t LOW = (127u - 66u) << 24;
+  float check = 0.f;
+  uint32_t low = 0;  // 0 < |sum| < 2^-66: above 0 - LOW, a sum of zero exactly that
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int m = m0 + wm * 32 * TM + i * 32 + 8 * (v / 4) + 4 * h + (v % 4);
-        if (full || (n < a.N && m < a.M)) put(m, n, acc[i][j][v]);
+        check = fmaf(acc[i][j][v], 0.f, check);
+        low = max(low, (__float_as_uint(acc[i][j][v]) << 1) - LOW);
       }
+  if (__syncthreads_or(check != 0.f || most >= 0x1p30f || (low > 0u - LOW))) {
+    float *sA = reinterpret_cast<float*>(smem), *sB = sA + TileA::SIZE;
+    TileA ta;
+    TileB tb;
+    clear();
+    ta.start(A, m0, a.M, a.K);
+    tb.start(B, n0, a.N, a.K);
+#pragma unroll 1
+    for (int k = 0; k < a.K; k += 32) {
+      ta.load(A, m0, k, a.M, a.K);
+      tb.load(B, n0, k, a.N, a.K);
+      __syncthreads();
+      ta.store(sA);
+      tb.store(sB);
+      __syncthreads();
+      mm_f32_step<TileA, TileB, TM, TN>(sA, sB, wm, wn, r, h, acc);
+    }
+    mm_store<MLLM_HIP_F32, TM, TN, BM, BN>(a, C, m0, n0, wm, wn, r, h, acc);
+    return;
+  }
+  // 32x32 accumulator layout as in mm_store; rows past the end lie past the end of the buffer
+  const __amdgpu_buffer_rsrc_t rC = __builtin_amdgcn_make_buffer_rsrc(C, 0, (uint32_t)a.M * (uint32_t)a.N * 4u, 0x00020000);
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = n0 + wn * 32 * TN + j * 32 + r;
+    if (n < a.N) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const uint32_t at = ((uint32_t)(m0 + wm * 32 * TM + i * 32 + 4 * h) * (uint32_t)a.N + n) * 4u;
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][v]), rC, at + (uint32_t)(8 * (v / 4) + v % 4) * (uint32_t)a.N * 4u, 0, 0);
+      }
+    }
   }
 }
 
@@ -496,7 +734,8 @@ static bool launch_matmul_dots(const MMArgs& a, hipStream_t st, int* rc) {
 //     small; 3000 x 3000 x 3000 (2.25 rounds): 604 / 527; K = 64 is mostly epilogue: 4 x 4000 x 1000 x 64: 34 / 31
 //   16 bits (bound by loads and LDS, more workgroups per CU hide them): us of a K of 2048 against tiles per CU, B [N][K]: 4096 x 4096 x 4096
 //     180 large, 298 small, 1000 x 3000 x 700: 24 / 20; where an operand is [K][rows] the large tile gains less (4096^3: 340 / 371)
-static int g_matmul_tile = 0;  // mllm_hip_matmul_set_tile
+static int g_matmul_tile = 0;   // mllm_hip_matmul_set_tile
+static int g_matmul_split = 0;  // mllm_hip_matmul_set_split
 template <int DT, bool TA, bool TB>
 static bool matmul_large_tile(const MMArgs& a) {
   if (g_matmul_tile) return g_matmul_tile == 128;
@@ -527,6 +766,24 @@ static bool mm_narrow(const MMArgs& a) {
   return DT == MLLM_HIP_F32 && !TA && TB && a.M <= 32 && (int64_t)((a.N + 63) / 64) * a.batch >= 800;
 }
 
+// fp32: the side of the tile of matmul_split_kernel, 0 where fp32 instructions are as fast or needed.  Costs in us fitted to 400 random shapes in
+// all orders (1 to 64 x 5 to 4096 x 5 to 4096 x 16 to 2048); of the launches above 12 us the choice takes 0.85 of the fp32 instructions' time on
+// average and at most 1.09 (10 x 3266 x 3871 x 64: 255 / 278).  Up to one small tile per CU a step's latency is the same either way (3 x 80 x
+// 126 x 1670: 44.9 us with fp32 instructions, 39.2 small, 67.1 large; 2 x 168 x 238 x 1975: 45.3, 48.7, 81.9), and the shortest launches are
+// bound by their start.  Few rows x [N][K] over many tiles stay with the form for those.
+static int mm_split_side(const MMArgs& a, bool nt) {
+  constexpr int64_t LIMIT = (int64_t)1 << 32;  // byte offsets in 32 bits
+  if (a.K < 16 || (int64_t)a.M * a.K * 4 >= LIMIT || (int64_t)a.N * a.K * 4 >= LIMIT || ((int64_t)a.M + 128) * a.N * 4 >= LIMIT) return 0;
+  if (g_matmul_split) return g_matmul_split < 0 ? 0 : g_matmul_split;
+  if (g_matmul_tile) return 0;
+  if (nt && mm_narrow<MLLM_HIP_F32, false, true>(a)) return 0;
+  const double K = a.K, t64 = (double)((a.M + 63) / 64) * ((a.N + 63) / 64) * a.batch / 256, t128 = (double)((a.M + 127) / 128) * ((a.N + 127) / 128) * a.batch / 256;
+  if (t64 <= 1. || t64 * K < 150.) return 0;
+  const double us64 = 5.1 + 0.46 * t64 + K * (0.0194 + 0.0144 * (0.2 * std::ceil(t64) + 0.8 * t64 - 1.));
+  const double us128 = 3.0 + 2.6 * std::max(t128, 1.) + 0.037 * K + (0.5 + 0.0435 * K) * (0.85 * std::ceil(t128) + 0.15 * std::max(t128, 1.) - 1.);
+  return us128 < us64 ? 128 : 64;
+}
+
 template <int DT, bool TA, bool TB>
 static int launch_matmul(const MMArgs& a, hipStream_t st) {
   if constexpr (!TA && !TB) {
@@ -537,8 +794,8 @@ static int launch_matmul(const MMArgs& a, hipStream_t st) {
     int rc = 0;
     if (launch_matmul_dots<DT>(a, st, &rc)) return rc;
   }
-  auto go = [&](auto kern, int side) {
-    const int64_t tilesM = (a.M + side - 1) / side, tiles = tilesM * ((a.N + side - 1) / side);
+  auto run = [&](auto kern, int bm, int bn, int threads) {
+    const int64_t tilesM = (a.M + bm - 1) / bm, tiles = tilesM * ((a.N + bn - 1) / bn);
     if (tiles > 0x7fffffff) return MLLM_HIP_E_SHAPE;
     const int most = (int)std::min<int64_t>(a.batch, 0x7fffffff / tiles);  // batch entries per launch
     using E = typename MMElem<DT>::type;
@@ -548,10 +805,17 @@ static int launch_matmul(const MMArgs& a, hipStream_t st) {
       p.B = reinterpret_cast<const E*>(a.B) + z * a.sB;
       p.C = reinterpret_cast<E*>(a.C) + z * a.sC;
       p.batch = std::min(most, a.batch - z);
-      hipLaunchKernelGGL(kern, mm_grid(tiles * p.batch), dim3(256), 0, st, p, (int)tiles, (int)tilesM, mm_inv(tiles, tiles * p.batch), mm_inv(tilesM, tiles));
+      hipLaunchKernelGGL(kern, mm_grid(tiles * p.batch), dim3(threads), 0, st, p, (int)tiles, (int)tilesM, mm_inv(tiles, tiles * p.batch), mm_inv(tilesM, tiles));
     }
     return (int)hipGetLastError();
   };
+  auto go = [&](auto kern, int side) { return run(kern, side, side, 256); };
+  if constexpr (DT == MLLM_HIP_F32) {
+    switch (mm_split_side(a, !TA && TB)) {
+      case 64: return run(matmul_split_kernel<TA, TB, 2, 2, 1, 1>, 64, 64, 256);
+      case 128: return run(matmul_split_kernel<TA, TB, 4, 2, 1, 2>, 128, 128, 512);
+    }
+  }
   if (matmul_large_tile<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 2, 2, MM_ANY>, 128);
   if constexpr (DT == MLLM_HIP_F32 && !TA && TB) {
     if (a.K > 32 && mm_narrow<DT, TA, TB>(a)) return go(matmul_kernel<DT, TA, TB, 1, 1, MM_NARROW>, 64);
@@ -603,6 +867,19 @@ MLLM_API int mllm_hip_matmul_set_tile(int side) {
   if (side != 0 && side != 64 && side != 128) return MLLM_HIP_E_BADARG;
   g_matmul_tile = side;
   return 0;
+}
+
+MLLM_API int mllm_hip_matmul_set_split(int side) {
+  if (side != -1 && side != 0 && side != 64 && side != 128) return MLLM_HIP_E_BADARG;
+  g_matmul_split = side;
+  return 0;
+}
+
+MLLM_API int mllm_hip_matmul_split_side(int64_t batch, int64_t M, int64_t N, int64_t K, int transpose_a, int transpose_b) {
+  if (batch < 1 || M < 1 || N < 1 || K < 1 || batch > INT32_MAX || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return 0;
+  MMArgs a{};
+  a.batch = (int)batch, a.M = (int)M, a.N = (int)N, a.K = (int)K;
+  return mm_split_side(a, !transpose_a && transpose_b);
 }
 
 MLLM_API int mllm_hip_matmul_f32(const float* A, const float* B, float* C, int64_t M, int64_t N, int64_t K, int transpose_a,

@@ -191,6 +191,76 @@ def test_matmul_keeps_infinities_and_nan_in_their_rows(M, N, K, ta, tb, dtype, s
     assert torch.equal(c.isnan(), want.isnan()) and torch.equal(c.nan_to_num(nan=0.), want.nan_to_num(nan=0.))
 
 
+def _split(side, a, b, ta, tb):
+    try:
+        assert _lib.lib().mllm_hip_matmul_set_split(side) == 0
+        return ql.matmul(a.cuda(), b.cuda(), ta, tb).cpu()
+    finally:
+        assert _lib.lib().mllm_hip_matmul_set_split(0) == 0
+
+
+@pytest.mark.parametrize("side", [64, 128])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("batch,M,N,K", [(1, 5, 7, 16), (3, 65, 63, 17), (2, 64, 128, 32), (2, 129, 127, 47), (3, 128, 64, 48), (1, 257, 130, 63), (5, 70, 129, 31),
+                                         (1, 200, 333, 1000)])
+def test_matmul_fp32_from_bf16_parts(batch, M, N, K, ta, tb, side):
+    """one to four K steps (all stages of the loop's start and end), last steps of one to sixteen k, ragged and whole tiles, in every order.  A
+    product of floats has 48 bits and three bf16 parts hold a float exactly: integers below 2^12 by powers of two are exact, a one-hot
+    operand returns the other one bit for bit, and random floats are within the bound of the fp32 instructions"""
+    rng = synth.rng_for(6, 8000 + batch + M + N + K)
+    put = lambda a, b: (torch.from_numpy(np.ascontiguousarray(np.swapaxes(a, 1, 2) if ta else a)), torch.from_numpy(np.ascontiguousarray(b if tb else np.swapaxes(b, 1, 2))))  # noqa: E731
+    announce("matmul from parts %s ta=%d tb=%d side %d" % ((batch, M, N, K), ta, tb, side))
+    a = (rng.integers(-4095, 4096, (batch, M, K)) * 2.0 ** rng.integers(-20, 20, (batch, M, 1))).astype(np.float32)
+    b = rng.integers(-1, 2, (batch, N, K)).astype(np.float32)
+    want = a.astype(np.float64) @ np.swapaxes(b, 1, 2)
+    assert np.array_equal(_split(side, *put(a, b), ta, tb).numpy(), want.astype(np.float32))
+    a = rng.standard_normal((batch, M, K)).astype(np.float32)
+    pick = rng.integers(0, K, (batch, N))
+    b = (np.arange(K) == pick[..., None]).astype(np.float32)
+    assert np.array_equal(_split(side, *put(a, b), ta, tb).numpy(), np.take_along_axis(a, pick[:, None, :].repeat(M, 1), 2))
+    b = rng.standard_normal((batch, N, K)).astype(np.float32)
+    assert rel_l2(_split(side, *put(a, b), ta, tb).numpy(), a.astype(np.float64) @ np.swapaxes(b.astype(np.float64), 1, 2)) <= 2e-6
+
+
+@pytest.mark.parametrize("side", [64, 128])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(70, 130, 37), (129, 66, 64), (5, 133, 100)])
+def test_matmul_from_bf16_parts_outside_their_range(M, N, K, ta, tb, side):
+    """infinities, NaN, floats that round to an infinity in bf16, sums that overflow, elements whose parts are below the smallest bf16 number and
+    operands of any size: the tile takes fp32 instructions, and no other row or column changes"""
+    rng = synth.rng_for(6, 9000 + M + N + K)
+    a = torch.from_numpy(rng.integers(1, 9, (M, K)).astype(np.float32))
+    b = torch.from_numpy(rng.integers(1, 9, (N, K)).astype(np.float32))
+    a[M - 1, K - 1], a[0, 0], b[N - 1, K - 2], b[1, 0] = float("inf"), float("nan"), float("-inf"), float("inf")
+    order = lambda a, b: (a.t().contiguous() if ta else a, b if tb else b.t().contiguous())  # noqa: E731
+    announce("matmul from parts of infinities %s ta=%d tb=%d side %d" % ((M, N, K), ta, tb, side))
+    c, want = _split(side, *order(a, b), ta, tb), torch.matmul(a, b.t().contiguous())
+    assert want.isfinite().sum() == (M - 2) * (N - 2)
+    assert torch.equal(c.isnan(), want.isnan()) and torch.equal(c.nan_to_num(nan=0.), want.nan_to_num(nan=0.))
+    for scale in (2.0 ** -120, 2.0 ** -104, 2.0 ** 60, 2.0 ** 107):  # a row of A; integers times a power of two: exact (sums below 2^12 2 100 2^107 < 2^127)
+        a = torch.from_numpy(rng.integers(1, 1 << 12, (M, K)).astype(np.float32))
+        b = torch.from_numpy(rng.integers(-2, 3, (N, K)).astype(np.float32))
+        a[M // 2] *= scale
+        assert torch.equal(_split(side, *order(a, b), ta, tb), torch.matmul(a.double(), b.double().t().contiguous()).float())
+    a = torch.full((M, K), 3.3961775e38)  # below the largest float, an infinity in bf16
+    b = torch.zeros((N, K))
+    b[:, 0] = 1.
+    assert torch.equal(_split(side, *order(a, b), ta, tb), a[:, :1].expand(M, N))
+
+
+def test_matmul_of_attention_sizes_takes_the_bf16_parts():
+    side = _lib.lib().mllm_hip_matmul_split_side
+    assert side(8, 3108, 777, 128, 0, 1) == 64 and side(8, 3108, 128, 777, 0, 0) == 128 and side(8, 1000, 520, 128, 0, 1) == 64
+    assert side(8, 64, 64, 64, 0, 1) == 0 and side(1, 1 << 15, 1 << 15, 128, 0, 1) == 0 and side(8, 3108, 777, 15, 0, 1) == 0
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a, b = torch.randn((8, 1000, 128), device="cuda", generator=g), torch.randn((8, 520, 128), device="cuda", generator=g)
+    announce("matmul of 8 x 1000 x 520 x 128")
+    c = ql.matmul(a, b, transpose_b=True)
+    want = torch.matmul(a.double(), b.double().transpose(1, 2).contiguous())
+    err = lambda c: float((c.double() - want).norm() / want.norm())  # noqa: E731
+    assert side(8, 1000, 520, 128, 0, 1) and err(c) <= err(_split(-1, a, b, False, True).cuda()) <= 3e-7
+
+
 def test_matmul_batches_beyond_a_grid_dimension():
     """more workgroups than a grid dimension's 32 bits of work-items hold (2^24 of 256 threads, 2^22 of 1024), once per kernel: tiles,
     dot products, values; small integers, exact"""
