@@ -604,25 +604,28 @@ __device__ __forceinline__ f16x2 qg_offset2(const uint32_t (&s)[qg_scale_dwords(
 // the rounding residual of the product (exact: the error of a product of two fp16 numbers is an fp16 number).
 // Q4_K: the sub-block's value is ds * q - dm (q = 0..15): one fused multiply-add, one rounding; Q6_K: codes widened to
 // int8 at load time, ds the scale of the step's 16 elements: the Q8_0 arithmetic.
+// These instructions and the MFMAs take turns (4 clocks each but 2 for a shift, and / or), so: nibbles at bits 4 b + 0..3 go into the mantissa of
+// 1024 (b even) or as they are into that of 64 (b odd), one shift for two of the four pairs instead of three; bytes are put under the mantissa
+// of 1024 by a permutation.  Three shifts and and / or on bytes took 117.2 us at 2048 x 9728 x 2560 Q6_K (113.7 now), 27.8 at 131 x 2560 x 9728 Q6_K (25.4), 26.2 Q4_0 (25.2).
 template <int WT, int PREC>
 __device__ __forceinline__ uint32_t qg_pair(const u32x4 (&rq)[qg_nibbles(WT) ? 1 : 2], int d, int b, f16x2 dd, f16x2 dm, uint32_t& lo) {
   uint32_t t;
-  f16x2 off;
-  if (WT == MLLM_HIP_Q4_K) {
-    static_assert(WT != MLLM_HIP_Q4_K || PREC == 1, "one-term operands only");
-    t = ((rq[0][d] >> (4 * b)) & 0x000f000fu) | 0x64006400u;       // (1024 + q) in both halves
-    const f16x2 c = __builtin_bit_cast(f16x2, t) - f16x2{(_Float16)1024.f, (_Float16)1024.f};  // q, exact
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(c, dd, -dm));                // v_pk_fma_f16
-  }
-  if (WT == MLLM_HIP_Q4_0) {
-    t = ((rq[0][d] >> (4 * b)) & 0x000f000fu) | 0x64006400u;       // (1024 + q) in both halves
-    off = f16x2{(_Float16)1032.f, (_Float16)1032.f};               // ... - 1032 = q - 8, exact
+  float off;
+  if (qg_nibbles(WT)) {
+    const uint32_t w = b < 2 ? rq[0][d] : rq[0][d] >> 8;
+    t = b & 1 ? (w & 0x00f000f0u) | 0x54005400u : (w & 0x000f000fu) | 0x64006400u;  // 64 + q or 1024 + q in both halves
+    off = b & 1 ? 64.f : 1024.f;
+    if (WT == MLLM_HIP_Q4_0) off += 8.f;
   } else {
     const uint32_t w = rq[d >> 1][2 * (d & 1) + (b >> 1)] ^ 0x80808080u;  // codes + 128, bytes e0 e2 e1 e3
-    t = ((w >> (8 * (b & 1))) & 0x00ff00ffu) | 0x64006400u;
-    off = f16x2{(_Float16)1152.f, (_Float16)1152.f};
+    t = __builtin_amdgcn_perm(0x64646464u, w, b & 1 ? 0x04030401u : 0x04020400u);
+    off = 1152.f;
   }
-  const f16x2 c = __builtin_bit_cast(f16x2, t) - off;              // v_pk_add_f16, exact
+  const f16x2 c = __builtin_bit_cast(f16x2, t) - f16x2{(_Float16)off, (_Float16)off};  // v_pk_add_f16: the code, exact
+  if (WT == MLLM_HIP_Q4_K) {
+    static_assert(WT != MLLM_HIP_Q4_K || PREC == 1, "one-term operands only");
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(c, dd, -dm));  // v_pk_fma_f16
+  }
   const f16x2 r = c * dd;                                          // v_pk_mul_f16: one rounding
   if (PREC == 2) lo = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(c, dd, -r));  // v_pk_fma_f16
   return __builtin_bit_cast(uint32_t, r);
