@@ -316,8 +316,8 @@ __global__ __launch_bounds__(SOFTMAX_WG) void softmax_long_rows_kernel(const flo
 // Few long rows spread over the chip (mllm_hip_softmax_ws): a row is cut into pieces of SOFTMAX_PIECE elements with a
 // workgroup each, and the row's maximum and sum meet in the caller's workspace, so the operator is three launches: maxima of
 // the pieces, sums of the pieces (which need the row's maximum: the reference's polynomial is not exp(a) exp(b) = exp(a + b)
-// to fp32), results.  A workgroup per row is bound by what one CU can load and by its vector ALU: eight rows of 151 936 take
-// 49 us there and 11.4 here (one row 47 -> 9.3; a launch costs about 2.5 us whatever it does).  A piece inside the polynomial's
+// to fp32), results -- or two, see STAGE 3 below.  A workgroup per row is bound by what one CU can load and by its vector ALU: eight rows of
+// 151 936 take 49 us there and 9.7 here (one row 47 -> 8.0; a launch costs about 2.5 us whatever it does).  A piece inside the polynomial's
 // range has no branch per element, so that its exponentials overlap (with the branches: 14.8 and 13.5); pieces of 2048 elements
 // are no faster.
 constexpr int SOFTMAX_PIECE = 4096;
@@ -348,10 +348,20 @@ __device__ __forceinline__ float block_sum_256(float v, float* s_red) {
   __syncthreads();
   return v;
 }
-// STAGE 0: pmax[row][piece];  1: psum[row][piece];  2: y.  ws: pmax, then psum, of rows * pieces floats each.
+// STAGE 0: pmax[row][piece], and psum[row][piece] = SOFTMAX_NO_SUM;  1: psum[row][piece];  2: y;  3: both in one launch.  ws: pmax, then psum, of
+// rows * pieces floats each.
+// STAGE 3: a workgroup keeps its exponentials in registers, publishes their sum and reads the other pieces' as they appear (the value is its
+// own flag; stores and loads of device scope, since every XCD has an L2 of its own).  It runs for up to SOFTMAX_WAIT workgroups, a quarter of what
+// the chip holds at once, so they run together.  Where they should not (other work on the chip), a workgroup gives up after `polls` looks
+// and adds up the row by itself: nobody waits for long, the bits are the same.  In a graph, us, stages 1 and 2 / 3 (with more workgroups, or more
+// pieces to look at, the looks cost more than a launch): 1 x 50 000 8.9 / 7.2, 4 x 64 000 9.7 / 7.9, 8 x 151 936 10.6 / 9.7, 16 x 151 936 (608)
+// 12.0 / 12.4, 512 x 151 936 225 / 255, 1 x 1 000 000 (245 pieces) 9.9 / 11.4; a launch less for the host.
+constexpr uint32_t SOFTMAX_NO_SUM = 0xffffffffu;
+constexpr int SOFTMAX_WAIT = 512, SOFTMAX_WAIT_PIECES = 64;
+static int g_softmax_polls = 4096;  // mllm_hip_softmax_set_wait; a look takes about a microsecond
 template <int STAGE>
 __global__ __launch_bounds__(256) void softmax_pieces_kernel(const float* __restrict__ x, float* __restrict__ y, float* __restrict__ ws,
-                                                             int len, int exp_accurate) {
+                                                             int len, int exp_accurate, int polls) {
   __shared__ float s_red[4];
   constexpr int R = SOFTMAX_PIECE / 256;
   const int tid = threadIdx.x, piece = blockIdx.x, pieces = gridDim.x;
@@ -359,16 +369,22 @@ __global__ __launch_bounds__(256) void softmax_pieces_kernel(const float* __rest
   float* pmax = ws + row * pieces;
   float* psum = ws + ((int64_t)gridDim.y + row) * pieces;
   const float* xr = x + row * len;
-  const int i0 = piece * SOFTMAX_PIECE + tid;
   float v[R];
+  auto load = [&](int i0) {
 #pragma unroll
-  for (int j = 0; j < R; j++) v[j] = i0 + 256 * j < len ? xr[i0 + 256 * j] : -3.402823466e+38f;
+    for (int j = 0; j < R; j++) v[j] = i0 + 256 * j < len ? xr[i0 + 256 * j] : -3.402823466e+38f;
+  };
+  const int i0 = piece * SOFTMAX_PIECE + tid;
+  load(i0);
   if (STAGE == 0) {
     float mx = v[0];
 #pragma unroll
     for (int j = 1; j < R; j++) mx = fmaxf(mx, v[j]);
     mx = block_max_256(mx, s_red);
-    if (tid == 0) pmax[piece] = mx;
+    if (tid == 0) {
+      pmax[piece] = mx;
+      psum[piece] = __uint_as_float(SOFTMAX_NO_SUM);
+    }
     return;
   }
   const bool poly = !exp_accurate;
@@ -378,33 +394,55 @@ __global__ __launch_bounds__(256) void softmax_pieces_kernel(const float* __rest
   if (STAGE == 2)
     for (int p = tid; p < pieces; p += 256) total += psum[p];
   mx = block_max_256(mx, s_red);
-  float sum = 0.f;
-  if (poly && (int64_t)(piece + 1) * SOFTMAX_PIECE <= (len & ~7)) {  // (uniform) the whole piece takes the polynomial
+  auto exponentials = [&](int p, int i0) {  // of piece p, in v; returns the thread's sum
+    float sum = 0.f;
+    if (poly && (int64_t)(p + 1) * SOFTMAX_PIECE <= (len & ~7)) {  // (uniform) the whole piece takes the polynomial
 #pragma unroll
-    for (int j = 0; j < R; j++) {
-      v[j] = exp_poly(v[j] - mx);
-      sum += v[j];
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < R; j++) {
-      const int i = i0 + 256 * j;
-      if (i < len) {
-        v[j] = softmax_exp(v[j] - mx, poly && i < (len & ~7));
+      for (int j = 0; j < R; j++) {
+        v[j] = exp_poly(v[j] - mx);
         sum += v[j];
       }
+    } else {
+#pragma unroll
+      for (int j = 0; j < R; j++) {
+        const int i = i0 + 256 * j;
+        if (i < len) {
+          v[j] = softmax_exp(v[j] - mx, poly && i < (len & ~7));
+          sum += v[j];
+        }
+      }
+    }
+    return sum;
+  };
+  float sum = exponentials(piece, i0);
+  if (STAGE == 1 || STAGE == 3) {
+    sum = block_sum_256(sum, s_red);
+    if (tid == 0) {
+      if (STAGE == 1) psum[piece] = sum;
+      else __hip_atomic_store(&psum[piece], sum == sum ? sum : __uint_as_float(0x7fc00000u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (STAGE == 1) return;
+    bool missing = tid < pieces;  // (at most 64 pieces)
+    for (int n = 0; missing && n <= polls; n++) {
+      total = __hip_atomic_load(&psum[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      missing = __float_as_uint(total) == SOFTMAX_NO_SUM;
+    }
+    if (__syncthreads_or(missing)) {
+      total = 0.f;
+      for (int p = 0; p < pieces; p++) {
+        load(p * SOFTMAX_PIECE + tid);
+        const float s = block_sum_256(exponentials(p, p * SOFTMAX_PIECE + tid), s_red);
+        if (tid == p) total += s;
+      }
+      load(i0);
+      exponentials(piece, i0);
     }
   }
-  if (STAGE == 1) {
-    sum = block_sum_256(sum, s_red);
-    if (tid == 0) psum[piece] = sum;
-  } else {
-    const float inv = 1.f / block_sum_256(total, s_red);
-    float* yr = y + row * len;
+  const float inv = 1.f / block_sum_256(total, s_red);
+  float* yr = y + row * len;
 #pragma unroll
-    for (int j = 0; j < R; j++)
-      if (i0 + 256 * j < len) yr[i0 + 256 * j] = v[j] * inv;
-  }
+  for (int j = 0; j < R; j++)
+    if (i0 + 256 * j < len) yr[i0 + 256 * j] = v[j] * inv;
 }
 
 // Rows between the two (2049 to 16 384 elements: the keys of an attention row): a workgroup of four waves per row, the row in
@@ -1282,6 +1320,11 @@ MLLM_API size_t mllm_hip_softmax_workspace_bytes(int64_t rows, int64_t len) {
   if (rows <= 0 || len <= 0) return 0;
   return (size_t)rows * softmax_pieces(rows, len) * 2 * sizeof(float);
 }
+MLLM_API int mllm_hip_softmax_set_wait(int polls) {
+  if (polls < -1) return MLLM_HIP_E_BADARG;
+  g_softmax_polls = polls;
+  return 0;
+}
 MLLM_API int mllm_hip_softmax_ws(const float* x, float* y, int64_t rows, int64_t len, void* workspace, void* stream) {
   const int pieces = workspace && rows > 0 && len > 0 ? softmax_pieces(rows, len) : 0;
   if (!pieces) return mllm_hip_softmax(x, y, rows, len, stream);
@@ -1290,9 +1333,14 @@ MLLM_API int mllm_hip_softmax_ws(const float* x, float* y, int64_t rows, int64_t
   const dim3 grid((unsigned)pieces, (unsigned)rows);
   hipStream_t st = (hipStream_t)stream;
   float* ws = reinterpret_cast<float*>(workspace);
-  hipLaunchKernelGGL(softmax_pieces_kernel<0>, grid, dim3(256), 0, st, x, y, ws, (int)len, g_exp_accurate);
-  hipLaunchKernelGGL(softmax_pieces_kernel<1>, grid, dim3(256), 0, st, x, y, ws, (int)len, g_exp_accurate);
-  hipLaunchKernelGGL(softmax_pieces_kernel<2>, grid, dim3(256), 0, st, x, y, ws, (int)len, g_exp_accurate);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, x, y, ws, (int)len, g_exp_accurate, g_softmax_polls); };
+  go(softmax_pieces_kernel<0>);
+  if (pieces <= SOFTMAX_WAIT_PIECES && pieces * rows <= SOFTMAX_WAIT && g_softmax_polls >= 0) {
+    go(softmax_pieces_kernel<3>);
+  } else {
+    go(softmax_pieces_kernel<1>);
+    go(softmax_pieces_kernel<2>);
+  }
   return (int)hipGetLastError();
 }
 

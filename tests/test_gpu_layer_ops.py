@@ -337,6 +337,24 @@ def test_softmax_pieces_treat_infinities_and_nan_as_whole_rows_do(ln):
     assert ((y[ok] - want[ok]).abs() <= 124 * 2.0 ** -24 * want[ok]).all()
 
 
+@pytest.mark.parametrize("rows,ln", [(1, 40961), (5, 45057), (8, 151936), (13, 151931), (14, 151936), (2, 262144), (2, 262145)])
+def test_softmax_pieces_that_wait_for_each_other(rows, ln):
+    """sums looked for by the workgroups, added up by each where none is seen in time (no look but the first), and by a launch of their
+    own (also the last sizes, more than 512 workgroups or 64 pieces of a row): the same bits, with a row of NaN and one of infinities"""
+    x = torch.randn((rows, ln), generator=torch.Generator().manual_seed(rows + ln)) * 3
+    x[rows - 1, ln // 2] = float("inf")
+    x[0, 4097] = float("nan") if rows > 1 else 0.
+    xd, got = x.cuda(), []
+    for polls in (4096, 0, -1):
+        announce("softmax pieces with %d looks" % polls, rows, ln)
+        try:
+            assert _lib.lib().mllm_hip_softmax_set_wait(polls) == 0
+            got.append(ql.softmax(xd).cpu())
+        finally:
+            assert _lib.lib().mllm_hip_softmax_set_wait(4096) == 0
+    assert torch.equal(got[0].view(torch.int32), got[1].view(torch.int32)) and torch.equal(got[0].view(torch.int32), got[2].view(torch.int32))
+
+
 @pytest.mark.parametrize("ln", [4100, 8193, 151_936])
 @pytest.mark.parametrize("k", [1, 50, 128])
 def test_topk_pieces_order_infinities_nan_and_zeros_as_whole_rows_do(ln, k):
