@@ -7,6 +7,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libmllm_hip_qlinear.so")
+CALLS_PATH = os.path.join(_HERE, "lib", "mllm_calls.so")  # the short calls of qlinear.py
 
 _lib = None
 

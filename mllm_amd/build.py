@@ -14,6 +14,7 @@ LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libmllm_hip_qlinear.so")
 HOST_LIB = os.path.join(LIBDIR, "libmllm_hip_backend.so")  # C++ op-factory layer on top of the C ABI
 HOST = os.path.join(CSRC, "host")
+CALLS_LIB = os.path.join(LIBDIR, "mllm_calls.so")  # the short calls of qlinear.py (a Python extension module)
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # no fast-math: the activation quantization needs correctly rounded fp32 division and plain multiplies;
@@ -50,6 +51,7 @@ def build(keep_asm=False, jobs=8):
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stderr)
     build_host()
+    build_calls()
     return LIB
 
 
@@ -66,6 +68,25 @@ def build_host():
     if err.strip():
         sys.stderr.write(err + "\n")
     return HOST_LIB
+
+
+def build_calls():
+    """The Python extension module, linked against the kernel library and torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I" + os.path.join(ROOT, "include")]
+    cmd += ["-isystem" + d for d in cpp_extension.include_paths() + [sysconfig.get_paths()["include"]]]
+    cmd += [os.path.join(CSRC, "python", "calls.cpp"), "-o", CALLS_LIB, "-L" + LIBDIR, "-lmllm_hip_qlinear", "-Wl,-rpath,$ORIGIN"]
+    cmd += ["-L" + d for d in cpp_extension.library_paths()] + ["-lc10", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("extension module build failed:\n" + r.stderr)
+    if r.stderr.strip():
+        sys.stderr.write(r.stderr + "\n")
+    return CALLS_LIB
 
 
 if __name__ == "__main__":

@@ -4,6 +4,8 @@ torch is used for device memory and the current stream only; every computation i
 libmllm_hip_qlinear.so.  Enumerations mirror include/mllm_hip_qlinear.h.
 """
 import ctypes as C
+import importlib.util
+import os
 
 import torch
 
@@ -13,6 +15,21 @@ Q4_0, Q8_0 = 0, 1
 F32, BF16 = 0, 1
 SCALE_IEEE, SCALE_X86_REF = 0, 1
 BLOCK_BYTES = {Q4_0: 18, Q8_0: 34}
+
+
+_native = None
+
+
+def _calls():
+    """the extension module of the short calls (csrc/python/calls.cpp)"""
+    global _native
+    if _native is None:
+        _lib.lib()
+        if not os.path.exists(_lib.CALLS_PATH):
+            raise _lib.HipQLinearError("%s not found: build it with `python -m mllm_amd.build`" % _lib.CALLS_PATH)
+        spec = importlib.util.spec_from_file_location("mllm_calls", _lib.CALLS_PATH)
+        _native = importlib.util.module_from_spec(spec)
+    return _native
 
 
 def _stream():
@@ -82,13 +99,7 @@ class PackedQWeight:
 
 def linear_q_gemv(w, x, bias=None, act_scale_mode=SCALE_X86_REF, out=None):
     """y = Linear(x) with Q4_0/Q8_0 weights (more than eight rows: passes of eight).  x [M, K] fp32/bf16 on the GPU -> y fp32 [M, N]."""
-    assert x.is_cuda and x.is_contiguous() and x.dim() == 2 and x.shape[1] == w.K
-    M = x.shape[0]
-    y = out if out is not None else torch.empty((M, w.N), dtype=torch.float32, device="cuda")
-    _lib.check(_lib.lib().mllm_hip_linear_q_gemv(w.wtype, w.ptr, x.data_ptr(), _xdtype(x),
-                                                 bias.data_ptr() if bias is not None else None, y.data_ptr(), M, w.N,
-                                                 w.K, act_scale_mode, _stream()), "mllm_hip_linear_q_gemv")
-    return y
+    return _calls().linear_q_gemv(w.wtype, w.buf, w.N, w.K, x, bias, act_scale_mode, out)
 
 
 def gemv_workspace(M, K, n_total=None):
@@ -103,20 +114,7 @@ def gemv_workspace(M, K, n_total=None):
 def linear_q_gemv_multi(ws, x, biases=None, act_scale_mode=SCALE_X86_REF, outs=None, workspace=None):
     """Sibling projections (same x, same K) in one launch.  ws: list of PackedQWeight; returns the list of outputs.
     With a workspace (gemv_workspace) and M >= 3, x is quantized once by a small kernel instead of in every workgroup."""
-    assert 1 <= len(ws) <= 4 and x.is_cuda and x.is_contiguous() and x.dim() == 2
-    M, K = x.shape
-    if outs is None:
-        outs = [torch.empty((M, w.N), dtype=torch.float32, device="cuda") for w in ws]
-    parts = (_lib.GemvPart * len(ws))()
-    for i, w in enumerate(ws):
-        assert w.K == K and w.wtype == ws[0].wtype
-        b = biases[i] if biases is not None else None
-        parts[i] = _lib.GemvPart(w.ptr, b.data_ptr() if b is not None else None, outs[i].data_ptr(), w.N)
-    _lib.check(_lib.lib().mllm_hip_linear_q_gemv_multi_wsn(ws[0].wtype, len(ws), parts, x.data_ptr(), _xdtype(x), M, K,
-                                                           act_scale_mode, _p(workspace),
-                                                           workspace.numel() if workspace is not None else 0, _stream()),
-               "mllm_hip_linear_q_gemv_multi_wsn")
-    return outs
+    return _calls().linear_q_gemv_multi(ws, x, biases, act_scale_mode, outs, workspace)
 
 
 Q8_IMAGE = 2  # MLLM_HIP_Q8_IMAGE
@@ -237,16 +235,7 @@ def w8a8_gemm_packed(xq, x_scale, W_packed, N, w_scale, bias=None, want_acc=Fals
 
 def w8a8_linear_packed(x, W_packed, N, w_scale, bias=None, workspace=None, out=None):
     """As w8a8_linear, with the weights from w8a8_prepack."""
-    M, K = x.shape
-    L = _lib.lib()
-    assert W_packed.numel() == L.mllm_hip_w8a8_packed_bytes(N, K)
-    if workspace is None:
-        workspace = torch.empty(L.mllm_hip_w8a8_workspace_bytes(M, K), dtype=torch.uint8, device="cuda")
-    y = out if out is not None else torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
-    _lib.check(L.mllm_hip_w8a8_linear_packed(x.data_ptr(), _xdtype(x), W_packed.data_ptr(), w_scale.data_ptr(), _p(bias),
-                                             y.data_ptr(), M, N, K, workspace.data_ptr(), _stream()),
-               "mllm_hip_w8a8_linear_packed")
-    return y
+    return _calls().w8a8_linear_packed(x, W_packed, N, w_scale, bias, workspace, out)
 
 
 # ----------------------------------------------------------------------------- W4A16 (group-wise uint4 + zero point)
@@ -293,14 +282,7 @@ def w4a16_prepack(qw, scales, zeros, group=128):
 
 def w4a16_gemm_packed(a, packed, N, bias=None, group=128, out=None):
     """a bf16 [M, K] x packed weights (w4a16_prepack) -> bf16 [M, N]."""
-    assert a.dtype == torch.bfloat16 and a.is_contiguous()
-    M, K = a.shape
-    L = _lib.lib()
-    assert packed.numel() == L.mllm_hip_w4a16_packed_bytes(N, K, group)
-    y = out if out is not None else torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
-    _lib.check(L.mllm_hip_w4a16_gemm_packed(a.data_ptr(), packed.data_ptr(), _p(bias), y.data_ptr(), M, N, K, group,
-                                            _stream()), "mllm_hip_w4a16_gemm_packed")
-    return y
+    return _calls().w4a16_gemm_packed(a, packed, N, bias, group, out)
 
 
 def w4a16_dequantize_packed(packed, N, K, group=128):
@@ -502,27 +484,11 @@ def set_exp_mode(accurate):
 
 
 def softmax(x):
-    assert x.is_cuda and x.is_contiguous() and x.dtype == torch.float32
-    n = x.shape[-1]
-    y = torch.empty_like(x)
-    rows, L = x.numel() // n, _lib.lib()
-    need = L.mllm_hip_softmax_workspace_bytes(rows, n)
-    ws = torch.empty(need, dtype=torch.uint8, device="cuda") if need else None
-    _lib.check(L.mllm_hip_softmax_ws(x.data_ptr(), y.data_ptr(), rows, n, _p(ws), _stream()), "mllm_hip_softmax_ws")
-    return y
+    return _calls().softmax(x)
 
 
 def topk(x, k, largest=True, sorted=True):
-    assert x.is_cuda and x.is_contiguous() and x.dtype == torch.float32
-    n = x.shape[-1]
-    v = torch.empty(x.shape[:-1] + (k,), dtype=torch.float32, device="cuda")
-    i = torch.empty(x.shape[:-1] + (k,), dtype=torch.int32, device="cuda")
-    rows, L = x.numel() // n, _lib.lib()
-    need = L.mllm_hip_topk_workspace_bytes(rows, n, k)
-    ws = torch.empty(need, dtype=torch.uint8, device="cuda") if need else None
-    _lib.check(L.mllm_hip_topk_ws(x.data_ptr(), v.data_ptr(), i.data_ptr(), rows, n, k, int(largest), int(sorted), _p(ws), _stream()),
-               "mllm_hip_topk_ws")
-    return v, i
+    return _calls().topk(x, k, largest, sorted)
 
 
 def moe_gate(x, gate_weight, k, norm_topk_prob=True, want_scores=False, scores=None):
@@ -706,25 +672,9 @@ def quantize_q8_K(x):
 
 
 # ----------------------------------------------------------------------------- MatMul (activation x activation)
-_MM_DTYPE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 3}
 
 
 def matmul(a, b, transpose_a=False, transpose_b=False, out=None):
     """C[..., M, N] = op(a) @ op(b) for fp32 / bf16 / fp16 tensors of rank >= 2, the whole batch in one launch; b may be a
     single matrix shared by every batch entry.  mllm/backends/cpu/ops/MatMulOp.cpp:19-90."""
-    assert a.dtype == b.dtype and a.dtype in _MM_DTYPE and a.is_contiguous() and b.is_contiguous()
-    M, K = (a.shape[-1], a.shape[-2]) if transpose_a else (a.shape[-2], a.shape[-1])
-    N, Kb = (b.shape[-2], b.shape[-1]) if transpose_b else (b.shape[-1], b.shape[-2])
-    assert K == Kb
-    batch = 1
-    for d in a.shape[:-2]:
-        batch *= d
-    b_batch = 1
-    for d in b.shape[:-2]:
-        b_batch *= d
-    assert b_batch in (1, batch)
-    c = out if out is not None else torch.empty(tuple(a.shape[:-2]) + (M, N), dtype=a.dtype, device="cuda")
-    _lib.check(_lib.lib().mllm_hip_matmul_batched(a.data_ptr(), b.data_ptr(), c.data_ptr(), _MM_DTYPE[a.dtype], batch, M, N, K,
-                                                  M * K, N * K if b_batch == batch and batch > 1 else 0, M * N,
-                                                  int(transpose_a), int(transpose_b), _stream()), "mllm_hip_matmul_batched")
-    return c
+    return _calls().matmul(a, b, transpose_a, transpose_b, out)

@@ -1,0 +1,68 @@
+"""The short calls of qlinear.py in native code (csrc/python/calls.cpp): what they refuse, before any device call, and that they use the
+caller's outputs, workspaces and stream."""
+import numpy as np
+import pytest
+import torch
+
+from mllm_amd import _lib, qlinear as ql
+from gpu_util import announce
+
+
+class _W:
+    wtype, N, K, buf = 0, 64, 64, torch.zeros(1, dtype=torch.uint8)
+
+
+X = torch.zeros(3, 64)
+
+
+@pytest.mark.parametrize("call,error", [
+    (lambda: ql.linear_q_gemv(_W, X), AssertionError), (lambda: ql.linear_q_gemv(_W, None), TypeError),
+    (lambda: ql.linear_q_gemv_multi([], X), AssertionError), (lambda: ql.linear_q_gemv_multi([_W] * 5, X), AssertionError),
+    (lambda: ql.linear_q_gemv_multi([_W], X), AssertionError), (lambda: ql.linear_q_gemv_multi(None, X), TypeError),
+    (lambda: ql.softmax(X), AssertionError), (lambda: ql.topk(X, 3), AssertionError),
+    (lambda: ql.matmul(X, X), AssertionError), (lambda: ql.matmul(X, X.double()), AssertionError), (lambda: ql.matmul(X[0], X[0]), IndexError),
+    (lambda: ql.matmul(X.t(), X.t()), AssertionError), (lambda: ql.matmul(X.double(), X.double(), False, True), AssertionError),
+    (lambda: ql.matmul(torch.zeros(2, 3, 4), torch.zeros(3, 4, 5)), AssertionError),
+    (lambda: ql.w8a8_linear_packed(X, X, 64, X), AssertionError), (lambda: ql.w8a8_linear_packed(X[0], X, 64, X), ValueError),
+    (lambda: ql.w4a16_gemm_packed(X, X, 64), AssertionError), (lambda: ql.w4a16_gemm_packed(X.bfloat16(), X, 64), AssertionError)])
+def test_calls_refuse_what_the_kernels_do_not_take(call, error):
+    with pytest.raises(error):
+        call()
+
+
+def test_missing_module_fails_loudly(monkeypatch):
+    monkeypatch.setattr(ql, "_native", None)
+    monkeypatch.setattr(_lib, "CALLS_PATH", "/nonexistent/mllm_calls.so")
+    with pytest.raises(_lib.HipQLinearError):
+        ql.softmax(X)
+
+
+@pytest.mark.gpu
+def test_calls_use_the_callers_outputs_and_stream():
+    g = torch.Generator(device="cuda").manual_seed(2)
+    rand = lambda *s: torch.randn(s, device="cuda", generator=g)  # noqa: E731
+    w, x, a, b = ql.PackedQWeight.synthetic(ql.Q4_0, 256, 256, g), rand(3, 256), rand(2, 70, 40), rand(2, 40, 50)
+    bias, room = rand(256), ql.gemv_workspace(3, 256, 512)
+    out = lambda *s: torch.full(s, float("nan"), device="cuda")  # noqa: E731
+    announce("calls with and without outputs")
+    y, c = ql.linear_q_gemv(w, x, bias), ql.matmul(a, b)
+    ys = ql.linear_q_gemv_multi([w, w], x, [bias, None])
+    assert torch.equal(y, ys[0]) and torch.equal(y, ys[1] + bias) and y.shape == (3, 256) and c.shape == (2, 70, 50) and c.dtype == torch.float32
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(200_000_000)  # a call on the default stream would not wait for what follows
+        xs, outs = x * 1, [out(3, 256), out(3, 256)]
+        y1, c1 = out(3, 256), out(2, 70, 50)
+        assert ql.linear_q_gemv(w, xs, bias, out=y1) is y1 and ql.matmul(a * 1, b, out=c1) is c1
+        assert ql.linear_q_gemv_multi([w, w], xs, [bias, None], outs=outs, workspace=room) is outs
+        p = ql.softmax(xs)
+        values, ids = ql.topk(p, 7)
+    stream.synchronize()
+    assert torch.equal(y1, y) and torch.equal(c1, c) and float((outs[0] - y).norm() / y.norm()) < 1e-5
+    assert torch.equal(ids.long(), p.topk(7).indices) and torch.equal(values, p.topk(7).values)
+    with pytest.raises(_lib.HipQLinearError):
+        ql.topk(p, 257)
+    with pytest.raises(TypeError):
+        ql.linear_q_gemv(w, x.half())
+    assert np.isfinite(y.cpu().numpy()).all()
