@@ -867,16 +867,18 @@ __global__ __launch_bounds__(NT) void topk_select_rows_kernel(const float* __res
 // Few long rows spread over the chip (mllm_hip_topk_ws), k up to 128: a row is cut into equal pieces of at most TOPK_PIECE elements, a
 // workgroup selects the k largest keys of its piece into the caller's workspace, and a second launch selects among the
 // pieces' keys.  A workgroup per row is bound by what one CU loads per pass over the row: 20 of eight rows of 151 936 take
-// 110 us there and 12 here, 64 of them 111 and 15.
+// 110 us there and 9.7 here, 64 of them 111 and 12.5.
 //
 // Selection inside a workgroup: keys are unique (value, inverted index).  The k-th largest of the threads' own maxima (found a
 // bit at a time by counting, every wave on its own) is at most the k-th largest value, so the keys at or above it contain the
 // selection, and of keys that are spread over the threads in any order they are few more than k (about 180 at k = 128).  They
 // are collected in LDS and placed by rank, up to 64 of them in the registers of one wave; should they be more than TOPK_CAND
-// (many equal values, or one thread's keys all larger than the other threads'), the k-th key itself is found a bit at a time.
+// (many equal values, or one thread's keys all larger than the other threads'), the k-th key itself is found a bit at a time.  The bound
+// is taken as soon as at most twelve maxima more than k reach it, and the second launch takes values from the keys: with the exact bound and
+// the values read again 8 x 151 936 took 10.8 us for the largest 20 (9.7 now), 8.85 for one (7.3), 8 x 32 000 12.8 for 64 (10.3).
 // Equal pieces, so that every thread has elements: a last piece of 432 (12 720 cut at 4096s) gave 108 threads four each, all of them
 // candidates for the largest 128 (256 rows of 12 720: 37.8 us, 19.7 in equal pieces, 20.3 as a workgroup per row).
-// Limits, in a graph, us, a workgroup per row / pieces, the largest 1 | 50 | 128: 8 rows of 4100: 17.6 / 8.6 | 19.1 / 12.9 | 21.3 / 13.9 (up to
+// Limits, in a graph, us, a workgroup per row / pieces (with the exact bound, 0.4 to 2 us more than now), the largest 1 | 50 | 128: 8 rows of 4100: 17.6 / 8.6 | 19.1 / 12.9 | 21.3 / 13.9 (up to
 // 4096 a row is one piece, and the second launch has nothing to merge), of 151 936: 109 / 9.3 | 111 / 15.0 | 113 / 23.5; 512 rows of 4100: 19.0 /
 // 11.7 | 20.9 / 16.8 | 24.1 / 19.4, of 151 936: 256 / 76 | 260 / 101 | 264 / 143.  Pieces win on either side of 512 rows (1024 rows of 4100:
 // 38.2 / 23.5, of 151 936: 511 / 187, the largest 50); the limits bound the workspace, 512 x 38 pieces x 128 keys of 8 bytes: 20 MB.
@@ -907,11 +909,16 @@ __device__ __forceinline__ int block_topk_256(const unsigned long long (&key)[R]
   sh.maxima[tid] = (uint32_t)(mine >> 32);
   __syncthreads();
   const u32x4 m4 = *reinterpret_cast<const u32x4*>(&sh.maxima[4 * lane]);  // every wave on its own, four maxima per lane
+  // a bit costs about 100 clocks (four ballots, their counts and a branch); it need not be the k-th largest exactly: enough once few are left
   uint32_t b32 = 0;
-  for (int bit = 31; bit >= 0; bit--) {
+  int reach = 256;  // maxima at or above b32
+  for (int bit = 31; bit >= 0 && reach > k + 12; bit--) {
     const uint32_t t = b32 | (1u << bit);
     const int c = __popcll(__ballot(m4.x >= t)) + __popcll(__ballot(m4.y >= t)) + __popcll(__ballot(m4.z >= t)) + __popcll(__ballot(m4.w >= t));
-    if (c >= k) b32 = t;
+    if (c >= k) {
+      b32 = t;
+      reach = c;
+    }
   }
   unsigned long long bound = (unsigned long long)b32 << 32;
   if (bound == 0) bound = 1;  // fewer than k threads hold an element: every element is wanted
@@ -991,7 +998,7 @@ __global__ __launch_bounds__(256) void topk_pieces_kernel(const float* __restric
 template <int R>
 __global__ __launch_bounds__(256) void topk_merge_kernel(const float* __restrict__ x, const unsigned long long* __restrict__ ws,
                                                          float* __restrict__ values, int32_t* __restrict__ indices, int len, int n, int k,
-                                                         int sorted) {
+                                                         int largest, int sorted) {
   __shared__ TopkShared sh;
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x;
@@ -1007,7 +1014,11 @@ __global__ __launch_bounds__(256) void topk_merge_kernel(const float* __restrict
       for (int j = 0; j < k; j++) r += (uint32_t)sh.top[j] > (uint32_t)my ? 1 : 0;  // the inverted index: larger = earlier
     }
     const int idx = (int)~(uint32_t)my;
-    values[row * k + r] = x[row * len + idx];
+    uint32_t b = (uint32_t)(my >> 32);  // order_key undone: not for zeros (of either sign) and NaN, which are read again
+    if (!largest) b = ~b;
+    float v = __uint_as_float(b & 0x80000000u ? b ^ 0x80000000u : ~b);
+    if (v == 0.f || v != v) v = x[row * len + idx];
+    values[row * k + r] = v;
     indices[row * k + r] = idx;
   }
 }
@@ -1372,8 +1383,8 @@ MLLM_API int mllm_hip_topk_ws(const float* x, float* values, int32_t* indices, i
   const int units = (int)(vec ? len / 4 : len), per = (units + pieces - 1) / pieces;  // (at most TOPK_PIECE elements)
   if (vec) hipLaunchKernelGGL(topk_pieces_kernel<4>, grid, dim3(256), 0, st, x, ws, (int)len, per, k, largest);
   else hipLaunchKernelGGL(topk_pieces_kernel<1>, grid, dim3(256), 0, st, x, ws, (int)len, per, k, largest);
-  if (pieces * k <= 1024) hipLaunchKernelGGL(topk_merge_kernel<4>, dim3((unsigned)rows), dim3(256), 0, st, x, ws, values, indices, (int)len, pieces * k, k, sorted);
-  else hipLaunchKernelGGL(topk_merge_kernel<TOPK_MERGE_R>, dim3((unsigned)rows), dim3(256), 0, st, x, ws, values, indices, (int)len, pieces * k, k, sorted);
+  if (pieces * k <= 1024) hipLaunchKernelGGL(topk_merge_kernel<4>, dim3((unsigned)rows), dim3(256), 0, st, x, ws, values, indices, (int)len, pieces * k, k, largest, sorted);
+  else hipLaunchKernelGGL(topk_merge_kernel<TOPK_MERGE_R>, dim3((unsigned)rows), dim3(256), 0, st, x, ws, values, indices, (int)len, pieces * k, k, largest, sorted);
   return (int)hipGetLastError();
 }
 
