@@ -1056,19 +1056,30 @@ __device__ __forceinline__ void gate_stage_x(const GateArgs& a, int64_t tok0, in
     dst[1] = f32x4{v[4], v[5], v[6], v[7]};
   }
 }
-// logits of experts e0 + wave, e0 + wave + nwaves, ... < e1 for the ntok tokens in s_x; out[t * ostride + e]
+constexpr int GATE_CB = 8;  // pieces of a row a lane requests before it multiplies the first
+struct GatePieces {
+  f32x4 v[GATE_CB];
+};
+__device__ __forceinline__ void gate_request(const GateArgs& a, int e, int c0, GatePieces& p) {
+  const f32x4* wr = reinterpret_cast<const f32x4*>(a.w + (size_t)min(e, a.E - 1) * a.H);
+  const int last = (a.H >> 2) - 1;
+#pragma unroll
+  for (int u = 0; u < GATE_CB; u++) p.v[u] = wr[min(c0 + 64 * u, last)];
+}
+// logits of experts e0 + wave, e0 + wave + nwaves, ... < e1 for the ntok tokens in s_x; out[t * ostride + e].  first: the first of the
+// pieces, requested before x was staged
 __device__ __forceinline__ void gate_logits(const GateArgs& a, const float* s_x, int ntok, int e0, int e1, int wave, int nwaves, int lane,
-                                            float* out, size_t ostride) {
-  constexpr int CB = 8;  // pieces of a row a lane requests before it multiplies the first
+                                            const GatePieces& first, float* out, size_t ostride) {
+  constexpr int CB = GATE_CB;
   const int nc = a.H >> 2;
+  GatePieces w = first;
+  f32x4(&wv)[CB] = w.v;
+  bool have = true;
   for (int e = e0 + wave; e < e1; e += nwaves) {
     float acc[GATE_TOK] = {0.f, 0.f, 0.f, 0.f};
-    const f32x4* wr = reinterpret_cast<const f32x4*>(a.w + (size_t)e * a.H);
     for (int c0 = lane; c0 < nc; c0 += 64 * CB) {
-      f32x4 wv[CB];
-#pragma unroll
-      for (int u = 0; u < CB; u++)
-        if (c0 + 64 * u < nc) wv[u] = wr[c0 + 64 * u];
+      if (!have) gate_request(a, e, c0, w);  // (uniform)
+      have = false;
 #pragma unroll
       for (int u = 0; u < CB; u++) {
         const int c = c0 + 64 * u;
@@ -1093,6 +1104,86 @@ __device__ __forceinline__ void gate_logits(const GateArgs& a, const float* s_x,
         if (lane == 0) out[t * ostride + e] = s;
       }
     }
+  }
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, true));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, true));
+  const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  v = max((uint32_t)a[0], (uint32_t)a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return max((uint32_t)b[0], (uint32_t)b[1]);
+}
+// The same for up to 64 R experts, of which k is at most GATE_ROUNDS, without LDS but for the k selected: the lane keeps the logits of experts
+// lane + 64 j, and a round takes the largest of what is left (a butterfly within the wave and a ballot, some 120 clocks; by rank the token's
+// 128 scores were compared with every lane's through LDS, 3 us).  Same sums, selection and weights bit for bit.
+constexpr int GATE_ROUNDS = 16;
+template <int R>
+__device__ __forceinline__ void gate_select_rounds(const GateArgs& a, float (&v)[R], int64_t tok, float* tv, int* ti, int lane) {
+  const bool poly = a.E > 16 && !a.exp_accurate;
+  float mx = -3.402823466e+38f;
+#pragma unroll
+  for (int j = 0; j < R; j++)
+    if (lane + 64 * j < a.E) mx = fmaxf(mx, v[j]);
+  mx = wave_max(mx);
+  float sum = 0.f;
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    const int i = lane + 64 * j;
+    if (i < a.E) {
+      v[j] = softmax_exp(v[j] - mx, poly && i < (a.E & ~7));
+      sum += v[j];
+    }
+  }
+  sum = wave_sum(sum);
+  const float inv = 1.f / sum;
+  uint32_t key[R];
+  unsigned long long taken[R];
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    const int i = lane + 64 * j;
+    v[j] *= inv;
+    if (a.scores && i < a.E) a.scores[tok * a.E + i] = v[j];
+    key[j] = i < a.E ? max((uint32_t)(order_key(v[j], 0, true) >> 32), 1u) : 0u;
+    taken[j] = 0;
+  }
+  for (int r = 0; r < a.k; r++) {
+    uint32_t m = key[0];
+#pragma unroll
+    for (int j = 1; j < R; j++) m = max(m, key[j]);
+    m = wave_max_u32(m);
+    bool found = false;  // (uniform) the lowest index among equal ones
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const unsigned long long at = __ballot(key[j] == m);
+      if (!found && at) {
+        const unsigned long long one = at & (0ull - at);
+        taken[j] |= one;
+        if ((one >> lane) & 1) key[j] = 0u;
+        found = true;
+      }
+    }
+  }
+  int before = 0;
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    if ((taken[j] >> lane) & 1) {
+      const int pos = before + __popcll(taken[j] & ((1ull << lane) - 1ull));
+      tv[pos] = v[j];
+      ti[pos] = lane + 64 * j;
+    }
+    before += __popcll(taken[j]);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  float tsum = 0.f;
+  for (int r = 0; r < a.k; r++) tsum += tv[r];
+  if (lane < a.k) {
+    const float wv = tv[lane];
+    a.weights[tok * a.k + lane] = a.norm ? wv / tsum : wv;
+    a.ids[tok * a.k + lane] = ti[lane];
   }
 }
 // one wave finishes one token: softmax over its E logits in lg (LDS, overwritten), the k largest in index order, weights
@@ -1131,6 +1222,25 @@ __device__ __forceinline__ void gate_select(const GateArgs& a, float* lg, int64_
     a.ids[tok * a.k + r] = ti[r];
   }
 }
+// the logits of a token, in LDS or in memory -> its experts; lg: LDS for them
+__device__ __forceinline__ void gate_finish(const GateArgs& a, const float* logits, float* lg, int64_t tok, float* tv, int* ti, int lane) {
+  auto rounds = [&](auto held) {
+    float(&v)[sizeof(held) / sizeof(float)] = held.v;
+#pragma unroll
+    for (int j = 0; j < (int)(sizeof(held) / sizeof(float)); j++) v[j] = lane + 64 * j < a.E ? logits[lane + 64 * j] : 0.f;
+    gate_select_rounds(a, v, tok, tv, ti, lane);
+  };
+  struct Two { float v[2]; };
+  struct Four { float v[4]; };
+  if (a.k <= GATE_ROUNDS && a.E <= 128) return rounds(Two{});
+  if (a.k <= GATE_ROUNDS && a.E <= 256) return rounds(Four{});
+  if (logits != lg) {
+    for (int i = lane; i < a.E; i += 64) lg[i] = logits[i];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  gate_select(a, lg, tok, tv, ti, lane);
+}
 // everything in one launch: a workgroup per four tokens (callers that pass no scores buffer)
 template <int XT>
 __global__ __launch_bounds__(GATE_WAVES * 64) void moe_gate_kernel(GateArgs a) {
@@ -1142,12 +1252,14 @@ __global__ __launch_bounds__(GATE_WAVES * 64) void moe_gate_kernel(GateArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t tok0 = (int64_t)blockIdx.x * GATE_TOK;
   const int ntok = (int)min((int64_t)GATE_TOK, a.M - tok0);  // uniform
+  GatePieces first;
+  gate_request(a, wave, lane, first);
   gate_stage_x<XT>(a, tok0, ntok, s_x, tid, GATE_WAVES * 64);
   __syncthreads();
-  gate_logits(a, s_x, ntok, 0, a.E, wave, GATE_WAVES, lane, s_logit, (size_t)a.E);
+  gate_logits(a, s_x, ntok, 0, a.E, wave, GATE_WAVES, lane, first, s_logit, (size_t)a.E);
   __syncthreads();
   if (wave >= ntok) return;
-  gate_select(a, s_logit + wave * a.E, tok0 + wave, s_tv + wave * a.k, s_ti + wave * a.k, lane);
+  gate_finish(a, s_logit + wave * a.E, s_logit + wave * a.E, tok0 + wave, s_tv + wave * a.k, s_ti + wave * a.k, lane);
 }
 // The same in two launches for callers that pass a scores buffer, which holds the logits in between: with few tokens one
 // workgroup per four tokens leaves the chip to one CU (a decode token: 1 MB of gate weights through one workgroup), so the
@@ -1160,10 +1272,12 @@ __global__ __launch_bounds__(GATE_WAVES * 64) void moe_gate_logits_kernel(GateAr
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nthreads = blockDim.x;
   const int64_t tok0 = (int64_t)blockIdx.x * GATE_TOK;
   const int ntok = (int)min((int64_t)GATE_TOK, a.M - tok0);  // uniform
+  const int e0 = (int)blockIdx.y * epg;
+  GatePieces first;
+  gate_request(a, e0 + wave, lane, first);
   gate_stage_x<XT>(a, tok0, ntok, s_x, tid, nthreads);
   __syncthreads();
-  const int e0 = (int)blockIdx.y * epg;
-  gate_logits(a, s_x, ntok, e0, min(a.E, e0 + epg), wave, nthreads >> 6, lane, a.scores + tok0 * a.E, (size_t)a.E);
+  gate_logits(a, s_x, ntok, e0, min(a.E, e0 + epg), wave, nthreads >> 6, lane, first, a.scores + tok0 * a.E, (size_t)a.E);
 }
 __global__ __launch_bounds__(GATE_TOK * 64) void moe_gate_select_kernel(GateArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -1173,11 +1287,7 @@ __global__ __launch_bounds__(GATE_TOK * 64) void moe_gate_select_kernel(GateArgs
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t tok = (int64_t)blockIdx.x * GATE_TOK + wave;
   if (tok >= a.M) return;  // (no workgroup barrier below)
-  float* lg = s_logit + wave * a.E;
-  for (int i = lane; i < a.E; i += 64) lg[i] = a.scores[tok * a.E + i];
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  gate_select(a, lg, tok, s_tv + wave * a.k, s_ti + wave * a.k, lane);
+  gate_finish(a, a.scores + tok * a.E, s_logit + wave * a.E, tok, s_tv + wave * a.k, s_ti + wave * a.k, lane);
 }
 
 }  // namespace mllmhip

@@ -428,6 +428,21 @@ def test_topk_pieces_are_equal(rows, ln, k):
     assert torch.equal(i, wi) and torch.equal(v, wv)
 
 
+@pytest.mark.parametrize("E,k", [(1, 1), (16, 16), (17, 17), (63, 5), (64, 16), (65, 16), (127, 1), (128, 17), (129, 16), (256, 16), (257, 16), (300, 9)])
+def test_moe_gate_selection_at_the_edges_of_its_forms(E, k):
+    """up to 256 experts of which up to 16 are taken stay in registers, more go through LDS; equal logits (experts in threes) go lowest index
+    first; H that is not a whole batch of pieces"""
+    rng = synth.rng_for(6, 6100 + 3 * E + k)
+    w = np.repeat(rng.standard_normal(((E + 2) // 3, 2312)) * 0.05, 3, 0)[:E].astype(np.float32)
+    w[0] = w[E // 2]
+    xf = synth.make_x_fp32(rng, 9, 2312)
+    announce("moe gate edges", E, k)
+    ids, wt, sc = (t.cpu().numpy() for t in ql.moe_gate(to_dev(xf), to_dev(w), k, True, want_scores=True))
+    assert rel_l2(sc, orc.moe_gate(xf, w, k, True)[2]) < 1e-5
+    sv, si = orc.topk(sc, k, True, False)
+    assert np.array_equal(ids, si) and np.max(np.abs(wt - sv / sv.sum(-1, keepdims=True))) < 1e-6
+
+
 @pytest.mark.parametrize("M,H,E,k,dtype", [(512, 2048, 128, 8, "f32"), (1, 2048, 128, 8, "f32"), (7, 256, 60, 4, "f32"),
                                            (33, 2048, 128, 8, "bf16"), (5, 64, 8, 2, "f32")])
 def test_moe_gate(M, H, E, k, dtype):
