@@ -99,10 +99,11 @@ struct KrWeights {
 // TH = groups of four rows (Q4_K: always two).  ORDER: the sums, see above; pairs: one wave per tile.
 enum { KR_LINEAR, KR_TILES, KR_PAIRS };
 template <int WT, int XT, int TH, int ORDER>
-__global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
+__global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P_or_T) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr bool Q4 = WT == MLLM_HIP_Q4_K;
   constexpr bool TILES = ORDER == KR_TILES, PAIRS = ORDER == KR_PAIRS;
+  const int P = PAIRS ? 1 : P_or_T, T = PAIRS ? P_or_T : 1;  // waves per tile; tiles per wave
   static_assert(!PAIRS || (!Q4 && TH == 1), "pairs in groups: Q6_K, groups of four");
   constexpr int DEPTH = kr_depth(Q4, PAIRS ? 2 : TH);  // (pairs: sixteen accumulators)
   const int nsb = a.nsb, K = nsb * QK_K;
@@ -156,7 +157,7 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
 
   // ---- 1. activations requested, then the wave's first super-blocks of weights (memory requests return in order) ------------
   const int c = lane & 15, g = lane >> 4;
-  const int row0 = (((int)blockIdx.x - a.wg_start[pidx]) * tiles_wg + tl) * 16;
+  int row0 = (((int)blockIdx.x - a.wg_start[pidx]) * tiles_wg + tl) * T * 16;
   const uint32_t sbt = (uint32_t)N * (uint32_t)nsb;
   const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(kq_at(pt.w.a, mt.eoff)), 0, sbt * 128u, 0x00020000);
   const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(kq_at(Q4 ? pt.w.a : pt.w.h, mt.eoff)), 0, sbt * 64u, 0x00020000);
@@ -166,8 +167,13 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
   const int S = (nsb + sps - 1) / sps;
   const int sl0 = p * S / P, sl1 = (p + 1) * S / P;                // this wave's slices
   const int sb0 = sl0 * sps, sb1 = min(nsb, sl1 * sps);            // and super-blocks
-  const uint32_t rb8 = (uint32_t)(row0 + (lane >> 3)) * (uint32_t)nsb, rb4 = (uint32_t)(row0 + (lane >> 2)) * (uint32_t)nsb;
-  const bool ok8[2] = {row0 + (lane >> 3) < N, row0 + 8 + (lane >> 3) < N}, ok4 = row0 + (lane >> 2) < N;
+  uint32_t rb8, rb4;
+  bool ok8[2], ok4;
+  auto rows_of = [&](int r) {  // the rows that weights are requested of
+    rb8 = (uint32_t)(r + (lane >> 3)) * (uint32_t)nsb, rb4 = (uint32_t)(r + (lane >> 2)) * (uint32_t)nsb;
+    ok8[0] = r + (lane >> 3) < N, ok8[1] = r + 8 + (lane >> 3) < N, ok4 = r + (lane >> 2) < N;
+  };
+  rows_of(row0);
   KrWeights<WT, DEPTH> w;
   auto load_sb = [&](int i, int sb) {
 #pragma unroll
@@ -470,30 +476,70 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
     slice++;
     left = sps;
   };
-  constexpr int TRIPS = PAIRS ? 4 / DEPTH : 1;  // (pairs: the super-block modulo 4 is a constant)
-  for (int t0 = sb0; t0 < sb1; t0 += TRIPS * DEPTH) {
+  const auto bias_of = [&](int n) { return pt.bias ? pt.bias[n] : 0.f; };
+  auto write = [&]() {
+    const int n = row0 + c;
+    if (n >= N) return;
+    const float bias = bias_of(n);
 #pragma unroll
-    for (int t = 0; t < TRIPS; t++) {
-      const int sb = t0 + t * DEPTH;
-      if (t && sb >= sb1) break;  // uniform
-      put_scales();
-      load_scales(sb + DEPTH);  // (past the wave's last one: fetches nothing)
+    for (int k = 0; k < (PAIRS ? 1 : 2); k++) {
+      const int m = Q4 ? 4 * (g & 1) + (g >> 1) + 2 * k : (TILES ? g : 2 * (g & 1) + (g >> 1)) + 4 * k;
+      if (m >= mt.rows) continue;
+      const int64_t orow = a.slot_ids ? (int64_t)s_rows[m] : (int64_t)kq_tile_out_row(a, mt, m);
+      pt.y[orow * N + n] = pt.bias ? tot[k] + bias : tot[k];
+    }
+  };
+  if constexpr (PAIRS) {  // the wave's tiles one after the other; the next one's first super-block is requested with this one's last
+    for (int t = 0; t < T; t++) {
+#pragma unroll 1
+      for (int s4 = 0; s4 < nsb; s4 += 4) {
 #pragma unroll
-      for (int i = 0; i < DEPTH; i++) {
-        if (sb + i < sb1) {  // uniform
-          put_sb(i);
+        for (int i = 0; i < 4; i++) {  // (the super-block modulo 4 is a constant)
+          const int sb = s4 + i;
+          if (sb >= nsb) break;  // uniform
+          const bool last = sb + 1 == nsb;
+          int next = sb + 1;  // (past the wave's last one: fetches nothing)
+          if (last && t + 1 < T) {
+            rows_of(row0 + 16);
+            next = 0;
+          }
+          put_scales();
+          load_scales(next);
+          put_sb(0);
           __builtin_amdgcn_wave_barrier();
-          take_sb(i);
+          take_sb(0);
           __builtin_amdgcn_wave_barrier();
+          load_sb(0, next);
+          __builtin_amdgcn_sched_barrier(0);
+          compute(sb, i);
+          if (last) flush();
+          __builtin_amdgcn_sched_barrier(0);
         }
-        load_sb(i, sb + DEPTH + i);
-        __builtin_amdgcn_sched_barrier(0);
-        if (sb + i < sb1) {
-          compute(sb + i, t * DEPTH + i);
-          if (--left == 0 || sb + i + 1 == nsb) flush();
-        }
-        __builtin_amdgcn_sched_barrier(0);
       }
+      write();
+      row0 += 16;
+      slice = 0;
+    }
+    return;
+  }
+  for (int sb = sb0; sb < sb1; sb += DEPTH) {
+    put_scales();
+    load_scales(sb + DEPTH);  // (past the wave's last one: fetches nothing)
+#pragma unroll
+    for (int i = 0; i < DEPTH; i++) {
+      if (sb + i < sb1) {  // uniform
+        put_sb(i);
+        __builtin_amdgcn_wave_barrier();
+        take_sb(i);
+        __builtin_amdgcn_wave_barrier();
+      }
+      load_sb(i, sb + DEPTH + i);
+      __builtin_amdgcn_sched_barrier(0);
+      if (sb + i < sb1) {
+        compute(sb + i, i);
+        if (--left == 0 || sb + i + 1 == nsb) flush();
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 
@@ -511,16 +557,7 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P) {
       tot[1] += v.y;
     }
   }
-  const int n = row0 + c;
-  if (n >= N) return;
-  const float bias = pt.bias ? pt.bias[n] : 0.f;
-#pragma unroll
-  for (int k = 0; k < (PAIRS ? 1 : 2); k++) {
-    const int m = Q4 ? 4 * (g & 1) + (g >> 1) + 2 * k : (TILES ? g : 2 * (g & 1) + (g >> 1)) + 4 * k;
-    if (m >= mt.rows) continue;
-    const int64_t orow = a.slot_ids ? (int64_t)s_rows[m] : (int64_t)kq_tile_out_row(a, mt, m);
-    pt.y[orow * N + n] = pt.bias ? tot[k] + bias : tot[k];
-  }
+  write();
 }
 
 // Tiles per workgroup and waves per tile.  A plain Linear: about one workgroup per CU, up to sixteen waves in it, none with more
@@ -578,15 +615,20 @@ static int launch_kq_rows(const KGemvArgs& a_in, hipStream_t st, unsigned grid_y
   const size_t lds = kr_lds_bytes(WT == MLLM_HIP_Q4_K, a.nsb, tw, P);
   if (lds > KR_LDS_MAX) return MLLM_HIP_E_SHAPE;
   unsigned grid = 0;
+  // Pairs: two tiles per wave where one each would be more workgroups than the chip holds at once (1024 by their registers).  A second round repeats
+  // the search for the pairs and the quantization.  Two layers of 128 experts of 2048 x 768, top-8, 8 tokens (2048 workgroups, some 1650 of them
+  // with work): 131.7 -> 128.0 us, four tiles 128.6; 4 tokens (1024): 93.2 / 95.4.
+  const int64_t single = (int64_t)grid_y * (((a.part[0].N + 15) / 16 + tw - 1) / tw);
+  const int T = ORDER == KR_PAIRS && single >= 1536 ? 2 : 1;
   for (int i = 0; i < a.nparts; i++) {
     a.wg_start[i] = (int)grid;
-    grid += (unsigned)(((a.part[i].N + 15) / 16 + tw - 1) / tw);
+    grid += (unsigned)(((a.part[i].N + 15) / 16 + tw * T - 1) / (tw * T));
   }
   a.wg_start[a.nparts] = (int)grid;
   auto kern = kq_rows_kernel<WT, XT, TH, ORDER>;
   if (lds > 64 * 1024)
     HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(kern, dim3(grid, grid_y), dim3(tw * P * 64), lds, st, a, P);
+  hipLaunchKernelGGL(kern, dim3(grid, grid_y), dim3(tw * P * 64), lds, st, a, ORDER == KR_PAIRS ? T : P);
   return (int)hipGetLastError();
 }
 template <int XT, int ORDER = KR_LINEAR>
