@@ -548,7 +548,7 @@ int mllm_hip_topk(const float* x, float* values, int32_t* indices, int64_t rows,
                   void* stream);
 /* The same two with a workspace (its size from the *_bytes call; 0 or a NULL workspace: the calls above).  Few long rows -- the
  * logits of a vocabulary -- are then cut into pieces with a workgroup each that meet in the workspace, instead of one workgroup
- * per row: two launches, three for softmax of many pieces.  Same values and indices for top-k; softmax adds a row's terms in another order. */
+ * per row: two launches, three for softmax of many pieces or in place.  Same values and indices for top-k; softmax adds a row's terms in another order. */
 size_t mllm_hip_softmax_workspace_bytes(int64_t rows, int64_t len);
 int mllm_hip_softmax_ws(const float* x, float* y, int64_t rows, int64_t len, void* workspace, void* stream);
 /* How often a workgroup looks for the sums of a row's other pieces before it adds up the row by itself (default 4096); -1: the form of

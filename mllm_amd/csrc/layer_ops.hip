@@ -1456,7 +1456,10 @@ MLLM_API int mllm_hip_softmax_ws(const float* x, float* y, int64_t rows, int64_t
   float* ws = reinterpret_cast<float*>(workspace);
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, x, y, ws, (int)len, g_exp_accurate, g_softmax_polls); };
   go(softmax_pieces_kernel<0>);
-  if (pieces <= SOFTMAX_WAIT_PIECES && pieces * rows <= SOFTMAX_WAIT && g_softmax_polls >= 0) {
+  // results over the input: a workgroup that adds up the row by itself would read what another one has written already
+  const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(y), bytes = (uintptr_t)rows * (uintptr_t)len * 4;
+  const bool apart = xa + bytes <= ya || ya + bytes <= xa;
+  if (apart && pieces <= SOFTMAX_WAIT_PIECES && pieces * rows <= SOFTMAX_WAIT && g_softmax_polls >= 0) {
     go(softmax_pieces_kernel<3>);
   } else {
     go(softmax_pieces_kernel<1>);

@@ -355,6 +355,26 @@ def test_softmax_pieces_that_wait_for_each_other(rows, ln):
     assert torch.equal(got[0].view(torch.int32), got[1].view(torch.int32)) and torch.equal(got[0].view(torch.int32), got[2].view(torch.int32))
 
 
+@pytest.mark.parametrize("polls", [4096, 0])
+@pytest.mark.parametrize("rows,ln", [(8, 151936), (2, 262144), (3, 45057)])
+def test_softmax_pieces_in_place(rows, ln, polls):
+    """results in the input's place: the bits of separate buffers (with no look but the first, the workgroups of a row would add up all of it
+    at different times)"""
+    L = _lib.lib()
+    x = (torch.randn((rows, ln), generator=torch.Generator().manual_seed(rows + ln)) * 3).cuda()
+    ws = torch.empty(L.mllm_hip_softmax_workspace_bytes(rows, ln) // 4 + 1, dtype=torch.float32, device="cuda")
+    want = ql.softmax(x)
+    announce("softmax in place", rows, ln, polls)
+    try:
+        assert L.mllm_hip_softmax_set_wait(polls) == 0
+        torch.cuda.synchronize()
+        assert L.mllm_hip_softmax_ws(x.data_ptr(), x.data_ptr(), rows, ln, ws.data_ptr(), None) == 0
+        torch.cuda.synchronize()
+    finally:
+        assert L.mllm_hip_softmax_set_wait(4096) == 0
+    assert torch.equal(x.view(torch.int32), want.view(torch.int32))
+
+
 @pytest.mark.parametrize("ln", [4100, 8193, 151_936])
 @pytest.mark.parametrize("k", [1, 50, 128])
 def test_topk_pieces_order_infinities_nan_and_zeros_as_whole_rows_do(ln, k):
