@@ -44,6 +44,26 @@ __device__ __forceinline__ int quant1(float x, float scale) {
   r = fminf(127.f, fmaxf(-128.f, r));
   return (int)r;
 }
+// Eight codes of a row.  The IEEE division of every element is eleven instructions; with inv = 1 / scale, correctly rounded once per row, a
+// product, its remainder and one correction give the correctly rounded quotient (no difference beside any half-way point of the codes for any
+// significand of the scale; the remainder is exact unless |x| is below 2^-102, whose code is 0 either way: no scale is below 2^-41).
+// |x / scale| <= 127 but for rounding, so that adding 1.5 * 2^23 rounds half to even and leaves the code in the low byte; a NaN becomes -128 as
+// above.  scale is infinite only for a row that holds an infinity: inv is 0 then, and with rem_scale 0 in its place the quotients are 0, and
+// NaN where x / scale is.
+struct RowScale {
+  float rem_scale, inv;
+};
+__device__ __forceinline__ RowScale row_scale(float scale) { return {scale < __builtin_inff() ? scale : 0.f, 1.0f / scale}; }
+__device__ __forceinline__ uint2 quant8(const float (&v)[8], RowScale s) {
+  uint32_t b[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const float q0 = v[e] * s.inv, q = fmaf(fmaf(-q0, s.rem_scale, v[e]), s.inv, q0);
+    b[e] = __float_as_uint(fmaxf(-128.f, q) + 12582912.f);
+  }
+  return make_uint2(__builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u) | __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu),
+                    __builtin_amdgcn_perm(b[5], b[4], 0x0c0c0400u) | __builtin_amdgcn_perm(b[7], b[6], 0x04000c0cu));
+}
 
 // NI > 0: the row (K <= NI * 2048, K % 8 == 0) stays in registers between the maximum and the rounding, eight elements per
 // lane and item; NI == 0: any K, the row is read twice (the second time from cache).
@@ -87,24 +107,19 @@ __global__ __launch_bounds__(256) void per_token_quant_kernel(const void* __rest
   amax = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
   amax = fmaxf(amax, 1e-10f);
   const float sc = amax / 127.0f;
+  const RowScale rs = row_scale(sc);
   if (tid == 0) scale[row] = sc;
   if (NI > 0) {
 #pragma unroll
     for (int i = 0; i < NI; i++) {
       const int k = (tid + 256 * i) * 8;
-      uint32_t pk[2] = {0, 0};
-#pragma unroll
-      for (int e = 0; e < 8; e++) pk[e >> 2] |= ((uint32_t)quant1(held[i][e], sc) & 0xffu) << (8 * (e & 3));
-      if (k < K) *reinterpret_cast<uint2*>(q + base + k) = make_uint2(pk[0], pk[1]);
+      if (k < K) *reinterpret_cast<uint2*>(q + base + k) = quant8(held[i], rs);
     }
   } else if (vec) {
     for (int k = tid * 8; k < K; k += 256 * 8) {
       float v[8];
       load_x8v<XT>(x, base + k, v);
-      uint32_t pk[2] = {0, 0};
-#pragma unroll
-      for (int e = 0; e < 8; e++) pk[e >> 2] |= ((uint32_t)quant1(v[e], sc) & 0xffu) << (8 * (e & 3));
-      *reinterpret_cast<uint2*>(q + base + k) = make_uint2(pk[0], pk[1]);
+      *reinterpret_cast<uint2*>(q + base + k) = quant8(v, rs);
     }
   } else {
     for (int k = tid; k < K; k += 256) q[base + k] = (int8_t)quant1(load_x1<XT>(x, base + k), sc);
@@ -567,9 +582,15 @@ MLLM_API int mllm_hip_w8a8_set_tuning(int tile) {
 // the K blocks, eight 1 KB blocks requested per wave before the first is multiplied (the first batch ahead of the copy of
 // the tokens' codes into LDS, which it does not depend on); v_dot4_i32_i8 sums, the two K halves of a block met by a wave
 // shuffle, the waves through LDS.  Integer sums are exact: the epilogue is the tile kernels' and so are the bits.
+//
+// XT: the tokens themselves instead of their codes: every workgroup quantizes all of them while its first weights are on their way, the waves
+// divided among the tokens, in place of a launch of its own (about 2.5 us).  Same codes, scales and results.  us, quantized in a launch before /
+// here: one token of 1536 x 2048 5.6 / 4.2, 3584 x 3584 6.1 / 4.8, 18 944 x 3584 15.1 / 13.9, 3584 x 18 944 21.6 / 15.3; two of 4096 x 4096
+// 7.1 / 5.8; four of 2048 x 6144 9.7 / 8.8.  Two workgroups per CU have to fit (64 VGPRs): with 76, 18 944 x 3584 takes 16.8.
 constexpr int W8G_MAXW = 16;
-template <int MT>
-__global__ __launch_bounds__(W8G_MAXW * 64) void w8a8_gemv_packed_kernel(W8A8Args a) {
+constexpr int W8G_CODES = -1;
+template <int MT, int XT>
+__global__ __launch_bounds__(W8G_MAXW * 64) __attribute__((amdgpu_waves_per_eu(8))) void w8a8_gemv_packed_kernel(W8A8Args a, const void* x) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int Kp = (int)w8a8_packed_k(a.K), kbs = Kp / 32;
   u32x4* sx = reinterpret_cast<u32x4*>(smem);                          // [MT][Kp / 16] the tokens' codes, zero past K and M
@@ -590,6 +611,51 @@ __global__ __launch_bounds__(W8G_MAXW * 64) void w8a8_gemv_packed_kernel(W8A8Arg
   };
   load_batch(wave);
   const int cpr = Kp / 16;  // 16-byte pieces per token
+  __shared__ float s_max[W8G_MAXW], s_scale[MT];
+  if constexpr (XT != W8G_CODES) {
+    constexpr int HELD = 1;                                   // items of eight elements that stay in registers (two: 76 VGPRs)
+    const int wpt = nwaves / MT, step = wpt * 64;             // (at least one wave per token; nwaves a multiple of MT)
+    const int m = wave / wpt, t = tid - m * step;
+    const int64_t base = (int64_t)min(m, a.M - 1) * a.K;
+    float held[HELD][8], amax = 0.f;
+    auto item = [&](int c, float (&v)[8]) { load_x8v<XT>(x, base + min(c * 8, a.K - 8), v); };  // (past the row: its tail again)
+    auto most = [&](const float (&v)[8]) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
+    };
+#pragma unroll
+    for (int i = 0; i < HELD; i++) item(t + i * step, held[i]);
+#pragma unroll
+    for (int i = 0; i < HELD; i++) most(held[i]);
+    for (int c = t + HELD * step; c * 8 < a.K; c += step) {
+      float v[8];
+      item(c, v);
+      most(v);
+    }
+    amax = fmaxf(amax, dpp_f<0xB1>(amax));
+    amax = fmaxf(amax, dpp_f<0x4E>(amax));
+    amax = fmaxf(amax, dpp_f<0x141>(amax));
+    amax = fmaxf(amax, dpp_f<0x140>(amax));
+    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+    if (lane == 0) s_max[wave] = amax;
+    __syncthreads();
+    for (int w = 0; w < wpt; w++) amax = fmaxf(amax, s_max[m * wpt + w]);
+    const float sc = fmaxf(amax, 1e-10f) / 127.0f;
+    const RowScale rs = row_scale(sc);
+    if (t == 0) s_scale[m] = sc;
+    uint2* row = reinterpret_cast<uint2*>(sx + m * cpr);
+    auto put = [&](int c, const float (&v)[8]) {
+      if (c * 8 < Kp) row[c] = c * 8 < a.K && m < a.M ? quant8(v, rs) : make_uint2(0u, 0u);
+    };
+#pragma unroll
+    for (int i = 0; i < HELD; i++) put(t + i * step, held[i]);
+    for (int c = t + HELD * step; c * 8 < Kp; c += step) {
+      float v[8];
+      item(c, v);
+      put(c, v);
+    }
+  } else
   for (int i = tid; i < MT * cpr; i += nthreads) {
     const int m = i / cpr, c = i - m * cpr;
     u32x4 v = {0u, 0u, 0u, 0u};
@@ -632,7 +698,7 @@ __global__ __launch_bounds__(W8G_MAXW * 64) void w8a8_gemv_packed_kernel(W8A8Arg
       for (int w = 0; w < nwaves; w++) v += s_part[(w * MT + m) * 32 + (i & 31)];
       if (a.acc) a.acc[(int64_t)m * a.N + n] = v;
       if (a.C) {
-        float f = (float)v * (a.ws[n] * a.xs[m]);
+        float f = (float)v * (a.ws[n] * (XT == W8G_CODES ? a.xs[m] : s_scale[m]));
         if (a.bias) f += a.bias[n];
         a.C[(int64_t)m * a.N + n] = (uint16_t)pack_bf16(f, 0.f);
       }
@@ -694,23 +760,38 @@ struct W8A8Waves {
 static int g_w8a8_decode = 1;  // 0: only the weights-from-global tiles (comparison runs and tests)
 static int g_w8a8_decode_mfma_from = 5;  // token counts from this one up take the matrix cores (at four tokens the two are even: 6144 x 2048
                                          // 5.9 us here, 6.1 there; 2560 x 9728 10.4 against 9.5; at one 5.3 / 6.1 and 8.1 / 9.4)
-// false where the dot kernel does not apply
-static bool launch_w8a8_gemv_packed(const W8A8Args& a, hipStream_t st, int* rc) {
+// false where the dot kernel does not apply; x: the tokens (a.A and a.xs are not read then), null: their codes
+static bool launch_w8a8_gemv_packed(const W8A8Args& a, hipStream_t st, int* rc, const void* x = nullptr, int x_dtype = 0) {
   if (a.M >= g_w8a8_decode_mfma_from || !g_w8a8_decode) return false;
   const int Kp = (int)w8a8_packed_k(a.K), kbs = Kp / 32;
   const int nwaves = kbs >= 32 ? W8G_MAXW : 4;
-  if (a.M > 8) return false;
+  if (a.M > (x ? 4 : 8)) return false;
+  // Three and four tokens are quantized by every workgroup only while there are few of them: four of 4096 (weights' rows 8192 / 10 240 / 12 288)
+  // 8.6 -> 7.7 us, 13.1 -> 12.7, 12.3 -> 12.7; three of 3584 x 18 944 17.2 -> 18.4.  One and two gain up to 4748 workgroups.
+  if (x && a.M > 2 && w8a8_packed_n(a.N) / 32 > 320) return false;
   const int MT = a.M <= 1 ? 1 : (a.M <= 2 ? 2 : (a.M <= 4 ? 4 : 8));
   const size_t lds = (size_t)MT * Kp + (size_t)nwaves * MT * 32 * 4;
-  if (lds > 160 * 1024) return false;
+  if (lds > (x ? 159u : 160u) * 1024) return false;
   const dim3 grid((unsigned)(w8a8_packed_n(a.N) / 32));
   auto go = [&](auto kern) {
-    if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    if (lds > 63 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return (int)hipGetLastError();
-    hipLaunchKernelGGL(kern, grid, dim3(nwaves * 64), lds, st, a);
+    hipLaunchKernelGGL(kern, grid, dim3(nwaves * 64), lds, st, a, x);
     return (int)hipGetLastError();
   };
-  *rc = MT == 1 ? go(w8a8_gemv_packed_kernel<1>) : MT == 2 ? go(w8a8_gemv_packed_kernel<2>) : MT == 4 ? go(w8a8_gemv_packed_kernel<4>) : go(w8a8_gemv_packed_kernel<8>);
+  if (!x)
+    *rc = MT == 1   ? go(w8a8_gemv_packed_kernel<1, W8G_CODES>)
+          : MT == 2 ? go(w8a8_gemv_packed_kernel<2, W8G_CODES>)
+          : MT == 4 ? go(w8a8_gemv_packed_kernel<4, W8G_CODES>)
+                    : go(w8a8_gemv_packed_kernel<8, W8G_CODES>);
+  else if (x_dtype == MLLM_HIP_F32)
+    *rc = MT == 1   ? go(w8a8_gemv_packed_kernel<1, MLLM_HIP_F32>)
+          : MT == 2 ? go(w8a8_gemv_packed_kernel<2, MLLM_HIP_F32>)
+                    : go(w8a8_gemv_packed_kernel<4, MLLM_HIP_F32>);
+  else
+    *rc = MT == 1   ? go(w8a8_gemv_packed_kernel<1, MLLM_HIP_BF16>)
+          : MT == 2 ? go(w8a8_gemv_packed_kernel<2, MLLM_HIP_BF16>)
+                    : go(w8a8_gemv_packed_kernel<4, MLLM_HIP_BF16>);
   return true;
 }
 // Which matrix-core form runs against packed weights.  Waves that split K (wk_gemm.h) from a few tokens to about the batch whose
@@ -781,12 +862,16 @@ MLLM_API int mllm_hip_w8a8_nsplit_set_tuning(int tile) {
   return 0;
 }
 
-MLLM_API int mllm_hip_per_token_quant_int8(const void* x, int x_dtype, int8_t* q, float* scale, int64_t M, int64_t K,
-                                           void* stream) {
+static int check_per_token_quant(const void* x, int x_dtype, const int8_t* q, const float* scale, int64_t M, int64_t K) {
   if (!x || !q || !scale || M <= 0 || K <= 0 || (x_dtype != MLLM_HIP_F32 && x_dtype != MLLM_HIP_BF16))
     return MLLM_HIP_E_BADARG;
   if (M > INT32_MAX || K > INT32_MAX) return MLLM_HIP_E_SHAPE;
   if (K % 8 == 0 && (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(q) % 8)) return MLLM_HIP_E_ALIGN;
+  return 0;
+}
+MLLM_API int mllm_hip_per_token_quant_int8(const void* x, int x_dtype, int8_t* q, float* scale, int64_t M, int64_t K,
+                                           void* stream) {
+  RC_RET(check_per_token_quant(x, x_dtype, q, scale, M, K));
   const int ni = (K % 8 == 0 && K >= 8 && K <= 4 * 2048) ? (K <= 2048 ? 1 : (K <= 4096 ? 2 : 4)) : 0;
 #define PTQ(XT_, NI_) \
   hipLaunchKernelGGL((per_token_quant_kernel<XT_, NI_>), dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, x, q, scale, (int)K)
@@ -845,15 +930,20 @@ MLLM_API int mllm_hip_w8a8_prepack(const int8_t* W, int64_t N, int64_t K, void* 
   return (int)hipGetLastError();
 }
 
-MLLM_API int mllm_hip_w8a8_gemm_packed(const int8_t* xq, const float* x_scale, const void* W_packed, const float* w_scale,
-                                       const float* bias, void* out_bf16, int32_t* acc_out, int64_t M, int64_t N,
-                                       int64_t K, void* stream) {
+static int check_w8a8_gemm_packed(const int8_t* xq, const float* x_scale, const void* W_packed, const float* w_scale, const void* out_bf16,
+                                  const int32_t* acc_out, int64_t M, int64_t N, int64_t K) {
   if (!xq || !W_packed || M <= 0 || N <= 0 || K <= 0 || (!out_bf16 && !acc_out)) return MLLM_HIP_E_BADARG;
   if (out_bf16 && (!x_scale || !w_scale)) return MLLM_HIP_E_BADARG;
   if (K % 16) return MLLM_HIP_E_SHAPE;
   if (M * K >= ((int64_t)1 << 32) || w8a8_packed_n(N) * w8a8_packed_k(K) >= ((int64_t)1 << 32) || M > INT32_MAX || N > INT32_MAX)
     return MLLM_HIP_E_SHAPE;
   if (reinterpret_cast<uintptr_t>(xq) % 16 || reinterpret_cast<uintptr_t>(W_packed) % 16) return MLLM_HIP_E_ALIGN;
+  return 0;
+}
+MLLM_API int mllm_hip_w8a8_gemm_packed(const int8_t* xq, const float* x_scale, const void* W_packed, const float* w_scale,
+                                       const float* bias, void* out_bf16, int32_t* acc_out, int64_t M, int64_t N,
+                                       int64_t K, void* stream) {
+  RC_RET(check_w8a8_gemm_packed(xq, x_scale, W_packed, w_scale, out_bf16, acc_out, M, N, K));
   W8A8Args a{xq, reinterpret_cast<const int8_t*>(W_packed), x_scale, w_scale, bias, (uint16_t*)out_bf16, acc_out, (int)M, (int)N, (int)K};
   int rc = 0;
   if (launch_w8a8_gemv_packed(a, (hipStream_t)stream, &rc)) return rc;  // up to four tokens
@@ -887,7 +977,14 @@ MLLM_API int mllm_hip_w8a8_linear_packed(const void* x, int x_dtype, const void*
   if (reinterpret_cast<uintptr_t>(workspace) % 16 || reinterpret_cast<uintptr_t>(W_packed) % 16) return MLLM_HIP_E_ALIGN;
   int8_t* q = reinterpret_cast<int8_t*>(workspace);
   float* xs = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + align_up((size_t)M * K, 256));
-  int rc = mllm_hip_per_token_quant_int8(x, x_dtype, q, xs, M, K, stream);
-  if (rc) return rc;
+  RC_RET(check_per_token_quant(x, x_dtype, q, xs, M, K));
+  RC_RET(check_w8a8_gemm_packed(q, xs, W_packed, w_scale, out_bf16, nullptr, M, N, K));
+  W8A8Args a{q, reinterpret_cast<const int8_t*>(W_packed), xs, w_scale, bias, (uint16_t*)out_bf16, nullptr, (int)M, (int)N, (int)K};
+  int rc = 0;
+  // (results over the tokens: they are all read first)
+  const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(out_bf16);
+  const bool apart = xa + (uintptr_t)M * K * (x_dtype == MLLM_HIP_F32 ? 4 : 2) <= ya || ya + (uintptr_t)M * N * 2 <= xa;
+  if (apart && launch_w8a8_gemv_packed(a, (hipStream_t)stream, &rc, x, x_dtype)) return rc;
+  RC_RET(mllm_hip_per_token_quant_int8(x, x_dtype, q, xs, M, K, stream));
   return mllm_hip_w8a8_gemm_packed(q, xs, W_packed, w_scale, bias, out_bf16, nullptr, M, N, K, stream);
 }

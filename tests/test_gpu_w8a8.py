@@ -260,3 +260,42 @@ def _waves_cases(shapes):
         finally:
             assert L.mllm_hip_w8a8_set_decode(1) == 0
         assert torch.equal(y.view(torch.int16), yt.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 16), (2, 33, 144), (3, 65, 1008), (4, 31, 1024), (1, 96, 8208), (2, 40, 16400), (4, 10240, 528),
+                                   (3, 10272, 272), (4, 8, 38656), (4, 8, 38672)])
+def test_linear_that_quantizes_beside_its_sums(M, N, K):
+    """one to four tokens, quantized by every workgroup (the last four sizes: the most workgroups and one more, the longest tokens that LDS
+    takes and one past them): the bits of quantizing in a launch of its own, with a row of zeros, one with a NaN, one with an infinity, one
+    of ties, a tiny one, results over the tokens, fp32 and bf16"""
+    rng = synth.rng_for(3, M * 5 + N + K)
+    W = rng.integers(-127, 128, (N, K), dtype=np.int8)
+    ws = to_dev(((rng.random(N) + 0.01) * 0.01).astype(np.float32))
+    bias = to_dev((rng.standard_normal(N) * 0.01).astype(np.float32))
+    Wp = ql.w8a8_prepack(to_dev(W))
+    base = rng.standard_normal((M, K)).astype(np.float32)
+    forms = {"plain": base.copy()}
+    for name in ("zero", "nan", "inf", "ties", "tiny"):
+        x = base.copy()
+        if name == "zero": x[0] = 0
+        if name == "nan": x[M - 1, K // 2] = np.nan
+        if name == "inf": x[0, 0], x[0, K - 1] = -np.inf, np.inf
+        if name == "ties": x[M - 1] = np.arange(K) % 255 * 0.5 - 63.5
+        if name == "tiny": x[0] *= np.float32(1e-38)
+        forms[name] = x
+    for name, x in forms.items():
+        for xd in (to_dev(x), to_dev(x).bfloat16()):
+            announce("W8A8 Linear of few tokens", M, N, K, name, str(xd.dtype))
+            q, s = ql.per_token_quant_int8(xd)
+            for b in (None, bias):
+                want = _bits(ql.w8a8_gemm_packed(q, s, Wp, N, ws, b))
+                assert np.array_equal(_bits(ql.w8a8_linear_packed(xd, Wp, N, ws, b)), want)
+            if N <= K:
+                L, over = _lib.lib(), xd.clone()
+                scratch = torch.empty(L.mllm_hip_w8a8_workspace_bytes(M, K), dtype=torch.uint8, device="cuda")
+                torch.cuda.synchronize()
+                assert L.mllm_hip_w8a8_linear_packed(over.data_ptr(), ql.F32 if xd.dtype == torch.float32 else ql.BF16, Wp.data_ptr(),
+                                                     ws.data_ptr(), None, over.data_ptr(), M, N, K, scratch.data_ptr(), None) == 0
+                torch.cuda.synchronize()
+                assert np.array_equal(over.view(torch.int16).flatten()[:M * N].cpu().numpy().view(np.uint16).reshape(M, N),
+                                      _bits(ql.w8a8_gemm_packed(q, s, Wp, N, ws, None)))
