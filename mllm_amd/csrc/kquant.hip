@@ -122,8 +122,12 @@ __global__ void kq_dequantize_kernel(int wtype, KView v, float* __restrict__ w, 
 // ---- Q8_K quantization of activations ---------------------------------------------------------------------------------------
 // 32 neighbouring lanes (half a wave) hold one super-block, eight consecutive elements per lane; both halves of the wave
 // must be active or idle as a whole.  The reference takes the element of largest magnitude WITH its sign, the first one
-// when several are equal: the magnitude goes through a plain max butterfly, the sign comes from the first lane (lowest set
-// bit of a ballot) that holds an element of that magnitude and, in it, the first such element.  Codes: the product is
+// when several are equal.  Bit patterns as signed integers have the largest positive element as their maximum, as unsigned ones the
+// negative one of largest magnitude: two butterflies give both, and only where they are equal in magnitude the first element is looked
+// for (the lowest set bit of a ballot over the lanes that hold one, and in that lane its first; a search in every block was a third of
+// the instructions).  Quotients: a reciprocal estimate and one Newton step are the correctly rounded 1 / amax for every amax in the
+// range (checked for all of its floats), -128 times that is exact, and so is its reciprocal, from amax / 128 in the estimate's place; outside the range
+// IEEE divisions.  Codes: the product is
 // rounded to fp32, then adding 1.5 * 2^23 rounds to nearest-even as rintf does and leaves the two's-complement code in the
 // low byte; the clamp to 127 is an integer min on the bits of that (positive) sum.  Outputs of a lane: its eight codes (two dwords), the sum of its
 // eight codes, the block scale.
@@ -133,34 +137,58 @@ struct Q8KItem {
   float d;
 };
 __device__ __forceinline__ Q8KItem quantize_q8k_item(const float (&v)[8], int lane) {
-  // magnitudes compare as their bit patterns: the butterfly runs on unsigned integers
-  uint32_t am = 0u;
+  int pos = (int)__float_as_uint(v[0]);
+  uint32_t neg = __float_as_uint(v[0]);
 #pragma unroll
-  for (int e = 0; e < 8; e++) am = max(am, __float_as_uint(v[e]) & 0x7fffffffu);
-  am = max(am, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)am, 0xB1, 0xf, 0xf, true));   // lane ^ 1
-  am = max(am, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)am, 0x4E, 0xf, 0xf, true));   // lane ^ 2
-  am = max(am, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)am, 0x141, 0xf, 0xf, true));  // half-row mirror
-  am = max(am, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)am, 0x140, 0xf, 0xf, true));  // row mirror
-  am = max(am, (uint32_t)__shfl_xor((int)am, 16, 64));
+  for (int e = 1; e < 8; e++) {
+    pos = max(pos, (int)__float_as_uint(v[e]));
+    neg = max(neg, __float_as_uint(v[e]));
+  }
+#define Q8K_STEP(ctrl)                                                                                    \
+  pos = max(pos, __builtin_amdgcn_update_dpp((int)0x80000000u, pos, ctrl, 0xf, 0xf, false));              \
+  neg = max(neg, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)neg, ctrl, 0xf, 0xf, false));
+  Q8K_STEP(0xB1)   // lane ^ 1
+  Q8K_STEP(0x4E)   // lane ^ 2
+  Q8K_STEP(0x141)  // half-row mirror
+  Q8K_STEP(0x140)  // row mirror
+#undef Q8K_STEP
+  const auto p16 = __builtin_amdgcn_permlane16_swap((uint32_t)pos, (uint32_t)pos, false, false);  // lane ^ 16
+  const auto n16 = __builtin_amdgcn_permlane16_swap(neg, neg, false, false);
+  pos = max((int)p16[0], (int)p16[1]);
+  neg = max(n16[0], n16[1]);
+  // (no positive element: pos is negative, and neg's magnitude the larger one; no negative one: neg == pos)
+  const uint32_t nmag = neg & 0x7fffffffu, am = max((uint32_t)max(pos, 0), nmag);
+  bool negative = neg != (uint32_t)pos ? pos < (int)nmag : pos < 0;
+  if (__any(pos == (int)nmag && neg != (uint32_t)pos)) {
+    float sel = 0.f;  // the lane's first element of that magnitude
+#pragma unroll
+    for (int e = 7; e >= 0; e--) sel = ((__float_as_uint(v[e]) & 0x7fffffffu) == am) ? v[e] : sel;
+    const bool hit = (__float_as_uint(sel) & 0x7fffffffu) == am, below = (__float_as_uint(sel) >> 31) != 0u;
+    const unsigned long long mh = __ballot(hit), mn = __ballot(hit && below);
+    const uint32_t h32 = (lane & 32) ? (uint32_t)(mh >> 32) : (uint32_t)mh;
+    const uint32_t n32 = (lane & 32) ? (uint32_t)(mn >> 32) : (uint32_t)mn;
+    negative = (n32 & (h32 & (0u - h32))) != 0u;
+  }
   const float amax = __uint_as_float(am);
-  float sel = 0.f;  // the lane's first element of that magnitude
-#pragma unroll
-  for (int e = 7; e >= 0; e--) sel = ((__float_as_uint(v[e]) & 0x7fffffffu) == am) ? v[e] : sel;
-  const bool hit = (__float_as_uint(sel) & 0x7fffffffu) == am, neg = (__float_as_uint(sel) >> 31) != 0u;
-  const unsigned long long mh = __ballot(hit), mn = __ballot(hit && neg);
-  const uint32_t h32 = (lane & 32) ? (uint32_t)(mh >> 32) : (uint32_t)mh;
-  const uint32_t n32 = (lane & 32) ? (uint32_t)(mn >> 32) : (uint32_t)mn;
-  const bool negative = (n32 & (h32 & (0u - h32))) != 0u;
   Q8KItem r{0u, 0u, 0, 0.f};
-  if (amax == 0.f) return r;
-  const float iscale = -128.f / (negative ? -amax : amax);
+  const bool usual = am - 0x1f800000u < 0x40000000u;  // 2^-64 <= amax < 2^64
+  float iscale;
+  if (__all(usual)) {
+    const float y = __builtin_amdgcn_rcpf(amax);
+    iscale = fmaf(fmaf(-amax, y, 1.f), y, y) * (negative ? 128.f : -128.f);
+    const float w = amax * (negative ? 0x1p-7f : -0x1p-7f);
+    r.d = fmaf(fmaf(-iscale, w, 1.f), w, w);
+  } else {
+    if (amax == 0.f) return r;
+    iscale = -128.f / (negative ? -amax : amax);
+    r.d = 1.f / iscale;
+  }
   uint32_t b[8];
 #pragma unroll
   for (int e = 0; e < 8; e++) b[e] = (uint32_t)min((int)__float_as_uint(iscale * v[e] + 12582912.0f), 0x4B40007F);  // bits of 1.5 * 2^23 + 127
   r.q0 = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u) | __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu);
   r.q1 = __builtin_amdgcn_perm(b[5], b[4], 0x0c0c0400u) | __builtin_amdgcn_perm(b[7], b[6], 0x04000c0cu);
   r.sum8 = __builtin_amdgcn_sdot4((int)r.q1, 0x01010101, __builtin_amdgcn_sdot4((int)r.q0, 0x01010101, 0, false), false);
-  r.d = 1.f / iscale;
   return r;
 }
 
@@ -917,10 +945,12 @@ MLLM_API int mllm_hip_linear_kq_multi_ws(int wtype, int nparts, const mllm_hip_g
     // From three rows on the matrix cores, while the rows' codes fit the LDS.  The rule looks at the number of rows and the row
     // length only: a projection gives the same bits alone and as a part of a launch.
     if (rows >= 3 && g_kq_path != 1 && kr_fits(nsb)) {
-      // Quantized once, by a launch of its own, where every workgroup would have more than three items of eight elements per
-      // thread to quantize (q+k+v, gate+up of 2560 and o of 4096 elements, own launch / in the workgroups, us: three rows 7.8 / 6.7,
-      // 11.8 / 10.1, 7.5 / 6.9; five 8.0 / 7.6, 12.0 / 11.2, 7.5 / 8.2; eight 8.1 / 8.9, 12.3 / 12.4, 7.6 / 10.0).  Same bits.
-      if (workspace && rows * nsb * 32 > 3 * kr_threads(wtype, a)) {
+      // Quantized once, by a launch of its own, where every workgroup would have more than four items of eight elements per
+      // thread to quantize, as many as a thread requests ahead of the weights (own launch / in the workgroups, us: q+k+v of 2560 elements, three
+      // rows 8.2 / 7.0, five 8.2 / 7.4, eight (four items) 8.2 / 8.3; gate+up 12.0 / 10.2, 11.9 / 10.7, 11.9 / 11.6; o of 4096, four rows 7.5 / 7.1, five
+      // (five items) 7.6 / 7.8, eight 7.6 / 9.3; 2048 x 6144 Q6_K at four 9.8 / 9.2, at five (five items) 10.1 / 10.4; 1024 x 1024 at three 6.3 / 4.8,
+      // at eight 6.5 / 5.5).  Same bits.
+      if (workspace && rows * nsb * 32 > 4 * kr_threads(wtype, a)) {
         hipLaunchKernelGGL(kr_image_kernel, dim3((unsigned)((nsb * 32 + 255) / 256), (unsigned)rows), dim3(256), 0, st, xg, x_dtype,
                            reinterpret_cast<unsigned char*>(workspace), nsb, rows);
         a.x = workspace;

@@ -16,11 +16,12 @@
 // super-block, then d * dx) with the sums of a super-block split over two (Q4_K) or four lanes.
 //
 // What bounds it (time stamps written by the kernel, gate + up of 9728 x 2560 at five rows, us after the start): the codes back
-// 2.2, all waves past the barrier 3.8, the last wave's loop done 7.9, end 8.4 -- the weights, 28 MB, flow from 1.5 on.  Kept
+// 2.2, all waves past the barrier 3.8, the last wave's loop done 7.9, end 8.4 -- the weights, 28 MB, flow from 1.5 on; with a quantizer of
+// twice the instructions, whose third item per thread came back behind the weights: 0.4 more.  Kept
 // short by spreading K over the waves of a workgroup (one tile's waves meet in LDS, not in memory), by requests for activations ahead
 // of every wave's weights, and by loading whole lines: with weights loaded in the operand's own order (sixteen rows per instruction) the
 // L1's tags were the bottleneck and the last wave passed the barrier at 10.7.  Five rows, us with the quantization (before: K slices as
-// workgroups that met in memory, or scale tables in LDS): q+k+v 9.9 -> 7.5, o 9.6 -> 7.5, gate+up 14.7 -> 11.2, down (Q6_K, 2560 x
+// workgroups that met in memory, or scale tables in LDS): q+k+v 9.9 -> 7.4, o 9.6 -> 7.6, gate+up 14.7 -> 10.7, down (Q6_K, 2560 x
 // 9728) 17.3 -> 12.6; 20 MB of the last take 4 us at the copy rate of the card.
 // K is cut into slices of KR_SPS super-blocks whatever the launch shape; a slice is summed in one chain and the slices are added in
 // order, by one wave or over several: the bits depend on the weight type and K alone.
@@ -245,7 +246,7 @@ __global__ __launch_bounds__(1024) void kq_rows_kernel(KGemvArgs a, int P_or_T) 
     constexpr int XL = XT == KQ_IMAGE ? MLLM_HIP_F32 : XT;
     const int ipr = nsb * 32, nitems = mt.rows * ipr;
     const float inv = 1.0f / (float)ipr;
-    constexpr int U = 2;  // items a thread requests ahead of the weights
+    constexpr int U = 4;  // items a thread requests ahead of the weights: as many as there are in a plain Linear
     const bool prod = XT == MLLM_HIP_F32 && a.x2 != nullptr;  // uniform
     auto fetch = [&](int it, float (&v)[8], float (&f)[8]) {
       const int m = (int)(((float)it + 0.5f) * inv), i = it - m * ipr;  // it / ipr: far from rounding trouble
@@ -603,8 +604,8 @@ static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y, bool quant
   while (tw > 1 && kr_lds_bytes(q4, a.nsb, tw, P) > KR_LDS_MAX) tw--;
   return KrShape{tw, P};
 }
-static int kr_threads(int wtype, const KGemvArgs& a) {
-  const KrShape s = kr_shape(wtype == MLLM_HIP_Q4_K, a, 1);
+static int kr_threads(int wtype, const KGemvArgs& a) {  // of a workgroup that quantizes
+  const KrShape s = kr_shape(wtype == MLLM_HIP_Q4_K, a, 1, true);
   return s.tiles * s.waves * 64;
 }
 template <int WT, int XT, int TH, int ORDER>

@@ -44,6 +44,27 @@ def test_q8_K_quantization_bit_exact(dtype):
     assert np.array_equal(bs.cpu().numpy(), obs)
 
 
+def test_q8_K_quantization_signs_and_magnitudes():
+    """super-blocks of every magnitude (also past the range of the reciprocal's estimate), of one sign, of zeros of both
+    signs, with the largest magnitude in two places of either sign: in one lane's eight elements, in two lanes, in the two halves of sixteen
+    lanes, next to a block that has no such pair"""
+    rng = synth.rng_for(7, 2)
+    x = rng.standard_normal((24, 512)).astype(np.float32)
+    # from 128 / max_float = 3.8e-37 on: below it the scale 128 / amax is infinite and the reference's codes are no numbers
+    x[:16] *= np.float32(10.0) ** np.array([-36, -34, -30, -25, -20, -19.2, -19, -10, -1, 5, 10, 19, 19.3, 20, 30, 37.5], np.float32)[:, None]
+    x[16] = -np.abs(x[16])
+    x[17] = np.abs(x[17])
+    x[18, ::2], x[18, 1::2] = 0.0, -0.0
+    for r, (a, b) in zip(range(19, 24), ((3, 5), (8, 250), (127, 128), (0, 255), (40, 41))):
+        x[r, a], x[r, b] = 7.5, -7.5
+        x[r, 256 + b], x[r, 256 + a] = (7.5, -7.5) if r % 2 else (9.5, -3.0)
+    want = orc.quantize_rows_q8_K(x)
+    announce("q8_K signs and magnitudes")
+    for got, w in zip(ql.quantize_q8_K(to_dev(x)), want):
+        got = got.cpu().numpy()
+        assert np.array_equal(got.view(np.uint32) if got.dtype == np.float32 else got, w.view(np.uint32) if w.dtype == np.float32 else w)
+
+
 @pytest.mark.parametrize("wtype", [2, 3])
 def test_prepack_and_dequantize_bit_exact(wtype):
     rng = synth.rng_for(7, 10 + wtype)
