@@ -688,8 +688,8 @@ __global__ __launch_bounds__(256) void matmul_dots_kernel(MMArgs a, int g_log2, 
       v += dpp_f<0x4E>(v);
       if (g > 4) v += dpp_f<0x141>(v);
       if (g > 8) v += dpp_f<0x140>(v);
-      if (g > 16) v += __shfl_xor(v, 16, 64);
-      if (g > 32) v += __shfl_xor(v, 32, 64);
+      if (g > 16) v = sum16(v);
+      if (g > 32) v = sum32(v);
       if (sub == 0) s_out[m][u * groups + grp] = v;
     }
   __syncthreads();

@@ -384,7 +384,7 @@ __global__ __launch_bounds__(MODE == 1 ? 512 : 256) void qgemm_tile_kernel(QGemm
         amax = fmaxf(amax, dpp_f<0x4E>(amax));
         amax = fmaxf(amax, dpp_f<0x141>(amax));
         amax = fmaxf(amax, dpp_f<0x140>(amax));
-        amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+        amax = max16(amax);
         const float d = amax / 127.f;
         const float idv = (amax != 0.f) ? 127.f / amax : 0.f;
         int qi = (int)rintf(h * idv);
@@ -918,7 +918,7 @@ __device__ __forceinline__ void qg_tile(const QG2Args& a, const int e, const int
           h[q] = silu_f(acc[0][j][i][q]) * acc[NW - 1][j][i][q];
           amax = fmaxf(amax, fabsf(h[q]));
         }
-        amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+        amax = max32(amax);
         const float d = amax / 127.f;
         const float idv = (amax != 0.f) ? 127.f / amax : 0.f;
         uint16_t bits = f32_to_f16bits(d);
@@ -1379,7 +1379,7 @@ __device__ __forceinline__ void qx_tile(const QXArgs& a, const int e, const int 
           h[q] = silu_f(acc[0][j][i][q]) * acc[NW - 1][j][i][q];
           amax = fmaxf(amax, fabsf(h[q]));
         }
-        amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+        amax = max32(amax);
         const float d = amax / 127.f;
         const float idv = (amax != 0.f) ? 127.f / amax : 0.f;
         uint16_t bits = f32_to_f16bits(d);
@@ -1393,8 +1393,8 @@ __device__ __forceinline__ void qx_tile(const QXArgs& a, const int e, const int 
           if (q & 2) sb += qv[q];
           else sa += qv[q];
         }
-        sa += __shfl_xor(sa, 32, 64);
-        sb += __shfl_xor(sb, 32, 64);
+        sa = sum32(sa);
+        sb = sum32(sb);
         if (r < rows && blk < nblk) {
           uint16_t* hrow = a.hq + (int64_t)(row0 + r) * a.N;
 #pragma unroll
@@ -1664,8 +1664,8 @@ __device__ __forceinline__ void qx_tile16(const QXArgs& a, const int e, const in
         hv[q] = silu_f(acc[0][j][q >> 2][q & 3]) * acc[NW - 1][j][q >> 2][q & 3];
         amax = fmaxf(amax, fabsf(hv[q]));
       }
-      amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-      amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+      amax = max16(amax);
+      amax = max32(amax);
       const float d = amax / 127.f;
       const float idv = (amax != 0.f) ? 127.f / amax : 0.f;
       uint16_t bits = f32_to_f16bits(d);
@@ -1679,10 +1679,10 @@ __device__ __forceinline__ void qx_tile16(const QXArgs& a, const int e, const in
         if (q & 2) sb += qv[q];
         else sa += qv[q];
       }
-      sa += __shfl_xor(sa, 16, 64);
-      sa += __shfl_xor(sa, 32, 64);
-      sb += __shfl_xor(sb, 16, 64);
-      sb += __shfl_xor(sb, 32, 64);
+      sa = sum16(sa);
+      sa = sum32(sa);
+      sb = sum16(sb);
+      sb = sum32(sb);
       if (c16 < rows && blk < nblk) {
         uint16_t* hrow = a.hq + (int64_t)(row0 + c16) * a.N;
 #pragma unroll

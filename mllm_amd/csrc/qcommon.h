@@ -83,6 +83,21 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
+// A value and the one 16 (32) lanes away, in one swap of rows: a shuffle goes through LDS, 0.1 us at the end of a kernel of two.
+__device__ __forceinline__ u32x2 lanes16(uint32_t v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return u32x2{r[0], r[1]};
+}
+__device__ __forceinline__ u32x2 lanes32(uint32_t v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return u32x2{r[0], r[1]};
+}
+__device__ __forceinline__ float sum16(float v) { const u32x2 r = lanes16(__float_as_uint(v)); return __uint_as_float(r.x) + __uint_as_float(r.y); }
+__device__ __forceinline__ float sum32(float v) { const u32x2 r = lanes32(__float_as_uint(v)); return __uint_as_float(r.x) + __uint_as_float(r.y); }
+__device__ __forceinline__ float max16(float v) { const u32x2 r = lanes16(__float_as_uint(v)); return fmaxf(__uint_as_float(r.x), __uint_as_float(r.y)); }
+__device__ __forceinline__ float max32(float v) { const u32x2 r = lanes32(__float_as_uint(v)); return fmaxf(__uint_as_float(r.x), __uint_as_float(r.y)); }
+__device__ __forceinline__ int sum16(int v) { const u32x2 r = lanes16((uint32_t)v); return (int)(r.x + r.y); }
+__device__ __forceinline__ int sum32(int v) { const u32x2 r = lanes32((uint32_t)v); return (int)(r.x + r.y); }
 // Sum over aligned groups of G consecutive lanes; every lane of the group ends up with the total.
 template <int G>
 __device__ __forceinline__ float group_sum(float v) {
@@ -90,8 +105,8 @@ __device__ __forceinline__ float group_sum(float v) {
   if (G >= 4) v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
   if (G >= 8) v += dpp_f<0x141>(v);  // row_half_mirror
   if (G >= 16) v += dpp_f<0x140>(v); // row_mirror
-  if (G >= 32) v += __shfl_xor(v, 16, 64);
-  if (G >= 64) v += __shfl_xor(v, 32, 64);
+  if (G >= 32) v = sum16(v);
+  if (G >= 64) v = sum32(v);
   return v;
 }
 
@@ -172,8 +187,8 @@ __device__ __forceinline__ void quad_quantize_to_image(const float (&v)[8], cons
   for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
   amax = fmaxf(amax, dpp_f<0xB1>(amax));
   amax = fmaxf(amax, dpp_f<0x4E>(amax));
-  const float d = amax / 127.f;
-  const float idv = (amax != 0.f) ? 127.f / amax : 0.f;
+  float d, idv;
+  q8_scales(amax, d, idv);
   const uint32_t pk[2] = {q8_pack4(&v[0], idv), q8_pack4(&v[4], idv)};
   int sum = __builtin_amdgcn_sdot4((int)pk[0], 0x01010101, 0, false);
   sum = __builtin_amdgcn_sdot4((int)pk[1], 0x01010101, sum, false);

@@ -100,8 +100,8 @@ __global__ __launch_bounds__(256) void per_token_quant_kernel(const void* __rest
   amax = fmaxf(amax, dpp_f<0x4E>(amax));
   amax = fmaxf(amax, dpp_f<0x141>(amax));
   amax = fmaxf(amax, dpp_f<0x140>(amax));
-  amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-  amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+  amax = max16(amax);
+  amax = max32(amax);
   if ((tid & 63) == 0) s_max[tid >> 6] = amax;
   __syncthreads();
   amax = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
@@ -636,8 +636,8 @@ __global__ __launch_bounds__(W8G_MAXW * 64) __attribute__((amdgpu_waves_per_eu(8
     amax = fmaxf(amax, dpp_f<0x4E>(amax));
     amax = fmaxf(amax, dpp_f<0x141>(amax));
     amax = fmaxf(amax, dpp_f<0x140>(amax));
-    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+    amax = max16(amax);
+    amax = max32(amax);
     if (lane == 0) s_max[wave] = amax;
     __syncthreads();
     for (int w = 0; w < wpt; w++) amax = fmaxf(amax, s_max[m * wpt + w]);
@@ -687,7 +687,7 @@ __global__ __launch_bounds__(W8G_MAXW * 64) __attribute__((amdgpu_waves_per_eu(8
   }
 #pragma unroll
   for (int m = 0; m < MT; m++) {
-    acc[m] += __shfl_xor(acc[m], 32, 64);
+    acc[m] = sum32(acc[m]);
     if (h == 0) s_part[(wave * MT + m) * 32 + r] = acc[m];
   }
   __syncthreads();

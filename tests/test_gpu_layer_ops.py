@@ -148,6 +148,22 @@ def test_silu_mul_image(M, D):
     _check_image(img3, y3.cpu().numpy(), M, D, False)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_silu_of_few_elements_as_of_many(dtype):
+    """two elements per thread (up to 327 680 items of eight) and eight: the same bits, with infinities, NaN and large values of both signs"""
+    g = torch.Generator().manual_seed(5)
+    a, b = ((torch.randn((327_690, 8), generator=g) * 4) for _ in range(2))
+    a[:10] = torch.tensor([float("inf"), -float("inf"), float("nan"), 90.0, -90.0, 3e38, -0.0, 1e-40])
+    b[5:15, ::2] = float("inf")
+    a, b = a.to(dtype).cuda(), b.to(dtype).cuda()
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    announce("silu of few elements", dtype)
+    one, two = ql.silu(a), ql.silu_mul(a, b)
+    for rows in (1, 3, 32, 127, 4097, 327_680, 327_681):
+        assert torch.equal(ql.silu(a[:rows]).view(bits), one[:rows].view(bits)), rows
+        assert torch.equal(ql.silu_mul(a[:rows], b[:rows]).view(bits), two[:rows].view(bits)), rows
+
+
 @pytest.mark.parametrize("wtype", [0, 1])
 @pytest.mark.parametrize("M", [1, 2, 3, 8])
 def test_gemv_fused_equals_the_operators_it_replaces(wtype, M):
