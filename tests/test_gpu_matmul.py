@@ -242,6 +242,15 @@ def test_matmul_from_bf16_parts_outside_their_range(M, N, K, ta, tb, side):
         b = torch.from_numpy(rng.integers(-2, 3, (N, K)).astype(np.float32))
         a[M // 2] *= scale
         assert torch.equal(_split(side, *order(a, b), ta, tb), torch.matmul(a.double(), b.double().t().contiguous()).float())
+    for few in (False, True):  # elements below the smallest part, everywhere or one of an operand of zeros: the sums of the parts are zero
+        def pair(small, other):
+            x = torch.from_numpy(rng.integers(1, 1 << 9, (small, K)).astype(np.float32)) * 2.0 ** -143
+            if few:
+                x *= torch.arange(small * K).reshape(small, K) == (small - 1) * K + K // 2
+            return x, torch.from_numpy(rng.integers(-2, 3, (other, K)).astype(np.float32)) * 2.0 ** 20
+        for a, b in (pair(M, N), pair(N, M)[::-1]):
+            want = torch.matmul(a.double(), b.double().t().contiguous()).float()
+            assert torch.equal(_split(-1, *order(a, b), ta, tb), want) and torch.equal(_split(side, *order(a, b), ta, tb), want)
     a = torch.full((M, K), 3.3961775e38)  # below the largest float, an infinity in bf16
     b = torch.zeros((N, K))
     b[:, 0] = 1.
