@@ -50,6 +50,7 @@ struct Owned {  // a new reference
   ~Owned() { Py_DECREF(o); }
   Owned(const Owned&) = delete;
 };
+int64_t number(PyObject* o) { return integer(Owned(PyNumber_Long(o)).o); }  // int(o): flags that are no whole numbers (numpy's booleans)
 int64_t attribute(PyObject* o, PyObject* name) { return integer(Owned(PyObject_GetAttr(o, name)).o); }
 void* stream() {  // the current stream of the current device
   Owned device(PyObject_CallNoArgs(g_device));
@@ -160,7 +161,7 @@ PyObject* topk(Args a) {
   require(x.is_cuda() && x.is_contiguous() && x.scalar_type() == at::kFloat);
   need_rank(x, 1);
   const int64_t n = x.size(-1), k = integer(a[1]);
-  const int largest = (int)integer(a[2]), sorted = (int)integer(a[3]);
+  const int largest = (int)number(a[2]), sorted = (int)number(a[3]);
   at::DimVector shape(x.sizes().begin(), x.sizes().end());
   shape.back() = k;
   at::Tensor v = empty(shape, at::kFloat), i = empty(shape, at::kInt), work;

@@ -65,4 +65,5 @@ def test_calls_use_the_callers_outputs_and_stream():
         ql.topk(p, 257)
     with pytest.raises(TypeError):
         ql.linear_q_gemv(w, x.half())
+    assert torch.equal(ql.topk(p, 7, np.bool_(True), np.bool_(True))[1], ids)
     assert np.isfinite(y.cpu().numpy()).all()
