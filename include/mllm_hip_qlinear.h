@@ -574,7 +574,7 @@ int mllm_hip_moe_gate_set_form(int two_launches);
  * replaces: CPUMatMulOp::forward  mllm/backends/cpu/ops/MatMulOp.cpp:19-90 (shapes :30-44, default kernel choice :47-61)
  * C[b][M][N] = op(A[b]) * op(B[b]), op(X) = X or X^T; A[b] is [M][K] ([K][M] when transposed), B[b] is [K][N] ([N][K]
  * when transposed).  dtype MLLM_HIP_F32, MLLM_HIP_BF16 or MLLM_HIP_F16 for all three tensors; products are exact (larger fp32
- * calls: to within 2^-26 of a product) and summed in fp32, 16-bit results are rounded once to nearest even.  Batch entry b starts stride_x * b elements after
+ * calls: to within 2^-34 of a product) and summed in fp32, 16-bit results are rounded once to nearest even.  Batch entry b starts stride_x * b elements after
  * entry 0 (stride_b = 0 multiplies every A[b] by the same B); the whole batch is one launch.
  * ------------------------------------------------------------------------------------------------------- */
 int mllm_hip_matmul_batched(const void* A, const void* B, void* C, int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,

@@ -2,7 +2,7 @@
 // x values and the MoE gate logits of the reference run through it, mllm/backends/cpu/ops/MatMulOp.cpp:27-61 with the batch
 // loop of mllm/backends/cpu/kernels/common/ggml/matmul.cpp / mllm_blas).  Not a quantized path.
 //   fp32 operands   v_mfma_f32_32x32x2f32: exact fp32 products, fp32 accumulation (the CPU's arithmetic in another order); larger products from
-//                   three bf16 parts per operand, to within 2^-26 of a product (matmul_split_kernel)
+//                   three bf16 parts per operand, to within 2^-34 of a product (matmul_split_kernel)
 //   bf16 / fp16     v_mfma_f32_32x32x16_{bf16,f16}: exact products, fp32 accumulation, one rounding of the result
 // One launch covers the whole batch (a stride of 0 broadcasts an operand).
 //
@@ -305,14 +305,15 @@ __global__ __launch_bounds__(256, (TM * TN == 4 && DT != MLLM_HIP_F32) ? 4 : 1) 
 }
 
 // fp32 operands on the bf16 matrix instructions, which do sixteen times the products per clock.  A float is the sum of three bf16 numbers,
-// exactly: x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1.  Six of the nine products are multiplied, the smallest first; the three left out
-// are below 2^-26 of a product.  An instruction adds sixteen of them before it rounds, so the result is nearer to 64 bits than that of the fp32
-// instructions, which add two (8 x 3108 x 777 x 128: 1.63e-7 of the norm against 2.03e-7, x 128 x 777: 4.3e-7 against 5.0e-7).
-// Bound by the matrix pipe at the clock it holds under this load, by LDS reads (nine 16-byte reads per twelve instructions; a wave tile of 32 x
-// 64) and by the splitting (six vector instructions per element), which share the issue slots: about 27 us per 128 k of 8 x 3072 x 768, where the
-// matrix instructions alone take 17 and the fp32 ones 45.  K steps of sixteen in two LDS buffers, one barrier each; two (large tile) to five
-// workgroups per CU.  One LDS buffer with steps of 32, operands read a step ahead, and tiles of 64 x 128 with four waves were no faster.
-//   8 x 3108 x 777 x 128 (scores): 65 -> 46 us, x 128 x 777 (values): 66 -> 43; 8 x 4096 x 1024 x 128: 93 -> 62
+// exactly: x0 = bf16(x), x1 = bf16(x - x0), x2 = x - x0 - x1.  Eight of the nine products are multiplied; x2 y2 is below 2^-34 of a product.
+// An instruction cuts off what it adds to a larger sum where the fp32 ones round, so the products but x0 y0 have a sum of their own, the smallest first, which
+// is added at the end: a single product is within 0.506 ulp (fp32 instructions 0.5; without x1 y2 and x2 y1 and in one sum 1.43), the results are nearer to
+// 64 bits than theirs (8 x 3108 x 777 x 128: 0.65e-7 of the norm against 2.03e-7, x 128 x 777: 1.6e-7 against 5.0e-7).
+// Bound by the matrix pipe at the clock it holds under this load, by LDS reads (nine 16-byte reads per sixteen instructions; a wave tile of 32 x
+// 64) and by the splitting (six vector instructions per element), which share the issue slots; the matrix instructions alone take 23 us per 128 k of
+// 8 x 3072 x 768, the fp32 ones 45.  K steps of sixteen in two LDS buffers, one barrier each; one (large tile, two accumulators) to four workgroups
+// per CU.  One LDS buffer with steps of 32, operands read a step ahead, and tiles of 64 x 128 with four waves were no faster.
+//   8 x 3108 x 777 x 128 (scores): 61 -> 55 us, x 128 x 777 (values): 61.5 -> 48; 8 x 4096 x 1024 x 128: 85 -> 80
 struct MMParts {
   uint32_t p[3];
 };
@@ -395,7 +396,7 @@ struct MMSplitTile {
 };
 
 template <bool TA, bool TB, int WM, int WN, int TM, int TN>
-__global__ __launch_bounds__(WM * WN * 64, 4) void matmul_split_kernel(MMArgs a, int tiles, int tilesM, uint32_t inv_tiles, uint32_t inv_tilesM) {
+__global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_split_kernel(MMArgs a, int tiles, int tilesM, uint32_t inv_tiles, uint32_t inv_tilesM) {
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN, NT = WM * WN * 64;
   typedef MMSplitTile<BM, !TA, NT> SplitA;
   typedef MMSplitTile<BN, TB, NT> SplitB;
@@ -415,17 +416,19 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void matmul_split_kernel(MMArgs a,
   float* C = reinterpret_cast<float*>(a.C) + z * a.sC;
 
   mm_f32x16 acc[TM][TN];
-  auto clear = [&]() {
+  auto clear = [&](mm_f32x16 (&x)[TM][TN]) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+        for (int v = 0; v < 16; ++v) x[i][j][v] = 0.f;
   };
-  clear();
+  clear(acc);
   float most = 0.f;
   {
+    mm_f32x16 low[TM][TN];  // the products but x0 y0
+    clear(low);
     SplitA ta;
     SplitB tb;
     ta.start(A, m0, a.M, a.K);
@@ -462,13 +465,13 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void matmul_split_kernel(MMArgs a,
       store(1 - d, skip);
       load(1 - d, step + 3);
       __builtin_amdgcn_sched_barrier(0);
-      auto mma = [&](int u, int w) {
+      auto mul = [&](mm_f32x16 (&to)[TM][TN], int u, int w) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][u], fb[j][w], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < TN; ++j) to[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][u], fb[j][w], to[i][j], 0, 0, 0);
       };
-      mma(2, 0), mma(0, 2), mma(1, 1), mma(1, 0), mma(0, 1), mma(0, 0);
+      mul(low, 2, 1), mul(acc, 0, 0), mul(low, 1, 2), mul(low, 2, 0), mul(low, 0, 2), mul(low, 1, 1), mul(low, 1, 0), mul(low, 0, 1);
       __syncthreads();
     };
     int step = 0;
@@ -478,6 +481,12 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void matmul_split_kernel(MMArgs a,
       work(0, step, skip(step + 1));
       if (step + 1 < steps) work(1, step + 1, skip(step + 2));
     }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] += low[i][j][v];
   }
   // An infinity or a NaN in an operand, and a float that rounds to an infinity in bf16, leave a NaN here.  Parts below 2^-133 vanish: at most
   // 2^-103 of a product of operands below 2^30.  A tile with a NaN, an infinity, a larger operand or a sum between 0 and 2^-66 is multiplied
@@ -515,7 +524,7 @@ __global__ __launch_bounds__(WM * WN * 64, 4) void matmul_split_kernel(MMArgs a,
     float *sA = reinterpret_cast<float*>(smem), *sB = sA + TileA::SIZE;
     TileA ta;
     TileB tb;
-    clear();
+    clear(acc);
     ta.start(A, m0, a.M, a.K);
     tb.start(B, n0, a.N, a.K);
 #pragma unroll 1

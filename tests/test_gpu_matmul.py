@@ -224,6 +224,25 @@ def test_matmul_fp32_from_bf16_parts(batch, M, N, K, ta, tb, side):
 
 @pytest.mark.parametrize("side", [64, 128])
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("K", [16, 61, 160])
+def test_matmul_from_bf16_parts_single_products(K, ta, tb, side):
+    """diag(d) B: every result is one product of two 24-bit significands, rounded once by fp32 instructions.  The parts but x0 y0 are at most 2^-7 of
+    it; their seven instructions lose less than an ulp of that each, 2^-30 of the product or 2^-6 of its ulp: within 0.5 + 7 / 64 ulp"""
+    rng = synth.rng_for(6, 8500 + K)
+    some = lambda *s: ((rng.integers(1 << 23, 1 << 24, s) * rng.choice([-1, 1], s)) * 2.0 ** rng.integers(-33, -13, s)).astype(np.float32)  # noqa: E731
+    hard = np.float32(1 + 2.0 ** -8 - 2.0 ** -16 + 2.0 ** -17 - 2.0 ** -23)  # its square loses 2^-24 without x1 y2 and x2 y1
+    d, b = some(K), some(K, 150)
+    d[0], b[0] = hard, hard * 2.0 ** rng.integers(-9, 9, 150).astype(np.float32)
+    a = np.diag(d)
+    announce("matmul from parts of single products %d ta=%d tb=%d side %d" % (K, ta, tb, side))
+    c = _split(side, torch.from_numpy(a), torch.from_numpy(np.ascontiguousarray(b.T) if tb else b), ta, tb).numpy()
+    want = d[:, None].astype(np.float64) * b
+    ulps = np.abs(c - want) / np.exp2(np.floor(np.log2(np.abs(want))) - 23)
+    assert ulps.max() <= 0.5 + 7 / 64, ulps.max()
+
+
+@pytest.mark.parametrize("side", [64, 128])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("M,N,K", [(70, 130, 37), (129, 66, 64), (5, 133, 100)])
 def test_matmul_from_bf16_parts_outside_their_range(M, N, K, ta, tb, side):
     """infinities, NaN, floats that round to an infinity in bf16, sums that overflow, elements whose parts are below the smallest bf16 number and
