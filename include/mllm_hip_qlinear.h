@@ -576,6 +576,9 @@ int mllm_hip_moe_gate_set_form(int two_launches);
  * when transposed).  dtype MLLM_HIP_F32, MLLM_HIP_BF16 or MLLM_HIP_F16 for all three tensors; products are exact (larger fp32
  * calls: to within 2^-34 of a product) and summed in fp32, 16-bit results are rounded once to nearest even.  Batch entry b starts stride_x * b elements after
  * entry 0 (stride_b = 0 multiplies every A[b] by the same B); the whole batch is one launch.
+ * A result depends on its row of A, its column of B and the call's sizes, on nothing else in the operands.  On the sizes: the kernels for up to four rows,
+ * fp32 instructions and bf16 parts (by batch, M, N and K, mllm_hip_matmul_split_side) add in different orders, so the last bits of an fp32 row can
+ * differ between a prompt taken whole and in chunks, or alone and in a batch.
  * ------------------------------------------------------------------------------------------------------- */
 int mllm_hip_matmul_batched(const void* A, const void* B, void* C, int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
                             int64_t stride_a, int64_t stride_b, int64_t stride_c, int transpose_a, int transpose_b,

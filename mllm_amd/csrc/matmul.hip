@@ -425,7 +425,8 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
         for (int v = 0; v < 16; ++v) x[i][j][v] = 0.f;
   };
   clear(acc);
-  float most = 0.f;
+  static_assert(SplitA::NV == 1 && SplitB::NV == 1, "a thread loads of one row of either operand");
+  float mostA = 0.f, mostB = 0.f;  // of those rows
   {
     mm_f32x16 low[TM][TN];  // the products but x0 y0
     clear(low);
@@ -440,8 +441,8 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
       tb.load(d, k);
     };
     auto store = [&](int d, int skip) {  // d = step % 2
-      ta.store(smem + d * BUF, d, skip, most);
-      tb.store(smem + d * BUF + SplitA::SIZE, d, skip, most);
+      ta.store(smem + d * BUF, d, skip, mostA);
+      tb.store(smem + d * BUF + SplitA::SIZE, d, skip, mostB);
     };
     const unsigned char *pa = smem + (wm * 32 * TM + r) * SplitA::LD + 16 * h, *pb = smem + SplitA::SIZE + (wn * 32 * TN + r) * SplitB::LD + 16 * h;
     auto skip = [&](int step) { return max(step * 16 + 16 - a.K, 0); };
@@ -489,12 +490,14 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
         for (int v = 0; v < 16; ++v) acc[i][j][v] += low[i][j][v];
   }
   // An infinity or a NaN in an operand, and a float that rounds to an infinity in bf16, leave a NaN here.  Parts below 2^-133 vanish: at most
-  // 2^-103 of a product of operands below 2^30.  A tile with a NaN, an infinity, a larger operand or a sum between 0 and 2^-66 is multiplied
-  // again with fp32 instructions; so is a tile with a sum of zero and an element whose parts may be below the normal bf16 numbers (below 2^-103: the
-  // sum may be zero because they vanished).  Masked or padded tiles have zeros too: they take one more look at their operands.
+  // 2^-103 of a product of operands below 2^30.  Results that are no numbers, of rows or columns with a larger operand, or between 0 and 2^-66 are
+  // multiplied again with fp32 instructions; so are results of zero whose row or column has an element with parts that may be below the normal bf16
+  // numbers (below 2^-103: the sum may be zero because they vanished).  Every result is judged by its own row and column: what else its tile holds
+  // does not change its bits.
   constexpr uint32_t LOW = (127u - 66u) << 24;
+  auto twice = [](float f) { return (__float_as_uint(f) << 1) - 1u; };  // the magnitude's bits, less one: a zero is ~0u, 0 < |f| < 2^-66 below LOW - 1
   float check = 0.f;
-  uint32_t least = ~0u, greatest = 0;  // of twice the magnitude's bits less one: a sum of zero is ~0u, 0 < |sum| < 2^-66 below LOW - 1
+  uint32_t least = ~0u, greatest = 0;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -502,59 +505,86 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         check = fmaf(acc[i][j][v], 0.f, check);
-        const uint32_t u = (__float_as_uint(acc[i][j][v]) << 1) - 1u;
-        least = min(least, u), greatest = max(greatest, u);
+        least = min(least, twice(acc[i][j][v])), greatest = max(greatest, twice(acc[i][j][v]));
       }
-  const bool bad = check != 0.f || most >= 0x1p30f || least < LOW - 1u;
-  bool again = __syncthreads_or(bad || greatest == ~0u);  // (one vote: with two the attention of 777 tokens takes 118.3 to 120 us, 117.8 with one)
-  if (again) {
-    bool small = bad;
-    auto look = [&](const float* X, bool contig, int row0, int rows, int side) {
-      const int nr = min(side, rows - row0), outer = contig ? nr : a.K, inner = contig ? a.K : nr;
-      for (int o = wave; o < outer; o += WM * WN) {
-        const float* p = X + (contig ? (int64_t)(row0 + o) * a.K : (int64_t)o * rows + row0);
-        for (int i = lane; i < inner; i += 64) small |= (__float_as_uint(p[i]) << 1) - 1u < (24u << 24) - 1u;  // 0 < |x| < 2^-103
+  const bool look = __syncthreads_or(check != 0.f || fmaxf(mostA, mostB) >= 0x1p30f || least < LOW - 1u || greatest == ~0u);
+  {  // 32x32 accumulator layout as in mm_store; rows past the end lie past the end of the buffer
+    const __amdgpu_buffer_rsrc_t rC = __builtin_amdgcn_make_buffer_rsrc(C, 0, (uint32_t)a.M * (uint32_t)a.N * 4u, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = n0 + wn * 32 * TN + j * 32 + r;
+      if (n < a.N) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const uint32_t at = ((uint32_t)(m0 + wm * 32 * TM + i * 32 + 4 * h) * (uint32_t)a.N + n) * 4u;
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][v]), rC, at + (uint32_t)(8 * (v / 4) + v % 4) * (uint32_t)a.N * 4u, 0, 0);
+        }
       }
-    };
-    look(A, !TA, m0, a.M, BM);
-    look(B, TB, n0, a.N, BN);
-    again = __syncthreads_or(small);
-  }
-  if (again) {
-    float *sA = reinterpret_cast<float*>(smem), *sB = sA + TileA::SIZE;
-    TileA ta;
-    TileB tb;
-    clear(acc);
-    ta.start(A, m0, a.M, a.K);
-    tb.start(B, n0, a.N, a.K);
-#pragma unroll 1
-    for (int k = 0; k < a.K; k += 32) {
-      ta.load(A, m0, k, a.M, a.K);
-      tb.load(B, n0, k, a.N, a.K);
-      __syncthreads();
-      ta.store(sA);
-      tb.store(sB);
-      __syncthreads();
-      mm_f32_step<TileA, TileB, TM, TN>(sA, sB, wm, wn, r, h, acc);
     }
-    mm_store<MLLM_HIP_F32, TM, TN, BM, BN>(a, C, m0, n0, wm, wn, r, h, acc);
-    return;
   }
-  // 32x32 accumulator layout as in mm_store; rows past the end lie past the end of the buffer
-  const __amdgpu_buffer_rsrc_t rC = __builtin_amdgcn_make_buffer_rsrc(C, 0, (uint32_t)a.M * (uint32_t)a.N * 4u, 0x00020000);
+  if (!look) return;
+
+  enum : uint32_t { BIG = 1, SMALL = 2 };
+  uint32_t* flags = reinterpret_cast<uint32_t*>(smem);  // of the tile's rows of A, then of its columns of B
+  for (int i = threadIdx.x; i < BM + BN; i += NT) flags[i] = 0u;
+  __syncthreads();
+  if (mostA >= 0x1p30f) atomicOr(&flags[SplitA::row(0)], BIG);
+  if (mostB >= 0x1p30f) atomicOr(&flags[BM + SplitB::row(0)], BIG);
+  auto small = [&](uint32_t* flags, const float* X, bool contig, int row0, int rows, int side) {
+    const int nr = min(side, rows - row0), outer = contig ? nr : a.K, inner = contig ? a.K : nr;
+    for (int o = wave; o < outer; o += WM * WN) {
+      const float* p = X + (contig ? (int64_t)(row0 + o) * a.K : (int64_t)o * rows + row0);
+      for (int i = lane; i < inner; i += 64)
+        if (twice(p[i]) < (24u << 24) - 1u) atomicOr(&flags[contig ? o : i], SMALL);  // 0 < |x| < 2^-103
+    }
+  };
+  small(flags, A, !TA, m0, a.M, BM);
+  small(flags + BM, B, TB, n0, a.N, BN);
+  __syncthreads();
+  static_assert(TM * TN <= 2, "a bit per result of a lane");
+  uint32_t wanted = 0;
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int n = n0 + wn * 32 * TN + j * 32 + r;
-    if (n < a.N) {
+    const uint32_t column = flags[BM + wn * 32 * TN + j * 32 + r];
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const uint32_t at = ((uint32_t)(m0 + wm * 32 * TM + i * 32 + 4 * h) * (uint32_t)a.N + n) * 4u;
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int v = 0; v < 16; ++v)
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][j][v]), rC, at + (uint32_t)(8 * (v / 4) + v % 4) * (uint32_t)a.N * 4u, 0, 0);
+      for (int v = 0; v < 16; ++v) {
+        const uint32_t both = column | flags[wm * 32 * TM + i * 32 + 8 * (v / 4) + 4 * h + v % 4];
+        const float f = acc[i][j][v];
+        const bool w = !(fabsf(f) < __builtin_inff()) || (both & BIG) || twice(f) < LOW - 1u || (f == 0.f && (both & SMALL));
+        wanted |= (uint32_t)w << (16 * (i * TN + j) + v);
       }
-    }
   }
+  if (!__syncthreads_or(wanted != 0u)) return;
+
+  float *sA = reinterpret_cast<float*>(smem), *sB = sA + TileA::SIZE;
+  TileA ta;
+  TileB tb;
+  clear(acc);
+  ta.start(A, m0, a.M, a.K);
+  tb.start(B, n0, a.N, a.K);
+#pragma unroll 1
+  for (int k = 0; k < a.K; k += 32) {
+    ta.load(A, m0, k, a.M, a.K);
+    tb.load(B, n0, k, a.N, a.K);
+    __syncthreads();
+    ta.store(sA);
+    tb.store(sB);
+    __syncthreads();
+    mm_f32_step<TileA, TileB, TM, TN>(sA, sB, wm, wn, r, h, acc);
+  }
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int m = m0 + wm * 32 * TM + i * 32 + 8 * (v / 4) + 4 * h + v % 4, n = n0 + wn * 32 * TN + j * 32 + r;
+        if ((wanted >> (16 * (i * TN + j) + v) & 1) && m < a.M && n < a.N) C[(int64_t)m * a.N + n] = acc[i][j][v];
+      }
 }
 
 // Up to four rows of A [M][K] against B [K][N] (attention probabilities x values of a decode token): a GEMV per row, bound by

@@ -676,5 +676,6 @@ def quantize_q8_K(x):
 
 def matmul(a, b, transpose_a=False, transpose_b=False, out=None):
     """C[..., M, N] = op(a) @ op(b) for fp32 / bf16 / fp16 tensors of rank >= 2, the whole batch in one launch; b may be a
-    single matrix shared by every batch entry.  mllm/backends/cpu/ops/MatMulOp.cpp:19-90."""
+    single matrix shared by every batch entry.  Last bits of fp32 results depend on the call's sizes (which instructions it
+    takes), never on other rows or columns.  mllm/backends/cpu/ops/MatMulOp.cpp:19-90."""
     return _calls().matmul(a, b, transpose_a, transpose_b, out)

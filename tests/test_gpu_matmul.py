@@ -246,7 +246,7 @@ def test_matmul_from_bf16_parts_single_products(K, ta, tb, side):
 @pytest.mark.parametrize("M,N,K", [(70, 130, 37), (129, 66, 64), (5, 133, 100)])
 def test_matmul_from_bf16_parts_outside_their_range(M, N, K, ta, tb, side):
     """infinities, NaN, floats that round to an infinity in bf16, sums that overflow, elements whose parts are below the smallest bf16 number and
-    operands of any size: the tile takes fp32 instructions, and no other row or column changes"""
+    operands of any size: fp32 instructions multiply them again, and no other row or column is infinite or NaN"""
     rng = synth.rng_for(6, 9000 + M + N + K)
     a = torch.from_numpy(rng.integers(1, 9, (M, K)).astype(np.float32))
     b = torch.from_numpy(rng.integers(1, 9, (N, K)).astype(np.float32))
@@ -274,6 +274,37 @@ def test_matmul_from_bf16_parts_outside_their_range(M, N, K, ta, tb, side):
     b = torch.zeros((N, K))
     b[:, 0] = 1.
     assert torch.equal(_split(side, *order(a, b), ta, tb), a[:, :1].expand(M, N))
+
+
+@pytest.mark.parametrize("side", [64, 128])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(70, 130, 37), (129, 66, 64), (200, 133, 100)])
+def test_matmul_from_bf16_parts_depends_on_one_row_and_one_column(M, N, K, ta, tb, side):
+    """random floats with a row of A, then a column of B, out of the parts' range or of zeros: its results are those of the fp32 instructions,
+    every other result keeps its bits"""
+    g = torch.Generator().manual_seed(M + N + K)
+    a, b = torch.randn((M, K), generator=g), torch.randn((N, K), generator=g)
+    run = lambda side, a, b: _split(side, a.t().contiguous() if ta else a, b if tb else b.t().contiguous(), ta, tb)  # noqa: E731
+    announce("matmul from parts beside rows out of their range %s ta=%d tb=%d side %d" % ((M, N, K), ta, tb, side))
+    plain = run(side, a, b)
+    bits = lambda t: t.contiguous().view(torch.int32)  # noqa: E731
+    for value in (float("nan"), float("inf"), 2. ** 31, 2. ** 100, 2. ** -80, 2. ** -140, 0., "one NaN", "one infinity", "one large", "zeros and one small"):
+        for rows, of_b in ((M, False), (N, True)):
+            x, at = (b if of_b else a).clone(), rows - 2
+            if isinstance(value, float):
+                x[at] *= value
+            else:
+                if value == "zeros and one small":
+                    x[at] = 0.
+                x[at, K // 2] = {"one NaN": float("nan"), "one infinity": -float("inf"), "one large": 2. ** 40, "zeros and one small": 2. ** -141}[value]
+            got, want = (run(s, *((a, x) if of_b else (x, b))) for s in (side, -1))
+            if of_b:
+                got, want, rest = got.t(), want.t(), plain.t()
+            else:
+                rest = plain
+            keep = torch.arange(rows) != at
+            assert torch.equal(bits(got[keep]), bits(rest[keep])), (value, of_b)
+            assert torch.equal(got[at].nan_to_num(nan=7.), want[at].nan_to_num(nan=7.)), (value, of_b)
 
 
 def test_matmul_of_attention_sizes_takes_the_bf16_parts():
