@@ -491,8 +491,8 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
   }
   // An infinity or a NaN in an operand, and a float that rounds to an infinity in bf16, leave a NaN here.  Parts below 2^-133 vanish: at most
   // 2^-103 of a product of operands below 2^30.  Results that are no numbers, of rows or columns with a larger operand, or between 0 and 2^-66 are
-  // multiplied again with fp32 instructions; so are results of zero whose row or column has an element with parts that may be below the normal bf16
-  // numbers (below 2^-103: the sum may be zero because they vanished).  Every result is judged by its own row and column: what else its tile holds
+  // multiplied again with fp32 instructions; so are results of zero of a row and a column that are not all zeros, of which one has an element with parts that may be
+  // below the normal bf16 numbers (below 2^-103: the sum may be zero because they vanished).  Every result is judged by its own row and column: what else its tile holds
   // does not change its bits.
   constexpr uint32_t LOW = (127u - 66u) << 24;
   auto twice = [](float f) { return (__float_as_uint(f) << 1) - 1u; };  // the magnitude's bits, less one: a zero is ~0u, 0 < |f| < 2^-66 below LOW - 1
@@ -526,23 +526,54 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
   }
   if (!look) return;
 
-  enum : uint32_t { BIG = 1, SMALL = 2 };
+  enum : uint32_t { BIG = 1, SMALL = 2, NONZERO = 4 };
   uint32_t* flags = reinterpret_cast<uint32_t*>(smem);  // of the tile's rows of A, then of its columns of B
   for (int i = threadIdx.x; i < BM + BN; i += NT) flags[i] = 0u;
   __syncthreads();
-  if (mostA >= 0x1p30f) atomicOr(&flags[SplitA::row(0)], BIG);
-  if (mostB >= 0x1p30f) atomicOr(&flags[BM + SplitB::row(0)], BIG);
-  auto small = [&](uint32_t* flags, const float* X, bool contig, int row0, int rows, int side) {
-    const int nr = min(side, rows - row0), outer = contig ? nr : a.K, inner = contig ? a.K : nr;
-    for (int o = wave; o < outer; o += WM * WN) {
-      const float* p = X + (contig ? (int64_t)(row0 + o) * a.K : (int64_t)o * rows + row0);
-      for (int i = lane; i < inner; i += 64)
-        if (twice(p[i]) < (24u << 24) - 1u) atomicOr(&flags[contig ? o : i], SMALL);  // 0 < |x| < 2^-103
-    }
-  };
-  small(flags, A, !TA, m0, a.M, BM);
-  small(flags + BM, B, TB, n0, a.N, BN);
+  const int rowA = SplitA::row(0), rowB = BM + SplitB::row(0);  // the rows that this thread loads of
+  if (mostA > 0.f) atomicOr(&flags[rowA], mostA >= 0x1p30f ? BIG | NONZERO : NONZERO);
+  if (mostB > 0.f) atomicOr(&flags[rowB], mostB >= 0x1p30f ? BIG | NONZERO : NONZERO);
   __syncthreads();
+  // Small elements are looked for only where a result is zero though neither its row nor its column is: padded rows, caches not yet filled and
+  // zero columns cost nothing, the look where zeros come of other elements 17 % of a tile (8 x 3108 x 128 x 777: dense 49 us, a zero row, column or
+  // unfilled rows 49 to 52, other zeros in each tile 58).  Keeping the smallest element as well would cost the staging 1.5 instructions per element.
+  bool open = false;
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const uint32_t column = flags[BM + wn * 32 * TN + j * 32 + r];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) open |= acc[i][j][v] == 0.f && (column & flags[wm * 32 * TM + i * 32 + 8 * (v / 4) + 4 * h + v % 4] & NONZERO);
+  }
+  if (__syncthreads_or(open)) {
+    SplitA ta;
+    SplitB tb;
+    ta.start(A, m0, a.M, a.K);
+    tb.start(B, n0, a.N, a.K);
+    constexpr int U = 4;  // K steps on their way at once
+    uint32_t leastA = ~0u, leastB = ~0u;
+    auto low = [&](uint32_t& l, u32x4 x) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) l = min(l, (x[e] << 1) - 1u);
+    };
+#pragma unroll 1
+    for (int k = 0; k < a.K; k += 16 * U) {
+      u32x4 xa[U], xb[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {  // (past the end: the last 16 k again)
+        ta.load(0, min(k + 16 * u, a.K - 16)), xa[u] = ta.v[0][0];
+        tb.load(0, min(k + 16 * u, a.K - 16)), xb[u] = tb.v[0][0];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < U; u++) low(leastA, xa[u]), low(leastB, xb[u]);
+    }
+    constexpr uint32_t PARTS = (24u << 24) - 1u;  // |x| < 2^-103
+    if (leastA < PARTS) atomicOr(&flags[rowA], SMALL);
+    if (leastB < PARTS) atomicOr(&flags[rowB], SMALL);
+    __syncthreads();
+  }
   static_assert(TM * TN <= 2, "a bit per result of a lane");
   uint32_t wanted = 0;
 #pragma unroll
@@ -552,9 +583,9 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const uint32_t both = column | flags[wm * 32 * TM + i * 32 + 8 * (v / 4) + 4 * h + v % 4];
+        const uint32_t row = flags[wm * 32 * TM + i * 32 + 8 * (v / 4) + 4 * h + v % 4], either = row | column;
         const float f = acc[i][j][v];
-        const bool w = !(fabsf(f) < __builtin_inff()) || (both & BIG) || twice(f) < LOW - 1u || (f == 0.f && (both & SMALL));
+        const bool w = !(fabsf(f) < __builtin_inff()) || (either & BIG) || twice(f) < LOW - 1u || (f == 0.f && (row & column & NONZERO) && (either & SMALL));
         wanted |= (uint32_t)w << (16 * (i * TN + j) + v);
       }
   }
