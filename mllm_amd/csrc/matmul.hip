@@ -591,21 +591,28 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
   }
   if (!__syncthreads_or(wanted != 0u)) return;
 
+  // The next K step is loaded during this one's instructions, as in matmul_kernel; waves of which nothing is wanted multiply nothing.  8 x 3108 x 128 x
+  // 777: one NaN row 81 us, a large or tiny row in every tile 102 (dense 49, fp32 instructions 61.5); a step loaded when it is needed: 109, 110.
   float *sA = reinterpret_cast<float*>(smem), *sB = sA + TileA::SIZE;
   TileA ta;
   TileB tb;
   clear(acc);
   ta.start(A, m0, a.M, a.K);
   tb.start(B, n0, a.N, a.K);
+  ta.load(A, m0, 0, a.M, a.K);
+  tb.load(B, n0, 0, a.N, a.K);
+  const bool mine = __any(wanted != 0u);
 #pragma unroll 1
   for (int k = 0; k < a.K; k += 32) {
-    ta.load(A, m0, k, a.M, a.K);
-    tb.load(B, n0, k, a.N, a.K);
-    __syncthreads();
     ta.store(sA);
     tb.store(sB);
     __syncthreads();
-    mm_f32_step<TileA, TileB, TM, TN>(sA, sB, wm, wn, r, h, acc);
+    if (k + 32 < a.K) {
+      ta.load(A, m0, k + 32, a.M, a.K);
+      tb.load(B, n0, k + 32, a.N, a.K);
+    }
+    if (mine) mm_f32_step<TileA, TileB, TM, TN>(sA, sB, wm, wn, r, h, acc);
+    __syncthreads();
   }
 #pragma unroll
   for (int j = 0; j < TN; ++j)
