@@ -860,11 +860,13 @@ static bool mm_narrow(const MMArgs& a) {
   return DT == MLLM_HIP_F32 && !TA && TB && a.M <= 32 && (int64_t)((a.N + 63) / 64) * a.batch >= 800;
 }
 
-// fp32: the side of the tile of matmul_split_kernel, 0 where fp32 instructions are as fast or needed.  Costs in us fitted to 400 random shapes in
-// all orders (1 to 64 x 5 to 4096 x 5 to 4096 x 16 to 2048); of the launches above 12 us the choice takes 0.85 of the fp32 instructions' time on
-// average and at most 1.09 (10 x 3266 x 3871 x 64: 255 / 278).  Up to one small tile per CU a step's latency is the same either way (3 x 80 x
-// 126 x 1670: 44.9 us with fp32 instructions, 39.2 small, 67.1 large; 2 x 168 x 238 x 1975: 45.3, 48.7, 81.9), and the shortest launches are
-// bound by their start.  Few rows x [N][K] over many tiles stay with the form for those.
+// fp32: the side of the tile of matmul_split_kernel, 0 where fp32 instructions are as fast or needed.  Costs in us of the three forms fitted to 4800
+// random shapes in all orders (1 to 64 x 5 to 4096 x 5 to 4096 x 16 to 2048, a third of them attention of 64 to 1024 tokens): the choice takes 0.945 of the
+// fp32 instructions' time on average over all of them, the best of the three 0.930; 9 shapes are more than 5 % slower.  A gain of less than 4 % in the costs stays with
+// fp32 instructions, and so do K below 32 (59 x 397 x 1677 x 24: 45.4 us, 57 with parts) and up to one small tile per CU, where the order decides
+// and tiles do not (1 x 1701 x 245 x 1964 with A [K][M] 74 / 56, 8 x 20 x 168 x 1765 42 / 50).  With costs of the parts alone every launch
+// above a floor took them, and the large tile too early: 8 x 504 x 504 x 128 9.4 / 12.2 us, 8 x 1308 x 327 x 64 11.2 / 16.1.  Few rows x
+// [N][K] over many tiles stay with the form for those.
 static int mm_split_side(const MMArgs& a, bool nt) {
   constexpr int64_t LIMIT = (int64_t)1 << 32;  // byte offsets in 32 bits
   if (a.K < 16 || (int64_t)a.M * a.K * 4 >= LIMIT || (int64_t)a.N * a.K * 4 >= LIMIT || ((int64_t)a.M + 128) * a.N * 4 >= LIMIT) return 0;
@@ -872,9 +874,11 @@ static int mm_split_side(const MMArgs& a, bool nt) {
   if (g_matmul_tile) return 0;
   if (nt && mm_narrow<MLLM_HIP_F32, false, true>(a)) return 0;
   const double K = a.K, t64 = (double)((a.M + 63) / 64) * ((a.N + 63) / 64) * a.batch / 256, t128 = (double)((a.M + 127) / 128) * ((a.N + 127) / 128) * a.batch / 256;
-  if (t64 <= 1. || t64 * K < 150.) return 0;
-  const double us64 = 5.1 + 0.46 * t64 + K * (0.0194 + 0.0144 * (0.2 * std::ceil(t64) + 0.8 * t64 - 1.));
-  const double us128 = 3.0 + 2.6 * std::max(t128, 1.) + 0.037 * K + (0.5 + 0.0435 * K) * (0.85 * std::ceil(t128) + 0.15 * std::max(t128, 1.) - 1.);
+  if (t64 <= 1. || a.K < 32) return 0;
+  const double us64 = 3.6 + 0.80 * t64 + K * (0.0225 + 0.0152 * (0.49 * std::ceil(t64) + 0.51 * t64 - 1.));
+  const double us128 = 1.6 + 4.66 * std::max(t128, 1.) + K * (0.0502 + 0.0579 * (std::ceil(t128) - 1.));
+  const double f32 = 3.06 + 0.869 * t64 + K * (0.024 + 0.020 * (0.93 * std::ceil(t64) + 0.07 * t64 - 1.));
+  if (std::min(us64, us128) > 0.96 * f32) return 0;
   return us128 < us64 ? 128 : 64;
 }
 

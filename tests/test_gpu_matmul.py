@@ -307,6 +307,17 @@ def test_matmul_from_bf16_parts_depends_on_one_row_and_one_column(M, N, K, ta, t
             assert torch.equal(got[at].nan_to_num(nan=7.), want[at].nan_to_num(nan=7.)), (value, of_b)
 
 
+def test_matmul_takes_the_bf16_parts_where_they_are_faster():
+    """host-only query of the rule.  us, fp32 instructions / parts on small / large tiles: 8 x 504 x 504 x 128 9.4 / 9.5 / 12.2, 8 x 1308 x 327 x 64 11.2 /
+    10.8 / 16.1, 4 x 2060 x 515 x 64 12.1 / 12.4 / 16.2, 59 x 397 x 1677 x 24 45.4 / 57.0 / 63.5, 8 x 1024 x 128 x 1024 26 / 30 / 53"""
+    side = _lib.lib().mllm_hip_matmul_split_side
+    for shape in ((8, 504, 504, 128), (8, 1308, 327, 64), (4, 2060, 515, 64)):
+        assert side(*shape, 0, 0) != 128
+    for shape in ((59, 397, 1677, 24), (8, 1024, 128, 1024), (8, 500, 500, 128), (1, 5, 4096, 2048), (8, 64, 64, 2048)):
+        assert side(*shape, 0, 0) == 0
+    assert side(8, 4096, 1024, 128, 0, 1) == 64 and side(1, 2048, 2048, 2048, 0, 0) == 128
+
+
 def _graph_time(call, n=20):
     """median of seven replays of n calls, in us per call"""
     call()
