@@ -332,34 +332,27 @@ __device__ __forceinline__ MMParts mm_split(float a, float b) {  // two neighbou
 template <int ROWS, bool CONTIG_K, int NT>
 struct MMSplitTile {
   static constexpr int LD = 3 * 32 + 16, SIZE = ROWS * LD;  // bytes
-  static constexpr int NV = ROWS * 4 / NT;                  // vectors of four k per thread: of as many rows, or [K][rows] of one row
-  static_assert(ROWS * 4 % NT == 0 && NT % ROWS == 0, "tile must split evenly over the threads");
+  static_assert(ROWS * 4 == NT && ROWS >= 64, "four k of one row per thread");
   __amdgpu_buffer_rsrc_t rsrc;
-  uint32_t off[CONTIG_K ? NV : 1], ld;
-  u32x4 v[2][NV];  // two K steps in flight
-  static __device__ __forceinline__ int row(int c) { return CONTIG_K ? (int)threadIdx.x / 4 + c * (NT / 4) : (int)threadIdx.x % ROWS; }
-  static __device__ __forceinline__ int kfirst(int c) {  // of the step's 16
-    return CONTIG_K ? (int)threadIdx.x % 4 * 4 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / ROWS) * 4 * NV + 4 * c;  // (the same in a wave: ROWS >= 64)
+  uint32_t off, ld;
+  u32x4 v[2];  // two K steps in flight
+  static __device__ __forceinline__ int row() { return CONTIG_K ? (int)threadIdx.x / 4 : (int)threadIdx.x % ROWS; }
+  static __device__ __forceinline__ int kfirst() {  // of the step's 16
+    return CONTIG_K ? (int)threadIdx.x % 4 * 4 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / ROWS) * 4;  // (the same in a wave)
   }
   __device__ __forceinline__ void start(const float* X, int row0, int rows, int K) {
     rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(X), 0, (uint32_t)rows * (uint32_t)K * 4u, 0x00020000);
-#pragma unroll
-    for (int c = 0; c < (CONTIG_K ? NV : 1); c++) {
-      const uint32_t r = (uint32_t)min(row0 + row(c), rows - 1);
-      off[c] = CONTIG_K ? (r * (uint32_t)K + kfirst(c)) * 4u : r * 4u;
-    }
+    const uint32_t r = (uint32_t)min(row0 + row(), rows - 1);
+    off = CONTIG_K ? (r * (uint32_t)K + kfirst()) * 4u : r * 4u;
     ld = (uint32_t)rows * 4u;
   }
   __device__ __forceinline__ void load(int d, int k) {  // k: the first of the step's 16
+    if constexpr (CONTIG_K) {
+      v[d] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, k * 4, 0);
+    } else {
+      const uint32_t at = (uint32_t)(k + kfirst()) * ld;
 #pragma unroll
-    for (int c = 0; c < NV; c++) {
-      if constexpr (CONTIG_K) {
-        v[d][c] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[c], k * 4, 0);
-      } else {
-        const uint32_t at = (uint32_t)(k + kfirst(c)) * ld;
-#pragma unroll
-        for (int e = 0; e < 4; e++) v[d][c][e] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, off[0], at + e * ld, 0);
-      }
+      for (int e = 0; e < 4; e++) v[d][e] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, off, at + e * ld, 0);
     }
   }
   // skip: how many k of the step are not its own
@@ -367,31 +360,16 @@ struct MMSplitTile {
     if (__builtin_expect(skip != 0, 0)) {
       asm volatile("");  // (a branch: selects in every step cost more)
 #pragma unroll
-      for (int c = 0; c < NV; c++)
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-          if (kfirst(c) + e < skip) v[d][c][e] = 0u;
+      for (int e = 0; e < 4; e++)
+        if (kfirst() + e < skip) v[d][e] = 0u;
     }
-    MMParts a[2 * NV];
+    const f32x4 x = __builtin_bit_cast(f32x4, v[d]);
+    most = fmaxf(fmaxf(most, fabsf(x[0])), fabsf(x[1]));
+    most = fmaxf(fmaxf(most, fabsf(x[2])), fabsf(x[3]));
+    const MMParts a = mm_split(x[0], x[1]), b = mm_split(x[2], x[3]);
+    unsigned char* at = s + row() * LD + kfirst() * 2;
 #pragma unroll
-    for (int c = 0; c < NV; c++) {
-      const f32x4 x = __builtin_bit_cast(f32x4, v[d][c]);
-      most = fmaxf(fmaxf(most, fabsf(x[0])), fabsf(x[1]));
-      most = fmaxf(fmaxf(most, fabsf(x[2])), fabsf(x[3]));
-      a[2 * c] = mm_split(x[0], x[1]), a[2 * c + 1] = mm_split(x[2], x[3]);
-    }
-    if constexpr (!CONTIG_K && NV == 2) {
-      unsigned char* at = s + row(0) * LD + kfirst(0) * 2;
-#pragma unroll
-      for (int i = 0; i < 3; i++) *reinterpret_cast<u32x4*>(at + 32 * i) = u32x4{a[0].p[i], a[1].p[i], a[2].p[i], a[3].p[i]};
-    } else {
-#pragma unroll
-      for (int c = 0; c < NV; c++) {
-        unsigned char* at = s + row(c) * LD + kfirst(c) * 2;
-#pragma unroll
-        for (int i = 0; i < 3; i++) *reinterpret_cast<u32x2*>(at + 32 * i) = u32x2{a[2 * c].p[i], a[2 * c + 1].p[i]};
-      }
-    }
+    for (int i = 0; i < 3; i++) *reinterpret_cast<u32x2*>(at + 32 * i) = u32x2{a.p[i], b.p[i]};
   }
 };
 
@@ -425,8 +403,7 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
         for (int v = 0; v < 16; ++v) x[i][j][v] = 0.f;
   };
   clear(acc);
-  static_assert(SplitA::NV == 1 && SplitB::NV == 1, "a thread loads of one row of either operand");
-  float mostA = 0.f, mostB = 0.f;  // of those rows
+  float mostA = 0.f, mostB = 0.f;  // of the rows that this thread loads of
   {
     mm_f32x16 low[TM][TN];  // the products but x0 y0
     clear(low);
@@ -530,7 +507,7 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
   uint32_t* flags = reinterpret_cast<uint32_t*>(smem);  // of the tile's rows of A, then of its columns of B
   for (int i = threadIdx.x; i < BM + BN; i += NT) flags[i] = 0u;
   __syncthreads();
-  const int rowA = SplitA::row(0), rowB = BM + SplitB::row(0);  // the rows that this thread loads of
+  const int rowA = SplitA::row(), rowB = BM + SplitB::row();
   if (mostA > 0.f) atomicOr(&flags[rowA], mostA >= 0x1p30f ? BIG | NONZERO : NONZERO);
   if (mostB > 0.f) atomicOr(&flags[rowB], mostB >= 0x1p30f ? BIG | NONZERO : NONZERO);
   __syncthreads();
@@ -562,8 +539,8 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
       u32x4 xa[U], xb[U];
 #pragma unroll
       for (int u = 0; u < U; u++) {  // (past the end: the last 16 k again)
-        ta.load(0, min(k + 16 * u, a.K - 16)), xa[u] = ta.v[0][0];
-        tb.load(0, min(k + 16 * u, a.K - 16)), xb[u] = tb.v[0][0];
+        ta.load(0, min(k + 16 * u, a.K - 16)), xa[u] = ta.v[0];
+        tb.load(0, min(k + 16 * u, a.K - 16)), xb[u] = tb.v[0];
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
