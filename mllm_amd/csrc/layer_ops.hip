@@ -1096,15 +1096,16 @@ __device__ __forceinline__ void gate_request(const GateArgs& a, int e, int c0, G
 #pragma unroll
   for (int u = 0; u < GATE_CB; u++) p.v[u] = wr[min(c0 + 64 * u, last)];
 }
-// logits of experts e0 + wave, e0 + wave + nwaves, ... < e1 for the ntok tokens in s_x; out[t * ostride + e].  first: the first of the
+// logits of experts e0 + wave, e0 + wave + nwaves, ... < e1 for the ntok tokens in s_x; out[t * ostride + e].  AHEAD: first holds the first of the
 // pieces, requested before x was staged
+template <bool AHEAD>
 __device__ __forceinline__ void gate_logits(const GateArgs& a, const float* s_x, int ntok, int e0, int e1, int wave, int nwaves, int lane,
                                             const GatePieces& first, float* out, size_t ostride) {
   constexpr int CB = GATE_CB;
   const int nc = a.H >> 2;
   GatePieces w = first;
   f32x4(&wv)[CB] = w.v;
-  bool have = true;
+  bool have = AHEAD;
   for (int e = e0 + wave; e < e1; e += nwaves) {
     float acc[GATE_TOK] = {0.f, 0.f, 0.f, 0.f};
     for (int c0 = lane; c0 < nc; c0 += 64 * CB) {
@@ -1272,7 +1273,7 @@ __device__ __forceinline__ void gate_finish(const GateArgs& a, const float* logi
   gate_select(a, lg, tok, tv, ti, lane);
 }
 // everything in one launch: a workgroup per four tokens (callers that pass no scores buffer)
-template <int XT>
+template <int XT, bool AHEAD>
 __global__ __launch_bounds__(GATE_WAVES * 64) void moe_gate_kernel(GateArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   float* s_x = reinterpret_cast<float*>(smem);     // [GATE_TOK][H]
@@ -1283,10 +1284,10 @@ __global__ __launch_bounds__(GATE_WAVES * 64) void moe_gate_kernel(GateArgs a) {
   const int64_t tok0 = (int64_t)blockIdx.x * GATE_TOK;
   const int ntok = (int)min((int64_t)GATE_TOK, a.M - tok0);  // uniform
   GatePieces first;
-  gate_request(a, wave, lane, first);
+  if (AHEAD) gate_request(a, wave, lane, first);
   gate_stage_x<XT>(a, tok0, ntok, s_x, tid, GATE_WAVES * 64);
   __syncthreads();
-  gate_logits(a, s_x, ntok, 0, a.E, wave, GATE_WAVES, lane, first, s_logit, (size_t)a.E);
+  gate_logits<AHEAD>(a, s_x, ntok, 0, a.E, wave, GATE_WAVES, lane, first, s_logit, (size_t)a.E);
   __syncthreads();
   if (wave >= ntok) return;
   gate_finish(a, s_logit + wave * a.E, s_logit + wave * a.E, tok0 + wave, s_tv + wave * a.k, s_ti + wave * a.k, lane);
@@ -1295,7 +1296,7 @@ __global__ __launch_bounds__(GATE_WAVES * 64) void moe_gate_kernel(GateArgs a) {
 // workgroup per four tokens leaves the chip to one CU (a decode token: 1 MB of gate weights through one workgroup), so the
 // experts are spread over the grid's y -- epg experts and as many waves per workgroup -- and a second, small launch
 // finishes each token.  Same logits, same selection.
-template <int XT>
+template <int XT, bool AHEAD>
 __global__ __launch_bounds__(GATE_WAVES * 64) void moe_gate_logits_kernel(GateArgs a, int epg) {
   extern __shared__ __align__(16) unsigned char smem[];
   float* s_x = reinterpret_cast<float*>(smem);  // [GATE_TOK][H]
@@ -1304,10 +1305,10 @@ __global__ __launch_bounds__(GATE_WAVES * 64) void moe_gate_logits_kernel(GateAr
   const int ntok = (int)min((int64_t)GATE_TOK, a.M - tok0);  // uniform
   const int e0 = (int)blockIdx.y * epg;
   GatePieces first;
-  gate_request(a, e0 + wave, lane, first);
+  if (AHEAD) gate_request(a, e0 + wave, lane, first);
   gate_stage_x<XT>(a, tok0, ntok, s_x, tid, nthreads);
   __syncthreads();
-  gate_logits(a, s_x, ntok, e0, min(a.E, e0 + epg), wave, nthreads >> 6, lane, first, a.scores + tok0 * a.E, (size_t)a.E);
+  gate_logits<AHEAD>(a, s_x, ntok, e0, min(a.E, e0 + epg), wave, nthreads >> 6, lane, first, a.scores + tok0 * a.E, (size_t)a.E);
 }
 __global__ __launch_bounds__(GATE_TOK * 64) void moe_gate_select_kernel(GateArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -1566,7 +1567,13 @@ MLLM_API int mllm_hip_moe_gate(const void* x, int x_dtype, const float* gate_wei
       hipLaunchKernelGGL(kern, dim3(grid, (unsigned)((E + epg - 1) / epg)), dim3(64 * epg), lds1, st, a, epg);
       return (int)hipGetLastError();
     };
-    RC_RET(x_dtype == MLLM_HIP_F32 ? go(moe_gate_logits_kernel<MLLM_HIP_F32>) : go(moe_gate_logits_kernel<MLLM_HIP_BF16>));
+    // weights ahead of x: 78 registers, so that a CU holds one workgroup of sixteen waves instead of two.  us without / with: 512 tokens, 128 experts of 2048
+    // 16.2 / 20.9, 2048 tokens 45 / 65, 512 tokens, 300 experts 50 / 62; in one round 7.4 / 7.4 (256 tokens, 64 of 1024).  Workgroups of four waves do not
+    // mind: 8 tokens 8.4 / 8.3, 192 13.2 / 13.6
+    const bool ahead = epg == 4;
+    RC_RET(x_dtype == MLLM_HIP_F32 ? ahead ? go(moe_gate_logits_kernel<MLLM_HIP_F32, true>) : go(moe_gate_logits_kernel<MLLM_HIP_F32, false>)
+           : ahead                 ? go(moe_gate_logits_kernel<MLLM_HIP_BF16, true>)
+                                   : go(moe_gate_logits_kernel<MLLM_HIP_BF16, false>));
     if (lds2 > 64 * 1024)
       HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(moe_gate_select_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds2));
     hipLaunchKernelGGL(moe_gate_select_kernel, dim3(grid), dim3(GATE_TOK * 64), lds2, st, a);
@@ -1578,5 +1585,10 @@ MLLM_API int mllm_hip_moe_gate(const void* x, int x_dtype, const float* gate_wei
     hipLaunchKernelGGL(kern, dim3(grid), dim3(GATE_WAVES * 64), lds, st, a);
     return (int)hipGetLastError();
   };
-  return x_dtype == MLLM_HIP_F32 ? launch(moe_gate_kernel<MLLM_HIP_F32>) : launch(moe_gate_kernel<MLLM_HIP_BF16>);
+  // weights ahead of x while there is one workgroup per CU at most (84 registers, see above): 128 experts of 2048, us without / with: 8 tokens 23.8 / 22.1,
+  // 1024 24.6 / 23.8, 2048 37 / 43
+  const bool ahead = grid <= 256;
+  return x_dtype == MLLM_HIP_F32 ? ahead ? launch(moe_gate_kernel<MLLM_HIP_F32, true>) : launch(moe_gate_kernel<MLLM_HIP_F32, false>)
+         : ahead                 ? launch(moe_gate_kernel<MLLM_HIP_BF16, true>)
+                                 : launch(moe_gate_kernel<MLLM_HIP_BF16, false>);
 }
