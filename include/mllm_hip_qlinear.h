@@ -551,9 +551,11 @@ int mllm_hip_topk(const float* x, float* values, int32_t* indices, int64_t rows,
  * per row: two launches, three for softmax of many pieces or in place.  Same values and indices for top-k; softmax adds a row's terms in another order. */
 size_t mllm_hip_softmax_workspace_bytes(int64_t rows, int64_t len);
 int mllm_hip_softmax_ws(const float* x, float* y, int64_t rows, int64_t len, void* workspace, void* stream);
-/* How often a workgroup looks for the sums of a row's other pieces before it adds up the row by itself (default 4096); -1: the form of
- * three launches, whose workgroups do not look.  Comparison runs and tests: the same bits. */
+/* How often a workgroup looks for the sums of a row's other pieces before it adds up the row by itself (by default and at most 64 times, about
+ * 30 us); -1: the form of three launches, whose workgroups do not look.  Comparison runs and tests: the same bits.  mllm_hip_softmax_wait: the
+ * setting. */
 int mllm_hip_softmax_set_wait(int polls);
+int mllm_hip_softmax_wait(void);
 size_t mllm_hip_topk_workspace_bytes(int64_t rows, int64_t len, int k);
 int mllm_hip_topk_ws(const float* x, float* values, int32_t* indices, int64_t rows, int64_t len, int k, int largest, int sorted,
                      void* workspace, void* stream);

@@ -76,6 +76,7 @@ def lib():
         L.mllm_hip_softmax.argtypes = [vp, vp, i64, i64, vp]
         L.mllm_hip_topk.argtypes = [vp, vp, vp, i64, i64, ci, ci, ci, vp]
         L.mllm_hip_softmax_set_wait.argtypes = [ci]
+        L.mllm_hip_softmax_wait.argtypes = []
         L.mllm_hip_softmax_workspace_bytes.restype = C.c_size_t
         L.mllm_hip_softmax_workspace_bytes.argtypes = [i64, i64]
         L.mllm_hip_softmax_ws.argtypes = [vp, vp, i64, i64, vp, vp]

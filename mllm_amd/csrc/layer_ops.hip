@@ -383,12 +383,16 @@ __device__ __forceinline__ float block_sum_256(float v, float* s_red) {
 // STAGE 3: a workgroup keeps its exponentials in registers, publishes their sum and reads the other pieces' as they appear (the value is its
 // own flag; stores and loads of device scope, since every XCD has an L2 of its own).  It runs for up to SOFTMAX_WAIT workgroups, a quarter of what
 // the chip holds at once, so they run together.  Where they should not (other work on the chip), a workgroup gives up after `polls` looks
-// and adds up the row by itself: nobody waits for long, the bits are the same.  In a graph, us, stages 1 and 2 / 3 (with more workgroups, or more
+// and adds up the row by itself: the wait is bounded, the bits are the same.  In a graph, us, stages 1 and 2 / 3 (with more workgroups, or more
 // pieces to look at, the looks cost more than a launch): 1 x 50 000 8.9 / 7.2, 4 x 64 000 9.7 / 7.9, 8 x 151 936 10.6 / 9.7, 16 x 151 936 (608)
 // 12.0 / 12.4, 512 x 151 936 225 / 255, 1 x 1 000 000 (245 pieces) 9.9 / 11.4; a launch less for the host.
 constexpr uint32_t SOFTMAX_NO_SUM = 0xffffffffu;
 constexpr int SOFTMAX_WAIT = 512, SOFTMAX_WAIT_PIECES = 64;
-static int g_softmax_polls = 4096;  // mllm_hip_softmax_set_wait; a look takes about a microsecond
+// Looks: sixteen were too few in some of the runs of 8 x 151 936 and 13 x 151 931, 32 and more in none.  64 take about 30 us, less than to
+// add up the row (50 to 90 us with no wait: 8 x 151 936, 1 x 262 144), so that a workgroup whose row is not on the chip all at once gives its
+// place up soon.
+constexpr int SOFTMAX_LOOKS = 64;
+static int g_softmax_polls = SOFTMAX_LOOKS;  // mllm_hip_softmax_set_wait
 template <int STAGE>
 __global__ __launch_bounds__(256) void softmax_pieces_kernel(const float* __restrict__ x, float* __restrict__ y, float* __restrict__ ws,
                                                              int len, int exp_accurate, int polls) {
@@ -1482,9 +1486,10 @@ MLLM_API size_t mllm_hip_softmax_workspace_bytes(int64_t rows, int64_t len) {
 }
 MLLM_API int mllm_hip_softmax_set_wait(int polls) {
   if (polls < -1) return MLLM_HIP_E_BADARG;
-  g_softmax_polls = polls;
+  g_softmax_polls = std::min(polls, SOFTMAX_LOOKS);
   return 0;
 }
+MLLM_API int mllm_hip_softmax_wait(void) { return g_softmax_polls; }
 MLLM_API int mllm_hip_softmax_ws(const float* x, float* y, int64_t rows, int64_t len, void* workspace, void* stream) {
   const int pieces = workspace && rows > 0 && len > 0 ? softmax_pieces(rows, len) : 0;
   if (!pieces) return mllm_hip_softmax(x, y, rows, len, stream);

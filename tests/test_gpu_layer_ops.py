@@ -371,6 +371,14 @@ def test_softmax_pieces_that_wait_for_each_other(rows, ln):
     assert torch.equal(got[0].view(torch.int32), got[1].view(torch.int32)) and torch.equal(got[0].view(torch.int32), got[2].view(torch.int32))
 
 
+def test_softmax_pieces_wait_less_than_adding_up_the_row_takes():
+    """host-only query: a workgroup looks at most 64 times (30 us), whatever is asked for; 50 to 90 us is what it does instead of waiting on"""
+    L = _lib.lib()
+    for polls, looks in ((4096, 64), (65, 64), (7, 7), (0, 0), (-1, -1), (64, 64)):
+        assert L.mllm_hip_softmax_set_wait(polls) == 0 and L.mllm_hip_softmax_wait() == looks
+    assert L.mllm_hip_softmax_set_wait(-2) != 0 and L.mllm_hip_softmax_wait() == 64
+
+
 @pytest.mark.parametrize("polls", [4096, 0])
 @pytest.mark.parametrize("rows,ln", [(8, 151936), (2, 262144), (3, 45057)])
 def test_softmax_pieces_in_place(rows, ln, polls):
