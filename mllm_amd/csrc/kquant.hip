@@ -1139,3 +1139,15 @@ MLLM_API int mllm_hip_linear_kq_gemm_short(int wtype, const void* gemm_packed, c
   void* partial = qg_partial_bytes(MLLM_HIP_Q4_K, M, N, K) ? base + mllm_hip_linear_kq_gemm_workspace_bytes(M, K) : nullptr;
   return qg_linear_run(wtype, gemm_packed, xh, bias, y, M, N, K, partial, st);
 }
+
+MLLM_API int mllm_hip_kq_moe_pair_tiles(int nparts, int64_t N, int64_t K, int slots) {
+  if (nparts < 1 || nparts > KQ_MAX_PARTS || slots < 1 || slots > 65535 || N <= 0 || N > 0x7fffffff || K <= 0 || !kq_moe_groups_fit(MLLM_HIP_Q6_K, nparts * N, K, slots)) return 0;
+  const int id = 0;
+  KGemvArgs a{};
+  a.slot_ids = &id;
+  a.M = 4;
+  a.nsb = (int)(K / QK_K);
+  a.nparts = nparts;
+  for (int p = 0; p < nparts; p++) a.part[p].N = (int)N;
+  return kr_pair_tiles(a, (unsigned)slots, kr_shape(false, a, (unsigned)slots, true, true).tiles);
+}

@@ -585,7 +585,7 @@ static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y, bool quant
   // on).  13 to 16 slices, 128 to 4096 channels, us, a slice / two per wave: 3 x 2048 x 8192 Q4_K 10.1 / 8.8, Q6_K 10.8 / 9.5; 6 x 1024 x
   // 7168 8.84 / 8.67, 10.1 / 9.9; eight rows 8.96 / 9.26, 10.2 / 10.5; with twelve slices 8.36 / 8.46, 9.1 / 9.9.
   if (!quantizes && !moe && tw == 1 && P > 12 && P == S && a.M <= 6) P = (S + 1) / 2;
-  // one tile per workgroup that quantizes x itself: waves without a slice share that, two items per thread (up to eight waves; 1024 x 1024
+  // one tile per workgroup that quantizes x itself: waves without a slice share that, two items per thread of the four that it requests ahead (up to eight waves; 1024 x 1024
   // Q6_K at three / four / eight rows 5.8 / 6.3 / 8.9 -> 5.2 / 5.3 / 6.5 us, Q4_K at eight 8.3 -> 6.0; with more tiles the added waves cost
   // more than they take over, 6144 x 2048 Q6_K at eight rows 8.4 -> 9.5)
   if (quantizes && !moe && tw == 1) P = std::max(P, std::min(8, (a.M * a.nsb * 32 + 127) / 128));
@@ -608,6 +608,16 @@ static int kr_threads(int wtype, const KGemvArgs& a) {  // of a workgroup that q
   const KrShape s = kr_shape(wtype == MLLM_HIP_Q4_K, a, 1, true);
   return s.tiles * s.waves * 64;
 }
+// Pairs: tiles per wave.  Two save the second round of workgroups, which repeat the search for the pairs and the quantization, but a wave waits for
+// twice the weights.  us of a layer of 128 experts, top-8 (top-4 for 768 x 2048), one tile / two (workgroups of the launch with one, all parts; the chip holds 1024 by their registers):
+// down of 768 elements, 2048 rows: 30.4 / 32.0 (1280), 33.7 / 34.4 (1536), 42.1 / 41.4 (2048), 49.7 / 48.4 (2560), 57.2 / 57.4 (4096); gate + up of
+// 768 elements, 2 x 2048 rows: 26.0 / 25.9 (1536), 29.8 / 28.4 (2048), 34.5 / 33.2 (2560), 44.8 / 45.5 (4096).  Longer rows gain nothing: 1024 elements 41.3 / 42.2
+// (1536), 51.5 / 52.4 (2048), 60.5 / 60.7 (3072), 1536 elements 57.9 / 60.2, 73.7 / 75.9, 84.4 / 84.3.  (N is a multiple of 256 here: whole tiles.)
+static int kr_pair_tiles(const KGemvArgs& a, unsigned grid_y, int tw) {
+  int64_t workgroups = 0;
+  for (int i = 0; i < a.nparts; i++) workgroups += (int64_t)grid_y * (((a.part[i].N + 15) / 16 + tw - 1) / tw);
+  return a.nsb <= 3 && workgroups >= 2048 ? 2 : 1;
+}
 template <int WT, int XT, int TH, int ORDER>
 static int launch_kq_rows(const KGemvArgs& a_in, hipStream_t st, unsigned grid_y = 1) {
   KGemvArgs a = a_in;
@@ -616,11 +626,7 @@ static int launch_kq_rows(const KGemvArgs& a_in, hipStream_t st, unsigned grid_y
   const size_t lds = kr_lds_bytes(WT == MLLM_HIP_Q4_K, a.nsb, tw, P);
   if (lds > KR_LDS_MAX) return MLLM_HIP_E_SHAPE;
   unsigned grid = 0;
-  // Pairs: two tiles per wave where one each would be more workgroups than the chip holds at once (1024 by their registers).  A second round repeats
-  // the search for the pairs and the quantization.  Two layers of 128 experts of 2048 x 768, top-8, 8 tokens (2048 workgroups, some 1650 of them
-  // with work): 131.7 -> 128.0 us, four tiles 128.6; 4 tokens (1024): 93.2 / 95.4.
-  const int64_t single = (int64_t)grid_y * (((a.part[0].N + 15) / 16 + tw - 1) / tw);
-  const int T = ORDER == KR_PAIRS && single >= 1536 ? 2 : 1;
+  const int T = ORDER == KR_PAIRS ? kr_pair_tiles(a, grid_y, tw) : 1;
   for (int i = 0; i < a.nparts; i++) {
     a.wg_start[i] = (int)grid;
     grid += (unsigned)(((a.part[i].N + 15) / 16 + tw * T - 1) / (tw * T));

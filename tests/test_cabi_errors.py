@@ -170,6 +170,16 @@ def test_moe_tiles_of_long_rows_spread_their_slices_over_waves():
     assert shape(Q4_K, 8, 2 * 768, 4096, 10) == (4, 2) and shape(Q6_K, 8, 2 * 768, 4096, 10) == (2, 4)
 
 
+def test_moe_pairs_take_two_tiles_per_wave_where_that_is_faster():
+    """from 2048 workgroups of all parts on, and for rows of three super-blocks: longer ones were up to 5 % slower with two (1536 and 2048 workgroups of 1024
+    and 1536 elements), and so were three (1536 workgroups)"""
+    tiles = _lib.lib().mllm_hip_kq_moe_pair_tiles
+    for parts, N in ((1, 2048), (2, 1024)):
+        assert [tiles(parts, N, 768, slots) for slots in (16, 48, 63, 64, 128)] == [1, 1, 1, 2, 2]
+        assert [tiles(parts, N, K, 64) for K in (512, 1024, 1280, 1536, 1792)] == [0, 1, 1, 1, 0]
+    assert tiles(1, 1024, 768, 127) == 1 and tiles(1, 1024, 768, 128) == 2 and tiles(0, 2048, 768, 64) == 0 and tiles(1, 2048, 768, 15) == 0
+
+
 def test_softmax_is_cut_into_pieces_only_where_that_is_not_slower():
     """193 to 256 rows, one whole round of workgroups, stay a workgroup per row up to 50 000 elements"""
     room = _lib.lib().mllm_hip_softmax_workspace_bytes

@@ -280,6 +280,7 @@ def test_rows_kernel_edges(wtype, M, Ns, K):
 @pytest.mark.parametrize("wtype,H,I,T,E,k,shared,same_as", [
     # pairs one by one, pairs in groups of four (Q6_K, three to six super-blocks; gate / up, down or both), at the edges of that rule
     (2, 768, 1024, 16, 64, 2, 19, 1), (3, 2048, 768, 8, 64, 2, 0, 1), (3, 1024, 512, 11, 64, 2, 9, 1), (3, 1024, 2048, 4, 64, 4, 5, 1),
+    ((2, 3), 2048, 768, 32, 256, 2, 21, 1), ((2, 3), 2048, 768, 63, 256, 1, 13, 1), ((3, 2), 768, 1024, 32, 256, 2, 21, 1), ((3, 3), 768, 1024, 31, 256, 2, 9, 1),  # (two tiles per wave, one)
     ((2, 3), 2048, 768, 9, 64, 3, 19, 1), ((2, 3), 2048, 1536, 31, 256, 4, 124, 1), ((3, 2), 1536, 1024, 15, 64, 2, 30, 1), (3, 1280, 1280, 13, 128, 2, 13, 1),
     # less than one pair per expert, with the sums of the sorted tiles
     (3, 256, 512, 20, 256, 8, 9, 2), ((2, 3), 512, 256, 17, 64, 3, 0, 2), ((3, 2), 1792, 256, 31, 128, 4, 124, 2)])
