@@ -32,6 +32,65 @@ def test_per_token_quant_bit_exact_special_rows():
         assert np.array_equal(s.cpu().numpy().view(np.uint32), wsc.view(np.uint32))
 
 
+def _codes_by_division(x):
+    """numpy, one IEEE division per element: the maximum passes over NaN, the code of NaN is -128"""
+    amax = np.fmax(np.nanmax(np.abs(x), axis=1, initial=0.0), np.float32(1e-10)).astype(np.float32)
+    scale = amax / np.float32(127.0)
+    with np.errstate(invalid="ignore"):
+        q = np.rint(x / scale[:, None])
+    return np.where(np.isnan(q), -128.0, np.clip(q, -128.0, 127.0)).astype(np.int8), scale
+
+
+def _hard_rows(rows, K):
+    """rows with NaN, infinities, zeros, tiny and largest magnitudes, and rows of every code's half-way points (scale * (n + 1/2), one ulp below and above,
+    both signs) under scales of random significands"""
+    rng = synth.rng_for(3, 77 + K)
+    x = rng.standard_normal((rows, K)).astype(np.float32)
+    x[0, K // 2], x[0, 0] = np.nan, -np.nan
+    x[1, 1], x[1, K - 1], x[1, 5] = np.inf, -np.inf, np.nan
+    x[2] = 0.0
+    x[3] *= np.float32(1e-38)
+    x[4] = np.where(np.arange(K) % 3, -3.4028235e38, 1e36).astype(np.float32)
+    x[5] *= np.float32(2.0 ** -42)
+    x[6] = np.nan
+    x[7] = np.float32(-1e-10) * (np.arange(K) % 255).astype(np.float32) / 254
+    half = np.arange(127, dtype=np.float64) + 0.5
+    for r in range(8, rows):
+        amax = np.float32((1 + rng.random()) * 2.0 ** int(rng.integers(-30, 100)))
+        mid = (half * float(amax / np.float32(127.0))).astype(np.float32)
+        mid = np.concatenate([mid, np.nextafter(mid, np.float32(0)), np.nextafter(mid, np.float32(np.inf))])
+        mid = np.concatenate([mid, -mid])
+        mid = mid[np.abs(mid) <= amax][:K - 1]
+        x[r] = 0.0
+        x[r, :mid.size], x[r, K - 1] = mid, amax
+    return x
+
+
+@pytest.mark.parametrize("K", [768, 2816, 9728])
+def test_per_token_codes_are_those_of_a_division(K):
+    """the rows above through the launch that quantizes (a row in registers, and read twice) and through the Linear of one to four tokens, whose one-hot
+    weights return the codes times the scales"""
+    x = _hard_rows(48, K)
+    for xd in (to_dev(x), to_dev(x).bfloat16()):
+        xf = xd.float().cpu().numpy()
+        want, scale = _codes_by_division(xf)
+        announce("per-token codes beside a division", K, str(xd.dtype))
+        q, s = ql.per_token_quant_int8(xd)
+        assert np.array_equal(s.cpu().numpy().view(np.uint32), scale.view(np.uint32))
+        assert np.array_equal(q.cpu().numpy(), want)
+        if K > 768:
+            continue
+        W = ql.w8a8_prepack(torch.eye(K, dtype=torch.int8, device="cuda"))
+        one = torch.ones(K, device="cuda")
+        with np.errstate(invalid="ignore", over="ignore"):
+            f = torch.from_numpy(want.astype(np.float32) * (np.float32(1.0) * scale[:, None]))
+        for M in (1, 2, 3, 4):
+            for r in range(0, 48, M):
+                y = ql.w8a8_linear_packed(xd[r:r + M].contiguous(), W, K, one).float().cpu()
+                w = f[r:r + M].bfloat16().float()
+                assert torch.equal(y.nan_to_num(nan=3e38), w.nan_to_num(nan=3e38)), (M, r)
+
+
 @pytest.mark.parametrize("M,K", [(2048, 2048), (7, 100), (3, 8), (5, 6144 + 24)])
 def test_per_token_quant_bit_exact(M, K):
     rng = synth.rng_for(3, M + K)
