@@ -283,7 +283,8 @@ int mllm_hip_w8a8_linear(const void* x, int x_dtype, const int8_t* W, const floa
  * pymllm/quantization/methods/compressed_tensors.py:429-448, where it re-lays the matrix for its CUTLASS kernel): the
  * [N][K] int8 matrix in the operand order of v_mfma_i32_32x32x32_i8, N padded to 32 and K to 128 with zeros, so that the
  * GEMM's waves fetch their weight operands from global memory with fully contiguous 1 KB loads and skip LDS for them.
- * Same arithmetic and results as mllm_hip_w8a8_gemm / _linear; this is the fast path for prefill-sized M. */
+ * Same arithmetic and results as mllm_hip_w8a8_gemm / _linear; this is the fast path for prefill-sized M.  _linear_packed takes the same
+ * workspace at any M, but leaves the codes there only where it quantizes in a launch of its own (not with one to four tokens). */
 size_t mllm_hip_w8a8_packed_bytes(int64_t N, int64_t K);
 int mllm_hip_w8a8_prepack(const int8_t* W, int64_t N, int64_t K, void* packed, void* stream);
 int mllm_hip_w8a8_gemm_packed(const int8_t* xq, const float* x_scale, const void* W_packed, const float* w_scale,

@@ -606,7 +606,8 @@ __device__ __forceinline__ f16x2 qg_offset2(const uint32_t (&s)[qg_scale_dwords(
 // int8 at load time, ds the scale of the step's 16 elements: the Q8_0 arithmetic.
 // These instructions and the MFMAs take turns (4 clocks each but 2 for a shift, and / or), so: nibbles at bits 4 b + 0..3 go into the mantissa of
 // 1024 (b even) or as they are into that of 64 (b odd), one shift for two of the four pairs instead of three; bytes are put under the mantissa
-// of 1024 by a permutation.  Three shifts and and / or on bytes took 117.2 us at 2048 x 9728 x 2560 Q6_K (113.7 now), 27.8 at 131 x 2560 x 9728 Q6_K (25.4), 26.2 Q4_0 (25.2).
+// of 1024 by a permutation.  In a graph, three shifts and and / or on bytes / this, us: 2048 x 9728 x 2560 Q6_K 119.3 / 117.7, Q4_0 115.9 / 113.0; 131 x 2560 x 9728 Q6_K
+// 28.3 / 25.9 (one call after the other 23.4 / 21.5), Q8_0 27.7 / 25.4, Q4_0 26.0 / 25.0, Q4_K 25.4 / 24.4.
 template <int WT, int PREC>
 __device__ __forceinline__ uint32_t qg_pair(const u32x4 (&rq)[qg_nibbles(WT) ? 1 : 2], int d, int b, f16x2 dd, f16x2 dm, uint32_t& lo) {
   uint32_t t;

@@ -1,7 +1,7 @@
 // The short calls of mllm_amd/qlinear.py in native code: argument checks, output tensors and the call into the C ABI.  A decode-size launch
 // takes the host 2.5 us; the same checks in Python and a ctypes call took another 2.3 (one projection of a token: 4.8 us, 3.3 now), a torch.empty
-// 1.7 of which the allocator needs a third.  Same checks, exceptions, results and streams as the Python code had; the interpreter's lock is
-// released for the call, as ctypes does.
+// 1.7 of which the allocator needs a third.  Same checks, results and streams as the Python code had, and the same exceptions but
+// one: an argument that is no tensor is a TypeError (AttributeError before).  The interpreter's lock is released for the call, as ctypes does.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
