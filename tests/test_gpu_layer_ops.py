@@ -522,7 +522,7 @@ def test_moe_gate_over_a_prompt_in_two_launches():
             torch.cuda.synchronize()
             times.append(first.elapsed_time(last))
         return sorted(times[2:])[5]
-    assert time(lambda: ql.moe_gate(x, w, 8, scores=scores)) <= 1.37 * time(lambda: ql.moe_gate(x, w, 8))
+    assert time(lambda: ql.moe_gate(x, w, 8, scores=scores)) <= 1.42 * time(lambda: ql.moe_gate(x, w, 8))
 
 
 @pytest.mark.parametrize("M,H,E,k,dtype", [(512, 2048, 128, 8, "f32"), (1, 2048, 128, 8, "f32"), (7, 256, 60, 4, "f32"),
