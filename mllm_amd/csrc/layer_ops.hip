@@ -943,15 +943,18 @@ __device__ __forceinline__ int block_topk_256(const unsigned long long (&key)[R]
   sh.maxima[tid] = (uint32_t)(mine >> 32);
   __syncthreads();
   const u32x4 m4 = *reinterpret_cast<const u32x4*>(&sh.maxima[4 * lane]);  // every wave on its own, four maxima per lane
-  // a bit costs about 100 clocks (four ballots, their counts and a branch); it need not be the k-th largest exactly: enough once few are left
+  // a bit costs about 100 clocks (four ballots and their counts); it need not be the k-th largest exactly: enough once few are left.  Four bits
+  // between two looks at that: with a branch per bit equal values, which take all 32, were up to 16 % slower than without any (largest 20 of 2 x 48 496 with
+  // ten values: 12.6 us without, 14.5 with, 12.8 now; normal ones, 8 x 151 936: 10.9, 9.7, 9.5)
   uint32_t b32 = 0;
   int reach = 256;  // maxima at or above b32
-  for (int bit = 31; bit >= 0 && reach > k + 12; bit--) {
-    const uint32_t t = b32 | (1u << bit);
-    const int c = __popcll(__ballot(m4.x >= t)) + __popcll(__ballot(m4.y >= t)) + __popcll(__ballot(m4.z >= t)) + __popcll(__ballot(m4.w >= t));
-    if (c >= k) {
-      b32 = t;
-      reach = c;
+  for (int bit = 31; bit >= 0 && reach > k + 12; bit -= 4) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t t = b32 | (1u << (bit - i));
+      const int c = __popcll(__ballot(m4.x >= t)) + __popcll(__ballot(m4.y >= t)) + __popcll(__ballot(m4.z >= t)) + __popcll(__ballot(m4.w >= t));
+      b32 = c >= k ? t : b32;
+      reach = c >= k ? c : reach;
     }
   }
   unsigned long long bound = (unsigned long long)b32 << 32;

@@ -525,6 +525,22 @@ def test_moe_gate_over_a_prompt_in_two_launches():
     assert time(lambda: ql.moe_gate(x, w, 8, scores=scores)) <= 1.42 * time(lambda: ql.moe_gate(x, w, 8))
 
 
+@pytest.mark.parametrize("rows,ln", [(1, 4100), (3, 48496), (8, 32001)])
+@pytest.mark.parametrize("k", [1, 20, 57, 64, 100, 128])
+def test_topk_pieces_of_equal_and_sorted_rows(rows, ln, k):
+    """ten values, rows in order both ways, one value, 16-bit values: the bound of the candidates is found with every bit of it or is left early; values and
+    lowest indices first"""
+    g = torch.Generator(device="cuda").manual_seed(rows + ln)
+    x = torch.randn((rows, ln), device="cuda", generator=g)
+    announce("topk of equal and sorted rows", rows, ln, k)
+    for r in ((2 * x).round(), x.sort(-1).values, x.sort(-1, descending=True).values, torch.full_like(x, -2.5), x.bfloat16().float(), (x > 2.5).float()):
+        r = r.contiguous()
+        for largest in (True, False):
+            v, i = ql.topk(r, k, largest)
+            want, at = torch.sort(r, dim=-1, descending=largest, stable=True)
+            assert torch.equal(v, want[:, :k]) and torch.equal(i.long(), at[:, :k])
+
+
 @pytest.mark.parametrize("M,H,E,k,dtype", [(512, 2048, 128, 8, "f32"), (1, 2048, 128, 8, "f32"), (7, 256, 60, 4, "f32"),
                                            (33, 2048, 128, 8, "bf16"), (5, 64, 8, 2, "f32")])
 def test_moe_gate(M, H, E, k, dtype):
