@@ -475,6 +475,8 @@ int mllm_hip_kq_set_rows_shape(int tiles, int waves);
 /* What a Linear of three to eight rows takes where a workspace is given (row_tiles > 0: a launch over that many row tiles of an MoE layer, N =
  * the channels of gate and up, or of down): 16 * tiles + waves per tile; 0: not that kernel.  Host only. */
 int mllm_hip_kq_rows_shape(int wtype, int64_t M, int64_t N, int64_t K, int row_tiles);
+/* 1 where that Linear's rows are quantized by a launch of its own, 0 where its workgroups do that (or it is not that kernel).  Host only. */
+int mllm_hip_kq_rows_image(int wtype, int64_t M, int64_t N, int64_t K);
 /* Tiles per wave where Q6_K MoE pairs run in groups (nparts matrices of N rows of K elements per expert); 0: they do not.  Host only. */
 int mllm_hip_kq_moe_pair_tiles(int nparts, int64_t N, int64_t K, int slots);
 int mllm_hip_linear_kq(int wtype, const void* packed, const void* x, int x_dtype, const float* bias, float* y, int64_t M, int64_t N,

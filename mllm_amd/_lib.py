@@ -116,6 +116,7 @@ def lib():
         L.mllm_hip_kq_set_slice_meeting.argtypes = [ci, ci]
         L.mllm_hip_kq_set_rows_shape.argtypes = [ci, ci]
         L.mllm_hip_kq_rows_shape.argtypes = [ci, i64, i64, i64, ci]
+        L.mllm_hip_kq_rows_image.argtypes = [ci, i64, i64, i64]
         L.mllm_hip_kq_moe_pair_tiles.argtypes = [ci, i64, i64, ci]
         L.mllm_hip_kq_workspace_bytes_n.restype = C.c_size_t
         L.mllm_hip_kq_workspace_bytes_n.argtypes = [i64, i64, i64]

@@ -945,12 +945,7 @@ MLLM_API int mllm_hip_linear_kq_multi_ws(int wtype, int nparts, const mllm_hip_g
     // From three rows on the matrix cores, while the rows' codes fit the LDS.  The rule looks at the number of rows and the row
     // length only: a projection gives the same bits alone and as a part of a launch.
     if (rows >= 3 && g_kq_path != 1 && kr_fits(nsb)) {
-      // Quantized once, by a launch of its own, where every workgroup would have more than four items of eight elements per
-      // thread to quantize, as many as a thread requests ahead of the weights (own launch / in the workgroups, us: q+k+v of 2560 elements, three
-      // rows 8.2 / 7.0, five 8.2 / 7.4, eight (four items) 8.2 / 8.3; gate+up 12.0 / 10.2, 11.9 / 10.7, 11.9 / 11.6; o of 4096, four rows 7.5 / 7.1, five
-      // (five items) 7.6 / 7.8, eight 7.6 / 9.3; 2048 x 6144 Q6_K at four 9.8 / 9.2, at five (five items) 10.1 / 10.4; 1024 x 1024 at three 6.3 / 4.8,
-      // at eight 6.5 / 5.5).  Same bits.
-      if (workspace && rows * nsb * 32 > 4 * kr_threads(wtype, a)) {
+      if (workspace && kr_image(wtype, a)) {
         hipLaunchKernelGGL(kr_image_kernel, dim3((unsigned)((nsb * 32 + 255) / 256), (unsigned)rows), dim3(256), 0, st, xg, x_dtype,
                            reinterpret_cast<unsigned char*>(workspace), nsb, rows);
         a.x = workspace;
@@ -1150,4 +1145,14 @@ MLLM_API int mllm_hip_kq_moe_pair_tiles(int nparts, int64_t N, int64_t K, int sl
   a.nparts = nparts;
   for (int p = 0; p < nparts; p++) a.part[p].N = (int)N;
   return kr_pair_tiles(a, (unsigned)slots, kr_shape(false, a, (unsigned)slots, true, true).tiles);
+}
+
+MLLM_API int mllm_hip_kq_rows_image(int wtype, int64_t M, int64_t N, int64_t K) {
+  if (!mllm_hip_kq_rows_shape(wtype, M, N, K, 0)) return 0;
+  KGemvArgs a{};
+  a.M = (int)M;
+  a.nsb = (int)(K / QK_K);
+  a.nparts = 1;
+  a.part[0].N = (int)N;
+  return kr_image(wtype, a);
 }

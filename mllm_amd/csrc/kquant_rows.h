@@ -604,9 +604,17 @@ static KrShape kr_shape(bool q4, const KGemvArgs& a, unsigned grid_y, bool quant
   while (tw > 1 && kr_lds_bytes(q4, a.nsb, tw, P) > KR_LDS_MAX) tw--;
   return KrShape{tw, P};
 }
-static int kr_threads(int wtype, const KGemvArgs& a) {  // of a workgroup that quantizes
-  const KrShape s = kr_shape(wtype == MLLM_HIP_Q4_K, a, 1, true);
-  return s.tiles * s.waves * 64;
+// Whether three to eight rows are quantized once, by a launch of its own (given a workspace): where every workgroup would have more than four items of
+// eight elements per thread to quantize, as many as a thread requests ahead of the weights (own launch / in the workgroups, us: q+k+v of 2560 elements,
+// three rows 8.2 / 7.0, five 8.2 / 7.4, eight (four items) 8.2 / 8.3; gate+up 12.0 / 10.2, 11.9 / 10.7, 11.9 / 11.6; o of 4096, four rows 7.5 / 7.1,
+// five (five items) 7.6 / 7.8, eight 7.6 / 9.3; 2048 x 6144 Q6_K at four 9.8 / 9.2, at five (five items) 10.1 / 10.4; 1024 x 1024 at three 6.3 / 4.8, at
+// eight 6.5 / 5.5).  And where the launch lets waves take two slices each (thirteen and more, kr_shape): three rows of 2560 x 7168 Q4_K 8.3 / 8.6, Q6_K
+// 8.9 / 9.5, four 8.5 / 9.4, 9.1 / 10.1; 4096 x 6656 Q6_K 8.9 / 9.5, 9.0 / 10.1.  Same bits.
+static bool kr_image(int wtype, const KGemvArgs& a) {
+  const bool q4 = wtype == MLLM_HIP_Q4_K;
+  const KrShape with = kr_shape(q4, a, 1), without = kr_shape(q4, a, 1, true);
+  const int slices = kr_slices(a.nsb);
+  return a.M * a.nsb * 32 > 4 * without.tiles * without.waves * 64 || (with.tiles == 1 && slices > 12 && with.waves == (slices + 1) / 2);
 }
 // Pairs: tiles per wave.  Two save the second round of workgroups, which repeat the search for the pairs and the quantization, but a wave waits for
 // twice the weights.  us of a layer of 128 experts, top-8 (top-4 for 768 x 2048), one tile / two (workgroups of the launch with one, all parts; the chip holds 1024 by their registers):

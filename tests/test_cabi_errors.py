@@ -160,6 +160,16 @@ def test_long_rows_of_few_channels_take_two_slices_per_wave(wtype, N):
     assert shape(wtype, 8, N, 8192, 0) == 16 + 16 and shape(wtype, 3, 4112, 8192, 0) == 2 * 16 + 8
 
 
+@pytest.mark.parametrize("wtype", [Q4_K, Q6_K])
+def test_rows_that_take_two_slices_per_wave_are_quantized_once(wtype):
+    """three and four rows of 13 to 16 slices were up to 13 % slower where every workgroup quantizes them (four items per thread with a wave per slice)"""
+    image = _lib.lib().mllm_hip_kq_rows_image
+    for N in (80, 2560, 4096):
+        assert [image(wtype, M, N, K) for K in (6400, 6656, 7168, 8192) for M in (3, 4, 6)] == [1] * 12
+        assert [image(wtype, M, N, K) for K in (1024, 2560, 4096) for M in (3, 4)] == [0] * 6
+    assert image(wtype, 5, 2560, 4096) == 1 and image(wtype, 4, 2048, 6144) == 0 and image(wtype, 2, 2560, 4096) == 0 and image(wtype, 5, 2560, 9728) == 1
+
+
 def test_moe_tiles_of_long_rows_spread_their_slices_over_waves():
     """one wave per tile walked all of K: 4 to 21 % slower than a workgroup per slice with eight experts of 3584 or 4096 elements"""
     shape = lambda *a: divmod(_lib.lib().mllm_hip_kq_rows_shape(*a), 16)  # noqa: E731
