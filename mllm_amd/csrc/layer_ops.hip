@@ -901,7 +901,7 @@ __global__ __launch_bounds__(NT) void topk_select_rows_kernel(const float* __res
 // Few long rows spread over the chip (mllm_hip_topk_ws), k up to 128: a row is cut into equal pieces of at most TOPK_PIECE elements, a
 // workgroup selects the k largest keys of its piece into the caller's workspace, and a second launch selects among the
 // pieces' keys.  A workgroup per row is bound by what one CU loads per pass over the row: 20 of eight rows of 151 936 take
-// 110 us there and 9.7 here, 64 of them 111 and 12.5.
+// 110 us there and 9.5 here, 64 of them 111 and 12.5.
 //
 // Selection inside a workgroup: keys are unique (value, inverted index).  The k-th largest of the threads' own maxima (found a
 // bit at a time by counting, every wave on its own) is at most the k-th largest value, so the keys at or above it contain the
