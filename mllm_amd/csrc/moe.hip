@@ -443,6 +443,7 @@ __global__ __launch_bounds__(MODE == 1 ? 512 : 256) void qgemm_tile_kernel(QGemm
 // weights straight from global memory two K steps ahead, dequantized one MFMA step ahead in the shadows of the MFMAs.
 // =========================================================================================================
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
@@ -1045,38 +1046,39 @@ static int launch_qg(const QG2Args& a, unsigned max_tiles, hipStream_t st) {
 //
 //   y[row][n] = sum_b fp32(dW[n][b] * dX[row][b]) * float(sum_32 qW * qX)
 //
-// (llamafile_sgemm.cpp:697-743: Cv += set1(dW * dX) * float(int32 block sum)).  Per 32-row x 32-channel tile and block,
-// four v_mfma_f32_32x32x16_f16 and sixteen fp32 FMAs:
-//   * the block sum: two MFMAs whose operands are integers held as fp16 numbers.  The activation codes are stored that
-//     way; a weight code is OR-ed into the mantissa of 1024.0 (nibble at bits 0..3 of a half-word) or of 64.0 (bits
-//     4..7), i.e. it enters as 1024 + q or 64 + q (q = 0..15; Q8_0: 1024 + 128 + q), which costs five operations per
-//     eight 4-bit codes.  A third MFMA puts the correction in front: its operands are the constants -(1024 + 8),
-//     -(64 + 8) and the sums of the activation codes that meet each constant (two per row and block, from the producer
-//     of the activations), so the chain starts at -sum(offset * qX) and ends at sum((q - 8) * qX).  Every product and
-//     every partial sum is an integer below 2^24: the fp32 result IS the int32 block sum, already a float.
-//   * the 32 x 32 scale products dW[n] * dX[row]: a fourth MFMA, an outer product of the two fp16 scales sitting in one
-//     K slot of otherwise zero operands; an 11-bit by 11-bit product is exact in fp32.
-//   * acc = fma(dW * dX, block sum, acc): the reference's operation.  Only the order in which blocks are added differs
+// (llamafile_sgemm.cpp:697-743: Cv += set1(dW * dX) * float(int32 block sum)).  Per 32-row x 32-channel tile and block, two
+// matrix instructions, sixteen conversions and sixteen fp32 FMAs:
+//   * the block sum: one v_mfma_i32_32x32x32_i8 on the codes.  A nibble enters as the byte 16 (q - 8): the nibble in the high half,
+//     its top bit inverted, one three-input logic operation (and a shift for the low nibbles).  The 16 goes out behind the last
+//     block: a power of two moves through products and sums unrounded (|sum| <= 2^19, scales below 2^16: far from the ends of fp32).
+//   * the 32 x 32 scale products dW[n] * dX[row]: an outer product of the two fp16 scales sitting in one K slot of otherwise
+//     zero fp16 operands; an 11-bit by 11-bit product is exact in fp32.
+//   * acc = fma(dW * dX, float(block sum), acc): the reference's operation.  Only the order in which blocks are added differs
 //     from the CPU path.
-// Same gemm-packed weights and tile list as the fp16-operand kernel.  Activations: Q8_0 codes as fp16 integers
-// [rows][K] and one record of three dwords per row and K step of 64: the fp16 scales of the step's two blocks, then per
-// block the two partial code sums (elements with bit 1 of k clear | set) as fp16 integers.
+// Same gemm-packed weights and tile list as the fp16-operand kernel.  Activations: Q8_0 codes as bytes [rows][K] in the order in
+// which a lane's weights come out of their dwords (QX_ORDER below), and the fp16 scales of two blocks per dword.
+//
+// What bounds it: the vector ALU (160 instructions of 4 clocks per K step and wave, 32 clocks for each of the 8 matrix instructions beside
+// them: three waves per SIMD keep it busy), with few rows per expert the weights (5.8 TB/s for 128 tokens), and the last round of workgroups.
+// Codes as fp16 numbers (offsets in the mantissas of 1024 and 64) gave the sums as floats at 3.5 matrix instructions per block, but in
+// 242 registers, and more than there are for Q8_0: two waves per SIMD, and a wave's own chain of instructions was what a workgroup took, with a neighbour or
+// without (Q4_0 26 us, Q8_0 with registers in memory 70).  us of an FFN of 128 experts of 2048 x 768, top-8, before / now: 512 tokens
+// Q4_0 146 / 125, Q8_0 281 / 175; 128 tokens Q4_0 97 / 87; 317 tokens, top-4, 512 elements Q8_0 143 / 102.
 // =========================================================================================================
 struct QXArgs {
   const char* W0;        // gemm-packed weights of matrix 0 (gate, or the only matrix), expert e at W0 + e * wstride
   const char* W1;        // matrix 1 (up) in the gate/up mode
   size_t wstride;
-  const uint16_t* xq;    // Q8_0 codes of the activations as fp16 integers [a_rows][K]
-  const uint32_t* xd;    // [a_rows][KD][3] dwords: fp16 scales of blocks 2j | 2j+1, then per block fp16(sum of the codes
-                         // with (k & 2) == 0) | fp16(sum of the others) << 16; zeros past the end
+  const uint8_t* xq;     // Q8_0 codes of the activations [a_rows][K], a block's 32 in QX_ORDER
+  const uint32_t* xd;    // [a_rows][KD] fp16 scales of blocks 2j | 2j+1 (zero past the end)
   const int* a_index;    // activation row of sorted position pos is a_index[pos] / a_div ; null: pos itself
   int a_div;
   int a_rows;
   const int* o_index;    // output row of sorted position pos (null: pos itself)
   float* out;            // fp32 [..][N]       (one-matrix mode)
   const float* bias;     // [N] or null        (one-matrix mode)
-  uint16_t* hq;          // gate/up mode: Q8_0 codes of silu(g)*u as fp16 integers [rows][N]
-  uint32_t* hd;          // gate/up mode: their records [rows][ceil(N/64)][3], as xd
+  uint8_t* hq;           // gate/up mode: Q8_0 codes of silu(g)*u [rows][N], as xq
+  uint32_t* hd;          // gate/up mode: their scales [rows][ceil(N/64)], as xd
   const int* tile_expert;
   const int* tile_row0;
   const int* tile_rows;
@@ -1086,88 +1088,63 @@ struct QXArgs {
   int half_tiles;        // tiles of at most sixteen rows take the 16-row form (same bits; 0: comparison runs and tests)
 };
 
-// masks and exponent patterns of qx_codes, kept in registers (v_and_or_b32 takes no literal constants)
+// QX_ORDER: lane half hi of the 32-row operand takes the elements 8 hi .. 8 hi + 7 and 16 + 8 hi .. of a block (bytes 16 hi .. 16 hi + 15 of the
+// stored block), each eight in the order of the weights' dwords: Q4_0 low nibbles 0 4 1 5, high nibbles 2 6 3 7; Q8_0 0 2 1 3, 4 6 5 7.
+// lo, hi: the codes 0..3 and 4..7
+template <int WT>
+__device__ __forceinline__ u32x2 qx_order(uint32_t lo, uint32_t hi) {
+  if (WT == MLLM_HIP_Q4_0) return u32x2{__builtin_amdgcn_perm(hi, lo, 0x05010400u), __builtin_amdgcn_perm(hi, lo, 0x07030602u)};
+  return u32x2{__builtin_amdgcn_perm(0u, lo, 0x03010200u), __builtin_amdgcn_perm(0u, hi, 0x03010200u)};
+}
+// constants in registers (three-input logic takes no literal)
 struct QXConst {
-  uint32_t m_lo, m_hi, e_1024, e_64;
+  uint32_t m, x;
 };
-__device__ __forceinline__ QXConst qx_const(int wtype) {
-  QXConst c{wtype == MLLM_HIP_Q4_0 ? 0x000f000fu : 0x00ff00ffu, 0x00f000f0u, 0x64006400u, 0x54005400u};
-  asm volatile("" : "+v"(c.m_lo), "+v"(c.m_hi), "+v"(c.e_1024), "+v"(c.e_64));
+__device__ __forceinline__ QXConst qx_const() {
+  QXConst c{0xf0f0f0f0u, 0x80808080u};
+  asm volatile("" : "+v"(c.m), "+v"(c.x));
   return c;
 }
-// the eight weight codes of MFMA step d (16 K elements, this lane's half) as fp16 numbers offset + code:
-// Q4_0: 1024 + q for the elements with (k & 2) == 0, 64 + q for the others (q = 0..15); Q8_0: 1152 + q (q = -128..127)
-// ... from the dwords themselves: Q4_0 one dword (v1 unused), Q8_0 two
-template <int WT>
-__device__ __forceinline__ f16x8 qx_codes_dw(uint32_t v0, uint32_t v1, const QXConst& c) {
-  uint32_t o[4];
-  if (WT == MLLM_HIP_Q4_0) {
-    // pair i of the dword sits in nibbles i and 4 + i.  Nibbles at bits 0..3 of a half-word land in the mantissa of 1024.0
-    // (unit 1), nibbles at bits 4..7 in the mantissa of 64.0 (unit 1/16): pairs 0 and 1 need no shift, pairs 2 and 3 one
-    // shift by 8 for both.
-    const uint32_t t = v0 >> 8;
-    o[0] = (v0 & c.m_lo) | c.e_1024;
-    o[1] = (v0 & c.m_hi) | c.e_64;
-    o[2] = (t & c.m_lo) | c.e_1024;
-    o[3] = (t & c.m_hi) | c.e_64;
-  } else {
-    // two dwords of four codes each in byte order e0 e2 e1 e3; + 128 makes them unsigned
-    const uint32_t w0 = v0 ^ 0x80808080u, w1 = v1 ^ 0x80808080u;
-    o[0] = (w0 & c.m_lo) | c.e_1024;
-    o[1] = ((w0 >> 8) & c.m_lo) | c.e_1024;
-    o[2] = (w1 & c.m_lo) | c.e_1024;
-    o[3] = ((w1 >> 8) & c.m_lo) | c.e_1024;
-  }
-  return __builtin_bit_cast(f16x8, u32x4{o[0], o[1], o[2], o[3]});
-}
-template <int WT>
-__device__ __forceinline__ f16x8 qx_codes(const u32x4 (&rq)[WT == MLLM_HIP_Q4_0 ? 1 : 2], int d, const QXConst& c) {
-  if (WT == MLLM_HIP_Q4_0) return qx_codes_dw<WT>(rq[0][d], 0u, c);
-  return qx_codes_dw<WT>(rq[d >> 1][2 * (d & 1)], rq[d >> 1][2 * (d & 1) + 1], c);
-}
-// fp16 pair (-offset of the elements with (k & 2) == 0, -offset of the others) including the 8 of Q4_0's code offset
-__host__ __device__ constexpr uint32_t qx_offsets(int wtype) { return wtype == MLLM_HIP_Q4_0 ? 0xD480E408u : 0xE480E480u; }
+// four low / high nibbles of a dword as bytes 16 (q - 8)
+__device__ __forceinline__ uint32_t qx_high(uint32_t v, const QXConst& c) { return (v & c.m) ^ c.x; }
+__device__ __forceinline__ uint32_t qx_low(uint32_t v, const QXConst& c) { return qx_high(v << 4, c); }
+constexpr float QX_UNIT(int wt) { return wt == MLLM_HIP_Q4_0 ? 0.0625f : 1.f; }  // of the codes' products
+// K steps of weights and activations in flight per wave, in the 32-row and the 16-row form (512 tokens, Q4_0: 2 / 2 127.0 us for the FFN, 2 / 4
+// 125.3, 2 / 6 130; a Q8_0 wave has registers for two)
+constexpr int QX_ST(int) { return 2; }
+constexpr int QX_ST16(int wt) { return wt == MLLM_HIP_Q4_0 ? 4 : 2; }
 
-// One tile: `rows` (<= 32 TM) sorted positions from row0 x 128 TN channels from n0, NW weight matrices (1, or gate + up).
-template <int WT, int NW, int TM, int TN>
+// One tile: `rows` (<= 32) sorted positions from row0 x 128 TN channels from n0, NW weight matrices (1, or gate + up).
+template <int WT, int NW, int TN>
 __device__ __forceinline__ void qx_tile(const QXArgs& a, const int e, const int row0, const int rows, const int n0,
                                         unsigned char* smem) {
-  constexpr int BK = 64, LDK = 2 * BK + 16;
-  constexpr int BM = TM * 32, WN = TN * 32;
-  constexpr int CA = TM;                      // 16-byte activation chunks per thread and K step
-  constexpr int STAGE = BM * LDK + BM * 48;   // code rows, then per row the record's three dwords, each the first of a
-                                              // 16-byte MFMA operand whose other K slots are zero
+  constexpr int BK = 64, LDK = BK + 16;  // bytes of codes per row and K step; pitch in LDS (sixteen rows' reads cover all banks)
+  constexpr int BM = 32, WN = TN * 32;
+  constexpr int STAGE = BM * LDK + BM * 4;  // code rows, then the rows' scale pairs
   constexpr int QW = WT == MLLM_HIP_Q4_0 ? 1 : 2;
-  constexpr int ST = 4;                       // K steps of weights in flight per wave
+  constexpr int ST = QX_ST(WT);             // K steps of weights in flight per wave
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 31, hi = lane >> 5;
   const int Kp = (int)qg_kp(a.K), kbs = Kp / 64, nbs = (int)(qg_np(a.N) / 32), KD = (a.K + 63) / 64;
   const int64_t qbytes = qg_qbytes(WT, a.N, a.K), wbytes = qg_bytes(WT, a.N, a.K);
 
-  const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.xq), 0, (uint32_t)((int64_t)a.a_rows * a.K * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rD = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.xd), 0, (uint32_t)((int64_t)a.a_rows * KD * 12), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.xq), 0, (uint32_t)((int64_t)a.a_rows * a.K), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rD = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.xd), 0, (uint32_t)((int64_t)a.a_rows * KD * 4), 0x00020000);
   __amdgpu_buffer_rsrc_t rW[NW];
   rW[0] = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.W0 + (size_t)e * a.wstride), 0, (uint32_t)wbytes, 0x00020000);
   if (NW == 2) rW[NW - 1] = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.W1 + (size_t)e * a.wstride), 0, (uint32_t)wbytes, 0x00020000);
 
-  // activation chunk c of a thread: tile row (tid + 256 c) / 8, 16-byte column (tid + 256 c) % 8.  Rows past `rows` repeat
-  // the last one (never stored); columns past K read as zeros (out-of-range buffer offsets).
-  uint32_t offA[CA];
+  // activations of a thread: tile row tid / 8, eight codes from 8 (tid % 8).  Rows past `rows` repeat the last one (never
+  // stored); columns past K read as zeros (out-of-range buffer offsets).
   const int colA = (tid % 8) * 8;
-#pragma unroll
-  for (int c = 0; c < CA; c++) {
-    const int pos = row0 + min((tid + c * 256) / 8, rows - 1);
-    const int arow = a.a_index ? a.a_index[pos] / a.a_div : pos;
-    offA[c] = (uint32_t)(((int64_t)arow * a.K + colA) * 2);
-  }
-  // the record of a row and K step: threads 0 .. BM-1, one row each
-  uint32_t offD = 0xffffffffu;
-  if (tid < BM) {
-    const int pos = row0 + min(tid, rows - 1);
-    const int arow = a.a_index ? a.a_index[pos] / a.a_div : pos;
-    offD = (uint32_t)((int64_t)arow * KD * 12);
-  }
+  auto arow_of = [&](int r) -> uint32_t {
+    const int pos = row0 + min(r, rows - 1);
+    return (uint32_t)(a.a_index ? a.a_index[pos] / a.a_div : pos);
+  };
+  const uint32_t offA = arow_of(tid / 8) * (uint32_t)a.K + colA;
+  // the scales of a row and K step: threads 0 .. 31, one row each
+  const uint32_t offD = tid < BM ? arow_of(tid) * (uint32_t)(KD * 4) : 0xffffffffu;
   uint32_t offQ[TN], offS[TN];
 #pragma unroll
   for (int j = 0; j < TN; j++) {
@@ -1175,88 +1152,67 @@ __device__ __forceinline__ void qx_tile(const QXArgs& a, const int e, const int 
     offQ[j] = (uint32_t)((int64_t)nb * kbs * (1024 * QW) + lane * 16);
     offS[j] = (uint32_t)(qbytes + ((int64_t)nb * kbs * 32 + lrow) * 4);
   }
-  typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
-  // Activations travel two K steps ahead of their use, in two register sets.  Vector memory returns in order: the wait for
-  // a step's activations also waits for every load issued before them, so loading them only one step ahead would cut
-  // the weights' lead (ST steps) down to one step as well.
-  u32x4 ga[2][CA];
-  u32x3 gd[2] = {{0u, 0u, 0u}, {0u, 0u, 0u}};
+  // Activations travel as many K steps ahead of their use as the weights, in as many register sets.  Vector memory returns in order:
+  // the wait for a step's activations also waits for every load issued before them, and a shorter lead would be the weights' lead too.
+  u32x2 ga[ST];
+  uint32_t gd[ST] = {};
   auto loadA = [&](int set, int kt) {
-    const bool ok = kt * BK + colA < a.K;
-#pragma unroll
-    for (int c = 0; c < CA; c++) ga[set][c] = __builtin_amdgcn_raw_buffer_load_b128(rA, ok ? offA[c] : 0xffffffffu, kt * BK * 2, 0);
-    if (tid < BM) gd[set] = __builtin_amdgcn_raw_buffer_load_b96(rD, kt < KD ? offD : 0xffffffffu, kt * 12, 0);
+    ga[set] = __builtin_amdgcn_raw_buffer_load_b64(rA, kt * BK + colA < a.K ? offA : 0xffffffffu, kt * BK, 0);
+    if (tid < BM) gd[set] = __builtin_amdgcn_raw_buffer_load_b32(rD, kt < KD ? offD : 0xffffffffu, kt * 4, 0);
   };
   auto storeA = [&](int set, int buf) {
-#pragma unroll
-    for (int c = 0; c < CA; c++) {
-      const int idx = tid + c * 256;
-      *reinterpret_cast<u32x4*>(smem + buf * STAGE + (idx / 8) * LDK + (idx % 8) * 16) = ga[set][c];
-    }
-    if (tid < BM) {
-      u32x4* rec = reinterpret_cast<u32x4*>(smem + buf * STAGE + BM * LDK + tid * 48);
-      rec[0] = u32x4{gd[set].x, 0u, 0u, 0u};
-      rec[1] = u32x4{gd[set].y, 0u, 0u, 0u};
-      rec[2] = u32x4{gd[set].z, 0u, 0u, 0u};
-    }
+    *reinterpret_cast<u32x2*>(smem + buf * STAGE + (tid / 8) * LDK + colA) = ga[set];
+    if (tid < BM) *reinterpret_cast<uint32_t*>(smem + buf * STAGE + BM * LDK + tid * 4) = gd[set];
   };
 
-  v16f acc[NW][TN][TM];
+  v16f acc[NW][TN];
 #pragma unroll
   for (int w = 0; w < NW; w++)
 #pragma unroll
     for (int j = 0; j < TN; j++)
 #pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[w][j][i][r] = 0.f;
+      for (int r = 0; r < 16; r++) acc[w][j][r] = 0.f;
 
   u32x4 rq[ST][NW][TN][QW];  // packed codes of the K steps in flight (ring, slot = step % ST)
   uint32_t rs[ST][NW][TN];   // their scale dwords
-  auto loadW = [&](int slot, int kt) {
-    const bool ok = kt < kbs;  // steps past the end read nothing (zeros): the ring is always full
+  auto loadW1 = [&](int slot, int kt, int w, int j) {  // steps past the end read nothing (zeros): the ring is always full
 #pragma unroll
-    for (int w = 0; w < NW; w++)
-#pragma unroll
-      for (int j = 0; j < TN; j++) {
-#pragma unroll
-        for (int p = 0; p < QW; p++)
-          rq[slot][w][j][p] = __builtin_amdgcn_raw_buffer_load_b128(rW[w], ok ? offQ[j] : 0xffffffffu, (kt * QW + p) * 1024, 0);
-        rs[slot][w][j] = __builtin_amdgcn_raw_buffer_load_b32(rW[w], ok ? offS[j] : 0xffffffffu, kt * 128, 0);
-      }
+    for (int p = 0; p < QW; p++)
+      rq[slot][w][j][p] = __builtin_amdgcn_raw_buffer_load_b128(rW[w], kt < kbs ? offQ[j] : 0xffffffffu, (kt * QW + p) * 1024, 0);
+    rs[slot][w][j] = __builtin_amdgcn_raw_buffer_load_b32(rW[w], kt < kbs ? offS[j] : 0xffffffffu, kt * 128, 0);
   };
   // Scale operand of the weights: the fp16 scale of the step's first block in K slot 0 (low half of the first register), of
   // its second block in K slot 1 (high half), in the lanes of the low K half only; every other K slot is zero.  The
-  // activations' scale pair and code sums are used as they come (first register of an otherwise zero operand): what a K
-  // slot holds does not matter where the other operand is zero.
-  static_assert(TM == 1, "one row tile per workgroup");
+  // activations' scale pair is used as it comes (first register of an otherwise zero operand): what a K slot holds does not
+  // matter where the other operand is zero.
   const uint32_t msk0 = hi ? 0u : 0x0000ffffu, msk1 = hi ? 0u : 0xffff0000u;
   const v16f zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  const QXConst kc = qx_const(WT);
-  const f16x8 off_op = __builtin_bit_cast(f16x8, u32x4{hi ? 0u : qx_offsets(WT), 0u, 0u, 0u});
+  const QXConst kc = qx_const();
+  const v16i izero = {};
 
-  // A "group" is one (block, matrix, column tile): four MFMAs (offset correction, shared by the matrices of a block; two
-  // for the block sum; the scale product) and sixteen FMAs.  A wave issues in order and a dependent MFMA holds it until its
-  // input is ready, so everything else is slotted between the MFMAs of one group: the unpacking of the NEXT group's weight
-  // codes and the FMAs of the PREVIOUS group (whose MFMA results sit in the other of two register sets).  The matrix pipe
-  // then runs back to back while the vector ALU works in its shadow, within one wave.
+  // A "group" is one (block, matrix, column tile): two matrix instructions, in their shadow the unpacking of the NEXT group's weights,
+  // sixteen conversions and FMAs.
   constexpr int G = 2 * NW * TN;  // groups per K step: block-major, then matrix, then column tile
-  f16x8 fw[2][2];                 // unpacked codes of the current / next group (two MFMA steps each)
-  u32x4 sw[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};  // their scale operands
-  v16f T[2], S[2];                // block sums and scale products of the current / previous group
-  T[1] = zero16;
-  S[1] = zero16;
+  v4i fw;                         // codes of the next group
+  u32x2 sw = {0u, 0u}, rec = {0u, 0u};  // its scale operand, the rows' (K slots 0 to 3 of either half)
+  asm("" : "+v"(sw), "+v"(rec));        // (known to be zero, the upper register would be written again for every group)
+  auto unpack = [&](const u32x4 (&q)[QW], uint32_t s, int b) {
+    if (WT == MLLM_HIP_Q4_0) fw = v4i{(int)qx_low(q[0][2 * b], kc), (int)qx_high(q[0][2 * b], kc), (int)qx_low(q[0][2 * b + 1], kc), (int)qx_high(q[0][2 * b + 1], kc)};
+    else fw = __builtin_bit_cast(v4i, q[QW == 2 ? b : 0]);
+    sw.x = s & (b ? msk1 : msk0);
+  };
 
   const int nsteps = (kbs + ST - 1) / ST * ST;
-  loadA(0, 0);
-  loadA(1, 1);
 #pragma unroll
-  for (int s = 0; s < ST; s++) loadW(s, s);
+  for (int s = 0; s < ST; s++) {
+    loadA(s, s);
+#pragma unroll
+    for (int w = 0; w < NW; w++)
+#pragma unroll
+      for (int j = 0; j < TN; j++) loadW1(s, s, w, j);
+  }
   storeA(0, 0);
-  // the first group's operands
-  fw[0][0] = qx_codes<WT>(rq[0][0][0], 0, kc);
-  fw[0][1] = qx_codes<WT>(rq[0][0][0], 1, kc);
-  sw[0].x = rs[0][0][0] & msk0;
+  unpack(rq[0][0][0], rs[0][0][0], 0);
   __syncthreads();
 
   // one K step (64 elements = two blocks) with its weights in ring slot SLOT; refills the slot with step kt + ST
@@ -1264,158 +1220,111 @@ __device__ __forceinline__ void qx_tile(const QXArgs& a, const int e, const int 
     constexpr int SLOT = decltype(slot_tag)::value;
     constexpr int NSLOT = (SLOT + 1) % ST;
     const int buf = kt & 1;
-    loadA(SLOT & 1, kt + 2);  // the set whose step (kt) is in LDS already
-    f16x8 fb[2][2];
+    loadA(SLOT, kt + ST);  // the set whose step (kt) is in LDS already
+    v4i fb[2];
 #pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int d = 0; d < 2; d++)
-        fb[b][d] = *reinterpret_cast<const f16x8*>(smem + buf * STAGE + lrow * LDK + (2 * b + d) * 32 + hi * 16);
-    // the row's scale pair (both scales: the weight operand is zero in the other block's K slot) and its two code-sum pairs,
-    // each already an operand
-    f16x8 rec[3];
-#pragma unroll
-    for (int q = 0; q < 3; q++) rec[q] = *reinterpret_cast<const f16x8*>(smem + buf * STAGE + BM * LDK + lrow * 48 + q * 16);
-    v16f tc = zero16;
+    for (int b = 0; b < 2; b++) fb[b] = *reinterpret_cast<const v4i*>(smem + buf * STAGE + lrow * LDK + b * 32 + hi * 16);
+    rec.x = *reinterpret_cast<const uint32_t*>(smem + buf * STAGE + BM * LDK + lrow * 4);
 #pragma unroll
     for (int g = 0; g < G; g++) {
-      constexpr int cur = 0;  // the register sets alternate by the parity of g (G is even)
-      const int c = (g + cur) & 1, n = c ^ 1;
       const int b = g / (NW * TN), w = (g / TN) % NW, j = g % TN;
       // the next group: (b', w', j') in this step, or the first group of the next step (ring slot NSLOT)
       const bool last = g == G - 1;
       const int gn = last ? 0 : g + 1;
       const int bn = gn / (NW * TN), wn = (gn / TN) % NW, jn = gn % TN;
       __builtin_amdgcn_sched_barrier(0);
-      if (w == 0 && j == 0) {  // the block's correction, shared by all its groups
-        tc = __builtin_amdgcn_mfma_f32_32x32x16_f16(off_op, rec[1 + b], zero16, 0, 0, 0);
-      }
+      const v16i D = __builtin_amdgcn_mfma_i32_32x32x32_i8(fw, fb[b], izero, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
-      if (last) fw[n][0] = qx_codes<WT>(rq[NSLOT][wn][jn], 2 * bn, kc);
-      else fw[n][0] = qx_codes<WT>(rq[SLOT][wn][jn], 2 * bn, kc);
-      __builtin_amdgcn_sched_barrier(0);
-      T[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fw[c][0], fb[b][0], tc, 0, 0, 0);
+      const v16f T = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(f16x4, sw), __builtin_bit_cast(f16x4, rec), zero16, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       if (last) {
-        fw[n][1] = qx_codes<WT>(rq[NSLOT][wn][jn], 2 * bn + 1, kc);
-        sw[n].x = rs[NSLOT][wn][jn] & msk0;
+        unpack(rq[NSLOT][wn][jn], rs[NSLOT][wn][jn], bn);
       } else {
-        fw[n][1] = qx_codes<WT>(rq[SLOT][wn][jn], 2 * bn + 1, kc);
-        sw[n].x = rs[SLOT][wn][jn] & (bn ? msk1 : msk0);
-        if (bn == 1) {  // both blocks of (wn, jn) are unpacked: its ring registers are free, fetch K step kt + ST into them
-#pragma unroll
-          for (int p = 0; p < QW; p++)
-            rq[SLOT][wn][jn][p] = __builtin_amdgcn_raw_buffer_load_b128(rW[wn], kt + ST < kbs ? offQ[jn] : 0xffffffffu, ((kt + ST) * QW + p) * 1024, 0);
-          rs[SLOT][wn][jn] = __builtin_amdgcn_raw_buffer_load_b32(rW[wn], kt + ST < kbs ? offS[jn] : 0xffffffffu, (kt + ST) * 128, 0);
-        }
+        unpack(rq[SLOT][wn][jn], rs[SLOT][wn][jn], bn);
+        if (bn == 1) loadW1(SLOT, kt + ST, wn, jn);  // both blocks of (wn, jn) are unpacked: its ring registers are free
       }
       __builtin_amdgcn_sched_barrier(0);
-      S[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, sw[c]), rec[0], zero16, 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      // the FMAs of the previous group (of the previous step's last group when g == 0): first half
-      const int pg = g == 0 ? G - 1 : g - 1;
-      const int pw = (pg / TN) % NW, pj = pg % TN;
 #pragma unroll
-      for (int r = 0; r < 8; r++) acc[pw][pj][0][r] = fmaf(S[n][r], T[n][r], acc[pw][pj][0][r]);
-      asm volatile("" : "+v"(acc[pw][pj][0]));  // pins the FMAs here (the compiler otherwise sinks them to the end of the body)
-      __builtin_amdgcn_sched_barrier(0);
-      T[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fw[c][1], fb[b][1], T[c], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int r = 8; r < 16; r++) acc[pw][pj][0][r] = fmaf(S[n][r], T[n][r], acc[pw][pj][0][r]);
-      asm volatile("" : "+v"(acc[pw][pj][0]));
-      __builtin_amdgcn_sched_barrier(0);
+      for (int r = 0; r < 16; r++) acc[w][j][r] = fmaf(T[r], (float)D[r], acc[w][j][r]);
+      asm volatile("" : "+v"(acc[w][j]));  // pins the FMAs here (the compiler otherwise sinks them to the end of the body)
     }
-    storeA((SLOT & 1) ^ 1, buf ^ 1);
+    storeA(NSLOT, buf ^ 1);
     __syncthreads();
   };
   for (int kt = 0; kt < nsteps; kt += ST) {
     kstep(std::integral_constant<int, 0>{}, kt);
     kstep(std::integral_constant<int, 1>{}, kt + 1);
-    kstep(std::integral_constant<int, 2>{}, kt + 2);
-    kstep(std::integral_constant<int, 3>{}, kt + 3);
+    if constexpr (ST >= 4) {
+      kstep(std::integral_constant<int, 2>{}, kt + 2);
+      kstep(std::integral_constant<int, 3>{}, kt + 3);
+    }
   }
-  // the last group's FMAs (G even: its results are in set 1)
-#pragma unroll
-  for (int r = 0; r < 16; r++) acc[NW - 1][TN - 1][0][r] = fmaf(S[1][r], T[1][r], acc[NW - 1][TN - 1][0][r]);
 
-  // acc[w][j][i][4g+e] = result[row0 + 32i + lrow][n0 + wave*WN + 32j + 8g + 4hi + e]
+  if (QX_UNIT(WT) != 1.f) {
+#pragma unroll
+    for (int w = 0; w < NW; w++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[w][j][r] *= QX_UNIT(WT);
+  }
+  // acc[w][j][4g+e] = result[row0 + lrow][n0 + wave*WN + 32j + 8g + 4hi + e]
   if (NW == 1) {
+    if (lrow < rows) {
+      const int pos = row0 + lrow;
+      float* orow = a.out + (int64_t)(a.o_index ? a.o_index[pos] : pos) * a.N;
 #pragma unroll
-    for (int i = 0; i < TM; i++) {
-      const int r = i * 32 + lrow;
-      if (r < rows) {
-        const int pos = row0 + r;
-        float* orow = a.out + (int64_t)(a.o_index ? a.o_index[pos] : pos) * a.N;
+      for (int j = 0; j < TN; j++)
 #pragma unroll
-        for (int j = 0; j < TN; j++)
+        for (int g = 0; g < 4; g++) {
+          const int n = n0 + wave * WN + j * 32 + 8 * g + 4 * hi;
+          f32x4 v = {acc[0][j][4 * g], acc[0][j][4 * g + 1], acc[0][j][4 * g + 2], acc[0][j][4 * g + 3]};
+          if (n + 3 < a.N && a.N % 4 == 0) {
+            if (a.bias) v += *reinterpret_cast<const f32x4*>(a.bias + n);
+            *reinterpret_cast<f32x4*>(orow + n) = v;
+          } else {
 #pragma unroll
-          for (int g = 0; g < 4; g++) {
-            const int n = n0 + wave * WN + j * 32 + 8 * g + 4 * hi;
-            f32x4 v = {acc[0][j][i][4 * g], acc[0][j][i][4 * g + 1], acc[0][j][i][4 * g + 2], acc[0][j][i][4 * g + 3]};
-            if (n + 3 < a.N && a.N % 4 == 0) {
-              if (a.bias) v += *reinterpret_cast<const f32x4*>(a.bias + n);
-              *reinterpret_cast<f32x4*>(orow + n) = v;
-            } else {
-#pragma unroll
-              for (int e2 = 0; e2 < 4; e2++)
-                if (n + e2 < a.N) orow[n + e2] = a.bias ? v[e2] + a.bias[n + e2] : v[e2];
-            }
+            for (int e2 = 0; e2 < 4; e2++)
+              if (n + e2 < a.N) orow[n + e2] = a.bias ? v[e2] + a.bias[n + e2] : v[e2];
           }
-      }
+        }
     }
   } else {
     // h = silu(gate) * up, quantized to Q8_0 over each block of 32 channels (a block is one column tile j: 16 channels in
-    // this lane, 16 in lane ^ 32): codes as fp16 integers and the fp16 scale, the next Linear's activation format
+    // this lane, 16 in lane ^ 32): the next Linear's activation format
     const int nblk = a.N / QK, KDo = (a.N + 63) / 64;
 #pragma unroll
-    for (int i = 0; i < TM; i++) {
-      const int r = i * 32 + lrow;
+    for (int j = 0; j < TN; j++) {
+      float h[16];
+      float amax = 0.f;
 #pragma unroll
-      for (int j = 0; j < TN; j++) {
-        float h[16];
-        float amax = 0.f;
+      for (int q = 0; q < 16; q++) {
+        h[q] = silu_f(acc[0][j][q]) * acc[NW - 1][j][q];
+        amax = fmaxf(amax, fabsf(h[q]));
+      }
+      amax = max32(amax);
+      const float d = amax / 127.f;
+      const float idv = (amax != 0.f) ? 127.f / amax : 0.f;
+      uint16_t bits = f32_to_f16bits(d);
+      if (a.x86_scale) bits = x86_scale_bits(bits);
+      const int blk = (n0 + wave * WN) / 32 + j;
+      uint32_t p[4];  // the codes 8 g + 4 hi .. + 3
 #pragma unroll
-        for (int q = 0; q < 16; q++) {
-          h[q] = silu_f(acc[0][j][i][q]) * acc[NW - 1][j][i][q];
-          amax = fmaxf(amax, fabsf(h[q]));
-        }
-        amax = max32(amax);
-        const float d = amax / 127.f;
-        const float idv = (amax != 0.f) ? 127.f / amax : 0.f;
-        uint16_t bits = f32_to_f16bits(d);
-        if (a.x86_scale) bits = x86_scale_bits(bits);
-        const int blk = (n0 + wave * WN) / 32 + j;
-        // element 8g + 4hi + e of the block: bit 1 of its index is bit 1 of e
-        int qv[16], sa = 0, sb = 0;
+      for (int g = 0; g < 4; g++) {
+        p[g] = 0u;
 #pragma unroll
-        for (int q = 0; q < 16; q++) {
-          qv[q] = min(127, max(-128, (int)rintf(h[q] * idv)));
-          if (q & 2) sb += qv[q];
-          else sa += qv[q];
-        }
-        sa = sum32(sa);
-        sb = sum32(sb);
-        if (r < rows && blk < nblk) {
-          uint16_t* hrow = a.hq + (int64_t)(row0 + r) * a.N;
-#pragma unroll
-          for (int g = 0; g < 4; g++) {
-            const int n = n0 + wave * WN + j * 32 + 8 * g + 4 * hi;
-            uint32_t o[2];
-#pragma unroll
-            for (int e2 = 0; e2 < 2; e2++)
-              o[e2] = (uint32_t)f32_to_f16bits((float)qv[4 * g + 2 * e2]) | ((uint32_t)f32_to_f16bits((float)qv[4 * g + 2 * e2 + 1]) << 16);
-            *reinterpret_cast<uint2*>(hrow + n) = uint2{o[0], o[1]};
-          }
-          if (hi == 0) {
-            uint32_t* recp = a.hd + ((int64_t)(row0 + r) * KDo + (blk >> 1)) * 3;
-            reinterpret_cast<uint16_t*>(recp)[blk & 1] = bits;
-            recp[1 + (blk & 1)] = (uint32_t)f32_to_f16bits((float)sa) | ((uint32_t)f32_to_f16bits((float)sb) << 16);
-            if (blk == nblk - 1 && (nblk & 1)) {  // the unused half of the last record
-              reinterpret_cast<uint16_t*>(recp)[1] = 0;
-              recp[2] = 0;
-            }
-          }
+        for (int e2 = 0; e2 < 4; e2++) p[g] |= ((uint32_t)min(127, max(-128, (int)rintf(h[4 * g + e2] * idv))) & 0xffu) << (8 * e2);
+      }
+      // lane half hi takes the eights hi and 2 + hi: its own half of each and the other lane's
+      const auto r0 = __builtin_amdgcn_permlane32_swap(p[0], p[1], false, false);
+      const auto r1 = __builtin_amdgcn_permlane32_swap(p[2], p[3], false, false);
+      const u32x2 o0 = qx_order<WT>(r0[0], r0[1]), o1 = qx_order<WT>(r1[0], r1[1]);
+      if (lrow < rows && blk < nblk) {
+        *reinterpret_cast<u32x4*>(a.hq + (int64_t)(row0 + lrow) * a.N + blk * 32 + hi * 16) = u32x4{o0.x, o0.y, o1.x, o1.y};
+        if (hi == 0) {
+          uint16_t* hd = reinterpret_cast<uint16_t*>(a.hd + (int64_t)(row0 + lrow) * KDo);
+          hd[blk] = bits;
+          if (blk == nblk - 1 && (nblk & 1)) hd[blk + 1] = 0;  // the unused half of the last dword
         }
       }
     }
@@ -1423,51 +1332,45 @@ __device__ __forceinline__ void qx_tile(const QXArgs& a, const int e, const int 
 }
 
 
-// The same tile for at most SIXTEEN sorted positions: v_mfma_f32_16x16x32_f16 takes a whole block of 32 elements per
-// instruction for 16 channels x 16 rows, so a tile of up to 16 rows costs half the matrix time (and half the FMAs) of the
-// 32-row form above, which would pad it to 32.  Same packed weights: a lane of the 32-row layout holds, of channel lane % 32,
-// the block's elements 8 hi .. 8 hi + 7 (MFMA step 0) and 16 + 8 hi .. (step 1); the 16-row operand wants, in lane
-// (channel c, K group kg), eight elements of channel c [+ 16].  v_permlane16_swap on the PACKED dwords (step 0 as first
-// operand, step 1 as second) leaves in the first the channels 0..15 and in the second the channels 16..31, each with K
-// groups (hi 0, step 0), (hi 0, step 1), (hi 1, step 0), (hi 1, step 1); the activation operand is read from LDS in that
-// order of K, so the products that meet are the same and every sum is the same exact integer.  Same scale products,
-// same FMAs per block, same order of blocks: the same bits as the 32-row form row by row.
+// The same tile for at most SIXTEEN sorted positions: v_mfma_i32_16x16x32_i8 takes a block of 16 channels x 16 rows, so a tile of
+// up to 16 rows costs half the matrix time (and half the FMAs) of the 32-row form above, which would pad it to 32.  Same packed
+// weights: a lane of the 32-row layout holds, of channel lane % 32, the block's elements 8 hi .. 8 hi + 7 (first dword, or two)
+// and 16 + 8 hi .. (second); the 16-row operand wants, in lane (channel c, K group kg), eight elements of channel c [+ 16].
+// v_permlane16_swap on the PACKED dwords (first eight as first operand, second as second) leaves in the first the channels 0..15
+// and in the second the channels 16..31, each with the K groups (hi 0, first), (hi 0, second), (hi 1, first), (hi 1, second): bytes
+// 8 kg .. 8 kg + 7 of the stored activation block.  The products that meet are the same and every sum is the same exact integer.
+// Same scale products, same FMAs per block, same order of blocks: the same bits as the 32-row form row by row.
 template <int WT, int NW, int TN>
 __device__ __forceinline__ void qx_tile16(const QXArgs& a, const int e, const int row0, const int rows, const int n0,
                                           unsigned char* smem) {
-  constexpr int BK = 64, LDK = 2 * BK + 16;
+  constexpr int BK = 64, LDK = BK + 16;
   constexpr int BM = 16, WN = TN * 32;
-  constexpr int STAGE = BM * LDK + BM * 48;
+  constexpr int STAGE = BM * LDK + BM * 4;
   constexpr int QW = WT == MLLM_HIP_Q4_0 ? 1 : 2;
-  constexpr int ST = 4;  // K steps of weights in flight per wave
+  constexpr int ST = QX_ST16(WT);  // K steps of weights in flight per wave
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int lrow = lane & 31;             // channel of this lane in the packed layout
+  const int lrow = lane & 31;                 // channel of this lane in the packed layout
   const int c16 = lane & 15, kg = lane >> 4;  // 16-row operands: channel / row c16, K group kg
   const int Kp = (int)qg_kp(a.K), kbs = Kp / 64, nbs = (int)(qg_np(a.N) / 32), KD = (a.K + 63) / 64;
   const int64_t qbytes = qg_qbytes(WT, a.N, a.K), wbytes = qg_bytes(WT, a.N, a.K);
 
-  const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.xq), 0, (uint32_t)((int64_t)a.a_rows * a.K * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rD = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.xd), 0, (uint32_t)((int64_t)a.a_rows * KD * 12), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.xq), 0, (uint32_t)((int64_t)a.a_rows * a.K), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rD = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(a.xd), 0, (uint32_t)((int64_t)a.a_rows * KD * 4), 0x00020000);
   __amdgpu_buffer_rsrc_t rW[NW];
   rW[0] = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.W0 + (size_t)e * a.wstride), 0, (uint32_t)wbytes, 0x00020000);
   if (NW == 2) rW[NW - 1] = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(a.W1 + (size_t)e * a.wstride), 0, (uint32_t)wbytes, 0x00020000);
 
-  // activation chunk of threads 0 .. 127: tile row tid / 8, 16-byte column tid % 8; record of a row: threads 0 .. 15.
+  // activations of threads 0 .. 127: tile row tid / 8, eight codes from 8 (tid % 8); scales of a row: threads 0 .. 15.
   // Rows past `rows` repeat the last one (never stored); columns past K read as zeros.
   const bool ldA = tid < BM * 8;
   const int colA = (tid % 8) * 8;
-  uint32_t offA = 0xffffffffu, offD = 0xffffffffu;
-  if (ldA) {
-    const int pos = row0 + min(tid / 8, rows - 1);
-    const int arow = a.a_index ? a.a_index[pos] / a.a_div : pos;
-    offA = (uint32_t)(((int64_t)arow * a.K + colA) * 2);
-  }
-  if (tid < BM) {
-    const int pos = row0 + min(tid, rows - 1);
-    const int arow = a.a_index ? a.a_index[pos] / a.a_div : pos;
-    offD = (uint32_t)((int64_t)arow * KD * 12);
-  }
+  auto arow_of = [&](int r) -> uint32_t {
+    const int pos = row0 + min(r, rows - 1);
+    return (uint32_t)(a.a_index ? a.a_index[pos] / a.a_div : pos);
+  };
+  const uint32_t offA = ldA ? arow_of(tid / 8) * (uint32_t)a.K + colA : 0xffffffffu;
+  const uint32_t offD = tid < BM ? arow_of(tid) * (uint32_t)(KD * 4) : 0xffffffffu;
   uint32_t offQ[TN], offS[TN];
 #pragma unroll
   for (int j = 0; j < TN; j++) {
@@ -1475,21 +1378,15 @@ __device__ __forceinline__ void qx_tile16(const QXArgs& a, const int e, const in
     offQ[j] = (uint32_t)((int64_t)nb * kbs * (1024 * QW) + lane * 16);
     offS[j] = (uint32_t)(qbytes + ((int64_t)nb * kbs * 32 + lrow) * 4);
   }
-  typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
-  u32x4 ga[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
-  u32x3 gd[2] = {{0u, 0u, 0u}, {0u, 0u, 0u}};
-  auto loadA = [&](int set, int kt) {  // two K steps ahead of their use, as in the 32-row form
-    if (ldA) ga[set] = __builtin_amdgcn_raw_buffer_load_b128(rA, kt * BK + colA < a.K ? offA : 0xffffffffu, kt * BK * 2, 0);
-    if (tid < BM) gd[set] = __builtin_amdgcn_raw_buffer_load_b96(rD, kt < KD ? offD : 0xffffffffu, kt * 12, 0);
+  u32x2 ga[ST] = {};
+  uint32_t gd[ST] = {};
+  auto loadA = [&](int set, int kt) {  // as far ahead as the weights, as in the 32-row form
+    if (ldA) ga[set] = __builtin_amdgcn_raw_buffer_load_b64(rA, kt * BK + colA < a.K ? offA : 0xffffffffu, kt * BK, 0);
+    if (tid < BM) gd[set] = __builtin_amdgcn_raw_buffer_load_b32(rD, kt < KD ? offD : 0xffffffffu, kt * 4, 0);
   };
   auto storeA = [&](int set, int buf) {
-    if (ldA) *reinterpret_cast<u32x4*>(smem + buf * STAGE + (tid / 8) * LDK + (tid % 8) * 16) = ga[set];
-    if (tid < BM) {
-      u32x4* rec = reinterpret_cast<u32x4*>(smem + buf * STAGE + BM * LDK + tid * 48);
-      rec[0] = u32x4{gd[set].x, 0u, 0u, 0u};
-      rec[1] = u32x4{gd[set].y, 0u, 0u, 0u};
-      rec[2] = u32x4{gd[set].z, 0u, 0u, 0u};
-    }
+    if (ldA) *reinterpret_cast<u32x2*>(smem + buf * STAGE + (tid / 8) * LDK + colA) = ga[set];
+    if (tid < BM) *reinterpret_cast<uint32_t*>(smem + buf * STAGE + BM * LDK + tid * 4) = gd[set];
   };
 
   f32x4 acc[NW][TN][2];  // [matrix][column tile][channel half]
@@ -1502,38 +1399,35 @@ __device__ __forceinline__ void qx_tile16(const QXArgs& a, const int e, const in
 
   u32x4 rq[ST][NW][TN][QW];
   uint32_t rs[ST][NW][TN];
-  auto loadW = [&](int slot, int kt) {
-    const bool ok = kt < kbs;
+  auto loadW1 = [&](int slot, int kt, int w, int j) {
 #pragma unroll
-    for (int w = 0; w < NW; w++)
-#pragma unroll
-      for (int j = 0; j < TN; j++) {
-#pragma unroll
-        for (int p = 0; p < QW; p++)
-          rq[slot][w][j][p] = __builtin_amdgcn_raw_buffer_load_b128(rW[w], ok ? offQ[j] : 0xffffffffu, (kt * QW + p) * 1024, 0);
-        rs[slot][w][j] = __builtin_amdgcn_raw_buffer_load_b32(rW[w], ok ? offS[j] : 0xffffffffu, kt * 128, 0);
-      }
+    for (int p = 0; p < QW; p++)
+      rq[slot][w][j][p] = __builtin_amdgcn_raw_buffer_load_b128(rW[w], kt < kbs ? offQ[j] : 0xffffffffu, (kt * QW + p) * 1024, 0);
+    rs[slot][w][j] = __builtin_amdgcn_raw_buffer_load_b32(rW[w], kt < kbs ? offS[j] : 0xffffffffu, kt * 128, 0);
   };
   // scale operands: the fp16 scale of the step's first block in K slot 0, of its second block in K slot 1, in the lanes of K
   // group 0; everything else zero
   const uint32_t msk0 = kg ? 0u : 0x0000ffffu, msk1 = kg ? 0u : 0xffff0000u;
   const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
-  const QXConst kc = qx_const(WT);
-  const f16x8 off_op = __builtin_bit_cast(f16x8, u32x4{kg ? 0u : qx_offsets(WT), 0u, 0u, 0u});
+  const v4i izero = {};
+  const QXConst kc = qx_const();
 
   // the operands of one (block, matrix, column tile) from the packed registers: codes of the channels 0..15 | 16..31
-  auto unpack = [&](const u32x4 (&q)[QW], int b, f16x8 (&fw)[2]) {
+  auto unpack = [&](const u32x4 (&q)[QW], int b, int64_t (&fw)[2]) {
+    u32x2 o[2];
     if (WT == MLLM_HIP_Q4_0) {
       const auto r = __builtin_amdgcn_permlane16_swap(q[0][2 * b], q[0][2 * b + 1], false, false);
-      fw[0] = qx_codes_dw<WT>(r[0], 0u, kc);
-      fw[1] = qx_codes_dw<WT>(r[1], 0u, kc);
+#pragma unroll
+      for (int h = 0; h < 2; h++) o[h] = u32x2{qx_low(r[h], kc), qx_high(r[h], kc)};
     } else {
-      // block b: steps 2b (dwords 0, 1 of register b) and 2b + 1 (dwords 2, 3)
+      // block b: first eight in dwords 0, 1 of register b, second in 2, 3
       const auto r0 = __builtin_amdgcn_permlane16_swap(q[QW - 1 ? b : 0][0], q[QW - 1 ? b : 0][2], false, false);
       const auto r1 = __builtin_amdgcn_permlane16_swap(q[QW - 1 ? b : 0][1], q[QW - 1 ? b : 0][3], false, false);
-      fw[0] = qx_codes_dw<WT>(r0[0], r1[0], kc);
-      fw[1] = qx_codes_dw<WT>(r0[1], r1[1], kc);
+#pragma unroll
+      for (int h = 0; h < 2; h++) o[h] = u32x2{r0[h], r1[h]};
     }
+#pragma unroll
+    for (int h = 0; h < 2; h++) fw[h] = __builtin_bit_cast(int64_t, o[h]);
   };
   auto scales = [&](uint32_t s, int b, u32x4 (&sw)[2]) {
     const uint32_t up = __builtin_amdgcn_permlane16_swap(s, s, false, false)[1];  // lanes 0..15 <- lanes 16..31
@@ -1543,16 +1437,20 @@ __device__ __forceinline__ void qx_tile16(const QXArgs& a, const int e, const in
   };
 
   constexpr int G = 2 * NW * TN;  // groups per K step: block-major, then matrix, then column tile
-  f16x8 fw[2][2];                 // [current | next group][channel half]
+  int64_t fw[2][2];               // [current | next group][channel half]
   u32x4 sw[2][2] = {{{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}}, {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}}};
-  f32x4 T[2][2], S[2][2];         // block sums and scale products of the current / previous group
-  T[1][0] = T[1][1] = S[1][0] = S[1][1] = zero4;
+  u32x4 rec = {0u, 0u, 0u, 0u};
+  asm("" : "+v"(sw[0][0]), "+v"(sw[0][1]), "+v"(sw[1][0]), "+v"(sw[1][1]), "+v"(rec));
 
   const int nsteps = (kbs + ST - 1) / ST * ST;
-  loadA(0, 0);
-  loadA(1, 1);
 #pragma unroll
-  for (int s = 0; s < ST; s++) loadW(s, s);
+  for (int s = 0; s < ST; s++) {
+    loadA(s, s);
+#pragma unroll
+    for (int w = 0; w < NW; w++)
+#pragma unroll
+      for (int j = 0; j < TN; j++) loadW1(s, s, w, j);
+  }
   storeA(0, 0);
   unpack(rq[0][0][0], 0, fw[0]);
   scales(rs[0][0][0], 0, sw[0]);
@@ -1562,75 +1460,61 @@ __device__ __forceinline__ void qx_tile16(const QXArgs& a, const int e, const in
     constexpr int SLOT = decltype(slot_tag)::value;
     constexpr int NSLOT = (SLOT + 1) % ST;
     const int buf = kt & 1;
-    loadA(SLOT & 1, kt + 2);
-    f16x8 fb[2];
+    loadA(SLOT, kt + ST);
+    int64_t fb[2];
 #pragma unroll
-    for (int b = 0; b < 2; b++)
-      fb[b] = *reinterpret_cast<const f16x8*>(smem + buf * STAGE + c16 * LDK + (2 * b + (kg & 1)) * 32 + (kg >> 1) * 16);
-    f16x8 rec[3];
-#pragma unroll
-    for (int q = 0; q < 3; q++) rec[q] = *reinterpret_cast<const f16x8*>(smem + buf * STAGE + BM * LDK + c16 * 48 + q * 16);
-    f32x4 tc = zero4;
+    for (int b = 0; b < 2; b++) fb[b] = *reinterpret_cast<const int64_t*>(smem + buf * STAGE + c16 * LDK + b * 32 + kg * 8);
+    rec.x = *reinterpret_cast<const uint32_t*>(smem + buf * STAGE + BM * LDK + c16 * 4);
 #pragma unroll
     for (int g = 0; g < G; g++) {
       const int c = g & 1, n = c ^ 1;  // the register sets alternate (G is even)
-      const int b = g / (NW * TN);
+      const int b = g / (NW * TN), w = (g / TN) % NW, j = g % TN;
       const bool last = g == G - 1;
       const int gn = last ? 0 : g + 1;
       const int bn = gn / (NW * TN), wn = (gn / TN) % NW, jn = gn % TN;
-      const int pg = g == 0 ? G - 1 : g - 1;
-      const int pw = (pg / TN) % NW, pj = pg % TN;
+      v4i D[2];
+      f32x4 T[2];
       __builtin_amdgcn_sched_barrier(0);
-      if (g % (NW * TN) == 0) tc = __builtin_amdgcn_mfma_f32_16x16x32_f16(off_op, rec[1 + b], zero4, 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if (last) unpack(rq[NSLOT][wn][jn], bn, fw[n]);
-      else unpack(rq[SLOT][wn][jn], bn, fw[n]);
-      __builtin_amdgcn_sched_barrier(0);
-      T[c][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[c][0], fb[b], tc, 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      S[c][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, sw[c][0]), rec[0], zero4, 0, 0, 0);
+#pragma unroll
+      for (int h = 0; h < 2; h++) D[h] = __builtin_amdgcn_mfma_i32_16x16x32_i8(fw[c][h], fb[b], izero, 0, 0, 0);
+#pragma unroll
+      for (int h = 0; h < 2; h++) T[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, sw[c][h]), __builtin_bit_cast(f16x8, rec), zero4, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       if (last) {
+        unpack(rq[NSLOT][wn][jn], bn, fw[n]);
         scales(rs[NSLOT][wn][jn], bn, sw[n]);
       } else {
+        unpack(rq[SLOT][wn][jn], bn, fw[n]);
         scales(rs[SLOT][wn][jn], bn, sw[n]);
-        if (bn == 1) {  // both blocks of (wn, jn) are unpacked: fetch K step kt + ST into its ring registers
-#pragma unroll
-          for (int p = 0; p < QW; p++)
-            rq[SLOT][wn][jn][p] = __builtin_amdgcn_raw_buffer_load_b128(rW[wn], kt + ST < kbs ? offQ[jn] : 0xffffffffu, ((kt + ST) * QW + p) * 1024, 0);
-          rs[SLOT][wn][jn] = __builtin_amdgcn_raw_buffer_load_b32(rW[wn], kt + ST < kbs ? offS[jn] : 0xffffffffu, (kt + ST) * 128, 0);
-        }
+        if (bn == 1) loadW1(SLOT, kt + ST, wn, jn);  // both blocks of (wn, jn) are unpacked
       }
       __builtin_amdgcn_sched_barrier(0);
-      T[c][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fw[c][1], fb[b], tc, 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      // the FMAs of the previous group (of the previous step's last group when g == 0)
 #pragma unroll
-      for (int r = 0; r < 4; r++) acc[pw][pj][0][r] = fmaf(S[n][0][r], T[n][0][r], acc[pw][pj][0][r]);
-      asm volatile("" : "+v"(acc[pw][pj][0]));
-      __builtin_amdgcn_sched_barrier(0);
-      S[c][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, sw[c][1]), rec[0], zero4, 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int h = 0; h < 2; h++)
 #pragma unroll
-      for (int r = 0; r < 4; r++) acc[pw][pj][1][r] = fmaf(S[n][1][r], T[n][1][r], acc[pw][pj][1][r]);
-      asm volatile("" : "+v"(acc[pw][pj][1]));
-      __builtin_amdgcn_sched_barrier(0);
+        for (int r = 0; r < 4; r++) acc[w][j][h][r] = fmaf(T[h][r], (float)D[h][r], acc[w][j][h][r]);
+      asm volatile("" : "+v"(acc[w][j][0]), "+v"(acc[w][j][1]));
     }
-    storeA((SLOT & 1) ^ 1, buf ^ 1);
+    storeA(NSLOT, buf ^ 1);
     __syncthreads();
   };
   for (int kt = 0; kt < nsteps; kt += ST) {
     kstep(std::integral_constant<int, 0>{}, kt);
     kstep(std::integral_constant<int, 1>{}, kt + 1);
-    kstep(std::integral_constant<int, 2>{}, kt + 2);
-    kstep(std::integral_constant<int, 3>{}, kt + 3);
+    if constexpr (ST >= 4) {
+      kstep(std::integral_constant<int, 2>{}, kt + 2);
+      kstep(std::integral_constant<int, 3>{}, kt + 3);
+    }
   }
-  // the last group's FMAs (G even: its results are in set 1)
-#pragma unroll
-  for (int h = 0; h < 2; h++)
-#pragma unroll
-    for (int r = 0; r < 4; r++) acc[NW - 1][TN - 1][h][r] = fmaf(S[1][h][r], T[1][h][r], acc[NW - 1][TN - 1][h][r]);
 
+  if (QX_UNIT(WT) != 1.f) {
+#pragma unroll
+    for (int w = 0; w < NW; w++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) acc[w][j][h] *= QX_UNIT(WT);
+  }
   // acc[w][j][h][e] = result[row0 + c16][n0 + wave*WN + 32j + 16h + 4kg + e]
   if (NW == 1) {
     if (c16 < rows) {
@@ -1672,37 +1556,22 @@ __device__ __forceinline__ void qx_tile16(const QXArgs& a, const int e, const in
       uint16_t bits = f32_to_f16bits(d);
       if (a.x86_scale) bits = x86_scale_bits(bits);
       const int blk = (n0 + wave * WN) / 32 + j;
-      // element 16h + 4kg + e of the block: bit 1 of its index is bit 1 of e
-      int qv[8], sa = 0, sb = 0;
+      uint32_t p[2];  // the codes 16 h + 4 kg .. + 3
 #pragma unroll
-      for (int q = 0; q < 8; q++) {
-        qv[q] = min(127, max(-128, (int)rintf(hv[q] * idv)));
-        if (q & 2) sb += qv[q];
-        else sa += qv[q];
+      for (int h = 0; h < 2; h++) {
+        p[h] = 0u;
+#pragma unroll
+        for (int e2 = 0; e2 < 4; e2++) p[h] |= ((uint32_t)min(127, max(-128, (int)rintf(hv[4 * h + e2] * idv))) & 0xffu) << (8 * e2);
       }
-      sa = sum16(sa);
-      sa = sum32(sa);
-      sb = sum16(sb);
-      sb = sum32(sb);
+      // K group kg takes the eight 2 (kg % 2) + kg / 2: its own half and the half of the lane sixteen away
+      const auto r = __builtin_amdgcn_permlane16_swap(p[0], p[1], false, false);
+      const u32x2 o = qx_order<WT>(r[0], r[1]);
       if (c16 < rows && blk < nblk) {
-        uint16_t* hrow = a.hq + (int64_t)(row0 + c16) * a.N;
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-          const int n = n0 + wave * WN + j * 32 + 16 * h + 4 * kg;
-          uint32_t o[2];
-#pragma unroll
-          for (int e2 = 0; e2 < 2; e2++)
-            o[e2] = (uint32_t)f32_to_f16bits((float)qv[4 * h + 2 * e2]) | ((uint32_t)f32_to_f16bits((float)qv[4 * h + 2 * e2 + 1]) << 16);
-          *reinterpret_cast<uint2*>(hrow + n) = uint2{o[0], o[1]};
-        }
+        *reinterpret_cast<u32x2*>(a.hq + (int64_t)(row0 + c16) * a.N + blk * 32 + (kg >> 1) * 16 + (kg & 1) * 8) = o;
         if (kg == 0) {
-          uint32_t* recp = a.hd + ((int64_t)(row0 + c16) * KDo + (blk >> 1)) * 3;
-          reinterpret_cast<uint16_t*>(recp)[blk & 1] = bits;
-          recp[1 + (blk & 1)] = (uint32_t)f32_to_f16bits((float)sa) | ((uint32_t)f32_to_f16bits((float)sb) << 16);
-          if (blk == nblk - 1 && (nblk & 1)) {  // the unused half of the last record
-            reinterpret_cast<uint16_t*>(recp)[1] = 0;
-            recp[2] = 0;
-          }
+          uint16_t* hd = reinterpret_cast<uint16_t*>(a.hd + (int64_t)(row0 + c16) * KDo);
+          hd[blk] = bits;
+          if (blk == nblk - 1 && (nblk & 1)) hd[blk + 1] = 0;  // the unused half of the last dword
         }
       }
     }
@@ -1714,7 +1583,7 @@ constexpr int QX_DOWN_TN = 2;  // column tiles per wave in the one-matrix mode
 constexpr int QX_GROUP = 8;    // tiles per group of work items (see qx_kernel)
 // MODE 0: one matrix, up to 32 rows x 256 channels per workgroup.  MODE 1: gate and up together, 32 rows x 128 channels.
 template <int WT, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void qx_kernel(QXArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void qx_kernel(QXArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   // Work items in groups of QX_GROUP tiles (list order: an expert's tiles are neighbours) x all column blocks, inside a
   // group the tile index fastest.  Workgroup L runs on XCD L % 8, and every XCD has its own L2: XCD x takes a contiguous
@@ -1735,11 +1604,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if constexpr (MODE == 1) {
     const int n0 = by * 128;
     if (rows <= 16 && a.half_tiles) qx_tile16<WT, 2, 1>(a, e, row0, rows, n0, smem);
-    else qx_tile<WT, 2, 1, 1>(a, e, row0, rows, n0, smem);
+    else qx_tile<WT, 2, 1>(a, e, row0, rows, n0, smem);
   } else {
     const int n0 = by * (128 * QX_DOWN_TN);
     if (rows <= 16 && a.half_tiles) qx_tile16<WT, 1, QX_DOWN_TN>(a, e, row0, rows, n0, smem);
-    else qx_tile<WT, 1, 1, QX_DOWN_TN>(a, e, row0, rows, n0, smem);
+    else qx_tile<WT, 1, QX_DOWN_TN>(a, e, row0, rows, n0, smem);
   }
 }
 
@@ -1749,16 +1618,16 @@ template <int MODE>
 static int launch_qx(int wtype, const QXArgs& a, unsigned max_tiles, hipStream_t st) {
   const int wg_n = MODE == 1 ? 128 : 128 * QX_DOWN_TN;
   const dim3 grid(max_tiles, (unsigned)((a.N + wg_n - 1) / wg_n));
-  const size_t lds = 2 * (size_t)(QX_TILE_H * (2 * 64 + 16) + QX_TILE_H * 48);
+  const size_t lds = 2 * (size_t)(QX_TILE_H * (64 + 16) + QX_TILE_H * 4);
   if (wtype == MLLM_HIP_Q4_0) hipLaunchKernelGGL((qx_kernel<MLLM_HIP_Q4_0, MODE>), grid, dim3(256), lds, st, a);
   else hipLaunchKernelGGL((qx_kernel<MLLM_HIP_Q8_0, MODE>), grid, dim3(256), lds, st, a);
   return (int)hipGetLastError();
 }
 
-// activations for the kernel above: Q8_0 quantization (bit-exact codes and scale); codes as fp16 integers, and per row and K
-// step of 64 a record of three dwords: the two blocks' fp16 scales, then per block the code sums over the elements with
-// bit 1 of k clear | set, as fp16 integers (at most 16 x 127 each: exact).  The second half of a last, incomplete record is zero.
-__device__ __forceinline__ void qx_act_block(const void* __restrict__ x, int x_dtype, uint16_t* __restrict__ xq, uint32_t* __restrict__ xd,
+// activations for the kernel above: Q8_0 quantization (bit-exact codes and scale), a block's codes in QX_ORDER, the scales of two
+// blocks per dword (the second half of a last, incomplete one is zero)
+template <int WT>
+__device__ __forceinline__ void qx_act_block(const void* __restrict__ x, int x_dtype, uint8_t* __restrict__ xq, uint32_t* __restrict__ xd,
                                              int64_t i, int nb, int x86_scale) {
   float v[32];
   uint32_t q[8];
@@ -1766,32 +1635,23 @@ __device__ __forceinline__ void qx_act_block(const void* __restrict__ x, int x_d
   load_block_f32(x, x_dtype, i * QK, v);
   uint16_t bits = quantize_block_q8_0(v, q, sum);
   if (x86_scale) bits = x86_scale_bits(bits);
-  uint32_t o[16];
-  int sa = 0, sb = 0;
-#pragma unroll
-  for (int j = 0; j < 16; j++) {  // elements 2j, 2j+1
-    const int c0 = (int8_t)(q[j / 2] >> (16 * (j & 1))), c1 = (int8_t)(q[j / 2] >> (16 * (j & 1) + 8));
-    o[j] = (uint32_t)f32_to_f16bits((float)c0) | ((uint32_t)f32_to_f16bits((float)c1) << 16);
-    if (j & 1) sb += c0 + c1;
-    else sa += c0 + c1;
-  }
   u32x4* out = reinterpret_cast<u32x4*>(xq + i * QK);
 #pragma unroll
-  for (int j = 0; j < 4; j++) out[j] = u32x4{o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]};
+  for (int h = 0; h < 2; h++) {
+    const u32x2 lo = qx_order<WT>(q[2 * h], q[2 * h + 1]), hi = qx_order<WT>(q[4 + 2 * h], q[5 + 2 * h]);
+    out[h] = u32x4{lo.x, lo.y, hi.x, hi.y};
+  }
   const int64_t row = i / nb;
   const int b = (int)(i - row * nb), KD = (nb + 1) / 2;
-  uint32_t* rec = xd + (row * KD + (b >> 1)) * 3;
-  reinterpret_cast<uint16_t*>(rec)[b & 1] = bits;
-  rec[1 + (b & 1)] = (uint32_t)f32_to_f16bits((float)sa) | ((uint32_t)f32_to_f16bits((float)sb) << 16);
-  if (b == nb - 1 && (nb & 1)) {
-    reinterpret_cast<uint16_t*>(rec)[1] = 0;
-    rec[2] = 0;
-  }
+  uint16_t* rec = reinterpret_cast<uint16_t*>(xd + row * KD);
+  rec[b] = bits;
+  if (b == nb - 1 && (nb & 1)) rec[b + 1] = 0;
 }
 
 // the two independent preparations of the grouped FFN in one launch: workgroup 0 routes, the others quantize x
+template <int WT>
 __global__ __launch_bounds__(1024) void qx_prepare_kernel(const int32_t* __restrict__ ids, int n, int E, int tile_h, RouteOut o,
-                                                          const void* __restrict__ x, int x_dtype, uint16_t* __restrict__ xq,
+                                                          const void* __restrict__ x, int x_dtype, uint8_t* __restrict__ xq,
                                                           uint32_t* __restrict__ xd, int64_t nblocks, int nb, int x86_scale) {
   extern __shared__ int s_route[];
   if (blockIdx.x == 0) {
@@ -1799,7 +1659,7 @@ __global__ __launch_bounds__(1024) void qx_prepare_kernel(const int32_t* __restr
     return;
   }
   const int64_t i = (int64_t)(blockIdx.x - 1) * 1024 + threadIdx.x;
-  if (i < nblocks) qx_act_block(x, x_dtype, xq, xd, i, nb, x86_scale);
+  if (i < nblocks) qx_act_block<WT>(x, x_dtype, xq, xd, i, nb, x86_scale);
 }
 
 // y[t][h] = sum_j per[t*k + j][h] * w[t][j]   (multiply, then add in j order: modeling_qwen3_moe_fa2.hpp:233-236)
@@ -2386,19 +2246,19 @@ MLLM_API int mllm_hip_linear_q_gemm_short(int wtype, const void* gemm_packed, co
 
 namespace mllmhip {
 struct QXCarve {
-  uint16_t* xq;
+  uint8_t* xq;
   uint32_t* xd;
-  uint16_t* hq;
+  uint8_t* hq;
   uint32_t* hd;
   float* per;
   RouteOut ro;
 };
 static QXCarve carve_qx(Carver& c, int64_t T, int64_t H, int64_t I, int E, int k) {
   QXCarve r;
-  r.xq = c.take<uint16_t>((size_t)T * H);
-  r.xd = c.take<uint32_t>((size_t)T * 3 * ((H + 63) / 64));
-  r.hq = c.take<uint16_t>((size_t)T * k * I);
-  r.hd = c.take<uint32_t>((size_t)T * k * 3 * ((I + 63) / 64));
+  r.xq = c.take<uint8_t>((size_t)T * H);
+  r.xd = c.take<uint32_t>((size_t)T * ((H + 63) / 64));
+  r.hq = c.take<uint8_t>((size_t)T * k * I);
+  r.hd = c.take<uint32_t>((size_t)T * k * ((I + 63) / 64));
   r.per = c.take<float>((size_t)T * k * H);
   r.ro = carve_route(c, E, T * k, QX_TILE_H);
   return r;
@@ -2424,7 +2284,8 @@ static int moe_ffn_qx(int wtype, const void* gate_packed, const void* up_packed,
   const unsigned max_tiles = (unsigned)(E + (T * k) / QX_TILE_H + 1);
   if (E > MOE_MAX_EXPERTS) return MLLM_HIP_E_SHAPE;
   const int64_t nblocks = T * (H / QK);
-  hipLaunchKernelGGL(qx_prepare_kernel, dim3((unsigned)(1 + (nblocks + 1023) / 1024)), dim3(1024), 5 * (size_t)E * sizeof(int), st,
+  const auto prepare = wtype == MLLM_HIP_Q4_0 ? qx_prepare_kernel<MLLM_HIP_Q4_0> : qx_prepare_kernel<MLLM_HIP_Q8_0>;
+  hipLaunchKernelGGL(prepare, dim3((unsigned)(1 + (nblocks + 1023) / 1024)), dim3(1024), 5 * (size_t)E * sizeof(int), st,
                      topk_ids, (int)(T * k), E, QX_TILE_H, w.ro, x, x_dtype, w.xq, w.xd, nblocks, (int)(H / QK), x86);
   HIP_RET(hipGetLastError());
   QXArgs a{};

@@ -316,6 +316,43 @@ def test_moe_gemm_small(T, H, I, E, k, wtype):
     assert L.mllm_hip_moe_gemm_set_path(3) == -1
 
 
+@pytest.mark.parametrize("wtype", [0, 1])
+@pytest.mark.parametrize("T,H,I", [(33, 64, 32), (50, 160, 96), (49, 384, 320)])
+def test_moe_gemm_largest_codes(T, H, I, wtype):
+    """Every weight code at an end of its range (Q4_0: -8 and 7, Q8_0: -128 and 127) against activations of one magnitude (codes +-127):
+    the largest block sums, in the 16-row and the 32-row form, with K of one, two and three steps of 128 elements and odd block
+    counts.  Signs of x and of a channel's weights agree in half of the channels, so that whole blocks add up."""
+    rng = synth.rng_for(4, 9000 + T + H + I + wtype)
+    E, k = 3, 2
+    sign = np.where(rng.random(H) < 0.5, 1.0, -1.0).astype(np.float32)
+
+    def weights(n, kk, s):
+        W = synth.make_weight(rng, wtype, E * n, kk)
+        aligned = rng.random((E * n, 1)) < 0.5
+        positive = np.where(aligned, s[None, :] > 0, rng.random((E * n, kk)) < 0.5).reshape(E * n, kk // 32, 32)
+        if wtype == 0:
+            q = np.where(positive, 15, 0).astype(np.uint8)
+            W[..., 2:] = q[..., :16] | (q[..., 16:] << 4)
+        else:
+            W[..., 2:] = np.where(positive, 127, -128).astype(np.int8).view(np.uint8)
+        return W.reshape(E, n, kk // 32, -1)
+
+    Wg, Wu, Wd = weights(I, H, sign), weights(I, H, sign), weights(H, I, np.ones(I, np.float32))
+    ids, w = synth.make_moe_routing(rng, T, E, k)
+    x = (sign[None, :] * np.exp2(rng.integers(-3, 1, (T, 1)))).astype(np.float32)
+    g, u, d = (ql.PackedExperts(wtype, torch.from_numpy(m), layout="gemm") for m in (Wg, Wu, Wd))
+    want = orc.moe_ffn(x, ids, w, Wg, Wu, Wd, wtype)
+    announce("moe gemm largest codes", T, H, I, wtype)
+    y = ql.moe_ffn_q_gemm(g, u, d, to_dev(x), to_dev(ids), to_dev(w)).cpu().numpy()
+    assert rel_l2(y, want) < 2e-4, rel_l2(y, want)  # as test_moe_gemm_small
+    try:
+        assert _lib.lib().mllm_hip_moe_gemm_set_path(2) == 0
+        y32 = ql.moe_ffn_q_gemm(g, u, d, to_dev(x), to_dev(ids), to_dev(w)).cpu().numpy()
+    finally:
+        _lib.lib().mllm_hip_moe_gemm_set_path(0)
+    assert np.array_equal(y32, y)
+
+
 def test_moe_gemm_exact_form_is_the_block_arithmetic():
     """Form 0 against the block-dot kernels of mllm_hip_moe_ffn_q on the same inputs: both compute
     sum_b fp32(dW * dX) * float(int32 block sum) with exact block sums, so they differ by fp32 summation order only; and a
