@@ -312,8 +312,10 @@ __global__ __launch_bounds__(256, (TM * TN == 4 && DT != MLLM_HIP_F32) ? 4 : 1) 
 // Bound by the matrix pipe at the clock it holds under this load, by LDS reads (nine 16-byte reads per sixteen instructions; a wave tile of 32 x
 // 64) and by the splitting (six vector instructions per element), which share the issue slots; the matrix instructions alone take 23 us per 128 k of
 // 8 x 3072 x 768, the fp32 ones 45.  K steps of sixteen in two LDS buffers, one barrier each; one (large tile, two accumulators) to four workgroups
-// per CU.  One LDS buffer with steps of 32, operands read a step ahead, and tiles of 64 x 128 with four waves were no faster.
-//   8 x 3108 x 777 x 128 (scores): 61 -> 55 us, x 128 x 777 (values): 61.5 -> 48; 8 x 4096 x 1024 x 128: 85 -> 80
+// per CU.  On the large tile three of the splitting's instructions follow each matrix instruction: in front of them all, they took their time alone,
+// two waves per SIMD or not (8 x 3108 x 128 x 777: 50 -> 43 us, 2048 x 2048 x 2048 131 -> 112; on the small one, bound by LDS reads at 64 bytes
+// per clock, nothing).  Waves of 64 x 64 read less (4096 x 4096 x 1024 233 -> 220) but have 256 registers and, one per SIMD, nothing beside them (8 x 3108 x 128 x 777: 48).  One LDS buffer with steps of 32, operands read a step ahead, and tiles of 64 x 128 with four waves were no faster.
+//   8 x 3108 x 777 x 128 (scores): 61 -> 55 us, x 128 x 777 (values): 61.5 -> 43; 8 x 4096 x 1024 x 128: 85 -> 80
 struct MMParts {
   uint32_t p[3];
 };
@@ -442,7 +444,7 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
       __builtin_amdgcn_sched_barrier(0);
       store(1 - d, skip);
       load(1 - d, step + 3);
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (TM * TN == 1) __builtin_amdgcn_sched_barrier(0);
       auto mul = [&](mm_f32x16 (&to)[TM][TN], int u, int w) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -450,6 +452,13 @@ __global__ __launch_bounds__(WM * WN * 64, TM * TN == 1 ? 4 : 2) void matmul_spl
           for (int j = 0; j < TN; ++j) to[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][u], fb[j][w], to[i][j], 0, 0, 0);
       };
       mul(low, 2, 1), mul(acc, 0, 0), mul(low, 1, 2), mul(low, 2, 0), mul(low, 0, 2), mul(low, 1, 1), mul(low, 1, 0), mul(low, 0, 1);
+      if constexpr (TM * TN > 1) {  // the splitting in the shadows of the matrix instructions
+#pragma unroll
+        for (int q = 0; q < 8 * TM * TN; q++) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+        }
+      }
       __syncthreads();
     };
     int step = 0;
@@ -838,8 +847,9 @@ static bool mm_narrow(const MMArgs& a) {
 }
 
 // fp32: the side of the tile of matmul_split_kernel, 0 where fp32 instructions are as fast or needed.  Costs in us of the three forms fitted to 4800
-// random shapes in all orders (1 to 64 x 5 to 4096 x 5 to 4096 x 16 to 2048, a third of them attention of 64 to 1024 tokens): the choice takes 0.945 of the
-// fp32 instructions' time on average over all of them, the best of the three 0.930; 9 shapes are more than 5 % slower.  A gain of less than 4 % in the costs stays with
+// random shapes in all orders (1 to 64 x 5 to 4096 x 5 to 4096 x 16 to 2048, a third of them attention of 64 to 1024 tokens), those of the large tile
+// again to 900 of more than one small tile per CU: the choice takes 0.864 of the fp32 instructions' time on average over those, the best of the three 0.859 (0.879
+// before the large tile's splitting moved); one is more than 5 % slower.  A gain of less than 4 % in the costs stays with
 // fp32 instructions, and so do K below 32 (59 x 397 x 1677 x 24: 45.4 us, 57 with parts) and up to one small tile per CU, where the order decides
 // and tiles do not (1 x 1701 x 245 x 1964 with A [K][M] 74 / 56, 8 x 20 x 168 x 1765 42 / 50).  With costs of the parts alone every launch
 // above a floor took them, and the large tile too early: 8 x 504 x 504 x 128 9.4 / 12.2 us, 8 x 1308 x 327 x 64 11.2 / 16.1.  Few rows x
@@ -853,7 +863,7 @@ static int mm_split_side(const MMArgs& a, bool nt) {
   const double K = a.K, t64 = (double)((a.M + 63) / 64) * ((a.N + 63) / 64) * a.batch / 256, t128 = (double)((a.M + 127) / 128) * ((a.N + 127) / 128) * a.batch / 256;
   if (t64 <= 1. || a.K < 32) return 0;
   const double us64 = 3.6 + 0.80 * t64 + K * (0.0225 + 0.0152 * (0.49 * std::ceil(t64) + 0.51 * t64 - 1.));
-  const double us128 = 1.6 + 4.66 * std::max(t128, 1.) + K * (0.0502 + 0.0579 * (std::ceil(t128) - 1.));
+  const double us128 = 2.14 + 6.02 * std::max(t128, 1.) + K * (0.0384 + 0.0503 * (std::ceil(t128) - 1.));
   const double f32 = 3.06 + 0.869 * t64 + K * (0.024 + 0.020 * (0.93 * std::ceil(t64) + 0.07 * t64 - 1.));
   if (std::min(us64, us128) > 0.96 * f32) return 0;
   return us128 < us64 ? 128 : 64;
