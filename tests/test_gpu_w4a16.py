@@ -41,6 +41,22 @@ def test_dequant_table_exhaustive():
     assert _same_values(got, orc.w4a16_dequant(synth.pack_nibbles(q), s, synth.pack_nibbles(z)))
 
 
+def test_dequant_every_code_and_zero_point():
+    """all 256 pairs of a code and a zero point with scales from the smallest denormal to the largest number of fp16, bit for bit, in both
+    layouts: a nibble is converted as a number of 2^-9 times its value, the scale as 2^9 times its own"""
+    scales = np.array([0x0001, 0x03ff, 0x0400, 0x1234, 0x3555, 0x3c00, 0x7bff, 0x9555, 0xfbff], np.uint16)
+    N, K, group = 16 * len(scales), 64, 64
+    q = np.tile(np.arange(16, dtype=np.uint8), (N, K // 16))
+    z = np.tile(np.arange(16, dtype=np.uint8)[:, None], (len(scales), 1))
+    qw, zp = synth.pack_nibbles(q), synth.pack_nibbles(z)
+    s = np.repeat(scales, 16)[:, None].copy()
+    want = orc.w4a16_dequant(qw, s, zp, group)
+    announce("w4a16 every code and zero point")
+    args = _dev(qw, s, zp)
+    assert _same_values(_bits(ql.w4a16_dequantize(*args, group)), want)
+    assert _same_values(_bits(ql.w4a16_dequantize_packed(ql.w4a16_prepack(*args, group), N, K, group)), want)
+
+
 def test_dequant_full_size_bit_exact():
     rng = synth.rng_for(2)
     qw, s, zp, _, _ = synth.make_w4a16(rng, 9728, 2560)
