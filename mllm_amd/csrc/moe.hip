@@ -601,21 +601,27 @@ __device__ __forceinline__ f16x2 qg_offset2(const uint32_t (&s)[qg_scale_dwords(
   return __builtin_bit_cast(f16x2, h | (h << 16));
 }
 
+// (w & mask) | base in one instruction
+__device__ __forceinline__ uint32_t qg_under(uint32_t w, uint32_t mask, uint32_t base) {
+  return (uint32_t)__builtin_amdgcn_bitop3_b32((int)w, (int)mask, (int)base, 0xea);
+}
 // pair `b` (elements 2b, 2b+1) of the eight weights of one MFMA step, scaled: one dword of two fp16.  With PREC == 2 also
 // the rounding residual of the product (exact: the error of a product of two fp16 numbers is an fp16 number).
 // Q4_K: the sub-block's value is ds * q - dm (q = 0..15): one fused multiply-add, one rounding; Q6_K: codes widened to
 // int8 at load time, ds the scale of the step's 16 elements: the Q8_0 arithmetic.
-// These instructions and the MFMAs take turns (4 clocks each but 2 for a shift, and / or), so: nibbles at bits 4 b + 0..3 go into the mantissa of
-// 1024 (b even) or as they are into that of 64 (b odd), one shift for two of the four pairs instead of three; bytes are put under the mantissa
-// of 1024 by a permutation.  In a graph, three shifts and and / or on bytes / this, us: 2048 x 9728 x 2560 Q6_K 119.3 / 117.7, Q4_0 115.9 / 113.0; 131 x 2560 x 9728 Q6_K
-// 28.3 / 25.9 (one call after the other 23.4 / 21.5), Q8_0 27.7 / 25.4, Q4_0 26.0 / 25.0, Q4_K 25.4 / 24.4.
+// Nibbles at bits 4 b + 0..3 go into the mantissa of 1024 (b even) or as they are into that of 64 (b odd), one shift for two of the four
+// pairs; bytes are put under the mantissa of 1024 by a permutation.  Clocks of a wave per instruction, four waves per SIMD: 2.3 for a shift, an and / or / xor,
+// 2.5 for three-input logic, 4.2 for a permutation, packed fp16 and conversions: mask and exponent in one instruction take 2.5 instead of 4.6 (bytes
+// by a shift and three-input logic instead of the permutation: no faster).  In a graph, three shifts and and / or on bytes / one shift, permutations, us: 2048 x 9728 x 2560
+// Q6_K 119.3 / 117.7, Q4_0 115.9 / 113.0; 131 x 2560 x 9728 Q6_K 28.3 / 25.9, Q8_0 27.7 / 25.4, Q4_0 26.0 / 25.0, Q4_K 25.4 / 24.4.  And, or / three-input logic, Q4_0:
+// 111 x 5376 x 4736 21.7 / 20.3, 531 x 4144 x 2848 32.9 / 31.8, 2048 x 9728 x 2560 (bound by the matrix pipe at the clock that it holds) 117.2 / 115.0.
 template <int WT, int PREC>
 __device__ __forceinline__ uint32_t qg_pair(const u32x4 (&rq)[qg_nibbles(WT) ? 1 : 2], int d, int b, f16x2 dd, f16x2 dm, uint32_t& lo) {
   uint32_t t;
   float off;
   if (qg_nibbles(WT)) {
     const uint32_t w = b < 2 ? rq[0][d] : rq[0][d] >> 8;
-    t = b & 1 ? (w & 0x00f000f0u) | 0x54005400u : (w & 0x000f000fu) | 0x64006400u;  // 64 + q or 1024 + q in both halves
+    t = b & 1 ? qg_under(w, 0x00f000f0u, 0x54005400u) : qg_under(w, 0x000f000fu, 0x64006400u);  // 64 + q or 1024 + q in both halves
     off = b & 1 ? 64.f : 1024.f;
     if (WT == MLLM_HIP_Q4_0) off += 8.f;
   } else {

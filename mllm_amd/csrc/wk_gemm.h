@@ -31,8 +31,9 @@
 
 namespace mllmhip {
 
+// (one tile by eight waves: 128 registers, two workgroups per CU)
 template <class T, int TM, int TN, int NW, int D, int RP = 4>
-__global__ __launch_bounds__(NW * 64) void wk_gemm_kernel(typename T::Args a) {
+__global__ __launch_bounds__(NW * 64, TM * TN == 1 && NW == 8 ? 4 : 1) void wk_gemm_kernel(typename T::Args a) {
   typedef typename T::Acc Acc;  // sixteen 32-bit sums
   extern __shared__ __align__(16) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
