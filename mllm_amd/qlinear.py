@@ -369,17 +369,7 @@ def moe_ffn_q(gate, up, down, x, topk_ids, topk_w, act_scale_mode=SCALE_X86_REF,
 def linear_q_gemm(w, x, bias=None, act_scale_mode=SCALE_X86_REF, workspace=None, out=None, short=False):
     """Q4_0/Q8_0 Linear for many rows on the matrix cores (fp16 operands with the block scales folded in); w in the "gemm"
     layout.  short=True: the entry point for short batches (K cut into ranges that run as separate workgroups)."""
-    assert x.is_cuda and x.is_contiguous() and x.dim() == 2 and x.shape[1] == w.K and w.layout == "gemm"
-    M = x.shape[0]
-    L = _lib.lib()
-    if workspace is None:
-        size = L.mllm_hip_linear_q_gemm_short_workspace_bytes(M, w.N, w.K) if short else L.mllm_hip_linear_q_gemm_workspace_bytes(M, w.K)
-        workspace = torch.empty(size, dtype=torch.uint8, device="cuda")
-    y = out if out is not None else torch.empty((M, w.N), dtype=torch.float32, device="cuda")
-    fn = L.mllm_hip_linear_q_gemm_short if short else L.mllm_hip_linear_q_gemm
-    _lib.check(fn(w.wtype, w.ptr, x.data_ptr(), _xdtype(x), _p(bias), y.data_ptr(), M, w.N, w.K, act_scale_mode, workspace.data_ptr(),
-                  _stream()), "mllm_hip_linear_q_gemm")
-    return y
+    return _calls().linear_q_gemm(w, x, bias, act_scale_mode, workspace, out, short)
 
 
 def moe_ffn_q_gemm(gate, up, down, x, topk_ids, topk_w, act_scale_mode=SCALE_X86_REF, workspace=None, out=None):
@@ -614,17 +604,7 @@ def kq_workspace(M, K, N_total=0):
 
 def linear_kq_gemm(w, x, bias=None, out=None, workspace=None, short=False):
     """many rows on the matrix cores; w: PackedKWeight(layout="gemm"); short=True: the entry point for short batches"""
-    assert w.layout == "gemm" and x.is_cuda and x.is_contiguous() and x.dim() == 2 and x.shape[1] == w.K
-    M = x.shape[0]
-    L = _lib.lib()
-    y = out if out is not None else torch.empty((M, w.N), dtype=torch.float32, device="cuda")
-    if workspace is None:
-        size = L.mllm_hip_linear_kq_gemm_short_workspace_bytes(M, w.N, w.K) if short else L.mllm_hip_linear_kq_gemm_workspace_bytes(M, w.K)
-        workspace = torch.empty(size, dtype=torch.uint8, device="cuda")
-    fn = L.mllm_hip_linear_kq_gemm_short if short else L.mllm_hip_linear_kq_gemm
-    _lib.check(fn(w.wtype, w.ptr, x.data_ptr(), _xdtype(x), _p(bias), y.data_ptr(), M, w.N, w.K, workspace.data_ptr(), _stream()),
-               "mllm_hip_linear_kq_gemm")
-    return y
+    return _calls().linear_kq_gemm(w, x, bias, workspace, out, short)
 
 
 def linear_kq(w, x, bias=None, out=None, workspace=None):

@@ -12,6 +12,14 @@ class _W:
     wtype, N, K, buf = 0, 64, 64, torch.zeros(1, dtype=torch.uint8)
 
 
+class _G(_W):
+    layout = "gemm"
+
+
+class _V(_W):
+    layout = "gemv"
+
+
 X = torch.zeros(3, 64)
 
 
@@ -24,6 +32,8 @@ X = torch.zeros(3, 64)
     (lambda: ql.matmul(X.t(), X.t()), AssertionError), (lambda: ql.matmul(X.double(), X.double(), False, True), AssertionError),
     (lambda: ql.matmul(torch.zeros(2, 3, 4), torch.zeros(3, 4, 5)), AssertionError),
     (lambda: ql.w8a8_linear_packed(X, X, 64, X), AssertionError), (lambda: ql.w8a8_linear_packed(X[0], X, 64, X), ValueError),
+    (lambda: ql.linear_q_gemm(_G, X), AssertionError), (lambda: ql.linear_q_gemm(_V, X), AssertionError), (lambda: ql.linear_kq_gemm(_G, X, short=True), AssertionError),
+    (lambda: ql.linear_q_gemm(_G, None), TypeError), (lambda: ql.linear_kq_gemm(_W, None), TypeError),
     (lambda: ql.w4a16_gemm_packed(X, X, 64), AssertionError), (lambda: ql.w4a16_gemm_packed(X.bfloat16(), X, 64), AssertionError)])
 def test_calls_refuse_what_the_kernels_do_not_take(call, error):
     with pytest.raises(error):
@@ -35,6 +45,34 @@ def test_missing_module_fails_loudly(monkeypatch):
     monkeypatch.setattr(_lib, "CALLS_PATH", "/nonexistent/mllm_calls.so")
     with pytest.raises(_lib.HipQLinearError):
         ql.softmax(X)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("short", [False, True])
+@pytest.mark.parametrize("kq", [False, True])
+def test_many_row_calls_use_the_callers_outputs_workspaces_and_stream(kq, short):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    make, call = (ql.PackedKWeight, ql.linear_kq_gemm) if kq else (ql.PackedQWeight, ql.linear_q_gemm)
+    w, v = (make.synthetic(ql.Q6_K if kq else ql.Q4_0, 256, 512, g, layout=layout) for layout in ("gemm", "gemv"))
+    x, bias = torch.randn((70, 512), device="cuda", generator=g), torch.randn(256, device="cuda", generator=g)
+    L = _lib.lib()
+    size = ((L.mllm_hip_linear_kq_gemm_short_workspace_bytes if kq else L.mllm_hip_linear_q_gemm_short_workspace_bytes)(70, 256, 512) if short else
+            (L.mllm_hip_linear_kq_gemm_workspace_bytes if kq else L.mllm_hip_linear_q_gemm_workspace_bytes)(70, 512))
+    announce("many-row calls with and without outputs", kq, short)
+    y = call(w, x, bias, short=short)
+    assert y.shape == (70, 256) and y.dtype == torch.float32
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(200_000_000)  # a call on the default stream would not wait for what follows
+        out, work = torch.full((70, 256), float("nan"), device="cuda"), torch.empty(size, dtype=torch.uint8, device="cuda")
+        assert call(w, x * 1, bias, out=out, workspace=work, short=short) is out
+    stream.synchronize()
+    assert torch.equal(out, y)
+    for bad, error in ((lambda: call(v, x), AssertionError), (lambda: call(w, x[:, :256]), AssertionError), (lambda: call(w, x.half()), TypeError),
+                       (lambda: call(w, x[:0]), _lib.HipQLinearError)):
+        with pytest.raises(error):
+            bad()
 
 
 @pytest.mark.gpu
