@@ -312,22 +312,41 @@ struct KRsrc {
   __amdgpu_buffer_rsrc_t a, h, s, d;
 };
 
+// byte offsets of a lane's first unit in a row; units that are a multiple of eight further on lie a multiple of these steps on
+struct KOff {
+  uint32_t a, h, s, d;
+};
 template <int WT>
-__device__ __forceinline__ void load_unit(KUnit<WT>& u, const KRsrc& r, uint32_t sb_base, int unit, int units, bool row_ok) {
-  const bool ok = row_ok && unit < units;
+__device__ __forceinline__ KOff unit_offsets(uint32_t sb_base, int unit) {
+  KOff o{};
   if (WT == MLLM_HIP_Q4_K) {
     const uint32_t sb = sb_base + (uint32_t)(unit >> 3);
-    u.a = __builtin_amdgcn_raw_buffer_load_b128(r.a, ok ? (sb * 8u + (uint32_t)(unit & 7)) * 16u : KBUF_OOB, 0, KBUF_NT);
-    u.s.x = __builtin_amdgcn_raw_buffer_load_b32(r.s, ok ? sb * 16u + (uint32_t)((unit >> 1) & 3) * 4u : KBUF_OOB, 0, KBUF_NT);  // its pair's scales
-    u.s.y = __builtin_amdgcn_raw_buffer_load_b32(r.d, ok ? sb * 4u : KBUF_OOB, 0, KBUF_NT);                                      // d, dmin
+    o.a = (sb * 8u + (uint32_t)(unit & 7)) * 16u;
+    o.s = sb * 16u + (uint32_t)((unit >> 1) & 3) * 4u;  // its pair's scales
+    o.d = sb * 4u;
   } else {
     const uint32_t sb = sb_base + (uint32_t)(unit >> 2);
     const uint32_t n = (uint32_t)(unit >> 1) & 1u, t = (uint32_t)unit & 1u;
-    u.a = __builtin_amdgcn_raw_buffer_load_b128(r.a, ok ? (sb * 8u + 4u * n + t) * 16u : KBUF_OOB, 0, KBUF_NT);
-    u.b = __builtin_amdgcn_raw_buffer_load_b128(r.a, ok ? (sb * 8u + 4u * n + 2u + t) * 16u : KBUF_OOB, 0, KBUF_NT);
-    u.h = __builtin_amdgcn_raw_buffer_load_b128(r.h, ok ? (sb * 4u + 2u * n + t) * 16u : KBUF_OOB, 0, KBUF_NT);
-    u.s = __builtin_amdgcn_raw_buffer_load_b128(r.s, ok ? sb * 16u : KBUF_OOB, 0, KBUF_NT);
-    u.d = __builtin_amdgcn_raw_buffer_load_b16(r.d, ok ? sb * 2u : KBUF_OOB, 0, KBUF_NT);
+    o.a = (sb * 8u + 4u * n + t) * 16u;
+    o.h = (sb * 4u + 2u * n + t) * 16u;
+    o.s = sb * 16u;
+    o.d = sb * 2u;
+  }
+  return o;
+}
+// the unit `ahead` (uniform) units behind that of o; one that is not there fetches nothing
+template <int WT>
+__device__ __forceinline__ void load_unit(KUnit<WT>& u, const KRsrc& r, const KOff& o, int ahead, bool ok) {
+  if (WT == MLLM_HIP_Q4_K) {
+    u.a = __builtin_amdgcn_raw_buffer_load_b128(r.a, ok ? o.a : KBUF_OOB, ahead * 16, KBUF_NT);
+    u.s.x = __builtin_amdgcn_raw_buffer_load_b32(r.s, ok ? o.s : KBUF_OOB, ahead * 2, KBUF_NT);
+    u.s.y = __builtin_amdgcn_raw_buffer_load_b32(r.d, ok ? o.d : KBUF_OOB, ahead / 2, KBUF_NT);  // d, dmin
+  } else {
+    u.a = __builtin_amdgcn_raw_buffer_load_b128(r.a, ok ? o.a : KBUF_OOB, ahead * 32, KBUF_NT);
+    u.b = __builtin_amdgcn_raw_buffer_load_b128(r.a, ok ? o.a : KBUF_OOB, ahead * 32 + 32, KBUF_NT);
+    u.h = __builtin_amdgcn_raw_buffer_load_b128(r.h, ok ? o.h : KBUF_OOB, ahead * 16, KBUF_NT);
+    u.s = __builtin_amdgcn_raw_buffer_load_b128(r.s, ok ? o.s : KBUF_OOB, ahead * 4, KBUF_NT);
+    u.d = __builtin_amdgcn_raw_buffer_load_b16(r.d, ok ? o.d : KBUF_OOB, ahead / 2, KBUF_NT);
   }
 }
 
@@ -350,8 +369,10 @@ __device__ __forceinline__ void silu_mul8(float (&v)[8], const float* u, bool ac
 // Workgroup = NW waves; a wave is cut into 64 / G groups of G lanes; a group owns R consecutive weight rows and its lanes
 // stride over the row's units.  x is quantized to Q8_K once per workgroup into LDS: codes [MT][K], scales [MT][nsb], sums
 // of 16 as int16 [MT][nsb][16].
-// U = units a lane keeps in flight per row and trip.
-// ONE: the row's units fit one trip (units <= G U): no second set of registers for the next trip.
+// U = units a lane keeps in flight per row: a ring, a unit's registers take the one U further on as soon as it is multiplied.  (A second set
+// of registers for a whole next trip, copied over, took 220 registers for Q6_K with two units of two rows, 152 now; 2 x 9728 x 2560 at two rows, with the
+// offsets below and 24-bit products of sums and scales: Q4_K 11.2 -> 10.5 us, Q6_K 14.9 -> 13.9.)
+// ONE: the row's units fit one trip (units <= G U): nothing to refill.
 template <int WT, int XT, int MT, int G, int R, int U, int LB = 256, bool ONE = false>
 __global__ __launch_bounds__(LB) void kq_gemv_kernel(KGemvArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -428,11 +449,18 @@ __global__ __launch_bounds__(LB) void kq_gemv_kernel(KGemvArgs a) {
     __asm__ volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   }
+  KOff off[R];
+  bool row_ok[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    off[r] = unit_offsets<WT>((uint32_t)((row0 + r) * nsb), c0);
+    row_ok[r] = row0 + r < pt.N;
+  }
   KUnit<WT> cur[U][R];
 #pragma unroll
   for (int uu = 0; uu < U; uu++)
 #pragma unroll
-    for (int r = 0; r < R; r++) load_unit<WT>(cur[uu][r], rs, (uint32_t)((row0 + r) * nsb), uu * G + c0, units, row0 + r < pt.N);
+    for (int r = 0; r < R; r++) load_unit<WT>(cur[uu][r], rs, off[r], uu * G, row_ok[r] && uu * G + c0 < units);
 
   __asm__ volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
@@ -493,15 +521,7 @@ __global__ __launch_bounds__(LB) void kq_gemv_kernel(KGemvArgs a) {
     for (int m = 0; m < MT; m++) acc[r][m] = 0.f;
 
   for (int u0 = 0; u0 < units; u0 += G * U) {
-    KUnit<WT> nxt[U][R];
     const bool more = !ONE && u0 + G * U < units;  // uniform
-    if (more) {
-#pragma unroll
-      for (int uu = 0; uu < U; uu++)
-#pragma unroll
-        for (int r = 0; r < R; r++)
-          load_unit<WT>(nxt[uu][r], rs, (uint32_t)((row0 + r) * nsb), u0 + G * U + uu * G + c0, units, row0 + r < pt.N);
-    }
 #pragma unroll
     for (int uu = 0; uu < U; uu++) {
     const KUnit<WT>(&cu)[R] = cur[uu];
@@ -534,8 +554,9 @@ __global__ __launch_bounds__(LB) void kq_gemv_kernel(KGemvArgs a) {
           const int bs_lo = half16(bp.x, hh), bs_hi = half16(bp.y, hh);
 #pragma unroll
           for (int r = 0; r < R; r++) {
-            const int isum = sc_lo[r] * dot16(wlo[r], xlo) + sc_hi[r] * dot16(whi[r], xhi);
-            const int msum = mn_lo[r] * bs_lo + mn_hi[r] * bs_hi;
+            // (24-bit factors: one instruction instead of four times one)
+            const int isum = __mul24(sc_lo[r], dot16(wlo[r], xlo)) + __mul24(sc_hi[r], dot16(whi[r], xhi));
+            const int msum = __mul24(mn_lo[r], bs_lo) + __mul24(mn_hi[r], bs_hi);
             acc[r][m] = fmaf(yd * dw[r], (float)isum, acc[r][m]);
             acc[r][m] = fmaf(-yd * dmw[r], (float)msum, acc[r][m]);
           }
@@ -573,19 +594,19 @@ __global__ __launch_bounds__(LB) void kq_gemv_kernel(KGemvArgs a) {
             const u32x4 xq = s_q[m * (K >> 4) + sb * 16 + 8 * n + 2 * g + t];
             const int bs = half16(bw[g], t);
 #pragma unroll
-            for (int r = 0; r < R; r++) tot[r] += sc[r][g] * (dot16(wv[r][g], xq) - 32 * bs);
+            for (int r = 0; r < R; r++) tot[r] += __mul24(sc[r][g], dot16(wv[r][g], xq) - 32 * bs);
           }
 #pragma unroll
           for (int r = 0; r < R; r++) acc[r][m] = fmaf(yd * dw[r], (float)tot[r], acc[r][m]);
         }
       }
     }
+    if (more) {  // the next trip's unit into the registers of this one
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < R; r++) load_unit<WT>(cur[uu][r], rs, off[r], u0 + G * U + uu * G, row_ok[r] && u0 + G * U + uu * G + c0 < units);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (more) {
-#pragma unroll
-      for (int uu = 0; uu < U; uu++)
-#pragma unroll
-        for (int r = 0; r < R; r++) cur[uu][r] = nxt[uu][r];
     }
   }
 
@@ -640,6 +661,17 @@ static int launch_kq_g(const KGemvArgs& a, int NW, int U, bool r1, hipStream_t s
       // two rounds; asking the compiler for five waves, 96 registers, measured slower: gate + up 8.7 -> 9.1 us, q+k+v 5.35 -> 5.65)
       if constexpr (MT == 1)
         if (!r1 && units > 2 * G && units <= 3 * G) return launch_kq_u<WT, XT, MT, G, 3, false, true>(a, NW, st);
+    }
+  }
+  // MoE slots: the row's units at once where two per lane hold them (Q4_K rows of up to 1024 elements, Q6_K of up to 2048), Q4_K four at a time beyond that.
+  // us of a layer of 128 experts of 2048 x 768, top-8, two at a time with a second set of registers for the next trip / this: Q4_K / Q6_K one token
+  // 15.1 / 14.3, four 26.4 / 25.4, eight 40.8 / 39.8 (three at a time 44.4), Q6_K eight 53.5 / 47.2
+  if constexpr (MT == 1 && G == 16) {
+    const int units = a.nsb * (WT == MLLM_HIP_Q4_K ? 8 : 4);
+    if (a.slot_ids && U == 2 && !g_kq_U) {
+      if (units <= G) return launch_kq_u<WT, XT, MT, G, 1, false, true>(a, NW, st);
+      if (units <= 2 * G) return launch_kq_u<WT, XT, MT, G, 2, false, true>(a, NW, st);
+      if (WT == MLLM_HIP_Q4_K) return launch_kq_u<WT, XT, MT, G, WT == MLLM_HIP_Q4_K ? 4 : 2>(a, NW, st);
     }
   }
   if (r1 && MT <= 2 && G >= 32) return launch_kq_u<WT, XT, MT, G, (MT <= 2 && G >= 32 && WT == MLLM_HIP_Q4_K) ? 4 : 1, (MT <= 2 && G >= 32)>(a, NW, st);

@@ -397,6 +397,28 @@ def test_units_in_flight_do_not_change_the_bits(wtype):
                 assert L.mllm_hip_kq_set_tuning(0, 0, 0) == 0
 
 
+@pytest.mark.parametrize("wtype,H", [(2, 512), (2, 768), (2, 1024), (2, 1280), (2, 2048), (2, 2304), (3, 1024), (3, 1280), (3, 2048), (3, 2304)])
+def test_units_in_flight_of_expert_pairs_do_not_change_the_bits(wtype, H):
+    """a token's experts, a GEMV row per pair: rows whose units fit one or two per lane, the ring of several and its last, partly filled trip
+    against one unit at a time (mllm_hip_kq_set_tuning)"""
+    I, E, k = 256 + 256 * (H % 512 > 0), 5, 3
+    rng = synth.rng_for(9, 7900 + wtype + H)
+    L = _lib.lib()
+    Wg, Wu = (synth.make_weight(rng, wtype, E * I, H).reshape(E, I, H // 256, -1) for _ in range(2))
+    Wd = synth.make_weight(rng, wtype, E * H, I).reshape(E, H, I // 256, -1)
+    g, u, d = (ql.PackedKExperts(wtype, torch.from_numpy(W)) for W in (Wg, Wu, Wd))
+    ids, w = synth.make_moe_routing(rng, 1, E, k)
+    ids, w, x = to_dev(ids), to_dev(w), to_dev(synth.make_x_fp32(rng, 1, H))
+    announce("moe k-quant pairs, units in flight", wtype, H, I)
+    want = ql.moe_ffn_kq(g, u, d, x, ids, w)
+    assert torch.isfinite(want).all() and want.abs().max() > 0
+    try:
+        assert L.mllm_hip_kq_set_tuning(0, 0, 1) == 0
+        assert torch.equal(want, ql.moe_ffn_kq(g, u, d, x, ids, w))
+    finally:
+        assert L.mllm_hip_kq_set_tuning(0, 0, 0) == 0
+
+
 def test_argument_checks():
     L = _lib.lib()
     buf = torch.zeros(1 << 16, dtype=torch.uint8, device="cuda")
