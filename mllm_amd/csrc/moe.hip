@@ -1812,7 +1812,7 @@ static int launch_q_waves(int form, const QWavesArgs& a, hipStream_t st) {
   switch (form) {
     case 0: return wk_gemm_launch<QWaves<WT>, 1, 1, 8, 2>(a, st);
     case 1: return wk_gemm_launch<QWaves<WT>, 1, 2, 8, 1>(a, st);
-    default: return wk_gemm_launch<QWaves<WT>, 2, 2, 4, 2>(a, st);
+    default: return wk_gemm_64x64<QWaves<WT>>(a, st);
   }
 }
 
@@ -1855,6 +1855,7 @@ static bool q_ranges_exist(int64_t N, int64_t blocks, int z) {  // whole even ra
 struct QFormCost {
   float waves[3][6];  // per form: how a partly filled last round counts, fixed, round, round and 64 of K, 1e6 M K (read again by every
   float halves[6];    // column tile), 1e6 M N
+  float eight;        // 64 of K less in the third of the waves' forms where it runs by eight waves (fitted to 34 shapes each, 1.3 to 2.6 % rms)
   float ranges[8];    // two workgroups on a CU, part of a last round; fixed, round, round and 64 of K, M K, M N, M N per partial result
 };
 static const QFormCost& q_form_cost(int wtype) {
@@ -1863,21 +1864,25 @@ static const QFormCost& q_form_cost(int wtype) {
         {0.75f, 5.554f, 0.1751f, 0.1086f, 1.942f, 1.997f},
         {0.5f, 6.718f, 0.f, 0.1817f, 1.876f, 1.659f}},
        {1.f, 8.318f, 0.3028f, 0.6705f, 0.6885f, 1.894f},
+       0.0238f,
        {1.5f, 0.5f, 11.4f, 0.005467f, 0.7897f, 1.398f, 0.7408f, 1.058f}},  // Q4_0: 4 / 4 / 5 / 4 / 6 %
       {{{0.75f, 5.465f, 0.4136f, 0.0751f, 3.046f, 1.154f},
         {1.f, 5.928f, 0.f, 0.1192f, 1.86f, 2.248f},
         {0.5f, 7.359f, 0.f, 0.2f, 1.889f, 1.413f}},
        {1.f, 6.389f, 2.611f, 0.6195f, 1.174f, 1.848f},
+       0.0234f,
        {1.6f, 0.5f, 11.23f, 0.f, 0.7656f, 1.514f, 0.6784f, 1.075f}},  // Q8_0: 4 / 4 / 5 / 7 / 7 %
       {{{0.75f, 5.412f, 0.5444f, 0.06797f, 3.148f, 0.8011f},
         {1.f, 5.739f, 0.04121f, 0.1086f, 1.952f, 2.302f},
         {0.5f, 7.01f, 0.f, 0.1872f, 1.97f, 1.559f}},
        {1.f, 10.17f, 0.05216f, 0.6293f, 0.906f, 1.662f},
+       0.025f,
        {1.5f, 0.75f, 12.58f, 0.f, 0.763f, 1.45f, 0.7756f, 1.005f}},  // Q4_K: 3 / 3 / 5 / 4 / 6 %
       {{{1.f, 4.986f, 0.6891f, 0.08025f, 3.059f, 2.38f},
         {1.f, 6.076f, 0.f, 0.1191f, 1.771f, 2.268f},
         {0.5f, 7.235f, 0.f, 0.2001f, 1.852f, 1.482f}},
        {1.f, 2.535f, 7.217f, 0.6381f, 1.067f, 1.459f},
+       0.0193f,
        {1.7f, 0.5f, 12.05f, 0.f, 0.7532f, 1.344f, 0.6954f, 1.035f}},  // Q6_K: 4 / 3 / 5 / 4 / 6 %
   };
   return cost[wtype == MLLM_HIP_Q4_0 ? 0 : wtype == MLLM_HIP_Q8_0 ? 1 : wtype == MLLM_HIP_Q4_K ? 2 : 3];
@@ -1906,7 +1911,12 @@ static QLinearPlan q_linear_plan(int wtype, int64_t M, int64_t N, int64_t K, boo
   static const int rows[3] = {32, 32, 64}, chans[3] = {32, 64, 64};
   for (int f = 0; f < 3; f++) {
     const int64_t tiles = ((M + rows[f] - 1) / rows[f]) * ((N + chans[f] - 1) / chans[f]);
-    offer(whole(c.waves[f], (float)((tiles + 255) / 256), (float)tiles / 256.f), QLinearPlan{f, 0, 1});
+    const float cost = whole(c.waves[f], (float)((tiles + 255) / 256), (float)tiles / 256.f);
+    const float eight = f == 2 && tiles <= WK_EIGHT_TILES ? c.eight * (float)blocks : 0.f;
+    offer(cost - eight, QLinearPlan{f, 0, 1});
+    // Tiles of 128 x 256 give way to the eight waves only where the costs differ by more than their errors.  Over 479 shapes 0.992 of the time with
+    // four waves throughout, 44 of them 3 to 18 % faster (180 x 3120 x 7680 Q4_0 33.6 -> 27.6 us), none slower.
+    if (best.waves == 2 && eight > 0.f) least = std::min(cost, 1.06f * least);
   }
   // a ragged last tile of 128 rows runs as 64 or 32
   const int64_t rest = M % QG_TILE_H;

@@ -165,6 +165,33 @@ def test_q_gemm_every_form_exact(wtype, M, N, K):
         assert L.mllm_hip_q_gemm_set_form(0) == 0
 
 
+@pytest.mark.parametrize("M,N,K", [(1024, 1024, 96), (1025, 1024, 96), (97, 8192, 800), (97, 8193, 800)])
+def test_linear_q_gemm_64x64_tiles_by_eight_and_four_waves(M, N, K):
+    """either side of 256 tiles: fewer K blocks than waves and blocks that do not divide among them; integers whose sums are exact in any order
+    (scales of one, no partial sum leaves 2^24)"""
+    L = _lib.lib()
+    rng = synth.rng_for(4, 1700 + M + N + K)
+    W = synth.make_weight(rng, 0, N, K)
+    W.reshape(N, K // 32, -1)[:, :, 0:2] = np.array([0x00, 0x3c], np.uint8)
+    b = W.reshape(N, K // 32, -1)[:, :, 2:]
+    wd = (np.concatenate([b & 15, b >> 4], 2).astype(np.float32) - 8).reshape(N, K)
+    x = rng.integers(-3, 4, (M, K)).astype(np.float32)
+    x[:, ::32] = 127.0
+    w = ql.PackedQWeight(0, torch.from_numpy(W), layout="gemm")
+    announce("q gemm 64 x 64", M, N, K)
+    try:
+        assert L.mllm_hip_q_gemm_set_form(3) == 0
+        assert np.array_equal(ql.linear_q_gemm(w, to_dev(x), None, ql.SCALE_IEEE, short=True).cpu().numpy(), x @ wd.T)
+    finally:
+        assert L.mllm_hip_q_gemm_set_form(0) == 0
+
+
+@pytest.mark.parametrize("wtype,M,N,K", [(0, 180, 3120, 7680), (2, 179, 2872, 1792), (3, 112, 4336, 1280)])
+def test_linear_q_gemm_takes_64x64_tiles_by_eight_waves(wtype, M, N, K):
+    """host-only query: sizes at which ranges of K or tiles of 32 rows took 5 to 22 % longer"""
+    assert _lib.lib().mllm_hip_q_gemm_form(wtype, M, N, K, 1) == 3
+
+
 def test_linear_q_gemm_exact_when_operands_fit_fp16():
     """Weights and activations chosen so that dW*qW and dX*qX are exactly representable in fp16 and every partial sum in
     fp32: then the matrix-core path must equal the reference arithmetic bit for bit (a wrong nibble order, scale pairing,

@@ -274,6 +274,13 @@ def test_waves_that_split_k_of_larger_tiles():
     _waves_cases(shapes)
 
 
+def test_waves_that_split_k_of_64x64_tiles_by_eight_and_four_waves():
+    """256 such tiles (eight waves) and 258 (four), K blocks that do not divide among the waves"""
+    shapes = ((128, 8192, 1984, 64), (128, 8193, 1984, 64))
+    assert [_lib.lib().mllm_hip_w4a16_packed_form(*s[:3]) for s in shapes] == [4, 4]
+    _waves_cases(shapes)
+
+
 def _waves_cases(shapes):
     for M, N, K, group in shapes:
         rng = synth.rng_for(2, 1300 + 3 * M + N + K + group)
