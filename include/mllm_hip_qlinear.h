@@ -367,7 +367,8 @@ int mllm_hip_w4a16_set_decode_mfma_from(int tokens);
  * + 16 switches off the half-height tiles that shorten a partly filled last round. */
 int mllm_hip_w4a16_packed_set_tuning(int tile);
 /* The form that a product of this size takes: waves that split K of a tile of 32x32 by 1: sixteen, 2: eight, 10: four, 3: 32x64, 4: 64x64; tiles of
- * 5: 128x128, 6: 128x256, 7: 128x384, 8: 64x128, 9: 64x384.  Host only, overrides aside.  No counterpart in the reference. */
+ * 5: 128x128, 6: 128x256, 7: 128x384, 8: 64x128, 9: 64x384 (all but 7 by eight waves with half of K each while every tile has a CU to itself).
+ * Host only, overrides aside.  No counterpart in the reference. */
 int mllm_hip_w4a16_packed_form(int64_t M, int64_t N, int64_t K);
 
 /* ---------------------------------------------------------------------------------------------------------

@@ -13,6 +13,8 @@
 // Weights are fetched packed (16 bytes = 32 elements per lane), dequantized once per workgroup in registers and staged
 // as bf16 in LDS next to the activation tile; the matrix cores read both operands from LDS.
 #include "qcommon.h"
+#include <algorithm>
+
 #include "wk_gemm.h"
 
 namespace mllmhip {
@@ -274,9 +276,10 @@ struct W4A16PArgs {
 };
 
 
-// One output tile (32 TM rows from m0) x (128 TN columns from n0) by the four waves of a workgroup.
-template <int TM, int TN, int BK>
-__device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int m0, const int n0, unsigned char* smem) {
+// One output tile (32 TM rows from m0) x (128 TN columns from n0) by the four waves of a workgroup.  G == 2: by eight, the second four take the
+// second half of K with a stage of their own; their sums join the first's in LDS.
+template <int TM, int TN, int BK, int G = 1>
+__device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int m0, const int n0, unsigned char* smem_all) {
   static_assert(BK == 64 || BK == 128, "K step of one or two 64-element weight blocks");
   constexpr int LDK = 2 * BK + 16, KS = BK / 16, NH = BK / 64;  // LDS row in bytes; MFMA steps; weight blocks per K step
   constexpr int CPRA = BK / 8;                                  // 16-byte activation chunks per row and K step
@@ -285,15 +288,17 @@ __device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int
   static_assert(CA >= 1, "tile too small for 256 threads");
   constexpr int STAGE = BM * LDK;
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  unsigned char* const smem = smem_all + group * 2 * STAGE;
+  const int tid = G == 1 ? threadIdx.x : threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 31, hi = lane >> 5;
 
-  const int Kp = (int)w4a16_packed_k(a.K), kbs = Kp / 64, G = a.K / a.group, g64 = a.group / 64;
+  const int Kp = (int)w4a16_packed_k(a.K), kbs = Kp / 64, groups = a.K / a.group, g64 = a.group / 64;
   const int64_t qbytes = w4a16_packed_qbytes(a.N, a.K);
   const int nbs = (int)(w4a16_packed_n(a.N) / 32);
   const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.A), 0, (uint32_t)((int64_t)a.M * a.K * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rQ = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.P), 0, (uint32_t)qbytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rS = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.P + qbytes), 0, (uint32_t)((int64_t)nbs * G * 256), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rS = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.P + qbytes), 0, (uint32_t)((int64_t)nbs * groups * 256), 0x00020000);
 
   // activation chunk: row idx / CPRA, 16-byte column idx % CPRA.  Rows past M are clamped (never stored); columns past K
   // read as zeros so that the zero-padded tail of the weights never meets another row's values.
@@ -310,7 +315,7 @@ __device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int
   for (int j = 0; j < TN; j++) {
     const int nb = min((n0 + wave * WN) / 32 + j, nbs - 1);
     offQ[j] = (uint32_t)((int64_t)nb * kbs * 1024 + lane * 16);
-    offS[j] = (uint32_t)(((int64_t)nb * G * 32 + lrow) * 8);
+    offS[j] = (uint32_t)(((int64_t)nb * groups * 32 + lrow) * 8);
   }
   auto loadA = [&](int k0, u32x4 (&ga)[CA]) {
 #pragma unroll
@@ -332,7 +337,7 @@ __device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int
   // the packed weights and the (scale, -zp*scale) pair of 64-element block kb of column block j
   auto loadQ = [&](int kb, int j) -> u32x4 { return __builtin_amdgcn_raw_buffer_load_b128(rQ, offQ[j], kb * 1024, 0); };
   auto loadS = [&](int kb, int j) -> u32x2 {
-    return __builtin_amdgcn_raw_buffer_load_b64(rS, offS[j], min(kb / g64, G - 1) * 256, 0);
+    return __builtin_amdgcn_raw_buffer_load_b64(rS, offS[j], min(kb / g64, groups - 1) * 256, 0);
   };
   auto dequant = [&](const u32x4& q, const u32x2& sz, int d) -> bf16x8 {
     uint32_t o[4];
@@ -348,19 +353,20 @@ __device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int
 #pragma unroll
       for (int r = 0; r < 16; r++) acc[j][i][r] = 0.f;
 
-  const int KT = Kp / BK;
+  // K steps of these waves: all of them, or one of the halves (idle: how many fewer the second has, whose barriers it keeps)
+  const int KT = Kp / BK, per = (KT + G - 1) / G, kt0 = group * per, kt1 = min(KT, kt0 + per), idle = G == 1 ? 0 : per - (kt1 - kt0);
   u32x4 ga[CA];
   u32x4 rq[NH][TN];  // packed weights of the 64-element blocks of a K step
   u32x2 rs[NH][TN];
   bf16x8 fb[2][TN];  // dequantized operands of MFMA step ks (set ks & 1)
   bf16x8 fa[2][TM];
-  loadA(0, ga);
+  loadA(kt0 * BK, ga);
 #pragma unroll
   for (int h = 0; h < NH; h++)
 #pragma unroll
     for (int j = 0; j < TN; j++) {
-      rq[h][j] = loadQ(h, j);
-      rs[h][j] = loadS(h, j);
+      rq[h][j] = loadQ(kt0 * NH + h, j);
+      rs[h][j] = loadS(kt0 * NH + h, j);
     }
   storeA(0, ga);
   __syncthreads();
@@ -368,8 +374,8 @@ __device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int
 #pragma unroll
   for (int j = 0; j < TN; j++) fb[0][j] = dequant(rq[0][j], rs[0][j], 0);
 
-  for (int kt = 0; kt < KT; kt++) {
-    const int buf = kt & 1, k1 = (kt + 1) * BK;
+  for (int kt = kt0; kt < kt1; kt++) {
+    const int buf = (kt - kt0) & 1, k1 = (kt + 1) * BK;
     loadA(k1, ga);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -408,14 +414,41 @@ __device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int
       }
     }
   }
+  for (int i = 0; i < idle; i++) __syncthreads();
   __syncthreads();  // all LDS reads done before the epilogue reuses the tiles
+  if constexpr (G == 2) {  // the second half's sums join the first's
+    f32x4* part = reinterpret_cast<f32x4*>(smem_all);
+    auto quad = [&](int j, int i, int g) -> f32x4& { return part[(((wave * TN + j) * TM + i) * 4 + g) * 64 + lane]; };
+    if (group == 1) {
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int g = 0; g < 4; g++) quad(j, i, g) = f32x4{acc[j][i][4 * g], acc[j][i][4 * g + 1], acc[j][i][4 * g + 2], acc[j][i][4 * g + 3]};
+    }
+    __syncthreads();
+    if (group == 0) {
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int g = 0; g < 4; g++) {
+            const f32x4 v = quad(j, i, g);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[j][i][4 * g + e] += v[e];
+          }
+    }
+    __syncthreads();
+  }
 
   // acc[j][i][4g+e] = C[m0 + 32i + lrow][n0 + wave*WN + 32j + 8g + 4hi + e]
-  float* sBi = reinterpret_cast<float*>(smem);
+  float* sBi = reinterpret_cast<float*>(smem_all);
   for (int i = tid; i < BN; i += 256) sBi[i] = (a.bias && n0 + i < a.N) ? bf16_to_f32(a.bias[n0 + i]) : 0.f;
   __syncthreads();
   constexpr int ROWB = 2 * BN + 16;
-  unsigned char* patch = smem + 4096;
+  unsigned char* patch = smem_all + 4096;
   static_assert(BN * 4 <= 4096, "bias overlaps the store patch");
   const bool has_bias = a.bias != nullptr;
   // 16-byte pieces; those of ragged edges fall outside the buffer (whose end a row or column past the tile must not wrap over)
@@ -430,28 +463,31 @@ __device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int
 #pragma unroll
       for (int g = 0; g < 4; g++) bi4[j][g] = *reinterpret_cast<const f32x4*>(&sBi[wave * WN + j * 32 + 8 * g + 4 * hi]);
     constexpr int CPR = BN / 8;  // 16-byte pieces per row
-    static_assert((8 * CPR) % 64 == 0, "a wave stores whole rows");
+    constexpr int RPW = 8 / G;   // rows per wave
+    static_assert((RPW * CPR) % 64 == 0, "a wave stores whole rows");
 #pragma unroll
     for (int i = 0; i < TM; i++) {
+      if (group == 0) {
 #pragma unroll
-      for (int j = 0; j < TN; j++)
+        for (int j = 0; j < TN; j++)
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-          float f[4];
+          for (int g = 0; g < 4; g++) {
+            float f[4];
 #pragma unroll
-          for (int e = 0; e < 4; e++) f[e] = acc[j][i][4 * g + e];
-          if (has_bias) {
+            for (int e = 0; e < 4; e++) f[e] = acc[j][i][4 * g + e];
+            if (has_bias) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) f[e] += bi4[j][g][e];
+              for (int e = 0; e < 4; e++) f[e] += bi4[j][g][e];
+            }
+            *reinterpret_cast<uint2*>(patch + lrow * ROWB + (wave * WN + j * 32 + 8 * g + 4 * hi) * 2) =
+                uint2{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3])};
           }
-          *reinterpret_cast<uint2*>(patch + lrow * ROWB + (wave * WN + j * 32 + 8 * g + 4 * hi) * 2) =
-              uint2{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3])};
-        }
+      }
       __syncthreads();
 #pragma unroll
-      for (int t = 0; t < 8 * CPR / 64; t++) {  // wave w stores rows 8w .. 8w+7
+      for (int t = 0; t < RPW * CPR / 64; t++) {  // wave w stores rows RPW w .. RPW (w + 1) - 1
         const int c = lane + 64 * t;
-        const int row = wave * 8 + c / CPR, cc = c % CPR;
+        const int row = (group * 4 + wave) * RPW + c / CPR, cc = c % CPR;
         const u32x4 v = *reinterpret_cast<const u32x4*>(patch + row * ROWB + cc * 16);
         const int n = n0 + cc * 8;
         // (a row past M lies past the end of the buffer)
@@ -461,6 +497,7 @@ __device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int
     }
     return;
   }
+  if (group != 0) return;
 #pragma unroll
   for (int i = 0; i < TM; i++) {
     const int m = m0 + i * 32 + lrow;
@@ -487,8 +524,8 @@ __device__ __forceinline__ void w4a16_nsplit_tile(const W4A16PArgs& a, const int
 // duration; the half-height tiles are the FIRST workgroups of the grid (2048 x 9728 x 2560: 108 -> 101 us; as the last
 // workgroups 107).
 // WPS: waves per SIMD the register budget is held to (workgroups of 4 waves: WPS workgroups per CU).
-template <int TM, int TN, int BK, int WPS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPS, WPS))) void w4a16_gemm_nsplit_kernel(W4A16PArgs a, int big_cols) {
+template <int TM, int TN, int BK, int WPS, int G = 1>
+__global__ __launch_bounds__(256 * G) __attribute__((amdgpu_waves_per_eu(WPS, WPS))) void w4a16_gemm_nsplit_kernel(W4A16PArgs a, int big_cols) {
   constexpr int BM = TM * 32, BN = 4 * TN * 32;
   extern __shared__ __align__(16) unsigned char smem[];
   const int tilesM = (a.M + BM - 1) / BM;
@@ -515,9 +552,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPS, WPS)))
       tm = b % tilesM;
       tn = b / tilesM;
     }
-    w4a16_nsplit_tile<TM, TN, BK>(a, tm * BM, tn * BN, smem);
+    w4a16_nsplit_tile<TM, TN, BK, G>(a, tm * BM, tn * BN, smem);
   } else {
-    if constexpr (TM >= 2) {
+    if constexpr (TM >= 2 && G == 1) {
       b = (int)blockIdx.x;
       w4a16_nsplit_tile<TM / 2, TN, BK>(a, (b % tilesH) * HM, (big_cols + b / tilesH) * BN, smem);
     }
@@ -539,6 +576,21 @@ __global__ void w4a16_dequant_packed_kernel(const uint8_t* __restrict__ P, uint1
 }
 
 static int g_w4a16_tail = 1;  // half-height tiles for a short last round (0 switches the schedule off: tuning/tests)
+
+// K in halves, eight waves per tile
+template <int TM, int TN, int BK>
+static int launch_w4a16_halves(const W4A16PArgs& a, hipStream_t st) {
+  constexpr int BM = TM * 32, BN = 4 * TN * 32;
+  constexpr size_t stage = 4 * (size_t)BM * (2 * BK + 16), patch = 4096 + 32 * (2 * (size_t)BN + 16), sums = (size_t)BM * BN * 4;
+  constexpr size_t lds = std::max(stage, std::max(patch, sums));
+  static_assert(lds <= 160 * 1024, "LDS of a CU");
+  auto kern = w4a16_gemm_nsplit_kernel<TM, TN, BK, 2, 2>;
+  if (lds > 64 * 1024)
+    HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  const int tilesM = (a.M + BM - 1) / BM, tilesN = (a.N + BN - 1) / BN;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tilesM * tilesN)), dim3(512), lds, st, a, tilesN);
+  return (int)hipGetLastError();
+}
 
 template <int TM, int TN, int BK, int WPS>
 static int launch_w4a16_nsplit(const W4A16PArgs& a, hipStream_t st) {
@@ -631,6 +683,22 @@ static int g_w4a16_ptile = 0;  // packed path: 0 = heuristic, 1 = 128x384, 2 = 6
 
 static int g_w4a16_waves = 1;  // 0: only the weights-from-global tiles (comparison runs and tests)
 
+// us that halves of K (eight waves) save a tile form, 0 where the four waves run: up to 256 tiles every tile has a CU to itself, and one wave per
+// SIMD dequantizes and multiplies in turns; above that two workgroups share a CU and the four are faster (1.05 to 1.3 of the time with halves).
+// Fitted to 71 to 84 shapes each within 1.7 % (rms).  Halves / whole, median over 298 shapes of 65 to 1500 rows: K up to 1500 0.91 to 0.97, up to 4000 0.79
+// to 0.87, beyond 0.73 to 0.83; the sums of 128 x 384 do not fit the LDS.
+static float w4a16_halves_gain(int form, int64_t M, int64_t N, int64_t K) {
+  struct Gain {
+    int bm, bn;
+    float less, block;
+  };
+  static const Gain gains[] = {{128, 128, 1.23f, 0.1892f}, {128, 256, 1.553f, 0.1981f}, {}, {64, 128, 0.671f, 0.094f}, {64, 384, 1.781f, 0.173f}};  // forms 4 to 8
+  if (form < 4 || form > 8 || !gains[form - 4].bm) return 0.f;
+  const Gain& g = gains[form - 4];
+  if (((M + g.bm - 1) / g.bm) * ((N + g.bn - 1) / g.bn) > 256) return 0.f;
+  return std::max(0.f, g.block * (float)((K + 63) / 64) - g.less);
+}
+
 // Which form runs.  The waves-split-K forms (wk_gemm.h) serve from one token to about the batch whose large tiles fill the chip;
 // 93 x 2048 x 6144: 43.6 -> 10.5 us, 1 x 2560 x 9728: 15.9 (a GEMV of fp32 FMAs) -> 11.9, 300 x 9728 x 2560: 36 -> 28, 2048 rows as before.
 // Two tables: where tiles of 128 x 256 would be fewer than 192, costs fitted to 1703 random shapes (5 to 6000 rows, 64 to 22 000 channels, K 64
@@ -664,7 +732,7 @@ static int w4a16_packed_form(int64_t M, int64_t N, int64_t K, bool tiles_only) {
   int form = -1;
   float best = 0.f;
   for (int f = tiles_only ? waves : 0; f < forms; f++) {
-    float c = form_cost(cost[f], M, N, K, (K + 63) / 64);
+    float c = form_cost(cost[f], M, N, K, (K + 63) / 64) - w4a16_halves_gain(f, M, N, K);
     // 64 x 64 by eight waves: fitted to 70 shapes of 100 to 256 such tiles, 2.2 % rms; over 250 shapes the choice takes 0.981 of the time with
     // four waves throughout, 41 of them 3 to 20 % less (119 x 7224 x 4416 20.6 -> 17.1 us)
     if (f == 3 && ((M + 63) / 64) * ((N + 63) / 64) <= WK_EIGHT_TILES) c -= 0.0322f * (float)((K + 63) / 64);
@@ -678,6 +746,7 @@ static int w4a16_packed_form(int64_t M, int64_t N, int64_t K, bool tiles_only) {
 static int launch_w4a16_auto(const W4A16PArgs& a, hipStream_t st) {
   static const int tiles[] = {-1, 6, 8, 4, 7, 5};  // of g_w4a16_ptile
   const int form = g_w4a16_ptile ? tiles[g_w4a16_ptile] : w4a16_packed_form(a.M, a.N, a.K, !g_w4a16_waves);
+  const bool halves = !g_w4a16_ptile && w4a16_halves_gain(form, a.M, a.N, a.K) > 0.f;  // (a tile asked for runs by four waves)
   if (a.M <= 8) switch (form) {  // one piece of eight rows; faster at every size measured (512 to 22016 channels, K 512 to 11008)
     case 0: return wk_gemm_launch<W4A16Waves, 1, 1, 16, 2, 1>(a, st);
     case 1: return wk_gemm_launch<W4A16Waves, 1, 1, 8, 3, 1>(a, st);
@@ -689,11 +758,11 @@ static int launch_w4a16_auto(const W4A16PArgs& a, hipStream_t st) {
     case 1: return wk_gemm_launch<W4A16Waves, 1, 1, 8, 3>(a, st);
     case 2: return wk_gemm_launch<W4A16Waves, 1, 2, 8, 1>(a, st);
     case 3: return wk_gemm_64x64<W4A16Waves>(a, st);
-    case 4: return launch_w4a16_nsplit<4, 1, 64, 3>(a, st);
-    case 5: return launch_w4a16_nsplit<4, 2, 64, 2>(a, st);
+    case 4: return halves ? launch_w4a16_halves<4, 1, 64>(a, st) : launch_w4a16_nsplit<4, 1, 64, 3>(a, st);
+    case 5: return halves ? launch_w4a16_halves<4, 2, 64>(a, st) : launch_w4a16_nsplit<4, 2, 64, 2>(a, st);
     case 6: return launch_w4a16_nsplit<4, 3, 128, 1>(a, st);
-    case 7: return launch_w4a16_nsplit<2, 1, 128, 2>(a, st);
-    case 8: return launch_w4a16_nsplit<2, 3, 128, 2>(a, st);
+    case 7: return halves ? launch_w4a16_halves<2, 1, 128>(a, st) : launch_w4a16_nsplit<2, 1, 128, 2>(a, st);
+    case 8: return halves ? launch_w4a16_halves<2, 3, 128>(a, st) : launch_w4a16_nsplit<2, 3, 128, 2>(a, st);
     default: return wk_gemm_launch<W4A16Waves, 1, 1, 4, 1>(a, st);
   }
 }

@@ -275,9 +275,18 @@ def test_waves_that_split_k_of_larger_tiles():
 
 
 def test_waves_that_split_k_of_64x64_tiles_by_eight_and_four_waves():
-    """256 such tiles (eight waves) and 258 (four), K blocks that do not divide among the waves"""
-    shapes = ((128, 8192, 1984, 64), (128, 8193, 1984, 64))
+    """256 such tiles (eight waves) and 510 (four), ragged rows and channels, K blocks that do not divide among the waves"""
+    shapes = ((119, 8134, 1216, 64), (322, 5380, 576, 64))
     assert [_lib.lib().mllm_hip_w4a16_packed_form(*s[:3]) for s in shapes] == [4, 4]
+    _waves_cases(shapes)
+
+
+def test_halves_of_k():
+    """tiles of 128x128, 64x128, 128x256 and 64x384 that have a CU to themselves, by eight waves with half of K each: ragged rows and channels,
+    an odd number of K steps (the second half has one less), N % 8 != 0 (element stores); the last one past 256 tiles, by four"""
+    shapes = ((643, 4110, 576, 64), (643, 3856, 640, 64), (226, 4113, 576, 64), (225, 4104, 640, 128), (257, 3592, 576, 64),
+              (771, 7952, 576, 64), (515, 8256, 1152, 64), (451, 4110, 576, 64))
+    assert [_lib.lib().mllm_hip_w4a16_packed_form(*s[:3]) for s in shapes] == [5, 5, 8, 8, 8, 6, 9, 8]
     _waves_cases(shapes)
 
 
