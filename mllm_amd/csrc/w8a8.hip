@@ -9,6 +9,8 @@
 //                      y = out_dtype( float(acc_int32) * (w_scale[n] * x_scale[m]) + bias[n] )
 // The int32 accumulators are exact, so they match any other exact implementation bit for bit.
 #include "qcommon.h"
+#include <algorithm>
+
 #include "wk_gemm.h"
 
 namespace mllmhip {
@@ -327,15 +329,18 @@ __global__ __launch_bounds__(256) void w8a8_prepack_kernel(const int8_t* __restr
 // Scheduling barriers pin the hand-made software pipeline: left alone, the compiler sinks all global loads to the end
 // of the loop body and exposes their latency.
 // WPS: waves per SIMD the register budget is held to (workgroups of 4 waves: WPS workgroups per CU).
-template <int TM, int TN, bool PK, int WPS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPS, WPS))) void w8a8_gemm_nsplit_kernel(W8A8Args a) {
+// G == 2: eight waves, the second four take the second half of K with a stage of their own; their sums join the first's in LDS (exact).
+template <int TM, int TN, bool PK, int WPS, int G = 1>
+__global__ __launch_bounds__(256 * G) __attribute__((amdgpu_waves_per_eu(WPS, WPS))) void w8a8_gemm_nsplit_kernel(W8A8Args a) {
   constexpr int BK = 128, LDK = 144, KS = BK / 32;
   constexpr int BM = TM * 32, WN = TN * 32, BN = 4 * WN;
   constexpr int CA = BM * (BK / 16) / 256;  // 16-byte activation chunks per thread and K step
   constexpr int STAGE = BM * LDK;
-  extern __shared__ __align__(16) unsigned char smem[];
+  extern __shared__ __align__(16) unsigned char smem_all[];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  unsigned char* const smem = smem_all + group * 2 * STAGE;
+  const int tid = G == 1 ? threadIdx.x : threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 31, hi = lane >> 5;
   const int tilesN = (a.N + BN - 1) / BN, tilesM = (a.M + BM - 1) / BM;
   const int tile = xcd_run(blockIdx.x, tilesM * tilesN);           // one run of tiles per XCD ...
@@ -390,21 +395,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPS, WPS)))
 #pragma unroll
       for (int r = 0; r < 16; r++) acc[j][i][r] = 0;
 
-  const int KT = Kw / BK;
+  // K steps of these waves: all of them, or one of the halves (idle: how many fewer the second has, whose barriers it keeps)
+  const int KT = Kw / BK, per = (KT + G - 1) / G, kt0 = group * per, kt1 = min(KT, kt0 + per), idle = G == 1 ? 0 : per - (kt1 - kt0);
   u32x4 ga[CA];
   v4i fb[KS][TN];
   v4i fa[2][TM];
-  loadA(0, ga);
+  loadA(kt0 * BK, ga);
 #pragma unroll
   for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-    for (int j = 0; j < TN; j++) fb[ks][j] = loadB(0, ks, j);
+    for (int j = 0; j < TN; j++) fb[ks][j] = loadB(kt0 * BK, ks, j);
   storeA(0, ga);
   __syncthreads();
   readA(0, 0, fa[0]);
 
-  for (int kt = 0; kt < KT; kt++) {
-    const int buf = kt & 1, k1 = (kt + 1) * BK;
+  for (int kt = kt0; kt < kt1; kt++) {
+    const int buf = (kt - kt0) & 1, k1 = (kt + 1) * BK;
     loadA(k1, ga);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -427,10 +433,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPS, WPS)))
       }
     }
   }
+  for (int i = 0; i < idle; i++) __syncthreads();
   __syncthreads();  // all LDS reads done before the scales overwrite the tiles
+  if constexpr (G == 2) {
+    v4i* part = reinterpret_cast<v4i*>(smem_all);
+    auto quad = [&](int j, int i, int g) -> v4i& { return part[(((wave * TN + j) * TM + i) * 4 + g) * 64 + lane]; };
+    if (group == 1) {
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int g = 0; g < 4; g++) quad(j, i, g) = v4i{acc[j][i][4 * g], acc[j][i][4 * g + 1], acc[j][i][4 * g + 2], acc[j][i][4 * g + 3]};
+    }
+    __syncthreads();
+    if (group == 0) {
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int g = 0; g < 4; g++) {
+            const v4i v = quad(j, i, g);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[j][i][4 * g + e] += v[e];
+          }
+    }
+    __syncthreads();
+  }
 
   // acc[j][i][4g+e] = C[m0 + 32i + lrow][n0 + wave*WN + 32j + 8g + 4hi + e]
-  float* sXs = reinterpret_cast<float*>(smem);
+  float* sXs = reinterpret_cast<float*>(smem_all);
   float* sWs = sXs + BM;
   float* sBi = sWs + BN;
   for (int i = tid; i < BM; i += 256) sXs[i] = (a.xs && m0 + i < a.M) ? a.xs[m0 + i] : 0.f;
@@ -443,7 +476,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPS, WPS)))
   // of results is turned through LDS so that a wave stores whole rows of the workgroup's BN columns (runs of whole
   // cache lines, 16 bytes per lane).
   constexpr int ROWB = 2 * BN + 16;
-  unsigned char* patch = smem + 4096;
+  unsigned char* patch = smem_all + 4096;
   static_assert((BM + 2 * BN) * 4 <= 4096, "scales overlap the store patch");
   // 16-byte pieces; those of ragged edges fall outside the buffer (whose end a row or column past the tile must not wrap over)
   const bool pieces = a.N % 8 == 0 && reinterpret_cast<uintptr_t>(a.C) % 16 == 0 && ((int64_t)a.M + BM) * a.N * 2 < ((int64_t)1 << 32);
@@ -459,29 +492,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPS, WPS)))
       }
     const bool has_bias = a.bias != nullptr;
     constexpr int CPR = BN / 8;  // 16-byte pieces per row
-    static_assert((8 * CPR) % 64 == 0, "a wave stores whole rows");
+    constexpr int RPW = 8 / G;   // rows per wave
+    static_assert((RPW * CPR) % 64 == 0, "a wave stores whole rows");
 #pragma unroll
     for (int i = 0; i < TM; i++) {
       const float xsm = sXs[i * 32 + lrow];
+      if (group == 0) {
 #pragma unroll
-      for (int j = 0; j < TN; j++)
+        for (int j = 0; j < TN; j++)
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-          float f[4];
+          for (int g = 0; g < 4; g++) {
+            float f[4];
 #pragma unroll
-          for (int e = 0; e < 4; e++) f[e] = (float)acc[j][i][4 * g + e] * (ws4[j][g][e] * xsm);
-          if (has_bias) {
+            for (int e = 0; e < 4; e++) f[e] = (float)acc[j][i][4 * g + e] * (ws4[j][g][e] * xsm);
+            if (has_bias) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) f[e] += bi4[j][g][e];
+              for (int e = 0; e < 4; e++) f[e] += bi4[j][g][e];
+            }
+            *reinterpret_cast<uint2*>(patch + lrow * ROWB + (wave * WN + j * 32 + 8 * g + 4 * hi) * 2) =
+                uint2{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3])};
           }
-          *reinterpret_cast<uint2*>(patch + lrow * ROWB + (wave * WN + j * 32 + 8 * g + 4 * hi) * 2) =
-              uint2{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3])};
-        }
+      }
       __syncthreads();
 #pragma unroll
-      for (int t = 0; t < 8 * CPR / 64; t++) {  // wave w stores rows 8w .. 8w+7
+      for (int t = 0; t < RPW * CPR / 64; t++) {  // wave w stores rows RPW w .. RPW (w + 1) - 1
         const int c = lane + 64 * t;
-        const int row = wave * 8 + c / CPR, cc = c % CPR;
+        const int row = (group * 4 + wave) * RPW + c / CPR, cc = c % CPR;
         const u32x4 v = *reinterpret_cast<const u32x4*>(patch + row * ROWB + cc * 16);
         const int n = n0 + cc * 8;
         // (a row past M lies past the end of the buffer)
@@ -491,6 +527,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPS, WPS)))
     }
     return;
   }
+  if (group != 0) return;
 #pragma unroll
   for (int i = 0; i < TM; i++) {
     const int m = m0 + i * 32 + lrow;
@@ -527,6 +564,21 @@ static int launch_w8a8_nsplit(const W8A8Args& a, hipStream_t st) {
   const size_t lds = stage > patch ? stage : patch;
   const unsigned grid = (unsigned)(((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN));
   hipLaunchKernelGGL((w8a8_gemm_nsplit_kernel<TM, TN, PK, WPS>), dim3(grid), dim3(256), lds, st, a);
+  return (int)hipGetLastError();
+}
+
+// K in halves, eight waves per tile
+template <int TM, int TN>
+static int launch_w8a8_halves(const W8A8Args& a, hipStream_t st) {
+  constexpr int BM = TM * 32, BN = 4 * TN * 32;
+  constexpr size_t stage = 4 * (size_t)BM * 144, patch = 4096 + 32 * (2 * (size_t)BN + 16), sums = (size_t)BM * BN * 4;
+  constexpr size_t lds = std::max(stage, std::max(patch, sums));
+  static_assert(lds <= 160 * 1024, "LDS of a CU");
+  auto kern = w8a8_gemm_nsplit_kernel<TM, TN, true, 2, 2>;
+  if (lds > 64 * 1024)
+    HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  const unsigned grid = (unsigned)(((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN));
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), lds, st, a);
   return (int)hipGetLastError();
 }
 
@@ -794,6 +846,17 @@ static bool launch_w8a8_gemv_packed(const W8A8Args& a, hipStream_t st, int* rc, 
                     : go(w8a8_gemv_packed_kernel<4, MLLM_HIP_BF16>);
   return true;
 }
+// us that halves of K (eight waves) save a tile form, 0 where the four waves run: up to 256 tiles every tile has a CU to itself, and one wave per
+// SIMD waits for its own loads; above that two workgroups share a CU and the four are faster (1.13 to 1.28 of the time with halves).  Fitted to 108 shapes each
+// within 2.6 % (rms).  Halves / whole, median over 299 shapes of 65 to 2048 rows, K up to 1500 / 4000 / beyond: 64 x 128 0.98 / 0.89 / 0.83, 128 x 128 1.02 / 0.94 /
+// 0.87; 128 x 256 1.10 / 1.02 / 0.97 and 64 x 384 1.11 / 1.06 / 1.03 stay with four.
+static float w8a8_halves_gain(int form, int64_t M, int64_t N, int64_t K) {
+  if (form != 3 && form != 4) return 0.f;
+  const int bm = form == 3 ? 64 : 128;
+  if (((M + bm - 1) / bm) * ((N + 127) / 128) > 256) return 0.f;
+  const float blocks = (float)((K + 127) / 128);
+  return std::max(0.f, form == 3 ? 0.1193f * blocks - 0.55f : 0.1264f * blocks - 1.111f);
+}
 // Which matrix-core form runs against packed weights.  Waves that split K (wk_gemm.h) from a few tokens to about the batch whose
 // large tiles fill the chip (93 x 2560 x 9728: 38 -> 11 us, 300 x 2560 x 9728: 41 -> 20, 32 x 4096 x 4096: 13.5 -> 7.6), then the
 // weights-from-global tiles.  Over 1850 random shapes (5 to 6000 rows, 64 to 22 000 channels, K 64 to 10 000) the choice takes 1.008 times the
@@ -820,7 +883,10 @@ static int w8a8_packed_form(int64_t M, int64_t N, int64_t K) {
   int form = 0;
   float best = 0.f;
   for (int f = 0; f < forms; f++) {
-    const float c = form_cost(cost[f], M, N, K, (K + 127) / 128);
+    float c = form_cost(cost[f], M, N, K, (K + 127) / 128);
+    // (fewer than half a round of tiles: their cost is up to 40 % more than the table's on long rows, and the waves' forms are the better ones)
+    if (M > 32 && ((M + cost[f].bm - 1) / cost[f].bm) * ((N + cost[f].bn - 1) / cost[f].bn) > 128)
+      c -= std::max(0.f, w8a8_halves_gain(f, M, N, K) - (f == 4 ? 1.2f : 0.f));  // (or it took the place of more tiles of 64 x 128 that were 3 to 7 % faster)
     if (f == 0 || c < best) {
       best = c;
       form = f;
@@ -830,12 +896,14 @@ static int w8a8_packed_form(int64_t M, int64_t N, int64_t K) {
 }
 static int launch_w8a8_packed_auto(const W8A8Args& a, hipStream_t st) {
   if (g_w8a8_ntile || !g_w8a8_decode) return launch_w8a8_nsplit_auto<true>(a, st);
-  switch (w8a8_packed_form(a.M, a.N, a.K)) {
+  const int form = w8a8_packed_form(a.M, a.N, a.K);
+  const bool halves = w8a8_halves_gain(form, a.M, a.N, a.K) > 0.f;
+  switch (form) {
     case 0: return wk_gemm_launch<W8A8Waves, 1, 1, 8, 2>(a, st);
     case 1: return wk_gemm_launch<W8A8Waves, 1, 2, 8, 1>(a, st);
     case 2: return wk_gemm_launch<W8A8Waves, 2, 2, 8, 1>(a, st);
-    case 3: return launch_w8a8_nsplit<2, 1, true, 2>(a, st);
-    case 4: return launch_w8a8_nsplit<4, 1, true, 2>(a, st);
+    case 3: return halves ? launch_w8a8_halves<2, 1>(a, st) : launch_w8a8_nsplit<2, 1, true, 2>(a, st);
+    case 4: return halves ? launch_w8a8_halves<4, 1>(a, st) : launch_w8a8_nsplit<4, 1, true, 2>(a, st);
     case 5: return launch_w8a8_nsplit<4, 2, true, 2>(a, st);
     case 6: return launch_w8a8_nsplit<2, 3, true, 2>(a, st);
     default: return launch_w8a8_nsplit<4, 3, true, 1>(a, st);

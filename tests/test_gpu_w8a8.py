@@ -301,6 +301,15 @@ def test_waves_that_split_k_of_larger_tiles():
     _waves_cases(small + large)
 
 
+def test_halves_of_k():
+    """tiles of 64x128 and 128x128 that have a CU to themselves, by eight waves with half of K each: ragged rows and channels, an odd number of K
+    steps (the second half has one less), N % 8 != 0 (element stores); the last one of each past 256 tiles, by four"""
+    shapes = ((99, 4116, 704), (98, 4172, 640), (129, 3288, 704), (105, 4128, 640), (451, 4110, 640),
+              (834, 3869, 1216), (833, 3872, 1216), (900, 3723, 1088), (841, 3984, 1088), (838, 4100, 704))
+    assert [_lib.lib().mllm_hip_w8a8_packed_form(*s) for s in shapes] == [4] * 5 + [5] * 5
+    _waves_cases(shapes)
+
+
 def _waves_cases(shapes):
     L = _lib.lib()
     for M, N, K in shapes:
