@@ -165,10 +165,11 @@ def test_q_gemm_every_form_exact(wtype, M, N, K):
         assert L.mllm_hip_q_gemm_set_form(0) == 0
 
 
-@pytest.mark.parametrize("M,N,K", [(1024, 1024, 96), (1025, 1024, 96), (97, 8192, 800), (97, 8193, 800)])
-def test_linear_q_gemm_64x64_tiles_by_eight_and_four_waves(M, N, K):
-    """either side of 256 tiles: fewer K blocks than waves and blocks that do not divide among them; integers whose sums are exact in any order
-    (scales of one, no partial sum leaves 2^24)"""
+@pytest.mark.parametrize("M,N,K,form", [(1024, 1024, 96, 3), (1025, 1024, 96, 3), (97, 8192, 800, 3), (97, 8193, 800, 3), (100, 8188, 1024, 12),
+                                        (100, 8448, 1024, 12), (129, 4100, 1184, 8), (129, 8448, 1184, 8)])
+def test_linear_q_gemm_by_eight_and_four_waves(M, N, K, form):
+    """either side of 256 tiles of 64 x 64 (fewer K blocks than waves and blocks that do not divide among them) and of 256 workgroups of ranges
+    of K (ranges of two and of four K steps, the last one shorter); integers whose sums are exact in any order (scales of one, no partial sum leaves 2^24)"""
     L = _lib.lib()
     rng = synth.rng_for(4, 1700 + M + N + K)
     W = synth.make_weight(rng, 0, N, K)
@@ -178,9 +179,9 @@ def test_linear_q_gemm_64x64_tiles_by_eight_and_four_waves(M, N, K):
     x = rng.integers(-3, 4, (M, K)).astype(np.float32)
     x[:, ::32] = 127.0
     w = ql.PackedQWeight(0, torch.from_numpy(W), layout="gemm")
-    announce("q gemm 64 x 64", M, N, K)
+    announce("q gemm by eight and four waves", M, N, K, form)
     try:
-        assert L.mllm_hip_q_gemm_set_form(3) == 0
+        assert L.mllm_hip_q_gemm_set_form(form) == 0 and L.mllm_hip_q_gemm_form(0, M, N, K, 1) == form
         assert np.array_equal(ql.linear_q_gemm(w, to_dev(x), None, ql.SCALE_IEEE, short=True).cpu().numpy(), x @ wd.T)
     finally:
         assert L.mllm_hip_q_gemm_set_form(0) == 0
