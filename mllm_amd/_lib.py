@@ -136,6 +136,7 @@ def lib():
         L.mllm_hip_w8a8_set_tuning.argtypes = [ci]
         L.mllm_hip_w8a8_nsplit_set_tuning.argtypes = [ci]
         L.mllm_hip_w8a8_packed_form.argtypes = [i64, i64, i64]
+        L.mllm_hip_w8a8_packed_halves.argtypes = [i64, i64, i64]
         L.mllm_hip_w8a8_packed_bytes.restype = C.c_size_t
         L.mllm_hip_w8a8_packed_bytes.argtypes = [i64, i64]
         L.mllm_hip_w8a8_prepack.argtypes = [vp, i64, i64, vp, vp]

@@ -846,16 +846,17 @@ static bool launch_w8a8_gemv_packed(const W8A8Args& a, hipStream_t st, int* rc, 
                     : go(w8a8_gemv_packed_kernel<4, MLLM_HIP_BF16>);
   return true;
 }
-// us that halves of K (eight waves) save a tile form, 0 where the four waves run: up to 256 tiles every tile has a CU to itself, and one wave per
-// SIMD waits for its own loads; above that two workgroups share a CU and the four are faster (1.13 to 1.28 of the time with halves).  Fitted to 108 shapes each
-// within 2.6 % (rms).  Halves / whole, median over 299 shapes of 65 to 2048 rows, K up to 1500 / 4000 / beyond: 64 x 128 0.98 / 0.89 / 0.83, 128 x 128 1.02 / 0.94 /
-// 0.87; 128 x 256 1.10 / 1.02 / 0.97 and 64 x 384 1.11 / 1.06 / 1.03 stay with four.
-static float w8a8_halves_gain(int form, int64_t M, int64_t N, int64_t K) {
-  if (form != 3 && form != 4) return 0.f;
+// Whether a tile form runs as halves of K by eight waves: up to 256 tiles every tile has a CU to itself, and one wave per SIMD waits for its own
+// loads; above that two workgroups share a CU and the four are faster (1.13 to 1.28 of the time with halves).  Halves / whole over 1500 shapes of 5 to 3000 rows,
+// mean (most): 64 x 128 five blocks of 128 1.01 (1.03), six 0.98 (1.00), sixteen 0.94, more 0.85 to 0.90; 128 x 128 eight 1.01 (1.03), nine to sixteen 0.98 (1.025),
+// up to 32 0.94, more 0.90.  One tile of rows and more than 192 of channels, where the weights' bytes are the bound: 1.02 (1.05) up to 23 blocks, 0.94 beyond.
+// 128 x 256 (1.10 to 0.97) and 64 x 384 (1.11 to 1.03) stay with four.
+static bool w8a8_halves(int form, int64_t M, int64_t N, int64_t K) {
+  if (form != 3 && form != 4) return false;
   const int bm = form == 3 ? 64 : 128;
-  if (((M + bm - 1) / bm) * ((N + 127) / 128) > 256) return 0.f;
-  const float blocks = (float)((K + 127) / 128);
-  return std::max(0.f, form == 3 ? 0.1193f * blocks - 0.55f : 0.1264f * blocks - 1.111f);
+  const int64_t tiles = ((M + bm - 1) / bm) * ((N + 127) / 128), blocks = (K + 127) / 128;
+  if (M <= 64 && tiles > 192 && blocks < 24) return false;
+  return tiles <= 256 && blocks >= (form == 3 ? 6 : 10);
 }
 // Which matrix-core form runs against packed weights.  Waves that split K (wk_gemm.h) from a few tokens to about the batch whose
 // large tiles fill the chip (93 x 2560 x 9728: 38 -> 11 us, 300 x 2560 x 9728: 41 -> 20, 32 x 4096 x 4096: 13.5 -> 7.6), then the
@@ -864,6 +865,8 @@ static float w8a8_halves_gain(int form, int64_t M, int64_t N, int64_t K) {
 // rows and columns alone that ran before in 17 (2806 x 208 x 3968: 14.7, 11.5 at most).  More than 32 rows: fitted to 1300 of them within 5 to
 // 8 % (rms, where a form is near the best); a table fitted to 170 shapes of 93 rows and more, without the prices of M K and M N, made the
 // choice 1.021, 169 and 97 (1811 x 264 x 1280 7.6 us, 6.4 now), but is as good up to 32 rows (1.009 of the best) and stays there.
+// Costs are those of four waves: with a gain of halves taken off them, 190 of 1500 shapes went from tiles of 64 x 128 (or 64 x 64 by eight waves) to halves of larger
+// ones, 1.01 of their time on average, 71 of them 3 to 22 % slower and 34 3 to 15 % faster (1155 x 1912 x 4288 28.7 -> 31.3 us, 927 x 1032 x 9728 33.5 -> 40.9).
 static int w8a8_packed_form(int64_t M, int64_t N, int64_t K) {
   constexpr int forms = 8;
   static const FormCost many[forms] = {
@@ -883,10 +886,7 @@ static int w8a8_packed_form(int64_t M, int64_t N, int64_t K) {
   int form = 0;
   float best = 0.f;
   for (int f = 0; f < forms; f++) {
-    float c = form_cost(cost[f], M, N, K, (K + 127) / 128);
-    // (fewer than half a round of tiles: their cost is up to 40 % more than the table's on long rows, and the waves' forms are the better ones)
-    if (M > 32 && ((M + cost[f].bm - 1) / cost[f].bm) * ((N + cost[f].bn - 1) / cost[f].bn) > 128)
-      c -= std::max(0.f, w8a8_halves_gain(f, M, N, K) - (f == 4 ? 1.2f : 0.f));  // (or it took the place of more tiles of 64 x 128 that were 3 to 7 % faster)
+    const float c = form_cost(cost[f], M, N, K, (K + 127) / 128);
     if (f == 0 || c < best) {
       best = c;
       form = f;
@@ -897,7 +897,7 @@ static int w8a8_packed_form(int64_t M, int64_t N, int64_t K) {
 static int launch_w8a8_packed_auto(const W8A8Args& a, hipStream_t st) {
   if (g_w8a8_ntile || !g_w8a8_decode) return launch_w8a8_nsplit_auto<true>(a, st);
   const int form = w8a8_packed_form(a.M, a.N, a.K);
-  const bool halves = w8a8_halves_gain(form, a.M, a.N, a.K) > 0.f;
+  const bool halves = w8a8_halves(form, a.M, a.N, a.K);
   switch (form) {
     case 0: return wk_gemm_launch<W8A8Waves, 1, 1, 8, 2>(a, st);
     case 1: return wk_gemm_launch<W8A8Waves, 1, 2, 8, 1>(a, st);
@@ -912,6 +912,9 @@ static int launch_w8a8_packed_auto(const W8A8Args& a, hipStream_t st) {
 MLLM_API int mllm_hip_w8a8_packed_form(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || N < 1 || K < 1) return 0;
   return M < 5 ? 9 : 1 + w8a8_packed_form(M, N, K);
+}
+MLLM_API int mllm_hip_w8a8_packed_halves(int64_t M, int64_t N, int64_t K) {
+  return M >= 5 && N >= 1 && K >= 1 && w8a8_halves(w8a8_packed_form(M, N, K), M, N, K);
 }
 MLLM_API int mllm_hip_w8a8_set_decode(int gemv) {
   if (gemv != 0 && gemv != 1) return MLLM_HIP_E_BADARG;

@@ -93,6 +93,7 @@ def _cases():
         "mllm_hip_w4a16_set_decode_mfma_from": ([2], [(0, 0, BADARG), (0, 34, BADARG)]),
         "mllm_hip_q_gemm_set_form": ([0], [(0, 13, BADARG), (0, -1, BADARG)]),
         "mllm_hip_w8a8_packed_form": ([64, 64, 64], [(0, 0, 0), (1, -1, 0), (2, 0, 0)]),
+        "mllm_hip_w8a8_packed_halves": ([64, 64, 64], [(0, 0, 0), (1, -1, 0), (2, 0, 0)]),
         "mllm_hip_w4a16_packed_form": ([64, 64, 64], [(0, 0, 0), (1, -1, 0), (2, 0, 0)]),
         "mllm_hip_q_gemm_form": ([Q4_0, 64, 64, 256, 1], [(0, 5, 0), (1, 0, 0), (2, 0, 0), (3, -1, 0)]),
         "mllm_hip_moe_gate_set_form": ([1], [(0, 2, BADARG), (0, -1, BADARG)]),
@@ -205,6 +206,24 @@ def test_w8a8_takes_a_form_that_measures_fast(M, N, K, form):
     L = _lib.lib()
     assert L.mllm_hip_w8a8_packed_form(M, N, K) == form
     assert [L.mllm_hip_w8a8_packed_form(t, N, K) for t in (1, 4)] == [9, 9] and len({L.mllm_hip_w8a8_packed_form(t, N, K) for t in (5, 17, 32)}) == 1
+
+
+@pytest.mark.parametrize("M,N,K,form", [(1155, 1912, 4288, 4), (338, 5456, 4928, 4), (998, 2488, 3904, 4), (927, 1032, 9728, 3), (270, 3232, 7040, 3), (1204, 803, 6592, 3)])
+def test_w8a8_keeps_the_form_that_halves_of_larger_tiles_do_not_beat(M, N, K, form):
+    """shapes at which a gain of halves of K in the choice took larger tiles, 8 to 22 % slower"""
+    assert _lib.lib().mllm_hip_w8a8_packed_form(M, N, K) == form
+
+
+def test_w8a8_runs_halves_of_k_where_they_are_faster():
+    """from six (64 x 128) and ten (128 x 128) blocks of 128 on, up to 256 tiles; with fewer blocks halves took up to 1.07 and 1.12 of the time"""
+    L = _lib.lib()
+    for M, N, block, form in ((99, 16384, 6, 4), (128, 12288, 6, 4), (728, 5064, 10, 5), (488, 8184, 10, 5)):
+        for blocks, halves in ((block - 1, 0), (block, 1)):
+            assert (L.mllm_hip_w8a8_packed_form(M, N, 128 * blocks), L.mllm_hip_w8a8_packed_halves(M, N, 128 * blocks)) == (form, halves)
+    assert (L.mllm_hip_w8a8_packed_form(128, 16512, 768), L.mllm_hip_w8a8_packed_halves(128, 16512, 768)) == (4, 0)  # 258 tiles
+    for N, blocks, halves in ((24576, 23, 1), (24584, 23, 0), (24584, 24, 1)):  # one tile of rows and more than 192 of channels
+        assert (L.mllm_hip_w8a8_packed_form(33, N, 128 * blocks), L.mllm_hip_w8a8_packed_halves(33, N, 128 * blocks)) == (4, halves)
+    assert L.mllm_hip_w8a8_packed_halves(4, 4096, 4096) == 0 and L.mllm_hip_w8a8_packed_halves(2048, 6144, 2048) == 0
 
 
 @pytest.mark.parametrize("M,N,K,form", [(3500, 456, 1280, 8), (4580, 576, 512, 8), (5226, 376, 2688, 8), (738, 2720, 384, 8), (2048, 9728, 2560, 6), (93, 2048, 6144, 2),
