@@ -370,9 +370,11 @@ int mllm_hip_w4a16_set_decode_mfma_from(int tokens);
  * + 16 switches off the half-height tiles that shorten a partly filled last round. */
 int mllm_hip_w4a16_packed_set_tuning(int tile);
 /* The form that a product of this size takes: waves that split K of a tile of 32x32 by 1: sixteen, 2: eight, 10: four, 3: 32x64, 4: 64x64; tiles of
- * 5: 128x128, 6: 128x256, 7: 128x384, 8: 64x128, 9: 64x384 (all but 7 by eight waves with half of K each while every tile has a CU to itself).
- * Host only, overrides aside.  No counterpart in the reference. */
+ * 5: 128x128, 6: 128x256, 7: 128x384, 8: 64x128, 9: 64x384.  mllm_hip_w4a16_packed_eight: 1 where forms 4, 5, 6, 8 and 9 run by eight waves (4: an eighth
+ * of K each, the others half of it) instead of four: every tile has a CU to itself and K is more than 384 (4, 5), 448 (6, 8) or 640 (9).  Host only, overrides
+ * aside.  No counterpart in the reference. */
 int mllm_hip_w4a16_packed_form(int64_t M, int64_t N, int64_t K);
+int mllm_hip_w4a16_packed_eight(int64_t M, int64_t N, int64_t K);
 
 /* ---------------------------------------------------------------------------------------------------------
  * MoE expert FFN over expert-sorted tokens, Q4_0 / Q8_0 expert weights

@@ -148,6 +148,7 @@ def lib():
         L.mllm_hip_w4a16_set_tuning.argtypes = [ci]
         L.mllm_hip_w4a16_packed_set_tuning.argtypes = [ci]
         L.mllm_hip_w4a16_packed_form.argtypes = [i64, i64, i64]
+        L.mllm_hip_w4a16_packed_eight.argtypes = [i64, i64, i64]
         L.mllm_hip_w4a16_packed_bytes.restype = C.c_size_t
         L.mllm_hip_w4a16_packed_bytes.argtypes = [i64, i64, ci]
         L.mllm_hip_w4a16_prepack.argtypes = [vp, vp, vp, i64, i64, ci, vp, vp]

@@ -1766,7 +1766,7 @@ struct QWaves {
   struct Col {
     uint32_t q, s;
   };
-  static __device__ __forceinline__ int kblocks(const Args& a) { return (a.K + 63) / 64; }
+  static __host__ __device__ __forceinline__ int kblocks(const Args& a) { return (a.K + 63) / 64; }
   static __device__ __forceinline__ int row_bytes(const Args& a) { return a.K * 2; }
   static __device__ __forceinline__ const void* activations(const Args& a) { return a.xh; }
   static __device__ __forceinline__ __amdgpu_buffer_rsrc_t weights(const Args& a) {
@@ -1913,7 +1913,7 @@ static QLinearPlan q_linear_plan(int wtype, int64_t M, int64_t N, int64_t K, boo
   for (int f = 0; f < 3; f++) {
     const int64_t tiles = ((M + rows[f] - 1) / rows[f]) * ((N + chans[f] - 1) / chans[f]);
     const float cost = whole(c.waves[f], (float)((tiles + 255) / 256), (float)tiles / 256.f);
-    const float eight = f == 2 && tiles <= WK_EIGHT_TILES ? c.eight * (float)blocks : 0.f;
+    const float eight = f == 2 && wk_eight(M, N, blocks) ? c.eight * (float)blocks : 0.f;
     offer(cost - eight, QLinearPlan{f, 0, 1});
     // Tiles of 128 x 256 give way to the eight waves only where the costs differ by more than their errors.  Over 479 shapes 0.992 of the time with
     // four waves throughout, 44 of them 3 to 18 % faster (180 x 3120 x 7680 Q4_0 33.6 -> 27.6 us), none slower.

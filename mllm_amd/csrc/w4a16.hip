@@ -640,7 +640,7 @@ struct W4A16Waves {
     uint32_t q, sz;
     int g64, last;
   };
-  static __device__ __forceinline__ int kblocks(const Args& a) { return (a.K + 63) / 64; }
+  static __host__ __device__ __forceinline__ int kblocks(const Args& a) { return (a.K + 63) / 64; }
   static __device__ __forceinline__ int row_bytes(const Args& a) { return a.K * 2; }
   static __device__ __forceinline__ const void* activations(const Args& a) { return a.A; }
   static __device__ __forceinline__ __amdgpu_buffer_rsrc_t weights(const Args& a) {
@@ -729,19 +729,31 @@ static int w4a16_packed_form(int64_t M, int64_t N, int64_t K, bool tiles_only) {
   const bool large = ((M + 127) / 128) * ((N + 255) / 256) >= 192;
   const FormCost* cost = large ? many : few;
   const int forms = large ? 7 : most;
-  int form = -1;
-  float best = 0.f;
-  for (int f = tiles_only ? waves : 0; f < forms; f++) {
-    float c = form_cost(cost[f], M, N, K, (K + 63) / 64) - w4a16_halves_gain(f, M, N, K);
-    // 64 x 64 by eight waves: fitted to 70 shapes of 100 to 256 such tiles, 2.2 % rms; over 250 shapes the choice takes 0.981 of the time with
-    // four waves throughout, 41 of them 3 to 20 % less (119 x 7224 x 4416 20.6 -> 17.1 us)
-    if (f == 3 && ((M + 63) / 64) * ((N + 63) / 64) <= WK_EIGHT_TILES) c -= 0.0322f * (float)((K + 63) / 64);
-    if (form < 0 || c < best) {
-      best = c;
-      form = f;
+  // What eight waves save comes off: halves of K as above; 64 x 64 fitted to 70 shapes of 100 to 256 such tiles, 2.2 % rms; over 250 shapes the choice takes
+  // 0.981 of the time with four waves throughout, 41 of them 3 to 20 % less (119 x 7224 x 4416 20.6 -> 17.1 us).  Where a form of the waves that split K is the
+  // cheapest by four, halves of K of a tile take its place only
+  //  * with 2 us per million results added where rows are no multiple of 16 bytes: the tiles store those an element at a time (1.4 to 3 us by form, the
+  //    waves' forms nothing), which had 40 of 372 such shapes 3 to 25 % slower (778 x 1915 x 1792 15.2 -> 19.1 us); 6 are 3 to 7 % slower with it
+  //  * on 128 x 128 at 0.94 of the cost: at 0.95 to 0.975 of 32 x 64's 9 of 12 shapes were 2 to 7 % slower (258 x 6832 x 5120 39.8 -> 42.8)
+  auto cheapest = [&](bool eight, bool split) {
+    int form = -1;
+    float best = 0.f;
+    for (int f = tiles_only ? waves : 0; f < forms; f++) {
+      float c = form_cost(cost[f], M, N, K, (K + 63) / 64);
+      if (eight) {
+        c -= w4a16_halves_gain(f, M, N, K);
+        if (f == 3 && ((M + 63) / 64) * ((N + 63) / 64) <= WK_EIGHT_TILES) c -= 0.0322f * (float)((K + 63) / 64);
+        if (split && f >= waves && N % 8 != 0) c += 2e-6f * (float)(M > 32 ? M : 32) * (float)N;
+        if (split && f == waves) c *= 1.06f;
+      }
+      if (form < 0 || c < best) {
+        best = c;
+        form = f;
+      }
     }
-  }
-  return form;
+    return form;
+  };
+  return cheapest(true, cheapest(false, false) < waves);
 }
 static int launch_w4a16_auto(const W4A16PArgs& a, hipStream_t st) {
   static const int tiles[] = {-1, 6, 8, 4, 7, 5};  // of g_w4a16_ptile
@@ -793,6 +805,11 @@ MLLM_API int mllm_hip_w4a16_set_tuning(int tile) {
 
 MLLM_API int mllm_hip_w4a16_packed_form(int64_t M, int64_t N, int64_t K) {
   return M < 1 || N < 1 || K < 1 ? 0 : 1 + w4a16_packed_form(M, N, K, false);
+}
+MLLM_API int mllm_hip_w4a16_packed_eight(int64_t M, int64_t N, int64_t K) {
+  if (M < 1 || N < 1 || K < 1) return 0;
+  const int form = w4a16_packed_form(M, N, K, false);
+  return form == 3 ? wk_eight(M, N, (K + 63) / 64) : w4a16_halves_gain(form, M, N, K) > 0.f;
 }
 MLLM_API int mllm_hip_w4a16_packed_set_tuning(int tile) {
   if (tile < 0 || (tile & 15) > 5 || tile > 31) return MLLM_HIP_E_BADARG;

@@ -768,7 +768,7 @@ struct W8A8Waves {
     u32x4 q[4];
   };
   typedef uint32_t Col;
-  static __device__ __forceinline__ int kblocks(const Args& a) { return (a.K + 127) / 128; }
+  static __host__ __device__ __forceinline__ int kblocks(const Args& a) { return (a.K + 127) / 128; }
   static __device__ __forceinline__ int row_bytes(const Args& a) { return a.K; }
   static __device__ __forceinline__ const void* activations(const Args& a) { return a.A; }
   static __device__ __forceinline__ __amdgpu_buffer_rsrc_t weights(const Args& a) {

@@ -171,11 +171,14 @@ int wk_gemm_launch(const typename T::Args& a, hipStream_t st) {
 // Tiles of 64 x 64 by four waves, two blocks ahead, two workgroups per CU; where every tile has a CU to itself, by eight: one wave per SIMD
 // dequantizes and multiplies in turns, with a second one the two overlap.  Eight / four waves, median (range) over 730 shapes of Q4_0, Q8_0, Q4_K,
 // Q6_K and W4A16: 129 to 256 tiles 0.96 (0.91 to 1.02) up to K 1500, 0.93 (0.86 to 0.98) up to 4000, 0.87 (0.82 to 0.99) beyond; 257 to 384 tiles
-// 1.02 to 1.25, more 0.99 to 1.44.
-constexpr int64_t WK_EIGHT_TILES = 256;
+// 1.02 to 1.25, more 0.99 to 1.44.  Up to six blocks most waves have one block or none (W4A16: four 1.06, six 1.02, eight 0.99).
+constexpr int64_t WK_EIGHT_TILES = 256, WK_EIGHT_BLOCKS = 7;
+inline bool wk_eight(int64_t M, int64_t N, int64_t blocks) {
+  return ((M + 63) / 64) * ((N + 63) / 64) <= WK_EIGHT_TILES && blocks >= WK_EIGHT_BLOCKS;
+}
 template <class T>
 int wk_gemm_64x64(const typename T::Args& a, hipStream_t st) {
-  if ((int64_t)((a.M + 63) / 64) * ((a.N + 63) / 64) <= WK_EIGHT_TILES) return wk_gemm_launch<T, 2, 2, 8, 1>(a, st);
+  if (wk_eight(a.M, a.N, T::kblocks(a))) return wk_gemm_launch<T, 2, 2, 8, 1>(a, st);
   return wk_gemm_launch<T, 2, 2, 4, 2>(a, st);
 }
 

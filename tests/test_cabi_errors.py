@@ -95,6 +95,7 @@ def _cases():
         "mllm_hip_w8a8_packed_form": ([64, 64, 64], [(0, 0, 0), (1, -1, 0), (2, 0, 0)]),
         "mllm_hip_w8a8_packed_halves": ([64, 64, 64], [(0, 0, 0), (1, -1, 0), (2, 0, 0)]),
         "mllm_hip_w4a16_packed_form": ([64, 64, 64], [(0, 0, 0), (1, -1, 0), (2, 0, 0)]),
+        "mllm_hip_w4a16_packed_eight": ([64, 64, 64], [(0, 0, 0), (1, -1, 0), (2, 0, 0)]),
         "mllm_hip_q_gemm_form": ([Q4_0, 64, 64, 256, 1], [(0, 5, 0), (1, 0, 0), (2, 0, 0), (3, -1, 0)]),
         "mllm_hip_moe_gate_set_form": ([1], [(0, 2, BADARG), (0, -1, BADARG)]),
         "mllm_hip_kq_gemm_prepack": ([Q4_K, P, 0, P, 8, 256, None], [(0, Q8_0, BADARG), (1, None, BADARG), (5, 96, SHAPE)]),
@@ -234,6 +235,21 @@ def test_w4a16_takes_a_form_that_measures_fast(M, N, K, form):
     L = _lib.lib()
     assert L.mllm_hip_w4a16_packed_form(M, N, K) == form
     assert len({L.mllm_hip_w4a16_packed_form(t, N, K) for t in (1, 5, 9, 32)}) == 1
+
+
+@pytest.mark.parametrize("M,N,K,form", [(778, 1915, 1792, 3), (296, 4756, 1664, 3), (177, 7068, 1280, 4), (458, 4129, 4480, 3), (258, 6832, 5120, 3), (526, 3808, 8448, 3)])
+def test_w4a16_keeps_the_form_that_halves_of_larger_tiles_do_not_beat(M, N, K, form):
+    """shapes at which halves of K of larger tiles took 12 to 25 % longer (rows that are no multiple of 16 bytes) and 6 to 8 % (the last two)"""
+    assert _lib.lib().mllm_hip_w4a16_packed_form(M, N, K) == form
+
+
+def test_w4a16_runs_eight_waves_where_they_are_faster():
+    """from as many blocks of K on as pay for the meeting of the sums: 64 x 64 with six blocks took 1.02 of the time by eight, with four 1.06"""
+    L = _lib.lib()
+    take = lambda M, N, K: (L.mllm_hip_w4a16_packed_form(M, N, K), L.mllm_hip_w4a16_packed_eight(M, N, K))  # noqa: E731
+    for M, N, K, form in ((211, 2832, 448, 4), (1009, 624, 448, 4), (745, 4632, 448, 5), (1146, 6816, 512, 6), (138, 9376, 512, 8), (604, 2880, 512, 8)):
+        assert take(M, N, K - 64) == (form, 0) and take(M, N, K) == (form, 1)
+    assert take(8, 4096, 4096)[1] == 0 and take(2048, 9728, 2560) == (6, 0)
 
 
 def test_topk_is_cut_into_pieces_only_where_that_is_faster():

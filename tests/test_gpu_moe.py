@@ -165,10 +165,10 @@ def test_q_gemm_every_form_exact(wtype, M, N, K):
         assert L.mllm_hip_q_gemm_set_form(0) == 0
 
 
-@pytest.mark.parametrize("M,N,K,form", [(1024, 1024, 96, 3), (1025, 1024, 96, 3), (97, 8192, 800, 3), (97, 8193, 800, 3), (100, 8188, 1024, 12),
+@pytest.mark.parametrize("M,N,K,form", [(1024, 1024, 416, 3), (1024, 1024, 352, 3), (1025, 1024, 416, 3), (97, 8192, 800, 3), (97, 8193, 800, 3), (100, 8188, 1024, 12),
                                         (100, 8448, 1024, 12), (129, 4100, 1184, 8), (129, 8448, 1184, 8)])
 def test_linear_q_gemm_by_eight_and_four_waves(M, N, K, form):
-    """either side of 256 tiles of 64 x 64 (fewer K blocks than waves and blocks that do not divide among them) and of 256 workgroups of ranges
+    """either side of 256 tiles of 64 x 64 and of seven K blocks (fewer blocks than waves and blocks that do not divide among them) and of 256 workgroups of ranges
     of K (ranges of two and of four K steps, the last one shorter); integers whose sums are exact in any order (scales of one, no partial sum leaves 2^24)"""
     L = _lib.lib()
     rng = synth.rng_for(4, 1700 + M + N + K)
