@@ -373,7 +373,9 @@ __device__ __forceinline__ void silu_mul8(float (&v)[8], const float* u, bool ac
 // of registers for a whole next trip, copied over, took 220 registers for Q6_K with two units of two rows, 152 now; 2 x 9728 x 2560 at two rows, with the
 // offsets below and 24-bit products of sums and scales: Q4_K 11.2 -> 10.5 us, Q6_K 14.9 -> 13.9.)
 // ONE: the row's units fit one trip (units <= G U): nothing to refill.
-template <int WT, int XT, int MT, int G, int R, int U, int LB = 256, bool ONE = false>
+// AHEAD: a second set for the whole next trip, requested before this one is multiplied: its requests leave together, where the ring's leave one by one behind
+// the products (two trips of four units each, one row per group: the second trip comes 0.6 to 1.4 us later).
+template <int WT, int XT, int MT, int G, int R, int U, int LB = 256, bool ONE = false, bool AHEAD = false>
 __global__ __launch_bounds__(LB) void kq_gemv_kernel(KGemvArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int nsb = a.nsb;
@@ -522,6 +524,14 @@ __global__ __launch_bounds__(LB) void kq_gemv_kernel(KGemvArgs a) {
 
   for (int u0 = 0; u0 < units; u0 += G * U) {
     const bool more = !ONE && u0 + G * U < units;  // uniform
+    KUnit<WT> nxt[AHEAD ? U : 1][R];
+    if (AHEAD && more) {
+#pragma unroll
+      for (int uu = 0; uu < U; uu++)
+#pragma unroll
+        for (int r = 0; r < R; r++)
+          load_unit<WT>(nxt[AHEAD ? uu : 0][r], rs, off[r], u0 + G * U + uu * G, row_ok[r] && u0 + G * U + uu * G + c0 < units);
+    }
 #pragma unroll
     for (int uu = 0; uu < U; uu++) {
     const KUnit<WT>(&cu)[R] = cur[uu];
@@ -601,12 +611,18 @@ __global__ __launch_bounds__(LB) void kq_gemv_kernel(KGemvArgs a) {
         }
       }
     }
-    if (more) {  // the next trip's unit into the registers of this one
+    if (!AHEAD && more) {  // the next trip's unit into the registers of this one
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int r = 0; r < R; r++) load_unit<WT>(cur[uu][r], rs, off[r], u0 + G * U + uu * G, row_ok[r] && u0 + G * U + uu * G + c0 < units);
       __builtin_amdgcn_sched_barrier(0);
     }
+    }
+    if (AHEAD && more) {
+#pragma unroll
+      for (int uu = 0; uu < U; uu++)
+#pragma unroll
+        for (int r = 0; r < R; r++) cur[uu][r] = nxt[AHEAD ? uu : 0][r];
     }
   }
 
@@ -624,7 +640,7 @@ static int g_kq_G = 0, g_kq_NW = 0, g_kq_U = 0;  // tuning overrides (0 = heuris
 
 // R1: one weight row per lane group and up to 16 waves per workgroup (few rows of many units: o_proj, down_proj).  The
 // quantization of x is the long part of such a workgroup, so it is shared by as many rows as still fill the CUs.
-template <int WT, int XT, int MT, int G, int U, bool R1 = false, bool ONE = false>
+template <int WT, int XT, int MT, int G, int U, bool R1 = false, bool ONE = false, bool AHEAD = false>
 static int launch_kq_u(const KGemvArgs& a_in, int NW, hipStream_t st) {
   constexpr int R = R1 ? 1 : (WT == MLLM_HIP_Q4_K && MT >= 4) ? 4 : 2;  // wider row tiles reuse every LDS read for more weight rows
   constexpr int LB = R1 ? 1024 : 256;
@@ -641,7 +657,7 @@ static int launch_kq_u(const KGemvArgs& a_in, int NW, hipStream_t st) {
   }
   a.wg_start[a.nparts] = (int)grid;
   if (ONE && a_in.nsb * (WT == MLLM_HIP_Q4_K ? 8 : 4) > G * U) return MLLM_HIP_E_BADARG;
-  auto kern = kq_gemv_kernel<WT, XT, MT, G, R, U, LB, ONE>;
+  auto kern = kq_gemv_kernel<WT, XT, MT, G, R, U, LB, ONE, AHEAD>;
   if (lds > 64 * 1024)
     HIP_RET(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   const unsigned slots = (MT == 1 && a.slot_ids) ? (unsigned)a.slot_div_slots : 1u;
@@ -673,6 +689,13 @@ static int launch_kq_g(const KGemvArgs& a, int NW, int U, bool r1, hipStream_t s
       if (units <= 2 * G) return launch_kq_u<WT, XT, MT, G, 2, false, true>(a, NW, st);
       if (WT == MLLM_HIP_Q4_K) return launch_kq_u<WT, XT, MT, G, WT == MLLM_HIP_Q4_K ? 4 : 2>(a, NW, st);
     }
+  }
+  // Q4_K in the large workgroups, beyond one trip: a second set of registers, but for rows that want one unit more of a lane at most, whose request leaves first
+  // either way.  Without the offsets, 24-bit products and ring / ring / second set, us, one row: 1552 x 7936 6.9 / 8.1 / 6.8, 880 x 14 592 8.5 / 9.7 / 8.4; over 1500
+  // shapes by how far the last trip is filled, of the first: up to a quarter 0.94 / 0.98, a half 0.99 / 0.98, three quarters 1.04 / 0.98, more 1.06 / 0.98
+  if constexpr (WT == MLLM_HIP_Q4_K && MT <= 2 && G >= 32) {
+    const int units = a.nsb * 8;
+    if (r1 && !g_kq_U && (units <= 4 * G || units > 5 * G)) return launch_kq_u<WT, XT, MT, G, 4, true, false, true>(a, NW, st);
   }
   if (r1 && MT <= 2 && G >= 32) return launch_kq_u<WT, XT, MT, G, (MT <= 2 && G >= 32 && WT == MLLM_HIP_Q4_K) ? 4 : 1, (MT <= 2 && G >= 32)>(a, NW, st);
   if (WT == MLLM_HIP_Q4_K && U >= 4 && MT <= 2) return launch_kq_u<WT, XT, MT, G, (WT == MLLM_HIP_Q4_K && MT <= 2) ? 4 : 1>(a, NW, st);

@@ -397,6 +397,58 @@ def test_units_in_flight_do_not_change_the_bits(wtype):
                 assert L.mllm_hip_kq_set_tuning(0, 0, 0) == 0
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 300, 5120), (1, 300, 5376), (2, 70, 7936), (2, 70, 8192), (1, 33, 10240), (1, 33, 10496), (2, 130, 14592), (1, 130, 18944)])
+def test_whole_trips_ahead_do_not_change_the_bits(M, N, K):
+    """long Q4_K rows in the large workgroups: a second set of registers for the next trip, either side of the lengths that keep the ring, against
+    the ring (the units in flight stated)"""
+    rng = synth.rng_for(7, 1700 + N + K)
+    L = _lib.lib()
+    w = ql.PackedKWeight(2, torch.from_numpy(synth.make_weight(rng, 2, N, K)))
+    x = to_dev(synth.make_x_fp32(rng, M, K))
+    announce("kq trips ahead", M, N, K)
+    want = ql.linear_kq(w, x)
+    assert torch.isfinite(want).all() and want.abs().max() > 0
+    try:
+        assert L.mllm_hip_kq_set_tuning(0, 0, 4) == 0
+        assert torch.equal(want, ql.linear_kq(w, x))
+    finally:
+        assert L.mllm_hip_kq_set_tuning(0, 0, 0) == 0
+
+
+def _graph_time(call, n=24):
+    """median of nine replays of call(0) .. call(n - 1), in us per call"""
+    call(0)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for i in range(n):
+            call(i)
+    times = []
+    for _ in range(11):
+        first, last = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        first.record()
+        graph.replay()
+        last.record()
+        torch.cuda.synchronize()
+        times.append(first.elapsed_time(last) * 1e3 / n)
+    return sorted(times[2:])[4]
+
+
+def test_long_q4_k_rows_are_requested_a_trip_ahead():
+    """1552 x 7936, one row, weights that no cache of an XCD holds: 6.8 us, by the ring 8.1.  A bound with room for other noise"""
+    L = _lib.lib()
+    g = torch.Generator(device="cuda").manual_seed(1)
+    ws = [ql.PackedKWeight.synthetic(2, 1552, 7936, g) for _ in range(8)]
+    x, y = torch.randn((1, 7936), device="cuda", generator=g), torch.empty((1, 1552), device="cuda")
+    announce("kq trips ahead, time")
+    ahead = _graph_time(lambda i: ql.linear_kq(ws[i % 8], x, out=y))
+    try:
+        assert L.mllm_hip_kq_set_tuning(0, 0, 4) == 0
+        assert ahead <= 0.93 * _graph_time(lambda i: ql.linear_kq(ws[i % 8], x, out=y))
+    finally:
+        assert L.mllm_hip_kq_set_tuning(0, 0, 0) == 0
+
+
 @pytest.mark.parametrize("wtype,H", [(2, 512), (2, 768), (2, 1024), (2, 1280), (2, 2048), (2, 2304), (3, 1024), (3, 1280), (3, 2048), (3, 2304)])
 def test_units_in_flight_of_expert_pairs_do_not_change_the_bits(wtype, H):
     """a token's experts, a GEMV row per pair: rows whose units fit one or two per lane, the ring of several and its last, partly filled trip
