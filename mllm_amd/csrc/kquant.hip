@@ -679,15 +679,20 @@ static int launch_kq_g(const KGemvArgs& a, int NW, int U, bool r1, hipStream_t s
         if (!r1 && units > 2 * G && units <= 3 * G) return launch_kq_u<WT, XT, MT, G, 3, false, true>(a, NW, st);
     }
   }
-  // MoE slots: the row's units at once where two per lane hold them (Q4_K rows of up to 1024 elements, Q6_K of up to 2048), Q4_K four at a time beyond that.
-  // us of a layer of 128 experts of 2048 x 768, top-8, two at a time with a second set of registers for the next trip / this: Q4_K / Q6_K one token
-  // 15.1 / 14.3, four 26.4 / 25.4, eight 40.8 / 39.8 (three at a time 44.4), Q6_K eight 53.5 / 47.2
+  // MoE slots: the row's units at once where two per lane hold them (Q4_K rows of up to 1024 elements, Q6_K of up to 2048), Q4_K four at a time up to 2048.  us of a
+  // layer of 128 experts of 2048 x 768, top-8, two at a time with a second set of registers for the next trip / this: Q4_K / Q6_K one token 15.1 / 14.3, four
+  // 26.4 / 25.4, eight 40.8 / 39.8 (three at a time 44.4), Q6_K eight 53.5 / 47.2.  Longer rows of Q4_K keep the second set: over 900 layers of 2304 to 7168 elements,
+  // of the time before there was a ring, mean (most): four at a time by the ring 1.00 (1.09), the second set 0.97 (1.04); one token of 2560 x 3072, eight
+  // experts 31.2 / 34.0 / 30.9 us
   if constexpr (MT == 1 && G == 16) {
     const int units = a.nsb * (WT == MLLM_HIP_Q4_K ? 8 : 4);
     if (a.slot_ids && U == 2 && !g_kq_U) {
       if (units <= G) return launch_kq_u<WT, XT, MT, G, 1, false, true>(a, NW, st);
       if (units <= 2 * G) return launch_kq_u<WT, XT, MT, G, 2, false, true>(a, NW, st);
-      if (WT == MLLM_HIP_Q4_K) return launch_kq_u<WT, XT, MT, G, WT == MLLM_HIP_Q4_K ? 4 : 2>(a, NW, st);
+      if constexpr (WT == MLLM_HIP_Q4_K) {
+        if (units <= 4 * G) return launch_kq_u<WT, XT, MT, G, 4>(a, NW, st);
+        return launch_kq_u<WT, XT, MT, G, 2, false, false, true>(a, NW, st);
+      }
     }
   }
   // Q4_K in the large workgroups, beyond one trip: a second set of registers, but for rows that want one unit more of a lane at most, whose request leaves first

@@ -449,11 +449,12 @@ def test_long_q4_k_rows_are_requested_a_trip_ahead():
         assert L.mllm_hip_kq_set_tuning(0, 0, 0) == 0
 
 
-@pytest.mark.parametrize("wtype,H", [(2, 512), (2, 768), (2, 1024), (2, 1280), (2, 2048), (2, 2304), (3, 1024), (3, 1280), (3, 2048), (3, 2304)])
+@pytest.mark.parametrize("wtype,H", [(2, 512), (2, 768), (2, 1024), (2, 1280), (2, 2048), (2, 2304), (2, 2560), (2, 3072), (3, 1024), (3, 1280), (3, 2048), (3, 2304), (3, 4096)])
 def test_units_in_flight_of_expert_pairs_do_not_change_the_bits(wtype, H):
-    """a token's experts, a GEMV row per pair: rows whose units fit one or two per lane, the ring of several and its last, partly filled trip
-    against one unit at a time (mllm_hip_kq_set_tuning)"""
-    I, E, k = 256 + 256 * (H % 512 > 0), 5, 3
+    """a token's experts, a GEMV row per pair with sixteen lanes: rows whose units fit one or two per lane, Q4_K four at a time and beyond that a whole trip ahead,
+    Q6_K the ring of two, the last trip partly filled among them, against one unit at a time (mllm_hip_kq_set_tuning).  Eight pairs of 768 rows: more workgroups
+    than the form for few rows takes"""
+    I, E, k = 768, 8, 8
     rng = synth.rng_for(9, 7900 + wtype + H)
     L = _lib.lib()
     Wg, Wu = (synth.make_weight(rng, wtype, E * I, H).reshape(E, I, H // 256, -1) for _ in range(2))
@@ -462,11 +463,30 @@ def test_units_in_flight_of_expert_pairs_do_not_change_the_bits(wtype, H):
     ids, w = synth.make_moe_routing(rng, 1, E, k)
     ids, w, x = to_dev(ids), to_dev(w), to_dev(synth.make_x_fp32(rng, 1, H))
     announce("moe k-quant pairs, units in flight", wtype, H, I)
-    want = ql.moe_ffn_kq(g, u, d, x, ids, w)
-    assert torch.isfinite(want).all() and want.abs().max() > 0
     try:
+        assert L.mllm_hip_moe_kq_set_path(1) == 0  # (eight pairs of eight experts of Q6_K are tiles otherwise)
+        want = ql.moe_ffn_kq(g, u, d, x, ids, w)
+        assert torch.isfinite(want).all() and want.abs().max() > 0
         assert L.mllm_hip_kq_set_tuning(0, 0, 1) == 0
         assert torch.equal(want, ql.moe_ffn_kq(g, u, d, x, ids, w))
+    finally:
+        assert L.mllm_hip_kq_set_tuning(0, 0, 0) == 0 and L.mllm_hip_moe_kq_set_path(0) == 0
+
+
+def test_expert_pairs_of_long_q4_k_rows_are_requested_a_trip_ahead():
+    """eight experts of 2560 x 3072, one token of all eight: 30.9 us, four units at a time by the ring 34.0.  A bound with room for other noise"""
+    L = _lib.lib()
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    g, u, d = (ql.PackedKExperts.synthetic(2, 8, n, k, gen) for n, k in ((3072, 2560), (3072, 2560), (2560, 3072)))
+    ids, w = synth.make_moe_routing(synth.rng_for(9, 1), 1, 8, 8)
+    ids, w, x = to_dev(ids), to_dev(w), torch.randn((1, 2560), device="cuda", generator=gen)
+    y, ws = torch.empty_like(x), torch.empty(L.mllm_hip_moe_kq_workspace_bytes(1, 2560, 3072, 8, 8), dtype=torch.uint8, device="cuda")
+    call = lambda i: ql.moe_ffn_kq(g, u, d, x, ids, w, workspace=ws, out=y)  # noqa: E731
+    announce("moe k-quant pairs, time")
+    ahead = _graph_time(call)
+    try:
+        assert L.mllm_hip_kq_set_tuning(0, 0, 4) == 0
+        assert ahead <= 0.96 * _graph_time(call)
     finally:
         assert L.mllm_hip_kq_set_tuning(0, 0, 0) == 0
 
