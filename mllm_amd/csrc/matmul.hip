@@ -849,7 +849,9 @@ static bool mm_narrow(const MMArgs& a) {
 // fp32: the side of the tile of matmul_split_kernel, 0 where fp32 instructions are as fast or needed.  Costs in us of the three forms fitted to 4800
 // random shapes in all orders (1 to 64 x 5 to 4096 x 5 to 4096 x 16 to 2048, a third of them attention of 64 to 1024 tokens), those of the large tile
 // again to 900 of more than one small tile per CU: the choice takes 0.864 of the fp32 instructions' time on average over those, the best of the three 0.859 (0.879
-// before the large tile's splitting moved); one is more than 5 % slower.  A gain of less than 4 % in the costs stays with
+// before the large tile's splitting moved).  Large tiles whose edges cover more than 1.2 of what small ones do cost 6 % more than that (42 x 157 x 721 x 1301 130 us on
+// small ones, 151), and the fp32 instructions no less than for 48 from 33 on (17 x 382 x 515 x 35 10.9 us, 8.4 from parts): over 2372 shapes near the limits 0.970 of the time of the
+// choice before those two costs and that move, 45 more than 3 % slower, up to 10 % (60, up to 18 %, without).  A gain of less than 4 % in the costs stays with
 // fp32 instructions, and so do K below 32 (59 x 397 x 1677 x 24: 45.4 us, 57 with parts) and up to one small tile per CU, where the order decides
 // and tiles do not (1 x 1701 x 245 x 1964 with A [K][M] 74 / 56, 8 x 20 x 168 x 1765 42 / 50).  With costs of the parts alone every launch
 // above a floor took them, and the large tile too early: 8 x 504 x 504 x 128 9.4 / 12.2 us, 8 x 1308 x 327 x 64 11.2 / 16.1.  Few rows x
@@ -862,9 +864,11 @@ static int mm_split_side(const MMArgs& a, bool nt) {
   if (nt && mm_narrow<MLLM_HIP_F32, false, true>(a)) return 0;
   const double K = a.K, t64 = (double)((a.M + 63) / 64) * ((a.N + 63) / 64) * a.batch / 256, t128 = (double)((a.M + 127) / 128) * ((a.N + 127) / 128) * a.batch / 256;
   if (t64 <= 1. || a.K < 32) return 0;
+  const double steps = a.K > 32 ? std::max(K, 48.) : K;  // the fp32 instructions' tiles take K in steps of 32: 33 elements cost as many as 48
+  const double pad = (double)((a.M + 127) / 128 * 2) * ((a.N + 127) / 128 * 2) / ((double)((a.M + 63) / 64) * ((a.N + 63) / 64));  // large tiles' area over small ones'
   const double us64 = 3.6 + 0.80 * t64 + K * (0.0225 + 0.0152 * (0.49 * std::ceil(t64) + 0.51 * t64 - 1.));
-  const double us128 = 2.14 + 6.02 * std::max(t128, 1.) + K * (0.0384 + 0.0503 * (std::ceil(t128) - 1.));
-  const double f32 = 3.06 + 0.869 * t64 + K * (0.024 + 0.020 * (0.93 * std::ceil(t64) + 0.07 * t64 - 1.));
+  const double us128 = (2.14 + 6.02 * std::max(t128, 1.) + K * (0.0384 + 0.0503 * (std::ceil(t128) - 1.))) * (pad > 1.2 ? 1.06 : 1.);
+  const double f32 = 3.06 + 0.869 * t64 + steps * (0.024 + 0.020 * (0.93 * std::ceil(t64) + 0.07 * t64 - 1.));
   if (std::min(us64, us128) > 0.96 * f32) return 0;
   return us128 < us64 ? 128 : 64;
 }

@@ -252,6 +252,13 @@ def test_w4a16_runs_eight_waves_where_they_are_faster():
     assert take(8, 4096, 4096)[1] == 0 and take(2048, 9728, 2560) == (6, 0)
 
 
+@pytest.mark.parametrize("shape,side", [((42, 157, 721, 1301, 0, 0), 64), ((9, 3206, 145, 1475, 0, 0), 64), ((19, 161, 1610, 1070, 1, 0), 64), ((50, 162, 589, 813, 1, 0), 64),
+                                        ((18, 1578, 99, 33, 0, 1), 64), ((17, 382, 515, 35, 0, 1), 64), ((8, 3108, 128, 777, 0, 0), 128), ((8, 504, 504, 128, 0, 0), 0)])
+def test_matmul_takes_a_form_that_measures_fast(shape, side):
+    """edges of large tiles (8 to 15 % slower than small ones at the first four) and K that fills a step of the fp32 instructions by a thirty-second (18 and 20 %)"""
+    assert _lib.lib().mllm_hip_matmul_split_side(*shape) == side
+
+
 def test_topk_is_cut_into_pieces_only_where_that_is_faster():
     """rows without whole vectors of up to 8192 elements stay one workgroup's work while that is one round of workgroups"""
     room = _lib.lib().mllm_hip_topk_workspace_bytes
