@@ -236,9 +236,12 @@ int mllm_hip_linear_q_gemm_short(int wtype, const void* gemm_packed, const void*
  * 1 / 2 / 3: waves that split K of a tile of 32 x 32 / 32 x 64 / 64 x 64; 4: tiles of 128 x 256, halves of K in one workgroup; 5: such
  * tiles whole, in half-height ones where a last round is short; 6 .. 12: K in two .. eight ranges (the calls with the larger workspace,
  * asked for its size under the same setting; where K has no such ranges, or N % 4, as 5).  mllm_hip_q_gemm_form: the form that a
- * Linear of this size takes, 1 .. 12 (host only).  No counterpart in the reference. */
+ * Linear of this size takes, 1 .. 12; mllm_hip_q_gemm_eight: 1 where its workgroups are eight waves (1, 2 and 4 always; 3 up to 256 tiles and from 385 elements of K
+ * on; 6 .. 12 up to 256 workgroups, of Q8_0 / Q6_K on more than 200 of them only in ranges of sixteen blocks of 64 and more), 0 where they are four (both host
+ * only).  No counterpart in the reference. */
 int mllm_hip_q_gemm_set_form(int form);
 int mllm_hip_q_gemm_form(int wtype, int64_t M, int64_t N, int64_t K, int short_call);
+int mllm_hip_q_gemm_eight(int wtype, int64_t M, int64_t N, int64_t K, int short_call);
 /* Same arguments as mllm_hip_moe_ffn_q; the three expert arrays are E gemm-packed matrices back to back
  * (stride mllm_hip_q_gemm_packed_bytes). */
 size_t mllm_hip_moe_gemm_workspace_bytes(int64_t T, int64_t H, int64_t I, int E, int k);

@@ -104,6 +104,7 @@ def lib():
         L.mllm_hip_linear_kq_gemm_short.argtypes = [ci, vp, vp, ci, vp, vp, i64, i64, i64, vp, vp]
         L.mllm_hip_q_gemm_set_form.argtypes = [ci]
         L.mllm_hip_q_gemm_form.argtypes = [ci, i64, i64, i64, ci]
+        L.mllm_hip_q_gemm_eight.argtypes = [ci, i64, i64, i64, ci]
         L.mllm_hip_kq_packed_bytes.restype = C.c_size_t
         L.mllm_hip_kq_packed_bytes.argtypes = [ci, i64, i64]
         L.mllm_hip_kq_prepack.argtypes = [ci, vp, ci, vp, i64, i64, vp]

@@ -1933,10 +1933,14 @@ static QLinearPlan q_linear_plan(int wtype, int64_t M, int64_t N, int64_t K, boo
   }
   return best;
 }
-// Ranges whose workgroups have a CU each run by eight waves, halves of a range each: one wave per SIMD dequantizes and multiplies in turns.  0.973 of the time
-// over 70 shapes that take ranges (0.94 to 1.01, one 1.04); more than 256 workgroups share CUs already.
-static bool q_ranges_in_halves(int64_t M, int64_t N, int ranges) {
-  return ranges > 1 && ((M + QG_TILE_H - 1) / QG_TILE_H) * ((N + 255) / 256) * ranges <= 256;
+// Ranges whose workgroups have a CU each run by eight waves, halves of a range each: one wave per SIMD dequantizes and multiplies in turns.  0.946 of the time
+// over 623 shapes that take ranges; more than 256 workgroups share CUs already.  Codes of a byte (less to unpack) on more than 200 CUs in ranges of fewer
+// than sixteen blocks, whose halves are as unequal as eight and six: 0.990, up to 1.04 (984 x 816 x 7040 Q8_0 38.1 -> 39.6 us), so they stay with four.
+static bool q_ranges_in_halves(int wtype, int64_t M, int64_t N, int64_t K, int ranges) {
+  const int64_t groups = ((M + QG_TILE_H - 1) / QG_TILE_H) * ((N + 255) / 256) * ranges;
+  if (ranges < 2 || groups > 256) return false;
+  const int64_t blocks = (K + 63) / 64, per = ((blocks + ranges - 1) / ranges + 1) / 2 * 2;
+  return qg_nibbles(wtype) || groups <= 200 || per >= 16;
 }
 size_t qg_partial_bytes(int wtype, int64_t M, int64_t N, int64_t K) {  // the same for both types of a call (their plans may differ)
   const bool kq = wtype == MLLM_HIP_Q4_K || wtype == MLLM_HIP_Q6_K;
@@ -1964,7 +1968,7 @@ int qg_linear_run(int wtype, const void* gemm_packed, const uint16_t* xh, const 
   a.o_index = nullptr; a.out = y; a.bias = bias;
   a.N = (int)N; a.K = (int)K; a.wtype = wtype; a.x86_scale = 0;
   a.ksplit = plan.ranges;
-  a.halves = plan.halves || q_ranges_in_halves(M, N, plan.ranges);
+  a.halves = plan.halves || q_ranges_in_halves(wtype, M, N, K, plan.ranges);
   a.partial = reinterpret_cast<float*>(partial_ws);
   const int64_t tilesM = (M + QG_TILE_H - 1) / QG_TILE_H, cols = (N + 255) / 256, total = tilesM * cols;
   a.big_cols = (int)cols;
@@ -2212,6 +2216,11 @@ MLLM_API int mllm_hip_q_gemm_form(int wtype, int64_t M, int64_t N, int64_t K, in
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const QLinearPlan p = q_linear_plan(wtype, M, N, K, short_call && qg_partial_bytes(wtype, M, N, K));
   return p.waves >= 0 ? 1 + p.waves : p.halves ? 4 : 4 + p.ranges;
+}
+MLLM_API int mllm_hip_q_gemm_eight(int wtype, int64_t M, int64_t N, int64_t K, int short_call) {
+  if (mllm_hip_q_gemm_form(wtype, M, N, K, short_call) == 0) return 0;
+  const QLinearPlan p = q_linear_plan(wtype, M, N, K, short_call && qg_partial_bytes(wtype, M, N, K));
+  return p.waves >= 0 ? p.waves < 2 || wk_eight(M, N, (K + 63) / 64) : p.halves || q_ranges_in_halves(wtype, M, N, K, p.ranges);
 }
 
 MLLM_API size_t mllm_hip_linear_q_gemm_workspace_bytes(int64_t M, int64_t K) {

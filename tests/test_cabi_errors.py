@@ -97,6 +97,7 @@ def _cases():
         "mllm_hip_w4a16_packed_form": ([64, 64, 64], [(0, 0, 0), (1, -1, 0), (2, 0, 0)]),
         "mllm_hip_w4a16_packed_eight": ([64, 64, 64], [(0, 0, 0), (1, -1, 0), (2, 0, 0)]),
         "mllm_hip_q_gemm_form": ([Q4_0, 64, 64, 256, 1], [(0, 5, 0), (1, 0, 0), (2, 0, 0), (3, -1, 0)]),
+        "mllm_hip_q_gemm_eight": ([Q4_0, 64, 64, 256, 1], [(0, 5, 0), (1, 0, 0), (2, 0, 0), (3, -1, 0)]),
         "mllm_hip_moe_gate_set_form": ([1], [(0, 2, BADARG), (0, -1, BADARG)]),
         "mllm_hip_kq_gemm_prepack": ([Q4_K, P, 0, P, 8, 256, None], [(0, Q8_0, BADARG), (1, None, BADARG), (5, 96, SHAPE)]),
         "mllm_hip_linear_kq_gemm": ([Q4_K, P, P, F32, None, P, 16, 8, 256, P, None],
@@ -274,6 +275,15 @@ def test_q_gemm_takes_a_form_that_measures_fast(wtype, M, N, K, forms):
     """shapes at which a choice by rows, columns and K steps alone was 10 to 23 % slower than the forms here (measured, all twelve)"""
     assert _lib.lib().mllm_hip_q_gemm_form(wtype, M, N, K, 1) in forms
     assert _lib.lib().mllm_hip_q_gemm_form(wtype, M, N, K, 0) <= 5  # no room for partial results: no ranges
+
+
+@pytest.mark.parametrize("wtype,M,N,K,form,eight", [
+    (Q8_0, 984, 816, 7040, 12, 0), (Q6_K, 99, 8480, 5376, 11, 0), (Q8_0, 162, 3888, 17472, 12, 1), (Q6_K, 394, 2560, 9728, 10, 1), (Q4_K, 1466, 752, 6912, 11, 1),
+    (Q4_0, 180, 3120, 7680, 3, 1), (Q6_K, 138, 2288, 1536, 2, 1), (Q4_0, 2048, 9728, 2560, 5, 0)])
+def test_q_gemm_runs_eight_waves_where_they_are_faster(wtype, M, N, K, form, eight):
+    """the first two: byte codes in ranges of fourteen and twelve blocks on nearly every CU, 4 and 2 % slower by eight"""
+    L = _lib.lib()
+    assert (L.mllm_hip_q_gemm_form(wtype, M, N, K, 1), L.mllm_hip_q_gemm_eight(wtype, M, N, K, 1)) == (form, eight)
 
 
 @pytest.mark.parametrize("M,N,K", [(200, 2560, 9728), (200, 2558, 9728), (70, 260, 160), (200, 1024, 640), (512, 512, 65536)])
