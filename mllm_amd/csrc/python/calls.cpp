@@ -66,6 +66,16 @@ int xdtype(const at::Tensor& x) {
   raise(PyExc_TypeError, "activations must be float32 or bfloat16");
 }
 at::Tensor empty(at::IntArrayRef sizes, at::ScalarType type) { return at::empty(sizes, at::TensorOptions().dtype(type).device(at::kCUDA)); }
+// the caller's workspace, which has to hold what the call writes (the C ABI takes its size on trust), or a new one
+void* workspace(PyObject* o, size_t bytes, at::Tensor& made) {
+  if (o == Py_None) return (made = empty({(int64_t)bytes}, at::kByte)).data_ptr();
+  const at::Tensor& t = tensor(o);
+  if (t.nbytes() < bytes) {
+    PyErr_Format(g_error, "a workspace of %zu bytes, %zu needed", (size_t)t.nbytes(), bytes);
+    throw Raised();
+  }
+  return t.data_ptr();
+}
 void need_rank(const at::Tensor& t, int64_t dims) {
   if (t.dim() < dims) raise(PyExc_IndexError, "tuple index out of range");
 }
@@ -218,10 +228,10 @@ PyObject* w8a8_linear_packed(Args a) {
   const int64_t M = x.size(0), K = x.size(1), N = integer(a[2]);
   require(w.numel() == (int64_t)mllm_hip_w8a8_packed_bytes(N, K));
   at::Tensor work, made;
-  if (a[5] == Py_None) work = empty({(int64_t)mllm_hip_w8a8_workspace_bytes(M, K)}, at::kByte);
+  void* sp = workspace(a[5], mllm_hip_w8a8_workspace_bytes(M, K), work);
   if (a[6] == Py_None) made = empty({M, N}, at::kBFloat16);
   const int xt = xdtype(x);
-  void *xp = x.data_ptr(), *wp = w.data_ptr(), *yp = a[6] == Py_None ? made.data_ptr() : pointer(a[6]), *sp = a[5] == Py_None ? work.data_ptr() : pointer(a[5]);
+  void *xp = x.data_ptr(), *wp = w.data_ptr(), *yp = a[6] == Py_None ? made.data_ptr() : pointer(a[6]);
   const float *scale = static_cast<const float*>(tensor(a[3]).data_ptr()), *bias = static_cast<const float*>(pointer(a[4]));
   void* st = stream();
   run("mllm_hip_w8a8_linear_packed", [&] { return mllm_hip_w8a8_linear_packed(xp, xt, wp, scale, bias, yp, M, N, K, sp, st); });
@@ -245,7 +255,7 @@ PyObject* w4a16_gemm_packed(Args a) {
 
 // a Linear over many rows: w, x, bias, workspace, out, short of both kinds of block formats
 template <typename Bytes, typename ShortBytes, typename Call>
-PyObject* linear_gemm(const char* what, PyObject* w, PyObject* xo, PyObject* bias, PyObject* workspace, PyObject* out, Bytes bytes, ShortBytes short_bytes,
+PyObject* linear_gemm(const char* what, PyObject* w, PyObject* xo, PyObject* bias, PyObject* room, PyObject* out, Bytes bytes, ShortBytes short_bytes,
                       bool shorter, Call call) {
   const at::Tensor& x = tensor(xo);
   require(x.is_cuda() && x.is_contiguous() && x.dim() == 2 && x.size(1) == attribute(w, s_K));
@@ -254,12 +264,12 @@ PyObject* linear_gemm(const char* what, PyObject* w, PyObject* xo, PyObject* bia
   const int64_t M = x.size(0), K = x.size(1), N = attribute(w, s_N);
   const int wtype = (int)attribute(w, s_wtype), xt = xdtype(x);
   at::Tensor work, made;
-  if (workspace == Py_None) work = empty({(int64_t)(shorter ? short_bytes(M, N, K) : bytes(M, K))}, at::kByte);
+  void* sp = workspace(room, shorter ? short_bytes(M, N, K) : bytes(M, K), work);
   if (out == Py_None) made = empty({M, N}, at::kFloat);
   const void *wp = pointer(buf.o), *xp = x.data_ptr();
   const float* bp = static_cast<const float*>(pointer(bias));
   float* yp = static_cast<float*>(out == Py_None ? made.data_ptr() : pointer(out));
-  void *sp = workspace == Py_None ? work.data_ptr() : pointer(workspace), *st = stream();
+  void* st = stream();
   run(what, [&] { return call(wtype, wp, xp, xt, bp, yp, M, N, K, sp, st); });
   return out == Py_None ? THPVariable_Wrap(made) : given(out);
 }

@@ -37,6 +37,15 @@ def _stream():
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
+def _workspace(given, size):
+    """the caller's workspace, which has to hold what the call writes (the C ABI takes its size on trust), or a new one"""
+    if given is None:
+        return torch.empty(size, dtype=torch.uint8, device="cuda")
+    if given.numel() * given.element_size() < size:
+        raise _lib.HipQLinearError("a workspace of %d bytes, %d needed" % (given.numel() * given.element_size(), size))
+    return given
+
+
 def _xdtype(x):
     if x.dtype == torch.float32:
         return F32
@@ -203,8 +212,7 @@ def w8a8_linear(x, W, w_scale, bias=None, workspace=None, out=None):
     M, K = x.shape
     N = W.shape[0]
     L = _lib.lib()
-    if workspace is None:
-        workspace = torch.empty(L.mllm_hip_w8a8_workspace_bytes(M, K), dtype=torch.uint8, device="cuda")
+    workspace = _workspace(workspace, L.mllm_hip_w8a8_workspace_bytes(M, K))
     y = out if out is not None else torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
     _lib.check(L.mllm_hip_w8a8_linear(x.data_ptr(), _xdtype(x), W.data_ptr(), w_scale.data_ptr(), _p(bias),
                                       y.data_ptr(), M, N, K, workspace.data_ptr(), _stream()), "mllm_hip_w8a8_linear")
@@ -307,8 +315,7 @@ def linear_q(w, x, bias=None, act_scale_mode=SCALE_X86_REF, workspace=None, out=
     assert x.is_cuda and x.is_contiguous() and x.dim() == 2 and x.shape[1] == w.K
     M = x.shape[0]
     L = _lib.lib()
-    if workspace is None:
-        workspace = torch.empty(L.mllm_hip_linear_q_workspace_bytes(M, w.K), dtype=torch.uint8, device="cuda")
+    workspace = _workspace(workspace, L.mllm_hip_linear_q_workspace_bytes(M, w.K))
     y = out if out is not None else torch.empty((M, w.N), dtype=torch.float32, device="cuda")
     _lib.check(L.mllm_hip_linear_q(w.wtype, w.ptr, x.data_ptr(), _xdtype(x), _p(bias), y.data_ptr(), M, w.N, w.K,
                                    act_scale_mode, workspace.data_ptr(), _stream()), "mllm_hip_linear_q")
@@ -357,8 +364,7 @@ def moe_ffn_q(gate, up, down, x, topk_ids, topk_w, act_scale_mode=SCALE_X86_REF,
     E, I = gate.E, gate.N
     assert gate.K == H and up.N == I and down.N == H and down.K == I and topk_ids.dtype == torch.int32
     L = _lib.lib()
-    if workspace is None:
-        workspace = torch.empty(L.mllm_hip_moe_workspace_bytes(T, H, I, E, k), dtype=torch.uint8, device="cuda")
+    workspace = _workspace(workspace, L.mllm_hip_moe_workspace_bytes(T, H, I, E, k))
     y = out if out is not None else torch.empty((T, H), dtype=torch.float32, device="cuda")
     _lib.check(L.mllm_hip_moe_ffn_q(gate.wtype, gate.ptr, up.ptr, down.ptr, x.data_ptr(), _xdtype(x), topk_ids.data_ptr(),
                                     topk_w.data_ptr(), y.data_ptr(), T, H, I, E, k, act_scale_mode, workspace.data_ptr(),
@@ -380,8 +386,7 @@ def moe_ffn_q_gemm(gate, up, down, x, topk_ids, topk_w, act_scale_mode=SCALE_X86
     assert gate.K == H and up.N == I and down.N == H and down.K == I and topk_ids.dtype == torch.int32
     assert gate.layout == up.layout == down.layout == "gemm"
     L = _lib.lib()
-    if workspace is None:
-        workspace = torch.empty(L.mllm_hip_moe_gemm_workspace_bytes(T, H, I, E, k), dtype=torch.uint8, device="cuda")
+    workspace = _workspace(workspace, L.mllm_hip_moe_gemm_workspace_bytes(T, H, I, E, k))
     y = out if out is not None else torch.empty((T, H), dtype=torch.float32, device="cuda")
     _lib.check(L.mllm_hip_moe_ffn_q_gemm(gate.wtype, gate.ptr, up.ptr, down.ptr, x.data_ptr(), _xdtype(x),
                                          topk_ids.data_ptr(), topk_w.data_ptr(), y.data_ptr(), T, H, I, E, k, act_scale_mode,
@@ -583,8 +588,7 @@ def moe_ffn_kq(gate, up, down, x, topk_ids, topk_w, workspace=None, out=None):
     assert gate.K == H and up.N == I and down.N == H and down.K == I and topk_ids.dtype == torch.int32
     assert gate.wtype == up.wtype
     L = _lib.lib()
-    if workspace is None:
-        workspace = torch.empty(L.mllm_hip_moe_kq_workspace_bytes(T, H, I, E, k), dtype=torch.uint8, device="cuda")
+    workspace = _workspace(workspace, L.mllm_hip_moe_kq_workspace_bytes(T, H, I, E, k))
     y = out if out is not None else torch.empty((T, H), dtype=torch.float32, device="cuda")
     if down.wtype == gate.wtype:
         _lib.check(L.mllm_hip_moe_ffn_kq(gate.wtype, gate.ptr, up.ptr, down.ptr, x.data_ptr(), _xdtype(x), topk_ids.data_ptr(),
@@ -612,7 +616,7 @@ def linear_kq(w, x, bias=None, out=None, workspace=None):
     assert w.layout == "gemv" and x.is_cuda and x.is_contiguous() and x.dim() == 2 and x.shape[1] == w.K
     M = x.shape[0]
     y = out if out is not None else torch.empty((M, w.N), dtype=torch.float32, device="cuda")
-    if workspace is not None and workspace.numel() > _lib.lib().mllm_hip_kq_workspace_bytes(M, w.K):
+    if workspace is not None and _workspace(workspace, _lib.lib().mllm_hip_kq_workspace_bytes(M, w.K)).numel() > _lib.lib().mllm_hip_kq_workspace_bytes(M, w.K):
         return linear_kq_multi([w], x, [bias], [y], workspace=workspace)[0]  # (the entry point that is told the workspace's size)
     _lib.check(_lib.lib().mllm_hip_linear_kq(w.wtype, w.ptr, x.data_ptr(), _xdtype(x), _p(bias), y.data_ptr(), M, w.N, w.K,
                                              _p(workspace), _stream()), "mllm_hip_linear_kq")

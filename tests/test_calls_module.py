@@ -1,5 +1,7 @@
 """The short calls of qlinear.py in native code (csrc/python/calls.cpp): what they refuse, before any device call, and that they use the
 caller's outputs, workspaces and stream."""
+import types
+
 import numpy as np
 import pytest
 import torch
@@ -38,6 +40,58 @@ X = torch.zeros(3, 64)
 def test_calls_refuse_what_the_kernels_do_not_take(call, error):
     with pytest.raises(error):
         call()
+
+
+def _moe(call, wtype, size):
+    """an MoE FFN call whose workspace is a byte short"""
+    E = types.SimpleNamespace(wtype=wtype, E=4, N=256, K=256, ptr=0, layout="gemm")
+    need = getattr(_lib.lib(), size)(3, 256, 256, 4, 2)
+    return lambda: call(E, E, E, torch.zeros(3, 256), torch.zeros((3, 2), dtype=torch.int32), torch.zeros(3, 2), workspace=torch.empty(need - 1, dtype=torch.uint8))
+
+
+def _short(size):
+    return torch.empty(size - 1, dtype=torch.uint8)
+
+
+@pytest.mark.parametrize("call", [
+    _moe(ql.moe_ffn_q, 0, "mllm_hip_moe_workspace_bytes"), _moe(ql.moe_ffn_q_gemm, 0, "mllm_hip_moe_gemm_workspace_bytes"), _moe(ql.moe_ffn_kq, 2, "mllm_hip_moe_kq_workspace_bytes"),
+    lambda: ql.w8a8_linear(X, torch.zeros((64, 64), dtype=torch.int8), X, workspace=_short(_lib.lib().mllm_hip_w8a8_workspace_bytes(3, 64))),
+    lambda: ql.w8a8_linear_packed(X, torch.zeros(_lib.lib().mllm_hip_w8a8_packed_bytes(64, 64), dtype=torch.uint8), 64, X,
+                                  workspace=_short(_lib.lib().mllm_hip_w8a8_workspace_bytes(3, 64)))])
+def test_a_workspace_that_is_too_small_is_refused(call):
+    """before any device call; the kernels wrote past it"""
+    with pytest.raises(_lib.HipQLinearError, match="needed"):
+        call()
+
+
+@pytest.mark.gpu
+def test_a_workspace_that_is_too_small_for_a_linear_is_refused():
+    """the calls that look at the device first: a byte short, and one sized under a form that needs no partial results.  One of another type counts in bytes"""
+    L, g = _lib.lib(), torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn((70, 512), device="cuda", generator=g)
+    room = lambda size: torch.empty(size, dtype=torch.uint8, device="cuda")  # noqa: E731
+    announce("workspaces that are too small")
+    for kq in (False, True):
+        make, wtype = (ql.PackedKWeight, ql.Q6_K) if kq else (ql.PackedQWeight, ql.Q4_0)
+        gemm, gemv = (make.synthetic(wtype, 256, 512, g, layout=layout) for layout in ("gemm", "gemv"))
+        call = ql.linear_kq_gemm if kq else ql.linear_q_gemm
+        plain = (L.mllm_hip_linear_kq_gemm_workspace_bytes if kq else L.mllm_hip_linear_q_gemm_workspace_bytes)(70, 512)
+        size = L.mllm_hip_linear_kq_gemm_short_workspace_bytes if kq else L.mllm_hip_linear_q_gemm_short_workspace_bytes
+        other, need = (ql.linear_kq, L.mllm_hip_kq_workspace_bytes(70, 512)) if kq else (ql.linear_q, L.mllm_hip_linear_q_workspace_bytes(70, 512))
+        want = call(gemm, x)
+        assert torch.equal(call(gemm, x, workspace=room(plain)), want) and torch.equal(call(gemm, x, workspace=torch.empty((plain + 3) // 4, device="cuda")), want)
+        assert torch.equal(other(gemv, x, workspace=torch.empty((need + 3) // 4, device="cuda")), other(gemv, x))
+        try:
+            assert L.mllm_hip_q_gemm_set_form(3) == 0
+            whole = size(70, 256, 512)
+            assert L.mllm_hip_q_gemm_set_form(8) == 0 and size(70, 256, 512) >= whole + 4 * 70 * 256 * 4
+            bad = [lambda: call(gemm, x, workspace=room(whole), short=True), lambda: call(gemm, x, workspace=room(size(70, 256, 512) - 1), short=True),
+                   lambda: call(gemm, x, workspace=room(plain - 1)), lambda: other(gemv, x, workspace=room(need - 1))]
+            for one in bad:
+                with pytest.raises(_lib.HipQLinearError, match="needed"):
+                    one()
+        finally:
+            assert L.mllm_hip_q_gemm_set_form(0) == 0
 
 
 def test_missing_module_fails_loudly(monkeypatch):
