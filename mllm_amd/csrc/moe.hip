@@ -1118,7 +1118,7 @@ __device__ __forceinline__ uint32_t qx_low(uint32_t v, const QXConst& c) { retur
 constexpr float QX_UNIT(int wt) { return wt == MLLM_HIP_Q4_0 ? 0.0625f : 1.f; }  // of the codes' products
 // K steps of weights and activations in flight per wave, in the 32-row and the 16-row form (512 tokens, Q4_0: 2 / 2 127.0 us for the FFN, 2 / 4
 // 125.3, 2 / 6 130; a Q8_0 wave has registers for two)
-constexpr int QX_ST(int) { return 2; }
+constexpr int QX_ST = 2;
 constexpr int QX_ST16(int wt) { return wt == MLLM_HIP_Q4_0 ? 4 : 2; }
 
 // One tile: `rows` (<= 32) sorted positions from row0 x 128 TN channels from n0, NW weight matrices (1, or gate + up).
@@ -1129,7 +1129,7 @@ __device__ __forceinline__ void qx_tile(const QXArgs& a, const int e, const int 
   constexpr int BM = 32, WN = TN * 32;
   constexpr int STAGE = BM * LDK + BM * 4;  // code rows, then the rows' scale pairs
   constexpr int QW = WT == MLLM_HIP_Q4_0 ? 1 : 2;
-  constexpr int ST = QX_ST(WT);             // K steps of weights in flight per wave
+  constexpr int ST = QX_ST;                 // K steps of weights in flight per wave
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 31, hi = lane >> 5;
@@ -1261,10 +1261,6 @@ __device__ __forceinline__ void qx_tile(const QXArgs& a, const int e, const int 
   for (int kt = 0; kt < nsteps; kt += ST) {
     kstep(std::integral_constant<int, 0>{}, kt);
     kstep(std::integral_constant<int, 1>{}, kt + 1);
-    if constexpr (ST >= 4) {
-      kstep(std::integral_constant<int, 2>{}, kt + 2);
-      kstep(std::integral_constant<int, 3>{}, kt + 3);
-    }
   }
 
   if (QX_UNIT(WT) != 1.f) {
