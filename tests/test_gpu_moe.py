@@ -73,7 +73,7 @@ def test_linear_q_gemm_any_m(wtype, M, N, K):
                                    (200, 2560, 9728), (256, 2560, 9728), (394, 2560, 9728)])
 def test_linear_q_gemm_short_batches(wtype, M, N, K):
     """short prompts with the larger workspace, against the oracle and the unsplit call; the long rows of 200 and more tokens run as K
-    ranges in separate workgroups + reduction, which the workspace has room for"""
+    ranges in separate workgroups + reduction, which the workspace has room for (256 of Q4_0 on 64 x 64 tiles by eight waves, 33.8 us against 34.8)"""
     rng = synth.rng_for(4, 600 + M + N % 97 + wtype)
     W = synth.make_weight(rng, wtype, N, K)
     w = ql.PackedQWeight(wtype, torch.from_numpy(W), layout="gemm")
@@ -81,7 +81,7 @@ def test_linear_q_gemm_short_batches(wtype, M, N, K):
     bias = rng.standard_normal(N).astype(np.float32)
     announce("linear_q_gemm short", wtype, M, N, K)
     ranges = _lib.lib().mllm_hip_q_gemm_form(wtype, M, N, K, 1) - 4
-    assert (ranges > 1) == (M >= 200 and K == 9728)
+    assert (ranges > 1) == (M >= 200 and K == 9728 and (M, wtype) != (256, 0))
     assert ranges <= 1 or (_lib.lib().mllm_hip_linear_q_gemm_short_workspace_bytes(M, N, K) >=
                            _lib.lib().mllm_hip_linear_q_gemm_workspace_bytes(M, K) + 256 + ranges * M * N * 4)
     ys = ql.linear_q_gemm(w, to_dev(x), to_dev(bias), short=True).cpu().numpy()
