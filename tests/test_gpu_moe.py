@@ -165,9 +165,9 @@ def test_q_gemm_every_form_exact(wtype, M, N, K):
         assert L.mllm_hip_q_gemm_set_form(0) == 0
 
 
-@pytest.mark.parametrize("M,N,K,form", [(1024, 1024, 416, 3), (1024, 1024, 352, 3), (1025, 1024, 416, 3), (97, 8192, 800, 3), (97, 8193, 800, 3), (100, 8188, 1024, 12),
-                                        (100, 8448, 1024, 12), (129, 4100, 1184, 8), (129, 8448, 1184, 8)])
-def test_linear_q_gemm_by_eight_and_four_waves(M, N, K, form):
+@pytest.mark.parametrize("M,N,K,form,eight", [(1024, 1024, 416, 3, 1), (1024, 1024, 352, 3, 0), (1025, 1024, 416, 3, 0), (97, 8192, 800, 3, 1), (97, 8193, 800, 3, 0),
+                                              (100, 8188, 1024, 12, 1), (100, 8448, 1024, 12, 0), (129, 4100, 1184, 8, 1), (129, 8448, 1184, 8, 0)])
+def test_linear_q_gemm_by_eight_and_four_waves(M, N, K, form, eight):
     """either side of 256 tiles of 64 x 64 and of seven K blocks (fewer blocks than waves and blocks that do not divide among them) and of 256 workgroups of ranges
     of K (ranges of two and of four K steps, the last one shorter); integers whose sums are exact in any order (scales of one, no partial sum leaves 2^24)"""
     L = _lib.lib()
@@ -181,7 +181,7 @@ def test_linear_q_gemm_by_eight_and_four_waves(M, N, K, form):
     w = ql.PackedQWeight(0, torch.from_numpy(W), layout="gemm")
     announce("q gemm by eight and four waves", M, N, K, form)
     try:
-        assert L.mllm_hip_q_gemm_set_form(form) == 0 and L.mllm_hip_q_gemm_form(0, M, N, K, 1) == form
+        assert L.mllm_hip_q_gemm_set_form(form) == 0 and (L.mllm_hip_q_gemm_form(0, M, N, K, 1), L.mllm_hip_q_gemm_eight(0, M, N, K, 1)) == (form, eight)
         assert np.array_equal(ql.linear_q_gemm(w, to_dev(x), None, ql.SCALE_IEEE, short=True).cpu().numpy(), x @ wd.T)
     finally:
         assert L.mllm_hip_q_gemm_set_form(0) == 0
@@ -189,8 +189,9 @@ def test_linear_q_gemm_by_eight_and_four_waves(M, N, K, form):
 
 @pytest.mark.parametrize("wtype,M,N,K", [(0, 180, 3120, 7680), (2, 179, 2872, 1792), (3, 112, 4336, 1280)])
 def test_linear_q_gemm_takes_64x64_tiles_by_eight_waves(wtype, M, N, K):
-    """host-only query: sizes at which ranges of K or tiles of 32 rows took 5 to 22 % longer"""
-    assert _lib.lib().mllm_hip_q_gemm_form(wtype, M, N, K, 1) == 3
+    """host-only queries: sizes at which ranges of K or tiles of 32 rows took 5 to 22 % longer"""
+    L = _lib.lib()
+    assert (L.mllm_hip_q_gemm_form(wtype, M, N, K, 1), L.mllm_hip_q_gemm_eight(wtype, M, N, K, 1)) == (3, 1)
 
 
 def test_linear_q_gemm_exact_when_operands_fit_fp16():

@@ -268,25 +268,29 @@ def test_waves_that_split_k(M):
 
 
 def test_waves_that_split_k_of_larger_tiles():
-    """tiles of 32x64, of 64x64 and of 64x128 (whole K): ragged rows and channels, N % 4 != 0, K blocks that do not divide"""
+    """tiles of 32x64, of 64x64 and of 64x128 (halves of K): ragged rows and channels, N % 4 != 0, K blocks that do not divide"""
     shapes = ((65, 3002, 576, 64), (45, 4101, 704, 64), (131, 4101, 576, 64), (97, 6002, 640, 128), (193, 6002, 576, 64), (300, 4101, 704, 64))
     assert [_lib.lib().mllm_hip_w4a16_packed_form(*s[:3]) for s in shapes] == [3, 3, 4, 4, 8, 8]
     _waves_cases(shapes)
 
 
 def test_waves_that_split_k_of_64x64_tiles_by_eight_and_four_waves():
-    """256 such tiles (eight waves) and 510 (four), ragged rows and channels, K blocks that do not divide among the waves"""
-    shapes = ((119, 8134, 1216, 64), (322, 5380, 576, 64))
-    assert [_lib.lib().mllm_hip_w4a16_packed_form(*s[:3]) for s in shapes] == [4, 4]
+    """256 such tiles (eight waves) and 510 (four), ragged rows and channels, K blocks that do not divide among the waves, and six blocks (four)"""
+    shapes = {(119, 8134, 1216, 64): 1, (322, 5380, 576, 64): 0, (66, 5457, 448, 64): 1, (65, 6419, 384, 64): 0}
+    L = _lib.lib()
+    assert {s: L.mllm_hip_w4a16_packed_eight(*s[:3]) for s in shapes} == shapes and {L.mllm_hip_w4a16_packed_form(*s[:3]) for s in shapes} == {4}
     _waves_cases(shapes)
 
 
 def test_halves_of_k():
-    """tiles of 128x128, 64x128, 128x256 and 64x384 that have a CU to themselves, by eight waves with half of K each: ragged rows and channels,
-    an odd number of K steps (the second half has one less), N % 8 != 0 (element stores); the last one past 256 tiles, by four"""
-    shapes = ((643, 4110, 576, 64), (643, 3856, 640, 64), (226, 4113, 576, 64), (225, 4104, 640, 128), (257, 3592, 576, 64),
-              (771, 7952, 576, 64), (515, 8256, 1152, 64), (451, 4110, 576, 64))
-    assert [_lib.lib().mllm_hip_w4a16_packed_form(*s[:3]) for s in shapes] == [5, 5, 8, 8, 8, 6, 9, 8]
+    """tiles of 128x128, 64x128, 128x256 and 64x384 that have a CU to themselves, by eight waves with half of K each: ragged rows and channels, N % 8 != 0
+    (element stores), 64x128 and 64x384 with an odd number of K steps (the second half has one less; K is padded to two steps of the others); one past 256 tiles and
+    one of six blocks, by four"""
+    shapes = {(643, 4110, 576, 64): (5, 1), (643, 3856, 640, 64): (5, 1), (226, 4113, 576, 64): (8, 1), (225, 4104, 640, 128): (8, 1), (257, 3592, 576, 64): (8, 1),
+              (97, 8220, 512, 64): (8, 1), (771, 7952, 576, 64): (6, 1), (642, 9729, 512, 64): (6, 1), (515, 8256, 1152, 64): (9, 1), (524, 8211, 1152, 64): (9, 1),
+              (393, 9994, 1280, 128): (9, 1), (451, 4110, 576, 64): (8, 0), (769, 9194, 384, 64): (6, 0)}
+    L = _lib.lib()
+    assert {s: (L.mllm_hip_w4a16_packed_form(*s[:3]), L.mllm_hip_w4a16_packed_eight(*s[:3])) for s in shapes} == shapes
     _waves_cases(shapes)
 
 

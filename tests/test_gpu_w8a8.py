@@ -303,10 +303,13 @@ def test_waves_that_split_k_of_larger_tiles():
 
 def test_halves_of_k():
     """tiles of 64x128 and 128x128 that have a CU to themselves, by eight waves with half of K each: ragged rows and channels, an odd number of K
-    steps (the second half has one less), N % 8 != 0 (element stores); the last one of each past 256 tiles, by four"""
-    shapes = ((99, 4116, 704), (98, 4172, 640), (129, 3288, 704), (105, 4128, 640), (451, 4110, 640),
-              (834, 3869, 1216), (833, 3872, 1216), (900, 3723, 1088), (841, 3984, 1088), (838, 4100, 704))
-    assert [_lib.lib().mllm_hip_w8a8_packed_form(*s) for s in shapes] == [4] * 5 + [5] * 5
+    steps (the second half has one less), N % 8 != 0 (element stores); beside them, by four, too few blocks of K and more than 256 tiles"""
+    shapes = {(99, 4116, 704): (4, 1), (98, 4172, 640): (4, 0), (129, 3288, 704): (4, 1), (105, 4128, 640): (4, 0), (451, 4110, 640): (4, 0),
+              (66, 5589, 832): (4, 1), (65, 5608, 832): (4, 1), (193, 8405, 768): (4, 0),
+              (834, 3869, 1216): (5, 1), (833, 3872, 1216): (5, 1), (900, 3723, 1088): (5, 0), (841, 3984, 1088): (5, 0), (838, 4100, 704): (5, 0),
+              (323, 8603, 1344): (5, 1), (327, 8592, 1344): (5, 1), (1163, 6408, 1216): (5, 0)}
+    L = _lib.lib()
+    assert {s: (L.mllm_hip_w8a8_packed_form(*s), L.mllm_hip_w8a8_packed_halves(*s)) for s in shapes} == shapes
     _waves_cases(shapes)
 
 
