@@ -1070,7 +1070,7 @@ static int launch_qg(const QG2Args& a, unsigned max_tiles, hipStream_t st) {
 // Codes as fp16 numbers (offsets in the mantissas of 1024 and 64) gave the sums as floats at 3.5 matrix instructions per block, but in
 // 242 registers, and more than there are for Q8_0: two waves per SIMD, and a wave's own chain of instructions was what a workgroup took, with a neighbour or
 // without (Q4_0 26 us, Q8_0 with registers in memory 70).  us of an FFN of 128 experts of 2048 x 768, top-8, before / now: 512 tokens
-// Q4_0 146 / 125, Q8_0 281 / 175; 128 tokens Q4_0 97 / 87; 317 tokens, top-4, 512 elements Q8_0 143 / 102.
+// Q4_0 145 / 122, Q8_0 269 / 173; 128 tokens Q4_0 102 / 95; 317 tokens, top-4, 512 elements Q8_0 149 / 105 (in a graph, routing and activations in it).
 // =========================================================================================================
 struct QXArgs {
   const char* W0;        // gemm-packed weights of matrix 0 (gate, or the only matrix), expert e at W0 + e * wstride
@@ -1116,8 +1116,8 @@ __device__ __forceinline__ QXConst qx_const() {
 __device__ __forceinline__ uint32_t qx_high(uint32_t v, const QXConst& c) { return (v & c.m) ^ c.x; }
 __device__ __forceinline__ uint32_t qx_low(uint32_t v, const QXConst& c) { return qx_high(v << 4, c); }
 constexpr float QX_UNIT(int wt) { return wt == MLLM_HIP_Q4_0 ? 0.0625f : 1.f; }  // of the codes' products
-// K steps of weights and activations in flight per wave, in the 32-row and the 16-row form (512 tokens, Q4_0: 2 / 2 127.0 us for the FFN, 2 / 4
-// 125.3, 2 / 6 130; a Q8_0 wave has registers for two)
+// K steps of weights and activations in flight per wave, in the 32-row and the 16-row form (512 tokens, Q4_0, of the FFN's time with 2 / 4: 2 / 2
+// 1.014, 2 / 6 1.04; a Q8_0 wave has registers for two)
 constexpr int QX_ST = 2;
 constexpr int QX_ST16(int wt) { return wt == MLLM_HIP_Q4_0 ? 4 : 2; }
 
@@ -1828,9 +1828,9 @@ __global__ __launch_bounds__(256) void qg_reduce_kernel(const float* __restrict_
 // 4B layer at 128 rows: 38, down: 10), so there is a choice:
 //   waves   the waves of a workgroup split K of a small tile (wk_gemm.h; forms 0..2 of launch_q_waves)
 //   halves  128 x 256 tiles by eight waves, four for each half of K: two waves per SIMD where a tile has a CU to itself
-//   ranges  128 x 256 tiles by four waves, K cut into up to eight ranges that run as separate workgroups, leave partial results and
-//           are added by a small second kernel in range order; one range: the plain form, with half-height tiles for a short
-//           last round
+//   ranges  128 x 256 tiles, K cut into up to eight ranges that run as separate workgroups (of eight waves, halves of a range each, while all have a CU to
+//           themselves, q_ranges_in_halves; else of four), leave partial results and are added by a small second kernel in range order; one range: the plain
+//           form by four waves, with half-height tiles for a short last round
 // 131 x 2560 x 9728 (Q6_K, with the activations' kernel): 33.6 -> 23.2 us, 93 x 6144 x 2048 (Q4_0) 27 -> 14, 700 x 6144 x 2048 43.7 -> 39,
 // 2048 x 2048 x 6144 102 -> 80.
 struct QLinearPlan {
@@ -1847,7 +1847,7 @@ static bool q_ranges_exist(int64_t N, int64_t blocks, int z) {  // whole even ra
 // weights of 512 to 9728 either way; the rms errors stand in the table).  Over 1360 such shapes the form chosen takes 1.005 times the best
 // form's time on average (19 % more at worst) and is more than 2 % slower than the one range or the ranges by rows and columns alone that
 // ran before in 5 of them (595 x 1016 x 8704 Q4_K 37.4 -> 39.3 us at most); from 33 to 4096 rows of up to 151 936 channels 3 of 520 (404 x
-// 17776 x 512 Q4_K 29.3 -> 32.9).  With one table for all formats, K products and ragged last tiles at a price, a choice was up to 18 %
+// 17776 x 512 Q4_K 29.3 -> 32.9).  The costs of ranges are those of four waves; eight take 0.95 of them.  With one table for all formats, K products and ragged last tiles at a price, a choice was up to 18 %
 // slower than those (63 x 9328 x 8704 Q6_K 41.4 -> 48.9, 345 x 1480 x 8704 Q6_K 33.9 -> 39.1, 424 x 6432 x 5376 Q4_K 56.2 -> 63.3).
 struct QFormCost {
   float waves[3][6];  // per form: how a partly filled last round counts, fixed, round, round and 64 of K, 1e6 M K (read again by every
