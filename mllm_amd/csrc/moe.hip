@@ -1909,13 +1909,16 @@ static QLinearPlan q_linear_plan(int wtype, int64_t M, int64_t N, int64_t K, boo
   for (int f = 0; f < 3; f++) {
     const int64_t tiles = ((M + rows[f] - 1) / rows[f]) * ((N + chans[f] - 1) / chans[f]);
     const float cost = whole(c.waves[f], (float)((tiles + 255) / 256), (float)tiles / 256.f);
-    const float eight = f == 2 && wk_eight(M, N, blocks) ? c.eight * (float)blocks : 0.f;
+    // (activation rows that straddle cache lines and lie within 256 bytes of a multiple of 16 KB apart share a few of the caches' sets, twice the lines each: with
+    // more than 512 rows 64 x 64 takes up to 1.42 of the time of ranges there, 1287 x 712 x 8160 Q4_0 64.3 us / 45.4; K a multiple of 64 0.87)
+    const bool crowded = M > 512 && K % 64 != 0 && (2 * K + 256) % 16384 <= 512;
+    const float eight = f == 2 && wk_eight(M, N, blocks) ? c.eight * (float)blocks - (crowded ? 0.4f * cost : 0.f) : 0.f;
     offer(cost - eight, QLinearPlan{f, 0, 1});
     // One tile of rows and long K, where the weights' bytes are the bound: ranges by eight waves are faster than their costs, which are those of four, by 6 %, and the
     // longer K is beyond the 9728 that they were fitted to, the more so: nibbles from there on (63 x 9224 x 15 456 Q4_0 43.1 us on 64 x 64, 35.6), bytes from about
     // 17 000 (47 x 15 080 x 18 976 Q8_0 83.2, 76.1; up to 16 000 64 x 64 is 0.91 of ranges).  A margin of 1.06 for all sizes kept ranges for 1400 shapes that were
     // 1.11 of the time of the eight waves on 64 x 64 (130 x 3544 x 5632 Q6_K 29.1 us, 22.5; 256 x 2560 x 9728 Q4_0 34.8, 33.8); without any, 8 shapes of more rows
-    // are 3 to 15 % slower, all of K near 8192.
+    // are 3 to 15 % slower, all of K near 8192 (above).
     if (best.waves == 2 && eight > 0.f && M <= 64 && blocks >= 120) {
       const float margin = qg_nibbles(wtype) ? 1.f + 0.0015f * (float)(blocks - 90) : blocks < 260 ? 1.06f : 1.2f;
       least = std::min(cost, margin * least);

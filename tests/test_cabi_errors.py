@@ -271,10 +271,12 @@ def test_topk_is_cut_into_pieces_only_where_that_is_faster():
 @pytest.mark.parametrize("wtype,M,N,K,forms", [
     (Q6_K, 54, 6144, 2048, (2,)), (Q6_K, 138, 2288, 1536, (2,)), (Q4_K, 394, 2560, 9728, (10,)), (Q4_0, 415, 5640, 8768, (9,)),
     (Q6_K, 316, 8880, 7424, (6, 8)), (Q4_0, 1956, 760, 4832, (8, 9, 10)), (Q6_K, 114, 2560, 9728, (2,)), (Q6_K, 130, 3544, 5632, (3,)),
-    (Q8_0, 135, 3856, 5760, (3,)), (Q4_0, 256, 2560, 9728, (3,)), (Q4_0, 41, 8504, 9600, (11,)), (Q4_K, 33, 8376, 8448, (11,))])
+    (Q8_0, 135, 3856, 5760, (3,)), (Q4_0, 256, 2560, 9728, (3,)), (Q4_0, 41, 8504, 9600, (11,)), (Q4_K, 33, 8376, 8448, (11,)),
+    (Q4_0, 1287, 712, 8160, (11,)), (Q4_0, 1028, 728, 8224, (12,)), (Q4_0, 1287, 712, 8192, (3,))])
 def test_q_gemm_takes_a_form_that_measures_fast(wtype, M, N, K, forms):
     """shapes at which a choice by rows, columns and K steps alone was 10 to 23 % slower than the forms here (measured, all twelve), and at which ranges by
-    a margin over 64 x 64 tiles took 3 to 29 % longer or, at the last two, those tiles 10 %"""
+    a margin over 64 x 64 tiles took 3 to 29 % longer or, at two of one tile of rows, those tiles 10 %; rows near 16 KB apart that straddle cache lines (42 and
+    31 %) and one that does not"""
     assert _lib.lib().mllm_hip_q_gemm_form(wtype, M, N, K, 1) in forms
     assert _lib.lib().mllm_hip_q_gemm_form(wtype, M, N, K, 0) <= 5  # no room for partial results: no ranges
 
