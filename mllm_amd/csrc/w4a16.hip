@@ -732,8 +732,9 @@ static int w4a16_packed_form(int64_t M, int64_t N, int64_t K, bool tiles_only) {
   // What eight waves save comes off: halves of K as above; 64 x 64 fitted to 70 shapes of 100 to 256 such tiles, 2.2 % rms; over 250 shapes the choice takes
   // 0.981 of the time with four waves throughout, 41 of them 3 to 20 % less (119 x 7224 x 4416 20.6 -> 17.1 us).  Where a form of the waves that split K is the
   // cheapest by four, halves of K of a tile take its place only
-  //  * with 2 us per million results added where rows are no multiple of 16 bytes: the tiles store those an element at a time (1.4 to 3 us by form, the
-  //    waves' forms nothing), which had 40 of 372 such shapes 3 to 25 % slower (778 x 1915 x 1792 15.2 -> 19.1 us); 6 are 3 to 7 % slower with it
+  //  * with 2.8 us per million results added where rows are no multiple of 16 bytes: the tiles store those an element at a time (1.4 to 3 us by form, the
+  //    waves' forms nothing), which had 40 of 372 such shapes 3 to 25 % slower (778 x 1915 x 1792 15.2 -> 19.1 us); not
+  //    for many rows of long K, where the waves' forms take more than their costs.  Over 1872 such shapes 0.896 of the time of four waves, 20 of them 3 to 9 % slower
   //  * on 128 x 128 at 0.94 of the cost: at 0.95 to 0.975 of 32 x 64's 9 of 12 shapes were 2 to 7 % slower (258 x 6832 x 5120 39.8 -> 42.8)
   auto cheapest = [&](bool eight, bool split) {
     int form = -1;
@@ -743,7 +744,7 @@ static int w4a16_packed_form(int64_t M, int64_t N, int64_t K, bool tiles_only) {
       if (eight) {
         c -= w4a16_halves_gain(f, M, N, K);
         if (f == 3 && ((M + 63) / 64) * ((N + 63) / 64) <= WK_EIGHT_TILES) c -= 0.0322f * (float)((K + 63) / 64);
-        if (split && f >= waves && N % 8 != 0) c += 2e-6f * (float)(M > 32 ? M : 32) * (float)N;
+        if (split && f >= waves && N % 8 != 0 && (M < 900 || K < 3000)) c += 2.8e-6f * (float)(M > 32 ? M : 32) * (float)N;
         if (split && f == waves) c *= 1.06f;
       }
       if (form < 0 || c < best) {
