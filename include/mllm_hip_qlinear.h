@@ -312,8 +312,8 @@ int mllm_hip_w8a8_set_decode_mfma_from(int tokens);
 int mllm_hip_w8a8_nsplit_set_tuning(int tile);
 /* The form that a product of this size takes against prepacked weights: 1 / 2 / 3 waves that split K of a tile of 32x32 / 32x64 / 64x64, 4 / 5 / 6 /
  * 7 / 8 tiles of 64x128 / 128x128 / 128x256 / 64x384 / 128x384, 9 the dot form.  mllm_hip_w8a8_packed_halves: 1 where the tile (of 64x128 or 128x128)
- * runs by eight waves with half of K each: every tile has a CU to itself and K more than 640 or 1152.  Host only, overrides aside.  No counterpart
- * in the reference. */
+ * runs by eight waves with half of K each: every tile has a CU to itself and K is more than 640 or 1152 (one tile of rows and more than 192 of channels:
+ * more than 2944).  Host only, overrides aside.  No counterpart in the reference. */
 int mllm_hip_w8a8_packed_form(int64_t M, int64_t N, int64_t K);
 int mllm_hip_w8a8_packed_halves(int64_t M, int64_t N, int64_t K);
 
